@@ -2,8 +2,9 @@
 
 The reference runs all of them through cuBLAS (nn.Linear / F.linear,
 lite_llama/models/llama.py:37-40,61,120,221). Here: float32 always goes through
-the package's own vector-FMA kernel (a true 32-bit product, no reduced-precision
-matrix mode can be switched on underneath it); bfloat16 uses the package's
+the package's own kernels (true 32-bit products and sums, on the matrix cores where
+rows are aligned; no reduced-precision matrix mode can be switched on underneath
+them); bfloat16 uses the package's
 skinny weight-streaming kernel for the few rows of a decode step and the
 library product (hipBLASLt, called directly: ops.gemm_library) for the many rows
 of a prompt.
@@ -16,7 +17,7 @@ import torch
 
 from .. import ops
 
-LINEAR_LIBRARIES = ("gemm", "gemm_rows", "blaslt")
+LINEAR_LIBRARIES = ("gemm", "gemm_f32", "gemm_rows", "blaslt")
 SKINNY_ROWS = 8          # rows up to which the skinny kernel takes a bfloat16 product
 SKINNY_ROWS_F32 = 16     # ... when float32 output is wanted (the head)
 

@@ -101,6 +101,36 @@ def test_gemm_nt(ops, dtype, mnk):
                                **tol(dtype))
 
 
+@pytest.mark.parametrize("mnk", [
+    # few rows: one piece of K, a row and a column past a tile, several waves with a short last one, 8-row tiles
+    # with one and with two tiles of x, 16-row tiles
+    (1, 8, 4), (8, 9, 68), (7, 2049, 2052), (9, 70, 1028), (16, 2048, 4100), (16, 3073, 516), (12, 5000, 260),
+    # many rows: one and just over one tile, K short of and past a step, cuts along K with a short last one
+    (17, 16, 4), (64, 64, 32), (65, 129, 36), (129, 66, 2052), (33, 515, 8196), (700, 1000, 96), (1030, 2100, 260)])
+def test_gemm_f32_matrix_cores(ops, mnk):
+    """The float32 products on the matrix cores, and the vector kernel on the same operands shifted by one
+    float (rows that are not aligned), element by element within the bound of a float32 sum of K products
+    in any order: (K + 1) 2^-24 sum |x w|."""
+    M, N, K = mnk
+    torch.manual_seed(9)
+    wide = torch.randn(M, K + 8, device="cuda")
+    w = torch.randn(N, K, device="cuda")
+    for x in (wide[:, 4:4 + K], wide[:, 4:4 + K].contiguous(), wide[:, 3:3 + K]):
+        want = x.double() @ w.double().T
+        bound = (K + 1) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)
+        out = torch.full((M, N + 3), 7.0, device="cuda")
+        y = ops.gemm_nt(x, w, out=out[:, :N])
+        assert ((y.double() - want).abs() <= bound).all()
+        assert (out[:, N:] == 7.0).all()
+    # what is not finite stays in its row of x and its row of w
+    x = wide[:, 4:4 + K].contiguous()
+    x[M - 1, K - 1] = float("inf")
+    w[N - 1, 0] = float("nan")
+    y = ops.gemm_nt(x, w)
+    assert torch.isnan(y[:, N - 1]).all() and torch.isfinite(y[:M - 1, :N - 1]).all()
+    assert (~torch.isfinite(y[M - 1])).all()
+
+
 @pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float32], ids=["to_bf16", "to_fp32"])
 @pytest.mark.parametrize("mnk", [(1, 300, 72), (7, 65, 136), (16, 3072, 2048), (17, 100, 200),
                                  (33, 16, 8192), (64, 1000, 64), (8, 2048, 8192), (5, 130, 2056),
@@ -128,6 +158,36 @@ def test_gemm_skinny(ops, out_dtype, mnk):
         ops.gemm_skinny(torch.zeros(65, K, device="cuda", dtype=torch.bfloat16), w)
     with pytest.raises(ops.KernelError):
         ops.gemm_skinny(x[:, :K - 4], w[:, :K - 4].contiguous())
+
+
+@pytest.mark.parametrize("mnk", [
+    # few rows: one piece of K, a row and a column past a tile, several waves with a short last one, 8-row tiles
+    # with one and with two tiles of x, 16-row tiles
+    (1, 8, 4), (8, 9, 68), (7, 2049, 2052), (9, 70, 1028), (16, 2048, 4100), (16, 3073, 516), (12, 5000, 260),
+    # many rows: one and just over one tile, K short of and past a step, cuts along K with a short last one
+    (17, 16, 4), (64, 64, 32), (65, 129, 36), (129, 66, 2052), (33, 515, 8196), (700, 1000, 96), (1030, 2100, 260)])
+def test_gemm_f32_matrix_cores(ops, mnk):
+    """The float32 products on the matrix cores, and the vector kernel on the same operands shifted by one
+    float (rows that are not aligned), element by element within the bound of a float32 sum of K products
+    in any order: (K + 1) 2^-24 sum |x w|."""
+    M, N, K = mnk
+    torch.manual_seed(9)
+    wide = torch.randn(M, K + 8, device="cuda")
+    w = torch.randn(N, K, device="cuda")
+    for x in (wide[:, 4:4 + K], wide[:, 4:4 + K].contiguous(), wide[:, 3:3 + K]):
+        want = x.double() @ w.double().T
+        bound = (K + 1) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)
+        out = torch.full((M, N + 3), 7.0, device="cuda")
+        y = ops.gemm_nt(x, w, out=out[:, :N])
+        assert ((y.double() - want).abs() <= bound).all()
+        assert (out[:, N:] == 7.0).all()
+    # what is not finite stays in its row of x and its row of w
+    x = wide[:, 4:4 + K].contiguous()
+    x[M - 1, K - 1] = float("inf")
+    w[N - 1, 0] = float("nan")
+    y = ops.gemm_nt(x, w)
+    assert torch.isnan(y[:, N - 1]).all() and torch.isfinite(y[:M - 1, :N - 1]).all()
+    assert (~torch.isfinite(y[M - 1])).all()
 
 
 @pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float32], ids=["to_bf16", "to_fp32"])
