@@ -7,6 +7,7 @@
 // matrix path of the true 32-bit mode (no reduced-precision matrix mode can
 // hide in it) and the fallback of the bfloat16 mode.
 #include "common.h"
+#include "device.h"
 #include <stdlib.h>
 
 #define TM 64
@@ -345,27 +346,6 @@ gemm_skinny_kernel(TY* __restrict__ y, const bf16_t* __restrict__ x, const bf16_
       if (4 * lg + i < ROWS && n < N) y[(size_t)m * ldy + n] = from_float<TY>(acc[t][i]);
     }
   }
-}
-
-// Compute units of the current device (256 on MI355X), asked for once a device: the launch
-// rules below were measured there and are stated in compute units, not as numbers of that chip.
-static int compute_units() {
-  constexpr int MAX_DEVICES = 64;
-  static int cached[MAX_DEVICES];
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= MAX_DEVICES) {
-    (void)hipGetLastError();
-    return 256;
-  }
-  if (cached[dev] == 0) {
-    int n = 0;
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) {
-      (void)hipGetLastError();
-      n = 256;
-    }
-    cached[dev] = n;
-  }
-  return cached[dev];
 }
 
 template <int MT, int U, int ROWS>

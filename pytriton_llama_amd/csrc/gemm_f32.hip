@@ -7,17 +7,10 @@
 // operands follow it, so a lane always loads four consecutive k in one 16-byte load and hands them
 // to four matrix instructions one after the other.
 #include "common.h"
+#include "device.h"
+#include "mfma_f32.h"
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
-
-union F4 {
-  uint4 u;
-  float f[4];
-};
-
-// (a value and not an lvalue: ``ok ? *p : zero`` of two lvalues would choose between addresses)
-__device__ __forceinline__ uint4 load16(const float* p) { return *reinterpret_cast<const uint4*>(p); }
-__device__ __forceinline__ uint4 zero16() { return make_uint4(0, 0, 0, 0); }
 
 // ===========================================================================
 // Few rows of x (M <= 16, a decode step): bound by reading W once. A workgroup owns ROWS rows of W;
@@ -116,27 +109,6 @@ gemm_f32_few_kernel(float* __restrict__ y, const float* __restrict__ x, const fl
   }
 }
 
-// Compute units of the current device (256 on MI355X), asked for once a device: the launch
-// rules below were measured there and are stated in compute units, not as numbers of that chip.
-static int compute_units() {
-  constexpr int MAX_DEVICES = 64;
-  static int cached[MAX_DEVICES];
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= MAX_DEVICES) {
-    (void)hipGetLastError();
-    return 256;
-  }
-  if (cached[dev] == 0) {
-    int n = 0;
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) {
-      (void)hipGetLastError();
-      n = 256;
-    }
-    cached[dev] = n;
-  }
-  return cached[dev];
-}
-
 static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
 // M <= 16, K % 4 == 0, ldx % 4 == 0, x and w 16-byte aligned.
@@ -171,14 +143,10 @@ extern "C" int ptl_gemm_f32_few(float* y, const float* x, const float* w, int M,
 
 // ===========================================================================
 // Many rows of x (a prompt portion): tiles of BN rows of W x BM rows of x a workgroup of four waves
-// (two along each side), BK columns of K at a time through LDS, two buffers: the next tile is on its
+// (two along each side), F32_BK columns of K at a time through LDS, two buffers: the next tile is on its
 // way from memory to registers while this one is multiplied, one barrier a tile.
-// v_mfma_f32_32x32x2_f32: lane l (r = l % 32, h = l / 32) holds A[r][k = h] and B[k = h][r], gets
-// D[8 (i / 4) + 4 h + i % 4][r], i = 0..15. A wave of the largest tile multiplies 64 x 64: for 8
-// columns it reads four 16-byte fragments a lane and issues 16 instructions of 64 clocks each, so the
-// matrix cores and nothing else bound it. Rows of 32 floats lie unpadded in LDS, the 16-byte pieces
-// of a row permuted by (row / 2) % 8: eight neighbouring lanes then touch all banks once, writing
-// along a row and reading down a column of pieces alike.
+// A wave of the largest tile multiplies 64 x 64: for 8 columns it reads four 16-byte fragments a lane and
+// issues 16 matrix instructions of 64 clocks each (mfma_f32.h), so the matrix cores bound it.
 //
 // A grid of few tiles is cut along K as well (blockIdx.y): the parts of the sums go to a workspace
 // [splits, M, N] and a second kernel adds them in order.
@@ -187,11 +155,6 @@ extern "C" int ptl_gemm_f32_few(float* y, const float* x, const float* w, int M,
 // 112 TFLOP/s (1,386), 700 x 2,048 x 8,192 230 (1,251), 700 x 3,072 x 2,048 100 (370), 483 x 1,536 x 2,048
 // 38 (224), 64 x 2,048 x 8,192 33 (967). Relative error against 64 bits at K = 2,048: 3.7e-7 (8.1e-7).
 // ===========================================================================
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-#define BK 32
-
-__device__ __forceinline__ int lds_piece(int row, int piece) { return row * 8 + (piece ^ ((row >> 1) & 7)); }
-
 template <int BN, int BM>
 __global__ void __launch_bounds__(256)
 gemm_f32_tile_kernel(float* __restrict__ y, const float* __restrict__ x, const float* __restrict__ w,
@@ -226,43 +189,30 @@ gemm_f32_tile_kernel(float* __restrict__ y, const float* __restrict__ x, const f
   };
   auto put = [&](int b) {
 #pragma unroll
-    for (int i = 0; i < BN / 32; ++i) ws[b][lds_piece(row + 32 * i, piece)] = wr[i];
+    for (int i = 0; i < BN / 32; ++i) ws[b][f32_piece(row + 32 * i, piece)] = wr[i];
 #pragma unroll
-    for (int i = 0; i < BM / 32; ++i) xs[b][lds_piece(row + 32 * i, piece)] = xr[i];
+    for (int i = 0; i < BM / 32; ++i) xs[b][f32_piece(row + 32 * i, piece)] = xr[i];
   };
-  f32x16 acc[TN][TM];
+  f32x16_t acc[TN][TM];
 #pragma unroll
   for (int a = 0; a < TN; ++a)
 #pragma unroll
     for (int b = 0; b < TM; ++b)
 #pragma unroll
       for (int i = 0; i < 16; ++i) acc[a][b][i] = 0.f;
-  F4 fa[2][TN], fb[2][TM];
-  auto read = [&](int set, int b, int g) {       // the fragments of columns 8 g .. 8 g + 7
+  int nrow[TN], mrow[TM];
 #pragma unroll
-    for (int a = 0; a < TN; ++a) fa[set][a].u = ws[b][lds_piece(wn + 32 * a + lr, 2 * g + lh)];
+  for (int a = 0; a < TN; ++a) nrow[a] = wn + 32 * a;
 #pragma unroll
-    for (int c = 0; c < TM; ++c) fb[set][c].u = xs[b][lds_piece(wm + 32 * c + lr, 2 * g + lh)];
-  };
+  for (int c = 0; c < TM; ++c) mrow[c] = wm + 32 * c;
   fetch(kb);
   put(0);
   __syncthreads();
   int buf = 0;
-  for (int k = kb; k < ke; k += BK, buf ^= 1) {
-    const bool more = k + BK < ke;
-    if (more) fetch(k + BK);
-    read(0, buf, 0);
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      if (g < 3) read((g + 1) & 1, buf, g + 1);
-#pragma unroll
-      for (int s = 0; s < 4; ++s)
-#pragma unroll
-        for (int a = 0; a < TN; ++a)
-#pragma unroll
-          for (int c = 0; c < TM; ++c)
-            acc[a][c] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[g & 1][a].f[s], fb[g & 1][c].f[s], acc[a][c], 0, 0, 0);
-    }
+  for (int k = kb; k < ke; k += F32_BK, buf ^= 1) {
+    const bool more = k + F32_BK < ke;
+    if (more) fetch(k + F32_BK);
+    f32_multiply<TN, TM>(acc, ws[buf], xs[buf], nrow, mrow, lane);
     if (more) put(buf ^ 1);
     __syncthreads();
   }
@@ -313,6 +263,11 @@ gemm_f32_sum_kernel(float* __restrict__ y, const float* __restrict__ parts, int 
   }
 }
 
+// Sums of fewer products than this are added up in one order whatever the number of rows (every tile
+// walks K alike), so that a request's results do not depend on what else is in its step; ops.gemm_nt
+// keeps them off the kernel for few rows as well.
+#define F32_ONE_ORDER_K 512
+
 struct TilePlan {
   int bn, bm, splits;
 };
@@ -320,11 +275,12 @@ struct TilePlan {
 // The tile and the number of cuts along K that a count of the work says are done first. The four
 // waves of a workgroup take the four SIMDs of a compute unit, so what counts is the fullest unit: r
 // workgroups, one after the other, at 0.5 TFLOP/s (128 TFLOP/s on 256 units), each with about two
-// steps of BK lost at its start and end; less than three at a time on a unit leave gaps (one alone
+// steps of F32_BK lost at its start and end; less than three at a time on a unit leave gaps (one alone
 // takes 1.6 times as long). A cut costs the second kernel and the traffic of the partial sums.
 // Against a sweep of the three tiles with 1 to 16 cuts (M 64 to 700, N 16 to 16,384, K 2,048 and
 // 8,192; one MI355X) the plan is within 6 % of the fastest; without cuts 483 x 1,536 x 2,048 takes 53
-// instead of 38 us, 64 x 2,048 x 8,192 takes 140 instead of 33.
+// instead of 38 us, 64 x 2,048 x 8,192 takes 140 instead of 33. Sums of fewer than F32_ONE_ORDER_K products
+// are never cut.
 static TilePlan tile_plan(int M, int N, int K) {
   const int cus = compute_units();
   static const struct { int bn, bm; } shapes[] = {{64, 64}, {128, 64}, {128, 128}};
@@ -333,9 +289,9 @@ static TilePlan tile_plan(int M, int N, int K) {
   for (const auto& s : shapes) {
     const long tiles = (long)((N + s.bn - 1) / s.bn) * ((M + s.bm - 1) / s.bm);
     for (int splits = 1; splits <= 16; ++splits) {
-      const int per = ((K + splits - 1) / splits + BK - 1) / BK * BK;
-      if (splits > 1 && (per < 4 * BK || (long)per * (splits - 1) >= K)) continue;
-      const double one = 2.0 * s.bn * s.bm * (per + 2 * BK) / 0.5e12;
+      const int per = ((K + splits - 1) / splits + F32_BK - 1) / F32_BK * F32_BK;
+      if (splits > 1 && (K < F32_ONE_ORDER_K || per < 4 * F32_BK || (long)per * (splits - 1) >= K)) continue;
+      const double one = 2.0 * s.bn * s.bm * (per + 2 * F32_BK) / 0.5e12;
       const double r = (double)((tiles * splits + cus - 1) / cus);
       double t = one * (r < 4 ? 0.8 * (r + 1) : r + 0.3);
       if (splits > 1) t += 4e-6 + 4.0 * M * N * (splits + 1) / 6e12;
@@ -366,7 +322,7 @@ extern "C" int ptl_gemm_f32(float* y, const float* x, const float* w, int M, int
   const int tiles_m = (M + p.bm - 1) / p.bm;
   const long tiles = (long)((N + p.bn - 1) / p.bn) * tiles_m;
   if (tiles > 0x3fffffff) return PTL_ERR_ARG;
-  const int per = ((K + p.splits - 1) / p.splits + BK - 1) / BK * BK;
+  const int per = ((K + p.splits - 1) / p.splits + F32_BK - 1) / F32_BK * F32_BK;
   float* out = p.splits > 1 ? parts : y;
   const long ld = p.splits > 1 ? N : ldy;
   const dim3 grid((unsigned)((tiles + 7) / 8 * 8), p.splits);

@@ -31,6 +31,7 @@
 // g' * sigmoid(1.702 g') * (u' + 1). Without a gate: 2: relu(u)^2.
 #include "common.h"
 #include "mfma.h"
+#include "mfma_f32.h"
 #include <math.h>
 
 #define MOE_TM 64
@@ -464,6 +465,89 @@ moe_gemm_kernel(T* __restrict__ out, long ldo, const T* __restrict__ x, long ldx
   }
 }
 
+// The same products in float32 on the matrix cores (K % 4 == 0, aligned rows): 64 sorted rows x 64
+// result columns a workgroup of four waves, each 32 x 32 of every product, F32_BK columns of K at a time
+// through LDS (mfma_f32.h), two buffers, the next step on its way to registers while this one is
+// multiplied. The gate and the up row of a result meet in one lane. 966 pairs of 16 experts of 2,048 x
+// 2,048 (one MI355X, us; the vector form in brackets): gate|up 251 (691), down 139 (419).
+template <int MODE>
+__global__ void __launch_bounds__(256)
+moe_gemm_f32_kernel(float* __restrict__ out, long ldo, const float* __restrict__ x, long ldx, const float* __restrict__ w,
+                    const int32_t* __restrict__ tile_expert, const int32_t* __restrict__ tile_row0,
+                    const int32_t* __restrict__ expert_end, const int32_t* __restrict__ sorted,
+                    const float* __restrict__ wgt, int top, int N, int K, int act, float limit) {
+  constexpr bool GATE_UP = MODE == MODE_GATE_UP;
+  constexpr bool GATHER = MODE != MODE_DOWN;
+  constexpr int G = GATE_UP ? 2 : 1;
+  const int e = tile_expert[blockIdx.y];
+  if (e < 0) return;
+  __shared__ uint4 ws[2][64 * G * 8];
+  __shared__ uint4 xs[2][64 * 8];
+  const int row0 = tile_row0[blockIdx.y];
+  const int rows = min(MOE_TM, expert_end[e] - row0);
+  const int n0 = blockIdx.x * 64;
+  w += (size_t)e * G * N * K;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int piece = tid & 7, row = tid >> 3;     // of a step's 16-byte pieces, those of rows row + 32 i
+  const float* wp[2 * G];
+  const float* xp[2];
+#pragma unroll
+  for (int i = 0; i < 2 * G; ++i)
+    wp[i] = w + ((size_t)(i >> 1) * N + min(n0 + row + 32 * (i & 1), N - 1)) * K + 4 * piece;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    // (a row past the tile's end repeats the last: its results are not stored)
+    const int at = row0 + min(row + 32 * i, rows - 1);
+    xp[i] = x + (size_t)(GATHER ? sorted[at] / top : at) * ldx + 4 * piece;
+  }
+  uint4 wr[2 * G], xr[2];
+  auto fetch = [&](int k) {
+    const bool ok = k + 4 * piece < K;
+#pragma unroll
+    for (int i = 0; i < 2 * G; ++i) wr[i] = ok ? load16(wp[i] + k) : zero16();
+#pragma unroll
+    for (int i = 0; i < 2; ++i) xr[i] = ok ? load16(xp[i] + k) : zero16();
+  };
+  auto put = [&](int b) {
+#pragma unroll
+    for (int i = 0; i < 2 * G; ++i) ws[b][f32_piece(row + 32 * i, piece)] = wr[i];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) xs[b][f32_piece(row + 32 * i, piece)] = xr[i];
+  };
+  f32x16_t acc[G][1];
+#pragma unroll
+  for (int g = 0; g < G; ++g)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc[g][0][i] = 0.f;
+  const int cn = 32 * (wave & 1), cm = 32 * (wave >> 1);
+  int wrow[G];
+#pragma unroll
+  for (int g = 0; g < G; ++g) wrow[g] = 64 * g + cn;
+  const int xrow[1] = {cm};
+  fetch(0);
+  put(0);
+  __syncthreads();
+  int buf = 0;
+  for (int k = 0; k < K; k += F32_BK, buf ^= 1) {
+    const bool more = k + F32_BK < K;
+    if (more) fetch(k + F32_BK);
+    f32_multiply<G, 1>(acc, ws[buf], xs[buf], wrow, xrow, lane);
+    if (more) put(buf ^ 1);
+    __syncthreads();
+  }
+  const int m = cm + (lane & 31), lh = lane >> 5;
+  if (m >= rows) return;
+  const float f = GATHER && wgt ? wgt[sorted[row0 + m]] : 1.f;
+  float* orow = out + (size_t)(row0 + m) * ldo;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const int n = n0 + cn + 8 * (i >> 2) + 4 * lh + (i & 3);
+    if (n >= N) continue;
+    orow[n] = GATE_UP ? gated_act(act, acc[0][0][i] * f, acc[G - 1][0][i] * f, limit)
+                      : (MODE == MODE_UP ? unary_act(act, acc[0][0][i] * f) : acc[0][0][i]);
+  }
+}
+
 // Matrix-core forms for bfloat16 (K % 8 == 0, aligned rows).
 //
 // Few pairs (a decode step): fragments straight from memory, FEW_COLS result columns a workgroup. A
@@ -754,6 +838,10 @@ static bool mfma_ok(const void* x, long ldx, const void* w, int K) {
   return K % 8 == 0 && ldx % 8 == 0 && ((uintptr_t)x | (uintptr_t)w) % 16 == 0;
 }
 
+static bool mfma_f32_ok(const void* x, long ldx, const void* w, int K) {
+  return K % 4 == 0 && ldx % 4 == 0 && ((uintptr_t)x | (uintptr_t)w) % 16 == 0;
+}
+
 // out [A, I] (sorted order) = act(w_a * x[token] Wg_e^T, w_a * x[token] Wu_e^T); w [E, 2 I, K];
 // wgt null: the routing weight is not applied here.
 extern "C" int ptl_moe_gate_up(void* out, long ldo, const void* x, long ldx, const void* w,
@@ -764,7 +852,10 @@ extern "C" int ptl_moe_gate_up(void* out, long ldo, const void* x, long ldx, con
   if (max_tiles <= 0) return PTL_OK;
   if (I <= 0 || K <= 0 || top <= 0 || max_tiles > 65535) return PTL_ERR_ARG;
   dim3 grid((I + 63) / 64, max_tiles), few((I + FEW_COLS - 1) / FEW_COLS, max_tiles);
-  if (dtype == PTL_DTYPE_F32)
+  if (dtype == PTL_DTYPE_F32 && mfma_f32_ok(x, ldx, w, K))
+    moe_gemm_f32_kernel<MODE_GATE_UP><<<grid, 256, 0, st>>>((float*)out, ldo, (const float*)x, ldx, (const float*)w, tile_expert,
+                                                  tile_row0, expert_end, sorted, wgt, top, I, K, act, limit);
+  else if (dtype == PTL_DTYPE_F32)
     moe_gemm_kernel<float, MODE_GATE_UP><<<grid, 256, 0, st>>>((float*)out, ldo, (const float*)x, ldx, (const float*)w,
                                                        tile_expert, tile_row0, expert_end, sorted, wgt, top, I,
                                                        K, act, limit);
@@ -796,7 +887,10 @@ extern "C" int ptl_moe_up(void* out, long ldo, const void* x, long ldx, const vo
   if (max_tiles <= 0) return PTL_OK;
   if (I <= 0 || K <= 0 || top <= 0 || max_tiles > 65535 || act != 2) return PTL_ERR_ARG;
   dim3 grid((I + 63) / 64, max_tiles), few((I + FEW_COLS - 1) / FEW_COLS, max_tiles);
-  if (dtype == PTL_DTYPE_F32)
+  if (dtype == PTL_DTYPE_F32 && mfma_f32_ok(x, ldx, w, K))
+    moe_gemm_f32_kernel<MODE_UP><<<grid, 256, 0, st>>>((float*)out, ldo, (const float*)x, ldx, (const float*)w, tile_expert,
+                                                  tile_row0, expert_end, sorted, wgt, top, I, K, act, 0.f);
+  else if (dtype == PTL_DTYPE_F32)
     moe_gemm_kernel<float, MODE_UP><<<grid, 256, 0, st>>>((float*)out, ldo, (const float*)x, ldx,
                                                           (const float*)w, tile_expert, tile_row0, expert_end,
                                                           sorted, wgt, top, I, K, act, 0.f);
@@ -825,7 +919,10 @@ extern "C" int ptl_moe_down(void* out, long ldo, const void* x, long ldx, const 
   if (max_tiles <= 0) return PTL_OK;
   if (N <= 0 || K <= 0 || max_tiles > 65535) return PTL_ERR_ARG;
   dim3 grid((N + 63) / 64, max_tiles), few((N + FEW_COLS - 1) / FEW_COLS, max_tiles);
-  if (dtype == PTL_DTYPE_F32)
+  if (dtype == PTL_DTYPE_F32 && mfma_f32_ok(x, ldx, w, K))
+    moe_gemm_f32_kernel<MODE_DOWN><<<grid, 256, 0, st>>>((float*)out, ldo, (const float*)x, ldx, (const float*)w, tile_expert,
+                                                  tile_row0, expert_end, nullptr, nullptr, 1, N, K, 0, 0.f);
+  else if (dtype == PTL_DTYPE_F32)
     moe_gemm_kernel<float, MODE_DOWN><<<grid, 256, 0, st>>>((float*)out, ldo, (const float*)x, ldx, (const float*)w,
                                                         tile_expert, tile_row0, expert_end, nullptr, nullptr, 1,
                                                         N, K, 0, 0.f);

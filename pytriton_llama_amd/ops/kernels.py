@@ -227,7 +227,7 @@ def gemm_nt(x: torch.Tensor, w: torch.Tensor, out_dtype: Optional[torch.dtype] =
     if x.dtype == torch.float32 and _gemm_f32_fits(x, w, M, K):
         lib = library.load("gemm_f32")
         ldx, ldy = ctypes.c_long(x.stride(0)), ctypes.c_long(y.stride(0))
-        if M <= F32_FEW_ROWS:
+        if M <= F32_FEW_ROWS and K >= F32_FEW_FROM_K:
             _check(lib.ptl_gemm_f32_few(_ptr(y), _ptr(x), _ptr(w), M, N, K, ldx, ldy, _stream()), "gemm_nt")
             return y
         lib.ptl_gemm_f32_workspace.restype = ctypes.c_long
@@ -242,7 +242,8 @@ def gemm_nt(x: torch.Tensor, w: torch.Tensor, out_dtype: Optional[torch.dtype] =
     return y
 
 
-F32_FEW_ROWS = 16          # rows of x up to which the kernel that streams W once takes a float32 product
+F32_FEW_ROWS = 16          # rows of x up to which the kernel that streams W once takes a float32 product,
+F32_FEW_FROM_K = 512       # and the K from which on: shorter sums are made in one order for any number of rows
 
 
 def _gemm_f32_fits(x: torch.Tensor, w: torch.Tensor, M: int, K: int) -> bool:

@@ -104,9 +104,9 @@ def test_gemm_nt(ops, dtype, mnk):
 @pytest.mark.parametrize("mnk", [
     # few rows: one piece of K, a row and a column past a tile, several waves with a short last one, 8-row tiles
     # with one and with two tiles of x, 16-row tiles
-    (1, 8, 4), (8, 9, 68), (7, 2049, 2052), (9, 70, 1028), (16, 2048, 4100), (16, 3073, 516), (12, 5000, 260),
+    (1, 9, 516), (8, 2049, 2052), (9, 70, 1028), (16, 2048, 4100), (16, 3073, 516), (12, 5000, 512),
     # many rows: one and just over one tile, K short of and past a step, cuts along K with a short last one
-    (17, 16, 4), (64, 64, 32), (65, 129, 36), (129, 66, 2052), (33, 515, 8196), (700, 1000, 96), (1030, 2100, 260)])
+    (1, 8, 4), (12, 300, 508), (17, 16, 512), (64, 64, 32), (65, 129, 36), (129, 66, 2052), (33, 515, 8196), (700, 1000, 96), (1030, 2100, 260)])
 def test_gemm_f32_matrix_cores(ops, mnk):
     """The float32 products on the matrix cores, and the vector kernel on the same operands shifted by one
     float (rows that are not aligned), element by element within the bound of a float32 sum of K products
@@ -129,6 +129,39 @@ def test_gemm_f32_matrix_cores(ops, mnk):
     y = ops.gemm_nt(x, w)
     assert torch.isnan(y[:, N - 1]).all() and torch.isfinite(y[:M - 1, :N - 1]).all()
     assert (~torch.isfinite(y[M - 1])).all()
+
+
+@pytest.mark.parametrize("sizes", [(1, 36, 8, 3, 2), (70, 132, 66, 2, 1), (200, 64, 130, 5, 2), (9, 30, 20, 4, 2)],
+                         ids=["one_row", "65_rows_an_expert", "edges", "unaligned"])
+@pytest.mark.parametrize("gated", [True, False])
+def test_moe_f32_matrix_cores(ops, sizes, gated):
+    """The routed experts in float32, within the bound that the sums of both products give: an element of the
+    first is off by (K + 2) 2^-24 sum |x w|, which the activation passes on with its slope, and the second adds
+    (I + 2) 2^-24 of its own sum."""
+    T, K, I, E, top = sizes
+    torch.manual_seed(K)
+    x = torch.randn(T, K, device="cuda")
+    gu = torch.randn(E, (2 if gated else 1) * I, K, device="cuda") / math.sqrt(K)
+    down = torch.randn(E, K, I, device="cuda") / math.sqrt(I)
+    r = ops.moe_route(torch.randn(T, E, device="cuda"), E, top)
+    got = ops.moe_experts(x, r, gu, down, 0 if gated else ops.ACT_RELU2, 0.0, False)
+    u = 2.0 ** -24
+    idx, wgt = r.idx.view(T, top).long(), r.wgt.view(T, top).double()
+    want, bound = torch.zeros(T, K, dtype=torch.float64, device="cuda"), torch.zeros(T, K, dtype=torch.float64, device="cuda")
+    for c in range(top):
+        w1, w2 = gu.double()[idx[:, c]], down.double()[idx[:, c]]
+        p = torch.bmm(w1, x.double()[:, :, None].contiguous())[:, :, 0]
+        e = (K + 2) * u * torch.bmm(w1.abs(), x.double().abs()[:, :, None].contiguous())[:, :, 0]
+        if gated:
+            g, v = p[:, :I], p[:, I:]
+            h = g * torch.sigmoid(g) * v
+            e = 1.1 * e[:, :I] * v.abs() + g.abs() * e[:, I:] + 8 * u * h.abs()
+        else:
+            h = p.clamp(min=0) ** 2
+            e = 2 * p.abs() * e + 4 * u * h
+        want += wgt[:, c:c + 1] * torch.bmm(w2, h[:, :, None].contiguous())[:, :, 0]
+        bound += wgt[:, c:c + 1] * torch.bmm(w2.abs(), (e + (I + 8) * u * h.abs())[:, :, None].contiguous())[:, :, 0]
+    assert ((got.double() - want).abs() <= bound * 1.01).all()
 
 
 @pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float32], ids=["to_bf16", "to_fp32"])
@@ -158,36 +191,6 @@ def test_gemm_skinny(ops, out_dtype, mnk):
         ops.gemm_skinny(torch.zeros(65, K, device="cuda", dtype=torch.bfloat16), w)
     with pytest.raises(ops.KernelError):
         ops.gemm_skinny(x[:, :K - 4], w[:, :K - 4].contiguous())
-
-
-@pytest.mark.parametrize("mnk", [
-    # few rows: one piece of K, a row and a column past a tile, several waves with a short last one, 8-row tiles
-    # with one and with two tiles of x, 16-row tiles
-    (1, 8, 4), (8, 9, 68), (7, 2049, 2052), (9, 70, 1028), (16, 2048, 4100), (16, 3073, 516), (12, 5000, 260),
-    # many rows: one and just over one tile, K short of and past a step, cuts along K with a short last one
-    (17, 16, 4), (64, 64, 32), (65, 129, 36), (129, 66, 2052), (33, 515, 8196), (700, 1000, 96), (1030, 2100, 260)])
-def test_gemm_f32_matrix_cores(ops, mnk):
-    """The float32 products on the matrix cores, and the vector kernel on the same operands shifted by one
-    float (rows that are not aligned), element by element within the bound of a float32 sum of K products
-    in any order: (K + 1) 2^-24 sum |x w|."""
-    M, N, K = mnk
-    torch.manual_seed(9)
-    wide = torch.randn(M, K + 8, device="cuda")
-    w = torch.randn(N, K, device="cuda")
-    for x in (wide[:, 4:4 + K], wide[:, 4:4 + K].contiguous(), wide[:, 3:3 + K]):
-        want = x.double() @ w.double().T
-        bound = (K + 1) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)
-        out = torch.full((M, N + 3), 7.0, device="cuda")
-        y = ops.gemm_nt(x, w, out=out[:, :N])
-        assert ((y.double() - want).abs() <= bound).all()
-        assert (out[:, N:] == 7.0).all()
-    # what is not finite stays in its row of x and its row of w
-    x = wide[:, 4:4 + K].contiguous()
-    x[M - 1, K - 1] = float("inf")
-    w[N - 1, 0] = float("nan")
-    y = ops.gemm_nt(x, w)
-    assert torch.isnan(y[:, N - 1]).all() and torch.isfinite(y[:M - 1, :N - 1]).all()
-    assert (~torch.isfinite(y[M - 1])).all()
 
 
 @pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float32], ids=["to_bf16", "to_fp32"])
