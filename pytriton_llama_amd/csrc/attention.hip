@@ -28,6 +28,7 @@
 // (float32 or bfloat16), any page size, any D up to 640 (beyond 256 with more LDS than a
 // kernel gets unasked: the launcher asks for it).
 #include "attention.h"
+#include "attention_f32.h"
 #include "common.h"
 #include "mfma.h"
 #include <math.h>
@@ -238,6 +239,10 @@ extern "C" int ptl_attention_generic_kv(void* out, long out_stride, int out_f32,
     if (Dk > 256 || Dv > 256) return GO(T, TO, 16, 40);                                           \
     return (Dk <= 128 && Dv <= 128) ? GO(T, TO, 32, 16) : GO(T, TO, 16, 16);                      \
   }
+  if (dtype == PTL_DTYPE_F32 && attn_f32_fits(out, out_stride, q, q_stride, k_cache, v_cache, Dk, Dv))
+    return attention_f32((float*)out, out_stride, (const float*)q, q_stride, (const float*)k_cache,
+                         (const float*)v_cache, q_start, ctx_len, block_table, bt_stride, work_seq, work_qoff, n_work,
+                         Hq, Hkv, maps, Dk, Dv, page_size, ex, scale, stream);
   if (dtype == PTL_DTYPE_F32) GO_SIZES(float, float)
   if (dtype == PTL_DTYPE_BF16) {
     if (out_f32) GO_SIZES(bf16_t, float)

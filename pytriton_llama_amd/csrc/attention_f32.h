@@ -1,0 +1,276 @@
+// Attention of prompt portions over a float32 paged cache on the matrix cores, float32 products and
+// sums throughout (v_mfma_f32_16x16x4_f32). What the vector kernel of attention.hip takes, for key and
+// value sizes that are multiples of 4 up to 128 and 16-byte aligned rows; included by attention.hip.
+//
+// A workgroup takes a block of 16 query rows and HPW query heads that read one key and value head
+// (HPW 2 or 1); its four waves are HPW heads x 4 / HPW parts of the keys. Tiles of BN keys and their
+// values come through LDS, two buffers: the next tile is on its way to registers while this one is
+// used, its page numbers a tile earlier still. A wave computes S^T = K Q^T, 16 keys x 16 queries at a
+// time: lane l (ln = l % 16, lg = l / 16) gets the scores of query ln with keys 4 lg + r, so maxima and
+// sums over keys stay in a lane but for two exchanges between lane groups, and the weights are where
+// O^T += V^T P^T wants them: the instruction's k = lg of step s is key 4 lg + s in both operands. Four
+// steps of a product take a lane's four consecutive floats of a row, read at once: of K and Q along the
+// head dimension; of V a lane reads floats 4 ln .. 4 ln + 3 of a group of 64, element t of them going to
+// the t-th of four result tiles (whose row i is then value column 4 i + t).
+//
+// Bound by the matrix cores: 16 keys x 16 queries cost (Dk + Dv) / 4 instructions of 32 clocks against 8 KB
+// of LDS reads at head size 64. Rows of keys lie 4 floats apart from a multiple of 64 banks, so that the
+// 16 rows of a fragment meet no bank twice; rows of values are read along the row and need no padding.
+//
+// Measured (one MI355X, us a launch; the vector kernel before in brackets): 700 tokens, 32 heads on 8, head
+// size 64: 58 (447); 150 and 333 tokens, 16 heads on one latent head of 128, values of 96: 38 (298).
+#pragma once
+#include "attention.h"
+#include "mfma.h"
+#include "mfma_f32.h"
+
+#define AF_ROWS 16
+
+template <int HPW, int NK, int BN>
+__global__ void __launch_bounds__(256)
+attn_f32_kernel(float* __restrict__ out, long out_stride, const float* __restrict__ q, long q_stride,
+                const float* __restrict__ k_cache, const float* __restrict__ v_cache,
+                const int32_t* __restrict__ q_start, const int32_t* __restrict__ ctx_len,
+                const int32_t* __restrict__ block_table, int bt_stride, const int32_t* __restrict__ work_seq,
+                const int32_t* __restrict__ work_qoff, int Hq, int Hkv, int maps, int Dk, int Dv, int page_size,
+                AttnExtras ex, float scale) {
+  constexpr int KS = 4 / HPW;                    // parts of the keys
+  constexpr int NG = BN / 16 / KS;               // groups of 16 keys of a tile that a wave takes
+  constexpr int D = 16 * NK, KLD = D + 4;        // padded sizes; floats between rows of keys in LDS
+  constexpr int PIECES = D / 4, PER_PASS = 256 / PIECES, P = BN / PER_PASS;
+  static_assert(NG >= 1 && P >= 1, "a tile has 16 keys a part and a row a thread");
+  extern __shared__ float lds[];
+  float* Ks = lds;                               // [2][BN][KLD]
+  float* Vs = lds + 2 * BN * KLD;                // [2][BN][D]
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, ln = lane & 15, lg = lane >> 4;
+  const int head = blockIdx.y * HPW + wave % HPW, part = wave / HPW;
+  const int seq = work_seq[blockIdx.x], qoff = work_qoff[blockIdx.x];
+  const int qs = q_start[seq], qlen = q_start[seq + 1] - qs, ctx = ctx_len[seq];
+  const int rows = min(AF_ROWS, qlen - qoff);
+  if (rows <= 0) return;
+  const int vh = (head / maps) / ((Hq / maps) / Hkv), kh = vh * maps + head % maps, Hk = Hkv * maps;
+  const int32_t* bt = block_table + (size_t)seq * bt_stride;
+  const int first_q = ctx - qlen + qoff, qpos = first_q + ln;
+  const int k_end = min(ctx, first_q + rows), k_lo = first_seen(ex, first_q), row_lo = first_seen(ex, qpos);
+  // the walk: the kept first keys left of the window, then the keys from the window's start on
+  const int n_kept = min(max(ex.keep_first, 0), k_lo), shift = k_lo - n_kept, n_walk = n_kept + (k_end - k_lo);
+  const bool row_valid = ln < rows;
+
+  F4 qf[NK];
+#pragma unroll
+  for (int c = 0; c < NK; ++c)
+    qf[c].u = row_valid && 16 * c + 4 * lg < Dk
+                  ? load16(q + (size_t)(qs + qoff + ln) * q_stride + (size_t)head * Dk + 16 * c + 4 * lg) : zero16();
+
+  const int piece = tid % PIECES, row0 = tid / PIECES;
+  int page[P], slot[P];
+  uint4 kr[P], vr[P];
+  auto pages = [&](int k0) {                     // where the rows of the tile from k0 on lie (page -1: nowhere)
+#pragma unroll
+    for (int i = 0; i < P; ++i) {
+      const int kw = k0 + row0 + i * PER_PASS, kp = kw < n_kept ? kw : kw + shift;
+      page[i] = kw < n_walk ? bt[kp / page_size] : -1;
+      slot[i] = kp % page_size;
+    }
+  };
+  auto fetch = [&]() {
+#pragma unroll
+    for (int i = 0; i < P; ++i) {
+      const bool ok = page[i] >= 0;
+      kr[i] = ok && 4 * piece < Dk
+                  ? load16(k_cache + (((size_t)page[i] * Hk + kh) * page_size + slot[i]) * Dk + 4 * piece) : zero16();
+      vr[i] = ok && 4 * piece < Dv
+                  ? load16(v_cache + (((size_t)page[i] * Hkv + vh) * page_size + slot[i]) * Dv + 4 * piece) : zero16();
+    }
+  };
+  auto put = [&](int b) {
+#pragma unroll
+    for (int i = 0; i < P; ++i) {
+      const int r = b * BN + row0 + i * PER_PASS;
+      *reinterpret_cast<uint4*>(Ks + r * KLD + 4 * piece) = kr[i];
+      *reinterpret_cast<uint4*>(Vs + r * D + 4 * piece) = vr[i];
+    }
+  };
+  f32x4_t acc[NK];
+#pragma unroll
+  for (int t = 0; t < NK; ++t) acc[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  float m_run = -INFINITY, l_run = 0.f;          // l_run: of this lane's keys only
+
+  if (n_walk > 0) {
+    pages(0);
+    fetch();
+    pages(BN);
+    put(0);
+  }
+  __syncthreads();
+  int buf = 0;
+  for (int k0 = 0; k0 < n_walk; k0 += BN, buf ^= 1) {
+    const bool more = k0 + BN < n_walk;
+    if (more) {
+      fetch();
+      pages(k0 + 2 * BN);
+    }
+    f32x4_t s[NG];
+    float tmax = -INFINITY;
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+      const int base = 16 * (g * KS + part);
+      const float* krow = Ks + (buf * BN + base + ln) * KLD + 4 * lg;
+      s[g] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int c = 0; c < NK; ++c) {
+        F4 kf;
+        kf.u = load16(krow + 16 * c);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          s[g] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf.f[i], qf[c].f[i], s[g], 0, 0, 0);
+      }
+    }
+#pragma unroll
+    for (int g = 0; g < NG; ++g)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int kw = k0 + 16 * (g * KS + part) + 4 * lg + r, kp = kw < n_kept ? kw : kw + shift;
+        const bool vis = row_valid && kw < n_walk && kp <= qpos && (kp >= row_lo || kp < ex.keep_first);
+        s[g][r] = vis ? cap_score(ex, s[g][r] * scale) : -INFINITY;
+        tmax = fmaxf(tmax, s[g][r]);
+      }
+    tmax = max_with_lane_xor32(max_with_lane_xor16(tmax));
+    const float m_new = fmaxf(m_run, tmax);
+    const float m_safe = m_new == -INFINITY ? 0.f : m_new;
+    const float alpha = expf(m_run - m_safe);
+    float psum = 0.f;
+#pragma unroll
+    for (int g = 0; g < NG; ++g)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        s[g][r] = expf(s[g][r] - m_safe);
+        psum += s[g][r];
+      }
+    l_run = l_run * alpha + psum;
+    m_run = m_new;
+#pragma unroll
+    for (int t = 0; t < NK; ++t) acc[t] *= alpha;
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+      const float* vrow = Vs + (buf * BN + 16 * (g * KS + part) + 4 * lg) * D;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        if (NK >= 4) {
+#pragma unroll
+          for (int v = 0; v < NK / 4; ++v) {
+            F4 vf;
+            vf.u = load16(vrow + r * D + 64 * v + 4 * ln);
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+              acc[4 * v + t] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf.f[t], s[g][r], acc[4 * v + t], 0, 0, 0);
+          }
+        } else {
+          const float2 vf = *reinterpret_cast<const float2*>(vrow + r * D + 2 * ln);
+          acc[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf.x, s[g][r], acc[0], 0, 0, 0);
+          acc[NK > 1 ? 1 : 0] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf.y, s[g][r], acc[NK > 1 ? 1 : 0], 0, 0, 0);
+        }
+      }
+    }
+    if (more) put(buf ^ 1);
+    __syncthreads();
+  }
+  l_run += __shfl_xor(l_run, 16, 64);
+  l_run += __shfl_xor(l_run, 32, 64);
+
+  {                                              // the parts of the keys meet in the first wave of a head
+    float* mine = lds + (size_t)wave * (NK * 256 + 128);
+    if (part > 0) {
+#pragma unroll
+      for (int t = 0; t < NK; ++t) *reinterpret_cast<f32x4_t*>(mine + (t * 64 + lane) * 4) = acc[t];
+      mine[NK * 256 + lane] = m_run;
+      mine[NK * 256 + 64 + lane] = l_run;
+    }
+    __syncthreads();
+    if (part > 0) return;
+#pragma unroll
+    for (int p = 1; p < KS; ++p) {
+      const float* other = lds + (size_t)(wave + p * HPW) * (NK * 256 + 128);
+      const float m_o = other[NK * 256 + lane], l_o = other[NK * 256 + 64 + lane];
+      const float m_new = fmaxf(m_run, m_o), m_safe = m_new == -INFINITY ? 0.f : m_new;
+      const float a = expf(m_run - m_safe), b = expf(m_o - m_safe);
+      l_run = l_run * a + l_o * b;
+      m_run = m_new;
+#pragma unroll
+      for (int t = 0; t < NK; ++t)
+        acc[t] = acc[t] * a + *reinterpret_cast<const f32x4_t*>(other + (t * 64 + lane) * 4) * b;
+    }
+  }
+  if (!row_valid) return;
+  float den = l_run, f = 1.f;
+  if (ex.sink) {                                 // one more term of the denominator: exp(sink)
+    const float sk = ex.sink[head], mx = fmaxf(m_run, sk);
+    f = expf(m_run - mx);
+    den = l_run * f + expf(sk - mx);
+  }
+  const float inv = den > 0.f ? f / den * head_gate(ex, qs + qoff + ln, head) : 0.f;
+  float* o = out + (size_t)(qs + qoff + ln) * out_stride + (size_t)head * Dv;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    if (NK >= 4) {
+#pragma unroll
+      for (int v = 0; v < NK / 4; ++v) {
+        const int d = 64 * v + 16 * lg + 4 * r;
+        if (d < Dv)
+          *reinterpret_cast<float4*>(o + d) = make_float4(acc[4 * v][r] * inv, acc[4 * v + 1][r] * inv,
+                                                          acc[4 * v + 2][r] * inv, acc[4 * v + 3][r] * inv);
+      }
+    } else {
+      const int d = 8 * lg + 2 * r;
+      if (d < Dv) *reinterpret_cast<float2*>(o + d) = make_float2(acc[0][r] * inv, acc[NK > 1 ? 1 : 0][r] * inv);
+    }
+  }
+}
+
+template <int HPW, int NK, int BN, typename... Args>
+static int launch_attn_f32(int n_work, int Hq, hipStream_t st, Args... args) {
+  constexpr int D = 16 * NK;
+  const size_t tiles = (size_t)2 * BN * (2 * D + 4) * sizeof(float);
+  const size_t merge = (size_t)4 * (NK * 256 + 128) * sizeof(float);
+  const size_t bytes = tiles > merge ? tiles : merge;
+  if (bytes > 64 * 1024 &&
+      hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_f32_kernel<HPW, NK, BN>),
+                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) != hipSuccess) {
+    (void)hipGetLastError();
+    return PTL_ERR_ARG;
+  }
+  attn_f32_kernel<HPW, NK, BN><<<dim3(n_work, Hq / HPW), 256, bytes, st>>>(args...);
+  return ptl_launch_status();
+}
+
+static bool attn_f32_fits(const void* out, long out_stride, const void* q, long q_stride, const void* k, const void* v,
+                          int Dk, int Dv) {
+  return Dk % 4 == 0 && Dv % 4 == 0 && Dk <= 128 && Dv <= 128 && out_stride % 4 == 0 && q_stride % 4 == 0 &&
+         (((uintptr_t)out | (uintptr_t)q | (uintptr_t)k | (uintptr_t)v) & 15) == 0;
+}
+
+// (arguments as ptl_attention_generic_kv, of attn_f32_fits)
+static int attention_f32(float* out, long out_stride, const float* q, long q_stride, const float* k_cache,
+                         const float* v_cache, const int32_t* q_start, const int32_t* ctx_len,
+                         const int32_t* block_table, int bt_stride, const int32_t* work_seq, const int32_t* work_qoff,
+                         int n_work, int Hq, int Hkv, int maps, int Dk, int Dv, int page_size, const AttnExtras& ex,
+                         float scale, hipStream_t st) {
+  // two heads that share a key head share its tiles; the other waves share the keys. (By the heads alone:
+  // how a row's keys are cut, and with it the order of its sums, does not depend on what else is in the step.)
+  const int hpw = maps == 1 && Hq / Hkv % 2 == 0 ? 2 : 1;
+  const int size = Dk > Dv ? Dk : Dv;
+#define GO(HPW, NK, BN)                                                                                            \
+  return launch_attn_f32<HPW, NK, BN>(n_work, Hq, st, out, out_stride, q, q_stride, k_cache, v_cache, q_start, ctx_len, \
+                                      block_table, bt_stride, work_seq, work_qoff, Hq, Hkv, maps, Dk, Dv, page_size, ex, \
+                                      scale)
+#define GO_HEADS(NK)             \
+  {                              \
+    if (hpw == 2) GO(2, NK, 32); \
+    GO(1, NK, 64);               \
+  }
+  if (size <= 32) GO_HEADS(2)
+  if (size <= 64) GO_HEADS(4)
+  GO_HEADS(8)
+#undef GO_HEADS
+#undef GO
+}

@@ -752,6 +752,21 @@ def test_attention_generic(ops, dtype, case):
     _attention_case(ops, dtype, **case)
 
 
+@pytest.mark.parametrize("case", [
+    # one and two heads a workgroup, tiles of 32, 64 and 128 columns with and without columns beyond the head,
+    # blocks of one row, keys one past and short of a tile
+    dict(seq_lens=[65, 33, 1], q_lens=[65, 1, 1], Hq=3, Hkv=1, D=64, P=16),
+    dict(seq_lens=[130, 31], q_lens=[17, 31], Hq=4, Hkv=4, D=20, P=3),
+    dict(seq_lens=[97, 64], q_lens=[97, 64], Hq=6, Hkv=3, D=128, P=16),
+    dict(seq_lens=[700, 333], q_lens=[650, 333], Hq=16, Hkv=2, D=64, P=16, window=100),
+    dict(seq_lens=[1200], q_lens=[1100], Hq=32, Hkv=8, D=32, P=8),
+    dict(seq_lens=[1100], q_lens=[1100], Hq=32, Hkv=8, D=100, P=16),
+    dict(seq_lens=[700], q_lens=[500], Hq=64, Hkv=32, D=64, P=16),
+])
+def test_attention_f32_matrix_cores(ops, case):
+    _attention_case(ops, torch.float32, **case)
+
+
 @pytest.mark.parametrize("dtype", DT, ids=IDS)
 @pytest.mark.parametrize("splits", [1, 3, 8])
 @pytest.mark.parametrize("case", [
