@@ -523,21 +523,27 @@ extern "C" int ptl_sample_top_p(int32_t* out, float* work, int want_probs, const
 // the kernel above passes over the row seven times. Here a row is cut into chunks of 4096
 // logits, a workgroup a chunk, and the passes become kernels:
 //   (1) minmax:  every chunk's largest and smallest finite logit;
-//   (2) exp:     e = exp(x/T - max) into the work buffer, the chunk's sum, and the chunk's
-//                histogram of mass over 2048 buckets of x, equally wide, from the row's max
-//                down to its min (at most 32 T below the max; what lies further goes to the
-//                last bucket). The histogram is summed in LDS in fixed point (2^-40) with
-//                integer atomics, so that it does not depend on the order of the threads;
-//   (3) combine: the chunks' histograms added in chunk order;
-//   (4) gather:  every workgroup finds the bucket in which the mass, most likely tokens first,
-//                passes top_p (same code, same numbers: same answer), adds up what its chunk
-//                has above that bucket and hands on its tokens inside it (at most 256);
+//   (2) hist:    the chunk's sum of e = exp(x/T - max) and its histogram of that mass over 2048
+//                buckets of x, equally wide, from the row's max down to its min (at most 32 T
+//                below the max; what lies further goes to the last bucket). The histogram is
+//                summed in LDS in fixed point (2^-40) with integer atomics, so that it does not
+//                depend on the order of the threads; the last bucket, where most of a
+//                vocabulary lies, in a register of every thread first (all of a wave's lanes
+//                adding to one address: 40 instead of 17 us for 64 rows of 128,256);
+//   (3) combine: one workgroup a row adds the chunks' histograms in chunk order and finds the
+//                bucket in which the mass, most likely tokens first, passes top_p;
+//   (4) gather:  every workgroup adds up what its chunk has above that bucket and hands on its
+//                tokens inside it (at most 256);
 //   (5) draw:    one workgroup a row bisects over the bit patterns of x among the tokens handed
 //                on (a few hundred) for the exact edge of the nucleus, adds the kept mass chunk
 //                by chunk, finds the chunk that holds u * kept and walks it;
 //   (6) probs:   only if asked for, the renormalised nucleus distribution.
 // A token is kept iff it lies in a bucket above the crossing one, or in it and above the edge;
-// equal logits are kept or dropped together. If a chunk has more than 256 tokens in the crossing
+// equal logits are kept or dropped together. e is worked out again from x wherever it is wanted
+// (one multiplication, one exp2, the same bits): keeping it would be a write and a read of the
+// whole row. 64 rows of 128,256 logits (one MI355X): 66 us for the five kernels, 12 to 17 for each of the
+// three passes over the logits; 97 us with e kept, the crossing found by every workgroup of the gather
+// kernel and the last bucket in LDS. If a chunk has more than 256 tokens in the crossing
 // bucket, or the row more than 4096 (many equal logits), the draw kernel bisects over the whole
 // row instead: slower, same result. Everything is added in a fixed order: the same logits,
 // parameters and u give the same token.
@@ -553,11 +559,11 @@ extern "C" int ptl_sample_top_p(int32_t* out, float* work, int want_probs, const
 
 // where a row's pieces lie in the workspace (all 4-byte words)
 struct SwRow {
-  float *cmax, *cmin, *csum, *ckept, *hist, *tot, *seg_x, *result;
+  float *cmax, *cmin, *csum, *ckept, *hist, *seg_x, *result;
   int32_t *ccount, *seg_i;
 };
 __host__ __device__ static inline size_t sw_row_words(int S) {
-  return (size_t)5 * S + (size_t)S * SW_BUCKETS + SW_BUCKETS + (size_t)2 * S * SW_SEG + 8;
+  return (size_t)5 * S + (size_t)S * SW_BUCKETS + (size_t)2 * S * SW_SEG + 8;
 }
 __device__ __forceinline__ SwRow sw_row(float* ws, int r, int S) {
   float* p = ws + (size_t)r * sw_row_words(S);
@@ -568,7 +574,6 @@ __device__ __forceinline__ SwRow sw_row(float* ws, int r, int S) {
   w.ckept = p; p += S;
   w.ccount = reinterpret_cast<int32_t*>(p); p += S;
   w.hist = p; p += (size_t)S * SW_BUCKETS;
-  w.tot = p; p += SW_BUCKETS;
   w.seg_x = p; p += (size_t)S * SW_SEG;
   w.seg_i = reinterpret_cast<int32_t*>(p); p += (size_t)S * SW_SEG;
   w.result = p;        // [0] edge key (bits), [1] crossing bucket (bits), [2] kept mass, [3] mass before
@@ -603,6 +608,9 @@ __device__ __forceinline__ SwScale sw_scale(const SwRow& w, int S, float T, bool
   s.inv_w = span > 0.f ? (float)SW_BUCKETS / span : 0.f;
   return s;
 }
+__device__ __forceinline__ float sw_exp(float x, const SwScale& s) {
+  return __builtin_amdgcn_exp2f(fmaf(x, s.c, -s.mc));
+}
 __device__ __forceinline__ int sw_bucket(float x, const SwScale& s) {
   const float fb = (s.mx - x) * s.inv_w;                 // (NaN when -inf meets inv_w 0: bucket 0)
   return (int)fminf(fmaxf(fb, 0.f), (float)(SW_BUCKETS - 1));
@@ -633,14 +641,13 @@ sw_minmax_kernel(float* __restrict__ ws, const float* __restrict__ logits, int V
 }
 
 __global__ void __launch_bounds__(SW_THREADS)
-sw_exp_hist_kernel(float* __restrict__ ws, float* __restrict__ work, const float* __restrict__ logits,
-                   int V, long stride, int S, const float* __restrict__ temperature) {
+sw_hist_kernel(float* __restrict__ ws, const float* __restrict__ logits, int V, long stride, int S,
+               const float* __restrict__ temperature) {
   __shared__ unsigned long long hist[SW_BUCKETS];
   __shared__ float scratch[16];
   const int r = blockIdx.y, c = blockIdx.x;
   const SwRow w = sw_row(ws, r, S);
   const float* row = logits + (size_t)r * stride;
-  float* ex = work + (size_t)r * V;
   const SwScale s = sw_scale(w, S, temperature[r], false);
   for (int b = threadIdx.x; b < SW_BUCKETS; b += SW_THREADS) hist[b] = 0ull;
   __syncthreads();
@@ -652,42 +659,33 @@ sw_exp_hist_kernel(float* __restrict__ ws, float* __restrict__ work, const float
     x[j] = i < V ? sw_clean(row[i]) : -INFINITY;
   }
   float z = 0.f;
+  unsigned long long last = 0ull;
 #pragma unroll
   for (int j = 0; j < SW_PER; ++j) {
     const int i = lo + j * SW_THREADS + threadIdx.x;
     if (i < V) {
-      const float e = __builtin_amdgcn_exp2f(fmaf(x[j], s.c, -s.mc));
-      ex[i] = e;
+      const float e = sw_exp(x[j], s);
       z += e;
-      atomicAdd(&hist[sw_bucket(x[j], s)], (unsigned long long)(e * SW_FIXED + 0.5f));
+      const unsigned long long fixed = (unsigned long long)(e * SW_FIXED + 0.5f);
+      const int b = sw_bucket(x[j], s);
+      if (b == SW_BUCKETS - 1) last += fixed;
+      else atomicAdd(&hist[b], fixed);
     }
   }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) last += __shfl_xor(last, o, 64);
+  if ((threadIdx.x & 63) == 0) atomicAdd(&hist[SW_BUCKETS - 1], last);
   z = block_sum(z, scratch);               // (its barriers also complete the histogram)
   if (threadIdx.x == 0) w.csum[c] = z;
   float* out = w.hist + (size_t)c * SW_BUCKETS;
   for (int b = threadIdx.x; b < SW_BUCKETS; b += SW_THREADS) out[b] = (float)hist[b] * (1.0f / SW_FIXED);
 }
 
-__global__ void __launch_bounds__(SW_THREADS)
-sw_combine_kernel(float* __restrict__ ws, int S) {
-  const SwRow w = sw_row(ws, blockIdx.y, S);
-  const int b = blockIdx.x * SW_THREADS + threadIdx.x;
-  float t = 0.f;
-  for (int c0 = 0; c0 < S; c0 += 8) {      // eight loads under way, added in chunk order
-    float v[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) v[j] = c0 + j < S ? w.hist[(size_t)(c0 + j) * SW_BUCKETS + b] : 0.f;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) t += v[j];
-  }
-  w.tot[b] = t;
-}
-
 // The bucket in which the mass, most likely tokens first, passes tp, and the mass before it;
 // SW_BUCKETS if it never does (everything is kept). The first SW_THREADS threads work, every
 // thread of the block must call (barriers). tmp: 8 floats and 2 ints of LDS.
-__device__ __forceinline__ void sw_crossing(const float* __restrict__ tot, float tp, float* tmp,
-                                            int* itmp, int* cross, float* before) {
+__device__ __forceinline__ void sw_crossing(const float* tot, float tp, float* tmp, int* itmp, int* cross,
+                                            float* before) {
   constexpr int PER = SW_BUCKETS / SW_THREADS;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const bool works = tid < SW_THREADS;
@@ -732,27 +730,77 @@ __device__ __forceinline__ void sw_crossing(const float* __restrict__ tot, float
   *before = cb < SW_BUCKETS ? tmp[4] : 0.f;
 }
 
-__global__ void __launch_bounds__(SW_THREADS)
-sw_gather_kernel(float* __restrict__ ws, const float* __restrict__ work, const float* __restrict__ logits,
-                 int V, long stride, int S, const float* __restrict__ temperature,
-                 const float* __restrict__ top_p) {
+// One workgroup a row; a thread adds two buckets, eight chunks' loads under way, in chunk order.
+#define SW_COMBINE_THREADS (SW_BUCKETS / 2)
+__global__ void __launch_bounds__(SW_COMBINE_THREADS)
+sw_combine_kernel(float* __restrict__ ws, int S, const float* __restrict__ temperature,
+                  const float* __restrict__ top_p) {
+  __shared__ float tot[SW_BUCKETS];
   __shared__ float tmp[17];
   __shared__ int itmp[2];
-  const int r = blockIdx.y, c = blockIdx.x;
+  const int r = blockIdx.x;
   const SwRow w = sw_row(ws, r, S);
-  const float* row = logits + (size_t)r * stride;
-  const float* ex = work + (size_t)r * V;
   const SwScale s = sw_scale(w, S, temperature[r], true);
   int cross = SW_BUCKETS;
   float before = 0.f;
-  if (top_p[r] < 1.0f) sw_crossing(w.tot, top_p[r] * s.z, tmp, itmp, &cross, &before);
+  if (top_p[r] < 1.0f) {
+    float2 t = make_float2(0.f, 0.f);
+    const float* mine = w.hist + 2 * threadIdx.x;
+    for (int c0 = 0; c0 < S; c0 += 8) {
+      float2 v[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        // (rows of the workspace begin at any multiple of four bytes)
+        const float* p = mine + (size_t)(c0 + j) * SW_BUCKETS;
+        v[j] = c0 + j < S ? make_float2(p[0], p[1]) : make_float2(0.f, 0.f);
+      }
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        t.x += v[j].x;
+        t.y += v[j].y;
+      }
+    }
+    tot[2 * threadIdx.x] = t.x;
+    tot[2 * threadIdx.x + 1] = t.y;
+    __syncthreads();
+    sw_crossing(tot, top_p[r] * s.z, tmp, itmp, &cross, &before);
+  }
+  if (threadIdx.x == 0) {
+    w.result[1] = __int_as_float(cross);
+    w.result[3] = before;
+    w.result[4] = s.mx;
+    w.result[5] = s.inv_w;
+    w.result[6] = s.z;
+  }
+}
+
+// What the combine kernel found for a row.
+__device__ __forceinline__ SwScale sw_found(const SwRow& w, float T, int* cross) {
+  *cross = __float_as_int(w.result[1]);
+  SwScale s;
+  s.mx = w.result[4];
+  s.inv_w = w.result[5];
+  s.z = w.result[6];
+  s.c = 1.4426950408889634f / T;
+  s.mc = s.mx * s.c;
+  return s;
+}
+
+__global__ void __launch_bounds__(SW_THREADS)
+sw_gather_kernel(float* __restrict__ ws, const float* __restrict__ logits, int V, long stride, int S,
+                 const float* __restrict__ temperature) {
+  __shared__ float tmp[17];
+  const int r = blockIdx.y, c = blockIdx.x;
+  const SwRow w = sw_row(ws, r, S);
+  const float* row = logits + (size_t)r * stride;
+  int cross;
+  const SwScale s = sw_found(w, temperature[r], &cross);
   const int lo = c * SW_CHUNK;
-  float x[SW_PER], e[SW_PER];
+  float x[SW_PER];
 #pragma unroll
   for (int j = 0; j < SW_PER; ++j) {
     const int i = lo + j * SW_THREADS + threadIdx.x;
     x[j] = i < V ? sw_clean(row[i]) : -INFINITY;
-    e[j] = i < V ? ex[i] : 0.f;
   }
   float sure = 0.f;
   int mine = 0;
@@ -762,7 +810,7 @@ sw_gather_kernel(float* __restrict__ ws, const float* __restrict__ work, const f
     const int i = lo + j * SW_THREADS + threadIdx.x;
     const int b = sw_bucket(x[j], s);
     in[j] = i < V && b == cross;
-    if (i < V && b < cross) sure += e[j];
+    if (i < V && b < cross) sure += sw_exp(x[j], s);
     mine += in[j] ? 1 : 0;
   }
   float total;
@@ -771,13 +819,6 @@ sw_gather_kernel(float* __restrict__ ws, const float* __restrict__ work, const f
   if (threadIdx.x == 0) {
     w.ckept[c] = sure;
     w.ccount[c] = (int)total;
-    if (c == 0) {                          // what every workgroup of the row found, for the draw
-      w.result[1] = __int_as_float(cross);
-      w.result[3] = before;
-      w.result[4] = s.mx;
-      w.result[5] = s.inv_w;
-      w.result[6] = s.z;
-    }
   }
   int at = at0;
 #pragma unroll
@@ -804,8 +845,8 @@ __device__ __forceinline__ float wave_inclusive_scan(float v) {
 }
 
 __global__ void __launch_bounds__(SW_THREADS)
-sw_draw_kernel(int32_t* __restrict__ out, float* __restrict__ ws, const float* __restrict__ work,
-               const float* __restrict__ logits, int V, long stride, int S,
+sw_draw_kernel(int32_t* __restrict__ out, float* __restrict__ ws, const float* __restrict__ logits, int V,
+               long stride, int S,
                const float* __restrict__ temperature, const float* __restrict__ top_p,
                const float* __restrict__ uniform) {
   __shared__ float tmp[17];
@@ -818,16 +859,9 @@ sw_draw_kernel(int32_t* __restrict__ out, float* __restrict__ ws, const float* _
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = blockIdx.x;
   const SwRow w = sw_row(ws, r, S);
   const float* row = logits + (size_t)r * stride;
-  const float* ex = work + (size_t)r * V;
-  // what the gather kernel's workgroups agreed on
-  const int cross = __float_as_int(w.result[1]);
+  int cross;
+  const SwScale s = sw_found(w, temperature[r], &cross);
   const float before = w.result[3];
-  SwScale s;
-  s.mx = w.result[4];
-  s.inv_w = w.result[5];
-  s.z = w.result[6];
-  s.c = 1.4426950408889634f / temperature[r];
-  s.mc = s.mx * s.c;
   const float tp = top_p[r] * s.z;
   const int my_count = lane < S ? w.ccount[lane] : 0;
   const float my_sure = lane < S ? w.ckept[lane] : 0.f;
@@ -850,9 +884,9 @@ sw_draw_kernel(int32_t* __restrict__ out, float* __restrict__ ws, const float* _
       for (int c = tid >> 3; c < S; c += SW_THREADS / 8) {            // eight threads a chunk
         const int base = seg_at[c], k = seg_at[c + 1] - base;
         for (int j = tid & 7; j < k; j += 8) {
-          const int i = w.seg_i[(size_t)c * SW_SEG + j];
-          list_x[base + j] = w.seg_x[(size_t)c * SW_SEG + j];
-          list_e[base + j] = ex[i];
+          const float x = w.seg_x[(size_t)c * SW_SEG + j];
+          list_x[base + j] = x;
+          list_e[base + j] = sw_exp(x, s);
         }
       }
       __syncthreads();
@@ -922,7 +956,7 @@ sw_draw_kernel(int32_t* __restrict__ out, float* __restrict__ ws, const float* _
         float mass = 0.f;
         for (int i = tid; i < V; i += SW_THREADS) {
           const float x = sw_clean(row[i]);
-          if (sw_bucket(x, s) == cross && sw_key(x) > mid) mass += ex[i];
+          if (sw_bucket(x, s) == cross && sw_key(x) > mid) mass += sw_exp(x, s);
         }
         mass = block_sum(mass, tmp) + before;
         if (mass <= tp) hi = mid; else lo = mid;
@@ -941,7 +975,7 @@ sw_draw_kernel(int32_t* __restrict__ out, float* __restrict__ ws, const float* _
       float part = 0.f;
       for (int i = c * SW_CHUNK + tid; i < min(V, (c + 1) * SW_CHUNK); i += SW_THREADS) {
         const float x = sw_clean(row[i]);
-        if (sw_bucket(x, s) == cross && sw_key(x) > edge) part += ex[i];
+        if (sw_bucket(x, s) == cross && sw_key(x) > edge) part += sw_exp(x, s);
       }
       part = block_sum(part, tmp);
       if (lane == c) extra = part;
@@ -981,7 +1015,7 @@ sw_draw_kernel(int32_t* __restrict__ out, float* __restrict__ ws, const float* _
   for (int k = 0; k < SW_PER; ++k) {
     const int i = c0 + SW_PER * tid + k;
     xv[k] = i < V ? sw_clean(row[i]) : -INFINITY;
-    v[k] = i < V ? ex[i] : 0.f;
+    v[k] = i < V ? sw_exp(xv[k], s) : 0.f;
   }
 #pragma unroll
   for (int k = 0; k < SW_PER; ++k) {
@@ -1018,16 +1052,16 @@ sw_probs_kernel(float* __restrict__ ws, float* __restrict__ work, const float* _
   const SwRow w = sw_row(ws, r, S);
   const float* row = logits + (size_t)r * stride;
   float* ex = work + (size_t)r * V;
-  SwScale s;
-  s.mx = w.result[4];
-  s.inv_w = w.result[5];
+  int cross;
+  const SwScale s = sw_found(w, temperature[r], &cross);
   const uint32_t edge = __float_as_uint(w.result[0]);
-  const int cross = __float_as_int(w.result[1]);
   const float inv_kept = 1.0f / w.result[2];
 #pragma unroll
   for (int j = 0; j < SW_PER; ++j) {
     const int i = c * SW_CHUNK + j * SW_THREADS + threadIdx.x;
-    if (i < V) ex[i] = sw_kept(sw_clean(row[i]), s, cross, edge) ? ex[i] * inv_kept : 0.f;
+    if (i >= V) continue;
+    const float x = sw_clean(row[i]);
+    ex[i] = sw_kept(x, s, cross, edge) ? sw_exp(x, s) * inv_kept : 0.f;
   }
 }
 
@@ -1037,7 +1071,8 @@ extern "C" size_t ptl_sample_top_p_wide_workspace(int R, int V) {
   return (size_t)R * sw_row_words(S) * sizeof(float);
 }
 
-// As ptl_sample_top_p; ws: ptl_sample_top_p_wide_workspace(R, V) bytes, 16-byte aligned.
+// As ptl_sample_top_p (work: only for the probabilities, if wanted); ws:
+// ptl_sample_top_p_wide_workspace(R, V) bytes, 16-byte aligned.
 // Rows of up to 64 chunks (262,144 logits).
 extern "C" int ptl_sample_top_p_wide(int32_t* out, float* work, int want_probs, const float* logits,
                                      int R, int V, long stride, const float* temperature,
@@ -1045,13 +1080,13 @@ extern "C" int ptl_sample_top_p_wide(int32_t* out, float* work, int want_probs, 
                                      hipStream_t stream) {
   if (R <= 0) return PTL_OK;
   const int S = (V + SW_CHUNK - 1) / SW_CHUNK;
-  if (V <= 0 || stride < V || !work || !ws || S > 64 || R > 65535) return PTL_ERR_ARG;
+  if (V <= 0 || stride < V || (want_probs && !work) || !ws || S > 64 || R > 65535) return PTL_ERR_ARG;
   const dim3 chunks(S, R);
   sw_minmax_kernel<<<chunks, SW_THREADS, 0, stream>>>(ws, logits, V, stride, S);
-  sw_exp_hist_kernel<<<chunks, SW_THREADS, 0, stream>>>(ws, work, logits, V, stride, S, temperature);
-  sw_combine_kernel<<<dim3(SW_BUCKETS / SW_THREADS, R), SW_THREADS, 0, stream>>>(ws, S);
-  sw_gather_kernel<<<chunks, SW_THREADS, 0, stream>>>(ws, work, logits, V, stride, S, temperature, top_p);
-  sw_draw_kernel<<<R, SW_THREADS, 0, stream>>>(out, ws, work, logits, V, stride, S, temperature, top_p, uniform);
+  sw_hist_kernel<<<chunks, SW_THREADS, 0, stream>>>(ws, logits, V, stride, S, temperature);
+  sw_combine_kernel<<<R, SW_COMBINE_THREADS, 0, stream>>>(ws, S, temperature, top_p);
+  sw_gather_kernel<<<chunks, SW_THREADS, 0, stream>>>(ws, logits, V, stride, S, temperature);
+  sw_draw_kernel<<<R, SW_THREADS, 0, stream>>>(out, ws, logits, V, stride, S, temperature, top_p, uniform);
   if (want_probs)
     sw_probs_kernel<<<chunks, SW_THREADS, 0, stream>>>(ws, work, logits, V, stride, S, temperature);
   return ptl_launch_status();
@@ -1059,28 +1094,59 @@ extern "C" int ptl_sample_top_p_wide(int32_t* out, float* work, int want_probs, 
 
 // ptl_token_logprob: out[r] = log_softmax(logits[r])[tokens[r]], the log-probability the
 // reference reports for a generated token (F.log_softmax of the step's logits gathered at
-// the token, lite_llama/generete_with_probs.py:154-165). One workgroup a row.
-__global__ void __launch_bounds__(1024)
-token_logprob_kernel(float* __restrict__ out, const float* __restrict__ logits,
-                     const int32_t* __restrict__ tokens, int V, long stride) {
+// the token, lite_llama/generete_with_probs.py:154-165). A workgroup a chunk of a row finds the
+// chunk's max and its sum of exp(x - max); a wave a row puts the chunks together. (One workgroup a row
+// reads a row of 128k logits at a small part of what the chip delivers: 64 rows 78 us,
+// now 12; one MI355X.)
+#define LP_CHUNK 4096
+#define LP_THREADS 256
+__global__ void __launch_bounds__(LP_THREADS)
+token_logprob_part_kernel(float2* __restrict__ parts, int chunks, const float* __restrict__ logits, int V, long stride) {
+  constexpr int PER = LP_CHUNK / LP_THREADS;
   __shared__ float scratch[16];
   const float* row = logits + (size_t)blockIdx.x * stride;
-  float mx = -INFINITY;
-  for (int i = threadIdx.x; i < V; i += blockDim.x) mx = fmaxf(mx, row[i]);
-  mx = block_max(mx, scratch);
-  float z = 0.f;
-  for (int i = threadIdx.x; i < V; i += blockDim.x) z += expf(row[i] - mx);
-  z = block_sum(z, scratch);
-  if (threadIdx.x == 0) {
-    const int t = tokens[blockIdx.x];
-    out[blockIdx.x] = (t >= 0 && t < V) ? row[t] - mx - logf(z) : -INFINITY;
+  for (int c = blockIdx.y; c < chunks; c += gridDim.y) {
+    float x[PER], mx = -INFINITY;
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+      const int i = c * LP_CHUNK + j * LP_THREADS + threadIdx.x;
+      x[j] = i < V ? row[i] : -INFINITY;
+      mx = fmaxf(mx, x[j]);
+    }
+    mx = block_max(mx, scratch);
+    const float at = mx == -INFINITY ? 0.f : mx;     // (a chunk of -inf adds nothing)
+    float z = 0.f;
+#pragma unroll
+    for (int j = 0; j < PER; ++j) z += expf(x[j] - at);
+    z = block_sum(z, scratch);
+    if (threadIdx.x == 0) parts[(size_t)blockIdx.x * chunks + c] = make_float2(mx, z);
   }
 }
 
-extern "C" int ptl_token_logprob(float* out, const float* logits, const int32_t* tokens, int R, int V,
+__global__ void __launch_bounds__(64)
+token_logprob_kernel(float* __restrict__ out, const float2* __restrict__ parts, int chunks,
+                     const float* __restrict__ logits, const int32_t* __restrict__ tokens, int V, long stride) {
+  const int r = blockIdx.x, lane = threadIdx.x;
+  parts += (size_t)r * chunks;
+  float mx = -INFINITY, z = 0.f;
+  for (int c = lane; c < chunks; c += 64) mx = fmaxf(mx, parts[c].x);
+  mx = wave_max(mx);
+  for (int c = lane; c < chunks; c += 64) z += parts[c].y * expf(parts[c].x - mx);
+  z = wave_sum(z);
+  if (lane == 0) {
+    const int t = tokens[r];
+    out[r] = (t >= 0 && t < V) ? logits[(size_t)r * stride + t] - mx - logf(z) : -INFINITY;
+  }
+}
+
+// parts: ceil(V / 4096) * 2 floats a row, 8-byte aligned
+extern "C" int ptl_token_logprob(float* out, float* parts, const float* logits, const int32_t* tokens, int R, int V,
                                  long stride, hipStream_t stream) {
   if (R <= 0) return PTL_OK;
-  if (V <= 0 || stride < V) return PTL_ERR_ARG;
-  token_logprob_kernel<<<R, 1024, 0, stream>>>(out, logits, tokens, V, stride);
+  if (V <= 0 || V > 0x7fffffff - LP_CHUNK || stride < V || !parts) return PTL_ERR_ARG;
+  const int chunks = (V + LP_CHUNK - 1) / LP_CHUNK;
+  token_logprob_part_kernel<<<dim3(R, chunks < 65535 ? chunks : 65535), LP_THREADS, 0, stream>>>(
+      (float2*)parts, chunks, logits, V, stride);
+  token_logprob_kernel<<<R, 64, 0, stream>>>(out, (const float2*)parts, chunks, logits, tokens, V, stride);
   return ptl_launch_status();
 }

@@ -981,7 +981,9 @@ def sample_top_p(logits: torch.Tensor, temperature: torch.Tensor, top_p: torch.T
     elif wide and V > SAMPLE_WIDE_UP_TO:
         raise KernelError(f"sample_top_p: the many-workgroup form takes rows up to {SAMPLE_WIDE_UP_TO}")
     out = torch.empty((R,), dtype=torch.int32, device=logits.device)
-    probs = torch.empty((R, V), dtype=torch.float32, device=logits.device)   # scratch, then result
+    # the result, if wanted, and the scratch of the one-workgroup form
+    probs = (torch.empty((R, V), dtype=torch.float32, device=logits.device) if return_probs or not wide
+             else None)
     lib = library.load("sampling")
     if wide:
         lib.ptl_sample_top_p_wide_workspace.restype = ctypes.c_size_t
@@ -1009,7 +1011,8 @@ def token_logprob(logits: torch.Tensor, tokens: torch.Tensor) -> torch.Tensor:
         raise KernelError("token_logprob: one token per row")
     out = torch.empty((R,), dtype=torch.float32, device=logits.device)
     lib = library.load("sampling")
-    _check(lib.ptl_token_logprob(_ptr(out), _ptr(logits), _ptr(tokens), R, V,
+    parts = torch.empty((R, -(-V // 4096), 2), dtype=torch.float32, device=logits.device)
+    _check(lib.ptl_token_logprob(_ptr(out), _ptr(parts), _ptr(logits), _ptr(tokens), R, V,
                                  ctypes.c_long(logits.stride(0)), _stream()), "token_logprob")
     return out
 

@@ -752,6 +752,23 @@ def test_attention_generic(ops, dtype, case):
     _attention_case(ops, dtype, **case)
 
 
+@pytest.mark.parametrize("V", [1, 4095, 4096, 4097, 3 * 4096 + 5])
+def test_token_logprob_at_the_edges_of_chunks(ops, V):
+    """Against 64 bits: the sum of V exponentials is off by (V / 256 + 16) 2^-24 of itself (a thread's share and
+    the tree) and two roundings of each, the logarithm and the two differences by a few ulps of |x - max|."""
+    torch.manual_seed(V)
+    x = 3 * torch.randn(3, V + 2, device="cuda")[:, :V]
+    if V > 4096:
+        x[1, :4096] = float("-inf")                  # a chunk without mass
+    t = torch.tensor([0, V - 1, V], dtype=torch.int32, device="cuda")
+    got = ops.token_logprob(x, t)
+    want = torch.log_softmax(x[:2].double(), -1).gather(1, t[:2, None].long())[:, 0]
+    assert float((got[:2].double() - want).abs().max()) <= (V / 256 + 24) * 2.0 ** -24 + 4 * 2.0 ** -24 * 30
+    assert got[2] == float("-inf")                   # a token outside the row
+    x[0, 0] = float("nan")
+    assert torch.isnan(ops.token_logprob(x, t)[0])
+
+
 @pytest.mark.parametrize("case", [
     # one and two heads a workgroup, tiles of 32, 64 and 128 columns with and without columns beyond the head,
     # blocks of one row, keys one past and short of a tile
