@@ -818,8 +818,9 @@ def attention_decode(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor,
     which brings exactly one query token (see csrc/attention.hip). Head sizes in
     steps of 16 up to 256, float32 or bfloat16. ``matrix_cores``: the MFMA
     variant (bfloat16, head sizes 32/64/96/128, at most 16 heads a kv head, a page
-    size that is a power of two); ``unroll``: its 16-key tiles per wave and turn
-    (1 or 2; 0 leaves the choice to the kernel)."""
+    size that is a power of two), which deals the keys of all sequences out in equal
+    shares; ``num_splits`` is there the most workgroups that a sequence and kv head are worth;
+    ``unroll``: its 16-key tiles per wave and turn (1 or 2; 0 leaves the choice to the kernel)."""
     T, Hq, Hkv, D, page_size = _attention_common(out, q, k_cache, v_cache, q_start, ctx_len,
                                                  block_table, "attention_decode")
     if D % 16 or D > 256:
@@ -829,10 +830,6 @@ def attention_decode(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor,
     if num_splits < 1:
         raise KernelError("attention_decode: num_splits must be >= 1")
     extras = _mask_extras("attention_decode", T, Hq, window, keep_first, chunk, sink, gate, softcap)
-    part_acc = part_ml = None
-    if num_splits > 1:
-        part_acc = torch.empty((n_seq, Hq, num_splits, D), dtype=torch.float32, device=q.device)
-        part_ml = torch.empty((n_seq, Hq, num_splits, 2), dtype=torch.float32, device=q.device)
     lib = library.load("attention")
     if matrix_cores:
         if (not attention_decode_mfma_fits(q.dtype, Hq, Hkv, D, page_size) or q.stride(0) % 8
@@ -840,13 +837,20 @@ def attention_decode(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor,
             raise KernelError("attention_decode: the matrix-core variant needs bfloat16, a head "
                               "size of 32/64/96/128, at most 16 heads a kv head, a page size that "
                               "is a power of two, aligned q rows")
+        lib.ptl_attention_decode_mfma_workspace.restype = ctypes.c_long
+        parts = torch.empty(lib.ptl_attention_decode_mfma_workspace(int(n_seq), Hq, Hkv, D, int(num_splits)),
+                            dtype=torch.float32, device=q.device)
         _check(lib.ptl_attention_decode_mfma(
             _ptr(out), ctypes.c_long(out.stride(0)), _ptr(q), ctypes.c_long(q.stride(0)),
             _ptr(k_cache), _ptr(v_cache), _ptr(q_start), _ptr(ctx_len), _ptr(block_table),
-            int(block_table.stride(0)), _ptr(part_acc), _ptr(part_ml), int(n_seq), Hq, Hkv, D,
+            int(block_table.stride(0)), _ptr(parts), int(n_seq), Hq, Hkv, D,
             page_size, *extras, ctypes.c_float(scale), int(num_splits), int(unroll),
             _stream()), "attention_decode_mfma")
         return
+    part_acc = part_ml = None
+    if num_splits > 1:
+        part_acc = torch.empty((n_seq, Hq, num_splits, D), dtype=torch.float32, device=q.device)
+        part_ml = torch.empty((n_seq, Hq, num_splits, 2), dtype=torch.float32, device=q.device)
     _check(lib.ptl_attention_decode(
         _ptr(out), ctypes.c_long(out.stride(0)), _ptr(q), ctypes.c_long(q.stride(0)),
         _ptr(k_cache), _ptr(v_cache), _ptr(q_start), _ptr(ctx_len), _ptr(block_table),

@@ -813,6 +813,51 @@ def test_attention_decode_mfma(ops, splits, case, unroll):
                     splits=splits, unroll=unroll, **case)
 
 
+@pytest.mark.parametrize("unroll", [1, 2])
+@pytest.mark.parametrize("case", [
+    # contexts that differ so much that the keys are dealt out in equal shares: pairs that begin and end inside
+    # shares and span several, the list in lanes (up to 64 sequences) and in LDS, wide and narrow heads, a window
+    dict(seq_lens=[3000] + [17 * i + 5 for i in range(19)], Hq=8, Hkv=2, D=64, P=16, splits=4),
+    dict(seq_lens=[7] * 5 + [2500, 1, 1900, 33], Hq=6, Hkv=3, D=128, P=16, splits=3),
+    dict(seq_lens=[40 + 3 * i for i in range(69)] + [4100], Hq=4, Hkv=1, D=32, P=8, splits=2),
+    dict(seq_lens=[1] * 64 + [3500], Hq=2, Hkv=2, D=96, P=16, splits=2),
+    dict(seq_lens=[4000] + [300] * 9, Hq=4, Hkv=2, D=64, P=16, window=3000, splits=2),
+    # and one key short of and past what the shares need: 16 sequences, two splits, 2 * (4 + 12) units of 32 keys
+    dict(seq_lens=[1024] + [5] * 15, Hq=4, Hkv=1, D=64, P=16, splits=2),
+    dict(seq_lens=[1025] + [5] * 15, Hq=4, Hkv=1, D=64, P=16, splits=2),
+])
+def test_attention_decode_mfma_shares(ops, case, unroll):
+    _attention_case(ops, torch.bfloat16, q_lens=[1] * len(case["seq_lens"]), kernel="decode_mfma", unroll=unroll,
+                    **case)
+
+
+@pytest.mark.parametrize("n", [12, 80])
+def test_attention_decode_mfma_shares_beside_empty_rows(ops, n):
+    """Rows without keys (padding of a recorded step) between sequences whose keys are dealt out in shares: zeros
+    there, and the other rows as without them."""
+    D, P = 64, 16
+    torch.manual_seed(n)
+    real = [(3 * i, 3000 if i == 1 else 20 + i) for i in range(n // 3)]
+    pages = 200
+    kc, vc = (torch.randn(pages, 2, P, D, device="cuda").to(torch.bfloat16) for _ in range(2))
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")
+    ctx = [0] * n
+    for r, c in real:
+        ctx[r] = c
+    q = torch.randn(n, 8, D, device="cuda").to(torch.bfloat16)
+    bt = torch.arange(pages, dtype=torch.int32, device="cuda").repeat(n, 1)
+
+    def run(rows):
+        out = torch.full((len(rows), 8, D), 9.0, dtype=torch.bfloat16, device="cuda")
+        ops.attention_decode(out, q[rows].contiguous(), kc, vc, i32(list(range(len(rows) + 1))), i32([ctx[r] for r in rows]),
+                             bt[rows].contiguous(), len(rows), 0.125, num_splits=2, matrix_cores=True)
+        return out.float()
+    out = run(list(range(n)))
+    for r, c in real:
+        torch.testing.assert_close(out[r], run([r])[0], atol=2e-2, rtol=2e-2)
+    assert all(bool((out[r] == 0).all()) for r in range(n) if ctx[r] == 0)
+
+
 def test_attention_decode_mfma_refuses_odd_page_size(ops):
     """A page size that is no power of two is for the general kernel; the fast one says so."""
     assert not ops.attention_decode_mfma_fits(torch.bfloat16, 8, 2, 96, 5)
