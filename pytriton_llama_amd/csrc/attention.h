@@ -32,6 +32,16 @@ __device__ __forceinline__ int first_seen(const AttnExtras& ex, int pos) {
   return 0;
 }
 
+// keys that the sequence's query reads (of the walk: the kept first keys, then the window)
+__device__ __forceinline__ int walk_of(const AttnExtras& ex, int ctx) {
+  const int lo = first_seen(ex, ctx - 1);
+  return ctx - lo + min(max(ex.keep_first, 0), lo);
+}
+// keys of a split, a multiple of ``tile``
+__device__ __forceinline__ int keys_a_split(int span, int num_splits, int tile) {
+  return max(1, ((span + num_splits - 1) / num_splits + tile - 1) / tile) * tile;
+}
+
 __device__ __forceinline__ float head_gate(const AttnExtras& ex, int row, int head) {
   return ex.gate ? 1.0f / (1.0f + expf(-ex.gate[(size_t)row * ex.gate_stride + head])) : 1.0f;
 }

@@ -481,16 +481,6 @@ attn_decode_kernel(TO* __restrict__ out, long out_stride, const T* __restrict__ 
   }
 }
 
-// keys that the sequence's query reads (of the walk: the kept first keys, then the window)
-__device__ __forceinline__ int walk_of(const AttnExtras& ex, int ctx) {
-  const int lo = first_seen(ex, ctx - 1);
-  return ctx - lo + min(max(ex.keep_first, 0), lo);
-}
-// keys of a split, a multiple of ``tile``
-__device__ __forceinline__ int keys_a_split(int span, int num_splits, int tile) {
-  return max(1, ((span + num_splits - 1) / num_splits + tile - 1) / tile) * tile;
-}
-
 template <typename T>
 __global__ void __launch_bounds__(64)
 attn_decode_merge_kernel(T* __restrict__ out, long out_stride, const int32_t* __restrict__ q_start,
@@ -593,6 +583,17 @@ extern "C" int ptl_attention_decode_kv(void* out, long out_stride, int out_f32, 
       Dk > 256 || Dv <= 0 || Dv % 16 || Dv > 256 || page_size <= 0 || num_splits < 1 ||
       num_splits > 1024 || (num_splits > 1 && (!part_acc || !part_ml)) || !extras_ok(ex))
     return PTL_ERR_ARG;
+  if (dtype == PTL_DTYPE_F32 && maps == 1 && Hq / Hkv <= 16 && Hkv <= 65535 &&
+      attn_f32_fits(out, out_stride, q, q_stride, k_cache, v_cache, Dk, Dv) && (num_splits == 1 || (uintptr_t)part_acc % 16 == 0)) {
+    const int rc = attention_f32_decode((float*)out, out_stride, (const float*)q, q_stride, (const float*)k_cache,
+                                        (const float*)v_cache, q_start, ctx_len, block_table, bt_stride,
+                                        SplitArgs{part_acc, part_ml, num_splits}, n_seq, Hq, Hkv, Dk, Dv, page_size, ex,
+                                        scale, stream);
+    if (rc != PTL_OK || num_splits == 1) return rc;
+    attn_decode_merge_kernel<float><<<dim3(n_seq, Hq), 64, 0, stream>>>((float*)out, out_stride, q_start, part_acc, part_ml, Hq,
+                                                                       Dv, num_splits, ex, ctx_len, AF_DECODE_TILE);
+    return ptl_launch_status();
+  }
   const int chunks = (Dk > Dv ? Dk : Dv) / 16;
   int lpk = 1;
   while (lpk < chunks) lpk <<= 1;

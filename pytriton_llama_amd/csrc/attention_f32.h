@@ -1,4 +1,4 @@
-// Attention of prompt portions over a float32 paged cache on the matrix cores, float32 products and
+// Attention over a float32 paged cache on the matrix cores, float32 products and
 // sums throughout (v_mfma_f32_16x16x4_f32). What the vector kernel of attention.hip takes, for key and
 // value sizes that are multiples of 4 up to 128 and 16-byte aligned rows; included by attention.hip.
 //
@@ -18,7 +18,8 @@
 // 16 rows of a fragment meet no bank twice; rows of values are read along the row and need no padding.
 //
 // Measured (one MI355X, us a launch; the vector kernel before in brackets): 700 tokens, 32 heads on 8, head
-// size 64: 58 (447); 150 and 333 tokens, 16 heads on one latent head of 128, values of 96: 38 (298).
+// size 64: 58 (447); 150 and 333 tokens, 16 heads on one latent head of 128, values of 96: 38 (298);
+// one token behind 333 to 601 keys of four sequences, 32 heads on 8, head size 64, 32 splits planned: 9.3 (24.9).
 #pragma once
 #include "attention.h"
 #include "mfma.h"
@@ -26,14 +27,23 @@
 
 #define AF_ROWS 16
 
-template <int HPW, int NK, int BN>
+// Where a decoded token's keys are cut (see below), of num_splits parts of multiples of AF_DECODE_TILE keys.
+#define AF_DECODE_TILE 128
+struct SplitArgs {
+  float *part_acc, *part_ml;     // [sequence][head][num_splits][Dv] and [2]
+  int num_splits;
+};
+
+// DECODE: sequence blockIdx.x brings one token, and the rows of the block are the query heads (up to 16) of kv head
+// blockIdx.y; the keys are shared by blockIdx.z workgroups as well. (HPW 1, maps 1.)
+template <int HPW, int NK, int BN, bool DECODE>
 __global__ void __launch_bounds__(256)
 attn_f32_kernel(float* __restrict__ out, long out_stride, const float* __restrict__ q, long q_stride,
                 const float* __restrict__ k_cache, const float* __restrict__ v_cache,
                 const int32_t* __restrict__ q_start, const int32_t* __restrict__ ctx_len,
                 const int32_t* __restrict__ block_table, int bt_stride, const int32_t* __restrict__ work_seq,
                 const int32_t* __restrict__ work_qoff, int Hq, int Hkv, int maps, int Dk, int Dv, int page_size,
-                AttnExtras ex, float scale) {
+                AttnExtras ex, float scale, SplitArgs sp) {
   constexpr int KS = 4 / HPW;                    // parts of the keys
   constexpr int NG = BN / 16 / KS;               // groups of 16 keys of a tile that a wave takes
   constexpr int D = 16 * NK, KLD = D + 4;        // padded sizes; floats between rows of keys in LDS
@@ -43,24 +53,34 @@ attn_f32_kernel(float* __restrict__ out, long out_stride, const float* __restric
   float* Ks = lds;                               // [2][BN][KLD]
   float* Vs = lds + 2 * BN * KLD;                // [2][BN][D]
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, ln = lane & 15, lg = lane >> 4;
-  const int head = blockIdx.y * HPW + wave % HPW, part = wave / HPW;
-  const int seq = work_seq[blockIdx.x], qoff = work_qoff[blockIdx.x];
-  const int qs = q_start[seq], qlen = q_start[seq + 1] - qs, ctx = ctx_len[seq];
-  const int rows = min(AF_ROWS, qlen - qoff);
+  const int part = wave / HPW, G = (Hq / maps) / Hkv;
+  const int seq = DECODE ? blockIdx.x : work_seq[blockIdx.x], qoff = DECODE ? 0 : work_qoff[blockIdx.x];
+  const int qs = q_start[seq], qlen = DECODE ? 1 : q_start[seq + 1] - qs, ctx = ctx_len[seq];
+  const int rows = DECODE ? G : min(AF_ROWS, qlen - qoff);
   if (rows <= 0) return;
-  const int vh = (head / maps) / ((Hq / maps) / Hkv), kh = vh * maps + head % maps, Hk = Hkv * maps;
+  // this lane's query: head and row of the batch
+  const int head = DECODE ? blockIdx.y * G + min(ln, G - 1) : blockIdx.y * HPW + wave % HPW;
+  const int row = qs + (DECODE ? 0 : qoff + ln);
+  const int vh = DECODE ? blockIdx.y : (head / maps) / G, kh = DECODE ? vh : vh * maps + head % maps, Hk = Hkv * maps;
   const int32_t* bt = block_table + (size_t)seq * bt_stride;
-  const int first_q = ctx - qlen + qoff, qpos = first_q + ln;
-  const int k_end = min(ctx, first_q + rows), k_lo = first_seen(ex, first_q), row_lo = first_seen(ex, qpos);
+  const int first_q = ctx - qlen + qoff, qpos = DECODE ? first_q : first_q + ln;
+  const int k_end = DECODE ? ctx : min(ctx, first_q + rows), k_lo = first_seen(ex, first_q), row_lo = first_seen(ex, qpos);
   // the walk: the kept first keys left of the window, then the keys from the window's start on
-  const int n_kept = min(max(ex.keep_first, 0), k_lo), shift = k_lo - n_kept, n_walk = n_kept + (k_end - k_lo);
+  const int n_kept = min(max(ex.keep_first, 0), k_lo), shift = k_lo - n_kept, n_all = n_kept + (k_end - k_lo);
+  int k_first = 0, n_walk = n_all;
+  if (DECODE) {
+    const int per = keys_a_split(n_all, sp.num_splits, AF_DECODE_TILE);
+    k_first = blockIdx.z * per;
+    n_walk = min(n_all, k_first + per);
+    if (blockIdx.z > 0 && k_first >= n_walk) return;     // (the first answers for a row without keys)
+  }
   const bool row_valid = ln < rows;
 
   F4 qf[NK];
 #pragma unroll
   for (int c = 0; c < NK; ++c)
     qf[c].u = row_valid && 16 * c + 4 * lg < Dk
-                  ? load16(q + (size_t)(qs + qoff + ln) * q_stride + (size_t)head * Dk + 16 * c + 4 * lg) : zero16();
+                  ? load16(q + (size_t)row * q_stride + (size_t)head * Dk + 16 * c + 4 * lg) : zero16();
 
   const int piece = tid % PIECES, row0 = tid / PIECES;
   int page[P], slot[P];
@@ -96,15 +116,15 @@ attn_f32_kernel(float* __restrict__ out, long out_stride, const float* __restric
   for (int t = 0; t < NK; ++t) acc[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   float m_run = -INFINITY, l_run = 0.f;          // l_run: of this lane's keys only
 
-  if (n_walk > 0) {
-    pages(0);
+  if (n_walk > k_first) {
+    pages(k_first);
     fetch();
-    pages(BN);
+    pages(k_first + BN);
     put(0);
   }
   __syncthreads();
   int buf = 0;
-  for (int k0 = 0; k0 < n_walk; k0 += BN, buf ^= 1) {
+  for (int k0 = k_first; k0 < n_walk; k0 += BN, buf ^= 1) {
     const bool more = k0 + BN < n_walk;
     if (more) {
       fetch();
@@ -202,14 +222,20 @@ attn_f32_kernel(float* __restrict__ out, long out_stride, const float* __restric
     }
   }
   if (!row_valid) return;
+  const bool split = DECODE && n_all > n_walk - k_first;     // a part of the keys: the merge kernel does the rest
+  const size_t place = DECODE ? ((size_t)seq * Hq + head) * sp.num_splits + blockIdx.z : 0;
   float den = l_run, f = 1.f;
-  if (ex.sink) {                                 // one more term of the denominator: exp(sink)
+  if (ex.sink && !split) {                                 // one more term of the denominator: exp(sink)
     const float sk = ex.sink[head], mx = fmaxf(m_run, sk);
     f = expf(m_run - mx);
     den = l_run * f + expf(sk - mx);
   }
-  const float inv = den > 0.f ? f / den * head_gate(ex, qs + qoff + ln, head) : 0.f;
-  float* o = out + (size_t)(qs + qoff + ln) * out_stride + (size_t)head * Dv;
+  const float inv = split ? 1.f : den > 0.f ? f / den * head_gate(ex, row, head) : 0.f;
+  float* o = split ? sp.part_acc + place * Dv : out + (size_t)row * out_stride + (size_t)head * Dv;
+  if (split && lg == 0) {
+    sp.part_ml[place * 2] = m_run;
+    sp.part_ml[place * 2 + 1] = l_run;
+  }
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     if (NK >= 4) {
@@ -227,19 +253,19 @@ attn_f32_kernel(float* __restrict__ out, long out_stride, const float* __restric
   }
 }
 
-template <int HPW, int NK, int BN, typename... Args>
-static int launch_attn_f32(int n_work, int Hq, hipStream_t st, Args... args) {
+template <int HPW, int NK, int BN, bool DECODE, typename... Args>
+static int launch_attn_f32(dim3 grid, hipStream_t st, Args... args) {
   constexpr int D = 16 * NK;
   const size_t tiles = (size_t)2 * BN * (2 * D + 4) * sizeof(float);
   const size_t merge = (size_t)4 * (NK * 256 + 128) * sizeof(float);
   const size_t bytes = tiles > merge ? tiles : merge;
   if (bytes > 64 * 1024 &&
-      hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_f32_kernel<HPW, NK, BN>),
+      hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_f32_kernel<HPW, NK, BN, DECODE>),
                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) != hipSuccess) {
     (void)hipGetLastError();
     return PTL_ERR_ARG;
   }
-  attn_f32_kernel<HPW, NK, BN><<<dim3(n_work, Hq / HPW), 256, bytes, st>>>(args...);
+  attn_f32_kernel<HPW, NK, BN, DECODE><<<grid, 256, bytes, st>>>(args...);
   return ptl_launch_status();
 }
 
@@ -260,9 +286,9 @@ static int attention_f32(float* out, long out_stride, const float* q, long q_str
   const int hpw = maps == 1 && Hq / Hkv % 2 == 0 ? 2 : 1;
   const int size = Dk > Dv ? Dk : Dv;
 #define GO(HPW, NK, BN)                                                                                            \
-  return launch_attn_f32<HPW, NK, BN>(n_work, Hq, st, out, out_stride, q, q_stride, k_cache, v_cache, q_start, ctx_len, \
-                                      block_table, bt_stride, work_seq, work_qoff, Hq, Hkv, maps, Dk, Dv, page_size, ex, \
-                                      scale)
+  return launch_attn_f32<HPW, NK, BN, false>(dim3(n_work, Hq / HPW), st, out, out_stride, q, q_stride, k_cache, v_cache, \
+                                             q_start, ctx_len, block_table, bt_stride, work_seq, work_qoff, Hq, Hkv,    \
+                                             maps, Dk, Dv, page_size, ex, scale, SplitArgs{nullptr, nullptr, 1})
 #define GO_HEADS(NK)             \
   {                              \
     if (hpw == 2) GO(2, NK, 32); \
@@ -272,5 +298,22 @@ static int attention_f32(float* out, long out_stride, const float* q, long q_str
   if (size <= 64) GO_HEADS(4)
   GO_HEADS(8)
 #undef GO_HEADS
+#undef GO
+}
+
+// One token a sequence (arguments as ptl_attention_decode_kv, of attn_f32_fits, one map, at most 16 heads a kv
+// head). Splits without keys leave at once; the caller merges what sequences of several splits left.
+static int attention_f32_decode(float* out, long out_stride, const float* q, long q_stride, const float* k_cache,
+                                const float* v_cache, const int32_t* q_start, const int32_t* ctx_len,
+                                const int32_t* block_table, int bt_stride, const SplitArgs& sp, int n_seq, int Hq, int Hkv,
+                                int Dk, int Dv, int page_size, const AttnExtras& ex, float scale, hipStream_t st) {
+  const int size = Dk > Dv ? Dk : Dv;
+#define GO(NK)                                                                                                    \
+  return launch_attn_f32<1, NK, 64, true>(dim3(n_seq, Hkv, sp.num_splits), st, out, out_stride, q, q_stride, k_cache, \
+                                          v_cache, q_start, ctx_len, block_table, bt_stride, (const int32_t*)nullptr, \
+                                          (const int32_t*)nullptr, Hq, Hkv, 1, Dk, Dv, page_size, ex, scale, sp)
+  if (size <= 32) GO(2);
+  if (size <= 64) GO(4);
+  GO(8);
 #undef GO
 }
