@@ -4,6 +4,7 @@
 // option (see max2 below).
 #include "attention.h"
 #include "common.h"
+#include "device.h"
 #include "mfma.h"
 #include <math.h>
 #include <type_traits>
@@ -11,7 +12,7 @@
 // ===========================================================================
 // ptl_attention_prefill_mfma: bfloat16 prompt portions on the matrix cores.
 //
-// A workgroup of four waves takes 64 or 128 query rows of one head (16 or 32 per
+// A workgroup of four waves (or of eight, which share the keys) takes 64 or 128 query rows of one head (16 or 32 per
 // wave) and walks the sequence's keys in tiles of 64. Key and value tiles go
 // through LDS as they lie in the cache (rows of D), in two buffers: while tile t
 // is used, tile t+1 is on its way from global memory straight into the other
@@ -69,8 +70,10 @@ template <> __device__ __forceinline__ void store4<float>(float* p, const float*
 // takes 64 * RT query rows. KEPT: a window that keeps the sequence's first keys (keep_first > 0):
 // the key tiles then walk a list of two stretches of positions instead of one. CAP: scores are capped:
 // tanh_exp2(raw score * cap_in) takes the place of the raw score and scale_log2 is softcap * log2 e.
-template <int NDK, int NDV, int RT, typename TO, bool KEPT, bool CAP>
-__global__ void __launch_bounds__(256, (NDK + NDV) <= 4 ? 3 : 2)
+// SIDES: groups of four waves in the workgroup. Two sides take the key tiles of a block in turn, each
+// with buffers, maxima and sums of its own, which meet through LDS at the end.
+template <int NDK, int NDV, int RT, typename TO, bool KEPT, bool CAP, int SIDES>
+__global__ void __launch_bounds__(256 * SIDES, SIDES == 1 && (NDK + NDV) <= 4 ? 3 : 2)
 attn_prefill_mfma_kernel(TO* __restrict__ out, long out_stride, const bf16_t* __restrict__ q,
                          long q_stride, const bf16_t* __restrict__ k_cache,
                          const bf16_t* __restrict__ v_cache, const int32_t* __restrict__ q_start,
@@ -87,15 +90,20 @@ attn_prefill_mfma_kernel(TO* __restrict__ out, long out_stride, const bf16_t* __
   // first product nor the transposing reads of the second meet in a bank. Two buffers each,
   // as separate arrays: the compiler then knows that a load into one does not touch the other.
   constexpr bool SW8K = CPRK % 8 == 0, SW8V = CPRV % 8 == 0;
-  __shared__ __attribute__((aligned(1024))) bf16_t Ks0[PF_BN * DK];
-  __shared__ __attribute__((aligned(1024))) bf16_t Ks1[PF_BN * DK];
-  __shared__ __attribute__((aligned(1024))) bf16_t Vs0[PF_BN * DV];
-  __shared__ __attribute__((aligned(1024))) bf16_t Vs1[PF_BN * DV];
+  __shared__ __attribute__((aligned(1024))) bf16_t Ks0[SIDES * PF_BN * DK];
+  __shared__ __attribute__((aligned(1024))) bf16_t Ks1[SIDES * PF_BN * DK];
+  __shared__ __attribute__((aligned(1024))) bf16_t Vs0[SIDES * PF_BN * DV];
+  __shared__ __attribute__((aligned(1024))) bf16_t Vs1[SIDES * PF_BN * DV];
   auto swzk = [](int row) { return SW8K ? (row & 7) : ((row >> 1) & 3); };
   auto swzv = [](int row) { return SW8V ? (row & 7) : ((row >> 1) & 3); };
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int side = SIDES == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+  const int tid = SIDES == 1 ? threadIdx.x : threadIdx.x & 255, lane = tid & 63, wave = tid >> 6;
   const int ln = lane & 15, lg = lane >> 4;
+  bf16_t* const Ka = Ks0 + side * (PF_BN * DK);
+  bf16_t* const Kc = Ks1 + side * (PF_BN * DK);
+  bf16_t* const Va = Vs0 + side * (PF_BN * DV);
+  bf16_t* const Vc = Vs1 + side * (PF_BN * DV);
   // Heads run along x, the fast index of the launch, so that workgroups started one after the
   // other land on the eight XCDs in turn; the heads are dealt out so that XCD c gets heads
   // c * Hq/8 .. (c+1) * Hq/8 - 1: the query heads of a kv head meet in one L2, which then holds
@@ -374,16 +382,16 @@ attn_prefill_mfma_kernel(TO* __restrict__ out, long out_stride, const bf16_t* __
         o[r][2 * NDV] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones.v, pb[r][half].v, o[r][2 * NDV], 0, 0, 0);
   };
 
-  // one turn: tile t + 1 sets out for the other buffer (everyone left it before the last
-  // barrier), tile t is used, and what was loaded is waited for before the barrier
+  // one turn: this side's next tile sets out for its other buffer (everyone left it before the
+  // last barrier), tile t is used, and what was loaded is waited for before the barrier
   auto turn = [&](int t, bf16_t* Kb, bf16_t* Vb, bf16_t* Kn, bf16_t* Vn) __attribute__((always_inline)) {
     const int k0 = k_begin + t * PF_BN;
-    if (t + 1 < n_tiles) {
-      fetch(t + 1, Kn, Vn);
-      load_pages(t + 2);
+    if (t + SIDES < n_tiles) {
+      fetch(t + SIDES, Kn, Vn);
+      load_pages(t + 2 * SIDES);
     }
     // a wave whose rows all lie before this tile has nothing to do in it
-    if (wave_has_rows && k0 <= wave_max_q - shift && (KEPT || k0 + PF_BN > wave_lo_first)) {
+    if ((SIDES == 1 || t < n_tiles) && wave_has_rows && k0 <= wave_max_q - shift && (KEPT || k0 + PF_BN > wave_lo_first)) {
       const bool need_mask = (k0 + PF_BN - 1 > wave_min_q - shift) || (k0 + PF_BN > k_end) || k0 < wave_lo_last;
       if (need_mask)
         tile(k0, Kb, Vb, std::true_type{});
@@ -393,14 +401,52 @@ attn_prefill_mfma_kernel(TO* __restrict__ out, long out_stride, const bf16_t* __
     __builtin_amdgcn_s_waitcnt(0x0F70);      // vmcnt(0): this wave's loads into LDS have landed
     __syncthreads();
   };
-  load_pages(0);
-  fetch(0, Ks0, Vs0);
-  load_pages(1);
+  if (SIDES == 1 || side < n_tiles) {
+    load_pages(side);
+    fetch(side, Ka, Va);
+    load_pages(side + SIDES);
+  }
   __builtin_amdgcn_s_waitcnt(0x0F70);
   __syncthreads();
-  for (int t = 0; t < n_tiles; t += 2) {
-    turn(t, Ks0, Vs0, Ks1, Vs1);
-    if (t + 1 < n_tiles) turn(t + 1, Ks1, Vs1, Ks0, Vs0);
+  // (the conditions count side 0's tiles, so that both sides meet at the same barriers)
+  for (int t = 0; t < n_tiles; t += 2 * SIDES) {
+    turn(t + side, Ka, Va, Kc, Vc);
+    if (t + SIDES < n_tiles) turn(t + SIDES + side, Kc, Vc, Ka, Va);
+  }
+  if constexpr (SIDES == 2) {
+    // Side 1 leaves its sums in the value buffers and the maxima and denominators in the key
+    // buffers (both free since the last barrier), side 0 adds them to its own.
+    static_assert(RT == 1, "the buffers hold the sums of one row tile a wave");
+    float4* const sums = reinterpret_cast<float4*>(Vs0);       // [2 NDV][256]: 256 DV bytes, all of Vs0
+    float2* const ends = reinterpret_cast<float2*>(Ks0);       // [256]
+    if (n_tiles > 1) {                       // (else side 0 has seen all keys there are)
+      if (side == 1) {
+#pragma unroll
+        for (int dt = 0; dt < 2 * NDV; ++dt)
+          sums[256 * dt + tid] = make_float4(o[0][dt][0], o[0][dt][1], o[0][dt][2], o[0][dt][3]);
+        ends[tid] = make_float2(m_run[0], o[0][2 * NDV][0]);
+      }
+      __syncthreads();
+      if (side == 0) {
+        const float2 end = ends[tid];
+        const float m = max2(m_run[0], end.x);
+        // (a side that has seen no key has zero sums; neither has: m is -inf, and so is the other side)
+        const float mine = m_run[0] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((m_run[0] - m) * scale_log2);
+        const float others = end.x == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((end.x - m) * scale_log2);
+#pragma unroll
+        for (int dt = 0; dt < 2 * NDV; ++dt) {
+          const float4 s = sums[256 * dt + tid];
+          o[0][dt][0] = o[0][dt][0] * mine + s.x * others;
+          o[0][dt][1] = o[0][dt][1] * mine + s.y * others;
+          o[0][dt][2] = o[0][dt][2] * mine + s.z * others;
+          o[0][dt][3] = o[0][dt][3] * mine + s.w * others;
+        }
+        o[0][2 * NDV][0] = o[0][2 * NDV][0] * mine + end.y * others;
+        m_run[0] = m;
+      }
+      __syncthreads();                         // the next item's tiles go where the sums lay
+    }
+    if (side == 1) continue;
   }
 
 #pragma unroll
@@ -424,7 +470,7 @@ attn_prefill_mfma_kernel(TO* __restrict__ out, long out_stride, const bf16_t* __
   }   // work items
 }
 
-template <int NDK, int NDV, int RT, typename TO>
+template <int NDK, int NDV, int RT, typename TO, int SIDES>
 static int launch_prefill_mfma(void* out, long out_stride, const void* q, long q_stride,
                                const void* k_cache, const void* v_cache, const int32_t* q_start,
                                const int32_t* ctx_len, const int32_t* block_table, int bt_stride,
@@ -440,7 +486,7 @@ static int launch_prefill_mfma(void* out, long out_stride, const void* q, long q
   const float log2e = 1.4426950408889634f;
   const float scale_log2 = (cap ? ex.softcap : scale) * log2e, cap_in = cap ? 2.0f * log2e * scale / ex.softcap : 0.f;
 #define GO(KEPT, CAP)                                                                                       \
-  attn_prefill_mfma_kernel<NDK, NDV, RT, TO, KEPT, CAP><<<grid, 256, 0, stream>>>(                          \
+  attn_prefill_mfma_kernel<NDK, NDV, RT, TO, KEPT, CAP, SIDES><<<grid, 256 * SIDES, 0, stream>>>(           \
       (TO*)out, out_stride, (const bf16_t*)q, q_stride, (const bf16_t*)k_cache, (const bf16_t*)v_cache,     \
       q_start, ctx_len, block_table, bt_stride, work_seq, work_qoff, n_work, Hq, Hkv, maps, page_size,      \
       page_shift, ex, scale_log2, cap_in)
@@ -453,14 +499,14 @@ static int launch_prefill_mfma(void* out, long out_stride, const void* q, long q
 
 // Keys and values of one size, one score map a head, bfloat16 result: the sizes every model
 // with ordinary heads brings.
-template <int RT>
+template <int RT, int SIDES>
 static int prefill_same_size(int nd, void* out, long out_stride, const void* q, long q_stride,
                              const void* k_cache, const void* v_cache, const int32_t* q_start,
                              const int32_t* ctx_len, const int32_t* block_table, int bt_stride,
                              const int32_t* work_seq, const int32_t* work_qoff, int n_work, int n_groups,
                              int Hq, int Hkv, int page_size, const AttnExtras& ex, float scale,
                              hipStream_t stream) {
-#define GO(N) launch_prefill_mfma<N, N, RT, bf16_t>(out, out_stride, q, q_stride, k_cache, v_cache, q_start, \
+#define GO(N) launch_prefill_mfma<N, N, RT, bf16_t, SIDES>(out, out_stride, q, q_stride, k_cache, v_cache, q_start, \
                                                     ctx_len, block_table, bt_stride, work_seq, work_qoff,  \
                                                     n_work, n_groups, Hq, Hkv, 1, page_size, ex, scale,  \
                                                     stream)
@@ -494,11 +540,23 @@ extern "C" int ptl_attention_prefill_mfma(void* out, long out_stride, const void
       Hq > 65535 || n_groups < 1 || n_groups > n_work || q_stride % 8 || out_stride % 4 ||
       (block_rows != 64 && block_rows != 128) || !extras_ok(ex))
     return PTL_ERR_ARG;
+  // Two sides where there are no more workgroups than compute units. A block's time is that of its
+  // chain of key tiles, and a compute unit with one workgroup of four waves has one wave a SIMD, which
+  // nothing covers: eight waves on two chains of half the length hold the unit as well as a second
+  // workgroup would, and there is none. Beyond that a unit holds two workgroups of four waves (the
+  // buffers of two sides leave no room for a second one), and the chains overlap without this.
+  // 24 heads of 128, 512 rows: on 1,536 keys 40.7 -> 28.5 us, on 3,072 76.8 -> 50.9, a prompt of
+  // 512 16.8 -> 13.3; 32 heads of 64, 285 rows 8.5 -> 7.5. One tile of keys, where the second side only
+  // waits: 6.3 -> 6.7.
+  if (block_rows == 64 && (long)n_groups * Hq <= compute_units())
+    return prefill_same_size<1, 2>(D / 32, out, out_stride, q, q_stride, k_cache, v_cache, q_start, ctx_len,
+                                   block_table, bt_stride, work_seq, work_qoff, n_work, n_groups, Hq, Hkv,
+                                   page_size, ex, scale, stream);
   if (block_rows == 64)
-    return prefill_same_size<1>(D / 32, out, out_stride, q, q_stride, k_cache, v_cache, q_start, ctx_len,
+    return prefill_same_size<1, 1>(D / 32, out, out_stride, q, q_stride, k_cache, v_cache, q_start, ctx_len,
                                 block_table, bt_stride, work_seq, work_qoff, n_work, n_groups, Hq, Hkv,
                                 page_size, ex, scale, stream);
-  return prefill_same_size<2>(D / 32, out, out_stride, q, q_stride, k_cache, v_cache, q_start, ctx_len,
+  return prefill_same_size<2, 1>(D / 32, out, out_stride, q, q_stride, k_cache, v_cache, q_start, ctx_len,
                               block_table, bt_stride, work_seq, work_qoff, n_work, n_groups, Hq, Hkv,
                               page_size, ex, scale, stream);
 }
@@ -523,7 +581,7 @@ extern "C" int ptl_attention_prefill_mfma_kv(void* out, long out_stride, int out
       Hq > 65535 || n_groups < 1 || n_groups > n_work || q_stride % 8 || out_stride % 4 || !extras_ok(ex))
     return PTL_ERR_ARG;
 #define GO(NK, NV, TO)                                                                                  \
-  launch_prefill_mfma<NK, NV, 1, TO>(out, out_stride, q, q_stride, k_cache, v_cache, q_start, ctx_len, \
+  launch_prefill_mfma<NK, NV, 1, TO, 1>(out, out_stride, q, q_stride, k_cache, v_cache, q_start, ctx_len, \
                                      block_table, bt_stride, work_seq, work_qoff, n_work, n_groups, Hq, \
                                      Hkv, maps, page_size, ex, scale, stream)
 #define BY_V(NK, TO)                   \

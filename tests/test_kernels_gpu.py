@@ -918,6 +918,18 @@ def test_attention_prefill_mfma_workgroups_share_the_blocks(ops, kernel, groups)
                     window=100, kernel=kernel, groups=groups)
 
 
+@pytest.mark.parametrize("Hq", [2, 264], ids=["two_sides", "one_side"])
+@pytest.mark.parametrize("D", [32, 64, 96, 128])
+@pytest.mark.parametrize("window", [0, 70])
+def test_attention_prefill_mfma_sides(ops, D, Hq, window):
+    """Few workgroups: two groups of waves share the key tiles of a block (one to six of them, with
+    and without a masked last one, shared list and a workgroup a block); many: one group. Tolerance as
+    for the other cases: the sums differ in order only, in float32."""
+    case = dict(seq_lens=[1, 64, 65, 129, 200, 321], q_lens=[1, 64, 65, 66, 70, 65], Hq=Hq, Hkv=1, D=D, P=16)
+    for groups in (0, 3):
+        _attention_case(ops, torch.bfloat16, kernel="mfma", window=window, groups=groups, **case)
+
+
 def test_attention_prefill_mfma_plan(ops):
     """128-row blocks once there are 1.25 t of them (t: workgroups a head can have resident);
     a workgroup a block up to 2 t blocks, t workgroups beyond; never more workgroups than blocks."""
