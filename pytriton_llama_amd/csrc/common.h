@@ -28,6 +28,11 @@ __device__ __forceinline__ bf16_t float_to_bf16(float f) {
   return (bf16_t)(u >> 16);
 }
 
+// 16 bytes, or zeros, by value: ``ok ? *p : zero`` of two lvalues chooses between addresses, which puts the
+// zeros into scratch memory and makes every such load one that does not know where it points (flat).
+__device__ __forceinline__ uint4 load16(const void* p) { return *reinterpret_cast<const uint4*>(p); }
+__device__ __forceinline__ uint4 zero16() { return make_uint4(0, 0, 0, 0); }
+
 // 16 bytes that a kernel reads once (weights, the cache of a decoding request, a product's result
 // on its way through an elementwise kernel): a load marked as not to be used again, so that it
 // does not displace what later kernels find in the caches.

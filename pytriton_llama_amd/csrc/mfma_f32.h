@@ -21,10 +21,6 @@ union F4 {
   float f[4];
 };
 
-// (a value and not an lvalue: ``ok ? *p : zero`` of two lvalues would choose between addresses)
-__device__ __forceinline__ uint4 load16(const float* p) { return *reinterpret_cast<const uint4*>(p); }
-__device__ __forceinline__ uint4 zero16() { return make_uint4(0, 0, 0, 0); }
-
 __device__ __forceinline__ int f32_piece(int row, int piece) { return row * 8 + (piece ^ ((row >> 1) & 7)); }
 
 // acc[a][b] += A rows (arow[a] .. + 31) x B rows (brow[b] .. + 31)^T over the F32_BK columns in As and Bs:

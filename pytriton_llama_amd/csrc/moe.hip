@@ -598,18 +598,17 @@ moe_gemm_mfma_kernel(bf16_t* __restrict__ out, long ldo, const bf16_t* __restric
   for (int g = 0; g < G; ++g)
 #pragma unroll
     for (int j = 0; j < J; ++j) acc[g][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  const uint4 zero = make_uint4(0, 0, 0, 0);
   const size_t up = (size_t)N * K;
   struct Turn {
     Frag8 a, b[G][J];
   };
   auto load = [&](Turn& f, int k0, int ke) {
     const int k = k0 + 8 * lg;
-    f.a.u = k < ke ? *reinterpret_cast<const uint4*>(arow + k) : zero;
+    f.a.u = k < ke ? load16(arow + k) : zero16();
 #pragma unroll
     for (int j = 0; j < J; ++j) {
-      f.b[0][j].u = k < ke ? load_once(brow[j] + k) : zero;
-      if (GATE_UP) f.b[G - 1][j].u = k < ke ? load_once(brow[j] + up + k) : zero;
+      f.b[0][j].u = k < ke ? load_once(brow[j] + k) : zero16();
+      if (GATE_UP) f.b[G - 1][j].u = k < ke ? load_once(brow[j] + up + k) : zero16();
     }
   };
   auto multiply = [&](const Turn& f) {
