@@ -26,9 +26,13 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 // instruction, of W and of x, still brings 1 KB that is used. It gives twice the workgroups. MT tiles
 // of 8 rows of x share the loads of W.
 //
-// Measured (one MI355X, cold weights, 4 rows; the vector-FMA kernel that ran before in brackets):
-// 16,384 x 2,048 32 us = 4.2 TB/s (245), 2,048 x 8,192 18 us = 3.7 TB/s (928), 128,256 x 2,048 207 us =
-// 5.1 TB/s (680); a decode step of 4 rows at the Llama-3.2-1B shape 2.03 ms (28.2).
+// gemm_f32_few_kernel reads x again for every tile and takes the sums of any length;
+// gemm_f32_held_kernel keeps x in registers and walks several tiles.
+//
+// Measured (one MI355X, cold weights, 4 rows; in brackets the vector-FMA kernel that ran first and
+// gemm_f32_few_kernel): 16,384 x 2,048 25 us = 5.4 TB/s (245, 33), 2,048 x 8,192 17 us = 4.0 TB/s (928, 18.5),
+// 128,256 x 2,048 171 us = 6.1 TB/s (680, 214); a decode step of 4 rows at the Llama-3.2-1B shape 1.57 ms
+// (28.2, 1.78).
 // ===========================================================================
 template <int ROWS, int MT, int U>
 __global__ void __launch_bounds__(1024)
@@ -109,6 +113,71 @@ gemm_f32_few_kernel(float* __restrict__ y, const float* __restrict__ x, const fl
   }
 }
 
+// Up to 8 rows with a wave's share of the columns in registers: x [8, 32 NB] of every wave is read once, and
+// the workgroup then walks 8-row tiles of W (blockIdx.x, + gridDim.x, ...), so that W is all that is read in
+// the loop: read again for every tile, x comes through the same path from L2 as W does and is as many bytes
+// (128,256 x 2,048, us at 1, 4 and 8 rows: 185, 214, 254; held 165, 171, 177). The next tile's first columns are on their way while a tile's sums are
+// added up, in two buffers, one barrier a tile.
+template <int ROWS, int NB>
+__global__ void __launch_bounds__(1024)
+gemm_f32_held_kernel(float* __restrict__ y, const float* __restrict__ x, const float* __restrict__ w,
+                     int M, int N, int K, long ldx, long ldy, int k_per_wave, int tiles) {
+  constexpr int KB = ROWS == 8 ? 32 : 16;        // columns of a block (as above)
+  constexpr int U = 4, S = NB / U;               // blocks a turn, turns a tile
+  static_assert(S % 2 == 0, "the two sets of registers change places an even number of times a tile");
+  extern __shared__ float red[];                 // [2][waves][64][4]
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, ln = lane & 15, lg = lane >> 4;
+  const int nwaves = blockDim.x >> 6;
+  const int koff = 4 * lg + (ROWS == 8 ? 16 * (ln >> 3) : 0);
+  const int kb = wave * k_per_wave, ke = min(K, kb + k_per_wave);
+  const int left = ke - kb - koff;               // this lane's columns of block b are there if KB b < left
+  F4 xf[NB];
+  {
+    const float* xp = x + (size_t)min(ln % ROWS, M - 1) * ldx + kb + koff;
+    const bool row = ln % ROWS < M;
+#pragma unroll
+    for (int b = 0; b < NB; ++b) xf[b].u = row && KB * b < left ? load16(xp + KB * b) : zero16();
+  }
+  F4 wa[U], wb[U];
+  auto load_w = [&](F4 (&f)[U], int tile, int b0) __attribute__((always_inline)) {
+    const float* wp = w + (size_t)min(ROWS * tile + ln % ROWS, N - 1) * K + kb + koff;
+#pragma unroll
+    for (int u = 0; u < U; ++u) f[u].u = KB * (b0 + u) < left ? load_once(wp + KB * (b0 + u)) : zero16();
+  };
+  load_w(wa, blockIdx.x, 0);
+  int at = 0;
+  for (int tile = blockIdx.x; tile < tiles; tile += gridDim.x, at ^= 1) {
+    f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+      F4 (&cur)[U] = s % 2 ? wb : wa;
+      F4 (&next)[U] = s % 2 ? wa : wb;
+      if (s + 1 < S) load_w(next, tile, U * (s + 1));
+      else if (tile + (int)gridDim.x < tiles) load_w(next, tile + gridDim.x, 0);
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          acc = __builtin_amdgcn_mfma_f32_16x16x4f32(cur[u].f[i], xf[U * s + u].f[i], acc, 0, 0, 0);
+    }
+    float* const sums = red + at * nwaves * 256;
+    *reinterpret_cast<f32x4*>(sums + (wave * 64 + lane) * 4) = acc;
+    __syncthreads();
+    for (int i = threadIdx.x; i < ROWS * ROWS; i += blockDim.x) {   // a thread a result, the waves' sums in order
+      const int n = i % ROWS, m = i / ROWS;
+      if (m < M && ROWS * tile + n < N) {
+        float r = 0.f;
+        for (int wv = 0; wv < nwaves; ++wv) {
+          const float* p = sums + wv * 256;
+          r += p[((n >> 2) * 16 + m) * 4 + (n & 3)];
+          if (ROWS == 8) r += p[(((n + 8) >> 2) * 16 + m + 8) * 4 + (n & 3)];
+        }
+        y[(size_t)m * ldy + ROWS * tile + n] = r;
+      }
+    }
+  }
+}
+
 static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
 // M <= 16, K % 4 == 0, ldx % 4 == 0, x and w 16-byte aligned.
@@ -117,7 +186,7 @@ extern "C" int ptl_gemm_f32_few(float* y, const float* x, const float* w, int M,
   if (M <= 0 || N <= 0) return PTL_OK;
   if (M > 16 || K <= 0 || K % 4 || (M > 1 && ldx % 4) || ldx < K || ldy < N || !aligned16(x) || !aligned16(w))
     return PTL_ERR_ARG;
-  // up to 8 rows 8-row tiles (us at 4 rows, 8- against 16-row tiles: 2,048 x 2,048 7.3 / 9.5, 16,384 x 2,048
+  // up to 8 rows 8-row tiles (gemm_f32_few_kernel, us at 4 rows, 8- against 16-row tiles: 2,048 x 2,048 7.3 / 9.5, 16,384 x 2,048
   // 31.7 / 33.0, 2,048 x 8,192 18.0 / 32.7, 128,256 x 2,048 208 / 228); beyond, where they cost a second load of
   // x, only while 16-row tiles leave a third of the compute units empty (us at 16 rows: 2,048 x 8,192 29 / 37,
   // 3,072 x 2,048 16.2 / 11.9, 16,384 x 2,048 54.6 / 39.9). At 16 rows the kernel for many rows takes 32, 18
@@ -134,6 +203,25 @@ extern "C" int ptl_gemm_f32_few(float* y, const float* x, const float* w, int M,
 #define GO(ROWS, MT)                                                                                            \
   gemm_f32_few_kernel<ROWS, MT, 8 / MT><<<(unsigned)blocks, waves * 64, (size_t)waves * MT * 1024, st>>>(          \
       y, x, w, M, N, K, ldx, ldy, per)
+  // x in registers where it fits, up to 512 columns a wave of 8 rows or 256 of 16, 16 waves a compute unit. In
+  // 16-row tiles (us at 16 rows, read again against held): 16,384 x 2,048 43 / 35, 3,072 x 2,048 12.0 / 11.7,
+  // 128,256 x 2,048 317 / 239; not where 8-row tiles are taken for more than 8 rows (2,048 x 2,048 10.0 / 11.3).
+  const int most = rows == 8 ? 512 : 256;
+  if (K <= 16 * most && (M <= 8 || rows == 16)) {
+    const int tiles = (int)blocks;
+    const int hw = max(rows == 8 ? waves : 1, (K + most - 1) / most);
+    const int share = ((K + hw - 1) / hw + 31) / 32 * 32;
+    const long resident = (long)cus * (16 / hw);
+    const long each = (tiles + resident - 1) / resident;
+    const unsigned grid = (unsigned)((tiles + each - 1) / each);
+#define HELD(ROWS, NB) \
+  gemm_f32_held_kernel<ROWS, NB><<<grid, hw * 64, (size_t)hw * 2048, st>>>(y, x, w, M, N, K, ldx, ldy, share, tiles)
+    if (rows == 16) HELD(16, 16);
+    else if (share <= 256) HELD(8, 8);
+    else HELD(8, 16);
+#undef HELD
+    return ptl_launch_status();
+  }
   if (rows == 16) GO(16, 1);
   else if (M <= 8) GO(8, 1);
   else GO(8, 2);

@@ -131,6 +131,14 @@ def test_gemm_f32_matrix_cores(ops, mnk):
     assert (~torch.isfinite(y[M - 1])).all()
 
 
+# rows of x kept in registers: several tiles a workgroup, the longest sums that are kept (16 waves), a wave with
+# fewer columns than the others and one without any, 16-row tiles; just too long to be kept
+@pytest.mark.parametrize("mnk", [(3, 17001, 516), (8, 40, 8192), (5, 2100, 2564), (11, 9001, 4096), (16, 2731, 1028),
+                                 (5, 70, 8196), (9, 2800, 4100)])
+def test_gemm_f32_rows_kept(ops, mnk):
+    test_gemm_f32_matrix_cores(ops, mnk)
+
+
 @pytest.mark.parametrize("sizes", [(1, 36, 8, 3, 2), (70, 132, 66, 2, 1), (200, 64, 130, 5, 2), (9, 30, 20, 4, 2)],
                          ids=["one_row", "65_rows_an_expert", "edges", "unaligned"])
 @pytest.mark.parametrize("gated", [True, False])
