@@ -179,6 +179,10 @@ attn_prefill_mfma_kernel(TO* __restrict__ out, long out_stride, const bf16_t* __
   const int k_end = min(ctx, first_q + rows) - shift;
   const int k_begin = (k_lo / PF_BN) * PF_BN;
   const int n_tiles = (k_end - k_begin + PF_BN - 1) / PF_BN;
+  // Below four tiles side 0 takes them all and side 1 only keeps to the barriers: a turn saved would be the
+  // merge's price. (both: tiles between two turns of a side, side 1's first tile)
+  const int stride = SIDES == 2 && n_tiles >= 4 ? 2 : 1;
+  const int first = side == 0 ? 0 : (stride == 2 ? 1 : n_tiles);
   auto key_at = [&](int kw) { return KEPT ? (kw < n_kept ? kw : kw + shift) : kw; };
   // What a row sees, in indices: its own key is index qw; with kept keys, an index from n_kept on
   // is a key of the window (position index + shift, which is no kept position when shift > 0),
@@ -386,9 +390,9 @@ attn_prefill_mfma_kernel(TO* __restrict__ out, long out_stride, const bf16_t* __
   // last barrier), tile t is used, and what was loaded is waited for before the barrier
   auto turn = [&](int t, bf16_t* Kb, bf16_t* Vb, bf16_t* Kn, bf16_t* Vn) __attribute__((always_inline)) {
     const int k0 = k_begin + t * PF_BN;
-    if (t + SIDES < n_tiles) {
-      fetch(t + SIDES, Kn, Vn);
-      load_pages(t + 2 * SIDES);
+    if (t + stride < n_tiles) {
+      fetch(t + stride, Kn, Vn);
+      load_pages(t + 2 * stride);
     }
     // a wave whose rows all lie before this tile has nothing to do in it
     if ((SIDES == 1 || t < n_tiles) && wave_has_rows && k0 <= wave_max_q - shift && (KEPT || k0 + PF_BN > wave_lo_first)) {
@@ -401,17 +405,17 @@ attn_prefill_mfma_kernel(TO* __restrict__ out, long out_stride, const bf16_t* __
     __builtin_amdgcn_s_waitcnt(0x0F70);      // vmcnt(0): this wave's loads into LDS have landed
     __syncthreads();
   };
-  if (SIDES == 1 || side < n_tiles) {
-    load_pages(side);
-    fetch(side, Ka, Va);
-    load_pages(side + SIDES);
+  if (SIDES == 1 || first < n_tiles) {
+    load_pages(first);
+    fetch(first, Ka, Va);
+    load_pages(first + stride);
   }
   __builtin_amdgcn_s_waitcnt(0x0F70);
   __syncthreads();
   // (the conditions count side 0's tiles, so that both sides meet at the same barriers)
-  for (int t = 0; t < n_tiles; t += 2 * SIDES) {
-    turn(t + side, Ka, Va, Kc, Vc);
-    if (t + SIDES < n_tiles) turn(t + SIDES + side, Kc, Vc, Ka, Va);
+  for (int t = 0; t < n_tiles; t += 2 * stride) {
+    turn(t + first, Ka, Va, Kc, Vc);
+    if (t + stride < n_tiles) turn(t + stride + first, Kc, Vc, Ka, Va);
   }
   if constexpr (SIDES == 2) {
     // Side 1 leaves its sums in the value buffers and the maxima and denominators in the key
@@ -419,7 +423,7 @@ attn_prefill_mfma_kernel(TO* __restrict__ out, long out_stride, const bf16_t* __
     static_assert(RT == 1, "the buffers hold the sums of one row tile a wave");
     float4* const sums = reinterpret_cast<float4*>(Vs0);       // [2 NDV][256]: 256 DV bytes, all of Vs0
     float2* const ends = reinterpret_cast<float2*>(Ks0);       // [256]
-    if (n_tiles > 1) {                       // (else side 0 has seen all keys there are)
+    if (stride == 2) {                       // (else side 0 has seen all keys there are)
       if (side == 1) {
 #pragma unroll
         for (int dt = 0; dt < 2 * NDV; ++dt)
@@ -545,9 +549,10 @@ extern "C" int ptl_attention_prefill_mfma(void* out, long out_stride, const void
   // nothing covers: eight waves on two chains of half the length hold the unit as well as a second
   // workgroup would, and there is none. Beyond that a unit holds two workgroups of four waves (the
   // buffers of two sides leave no room for a second one), and the chains overlap without this.
-  // 24 heads of 128, 512 rows: on 1,536 keys 40.7 -> 28.5 us, on 3,072 76.8 -> 50.9, a prompt of
-  // 512 16.8 -> 13.3; 32 heads of 64, 285 rows 8.5 -> 7.5. One tile of keys, where the second side only
-  // waits: 6.3 -> 6.7.
+  // 24 heads of 128, 512 rows: on 1,536 keys 40.7 -> 29.5 us, on 3,072 76.5 -> 52.5, a prompt of 512
+  // 17.0 -> 13.8; 64 rows on 256 keys 10.6 -> 9.7; 32 heads of 64, 285 rows 8.5 -> 7.7. Below 256 keys the
+  // larger workgroup costs 0.8 us (64 rows on 64 keys 6.3 -> 7.1); how many keys a recorded step will
+  // have is not known at its launch.
   if (block_rows == 64 && (long)n_groups * Hq <= compute_units())
     return prefill_same_size<1, 2>(D / 32, out, out_stride, q, q_stride, k_cache, v_cache, q_start, ctx_len,
                                    block_table, bt_stride, work_seq, work_qoff, n_work, n_groups, Hq, Hkv,
