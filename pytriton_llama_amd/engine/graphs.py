@@ -25,14 +25,6 @@ context (q_start above all) say where the real tokens end; the host copies in th
 a recorded step (q_lens, ctx_lens and the maxima) are the bucket's upper bounds. A mixer with
 state of its own must stop at q_start[i + 1], not at the padded length.
 
-A step with several entries of several tokens (the prompts of a batch that comes in at once) is
-as many launches as one with a single portion and ran at the host's speed (2.65 ms for eight
-prompts of 285 tokens in all, of which the GPU needs 1.9). It runs through a graph captured once
-per bucket of single-token entries, of portions (2, 4, 8, 16) and of tokens in all (every 64 up
-to 512, then as above), the second time a step falls into it: sizes that come once are not worth
-a capture. Models with state of their own beside pages run such steps kernel by kernel (their
-kernels' grids follow the longest portion, which a recorded step would have to assume of all).
-
 All graphs of a runner share one memory pool: they are replayed one at a time on one stream,
 so what a step needs while it runs is the most that any of them needs, not the sum.
 
@@ -266,83 +258,6 @@ class PortionGraphs(_Graphs):
         row_of = {i: j for j, i in enumerate(ones)}
         row_of[portion] = B
         rows = [row_of[i] for i, x in enumerate(entries) if len(x.want)]
-        if not rows:
-            return b.logits[:0]
-        return b.logits.index_select(0, ops.to_device(rows, torch.int32, b.logits.device))
-
-
-# Tokens of several portions in all: finer than for one portion, whose steps of up to 512 tokens all take
-# about the same time. At 285 tokens of eight prompts 320 rows cost 1.9 ms, 512 rows 2.5.
-PROMPT_BUCKETS = tuple(range(64, 512, 64)) + tuple(t for t in PORTION_BUCKETS if t >= 512)
-PROMPT_COUNTS = (2, 4, 8, 16)
-MAX_PROMPT_GRAPHS = 24           # triples (decoding rows, portions, tokens) kept; others run eagerly
-
-
-class PromptGraphs(_Graphs):
-    """Steps of single-token entries (any number up to the largest decode bucket, also none)
-    and 2 to 16 entries of several tokens, up to 2,048 in all, with at most one wanted place
-    each."""
-
-    def __init__(self, *args, **kwargs):
-        super().__init__(*args, **kwargs)
-        self.row_sizes = [0] + bucket_sizes(self.manager.max_num_seqs)
-        self.buckets: Dict[tuple, _Recorded] = {}
-        self.seen: set = set()           # size classes that have come once
-
-    def _key(self, entries):
-        """The size class of a step, or None."""
-        ones = sum(1 for e in entries if len(e.tokens) == 1)
-        m, tokens = len(entries) - ones, sum(len(e.tokens) for e in entries) - ones
-        if (not 2 <= m <= PROMPT_COUNTS[-1] or tokens > PROMPT_BUCKETS[-1] or ones > self.row_sizes[-1]
-                or any(len(e.want) > 1 for e in entries)):
-            return None
-        key = (next(r for r in self.row_sizes if r >= ones), next(c for c in PROMPT_COUNTS if c >= m),
-               next(t for t in PROMPT_BUCKETS if t >= tokens))
-        # (the pool is sized for the logits of max_num_seqs + 1 rows)
-        return key if key[0] + key[1] <= self.manager.max_num_seqs + 1 else None
-
-    def fits(self, entries: Sequence[StepEntry]) -> bool:
-        """Also counts: a size class is recorded the second time it comes."""
-        if len(entries) < 2 or self.manager.states:
-            return False
-        key = self._key(entries)
-        if key is None or not all(self.manager.num_tokens.get(e.request, 0) + len(e.tokens) <= self.max_model_len
-                                  for e in entries):
-            return False
-        if key in self.buckets:
-            return True
-        if key not in self.seen:
-            self.seen.add(key)
-            return False
-        return len(self.buckets) < MAX_PROMPT_GRAPHS
-
-    def step(self, entries: Sequence[StepEntry]) -> torch.Tensor:
-        """Logits [wanted, vocab] in the order of the entries."""
-        key = self._key(entries)
-        tokens_of: list = []
-        starts = take_pages(entries, self.manager, self.model.vocab_size, tokens_of)
-        ones = [i for i, e in enumerate(entries) if len(e.tokens) == 1]
-        multi = [i for i, e in enumerate(entries) if len(e.tokens) != 1]
-        b = self.buckets.get(key)
-        if b is None:
-            B, m, T = key
-            b = self.buckets[key] = _Recorded(self.manager, self.work_lists, self.device,
-                                              StepSizes(B, m, T, self.width, B + m), self.max_model_len)
-        B = b.sizes.decode_rows
-        b.wait_for_last_copy()
-        # the logits of every single-token row and of one row of each portion are computed
-        wanted, row, row_of = list(range(B)), B, {i: j for j, i in enumerate(ones)}
-        for j, i in enumerate(multi):
-            want = entries[i].want
-            wanted.append(row + (want[0] if want else len(tokens_of[i]) - 1))
-            row += len(tokens_of[i])
-            row_of[i] = B + j
-        b.layout.fill([SeqInput(entries[i].request, int(tokens_of[i][0]), starts[i]) for i in ones],
-                      [SeqInput(entries[i].request, tokens_of[i], starts[i]) for i in multi], wanted)
-        self._replay(b, lambda: b.layout.dev.copy_(b.layout.host, non_blocking=True))
-        # rows of the graph's logits in the caller's order of entries (a copy: the next replay
-        # of this bucket overwrites the graph's own buffer)
-        rows = [row_of[i] for i, e in enumerate(entries) if len(e.want)]
         if not rows:
             return b.logits[:0]
         return b.logits.index_select(0, ops.to_device(rows, torch.int32, b.logits.device))

@@ -34,17 +34,14 @@ class ModelRunner:
         # decode-only steps replay a HIP graph when the longest request is known
         self.graphs = None
         self.portion_graphs = None
-        self.prompt_graphs = None
         if (use_graphs and max_model_len and self.device.type == "cuda"
                 and model.graph_capturable()):
-            from .graphs import DecodeGraphs, PortionGraphs, PromptGraphs
+            from .graphs import DecodeGraphs, PortionGraphs
             pool = torch.cuda.graph_pool_handle()
             self.graphs = DecodeGraphs(model, self.manager, self.storage, max_model_len, self.device,
                                        pool, timed_library_products)
             self.portion_graphs = PortionGraphs(model, self.manager, self.storage, max_model_len,
                                                 self.device, pool, timed_library_products)
-            self.prompt_graphs = PromptGraphs(model, self.manager, self.storage, max_model_len, self.device,
-                                              pool, timed_library_products)
 
     def admit(self, request: Hashable) -> None:
         slot = self.manager.admit(request)
@@ -71,8 +68,6 @@ class ModelRunner:
             raise ValueError("only steps that replay a graph can take their tokens from the device")
         elif self.portion_graphs is not None and self.portion_graphs.fits(entries):
             logits = self.portion_graphs.step(entries)
-        elif self.prompt_graphs is not None and self.prompt_graphs.fits(entries):
-            logits = self.prompt_graphs.step(entries)
         else:
             ctx, _ = build_context(entries, self.manager, self.device, self.model.vocab_size,
                                    self.model.work_lists())

@@ -339,55 +339,6 @@ def test_portion_graphs_match_eager_steps(folder_a, folder_b, which, dtype):
     assert all(b.graph is not None for b in used.values())
 
 
-@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
-def test_prompt_graphs_match_eager_steps(folder_b, dtype):
-    """Steps that bring portions of several prompts, alone or beside decoding requests, give the logits of the
-    same steps launched kernel by kernel: recorded the second time a size class comes, replayed with other
-    prompts, fewer portions than the class holds, wanted places anywhere or absent, and pages used again."""
-    from pytriton_llama_amd.config import build_model, read_config_json
-    from pytriton_llama_amd.engine.batch import StepEntry
-    from pytriton_llama_amd.engine.runner import ModelRunner
-    from pytriton_llama_amd.weights import load_weights
-    folder, page = folder_b
-    model = build_model(read_config_json(folder))
-    load_weights(model, folder, dtype, "cuda:0")
-    eager = ModelRunner(model, page, 64, 8)
-    graphed = ModelRunner(model, page, 64, 8, max_model_len=260, use_graphs=True)
-    g = torch.Generator().manual_seed(17)
-    tol = 1e-5 if dtype == torch.float32 else 4e-2       # (as for one portion, above)
-    names = iter(range(1000))
-
-    def both(spec):
-        """spec: (name or None for a new request, tokens, wanted places)"""
-        entries = []
-        for r, n, want in spec:
-            entries.append(StepEntry(next(names) if r is None else r,
-                                     torch.randint(0, model.vocab_size, (n,), generator=g).tolist(), want))
-        le, lg = eager.step(entries).float().cpu(), graphed.step(entries).float().cpu()
-        assert le.shape == lg.shape
-        if le.numel():
-            assert float((le - lg).abs().max()) / float(le.abs().max()) < tol
-        return [e.request for e in entries]
-
-    def end(requests):
-        for r in requests:
-            eager.end(r)
-            graphed.end(r)
-    kept = graphed.prompt_graphs.buckets
-    for i in range(4):                                   # 64 tokens in 4 places: eager, recorded, replayed
-        end(both([(None, 5 + i, [4 + i]), (None, 30, [3]), (None, 9, [8])]))
-        assert set(kept) == ({(0, 4, 64)} if i else set())
-        torch.cuda.synchronize()
-    held = both([(None, 2, [1]), (None, 62, [])])        # two portions have a class of their own: eager
-    for i in range(3):                                   # behind a prefix, beside decoding rows
-        both([(held[0], 1, [0]), (held[1], 7, [6]), (None, 40, [39])])
-        end([held[1]])
-        held[1] = both([(None, 20, [19])])[0]            # (one portion)
-        both([(held[0], 1, [0]), (held[1], 1, [0])])     # (decode)
-    assert (1, 2, 64) in kept and all(b.graph is not None for b in kept.values())
-    assert both([(None, 33, []), (None, 32, [])])        # 65 tokens, nothing wanted: the next class
-
-
 def test_warm_up_captures_the_graphs_and_changes_nothing(folder_b):
     """Engine.warm_up makes the graphs of every bucket the limits allow and gives everything
     back; generation afterwards is what it is without it."""

@@ -76,3 +76,27 @@ def test_wide_model_graph_replays_of_long_portions(wide):
         for a, b in zip(got, want):
             err = float((a - b).abs().max()) / float(b.abs().max())
             assert err < 2e-2, f"replay {i} ({n} tokens): {err}"
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+def test_prompts_that_come_together_give_the_same_bits_every_time(wide, dtype, monkeypatch):
+    """A batch of prompts that comes again and again, on an engine that records its other steps: the same
+    logits bit for bit each time, and nothing is recorded in the middle of serving it."""
+    from pytriton_llama_amd.engine import graphs
+    from pytriton_llama_amd.engine.batch import StepEntry
+    from pytriton_llama_amd.engine.runner import ModelRunner
+    folder, seqs, _ = wide
+    model = load_runner(folder, dtype, 16, 8).model
+    runner = ModelRunner(model, 16, 64, 8, max_model_len=320, use_graphs=True)
+    recorded = []
+    capture = graphs.capture_forward
+    monkeypatch.setattr(graphs, "capture_forward", lambda *a, **k: recorded.append(1) or capture(*a, **k))
+    first = None
+    for _ in range(4):
+        entries = [StepEntry(r, t[:n], [n - 1]) for (r, t), n in zip(seqs.items(), (31, 60, 9))]
+        logits = runner.step(entries).clone()
+        for e in entries:
+            runner.end(e.request)
+        first = logits if first is None else first
+        assert torch.equal(logits, first)
+    assert not recorded
