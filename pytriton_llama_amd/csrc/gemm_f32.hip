@@ -1,49 +1,79 @@
 // y = x W^T in float32 on the matrix cores: row-major x [M, K] (row stride ldx) and W [N, K],
-// float32 products and sums (v_mfma_f32_*_f32 multiplies and adds in float32, so this is the same
+// float32 products and sums (v_mfma_f32_16x16x4_f32 multiplies and adds in float32, so this is the same
 // true 32-bit arithmetic as the vector-FMA kernel of gemm.hip, in another order).
 //
-// Both kernels need K % 4 == 0 and 16-byte aligned rows of x and W; everything else stays with the
-// vector-FMA kernel. Inside a block of k the order of the products is free as long as both
-// operands follow it, so a lane always loads four consecutive k in one 16-byte load and hands them
-// to four matrix instructions one after the other.
+// All kernels need K % 4 == 0 and 16-byte aligned rows of x and W; everything else stays with the
+// vector-FMA kernel.
+//
+// One order of sums. The bits of a result do not depend on the other rows of x, nor on how many there are, so
+// that a request's float32 results are the same alone and in a batch: all kernels add the products of a result
+// in an order that K alone fixes. The columns are cut into spans of span_width(K) (at most 16). A span's sum is
+// that of its even plus that of its odd blocks of 16 columns; either starts from zero and takes its blocks one
+// after the other, four matrix instructions a block, of which number s multiplies columns 3 - s, 7 - s, 11 - s and
+// 15 - s (a lane loads four consecutive columns at once and hands them to the four instructions). The spans'
+// sums are added in order. Which wave, workgroup or lane computes a span is free. (Measured, in us, against
+// kernels whose order followed M: level at up to 8 rows; 64 x 2,048 x 2,048 19.0 -> 15.0, 700 x 2,048 x 2,048 76 -> 80,
+// 300 x 4,096 x 4,096 116 -> 128, 17 x 16 x 2,048 8.9 -> 10.9; a prompt of 700 tokens and a decode step of four rows at
+// the Llama-3.2-1B shape are level, their errors against 64 bits 1.1e-6 -> 4.1e-7 and 4.5e-7 -> 3.9e-7.)
 #include "common.h"
 #include "device.h"
 #include "mfma_f32.h"
 
-typedef float f32x4 __attribute__((ext_vector_type(4)));
+// columns of a span: 256, doubled until there are no more than 16; 128 of short sums, which have few spans to share
+__host__ __device__ static inline int span_width(int K) {
+  int w = K <= 1024 ? 128 : 256;
+  while ((long)w * 16 < K) w <<= 1;
+  return w;
+}
 
 // ===========================================================================
 // Few rows of x (M <= 16, a decode step): bound by reading W once. A workgroup owns ROWS rows of W;
-// its waves split K among themselves, every wave keeps up to 16 KB of W under way (two sets of U
-// loads of 1 KB), and their partial sums meet in LDS. v_mfma_f32_16x16x4_f32: lane l (ln = l % 16,
+// its waves take the spans, every wave keeps up to 16 KB of W under way (two sets of U
+// loads of 1 KB), and the spans' sums meet in LDS. v_mfma_f32_16x16x4_f32: lane l (ln = l % 16,
 // lg = l / 16) holds A[ln][k = lg] and B[k = lg][ln] and gets D[4 lg + i][ln].
 //
 // ROWS 16: A is 16 rows of W x 16 columns, a load instruction reads 64 bytes of each row; B the same
-// columns of 16 rows of x, from L2.
+// columns of 16 rows of x, from L2. Even and odd blocks have sums of their own.
 // ROWS 8: with at most 8 rows of x half of such a tile would be empty, so the tile holds two blocks of
-// 16 columns of the same 8 rows (lanes ln < 8 the first block, ln >= 8 the second), of W and of x
-// alike. The products that matter are then D[n < 8][m < 8] and D[n >= 8][m >= 8], and every load
-// instruction, of W and of x, still brings 1 KB that is used. It gives twice the workgroups. MT tiles
-// of 8 rows of x share the loads of W.
+// 16 columns of the same 8 rows (lanes ln < 8 the even block, ln >= 8 the odd one), of W and of x
+// alike. The products that matter are then D[n < 8][m < 8] and D[n >= 8][m >= 8], the sums of the even and
+// of the odd blocks, and every load instruction, of W and of x, still brings 1 KB that is used. It gives twice
+// the workgroups. MT tiles of 8 rows of x share the loads of W.
 //
 // gemm_f32_few_kernel reads x again for every tile and takes the sums of any length;
 // gemm_f32_held_kernel keeps x in registers and walks several tiles.
 //
-// Measured (one MI355X, cold weights, 4 rows; in brackets the vector-FMA kernel that ran first and
-// gemm_f32_few_kernel): 16,384 x 2,048 25 us = 5.4 TB/s (245, 33), 2,048 x 8,192 17 us = 4.0 TB/s (928, 18.5),
-// 128,256 x 2,048 171 us = 6.1 TB/s (680, 214); a decode step of 4 rows at the Llama-3.2-1B shape 1.57 ms
-// (28.2, 1.78).
+// Measured (one MI355X, cold weights, us at 4 rows; in brackets the vector-FMA kernel that ran first and
+// gemm_f32_few_kernel): 16,384 x 2,048 26 = 5.2 TB/s (240, 33), 2,048 x 8,192 17 = 4.0 TB/s (922, 18.5),
+// 128,256 x 2,048 171 = 6.1 TB/s (643, 214), 2,048 x 2,048 6.7 (209), 64 x 256 3.6 (25); a decode step of 4 rows at
+// the Llama-3.2-1B shape 1.57 ms (28.2).
 // ===========================================================================
+
+// A tile's results from the spans' sums in LDS ([span][MT][64 lanes][4], lane and element as in D; of 8-row tiles
+// the two halves).
+template <int ROWS, int MT>
+__device__ __forceinline__ void few_results(float* __restrict__ y, const float* sums, int spans, int M, int N, int n0,
+                                            long ldy) {
+  for (int i = threadIdx.x; i < ROWS * ROWS * MT; i += blockDim.x) {
+    const int n = i % ROWS, m = i / ROWS, t = m / ROWS, j = m % ROWS;
+    if (m >= M || n0 + n >= N) continue;
+    const float* p = sums + t * 256 + ((n >> 2) * 16 + j) * 4 + (n & 3);
+    constexpr int ODD = (2 * 16 + 8) * 4;          // from D[n][j] to D[n + 8][j + 8]
+    float s = 0.f;
+    for (int sp = 0; sp < spans; ++sp, p += MT * 256) s += ROWS == 8 ? p[0] + p[ODD] : p[0];
+    y[(size_t)m * ldy + n0 + n] = s;
+  }
+}
+
 template <int ROWS, int MT, int U>
 __global__ void __launch_bounds__(1024)
 gemm_f32_few_kernel(float* __restrict__ y, const float* __restrict__ x, const float* __restrict__ w,
-                    int M, int N, int K, long ldx, long ldy, int k_per_wave) {
-  extern __shared__ float red[];                 // [waves][MT][64][4]
-  static_assert(ROWS == 16 || ROWS == 8, "rows of W a tile");
-  constexpr int XR = ROWS;                       // rows of x in a tile
+                    int M, int N, int K, long ldx, long ldy, int width) {
+  extern __shared__ float red[];                 // [waves][MT][64][4]: a wave a span
+  static_assert((ROWS == 16 && MT == 1) || ROWS == 8, "rows of W a tile");
   constexpr int KB = ROWS == 8 ? 32 : 16;        // columns of W that one load instruction covers
+  constexpr int H = ROWS == 8 ? 1 : 2;           // sums a lane keeps of a tile
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, ln = lane & 15, lg = lane >> 4;
-  const int nwaves = blockDim.x >> 6;
   const int n0 = blockIdx.x * ROWS;
   const int koff = 4 * lg + (ROWS == 8 ? 16 * (ln >> 3) : 0);
   const float* wp = w + (size_t)min(n0 + ln % ROWS, N - 1) * K + koff;
@@ -51,15 +81,17 @@ gemm_f32_few_kernel(float* __restrict__ y, const float* __restrict__ x, const fl
   bool xok[MT];
 #pragma unroll
   for (int t = 0; t < MT; ++t) {
-    const int m = XR * t + ln % ROWS;
+    const int m = ROWS * t + ln % ROWS;
     xok[t] = m < M;
     xp[t] = x + (size_t)min(m, M - 1) * ldx + koff;
   }
-  f32x4 acc[MT];
+  f32x4_t acc[MT][H];
 #pragma unroll
-  for (int t = 0; t < MT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const int kb = wave * k_per_wave;
-  const int ke = min(K, kb + k_per_wave);
+  for (int t = 0; t < MT; ++t)
+#pragma unroll
+    for (int h = 0; h < H; ++h) acc[t][h] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  const int kb = wave * width;
+  const int ke = min(K, kb + width);
   // two sets of weight registers: the next U blocks are under way while these are multiplied
   F4 wa[U], wb[U];
   auto load_w = [&](F4 (&f)[U], int k) {
@@ -84,7 +116,7 @@ gemm_f32_few_kernel(float* __restrict__ y, const float* __restrict__ x, const fl
       for (int s = 0; s < 4; ++s)
 #pragma unroll
         for (int t = 0; t < MT; ++t)
-          acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(f[u].f[s], xf[t][u].f[s], acc[t], 0, 0, 0);
+          acc[t][u % H] = __builtin_amdgcn_mfma_f32_16x16x4f32(f[u].f[3 - s], xf[t][u].f[3 - s], acc[t][u % H], 0, 0, 0);
   };
   if (kb < ke) load_w(wa, kb);
   for (int k = kb; k < ke; k += 2 * KB * U) {
@@ -96,58 +128,57 @@ gemm_f32_few_kernel(float* __restrict__ y, const float* __restrict__ x, const fl
     multiply(wb, k1);
   }
 #pragma unroll
-  for (int t = 0; t < MT; ++t)
-    *reinterpret_cast<f32x4*>(red + (((size_t)wave * MT + t) * 64 + lane) * 4) = acc[t];
-  __syncthreads();
-  // a thread a result; the sums of the waves (and of the two blocks of an 8-row tile) in order
-  for (int i = threadIdx.x; i < ROWS * XR * MT; i += blockDim.x) {
-    const int n = i % ROWS, m = i / ROWS, t = m / XR, j = m % XR;
-    if (m >= M || n0 + n >= N) continue;
-    float s = 0.f;
-    for (int wv = 0; wv < nwaves; ++wv) {
-      const float* p = red + ((size_t)wv * MT + t) * 256;
-      s += p[((n >> 2) * 16 + j) * 4 + (n & 3)];
-      if (ROWS == 8) s += p[(((n + 8) >> 2) * 16 + j + 8) * 4 + (n & 3)];
-    }
-    y[(size_t)m * ldy + n0 + n] = s;
+  for (int t = 0; t < MT; ++t) {
+    f32x4_t s = acc[t][0];
+    if (H == 2)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) s[i] += acc[t][H - 1][i];
+    *reinterpret_cast<f32x4_t*>(red + (((size_t)wave * MT + t) * 64 + lane) * 4) = s;
   }
+  __syncthreads();
+  few_results<ROWS, MT>(y, red, blockDim.x >> 6, M, N, n0, ldy);
 }
 
-// Up to 8 rows with a wave's share of the columns in registers: x [8, 32 NB] of every wave is read once, and
-// the workgroup then walks 8-row tiles of W (blockIdx.x, + gridDim.x, ...), so that W is all that is read in
-// the loop: read again for every tile, x comes through the same path from L2 as W does and is as many bytes
-// (128,256 x 2,048, us at 1, 4 and 8 rows: 185, 214, 254; held 165, 171, 177). The next tile's first columns are on their way while a tile's sums are
-// added up, in two buffers, one barrier a tile.
-template <int ROWS, int NB>
+// Up to 8 rows (16 of 16-row tiles) with a wave's share of the columns in registers: x [ROWS, KB NB] of every wave
+// is read once, and the workgroup then walks ROWS-row tiles of W (blockIdx.x, + gridDim.x, ...), so that W is all that
+// is read in the loop: read again for every tile, x comes through the same path from L2 as W does and is as many
+// bytes (128,256 x 2,048, us at 1, 4 and 8 rows: 185, 214, 254; held 161, 171, 177). The next tile's first columns are on their way while a tile's
+// sums are added up, in two buffers, one barrier a tile. SB: load blocks of a span.
+template <int ROWS, int NB, int SB>
 __global__ void __launch_bounds__(1024)
 gemm_f32_held_kernel(float* __restrict__ y, const float* __restrict__ x, const float* __restrict__ w,
-                     int M, int N, int K, long ldx, long ldy, int k_per_wave, int tiles) {
+                     int M, int N, int K, long ldx, long ldy, int tiles) {
   constexpr int KB = ROWS == 8 ? 32 : 16;        // columns of a block (as above)
+  constexpr int H = ROWS == 8 ? 1 : 2;
   constexpr int U = 4, S = NB / U;               // blocks a turn, turns a tile
+  constexpr int EACH = NB / SB;                  // spans of a wave
   static_assert(S % 2 == 0, "the two sets of registers change places an even number of times a tile");
-  extern __shared__ float red[];                 // [2][waves][64][4]
+  static_assert(NB % SB == 0 && SB % U == 0, "a turn does not cross a span's end, a wave's share ends with a span");
+  extern __shared__ float red[];                 // [2][waves][EACH][64][4]
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, ln = lane & 15, lg = lane >> 4;
   const int nwaves = blockDim.x >> 6;
-  const int koff = 4 * lg + (ROWS == 8 ? 16 * (ln >> 3) : 0);
-  const int kb = wave * k_per_wave, ke = min(K, kb + k_per_wave);
-  const int left = ke - kb - koff;               // this lane's columns of block b are there if KB b < left
+  const int kb = KB * NB * wave + 4 * lg + (ROWS == 8 ? 16 * (ln >> 3) : 0);
+  const int left = K - kb;                       // this lane's columns of block b are there if KB b < left
   F4 xf[NB];
   {
-    const float* xp = x + (size_t)min(ln % ROWS, M - 1) * ldx + kb + koff;
+    const float* xp = x + (size_t)min(ln % ROWS, M - 1) * ldx + kb;
     const bool row = ln % ROWS < M;
 #pragma unroll
     for (int b = 0; b < NB; ++b) xf[b].u = row && KB * b < left ? load16(xp + KB * b) : zero16();
   }
   F4 wa[U], wb[U];
   auto load_w = [&](F4 (&f)[U], int tile, int b0) __attribute__((always_inline)) {
-    const float* wp = w + (size_t)min(ROWS * tile + ln % ROWS, N - 1) * K + kb + koff;
+    const float* wp = w + (size_t)min(ROWS * tile + ln % ROWS, N - 1) * K + kb;
 #pragma unroll
     for (int u = 0; u < U; ++u) f[u].u = KB * (b0 + u) < left ? load_once(wp + KB * (b0 + u)) : zero16();
   };
   load_w(wa, blockIdx.x, 0);
   int at = 0;
   for (int tile = blockIdx.x; tile < tiles; tile += gridDim.x, at ^= 1) {
-    f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+    float* const sums = red + at * nwaves * EACH * 256;
+    f32x4_t acc[H];
+#pragma unroll
+    for (int h = 0; h < H; ++h) acc[h] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int s = 0; s < S; ++s) {
       F4 (&cur)[U] = s % 2 ? wb : wa;
@@ -158,23 +189,18 @@ gemm_f32_held_kernel(float* __restrict__ y, const float* __restrict__ x, const f
       for (int u = 0; u < U; ++u)
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-          acc = __builtin_amdgcn_mfma_f32_16x16x4f32(cur[u].f[i], xf[U * s + u].f[i], acc, 0, 0, 0);
-    }
-    float* const sums = red + at * nwaves * 256;
-    *reinterpret_cast<f32x4*>(sums + (wave * 64 + lane) * 4) = acc;
-    __syncthreads();
-    for (int i = threadIdx.x; i < ROWS * ROWS; i += blockDim.x) {   // a thread a result, the waves' sums in order
-      const int n = i % ROWS, m = i / ROWS;
-      if (m < M && ROWS * tile + n < N) {
-        float r = 0.f;
-        for (int wv = 0; wv < nwaves; ++wv) {
-          const float* p = sums + wv * 256;
-          r += p[((n >> 2) * 16 + m) * 4 + (n & 3)];
-          if (ROWS == 8) r += p[(((n + 8) >> 2) * 16 + m + 8) * 4 + (n & 3)];
-        }
-        y[(size_t)m * ldy + ROWS * tile + n] = r;
+          acc[u % H] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur[u].f[3 - i], xf[U * s + u].f[3 - i], acc[u % H], 0, 0, 0);
+      if ((s + 1) * U % SB == 0) {               // the end of a span
+        if (H == 2)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) acc[0][i] += acc[H - 1][i];
+        *reinterpret_cast<f32x4_t*>(sums + ((wave * EACH + s * U / SB) * 64 + lane) * 4) = acc[0];
+#pragma unroll
+        for (int h = 0; h < H; ++h) acc[h] = f32x4_t{0.f, 0.f, 0.f, 0.f};
       }
     }
+    __syncthreads();
+    few_results<ROWS, 1>(y, sums, nwaves * EACH, M, N, ROWS * tile, ldy);
   }
 }
 
@@ -186,42 +212,40 @@ extern "C" int ptl_gemm_f32_few(float* y, const float* x, const float* w, int M,
   if (M <= 0 || N <= 0) return PTL_OK;
   if (M > 16 || K <= 0 || K % 4 || (M > 1 && ldx % 4) || ldx < K || ldy < N || !aligned16(x) || !aligned16(w))
     return PTL_ERR_ARG;
-  // up to 8 rows 8-row tiles (gemm_f32_few_kernel, us at 4 rows, 8- against 16-row tiles: 2,048 x 2,048 7.3 / 9.5, 16,384 x 2,048
-  // 31.7 / 33.0, 2,048 x 8,192 18.0 / 32.7, 128,256 x 2,048 208 / 228); beyond, where they cost a second load of
-  // x, only while 16-row tiles leave a third of the compute units empty (us at 16 rows: 2,048 x 8,192 29 / 37,
-  // 3,072 x 2,048 16.2 / 11.9, 16,384 x 2,048 54.6 / 39.9). At 16 rows the kernel for many rows takes 32, 18
-  // and 46 us; at 32 rows this one is slower at every size.
+  // up to 8 rows 8-row tiles; beyond, where they cost a second load of x, only while 16-row tiles leave a third of
+  // the compute units empty (us at 16 rows, 8- against 16-row tiles: 2,048 x 8,192 29 / 37, 3,072 x 2,048 16.2 /
+  // 11.9, 16,384 x 2,048 54.6 / 39.9). At 32 rows gemm_f32_few_kernel is slower than the tiles below at every size.
   const int cus = compute_units();
   const int rows = M <= 8 || (N + 15) / 16 * 3 < 2L * cus ? 8 : 16;
   const long blocks = (N + rows - 1) / rows;
-  // waves a workgroup: at least 256 columns each (128 in 16-row tiles), until the chip has 32 a compute unit
-  // in 16-row tiles; 8-row tiles read less a wave and take four times as many
-  int waves = 1;
-  const int least = rows == 8 ? 256 : 128;
-  while (waves < 16 && K / (waves * 2) >= least && (waves < 4 || blocks * waves < (rows == 8 ? 64L : 32L) * cus)) waves <<= 1;
-  const int per = ((K + waves - 1) / waves + 31) / 32 * 32;
-#define GO(ROWS, MT)                                                                                            \
-  gemm_f32_few_kernel<ROWS, MT, 8 / MT><<<(unsigned)blocks, waves * 64, (size_t)waves * MT * 1024, st>>>(          \
-      y, x, w, M, N, K, ldx, ldy, per)
-  // x in registers where it fits, up to 512 columns a wave of 8 rows or 256 of 16, 16 waves a compute unit. In
-  // 16-row tiles (us at 16 rows, read again against held): 16,384 x 2,048 43 / 35, 3,072 x 2,048 12.0 / 11.7,
-  // 128,256 x 2,048 317 / 239; not where 8-row tiles are taken for more than 8 rows (2,048 x 2,048 10.0 / 11.3).
-  const int most = rows == 8 ? 512 : 256;
-  if (K <= 16 * most && (M <= 8 || rows == 16)) {
-    const int tiles = (int)blocks;
-    const int hw = max(rows == 8 ? waves : 1, (K + most - 1) / most);
-    const int share = ((K + hw - 1) / hw + 31) / 32 * 32;
-    const long resident = (long)cus * (16 / hw);
-    const long each = (tiles + resident - 1) / resident;
-    const unsigned grid = (unsigned)((tiles + each - 1) / each);
-#define HELD(ROWS, NB) \
-  gemm_f32_held_kernel<ROWS, NB><<<grid, hw * 64, (size_t)hw * 2048, st>>>(y, x, w, M, N, K, ldx, ldy, share, tiles)
-    if (rows == 16) HELD(16, 16);
-    else if (share <= 256) HELD(8, 8);
-    else HELD(8, 16);
+  const int width = span_width(K), spans = (K + width - 1) / width;
+  // x in registers where it fits, up to 512 columns a wave of 8 rows or 256 of 16, 16 waves a compute unit
+  // (16 rows, read again against held: 16,384 x 2,048 43 / 36, 3,072 x 2,048 12.0 / 12.2, 128,256 x 2,048 317 / 230;
+  // not where 8-row tiles are taken for more than 8 rows: 2,048 x 2,048 10.4 / 11.3)
+  if (rows == 8 ? M <= 8 && K <= 8192 : K <= 4096) {
+    // (8 rows: 512 columns a wave where that gives 64 waves a compute unit, else 256)
+    const bool half = rows == 8 && K <= 4096 && blocks * ((K + 511) / 512) < 64L * cus;
+    const int share = rows == 8 && !half ? 512 : 256;
+    const int waves = (K + share - 1) / share;
+    const long resident = (long)cus * (16 / waves);
+    const long walk = (blocks + resident - 1) / resident;
+    const unsigned grid = (unsigned)((blocks + walk - 1) / walk);
+#define HELD(ROWS, NB, SB)                                                                                      \
+  gemm_f32_held_kernel<ROWS, NB, SB><<<grid, waves * 64, (size_t)waves * (NB / SB) * 2048, st>>>(y, x, w, M, N, K, ldx, \
+                                                                                                 ldy, (int)blocks)
+    if (rows == 16 && width == 128) HELD(16, 16, 8);
+    else if (rows == 16) HELD(16, 16, 16);
+    else if (half && width == 128) HELD(8, 8, 4);
+    else if (half) HELD(8, 8, 8);
+    else if (width == 128) HELD(8, 16, 4);
+    else if (width == 256) HELD(8, 16, 8);
+    else HELD(8, 16, 16);
 #undef HELD
     return ptl_launch_status();
   }
+#define GO(ROWS, MT)                                                                                        \
+  gemm_f32_few_kernel<ROWS, MT, 8 / MT><<<(unsigned)blocks, spans * 64, (size_t)spans * MT * 1024, st>>>(y, x, w, M, N, K, \
+                                                                                                       ldx, ldy, width)
   if (rows == 16) GO(16, 1);
   else if (M <= 8) GO(8, 1);
   else GO(8, 2);
@@ -230,69 +254,88 @@ extern "C" int ptl_gemm_f32_few(float* y, const float* x, const float* w, int M,
 }
 
 // ===========================================================================
-// Many rows of x (a prompt portion): tiles of BN rows of W x BM rows of x a workgroup of four waves
-// (two along each side), F32_BK columns of K at a time through LDS, two buffers: the next tile is on its
-// way from memory to registers while this one is multiplied, one barrier a tile.
-// A wave of the largest tile multiplies 64 x 64: for 8 columns it reads four 16-byte fragments a lane and
-// issues 16 matrix instructions of 64 clocks each (mfma_f32.h), so the matrix cores bound it.
+// Many rows of x (a prompt portion): tiles of 64 rows of W x 64 rows of x a workgroup of four waves, each 32 x 32,
+// F32_BK columns of K at a time through LDS, two buffers: the next tile is on its way from memory to registers
+// while this one is multiplied, one barrier a tile. For 16 columns a wave reads four 16-byte fragments a lane and
+// issues 16 matrix instructions of 32 clocks each (mfma_f32.h), so the matrix cores bound it. A wave keeps its
+// results three times, the sums of the even blocks, of the odd blocks and of the spans so far; at the end of a
+// span the first two are added to the third. (Tiles of 128 x 64 and 128 x 128, M 17 to 2,048, N 1,536 to 28,672: at
+// most 5 % faster anywhere, up to 40 % slower.)
 //
-// A grid of few tiles is cut along K as well (blockIdx.y): the parts of the sums go to a workspace
-// [splits, M, N] and a second kernel adds them in order.
+// A grid of few tiles is cut along K as well (blockIdx.y, a number of spans each): the spans' sums go to a
+// workspace [spans, M, N] and a second kernel adds them in order.
 //
-// Measured (one MI355X, us; the vector-FMA kernel that ran before in brackets): 700 x 16,384 x 2,048 420 =
-// 112 TFLOP/s (1,386), 700 x 2,048 x 8,192 230 (1,251), 700 x 3,072 x 2,048 100 (370), 483 x 1,536 x 2,048
-// 38 (224), 64 x 2,048 x 8,192 33 (967). Relative error against 64 bits at K = 2,048: 3.7e-7 (8.1e-7).
+// Measured (one MI355X, us; the vector-FMA kernel that ran before in brackets): 700 x 16,384 x 2,048 432 =
+// 109 TFLOP/s (1,386), 700 x 2,048 x 8,192 237 (1,251), 700 x 3,072 x 2,048 115 (370), 64 x 2,048 x 8,192 30.5 (963),
+// 17 x 2,048 x 2,048 13.5 (228). Relative error against 64 bits of a 700-token prompt's logits at the Llama-3.2-1B shape
+// 4.1e-7 (1.5e-6).
 // ===========================================================================
-template <int BN, int BM>
-__global__ void __launch_bounds__(256)
+#define F32_TILE 64
+// (two workgroups a unit asked for: without it the sums go to accumulation registers and the occupancy falls)
+__global__ void __launch_bounds__(256, 2)
 gemm_f32_tile_kernel(float* __restrict__ y, const float* __restrict__ x, const float* __restrict__ w,
-                     int M, int N, int K, long ldx, long ldy, int tiles_m, int tiles, int k_per_split, long split_stride) {
-  constexpr int TN = BN / 64, TM = BM / 64;      // 32 x 32 results of a wave along each side
-  __shared__ uint4 ws[2][BN * 8];
-  __shared__ uint4 xs[2][BM * 8];
+                     int M, int N, int K, long ldx, long ldy, int tiles_m, int tiles, int width, int k_per_split,
+                     float* __restrict__ parts) {
+  constexpr int T = 2;                           // 16 x 16 results of a wave along each side
+  constexpr int L = F32_TILE / 32;               // 16-byte pieces of W and of x a thread loads, of rows 32 apart
+  __shared__ uint4 ws[2][F32_TILE * 8];
+  __shared__ uint4 xs[2][F32_TILE * 8];
   // Workgroups go to the eight XCDs in turn: each gets a run of tiles, neighbours in the run share
   // rows of W, so that W comes into one L2 once.
   const int per_xcd = (tiles + 7) / 8;
   const int tile = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
   if (tile >= tiles || (int)(blockIdx.x >> 3) >= per_xcd) return;
-  const int n0 = tile / tiles_m * BN, m0 = tile % tiles_m * BM;
+  const int n0 = tile / tiles_m * F32_TILE, m0 = tile % tiles_m * F32_TILE;
   const int kb = blockIdx.y * k_per_split, ke = min(K, kb + k_per_split);
-  y += (size_t)blockIdx.y * split_stride;
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, lr = lane & 31, lh = lane >> 5;
-  const int wn = (wave & 1) * (BN / 2), wm = (wave >> 1) * (BM / 2);
-  const int piece = tid & 7, row = tid >> 3;     // of the tile's 16-byte pieces, those of rows row + 32 i
-  const float* wp[BN / 32];
-  const float* xp[BM / 32];
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, ln = lane & 15, lg = lane >> 4;
+  const int wn = 32 * (wave & 1), wm = 32 * (wave >> 1);
+  const int piece = tid & 7, row = tid >> 3;
+  const float* wp[L];
+  const float* xp[L];
 #pragma unroll
-  for (int i = 0; i < BN / 32; ++i) wp[i] = w + (size_t)min(n0 + row + 32 * i, N - 1) * K + 4 * piece;
+  for (int i = 0; i < L; ++i) wp[i] = w + (size_t)min(n0 + row + 32 * i, N - 1) * K + 4 * piece;
 #pragma unroll
-  for (int i = 0; i < BM / 32; ++i) xp[i] = x + (size_t)min(m0 + row + 32 * i, M - 1) * ldx + 4 * piece;
-  uint4 wr[BN / 32], xr[BM / 32];
+  for (int i = 0; i < L; ++i) xp[i] = x + (size_t)min(m0 + row + 32 * i, M - 1) * ldx + 4 * piece;
+  uint4 wr[L], xr[L];
   auto fetch = [&](int k) {
     const bool ok = k + 4 * piece < ke;
 #pragma unroll
-    for (int i = 0; i < BN / 32; ++i) wr[i] = ok ? load16(wp[i] + k) : zero16();
+    for (int i = 0; i < L; ++i) wr[i] = ok ? load16(wp[i] + k) : zero16();
 #pragma unroll
-    for (int i = 0; i < BM / 32; ++i) xr[i] = ok ? load16(xp[i] + k) : zero16();
+    for (int i = 0; i < L; ++i) xr[i] = ok ? load16(xp[i] + k) : zero16();
   };
   auto put = [&](int b) {
 #pragma unroll
-    for (int i = 0; i < BN / 32; ++i) ws[b][f32_piece(row + 32 * i, piece)] = wr[i];
+    for (int i = 0; i < L; ++i) ws[b][f32_piece(row + 32 * i, piece)] = wr[i];
 #pragma unroll
-    for (int i = 0; i < BM / 32; ++i) xs[b][f32_piece(row + 32 * i, piece)] = xr[i];
+    for (int i = 0; i < L; ++i) xs[b][f32_piece(row + 32 * i, piece)] = xr[i];
   };
-  f32x16_t acc[TN][TM];
+  // results [M, N] of row stride ld, from D[n = 4 lg + i][m = ln] of every 16 x 16 tile
+  auto store = [&](float* to, long ld, const f32x4_t (&v)[T][T]) {
+    const bool four = (N & 3) == 0 && (ld & 3) == 0 && (reinterpret_cast<uintptr_t>(to) & 15) == 0;
 #pragma unroll
-  for (int a = 0; a < TN; ++a)
+    for (int c = 0; c < T; ++c) {
+      const int m = m0 + wm + 16 * c + ln;
+      if (m >= M) continue;
 #pragma unroll
-    for (int b = 0; b < TM; ++b)
+      for (int a = 0; a < T; ++a) {
+        const int n = n0 + wn + 16 * a + 4 * lg;
+        float* at = to + (size_t)m * ld + n;
+        if (four) {
+          if (n < N) *reinterpret_cast<f32x4_t*>(at) = v[a][c];
+        } else {
 #pragma unroll
-      for (int i = 0; i < 16; ++i) acc[a][b][i] = 0.f;
-  int nrow[TN], mrow[TM];
+          for (int i = 0; i < 4; ++i)
+            if (n + i < N) at[i] = v[a][c][i];
+        }
+      }
+    }
+  };
+  f32x4_t acc[2][T][T], sum[T][T];           // acc: of the span's even and of its odd blocks
 #pragma unroll
-  for (int a = 0; a < TN; ++a) nrow[a] = wn + 32 * a;
+  for (int a = 0; a < T; ++a)
 #pragma unroll
-  for (int c = 0; c < TM; ++c) mrow[c] = wm + 32 * c;
+    for (int c = 0; c < T; ++c) acc[0][a][c] = acc[1][a][c] = sum[a][c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   fetch(kb);
   put(0);
   __syncthreads();
@@ -300,42 +343,36 @@ gemm_f32_tile_kernel(float* __restrict__ y, const float* __restrict__ x, const f
   for (int k = kb; k < ke; k += F32_BK, buf ^= 1) {
     const bool more = k + F32_BK < ke;
     if (more) fetch(k + F32_BK);
-    f32_multiply<TN, TM>(acc, ws[buf], xs[buf], nrow, mrow, lane);
+    f32_multiply16<T, T>(acc, ws[buf], xs[buf], wn, wm, lane);
+    if (!more || (k + F32_BK) % width == 0) {    // the end of a span
+#pragma unroll
+      for (int a = 0; a < T; ++a)
+#pragma unroll
+        for (int c = 0; c < T; ++c) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const float s = acc[0][a][c][i] + acc[1][a][c][i];
+            sum[a][c][i] = parts ? s : sum[a][c][i] + s;
+          }
+          acc[0][a][c] = acc[1][a][c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        }
+      if (parts) store(parts + (size_t)(k / width) * M * N, N, sum);
+    }
     if (more) put(buf ^ 1);
     __syncthreads();
   }
-  const bool four = (N & 3) == 0 && (ldy & 3) == 0 && (reinterpret_cast<uintptr_t>(y) & 15) == 0;
-#pragma unroll
-  for (int c = 0; c < TM; ++c) {
-    const int m = m0 + wm + 32 * c + lr;
-    if (m >= M) continue;
-#pragma unroll
-    for (int a = 0; a < TN; ++a)
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int n = n0 + wn + 32 * a + 8 * q + 4 * lh;
-        float* at = y + (size_t)m * ldy + n;
-        if (four) {
-          if (n < N)
-            *reinterpret_cast<float4*>(at) = make_float4(acc[a][c][4 * q], acc[a][c][4 * q + 1], acc[a][c][4 * q + 2],
-                                                         acc[a][c][4 * q + 3]);
-        } else {
-#pragma unroll
-          for (int i = 0; i < 4; ++i)
-            if (n + i < N) at[i] = acc[a][c][4 * q + i];
-        }
-      }
-  }
+  if (!parts) store(y, ldy, sum);
 }
 
 __global__ void __launch_bounds__(256)
-gemm_f32_sum_kernel(float* __restrict__ y, const float* __restrict__ parts, int splits, int M, int N, long ldy) {
+gemm_f32_sum_kernel(float* __restrict__ y, const float* __restrict__ parts, int spans, int M, int N, long ldy) {
   const long total = (long)M * N;
   if ((N & 3) == 0 && (ldy & 3) == 0 && (reinterpret_cast<uintptr_t>(y) & 15) == 0) {
     const long i = ((long)blockIdx.x * 256 + threadIdx.x) * 4;
     if (i >= total) return;
-    float4 s = *reinterpret_cast<const float4*>(parts + i);
-    for (int p = 1; p < splits; ++p) {
+    float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll 4
+    for (int p = 0; p < spans; ++p) {
       const float4 v = *reinterpret_cast<const float4*>(parts + (size_t)p * total + i);
       s.x += v.x; s.y += v.y; s.z += v.z; s.w += v.w;
     }
@@ -346,47 +383,34 @@ gemm_f32_sum_kernel(float* __restrict__ y, const float* __restrict__ parts, int 
     const long i = (long)blockIdx.x * 1024 + j * 256 + threadIdx.x;
     if (i >= total) return;
     float s = 0.f;
-    for (int p = 0; p < splits; ++p) s += parts[(size_t)p * total + i];
+    for (int p = 0; p < spans; ++p) s += parts[(size_t)p * total + i];
     y[i / N * ldy + i % N] = s;
   }
 }
 
-// Sums of fewer products than this are added up in one order whatever the number of rows (every tile
-// walks K alike), so that a request's results do not depend on what else is in its step; ops.gemm_nt
-// keeps them off the kernel for few rows as well.
-#define F32_ONE_ORDER_K 512
-
-struct TilePlan {
-  int bn, bm, splits;
-};
-
-// The tile and the number of cuts along K that a count of the work says are done first. The four
-// waves of a workgroup take the four SIMDs of a compute unit, so what counts is the fullest unit: r
+// Columns that a workgroup takes (a number of spans; all: no second kernel): what a count of the work says is done
+// first. The waves of a workgroup take the four SIMDs of a compute unit, so what counts is the fullest unit: r
 // workgroups, one after the other, at 0.5 TFLOP/s (128 TFLOP/s on 256 units), each with about two
 // steps of F32_BK lost at its start and end; less than three at a time on a unit leave gaps (one alone
-// takes 1.6 times as long). A cut costs the second kernel and the traffic of the partial sums.
-// Against a sweep of the three tiles with 1 to 16 cuts (M 64 to 700, N 16 to 16,384, K 2,048 and
-// 8,192; one MI355X) the plan is within 6 % of the fastest; without cuts 483 x 1,536 x 2,048 takes 53
-// instead of 38 us, 64 x 2,048 x 8,192 takes 140 instead of 33. Sums of fewer than F32_ONE_ORDER_K products
-// are never cut.
-static TilePlan tile_plan(int M, int N, int K) {
+// takes 1.6 times as long). Cuts cost the second kernel and the traffic of the spans' sums, however many they are.
+// Against a sweep of all numbers of cuts (M 17 to 700, N 16 to 28,672, K 512 to 14,336; one MI355X) the plan is
+// within 6 % of the fastest; without cuts 64 x 2,048 x 8,192 takes 140 instead of 31.
+static int columns_a_split(int M, int N, int K) {
   const int cus = compute_units();
-  static const struct { int bn, bm; } shapes[] = {{64, 64}, {128, 64}, {128, 128}};
-  TilePlan best{64, 64, 1};
+  const int width = span_width(K), spans = (K + width - 1) / width;
+  const long tiles = (long)((N + F32_TILE - 1) / F32_TILE) * ((M + F32_TILE - 1) / F32_TILE);
+  int best = spans * width;
   double least = 1e30;
-  for (const auto& s : shapes) {
-    const long tiles = (long)((N + s.bn - 1) / s.bn) * ((M + s.bm - 1) / s.bm);
-    for (int splits = 1; splits <= 16; ++splits) {
-      const int per = ((K + splits - 1) / splits + F32_BK - 1) / F32_BK * F32_BK;
-      if (splits > 1 && (K < F32_ONE_ORDER_K || per < 4 * F32_BK || (long)per * (splits - 1) >= K)) continue;
-      const double one = 2.0 * s.bn * s.bm * (per + 2 * F32_BK) / 0.5e12;
-      const double r = (double)((tiles * splits + cus - 1) / cus);
-      double t = one * (r < 4 ? 0.8 * (r + 1) : r + 0.3);
-      if (splits > 1) t += 4e-6 + 4.0 * M * N * (splits + 1) / 6e12;
-      if (t < least) {
-        least = t;
-        best = TilePlan{s.bn, s.bm, splits};
-      }
+  for (int splits = 1; splits <= spans; ++splits) {
+    const int per = (spans + splits - 1) / splits * width;
+    if ((long)per * (splits - 1) >= K) continue;
+    const double one = 2.0 * F32_TILE * F32_TILE * (min(per, K) + 2 * F32_BK) / 0.5e12;
+    const double r = (double)((tiles * splits + cus - 1) / cus);
+    double t = one * (r < 4 ? 0.8 * (r + 1) : r + 0.3);
+    if (splits > 1) t += 4e-6 + 4.0 * M * N * (spans + 1) / 6e12;
+    if (t < least) {
+      least = t;
+      best = per;
     }
   }
   return best;
@@ -395,8 +419,8 @@ static TilePlan tile_plan(int M, int N, int K) {
 // floats of workspace ptl_gemm_f32 wants for these sizes (0: none)
 extern "C" long ptl_gemm_f32_workspace(int M, int N, int K) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
-  const TilePlan p = tile_plan(M, N, K);
-  return p.splits > 1 ? (long)p.splits * M * N : 0;
+  const int width = span_width(K);
+  return columns_a_split(M, N, K) < K ? (long)((K + width - 1) / width) * M * N : 0;
 }
 
 // K % 4 == 0, ldx % 4 == 0, x and w 16-byte aligned. ``parts``: workspace of ptl_gemm_f32_workspace(M, N, K)
@@ -405,23 +429,15 @@ extern "C" int ptl_gemm_f32(float* y, const float* x, const float* w, int M, int
                             float* parts, hipStream_t st) {
   if (M <= 0 || N <= 0) return PTL_OK;
   if (K <= 0 || K % 4 || (M > 1 && ldx % 4) || ldx < K || ldy < N || !aligned16(x) || !aligned16(w)) return PTL_ERR_ARG;
-  const TilePlan p = tile_plan(M, N, K);
-  if (p.splits > 1 && (parts == nullptr || !aligned16(parts))) return PTL_ERR_ARG;
-  const int tiles_m = (M + p.bm - 1) / p.bm;
-  const long tiles = (long)((N + p.bn - 1) / p.bn) * tiles_m;
+  const int width = span_width(K), per = columns_a_split(M, N, K);
+  const bool cut = per < K;
+  if (cut && (parts == nullptr || !aligned16(parts))) return PTL_ERR_ARG;
+  const int tiles_m = (M + F32_TILE - 1) / F32_TILE;
+  const long tiles = (long)((N + F32_TILE - 1) / F32_TILE) * tiles_m;
   if (tiles > 0x3fffffff) return PTL_ERR_ARG;
-  const int per = ((K + p.splits - 1) / p.splits + F32_BK - 1) / F32_BK * F32_BK;
-  float* out = p.splits > 1 ? parts : y;
-  const long ld = p.splits > 1 ? N : ldy;
-  const dim3 grid((unsigned)((tiles + 7) / 8 * 8), p.splits);
-#define GO(BN, BM)                                                                                         \
-  gemm_f32_tile_kernel<BN, BM><<<grid, 256, 0, st>>>(out, x, w, M, N, K, ldx, ld, tiles_m, (int)tiles, per, \
-                                                     p.splits > 1 ? (long)M * N : 0)
-  if (p.bm == 128) GO(128, 128);
-  else if (p.bn == 128) GO(128, 64);
-  else GO(64, 64);
-#undef GO
-  if (p.splits > 1)
-    gemm_f32_sum_kernel<<<(unsigned)(((long)M * N + 1023) / 1024), 256, 0, st>>>(y, parts, p.splits, M, N, ldy);
+  gemm_f32_tile_kernel<<<dim3((unsigned)((tiles + 7) / 8 * 8), (K + per - 1) / per), 256, 0, st>>>(
+      y, x, w, M, N, K, ldx, ldy, tiles_m, (int)tiles, width, per, cut ? parts : nullptr);
+  if (cut)
+    gemm_f32_sum_kernel<<<(unsigned)(((long)M * N + 1023) / 1024), 256, 0, st>>>(y, parts, (K + width - 1) / width, M, N, ldy);
   return ptl_launch_status();
 }

@@ -207,7 +207,8 @@ def rope_store(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, positions: tor
 def gemm_nt(x: torch.Tensor, w: torch.Tensor, out_dtype: Optional[torch.dtype] = None,
             out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """y = x @ w.T with float32 accumulation: float32 operands with 16-byte aligned rows through the
-    32-bit matrix instructions (csrc/gemm_f32.hip), everything else through the vector-FMA kernel.
+    32-bit matrix instructions (csrc/gemm_f32.hip), everything else through the vector-FMA kernel;
+    in both the bits of a row of y do not depend on the other rows of x, nor on how many there are.
     x [M, K] (rows may be strided), w [N, K] contiguous, same dtype."""
     _need_gpu(x, w)
     if x.dim() != 2 or w.dim() != 2 or x.shape[1] != w.shape[1]:
@@ -227,7 +228,7 @@ def gemm_nt(x: torch.Tensor, w: torch.Tensor, out_dtype: Optional[torch.dtype] =
     if x.dtype == torch.float32 and _gemm_f32_fits(x, w, M, K):
         lib = library.load("gemm_f32")
         ldx, ldy = ctypes.c_long(x.stride(0)), ctypes.c_long(y.stride(0))
-        if M <= F32_FEW_ROWS and K >= F32_FEW_FROM_K:
+        if M <= F32_FEW_ROWS:
             _check(lib.ptl_gemm_f32_few(_ptr(y), _ptr(x), _ptr(w), M, N, K, ldx, ldy, _stream()), "gemm_nt")
             return y
         lib.ptl_gemm_f32_workspace.restype = ctypes.c_long
@@ -242,8 +243,7 @@ def gemm_nt(x: torch.Tensor, w: torch.Tensor, out_dtype: Optional[torch.dtype] =
     return y
 
 
-F32_FEW_ROWS = 16          # rows of x up to which the kernel that streams W once takes a float32 product,
-F32_FEW_FROM_K = 512       # and the K from which on: shorter sums are made in one order for any number of rows
+F32_FEW_ROWS = 16          # rows of x up to which the kernel that streams W once takes a float32 product
 
 
 def _gemm_f32_fits(x: torch.Tensor, w: torch.Tensor, M: int, K: int) -> bool:

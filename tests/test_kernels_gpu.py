@@ -139,6 +139,23 @@ def test_gemm_f32_rows_kept(ops, mnk):
     test_gemm_f32_matrix_cores(ops, mnk)
 
 
+@pytest.mark.parametrize("nk", [
+    # one chunk of K and a part of one, chunks of 128, 256, 512 and 1,024 columns with a short last one, few and many
+    # tiles of W, columns past a tile, odd N
+    (16, 64), (37, 128), (70, 388), (2048, 512), (3073, 2052), (9001, 4096), (66, 4100), (2100, 8192), (40, 12292),
+    (515, 16388), (2048, 2048)])
+def test_gemm_f32_same_bits_alone_and_in_a_batch(ops, nk):
+    """A row's float32 results are the same bits whatever the number of rows beside it: every kernel and plan
+    adds the products in one order."""
+    N, K = nk
+    torch.manual_seed(4)
+    x, w = torch.randn(700, K, device="cuda"), torch.randn(N, K, device="cuda")
+    want = ops.gemm_nt(x, w)
+    for M in (1, 2, 8, 9, 16, 17, 33, 64, 65, 129, 300, 483):
+        for first in (0, 700 - M):
+            assert torch.equal(ops.gemm_nt(x[first:first + M], w), want[first:first + M]), (M, first)
+
+
 @pytest.mark.parametrize("sizes", [(1, 36, 8, 3, 2), (70, 132, 66, 2, 1), (200, 64, 130, 5, 2), (9, 30, 20, 4, 2)],
                          ids=["one_row", "65_rows_an_expert", "edges", "unaligned"])
 @pytest.mark.parametrize("gated", [True, False])
