@@ -583,7 +583,7 @@ extern "C" int ptl_attention_decode_kv(void* out, long out_stride, int out_f32, 
       Dk > 256 || Dv <= 0 || Dv % 16 || Dv > 256 || page_size <= 0 || num_splits < 1 ||
       num_splits > 1024 || (num_splits > 1 && (!part_acc || !part_ml)) || !extras_ok(ex))
     return PTL_ERR_ARG;
-  if (dtype == PTL_DTYPE_F32 && maps == 1 && Hq / Hkv <= 16 && Hkv <= 65535 &&
+  if (dtype == PTL_DTYPE_F32 && attn_f32_decodes(Hq, Hkv, maps, Dk, Dv) &&
       attn_f32_fits(out, out_stride, q, q_stride, k_cache, v_cache, Dk, Dv) && (num_splits == 1 || (uintptr_t)part_acc % 16 == 0)) {
     const int rc = attention_f32_decode((float*)out, out_stride, (const float*)q, q_stride, (const float*)k_cache,
                                         (const float*)v_cache, q_start, ctx_len, block_table, bt_stride,

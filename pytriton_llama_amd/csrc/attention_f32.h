@@ -21,6 +21,8 @@
 // size 64: 58 (447); 150 and 333 tokens, 16 heads on one latent head of 128, values of 96: 38 (298);
 // one token behind 333 to 601 keys of four sequences, 32 heads on 8, head size 64, 32 splits planned: 9.3 (24.9).
 #pragma once
+#include <atomic>
+
 #include "attention.h"
 #include "mfma.h"
 #include "mfma_f32.h"
@@ -259,11 +261,18 @@ static int launch_attn_f32(dim3 grid, hipStream_t st, Args... args) {
   const size_t tiles = (size_t)2 * BN * (2 * D + 4) * sizeof(float);
   const size_t merge = (size_t)4 * (NK * 256 + 128) * sizeof(float);
   const size_t bytes = tiles > merge ? tiles : merge;
-  if (bytes > 64 * 1024 &&
-      hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_f32_kernel<HPW, NK, BN, DECODE>),
-                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) != hipSuccess) {
-    (void)hipGetLastError();
-    return PTL_ERR_ARG;
+  if (bytes > 64 * 1024) {                       // more than a kernel gets unasked: asked for once a device
+    static std::atomic<unsigned long long> asked{0};
+    int dev = 64;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev > 63) dev = 64;
+    if (dev == 64 || !(asked.load(std::memory_order_relaxed) >> dev & 1)) {
+      if (hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_f32_kernel<HPW, NK, BN, DECODE>),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        return PTL_ERR_ARG;
+      }
+      if (dev < 64) asked.fetch_or(1ull << dev, std::memory_order_relaxed);
+    }
   }
   attn_f32_kernel<HPW, NK, BN, DECODE><<<grid, 256, bytes, st>>>(args...);
   return ptl_launch_status();
@@ -301,19 +310,28 @@ static int attention_f32(float* out, long out_stride, const float* q, long q_str
 #undef GO
 }
 
-// One token a sequence (arguments as ptl_attention_decode_kv, of attn_f32_fits, one map, at most 16 heads a kv
-// head). Splits without keys leave at once; the caller merges what sequences of several splits left.
+// Where a decoded token takes this kernel (sizes in steps of 16 come here), one map and at most 16 heads a kv head:
+// key and value sizes from 32 to 64. Against the vector kernel (one MI355X, 1 to 40 sequences of 60 to 2,000 keys, 1
+// to 16 heads a kv head): 1.25 to 1.67 times as fast in the mean of a shape, at worst level but for one head a kv head
+// over 32 kv heads and 2,000 keys (119 against 123 us). Above 64 the buffers leave room for one workgroup a compute unit
+// (133 KB; 16 sequences of 2,000 keys, 8 x 128: 89 against 66 us; 8 x 96: 87 against 56), below 32 half of every
+// tile is padding (40 of 2,000 keys, 32 x 16: 143 against 97).
+static bool attn_f32_decodes(int Hq, int Hkv, int maps, int Dk, int Dv) {
+  const int size = Dk > Dv ? Dk : Dv;
+  return maps == 1 && Hq / Hkv <= 16 && Hkv <= 65535 && size >= 32 && size <= 64;
+}
+
+// One token a sequence (arguments as ptl_attention_decode_kv, of attn_f32_fits and attn_f32_decodes). Splits without
+// keys leave at once; the caller merges what sequences of several splits left.
 static int attention_f32_decode(float* out, long out_stride, const float* q, long q_stride, const float* k_cache,
                                 const float* v_cache, const int32_t* q_start, const int32_t* ctx_len,
                                 const int32_t* block_table, int bt_stride, const SplitArgs& sp, int n_seq, int Hq, int Hkv,
                                 int Dk, int Dv, int page_size, const AttnExtras& ex, float scale, hipStream_t st) {
-  const int size = Dk > Dv ? Dk : Dv;
 #define GO(NK)                                                                                                    \
   return launch_attn_f32<1, NK, 64, true>(dim3(n_seq, Hkv, sp.num_splits), st, out, out_stride, q, q_stride, k_cache, \
                                           v_cache, q_start, ctx_len, block_table, bt_stride, (const int32_t*)nullptr, \
                                           (const int32_t*)nullptr, Hq, Hkv, 1, Dk, Dv, page_size, ex, scale, sp)
-  if (size <= 32) GO(2);
-  if (size <= 64) GO(4);
-  GO(8);
+  if (Dk <= 32 && Dv <= 32) GO(2);
+  GO(4);
 #undef GO
 }

@@ -883,6 +883,25 @@ def test_attention_decode_mfma_shares_beside_empty_rows(ops, n):
     assert all(bool((out[r] == 0).all()) for r in range(n) if ctx[r] == 0)
 
 
+@pytest.mark.parametrize("D", [16, 32, 48, 64, 80, 128])
+def test_attention_decode_float32_form_by_head_size(ops, D):
+    """float32 decode attention takes the matrix-core form for sizes 32 to 64 alone; the others give the bits
+    of the vector form, which rows of odd stride always take."""
+    n, Hq, Hkv, P, ctx = 3, 6, 2, 16, [5, 300, 70]
+    torch.manual_seed(D)
+    kc, vc = (torch.randn(60, Hkv, P, D, device="cuda") for _ in range(2))
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")
+    bt = torch.randperm(60)[:57].reshape(3, 19).to(dtype=torch.int32, device="cuda")
+    q = torch.randn(n, Hq, D, device="cuda")
+    outs = []
+    for stride in (Hq * D, Hq * D + 1):
+        out = torch.empty(n, stride, device="cuda")[:, :Hq * D].unflatten(1, (Hq, D))
+        ops.attention_decode(out, q, kc, vc, i32([0, 1, 2, 3]), i32(ctx), bt, n, D ** -0.5, num_splits=2)
+        outs.append(out)
+    torch.testing.assert_close(outs[0], outs[1], atol=1e-5, rtol=1e-5)
+    assert torch.equal(outs[0], outs[1]) == (D not in (32, 48, 64))
+
+
 def test_attention_decode_mfma_refuses_odd_page_size(ops):
     """A page size that is no power of two is for the general kernel; the fast one says so."""
     assert not ops.attention_decode_mfma_fits(torch.bfloat16, 8, 2, 96, 5)
