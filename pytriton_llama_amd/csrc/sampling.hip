@@ -1094,10 +1094,37 @@ extern "C" int ptl_sample_top_p_wide(int32_t* out, float* work, int want_probs, 
 
 // ptl_token_logprob: out[r] = log_softmax(logits[r])[tokens[r]], the log-probability the
 // reference reports for a generated token (F.log_softmax of the step's logits gathered at
-// the token, lite_llama/generete_with_probs.py:154-165). A workgroup a chunk of a row finds the
-// chunk's max and its sum of exp(x - max); a wave a row puts the chunks together. (One workgroup a row
-// reads a row of 128k logits at a small part of what the chip delivers: 64 rows 78 us,
-// now 12; one MI355X.)
+// the token, lite_llama/generete_with_probs.py:154-165). Rows of up to LP_ONE logits: one workgroup a row with the
+// row in registers, one launch, no workspace. Longer ones: a workgroup a chunk of a row finds the chunk's max and its
+// sum of exp(x - max); a wave a row puts the chunks together. (A workgroup reads a row of 128k logits at a small
+// part of what the chip delivers: 64 rows 78 us, by chunks 10. At 32,000 logits the chunks take 5.7 to 6.5 us on
+// the device and this form 7.1 to 7.5, but the second launch and the workspace cost the host 4 us, and a greedy
+// pass with log-probabilities is bound by the host there: 26.3 us by chunks, 22.6 so; one MI355X.)
+#define LP_ONE 32768
+__global__ void __launch_bounds__(1024)
+token_logprob_one_kernel(float* __restrict__ out, const float* __restrict__ logits, const int32_t* __restrict__ tokens,
+                         int V, long stride) {
+  constexpr int PER = LP_ONE / 1024;
+  __shared__ float scratch[16];
+  const float* row = logits + (size_t)blockIdx.x * stride;
+  float x[PER], mx = -INFINITY;
+#pragma unroll
+  for (int j = 0; j < PER; ++j) {
+    const int i = j * 1024 + threadIdx.x;
+    x[j] = i < V ? row[i] : -INFINITY;
+    mx = fmaxf(mx, x[j]);
+  }
+  mx = block_max(mx, scratch);
+  float z = 0.f;
+#pragma unroll
+  for (int j = 0; j < PER; ++j) z += expf(x[j] - mx);
+  z = block_sum(z, scratch);
+  if (threadIdx.x == 0) {
+    const int t = tokens[blockIdx.x];
+    out[blockIdx.x] = (t >= 0 && t < V) ? row[t] - mx - logf(z) : -INFINITY;
+  }
+}
+
 #define LP_CHUNK 4096
 #define LP_THREADS 256
 __global__ void __launch_bounds__(LP_THREADS)
@@ -1139,11 +1166,15 @@ token_logprob_kernel(float* __restrict__ out, const float2* __restrict__ parts, 
   }
 }
 
-// parts: ceil(V / 4096) * 2 floats a row, 8-byte aligned
+// parts: of rows of more than 32,768 logits ceil(V / 4096) * 2 floats a row, 8-byte aligned
 extern "C" int ptl_token_logprob(float* out, float* parts, const float* logits, const int32_t* tokens, int R, int V,
                                  long stride, hipStream_t stream) {
   if (R <= 0) return PTL_OK;
-  if (V <= 0 || V > 0x7fffffff - LP_CHUNK || stride < V || !parts) return PTL_ERR_ARG;
+  if (V <= 0 || V > 0x7fffffff - LP_CHUNK || stride < V || (V > LP_ONE && !parts)) return PTL_ERR_ARG;
+  if (V <= LP_ONE) {
+    token_logprob_one_kernel<<<R, 1024, 0, stream>>>(out, logits, tokens, V, stride);
+    return ptl_launch_status();
+  }
   const int chunks = (V + LP_CHUNK - 1) / LP_CHUNK;
   token_logprob_part_kernel<<<dim3(R, chunks < 65535 ? chunks : 65535), LP_THREADS, 0, stream>>>(
       (float2*)parts, chunks, logits, V, stride);

@@ -1004,6 +1004,9 @@ def sample_top_p(logits: torch.Tensor, temperature: torch.Tensor, top_p: torch.T
     return (out, probs) if return_probs else out
 
 
+LOGPROB_ONE_UP_TO = 32768     # rows up to this long: a workgroup a row (longer ones: many, and a second kernel)
+
+
 def token_logprob(logits: torch.Tensor, tokens: torch.Tensor) -> torch.Tensor:
     """log_softmax(logits[r])[tokens[r]] for float32 logits [R, V] and int32 tokens [R]."""
     _need_gpu(logits, tokens)
@@ -1015,7 +1018,8 @@ def token_logprob(logits: torch.Tensor, tokens: torch.Tensor) -> torch.Tensor:
         raise KernelError("token_logprob: one token per row")
     out = torch.empty((R,), dtype=torch.float32, device=logits.device)
     lib = library.load("sampling")
-    parts = torch.empty((R, -(-V // 4096), 2), dtype=torch.float32, device=logits.device)
+    # (short rows: one workgroup each, no workspace)
+    parts = torch.empty((R, -(-V // 4096), 2), dtype=torch.float32, device=logits.device) if V > LOGPROB_ONE_UP_TO else None
     _check(lib.ptl_token_logprob(_ptr(out), _ptr(parts), _ptr(logits), _ptr(tokens), R, V,
                                  ctypes.c_long(logits.stride(0)), _stream()), "token_logprob")
     return out

@@ -794,6 +794,18 @@ def test_token_logprob_at_the_edges_of_chunks(ops, V):
     assert torch.isnan(ops.token_logprob(x, t)[0])
 
 
+@pytest.mark.parametrize("V", [1023, 1025, 32000, 32768, 32769])
+def test_token_logprob_of_short_rows(ops, V):
+    """Rows of up to 32,768 logits take one launch and allocate their result alone; on both sides of the line the
+    bound of the test above, a thread's share being V / 1024 or V / 256 exponentials."""
+    test_token_logprob_at_the_edges_of_chunks(ops, V)
+    x, t = torch.randn(2, V, device="cuda"), torch.zeros(2, dtype=torch.int32, device="cuda")
+    before = torch.cuda.memory_stats()["allocation.all.allocated"]
+    out = ops.token_logprob(x, t)
+    assert torch.cuda.memory_stats()["allocation.all.allocated"] - before == (1 if V <= 32768 else 2)
+    assert out.shape == (2,)
+
+
 @pytest.mark.parametrize("case", [
     # one and two heads a workgroup, tiles of 32, 64 and 128 columns with and without columns beyond the head,
     # blocks of one row, keys one past and short of a tile
