@@ -524,15 +524,15 @@ static int prefill_same_size(int nd, void* out, long out_stride, const void* q, 
 }
 
 // work_seq / work_qoff list query blocks of ``block_rows`` rows (64 or 128), the longest first;
-// n_groups workgroups a head share them (1 <= n_groups <= n_work). bfloat16 only;
-// q rows must be 16-byte aligned and output rows 8-byte (q_stride % 8, out_stride % 4); the
+// n_groups workgroups a head share them (1 <= n_groups <= n_work). longest: rows of the longest portion, or the
+// most that a recorded step can bring (0: not known). bfloat16 only; q rows must be 16-byte aligned and output rows 8-byte (q_stride % 8, out_stride % 4); the
 // page size is a power of two and a page of all kv heads is smaller than 4 GiB.
 extern "C" int ptl_attention_prefill_mfma(void* out, long out_stride, const void* q, long q_stride,
                                           const void* k_cache, const void* v_cache,
                                           const int32_t* q_start, const int32_t* ctx_len,
                                           const int32_t* block_table, int bt_stride,
                                           const int32_t* work_seq, const int32_t* work_qoff,
-                                          int n_work, int n_groups, int block_rows, int Hq,
+                                          int n_work, int n_groups, int block_rows, int longest, int Hq,
                                           int Hkv, int D,
                                           int page_size, int window, int keep_first, int chunk,
                                           const float* sink, const float* gate, long gate_stride,
@@ -544,16 +544,18 @@ extern "C" int ptl_attention_prefill_mfma(void* out, long out_stride, const void
       Hq > 65535 || n_groups < 1 || n_groups > n_work || q_stride % 8 || out_stride % 4 ||
       (block_rows != 64 && block_rows != 128) || !extras_ok(ex))
     return PTL_ERR_ARG;
-  // Two sides where there are no more workgroups than compute units. A block's time is that of its
+  // Two sides where there are no more workgroups than compute units and portions are long enough to have long
+  // chains of key tiles by themselves. A block's time is that of its
   // chain of key tiles, and a compute unit with one workgroup of four waves has one wave a SIMD, which
   // nothing covers: eight waves on two chains of half the length hold the unit as well as a second
   // workgroup would, and there is none. Beyond that a unit holds two workgroups of four waves (the
   // buffers of two sides leave no room for a second one), and the chains overlap without this.
   // 24 heads of 128, 512 rows: on 1,536 keys 40.7 -> 29.5 us, on 3,072 76.5 -> 52.5, a prompt of 512
-  // 17.0 -> 13.8; 64 rows on 256 keys 10.6 -> 9.7; 32 heads of 64, 285 rows 8.5 -> 7.7. Below 256 keys the
-  // larger workgroup costs 0.8 us (64 rows on 64 keys 6.3 -> 7.1); how many keys a recorded step will
-  // have is not known at its launch.
-  if (block_rows == 64 && (long)n_groups * Hq <= compute_units())
+  // 17.4 -> 14.1, of 300 12.1 -> 11.3; 32 heads of 64, 300 rows 8.9 -> 8.0. Below 256 keys the larger workgroup
+  // costs 0.2 to 0.8 us (64 rows on 64 keys 6.3 -> 7.1, 128 on 128 7.9 -> 8.6, 200 on 200 level), which every short
+  // prompt would pay in every layer; a short portion behind a long prefix would gain (64 rows on 320 keys 12.1 ->
+  // 11.3, on 1,088 29.9 -> 22.8), but how many keys a recorded step will have is not known at its launch.
+  if (block_rows == 64 && (longest <= 0 || longest > 256) && (long)n_groups * Hq <= compute_units())
     return prefill_same_size<1, 2>(D / 32, out, out_stride, q, q_stride, k_cache, v_cache, q_start, ctx_len,
                                    block_table, bt_stride, work_seq, work_qoff, n_work, n_groups, Hq, Hkv,
                                    page_size, ex, scale, stream);

@@ -906,11 +906,12 @@ def attention_prefill_mfma(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Te
                            work_qoff: torch.Tensor, scale: float, window: int = 0,
                            block_rows: int = 64, groups: int = 0, keep_first: int = 0,
                            sink: Optional[torch.Tensor] = None, chunk: int = 0,
-                           gate: Optional[torch.Tensor] = None, softcap: float = 0.0) -> None:
+                           gate: Optional[torch.Tensor] = None, softcap: float = 0.0, longest: int = 0) -> None:
     """bfloat16 attention of prompt portions on the matrix cores; the work list
     names query blocks of ``block_rows`` (64 or 128) rows, those with the most
     keys first. ``groups`` workgroups a head share the list (0: one for every
-    block). Head sizes 32, 64, 96, 128."""
+    block). ``longest``: rows of the longest portion (0: not known), by which few blocks are
+    given two groups of waves each or one. Head sizes 32, 64, 96, 128."""
     T, Hq, Hkv, D, page_size = _attention_common(out, q, k_cache, v_cache, q_start, ctx_len,
                                                  block_table, "attention_prefill_mfma")
     if q.dtype != torch.bfloat16:
@@ -938,7 +939,7 @@ def attention_prefill_mfma(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Te
         _ptr(out), ctypes.c_long(out.stride(0)), _ptr(q), ctypes.c_long(q.stride(0)),
         _ptr(k_cache), _ptr(v_cache), _ptr(q_start), _ptr(ctx_len), _ptr(block_table),
         int(block_table.stride(0)), _ptr(work_seq), _ptr(work_qoff), n_work,
-        min(n_work, int(groups)) if groups > 0 else n_work, int(block_rows), Hq, Hkv, D, page_size,
+        min(n_work, int(groups)) if groups > 0 else n_work, int(block_rows), int(longest), Hq, Hkv, D, page_size,
         *extras, ctypes.c_float(scale), _stream()), "attention_prefill_mfma")
 
 

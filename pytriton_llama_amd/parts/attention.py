@@ -196,7 +196,7 @@ class PagedAttention(Part):
             ws, wo = ctx.work[PORTIONS_128 if rows == 128 else PORTIONS_64]
             ops.attention_prefill_mfma(out, q, k, v, ctx.q_start, ctx.ctx_len,
                                        group.block_table, ws, wo, self.scale, window, rows, groups,
-                                       sink=self.sink)
+                                       sink=self.sink, longest=max(ctx.q_lens[n_dec:]))
         else:
             ws, wo = ctx.work[PORTIONS_16 if n_dec else ALL_16]
             ops.attention_generic(out, q, k, v, ctx.q_start, ctx.ctx_len,

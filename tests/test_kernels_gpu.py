@@ -986,6 +986,29 @@ def test_attention_prefill_mfma_sides(ops, D, Hq, window):
         _attention_case(ops, torch.bfloat16, kernel="mfma", window=window, groups=groups, **case)
 
 
+@pytest.mark.parametrize("D", [64, 128])
+def test_attention_prefill_mfma_short_portions_keep_one_side(ops, D):
+    """Portions of up to 256 rows give the bits of one group of waves (which a launch of many heads always takes),
+    longer ones those of two; nothing known: two."""
+    P, total = 16, 400
+    for rows in (60, 256, 257):
+        kc, vc, bt, _, _ = _paged_setup([total], [rows], 1, D, P, torch.bfloat16, 3)
+        torch.manual_seed(rows)
+        q = torch.randn(rows, 1, D, device="cuda").to(torch.bfloat16)
+        i32 = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")
+        off = list(range(0, rows, 64))[::-1]
+
+        def run(heads, **kw):
+            out = torch.zeros(rows, heads, D, dtype=torch.bfloat16, device="cuda")
+            ops.attention_prefill_mfma(out, q.expand(rows, heads, D).contiguous(), kc.cuda(), vc.cuda(), i32([0, rows]),
+                                       i32([total]), bt.cuda(), i32([0] * len(off)), i32(off), D ** -0.5, **kw)
+            return out[:, 0]
+        one = run(264)
+        assert torch.equal(run(2, longest=rows), one) == (rows <= 256)
+        assert not torch.equal(run(2), one)
+        torch.testing.assert_close(run(2).float(), one.float(), atol=2e-2, rtol=2e-2)
+
+
 def test_attention_prefill_mfma_plan(ops):
     """128-row blocks once there are 1.25 t of them (t: workgroups a head can have resident);
     a workgroup a block up to 2 t blocks, t workgroups beyond; never more workgroups than blocks."""

@@ -100,3 +100,18 @@ def test_prompts_that_come_together_give_the_same_bits_every_time(wide, dtype, m
         first = logits if first is None else first
         assert torch.equal(logits, first)
     assert not recorded
+
+
+def test_attention_is_told_the_longest_portion(wide, monkeypatch):
+    """What the attention of prompt portions chooses its kernel by is the longest portion of the step."""
+    from pytriton_llama_amd import ops
+    from pytriton_llama_amd.engine.batch import StepEntry
+    folder, seqs, _ = wide
+    runner = load_runner(folder, torch.bfloat16, 16, 64)
+    told = []
+    real = ops.attention_prefill_mfma
+    monkeypatch.setattr(ops, "attention_prefill_mfma", lambda *a, **k: told.append(k["longest"]) or real(*a, **k))
+    r = list(seqs)
+    runner.step([StepEntry(r[0], seqs[r[0]][:40], []), StepEntry(r[1], seqs[r[1]], [])])
+    runner.step([StepEntry(r[0], seqs[r[0]][40:], []), StepEntry(r[2], seqs[r[2]][:9], [])])
+    assert told == [77, 77, 260, 260]
