@@ -637,21 +637,28 @@ extern "C" int ptl_attention_decode(void* out, long out_stride, const void* q, l
 // ===========================================================================
 // ptl_attention_decode_mfma: the bfloat16 decode case on the matrix cores.
 //
-// What bounds the kernel is the memory a compute unit keeps on its way (about 26 GB/s a unit, 6.6 TB/s in
-// all), so its time is that of the unit with the most bytes. Two ways to deal the keys out:
-//   equal parts   num_splits workgroups a (sequence, kv head) pair, each with the same share of that pair's
-//                 keys; those without keys leave at once, and a pair that the first one covers is done;
-//   shares        the keys of all pairs, in units of 16 UNR, form one list that is cut into as many equal
-//                 shares as the chip holds workgroups (their LDS is sized so that no unit takes more than
-//                 its number); a workgroup walks its share pair by pair, the first keys of the next pair on
-//                 their way while the waves of the last one are merged.
-// Shares are taken where a step's contexts differ so much that the longest one's equal parts would end well
-// after everybody else (flat_share; each workgroup finds that out from ctx_len, a recorded step does not know
-// it). The parts of a pair meet in a second kernel. Measured (one MI355X, us with the second kernel; equal parts
-// alone, as before, in brackets; * by shares): 20 sequences of 130 to 2,900 keys beside 12 empty rows, 8 kv heads
-// of 128, 35 * (62); 16 of 300 to 3,000 keys, 8 x 128, 32 * (40); 32 of 100 to 2,800 keys, 8 x 64, 28 * (34);
-// 24 of 100 to 2,900, 24 * (28.5); 32 of 2,048, 31.3 (31.5); 8 of 2,100, 15.7 (16.2); 64 of 2,048, 50 (52);
-// 64 of 100 to 450, 8 x 128, 22 (25); 1 of 60 with 32 splits planned 6.1 (8.6).
+// num_splits workgroups a (sequence, kv head) pair, each with an equal part of that pair's keys; those without keys
+// leave at once, and a pair that the first one covers is done. The parts of the others meet in a second kernel.
+//
+// What bounds the kernel is the memory a compute unit keeps on its way (about 26 GB/s a unit however many
+// workgroups it holds, 6.6 TB/s in all), so its time is that of the unit with the most keys. Workgroups go to the
+// units in turn, so with the sequences fastest in the grid the splits of a pair meet on one unit as soon as
+// n_seq * Hkv is a multiple of the units: the longest sequence's unit gets it num_splits times. Where contexts
+// differ (each workgroup finds that out from ctx_len, a recorded step does not know it) workgroups therefore take
+// their pairs by length, the longest first, every second turn of the units from the other end: a unit's second
+// workgroup is short where its first is long. Who computes a part is all that changes: a sequence's bits do not
+// depend on the others. From DECODE_ORDER_KEYS keys a split on (of the longest), where some context is a quarter
+// longer or shorter than the first, for 9 to 64 sequences and 2 to 4 splits: with more splits the parts are short and
+// the order costs 0.5 to 1.5 us (16 sequences, 2 heads of 96, 16 splits: 300 to 3,000 keys 15.0 -> 16.6, 500 each 10.2 ->
+// 11.4); equal contexts keep the order in which a pair's parts lie in the L2 that the second kernel reads them from
+// (48 of 1,000, 8 x 128: 40.9 against 45.0); at 400 keys a split it gains nothing yet (20 of 800 beside 12 empty rows,
+// 8 x 64: 14.5 against 15.8).
+// Measured (one MI355X, us with the second kernel; the sequences fastest in brackets): 20 of 130 to 2,900 keys
+// beside 12 empty rows, 8 kv heads of 128, 42 (55); 32 of 300 to 3,000, 8 x 128, 48 (60), 8 x 64, 29 (34); 16 of 300 to
+// 3,000, 8 x 128, 30 (36); 48 of 300 to 3,000, 8 x 128, 68 (86); 32 of 1,000 to 2,000, 8 x 128, 42 (45.5); one of 3,000
+// beside 31 of 100, 8 x 128, 39 (53); 32 of 2,048, 8 x 64, 27.5 (28.0).
+// (Cutting all pairs' keys as one list into equal shares gave 35, 52, 29, 31, 92, 49, 19 and 29: better only where a few
+// sequences have nearly all keys, worse by up to 1.4 times where a share crosses many short pairs.)
 //
 // A wave takes UNR tiles of 16 keys per turn and all query heads of a kv head at once (up to 16 of them
 // are the N side of the MFMA tiles, so grouped heads cost nothing extra):
@@ -680,84 +687,24 @@ __device__ __forceinline__ void wave_lds_fence() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// workgroups of four waves that a compute unit holds at once, by the registers of a wave
-constexpr int decode_held(int D) { return D <= 64 ? 3 : 2; }
-#define FLAT_MAX_SEQS 4096         // sequences of one launch (their places in the list lie in LDS)
+#define DECODE_ORDER_SEQS 64       // sequences of an ordered launch (one a lane)
+#define DECODE_ORDER_KEYS 512      // keys a split from which on the order matters
 
-// The list of all pairs' keys in units of KEYS: a sequence's pairs follow those of the sequences before it, kv
-// head by kv head. Every wave computes the same from the same numbers; a table ([n_seq] units of the sequences
-// before each, [n_seq] of its own, both of one kv head) is written by its first wave.
-struct FlatList {
-  int total, longest;      // units of one kv head, in all and of the longest sequence
-  int before, units;       // of the sequence asked for
-};
-template <int KEYS>
-__device__ __forceinline__ FlatList flat_list(const AttnExtras& ex, const int32_t* __restrict__ ctx_len, int n_seq,
-                                              int* table, int mine) {
-  const int lane = threadIdx.x & 63;
-  FlatList l{0, 0, 0, 0};
-  for (int s0 = 0; s0 < n_seq; s0 += 64) {
-    const int s = s0 + lane, c = s < n_seq ? ctx_len[s] : 0;
-    const int u = c > 0 ? (walk_of(ex, c) + KEYS - 1) / KEYS : 0;
-    int upto = u, most = u;
-    for (int o = 1; o < 64 && o < n_seq - s0; o <<= 1) {       // (no lane beyond n_seq - s0 adds anything)
-      const int below = __shfl_up(upto, o, 64);
-      if (lane >= o) upto += below;
-      most = max(most, __shfl_xor(most, o, 64));
-    }
-    if (table && s < n_seq && threadIdx.x < 64) {
-      table[s] = l.total + upto - u;
-      table[n_seq + s] = u;
-    }
-    if (mine >= s0 && mine < s0 + 64) {
-      l.before = l.total + __shfl(upto - u, mine - s0, 64);
-      l.units = __shfl(u, mine - s0, 64);
-    }
-    const int last = min(63, n_seq - 1 - s0);
-    l.total += __builtin_amdgcn_readlane(upto, last);
-    l.longest = max(l.longest, __builtin_amdgcn_readfirstlane(most));
-  }
-  return l;
-}
-// Units of the list a workgroup takes when the list is cut into equal shares (at least 128 keys), or 0 when the
-// workgroups of the longest sequence are about as soon done in num_splits equal parts a pair: beginning in the
-// middle of pairs costs a workgroup about as much as 12 units of 32 keys (8 of the wider heads).
-template <int KEYS, int D> struct FlatCost {
-  static constexpr int least = 128 / KEYS, begin = (D <= 64 ? 12 : 8) * 32 / KEYS;
-};
-template <int KEYS, int D>
-__device__ __forceinline__ int flat_share(const FlatList& l, int Hkv, int groups, int num_splits) {
-  const int share = max(FlatCost<KEYS, D>::least, (l.total * Hkv + groups - 1) / groups);
-  return (l.longest + num_splits - 1) / num_splits > share + FlatCost<KEYS, D>::begin ? share : 0;
-}
-// Whether any sequence is long enough for shares at all: what short contexts are spared the list by.
-template <int KEYS, int D>
-__device__ __forceinline__ bool flat_possible(const AttnExtras& ex, const int32_t* __restrict__ ctx_len, int n_seq,
-                                              int num_splits) {
-  const int limit = num_splits * (FlatCost<KEYS, D>::least + FlatCost<KEYS, D>::begin) * KEYS;
-  bool any = false;
-  for (int s = threadIdx.x & 63; s < n_seq; s += 64) any |= walk_of(ex, ctx_len[s]) > limit;
-  return __any(any);
-}
-
-// FLAT: the keys of all pairs may be cut into equal shares (flat_share); groups is the most of them. Otherwise, and
-// where flat_share says so, workgroups (sequence, kv head, split) take num_splits equal parts a pair, and those
-// without keys leave at once. A grid of one dimension, the sequences fastest.
+// A grid of one dimension: workgroups (sequence, kv head, split), the sequences fastest. ORDERED: by length where
+// contexts differ (above); cus: the compute units.
 // KEPT: a window that keeps the sequence's first keys (keep_first > 0). CAP: scores are capped; then
 // scale_log2 is softcap * log2 e and cap_in takes a raw score to tanh_exp2's argument.
-// parts: the results of the parts of pairs, [part][D], and part_ml their (max, denominator), [part][2]: of shares
-// part (2 workgroup + place) G + head of the pair, place 0 for the part that begins with the workgroup's share, 1
-// for one that begins inside; of equal parts (sequence Hq + head) num_splits + split. note [1 + 2 n_seq]: the
-// share, and for shares the list's table.
-template <int NDT, int UNR, bool FLAT, bool KEPT, bool CAP>
-__global__ void __launch_bounds__(256, decode_held(32 * NDT))
+// part_acc [sequence][head][num_splits][D], part_ml [sequence][head][num_splits][2]: the results of the splits of a
+// pair that has several, and their (max, denominator).
+template <int NDT, int UNR, bool ORDERED, bool KEPT, bool CAP>
+__global__ void __launch_bounds__(256, NDT <= 2 ? 3 : 2)
 attn_decode_mfma_kernel(bf16_t* __restrict__ out, long out_stride, const bf16_t* __restrict__ q,
                         long q_stride, const bf16_t* __restrict__ k_cache,
                         const bf16_t* __restrict__ v_cache, const int32_t* __restrict__ q_start,
                         const int32_t* __restrict__ ctx_len, const int32_t* __restrict__ block_table,
-                        int bt_stride, float* __restrict__ parts, float* __restrict__ part_ml, int n_seq, int Hq, int Hkv,
+                        int bt_stride, float* __restrict__ part_acc, float* __restrict__ part_ml, int n_seq, int Hq, int Hkv,
                         int page_size, int page_shift, AttnExtras ex, float scale_log2, float cap_in, int num_splits,
-                        int groups, int table_at, int* __restrict__ note) {
+                        int cus) {
   constexpr int D = 32 * NDT;
   constexpr int NT = 2 * NDT;             // 16-wide tiles of the head dimension
   constexpr int WAVES = 4;
@@ -781,74 +728,56 @@ attn_decode_mfma_kernel(bf16_t* __restrict__ out, long out_stride, const bf16_t*
     vrow[i] = c / CPR;
     vcol[i] = (c - vrow[i] * CPR) * 8;
   }
-  // The list: of up to 64 sequences in the lanes (u0 units of sequence lane, b0 before it), else in LDS; of it
-  // this workgroup takes begin .. stop - 1 and is at ``at``.
-  const bool in_lanes = n_seq <= 64;
-  int* table = reinterpret_cast<int*>(lds + table_at);
-  int b0 = 0, u0 = 0, begin = 0, stop = 1, at = 0, split = blockIdx.x / (n_seq * Hkv);
-  bool listed = false;
-
-  // The pair that holds place ``at`` and the part of its keys that lies in the share. The walk: the kept first
-  // keys left of the window, then the window; k_begin, k_end and the keys of a turn are indices of the walk,
-  // key_at gives the position.
-  int end, head0, row, n_kept, shift, k_begin, k_end, turns;
-  bool whole;
-  const int32_t* bt;
-  const char *k_head, *v_head;
-  auto key_at = [&](int kw) { return (KEPT && kw < n_kept) ? kw : kw + shift; };
-  Frag8 qf[NDT];
-  auto enter = [&]() {
-    // (of the last sequence with keys that begins at or before it)
-    int seq = 0, seq_before = 0, units = 1;
-    if (!FLAT || !listed) {
-      seq = blockIdx.x % n_seq;
-    } else if (in_lanes) {
-      seq = 63 - __clzll((long long)__ballot(u0 > 0 && b0 * Hkv <= at));
-      seq_before = __builtin_amdgcn_readlane(b0, seq) * Hkv;
-      units = __builtin_amdgcn_readlane(u0, seq);
-    } else {
-      for (int s0 = 0; s0 < n_seq; s0 += 64) {
-        const int s = s0 + lane;
-        const unsigned long long has = __ballot(s < n_seq && table[n_seq + s] > 0 && table[s] * Hkv <= at);
-        if (has) seq = s0 + 63 - __clzll((long long)has);
+  int seq = blockIdx.x % n_seq, kvh = blockIdx.x / n_seq % Hkv, split = blockIdx.x / (n_seq * Hkv);
+  if (ORDERED) {
+    const int c = lane < n_seq ? ctx_len[lane] : 0, keys = c > 0 ? walk_of(ex, c) : 0;
+    const unsigned long long some = __ballot(keys > 0);
+    const int one = some ? __builtin_amdgcn_readlane(keys, __ffsll(some) - 1) : 0;
+    if (__any(keys > DECODE_ORDER_KEYS * num_splits) && __any(keys > 0 && abs(keys - one) > one / 4)) {
+      // unit u: the workgroups of a sequence's split (one a kv head); turn: the units that all compute units take
+      const int u = blockIdx.x / Hkv, turn = max(1, cus / Hkv), first = u / turn * turn;
+      const int at = u / turn % 2 ? first + min(turn, n_seq * num_splits - first) - 1 - (u - first) : u;
+      kvh = blockIdx.x - u * Hkv;
+      split = at % num_splits;
+      int place = 0;                                      // of sequence ``lane``, the longest first
+      for (int s = 0; s < n_seq; ++s) {
+        const int other = __builtin_amdgcn_readlane(keys, s);
+        place += (other > keys || (other == keys && s < lane)) ? 1 : 0;
       }
-      seq = __builtin_amdgcn_readfirstlane(seq);
-      seq_before = __builtin_amdgcn_readfirstlane(table[seq]) * Hkv;
-      units = __builtin_amdgcn_readfirstlane(table[n_seq + seq]);
+      seq = __ffsll((unsigned long long)__ballot(lane < n_seq && place == at / num_splits)) - 1;
     }
-    const int kvh = FLAT && listed ? (at - seq_before) / units : blockIdx.x / n_seq % Hkv;
-    head0 = kvh * G;
-    row = q_start[seq];
-    const int ctx = ctx_len[seq], k_lo = first_seen(ex, ctx - 1);
-    n_kept = KEPT ? min(max(ex.keep_first, 0), k_lo) : 0;
-    shift = k_lo - n_kept;
-    if (FLAT && listed) {
-      const int pair0 = seq_before + kvh * units;
-      end = min(stop, pair0 + units);
-      whole = at == pair0 && end == pair0 + units;
-      k_begin = (at - pair0) * UNIT;
-      k_end = min(ctx - shift, (end - pair0) * UNIT);
-    } else {
-      const int per = keys_a_split(ctx - shift, num_splits, TILE);
-      end = stop;
-      whole = per >= ctx - shift;
-      k_begin = split * per;
-      k_end = min(ctx - shift, k_begin + per);
-    }
-    turns = (k_end - k_begin + TILE - 1) / TILE;
-    bt = block_table + (size_t)seq * bt_stride;
-    k_head = reinterpret_cast<const char*>(k_cache) + (size_t)kvh * page_size * D * 2;
-    v_head = reinterpret_cast<const char*>(v_cache) + (size_t)kvh * page_size * D * 2;
+  }
+  const int head0 = kvh * G;
+  const int row = q_start[seq];
+  const int ctx = ctx_len[seq];
+  const int k_lo = first_seen(ex, ctx - 1);
+  // the walk: the kept first keys left of the window, then the window; k_begin, k_end and the
+  // keys of a turn are indices of the walk, key_at gives the position
+  const int n_kept = KEPT ? min(max(ex.keep_first, 0), k_lo) : 0;
+  const int shift = k_lo - n_kept;
+  const int span = ctx - shift;
+  const int per = keys_a_split(span, num_splits, TILE);
+  const int k_begin = split * per;
+  const int k_end = min(span, k_begin + per);
+  if (split > 0 && k_begin >= k_end) return;              // (the first split answers for a row without keys)
+  const int turns = (k_end - k_begin + TILE - 1) / TILE;
+  auto key_at = [&](int kw) { return (KEPT && kw < n_kept) ? kw : kw + shift; };
+  const int32_t* bt = block_table + (size_t)seq * bt_stride;
+  const char* k_head = reinterpret_cast<const char*>(k_cache) + (size_t)kvh * page_size * D * 2;
+  const char* v_head = reinterpret_cast<const char*>(v_cache) + (size_t)kvh * page_size * D * 2;
+
+  Frag8 qf[NDT];
 #pragma unroll
-    for (int kk = 0; kk < NDT; ++kk) {
-      qf[kk].u = make_uint4(0, 0, 0, 0);
-      if (ln < G)
-        qf[kk].u = *reinterpret_cast<const uint4*>(q + (size_t)row * q_stride +
-                                                   (size_t)(head0 + ln) * D + 32 * kk + 8 * lg);
-    }
-  };
+  for (int kk = 0; kk < NDT; ++kk) {
+    qf[kk].u = make_uint4(0, 0, 0, 0);
+    if (ln < G)
+      qf[kk].u = *reinterpret_cast<const uint4*>(q + (size_t)row * q_stride +
+                                                 (size_t)(head0 + ln) * D + 32 * kk + 8 * lg);
+  }
   f32x4_t o[NT];
-  float m_run, l_part;
+#pragma unroll
+  for (int t = 0; t < NT; ++t) o[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  float m_run = -INFINITY, l_part = 0.f;
 
   int pk[UNR], pv[UNR][VCH];            // pages of the key row and of the value chunks' rows
   uint4 vg[UNR][VCH];                   // values on their way to LDS
@@ -952,47 +881,9 @@ attn_decode_mfma_kernel(bf16_t* __restrict__ out, long out_stride, const bf16_t*
   };
 
   Frag8 kfa[UNR][NDT], kfb[UNR][NDT];
-  enter();                                               // of equal parts; the contexts may say otherwise
   load_pages(0);
-  if (FLAT && flat_possible<UNIT, D>(ex, ctx_len, n_seq, num_splits)) {
-    const FlatList l = flat_list<UNIT>(ex, ctx_len, n_seq, in_lanes ? nullptr : table, lane);
-    const int share = flat_share<UNIT, D>(l, Hkv, groups, num_splits);
-    listed = share > 0;
-    if (blockIdx.x == 0 && tid == 0) note[0] = share;    // (what the merge needs to know)
-    if (listed) {
-      if (in_lanes) {
-        b0 = l.before;
-        u0 = l.units;
-        if (blockIdx.x == 0 && tid < n_seq) {
-          note[1 + tid] = b0;
-          note[1 + n_seq + tid] = u0;
-        }
-      } else {
-        __syncthreads();
-        if (blockIdx.x == 0)
-          for (int i = tid; i < 2 * n_seq; i += 64 * WAVES) note[1 + i] = table[i];
-      }
-      // rows without keys (they pad a step) get zeros, from the workgroups in turn
-      for (int s = blockIdx.x; s < n_seq; s += gridDim.x)
-        if ((in_lanes ? __builtin_amdgcn_readlane(u0, s) : table[n_seq + s]) == 0)
-          for (int j = tid; j < Hq * D; j += 64 * WAVES) out[(size_t)q_start[s] * out_stride + j] = 0;
-      split = 0;
-      at = begin = blockIdx.x * share;
-      stop = min(l.total * Hkv, begin + share);
-      if (at >= stop) return;
-      enter();
-      load_pages(0);
-    }
-  }
-  // (the first split answers for a row without keys)
-  if (split >= num_splits || (split > 0 && k_begin >= k_end)) return;
   issue_loads(0, kfa);
   load_pages(1);
- for (;;) {
-#pragma unroll
-  for (int t = 0; t < NT; ++t) o[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  m_run = -INFINITY;
-  l_part = 0.f;
   for (int turn = 0; turn < turns; turn += 2) {
     step(turn, kfa, kfb);
     if (turn + 1 < turns) step(turn + 1, kfb, kfa);
@@ -1000,17 +891,6 @@ attn_decode_mfma_kernel(bf16_t* __restrict__ out, long out_stride, const bf16_t*
   float l = l_part + __shfl_xor(l_part, 16, 64);
   l += __shfl_xor(l, 32, 64);
 
-  // this pair's results go on; the first keys and values of the next one are on their way meanwhile
-  const bool done = whole;
-  const int done_head0 = head0, done_row = row;
-  const size_t place = (size_t)blockIdx.x * 2 + (at == begin ? 0 : 1);
-  at = end;
-  if (FLAT && at < stop) {
-    enter();
-    load_pages(0);
-    issue_loads(0, kfa);
-    load_pages(1);
-  }
   // merge the waves: [wave][head][D] accumulators, [wave][head][2] (max, denominator);
   // the region takes the place of the value tiles, which every wave has left by now
   __syncthreads();
@@ -1036,8 +916,8 @@ attn_decode_mfma_kernel(bf16_t* __restrict__ out, long out_stride, const bf16_t*
       ll += w_ml[(w * 16 + h) * 2 + 1] * f;
       a += w_acc[(w * 16 + h) * D + d] * f;
     }
-    const int head = done_head0 + h;
-    if (done) {
+    const int head = head0 + h;
+    if (per >= span) {                     // the only split
       if (ex.sink) {                       // one more term of the denominator: exp(sink)
         const float sk = ex.sink[head] * 1.4426950408889634f;
         const float mx = fmaxf(mn, sk);
@@ -1045,177 +925,65 @@ attn_decode_mfma_kernel(bf16_t* __restrict__ out, long out_stride, const bf16_t*
         ll = ll * f + __builtin_amdgcn_exp2f(sk - mx);
         a *= f;
       }
-      out[(size_t)done_row * out_stride + (size_t)head * D + d] =
-          float_to_bf16(ll > 0.f ? a / ll * head_gate(ex, done_row, head) : 0.f);
+      out[(size_t)row * out_stride + (size_t)head * D + d] =
+          float_to_bf16(ll > 0.f ? a / ll * head_gate(ex, row, head) : 0.f);
     } else {
-      const size_t p = FLAT && listed ? place * G + h
-                                      : ((size_t)(blockIdx.x % n_seq) * Hq + head) * num_splits + split;
-      parts[p * D + d] = a;
+      const size_t p = ((size_t)seq * Hq + head) * num_splits + split;
+      part_acc[p * D + d] = a;
       // the merge works with natural exponents
       if (d == 0) { part_ml[p * 2] = mn * 0.6931471805599453f; part_ml[p * 2 + 1] = ll; }
     }
   }
-  if (!FLAT || at >= stop) break;
-  __syncthreads();                         // the region is read before the next pair's values come
- }
 }
 
-// One wave a (sequence, head) that several workgroups answered for: lanes take the parts' (max, denominator) side
-// by side, then the head dimension, with the parts' weights in LDS.
-template <int KEYS, int D>
-__global__ void __launch_bounds__(64)
-attn_decode_merge_flat_kernel(bf16_t* __restrict__ out, long out_stride, const int32_t* __restrict__ q_start,
-                              const int32_t* __restrict__ ctx_len, const float* __restrict__ parts,
-                              const float* __restrict__ part_ml, const int* __restrict__ note, int n_seq, int Hq, int Hkv,
-                              int num_splits, AttnExtras ex) {
-  constexpr int AHEAD = 16, J = (D + 63) / 64;
-  __shared__ float wgt[1024];
-  const int seq = blockIdx.x, head = blockIdx.y, lane = threadIdx.x;
-  const int G = Hq / Hkv, kvh = head / G, g = head - kvh * G;
-  const int row = q_start[seq], ctx = ctx_len[seq];
-  int share = 0, before = 0, units = 0;
-  if (flat_possible<KEYS, D>(ex, ctx_len, n_seq, num_splits)) {
-    share = note[0];
-    before = note[1 + seq];
-    units = note[1 + n_seq + seq];         // (of shares only)
-  }
-  // part s is part first + s * step, but for the first one of a pair that begins inside its workgroup's share
-  size_t first, step = 1, first_part;
-  int n;
-  if (share > 0) {
-    const int a0 = before * Hkv + kvh * units, w0 = a0 / share;
-    n = units ? (a0 + units - 1) / share - w0 + 1 : 1;
-    first = (size_t)w0 * 2 * G + g;
-    step = 2 * G;
-    first_part = first + (a0 == w0 * share ? 0 : G);
-  } else {
-    const int span = ctx > 0 ? walk_of(ex, ctx) : 0, per = keys_a_split(span, num_splits, KEYS * 4);
-    n = (span + per - 1) / per;
-    first = first_part = ((size_t)seq * Hq + head) * num_splits;
-  }
-  if (n <= 1) return;
-  auto part = [&](int s) { return s == 0 ? first_part : first + s * step; };
-  float ahead[J][AHEAD];
-#pragma unroll
-  for (int j = 0; j < J; ++j)
-#pragma unroll
-    for (int s = 0; s < AHEAD; ++s) ahead[j][s] = s < n && lane + 64 * j < D ? parts[part(s) * D + lane + 64 * j] : 0.f;
-  const float sk = ex.sink ? ex.sink[head] : -INFINITY;      // the denominator's term without a key
-  float mn = sk;
-  for (int s = lane; s < n; s += 64) mn = fmaxf(mn, part_ml[part(s) * 2]);
-  mn = wave_max(mn);
-  const float ms = mn == -INFINITY ? 0.f : mn;
-  float ll = 0.f;
-  for (int s = lane; s < n; s += 64) {
-    const float w = expf(part_ml[part(s) * 2] - ms);
-    wgt[s] = w;
-    ll += part_ml[part(s) * 2 + 1] * w;
-  }
-  ll = wave_sum(ll);
-  if (ex.sink) ll += expf(sk - ms);
-  __syncthreads();
-  const float inv = ll > 0.f ? head_gate(ex, row, head) / ll : 0.f;
-#pragma unroll
-  for (int j = 0; j < J; ++j) {
-    const int d = lane + 64 * j;
-    if (d >= D) continue;
-    float a = 0.f;
-#pragma unroll
-    for (int s = 0; s < AHEAD; ++s)
-      if (s < n) a = fmaf(ahead[j][s], wgt[s], a);
-#pragma unroll 8
-    for (int s = AHEAD; s < n; ++s) a = fmaf(parts[part(s) * D + d], wgt[s], a);
-    out[(size_t)row * out_stride + (size_t)head * D + d] = float_to_bf16(a * inv);
-  }
+static bool decode_ordered(int n_seq, int num_splits) {
+  return num_splits > 1 && num_splits <= 4 && n_seq > 8 && n_seq <= DECODE_ORDER_SEQS;
 }
 
-// Shares: as many workgroups as the chip holds at once.
-static int flat_groups(int D) {
-  const int n = decode_held(D) * compute_units();
-  return n < 1024 ? n : 1024;
-}
-
-// Where the shares are thought of at all (us in the better of both forms against equal parts alone): up to 8
-// sequences, which take many splits each, looking at all contexts costs more than it gives; with one
-// workgroup a pair the chip is full, and shares of 64 sequences, most of which cross pairs, gain 4 % where contexts
-// differ and lose 10 % where they do not.
-static bool decode_flat(int n_seq, int num_splits) { return num_splits > 1 && n_seq > 8; }
-
-// parts of the workspace
-static long decode_parts(int n_seq, int Hq, int Hkv, int D, int num_splits) {
-  if (num_splits <= 1) return 0;
-  const long equal = (long)n_seq * Hq * num_splits, shares = (long)flat_groups(D) * 2 * (Hq / Hkv);
-  return decode_flat(n_seq, num_splits) && shares > equal ? shares : equal;
-}
-
-template <int NDT, int UNR, bool FLAT, bool KEPT, bool CAP, typename... Args>
-static int launch_decode_form(dim3 grid, size_t lds, hipStream_t st, Args... args) {
-  if (lds > 64 * 1024 &&
-      hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_decode_mfma_kernel<NDT, UNR, FLAT, KEPT, CAP>),
-                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) {
-    (void)hipGetLastError();
-    return PTL_ERR_LAUNCH;
-  }
-  attn_decode_mfma_kernel<NDT, UNR, FLAT, KEPT, CAP><<<grid, 256, lds, st>>>(args...);
-  return hipGetLastError() == hipSuccess ? PTL_OK : PTL_ERR_LAUNCH;
-}
-
-template <int NDT, int UNR, bool FLAT>
+template <int NDT, int UNR, bool ORDERED>
 static int launch_decode_mfma(void* out, long out_stride, const void* q, long q_stride,
                               const void* k_cache, const void* v_cache, const int32_t* q_start,
                               const int32_t* ctx_len, const int32_t* block_table, int bt_stride,
                               float* parts, int n_seq, int Hq, int Hkv, int page_size, const AttnExtras& ex,
                               float scale, int num_splits, hipStream_t stream) {
-  constexpr int D = 32 * NDT, WAVES = 4;
-  const int groups = flat_groups(D);
-  const long equal = (long)n_seq * Hkv * num_splits;
-  if (equal > 0x7fffffff) return PTL_ERR_ARG;
-  const long n_parts = decode_parts(n_seq, Hq, Hkv, D, num_splits);
-  float* part_ml = parts ? parts + n_parts * D : nullptr;
-  int* note = parts ? reinterpret_cast<int*>(part_ml + n_parts * 2) : nullptr;
+  constexpr int D = 32 * NDT, WAVES = 4, TILE = 16 * UNR * WAVES;
+  const long groups = (long)n_seq * Hkv * num_splits;
+  if (groups > 0x7fffffff) return PTL_ERR_ARG;
+  float* part_ml = parts ? parts + (long)n_seq * Hq * num_splits * D : nullptr;
   int page_shift = 0;
   while ((1 << page_shift) < page_size) ++page_shift;
   const size_t lds_merge = (size_t)WAVES * 16 * (D + 2) * sizeof(float);
   const size_t lds_values = (size_t)WAVES * UNR * 16 * (D + 16) * sizeof(bf16_t);
-  const size_t used = lds_merge > lds_values ? lds_merge : lds_values;
-  size_t lds = used;
-  if (FLAT) {
-    // the list's table, and more of a compute unit's 160 KB than would let one workgroup too many in
-    const size_t one = 160 * 1024 / (decode_held(D) + 1) + 1024;
-    if (n_seq > 64) lds += (size_t)2 * n_seq * sizeof(int);
-    if (lds < one) lds = one;
-  }
+  const size_t lds = lds_merge > lds_values ? lds_merge : lds_values;
   const bool kept = ex.window > 0 && ex.keep_first > 0, cap = ex.softcap > 0.f;
   const float log2e = 1.4426950408889634f;
   const float scale_log2 = (cap ? ex.softcap : scale) * log2e, cap_in = cap ? 2.0f * log2e * scale / ex.softcap : 0.f;
 #define GO(KEPT, CAP)                                                                                              \
-  launch_decode_form<NDT, UNR, FLAT, KEPT, CAP>(                                                                   \
-      dim3((unsigned)(FLAT && groups > equal ? groups : equal)), lds, stream, (bf16_t*)out, out_stride,            \
-      (const bf16_t*)q, q_stride, (const bf16_t*)k_cache, (const bf16_t*)v_cache, q_start, ctx_len, block_table,   \
-      bt_stride, parts, part_ml, n_seq, Hq, Hkv, page_size, page_shift, ex, scale_log2, cap_in, num_splits, groups, \
-      (int)(used / sizeof(float)), note)
-  const int rc = kept ? (cap ? GO(true, true) : GO(true, false)) : (cap ? GO(false, true) : GO(false, false));
+  attn_decode_mfma_kernel<NDT, UNR, ORDERED, KEPT, CAP><<<(unsigned)groups, 64 * WAVES, lds, stream>>>(            \
+      (bf16_t*)out, out_stride, (const bf16_t*)q, q_stride, (const bf16_t*)k_cache, (const bf16_t*)v_cache, q_start, \
+      ctx_len, block_table, bt_stride, parts, part_ml, n_seq, Hq, Hkv, page_size, page_shift, ex, scale_log2, cap_in, \
+      num_splits, compute_units())
+  if (kept) {
+    if (cap) GO(true, true); else GO(true, false);
+  } else {
+    if (cap) GO(false, true); else GO(false, false);
+  }
 #undef GO
-  if (rc != PTL_OK) return rc;
-  if (FLAT)
-    attn_decode_merge_flat_kernel<16 * UNR, D><<<dim3(n_seq, Hq), 64, 0, stream>>>(
-        (bf16_t*)out, out_stride, q_start, ctx_len, parts, part_ml, note, n_seq, Hq, Hkv, num_splits, ex);
-  else if (num_splits > 1)
+  if (hipGetLastError() != hipSuccess) return PTL_ERR_LAUNCH;
+  if (num_splits > 1)
     attn_decode_merge_kernel<bf16_t><<<dim3(n_seq, Hq), 64, 0, stream>>>(
-        (bf16_t*)out, out_stride, q_start, parts, part_ml, Hq, D, num_splits, ex, ctx_len, 16 * UNR * WAVES);
+        (bf16_t*)out, out_stride, q_start, parts, part_ml, Hq, D, num_splits, ex, ctx_len, TILE);
   return ptl_launch_status();
 }
 
 // floats of workspace that ptl_attention_decode_mfma wants
 extern "C" long ptl_attention_decode_mfma_workspace(int n_seq, int Hq, int Hkv, int D, int num_splits) {
-  if (n_seq <= 0 || Hkv <= 0 || Hq % Hkv || num_splits < 1) return 0;
-  if (num_splits == 1) return 0;
-  return decode_parts(n_seq, Hq, Hkv, D, num_splits) * (D + 2) + (decode_flat(n_seq, num_splits) ? 1 + 2L * n_seq : 0);
+  if (n_seq <= 0 || Hkv <= 0 || Hq % Hkv || num_splits <= 1) return 0;
+  return (long)n_seq * Hq * num_splits * (D + 2);
 }
 
-// num_splits: the most workgroups that a sequence and kv head are worth, on average; parts:
-// ptl_attention_decode_mfma_workspace floats. unroll: 16-key tiles a wave takes per turn, 1 or 2 (0: the kernel's
-// choice).
+// parts: ptl_attention_decode_mfma_workspace floats. unroll: 16-key tiles a wave takes per turn, 1 or 2 (0: the
+// kernel's choice).
 extern "C" int ptl_attention_decode_mfma(void* out, long out_stride, const void* q, long q_stride,
                                          const void* k_cache, const void* v_cache,
                                          const int32_t* q_start, const int32_t* ctx_len,
@@ -1232,25 +1000,14 @@ extern "C" int ptl_attention_decode_mfma(void* out, long out_stride, const void*
       num_splits > 1024 || (num_splits > 1 && !parts) || unroll < 0 || unroll > 2 || !extras_ok(ex))
     return PTL_ERR_ARG;
   if (unroll == 0) unroll = 2;
-  const bool flat = decode_flat(n_seq, num_splits);
-  // (one launch after the other, one workspace)
-  for (; flat && n_seq > FLAT_MAX_SEQS + 8; n_seq -= FLAT_MAX_SEQS) {
-    const int rc = ptl_attention_decode_mfma(out, out_stride, q, q_stride, k_cache, v_cache, q_start, ctx_len,
-                                             block_table, bt_stride, parts, FLAT_MAX_SEQS, Hq, Hkv, D, page_size, window,
-                                             keep_first, chunk, sink, gate, gate_stride, softcap, scale, num_splits,
-                                             unroll, stream);
-    if (rc != PTL_OK) return rc;
-    q_start += FLAT_MAX_SEQS;
-    ctx_len += FLAT_MAX_SEQS;
-    block_table += (size_t)FLAT_MAX_SEQS * bt_stride;
-  }
 #define GO(N, U)                                                                                                \
-  (flat ? launch_decode_mfma<N, U, true>(out, out_stride, q, q_stride, k_cache, v_cache, q_start, ctx_len,      \
+  (decode_ordered(n_seq, num_splits)                                                                            \
+       ? launch_decode_mfma<N, U, true>(out, out_stride, q, q_stride, k_cache, v_cache, q_start, ctx_len,       \
+                                        block_table, bt_stride, parts, n_seq, Hq, Hkv, page_size, ex, scale,    \
+                                        num_splits, stream)                                                     \
+       : launch_decode_mfma<N, U, false>(out, out_stride, q, q_stride, k_cache, v_cache, q_start, ctx_len,      \
                                          block_table, bt_stride, parts, n_seq, Hq, Hkv, page_size, ex, scale,   \
-                                         num_splits, stream)                                                    \
-        : launch_decode_mfma<N, U, false>(out, out_stride, q, q_stride, k_cache, v_cache, q_start, ctx_len,     \
-                                          block_table, bt_stride, parts, n_seq, Hq, Hkv, page_size, ex, scale,  \
-                                          num_splits, stream))
+                                         num_splits, stream))
   if (unroll == 1) {
     switch (D / 32) {
       case 1: return GO(1, 1);

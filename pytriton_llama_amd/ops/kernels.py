@@ -818,9 +818,8 @@ def attention_decode(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor,
     which brings exactly one query token (see csrc/attention.hip). Head sizes in
     steps of 16 up to 256, float32 or bfloat16. ``matrix_cores``: the MFMA
     variant (bfloat16, head sizes 32/64/96/128, at most 16 heads a kv head, a page
-    size that is a power of two), which deals the keys of all sequences out in equal
-    shares; ``num_splits`` is there the most workgroups that a sequence and kv head are worth;
-    ``unroll``: its 16-key tiles per wave and turn (1 or 2; 0 leaves the choice to the kernel)."""
+    size that is a power of two); ``unroll``: its 16-key tiles per wave and turn
+    (1 or 2; 0 leaves the choice to the kernel)."""
     T, Hq, Hkv, D, page_size = _attention_common(out, q, k_cache, v_cache, q_start, ctx_len,
                                                  block_table, "attention_decode")
     if D % 16 or D > 256:

@@ -852,14 +852,14 @@ def test_attention_decode_mfma(ops, splits, case, unroll):
 
 @pytest.mark.parametrize("unroll", [1, 2])
 @pytest.mark.parametrize("case", [
-    # contexts that differ so much that the keys are dealt out in equal shares: pairs that begin and end inside
-    # shares and span several, the list in lanes (up to 64 sequences) and in LDS, wide and narrow heads, a window
+    # contexts that differ much: workgroups by length, or, beyond 64 sequences, as they come; wide and narrow heads, a
+    # window
     dict(seq_lens=[3000] + [17 * i + 5 for i in range(19)], Hq=8, Hkv=2, D=64, P=16, splits=4),
     dict(seq_lens=[7] * 5 + [2500, 1, 1900, 33], Hq=6, Hkv=3, D=128, P=16, splits=3),
     dict(seq_lens=[40 + 3 * i for i in range(69)] + [4100], Hq=4, Hkv=1, D=32, P=8, splits=2),
     dict(seq_lens=[1] * 64 + [3500], Hq=2, Hkv=2, D=96, P=16, splits=2),
     dict(seq_lens=[4000] + [300] * 9, Hq=4, Hkv=2, D=64, P=16, window=3000, splits=2),
-    # and one key short of and past what the shares need: 16 sequences, two splits, 2 * (4 + 12) units of 32 keys
+    # and the longest on both sides of 512 keys a split
     dict(seq_lens=[1024] + [5] * 15, Hq=4, Hkv=1, D=64, P=16, splits=2),
     dict(seq_lens=[1025] + [5] * 15, Hq=4, Hkv=1, D=64, P=16, splits=2),
 ])
@@ -870,7 +870,7 @@ def test_attention_decode_mfma_shares(ops, case, unroll):
 
 @pytest.mark.parametrize("n", [12, 80])
 def test_attention_decode_mfma_shares_beside_empty_rows(ops, n):
-    """Rows without keys (padding of a recorded step) between sequences whose keys are dealt out in shares: zeros
+    """Rows without keys (padding of a recorded step) between sequences of very different lengths: zeros
     there, and the other rows as without them."""
     D, P = 64, 16
     torch.manual_seed(n)
@@ -893,6 +893,64 @@ def test_attention_decode_mfma_shares_beside_empty_rows(ops, n):
     for r, c in real:
         torch.testing.assert_close(out[r], run([r])[0], atol=2e-2, rtol=2e-2)
     assert all(bool((out[r] == 0).all()) for r in range(n) if ctx[r] == 0)
+
+
+def _masked_attention(q, k, v, pos, scale, window=0, keep_first=0, chunk=0, sink=None, gate=None, softcap=0.0):
+    """One query [Hq, D] at position pos on keys [pos + 1, Hkv, D] under the masks, in float64."""
+    Hq, G = q.shape[0], q.shape[0] // k.shape[1]
+    s = torch.einsum("hd,khd->hk", q.double(), k.double().repeat_interleave(G, 1)) * scale
+    if softcap:
+        s = softcap * torch.tanh(s / softcap)
+    at = torch.arange(pos + 1)
+    first = max(0, pos + 1 - window) if window else pos // chunk * chunk if chunk else 0
+    s[:, ~((at >= first) | (at < keep_first))] = -math.inf
+    if sink is not None:
+        s = torch.cat([s, sink.double()[:, None]], 1)
+    p = torch.softmax(s, 1)[:, :pos + 1]
+    o = torch.einsum("hk,khd->hd", p, v.double().repeat_interleave(G, 1))
+    return o if gate is None else o * torch.sigmoid(gate.double())[:, None]
+
+
+@pytest.mark.parametrize("masks", ["none", "sink_gate", "softcap", "kept", "kept_softcap_sink_gate", "chunk_sink"])
+@pytest.mark.parametrize("n,splits,Hq,Hkv,D", [(9, 2, 4, 2, 64), (33, 4, 3, 1, 128), (64, 2, 8, 8, 32), (65, 3, 4, 2, 96)])
+def test_attention_decode_mfma_ragged_batch_gives_what_each_gives_alone(ops, n, splits, Hq, Hkv, D, masks):
+    """Workgroups in the order of very different lengths (up to 64 sequences), rows without keys among them, under
+    every mask: the bits of each sequence alone, and the plain result at the tolerance of the other cases."""
+    P, pages = 16, 300
+    g = torch.Generator().manual_seed(n)
+    ctx = [3 * i * i % 700 + 1 for i in range(n)]
+    ctx[n // 2], ctx[1], ctx[n - 1], ctx[3] = 512 * splits + 300, 512 * splits + 7, 1000, 0
+    kc, vc = (torch.randn(pages, Hkv, P, D, generator=g).to(torch.bfloat16) for _ in range(2))
+    bt = torch.stack([torch.randperm(pages, generator=g) for _ in range(n)]).to(torch.int32)
+    q = torch.randn(n, Hq, D, generator=g).to(torch.bfloat16)
+    sink, gate = torch.randn(Hq, generator=g), torch.randn(n, Hq, generator=g)
+    kw = {}
+    if "kept" in masks:
+        kw.update(window=512 * splits + 100, keep_first=21)
+    if "chunk" in masks:
+        kw.update(chunk=512 * splits + 200)
+    if "softcap" in masks:
+        kw.update(softcap=2.0)
+    dev = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")
+    kd, vd, scale = kc.cuda(), vc.cuda(), D ** -0.5
+
+    def run(rows):
+        out = torch.full((len(rows), Hq, D), 9.0, dtype=torch.bfloat16, device="cuda")
+        more = dict(kw, **({"sink": sink.cuda()} if "sink" in masks else {}),
+                    **({"gate": gate[rows].cuda()} if "gate" in masks else {}))
+        ops.attention_decode(out, q[rows].cuda(), kd, vd, dev(list(range(len(rows) + 1))), dev([ctx[r] for r in rows]),
+                             bt[rows].cuda(), len(rows), scale, num_splits=splits, matrix_cores=True, **more)
+        return out
+    out = run(list(range(n)))
+    for r in range(n):
+        assert torch.equal(out[r], run([r])[0]), f"sequence {r}"
+    assert bool((out[3] == 0).all())
+    for r in (0, 1, n // 2, n - 1):
+        c = ctx[r]
+        rows = [t[bt[r].long()].transpose(1, 2).reshape(pages * P, Hkv, D)[:c] for t in (kc, vc)]
+        want = _masked_attention(q[r], *rows, c - 1, scale, sink=sink if "sink" in masks else None,
+                                 gate=gate[r] if "gate" in masks else None, **kw)
+        torch.testing.assert_close(out[r].float().cpu(), want.float(), **tol(torch.bfloat16))
 
 
 @pytest.mark.parametrize("D", [16, 32, 48, 64, 80, 128])
@@ -984,6 +1042,37 @@ def test_attention_prefill_mfma_sides(ops, D, Hq, window):
     case = dict(seq_lens=[1, 64, 65, 129, 200, 321], q_lens=[1, 64, 65, 66, 70, 65], Hq=Hq, Hkv=1, D=D, P=16)
     for groups in (0, 3):
         _attention_case(ops, torch.bfloat16, kernel="mfma", window=window, groups=groups, **case)
+
+
+@pytest.mark.parametrize("rows,groups", [(300, 0), (300, 2), (257, 0)])
+@pytest.mark.parametrize("masks", ["kept", "kept_sink_gate", "softcap_sink_gate", "chunk_sink"])
+def test_attention_prefill_mfma_sides_with_masks(ops, masks, rows, groups):
+    """Two groups of waves on blocks of four and more key tiles whose walk is two stretches (kept first keys and a
+    window), with sinks and gates, and under capped scores and chunks."""
+    Hq, Hkv, D, P, total = 2, 1, 64, 16, 900
+    kc, vc, bt, dk, dv = _paged_setup([total], [rows], Hkv, D, P, torch.bfloat16, 5)
+    g = torch.Generator().manual_seed(rows)
+    q = torch.randn(rows, Hq, D, generator=g).to(torch.bfloat16)
+    sink, gate = torch.randn(Hq, generator=g), torch.randn(rows, Hq, generator=g)
+    kw = {}
+    if "kept" in masks:
+        kw.update(window=310, keep_first=70)
+    if "chunk" in masks:
+        kw.update(chunk=400)
+    if "softcap" in masks:
+        kw.update(softcap=2.0)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")
+    off = list(range(0, rows, 64))[::-1]
+    out = torch.zeros(rows, Hq, D, dtype=torch.bfloat16, device="cuda")
+    ops.attention_prefill_mfma(out, q.cuda(), kc.cuda(), vc.cuda(), i32([0, rows]), i32([total]), bt.cuda(),
+                               i32([0] * len(off)), i32(off), D ** -0.5, groups=groups,
+                               **kw, **({"sink": sink.cuda()} if "sink" in masks else {}),
+                               **({"gate": gate.cuda()} if "gate" in masks else {}))
+    for r in (0, 1, 63, 64, 100, 200, rows - 1):
+        pos = total - rows + r
+        want = _masked_attention(q[r], dk[0][:pos + 1], dv[0][:pos + 1], pos, D ** -0.5, sink=sink if "sink" in masks else None,
+                                 gate=gate[r] if "gate" in masks else None, **kw)
+        torch.testing.assert_close(out[r].float().cpu(), want.float(), **tol(torch.bfloat16))
 
 
 @pytest.mark.parametrize("D", [64, 128])
