@@ -917,7 +917,7 @@ attn_decode_mfma_kernel(bf16_t* __restrict__ out, long out_stride, const bf16_t*
       a += w_acc[(w * 16 + h) * D + d] * f;
     }
     const int head = head0 + h;
-    if (per >= span) {                     // the only split
+    if (num_splits == 1) {
       if (ex.sink) {                       // one more term of the denominator: exp(sink)
         const float sk = ex.sink[head] * 1.4426950408889634f;
         const float mx = fmaxf(mn, sk);
@@ -927,6 +927,13 @@ attn_decode_mfma_kernel(bf16_t* __restrict__ out, long out_stride, const bf16_t*
       }
       out[(size_t)row * out_stride + (size_t)head * D + d] =
           float_to_bf16(ll > 0.f ? a / ll * head_gate(ex, row, head) : 0.f);
+    } else if (per >= span) {              // the only split with keys: what the second kernel makes of it, bit for bit
+      const float m = mn * 0.6931471805599453f, sk = ex.sink ? ex.sink[head] : -INFINITY, mx = fmaxf(m, sk);
+      const float w = expf(m - (mx == -INFINITY ? 0.f : mx));
+      ll *= w;
+      if (ex.sink) ll += expf(sk - mx);
+      out[(size_t)row * out_stride + (size_t)head * D + d] =
+          float_to_bf16(a * w * (ll > 0.f ? head_gate(ex, row, head) / ll : 0.f));
     } else {
       const size_t p = ((size_t)seq * Hq + head) * num_splits + split;
       part_acc[p * D + d] = a;
