@@ -311,14 +311,16 @@ static int attention_f32(float* out, long out_stride, const float* q, long q_str
 }
 
 // Where a decoded token takes this kernel (sizes in steps of 16 come here), one map and at most 16 heads a kv head:
-// key and value sizes from 32 to 64. Against the vector kernel (one MI355X, 1 to 40 sequences of 60 to 2,000 keys, 1
-// to 16 heads a kv head): 1.25 to 1.67 times as fast in the mean of a shape, at worst level but for one head a kv head
-// over 32 kv heads and 2,000 keys (119 against 123 us). Above 64 the buffers leave room for one workgroup a compute unit
-// (133 KB; 16 sequences of 2,000 keys, 8 x 128: 89 against 66 us; 8 x 96: 87 against 56), below 32 half of every
-// tile is padding (40 of 2,000 keys, 32 x 16: 143 against 97).
+// key and value sizes from 32 to 64 always; above 64 from 8, below 32 from 4 heads a kv head on. Against the vector kernel (one
+// MI355X, 1 to 40 sequences of 60 to 2,000 keys), us before and with this kernel: sizes 32 to 64 1.25 to 1.67 times as fast
+// in the mean of a shape, at worst level but for one head a kv head over 32 kv heads and 2,000 keys (119, 123). Above 64
+// the buffers leave room for one workgroup a compute unit (133 KB), and how much of a tile's 16 rows are heads
+// decides: 16 on one latent head of 128, 14 sequences of 222 to 1,015 keys 33, 20, 16 of 2,000 40, 19; 16 on 2 x 128 44, 34;
+// 24 on 3 x 96 57, 46; but 16 on 4 x 128 46, 58 and 8 on 8 x 128 66, 89. Below 32 half of every tile is padding: 32 on 8 x 16,
+// 16 of 2,000 24 to 36 (4 and 8 splits planned), 25 to 23; 32 on 32 x 16, 40 of 2,000 97, 143.
 static bool attn_f32_decodes(int Hq, int Hkv, int maps, int Dk, int Dv) {
-  const int size = Dk > Dv ? Dk : Dv;
-  return maps == 1 && Hq / Hkv <= 16 && Hkv <= 65535 && size >= 32 && size <= 64;
+  const int size = Dk > Dv ? Dk : Dv, heads = Hq / Hkv;
+  return maps == 1 && heads <= 16 && Hkv <= 65535 && size <= 128 && heads >= (size > 64 ? 8 : size < 32 ? 4 : 1);
 }
 
 // One token a sequence (arguments as ptl_attention_decode_kv, of attn_f32_fits and attn_f32_decodes). Splits without
@@ -331,7 +333,9 @@ static int attention_f32_decode(float* out, long out_stride, const float* q, lon
   return launch_attn_f32<1, NK, 64, true>(dim3(n_seq, Hkv, sp.num_splits), st, out, out_stride, q, q_stride, k_cache, \
                                           v_cache, q_start, ctx_len, block_table, bt_stride, (const int32_t*)nullptr, \
                                           (const int32_t*)nullptr, Hq, Hkv, 1, Dk, Dv, page_size, ex, scale, sp)
-  if (Dk <= 32 && Dv <= 32) GO(2);
-  GO(4);
+  const int size = Dk > Dv ? Dk : Dv;
+  if (size <= 32) GO(2);
+  if (size <= 64) GO(4);
+  GO(8);
 #undef GO
 }

@@ -954,10 +954,12 @@ def test_attention_decode_mfma_ragged_batch_gives_what_each_gives_alone(ops, n, 
 
 
 @pytest.mark.parametrize("D", [16, 32, 48, 64, 80, 128])
-def test_attention_decode_float32_form_by_head_size(ops, D):
-    """float32 decode attention takes the matrix-core form for sizes 32 to 64 alone; the others give the bits
-    of the vector form, which rows of odd stride always take."""
-    n, Hq, Hkv, P, ctx = 3, 6, 2, 16, [5, 300, 70]
+@pytest.mark.parametrize("heads", [3, 4, 8, 16])
+def test_attention_decode_float32_form_by_head_size(ops, D, heads):
+    """float32 decode attention takes the matrix-core form for sizes 32 to 64, for larger ones from 8 and for
+    smaller ones from 4 heads a kv head on; the others give the bits of the vector form, which rows of odd stride
+    always take."""
+    n, Hq, Hkv, P, ctx = 3, 2 * heads, 2, 16, [5, 300, 70]
     torch.manual_seed(D)
     kc, vc = (torch.randn(60, Hkv, P, D, device="cuda") for _ in range(2))
     i32 = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")
@@ -969,7 +971,7 @@ def test_attention_decode_float32_form_by_head_size(ops, D):
         ops.attention_decode(out, q, kc, vc, i32([0, 1, 2, 3]), i32(ctx), bt, n, D ** -0.5, num_splits=2)
         outs.append(out)
     torch.testing.assert_close(outs[0], outs[1], atol=1e-5, rtol=1e-5)
-    assert torch.equal(outs[0], outs[1]) == (D not in (32, 48, 64))
+    assert torch.equal(outs[0], outs[1]) == (heads < (8 if D > 64 else 4 if D < 32 else 1))
 
 
 def test_attention_decode_mfma_refuses_odd_page_size(ops):
