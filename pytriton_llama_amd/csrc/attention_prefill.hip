@@ -553,8 +553,9 @@ extern "C" int ptl_attention_prefill_mfma(void* out, long out_stride, const void
   // 24 heads of 128, 512 rows: on 1,536 keys 40.7 -> 29.5 us, on 3,072 76.5 -> 52.5, a prompt of 512
   // 17.4 -> 14.1, of 300 12.1 -> 11.3; 32 heads of 64, 300 rows 8.9 -> 8.0. Below 256 keys the larger workgroup
   // costs 0.2 to 0.8 us (64 rows on 64 keys 6.3 -> 7.1, 128 on 128 7.9 -> 8.6, 200 on 200 level), which every short
-  // prompt would pay in every layer; a short portion behind a long prefix would gain (64 rows on 320 keys 12.1 ->
-  // 11.3, on 1,088 29.9 -> 22.8), but how many keys a recorded step will have is not known at its launch.
+  // prompt would pay in every layer; a short portion behind a long prefix gains (64 rows on 320 keys 12.1 ->
+  // 11.3, on 1,088 29.9 -> 22.8). How many keys a recorded step will have is not known at its launch: callers give
+  // the rows of what is most likely a prompt of its own, and 0 where a prefix is as likely.
   if (block_rows == 64 && (longest <= 0 || longest > 256) && (long)n_groups * Hq <= compute_units())
     return prefill_same_size<1, 2>(D / 32, out, out_stride, q, q_stride, k_cache, v_cache, q_start, ctx_len,
                                    block_table, bt_stride, work_seq, work_qoff, n_work, n_groups, Hq, Hkv,

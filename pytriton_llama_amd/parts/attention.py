@@ -194,9 +194,11 @@ class PagedAttention(Part):
                 q.device, self.num_heads, D, ctx.work[PORTIONS_64][0].numel(),
                 ctx.work[PORTIONS_128][0].numel(), min(keys, window) if window else keys)
             ws, wo = ctx.work[PORTIONS_128 if rows == 128 else PORTIONS_64]
+            # (a portion alone has about as many keys as rows: it is a prompt, or the largest piece of one. What comes
+            # beside decoding requests is as often the rest of a prompt behind a long prefix)
             ops.attention_prefill_mfma(out, q, k, v, ctx.q_start, ctx.ctx_len,
                                        group.block_table, ws, wo, self.scale, window, rows, groups,
-                                       sink=self.sink, longest=max(ctx.q_lens[n_dec:]))
+                                       sink=self.sink, longest=0 if n_dec else max(ctx.q_lens))
         else:
             ws, wo = ctx.work[PORTIONS_16 if n_dec else ALL_16]
             ops.attention_generic(out, q, k, v, ctx.q_start, ctx.ctx_len,

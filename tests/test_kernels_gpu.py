@@ -1077,6 +1077,43 @@ def test_attention_prefill_mfma_sides_with_masks(ops, masks, rows, groups):
         torch.testing.assert_close(out[r].float().cpu(), want.float(), **tol(torch.bfloat16))
 
 
+@pytest.mark.parametrize("n_dec", [0, 2])
+def test_short_portion_beside_decoding_requests_takes_two_sides(ops, n_dec):
+    """PagedAttention: a portion of 70 rows behind a prefix of 900, alone (the bits of one group of waves) and beside
+    decoding requests (of two); both near the plain result."""
+    from types import SimpleNamespace
+
+    from pytriton_llama_amd.parts import attention as part
+    D, P, rows, total = 64, 16, 70, 970
+    att = part.PagedAttention(128, 2, 1, D)
+    lens, q_lens = [40] * n_dec + [total], [1] * n_dec + [rows]
+    kc, vc, bt, dk, dv = _paged_setup(lens, q_lens, 1, D, P, torch.bfloat16, 3)
+    torch.manual_seed(0)
+    q = torch.randn(n_dec + rows, 2, D).to(torch.bfloat16)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")
+    q_start = [0]
+    for n in q_lens:
+        q_start.append(q_start[-1] + n)
+    off = [64, 0]
+    lists = (i32([n_dec] * 2), i32(off))
+    ctx = SimpleNamespace(num_decode_seqs=n_dec, num_seqs=n_dec + 1, q_start=i32(q_start), ctx_len=i32(lens), q_lens=q_lens,
+                          ctx_lens=lens, work={part.PORTIONS_64: lists, part.PORTIONS_128: lists})
+    out = torch.zeros(n_dec + rows, 2, D, dtype=torch.bfloat16, device="cuda")
+    att.attend(out, q.cuda(), SimpleNamespace(k=kc.cuda(), v=vc.cuda(), page_size=P), ctx, SimpleNamespace(block_table=bt.cuda()))
+    sides = []
+    for longest in (rows, 0):
+        o = torch.zeros_like(out)
+        ops.attention_prefill_mfma(o, q.cuda(), kc.cuda(), vc.cuda(), i32(q_start), i32(lens), bt.cuda(), *lists, D ** -0.5,
+                                   longest=longest)
+        sides.append(o[n_dec:])
+    assert not torch.equal(*sides)
+    assert torch.equal(out[n_dec:], sides[1 if n_dec else 0])
+    for r in (0, 69):
+        pos = total - rows + r
+        want = _masked_attention(q[n_dec + r], dk[-1][:pos + 1], dv[-1][:pos + 1], pos, D ** -0.5)
+        torch.testing.assert_close(out[n_dec + r].float().cpu(), want.float(), **tol(torch.bfloat16))
+
+
 @pytest.mark.parametrize("D", [64, 128])
 def test_attention_prefill_mfma_short_portions_keep_one_side(ops, D):
     """Portions of up to 256 rows give the bits of one group of waves (which a launch of many heads always takes),
