@@ -225,17 +225,22 @@ def gemm_nt(x: torch.Tensor, w: torch.Tensor, out_dtype: Optional[torch.dtype] =
     y = out if out is not None else torch.empty((M, N), dtype=out_dtype, device=x.device)
     if M == 0:
         return y
-    if x.dtype == torch.float32 and _gemm_f32_fits(x, w, M, K):
-        lib = library.load("gemm_f32")
-        ldx, ldy = ctypes.c_long(x.stride(0)), ctypes.c_long(y.stride(0))
-        if M <= F32_FEW_ROWS:
-            _check(lib.ptl_gemm_f32_few(_ptr(y), _ptr(x), _ptr(w), M, N, K, ldx, ldy, _stream()), "gemm_nt")
+    if x.dtype == torch.float32:
+        # (each of these is asked for once: at a few rows the host's part of a call is most of it)
+        xp, wp, ldx = x.data_ptr(), w.data_ptr(), x.stride(0)
+        # whole 16-byte pieces of K in aligned rows of both
+        if K > 0 and (4 * K | xp | wp) % 16 == 0 and ldx >= K and (M == 1 or ldx % 4 == 0):
+            lib = library.load("gemm_f32")
+            sizes = (M, N, K, ctypes.c_long(ldx), ctypes.c_long(y.stride(0)))
+            xp, wp = ctypes.c_void_p(xp), ctypes.c_void_p(wp)
+            if M <= F32_FEW_ROWS:
+                _check(lib.ptl_gemm_f32_few(_ptr(y), xp, wp, *sizes, _stream()), "gemm_nt")
+                return y
+            lib.ptl_gemm_f32_workspace.restype = ctypes.c_long
+            floats = lib.ptl_gemm_f32_workspace(M, N, K)
+            parts = torch.empty(floats, dtype=torch.float32, device=x.device) if floats else None
+            _check(lib.ptl_gemm_f32(_ptr(y), xp, wp, *sizes, _ptr(parts), _stream()), "gemm_nt")
             return y
-        lib.ptl_gemm_f32_workspace.restype = ctypes.c_long
-        floats = lib.ptl_gemm_f32_workspace(M, N, K)
-        parts = torch.empty(floats, dtype=torch.float32, device=x.device) if floats else None
-        _check(lib.ptl_gemm_f32(_ptr(y), _ptr(x), _ptr(w), M, N, K, ldx, ldy, _ptr(parts), _stream()), "gemm_nt")
-        return y
     lib = library.load("gemm")
     _check(lib.ptl_gemm_nt(_ptr(y), _ptr(x), _ptr(w), M, N, K, ctypes.c_long(x.stride(0)),
                            ctypes.c_long(y.stride(0)), _dtype_code(x),
@@ -244,13 +249,6 @@ def gemm_nt(x: torch.Tensor, w: torch.Tensor, out_dtype: Optional[torch.dtype] =
 
 
 F32_FEW_ROWS = 16          # rows of x up to which the kernel that streams W once takes a float32 product
-
-
-def _gemm_f32_fits(x: torch.Tensor, w: torch.Tensor, M: int, K: int) -> bool:
-    """Whether the float32 matrix-core kernels take x [M, K] and w: whole 16-byte pieces of K in
-    aligned rows of both."""
-    return (K > 0 and K % 4 == 0 and x.stride(0) >= K and (M == 1 or x.stride(0) % 4 == 0)
-            and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
 
 
 SKINNY_MAX_ROWS = 64
