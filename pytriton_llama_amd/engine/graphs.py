@@ -26,7 +26,8 @@ a recorded step (q_lens, ctx_lens and the maxima) are the bucket's upper bounds.
 state of its own must stop at q_start[i + 1], not at the padded length.
 
 All graphs of a runner share one memory pool: they are replayed one at a time on one stream,
-so what a step needs while it runs is the most that any of them needs, not the sum.
+so what a step needs while it runs is the most that any of them needs, not the sum. What stays
+for good is each graph's logits, one tensor a size class ([its rows, vocabulary] in float32).
 
 Nothing in a captured step clears memory with a memset node, and the buffers a
 replay reads are written by ordinary copies before it.

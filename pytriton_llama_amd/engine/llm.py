@@ -37,8 +37,9 @@ def pages_that_fit(usable_bytes: int, bytes_per_page: int, state_bytes: int, cap
 def graph_pool_bytes(model, engine: EngineConfig) -> int:
     """Memory the recorded steps' shared pool is allowed for when the cache is sized from free
     memory: the intermediate results of the largest step that is recorded (a portion of up to
-    2,048 tokens beside max_num_seqs decoding rows) and its float32 logits. Nothing when steps
-    are not recorded."""
+    2,048 tokens beside max_num_seqs decoding rows) and its float32 logits. (The logits that the
+    graphs of further size classes keep come from what gpu_memory_fraction leaves free.) Nothing
+    when steps are not recorded."""
     if not (engine.use_graphs and model.graph_capturable()):
         return 0
     from .graphs import PORTION_BUCKETS
