@@ -18,7 +18,8 @@
 // 16 rows of a fragment meet no bank twice; rows of values are read along the row and need no padding.
 //
 // Measured (one MI355X, us a launch; the vector kernel before in brackets): 700 tokens, 32 heads on 8, head
-// size 64: 58 (447); 150 and 333 tokens, 16 heads on one latent head of 128, values of 96: 38 (298);
+// size 64: 58 (447); 150 and 333 tokens, 16 heads on one latent head of 128, values of 96: 36 (253);
+// 700 tokens, 24 heads of 128 on 8: 146 (897), 16 heads of 16 on 4: 34 (207); 64 rows on 1,500 keys, 8 x 128: 98 (1,451);
 // one token behind 333 to 601 keys of four sequences, 32 heads on 8, head size 64, 32 splits planned: 9.3 (24.9).
 #pragma once
 #include <atomic>
