@@ -640,8 +640,8 @@ extern "C" int ptl_attention_decode(void* out, long out_stride, const void* q, l
 // num_splits workgroups a (sequence, kv head) pair, each with an equal part of that pair's keys; those without keys
 // leave at once, and a pair that the first one covers is done. The parts of the others meet in a second kernel.
 //
-// What bounds the kernel is the memory a compute unit keeps on its way (about 26 GB/s a unit however many
-// workgroups it holds, 6.6 TB/s in all), so its time is that of the unit with the most keys. Workgroups go to the
+// What bounds the kernel is the memory a compute unit keeps on its way (about 26 GB/s a unit, hardly more with two
+// workgroups than with one; 6.6 TB/s in all), so its time is that of the unit with the most keys. Workgroups go to the
 // units in turn, so with the sequences fastest in the grid the splits of a pair meet on one unit as soon as
 // n_seq * Hkv is a multiple of the units: the longest sequence's unit gets it num_splits times. Where contexts
 // differ (each workgroup finds that out from ctx_len, a recorded step does not know it) workgroups therefore take
