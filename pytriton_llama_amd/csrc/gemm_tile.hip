@@ -1,0 +1,325 @@
+// Products of some hundred rows of x (a batch of short prompts, a portion of a prompt beside decoding requests) in
+// bfloat16 on the matrix cores, where the library's product is far from what the card can do: x [M, K] times the
+// row-major W [N, K], transposed.
+//   ptl_tile_gemm_sums   the product as float32 partial sums over equal slices of K, which the norm that follows
+//                        adds up (ptl_rows_sum_add_rmsnorm): a matrix of few rows and a deep K (the down and output
+//                        projections) has too few tiles for the compute units otherwise
+//   ptl_tile_gate_up     act(x Wg^T) * (x Wu^T) for W = [Wg; Wu]: the rows of a gate and of its up lie in one wave's
+//                        tile, so the [M, 2 I] product is never stored
+// The reference runs these products through cuBLAS and the rest as kernels of their own
+// (lite_llama/models/llama.py:107-120, lite_llama/kernels/swiglu.py, skip_rmsnorm.py).
+//
+// Four waves multiply, each a part of the tile, and two bring the operands through LDS (tile_stream.h). What bounds it: with
+// few workgroups the latency of W on its way from HBM (a chunk a compute unit and 0.35 to 0.7 us, of which the matrix
+// instructions take 0.06 to 0.5), with all compute units at work what they read from L2, 11 to 16 TB/s. LDS is next: a
+// wave of 64 x 64 reads as many bytes as LDS gives in the time of its products, hence parts of 64 x 128 and 144 x 64 in the
+// larger tiles. The reads go between the products (tile_interleave), a workgroup walks several tiles where there are more than the chip
+// holds, and the loading waves run ahead into the next one.
+// Tried: W from the blocked copy straight into registers, x alone through LDS (2,048 x 2,048 x 8,192: 150 us for
+// 128 x 256, 85 for 128 x 128, against 103 and 67); a seventh wave that touches W 6 to 16 chunks ahead (10 to 35 % slower);
+// rows of x and W padded by 64 or 128 columns (level).
+//
+// Measured (one MI355X, cold weights, us; the library's product and the kernel behind it in brackets): down projection with
+// sum, residual and norm, 2,048 x 8,192, 80 / 285 / 532 / 1,024 rows: 16.5 / 26.4 / 32.0 / 47.5 (25.3 / 37.0 / 49.0 / 56.0);
+// 3,072 x 8,192 22.7 / 35.0 / 43.3 / 64.4 (44.0 / 40.1 / 56.3 / 71.7); 4,096 x 14,336 34.3 / 54.4 / 75.7 / 121 (49.9 / 85.2 /
+// 119 / 138); output projection, 2,048 x 2,048 10.6 / 14.4 / 17.3 / 21.8 (13.0 / 15.4 / 17.5 / 22.0). Gate-up with SiLU-multiply,
+// 2 x 8,192 x 2,048, 80 / 285 / 532 / 700 rows: 20.4 / 30.3 / 41.2 / 56.8 (24.5 / 34.9 / 46.4 / 53.3).
+#include "common.h"
+#include "device.h"
+#include "mfma.h"
+#include "tile_stream.h"
+
+#include <atomic>
+
+namespace {
+
+enum { OUT_SUMS = 0, OUT_GLU = 1 };
+
+constexpr int KC = TILE_ROW / 2;           // columns of a chunk
+
+// round to nearest even by the hardware's conversion
+__device__ __forceinline__ bf16_t to_bf16(float f) {
+  union { __bf16 b; bf16_t u; } r;
+  r.b = (__bf16)f;
+  return r.u;
+}
+__device__ __forceinline__ float rounded(float f) { return (float)(__bf16)f; }
+
+// The activation of a pair. SiLU by the hardware's exponential and reciprocal (1 ulp each, far below the rounding of the
+// result to bfloat16): the matrix cores stand still meanwhile, and with expf and a division 2,048 x 16,384 x 2,048 takes
+// 150 us instead of 136.
+__device__ __forceinline__ float pair_value(const GluArgs& a, float g, float u) {
+  if (a.act == GLU_SILU)
+    return g * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * g)) * u;
+  return glu(a, g, u);
+}
+
+struct TileArgs {
+  void* y;                   // OUT_SUMS: float32 [splits, M, N]; OUT_GLU: bfloat16 [M, N]
+  const bf16_t* x;
+  const bf16_t* w;
+  int M, N, K;               // N: columns of y
+  long ldx;
+  int splits, tiles_m, tiles_n;
+  GluArgs act;
+};
+
+struct Tile {
+  int m0, n0, split;
+};
+
+// Tile t of the list: slices of K slowest; then groups of eight tiles of rows, inside which the rows go fastest, so
+// that consecutive tiles share rows of W and of x.
+template <int BM, int COLS> __device__ __forceinline__ Tile tile_at(const TileArgs& a, int t) {
+  constexpr int GM = 8;
+  const int per_split = a.tiles_m * a.tiles_n;
+  Tile r;
+  r.split = t / per_split;
+  const int u = t - r.split * per_split;
+  const int group = u / (GM * a.tiles_n), in_group = u - group * (GM * a.tiles_n);
+  const int gm = min(GM, a.tiles_m - group * GM);
+  const int tn = in_group / gm;
+  r.m0 = (group * GM + in_group - tn * gm) * BM;
+  r.n0 = tn * COLS;
+  return r;
+}
+
+// BM x BN: rows of x and of W a tile; WGM x WGN waves share it; NB buffers, PW loading waves.
+template <int BM, int BN, int WGM, int WGN, int NB, int PW, int MODE>
+__global__ void __launch_bounds__(64 * (WGM * WGN + PW))
+gemm_tile_kernel(const TileArgs a) {
+  constexpr int WAVES = WGM * WGN;
+  constexpr int WM = BM / WGM, WN = BN / WGN;                // the wave's part of the tile
+  constexpr int TM = WM / 16, TN = WN / 16;
+  constexpr int COLS = MODE == OUT_GLU ? BN / 2 : BN;        // columns of y a tile gives
+  constexpr int CHUNK = (BM + BN) * TILE_ROW;                // rows of x, then rows of W
+  static_assert(MODE != OUT_GLU || TN % 2 == 0, "the two of a pair meet in a wave");
+  extern __shared__ __align__(16) unsigned char lds[];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  const int M = a.M, N = a.N, K = a.K;
+  // Workgroups go to the XCDs in turn; XCD c takes a run of consecutive tiles of every round, which share rows of x
+  // and of W in its L2.
+  const int total = a.tiles_m * a.tiles_n * a.splits, G = gridDim.x;
+  const int run = G >> 3, rest = G & 7, xcd = blockIdx.x & 7;
+  const int first_tile = xcd * run + min(xcd, rest) + (blockIdx.x >> 3);
+  const int my_tiles = (total - first_tile + G - 1) / G;     // (the grid has no more workgroups than there are tiles)
+  const int k_per_split = K / a.splits, chunks = k_per_split / KC;
+
+  if (wave >= WAVES) {
+    tile_bring<BM + BN, NB, PW>(lds, wave - WAVES, lane, my_tiles, chunks, [&](int i, int r) {
+      const Tile t = tile_at<BM, COLS>(a, first_tile + i * G);
+      const size_t k0 = (size_t)t.split * k_per_split;
+      if (r < BM) return reinterpret_cast<const char*>(a.x + (size_t)min(t.m0 + r, M - 1) * a.ldx + k0);
+      const int q = r - BM;
+      int row;
+      if (MODE == OUT_GLU) {                                 // a wave's rows: one half gate, the other half up
+        const int part = q / WN, at = q - part * WN, up = at >= WN / 2;
+        row = min(t.n0 + part * (WN / 2) + (up ? at - WN / 2 : at), N - 1) + (up ? N : 0);
+      } else {
+        row = min(t.n0 + q, N - 1);
+      }
+      return reinterpret_cast<const char*>(a.w + (size_t)row * K + k0);
+    });
+    return;
+  }
+
+  const int ln = lane & 15, lg = lane >> 4, wm = wave / WGN, wn = wave - wm * WGN;
+  const int x_at = (wm * WM + ln) * TILE_ROW, w_at = (BM + wn * WN + ln) * TILE_ROW;
+  const int p0 = 16 * (lg ^ (ln & 7)), p1 = 16 * ((4 + lg) ^ (ln & 7));
+  f32x4_t acc[TN][TM];
+  Frag8 xf[2][TM], wf[2][TN];                                // of the two halves of a chunk
+  auto read = [&](const unsigned char* at, int h) __attribute__((always_inline)) {
+    const int p = h ? p1 : p0;
+#pragma unroll
+    for (int j = 0; j < TN; ++j) wf[h][j].u = load16(at + w_at + j * 16 * TILE_ROW + p);
+#pragma unroll
+    for (int i = 0; i < TM; ++i) xf[h][i].u = load16(at + x_at + i * 16 * TILE_ROW + p);
+  };
+  auto multiply = [&](int h) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+        acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[h][j].v, xf[h][i].v, acc[j][i], 0, 0, 0);
+  };
+  int slot = 0;
+  for (int n = 0; n < my_tiles; ++n) {
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int i = 0; i < TM; ++i) acc[j][i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    tile_meet();
+    read(lds + slot * CHUNK, 0);
+    for (int c = 0; c + 1 < chunks; ++c) {
+      tile_wait_lds();
+      __builtin_amdgcn_sched_barrier(0);
+      read(lds + slot * CHUNK, 1);
+      multiply(0);
+      tile_interleave<TM + TN, TM * TN>();
+      tile_wait_lds();             // every read of the chunk has come back before the wave says that it is done with it
+      tile_meet();
+      slot = slot + 1 == NB ? 0 : slot + 1;
+      __builtin_amdgcn_sched_barrier(0);
+      read(lds + slot * CHUNK, 0);
+      multiply(1);
+      tile_interleave<TM + TN, TM * TN>();
+    }
+    tile_wait_lds();
+    __builtin_amdgcn_sched_barrier(0);
+    read(lds + slot * CHUNK, 1);
+    multiply(0);
+    tile_interleave<TM + TN, TM * TN>();
+    tile_wait_lds();
+    multiply(1);
+    slot = slot + 1 == NB ? 0 : slot + 1;
+
+    // the lane holds, of every 16 x 16 results, the columns 4 lg + i (rows of W) of row ln (of x)
+    const Tile t = tile_at<BM, COLS>(a, first_tile + n * G);
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+      const int m = t.m0 + wm * WM + 16 * i + ln;
+      if (m >= M) continue;
+      if (MODE == OUT_SUMS) {
+        float* row = reinterpret_cast<float*>(a.y) + ((size_t)t.split * M + m) * N;
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+          const int col = t.n0 + wn * WN + 16 * j + 4 * lg;
+          if (col < N) *reinterpret_cast<f32x4_t*>(row + col) = acc[j][i];
+        }
+      } else {
+        bf16_t* row = reinterpret_cast<bf16_t*>(a.y) + (size_t)m * N;
+#pragma unroll
+        for (int j = 0; j < TN / 2; ++j) {
+          const int col = t.n0 + wn * (WN / 2) + 16 * j + 4 * lg;
+          if (col >= N) continue;
+          union { uint2 u; bf16_t e[4]; } o;
+          // the two products are rounded to bfloat16 first, as a stored product is
+#pragma unroll
+          for (int k = 0; k < 4; ++k)
+            o.e[k] = to_bf16(pair_value(a.act, rounded(acc[j][i][k]), rounded(acc[j + TN / 2][i][k])));
+          *reinterpret_cast<uint2*>(row + col) = o.u;
+        }
+      }
+    }
+  }
+}
+
+// The tiles there are: rows of x and of W, waves along either, buffers, workgroups a compute unit (LDS), and what one
+// takes, in us: r rounds of workgroups with c chunks each, of which a share f of the chip's places is taken, take
+// r (c (chunk + full f) + tile). Fitted to 12 shapes of W (2,048 to 28,672 rows, 2,048 to 14,336 columns), 80 to 2,048 rows and
+// 1 to 8 slices; 6 to 14 % (root mean square) from the measured times, and the plan chosen by it is 1 % slower on average
+// than the fastest, 11 % at worst.
+#define TILES(T)                                     \
+  T(64, 64, 2, 2, 5, 2, 0.17f, 0.30f, 1.4f)          \
+  T(64, 128, 2, 2, 5, 1, 0.30f, 0.08f, 1.9f)         \
+  T(128, 64, 2, 2, 5, 1, 0.27f, 0.09f, 2.1f)         \
+  T(96, 128, 2, 2, 5, 1, 0.35f, 0.10f, 2.7f)         \
+  T(128, 128, 2, 2, 4, 1, 0.35f, 0.19f, 4.1f)        \
+  T(160, 128, 2, 2, 4, 1, 0.40f, 0.20f, 4.8f)        \
+  T(192, 128, 2, 2, 3, 1, 0.43f, 0.29f, 5.8f)        \
+  T(128, 192, 2, 2, 3, 1, 0.47f, 0.27f, 5.5f)        \
+  T(96, 256, 2, 2, 3, 1, 0.56f, 0.23f, 5.2f)         \
+  T(112, 256, 1, 4, 3, 1, 0.59f, 0.26f, 6.1f)        \
+  T(128, 256, 2, 2, 3, 1, 0.59f, 0.35f, 7.3f)        \
+  T(144, 256, 1, 4, 3, 1, 0.67f, 0.27f, 7.6f)
+
+struct Shape {
+  int rows, cols, per_unit;
+  float chunk, full, tile;
+};
+constexpr Shape SHAPES[] = {
+#define T(BM, BN, WGM, WGN, NB, OCC, CHUNK, FULL, TILE) {BM, BN, OCC, CHUNK, FULL, TILE},
+    TILES(T)
+#undef T
+};
+constexpr int N_SHAPES = sizeof(SHAPES) / sizeof(SHAPES[0]);
+
+struct Plan {
+  int shape, splits;
+  float us;
+};
+
+// rows_w: rows of W. Slices are equal, of at least 512 columns, at most eight; each costs the float32 sums once more on their
+// way out and in (5 TB/s).
+Plan plan_for(int M, int rows_w, int K, bool sums) {
+  const int cus = compute_units();
+  Plan best{0, 1, 1e30f};
+  for (int s = 1; s <= (sums ? 8 : 1); s *= 2) {
+    if ((K / KC) % s || (s > 1 && K / s < 512)) break;
+    const float extra = s > 1 ? 4.0f * s * M * rows_w / 5e6f : 0.f;
+    for (int i = 0; i < N_SHAPES; ++i) {
+      const Shape& h = SHAPES[i];
+      const long tiles = (long)((M + h.rows - 1) / h.rows) * ((rows_w + h.cols - 1) / h.cols) * s;
+      const long places = (long)h.per_unit * cus, rounds = (tiles + places - 1) / places;
+      const float fill = (float)tiles / (float)(rounds * places);
+      const float us = rounds * (K / KC / s * (h.chunk + h.full * fill) + h.tile) + extra;
+      if (us < best.us) best = Plan{i, s, us};
+    }
+  }
+  return best;
+}
+
+template <int BM, int BN, int WGM, int WGN, int NB, int OCC, int MODE>
+int launch(TileArgs a, hipStream_t stream) {
+  const size_t lds = (size_t)NB * (BM + BN) * TILE_ROW;
+  auto kernel = gemm_tile_kernel<BM, BN, WGM, WGN, NB, 2, MODE>;
+  static std::atomic<bool> raised{false};      // (per instantiation)
+  if (!raised.load(std::memory_order_relaxed)) {
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                            (int)lds) != hipSuccess) {
+      (void)hipGetLastError();
+      return PTL_ERR_LAUNCH;
+    }
+    raised.store(true, std::memory_order_relaxed);
+  }
+  const int cols = MODE == OUT_GLU ? BN / 2 : BN;
+  a.tiles_m = (a.M + BM - 1) / BM;
+  a.tiles_n = (a.N + cols - 1) / cols;
+  const long total = (long)a.tiles_m * a.tiles_n * a.splits, most = (long)OCC * compute_units();
+  if (total > 0x3fffffff) return PTL_ERR_ARG;
+  kernel<<<(unsigned)(total < most ? total : most), 64 * (WGM * WGN + 2), lds, stream>>>(a);
+  return ptl_launch_status();
+}
+
+template <int MODE> int run(int shape, const TileArgs& a, hipStream_t stream) {
+  int i = 0;
+#define T(BM, BN, WGM, WGN, NB, OCC, CHUNK, FULL, TILE) \
+  if (shape == i++) return launch<BM, BN, WGM, WGN, NB, OCC, MODE>(a, stream);
+  TILES(T)
+#undef T
+  return PTL_ERR_ARG;
+}
+
+bool aligned(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
+
+bool bad(const void* y, const void* x, const void* w, int M, int N, int K, long ldx) {
+  return M <= 0 || N <= 0 || N % 4 || K <= 0 || K % KC || ldx % 8 || ldx < K || !aligned(y) || !aligned(x) || !aligned(w);
+}
+
+}  // namespace
+
+// The slices of K that ptl_tile_gemm_sums should leave partial sums of.
+extern "C" int ptl_tile_gemm_splits(int M, int N, int K) {
+  if (M <= 0 || N <= 0 || K <= 0 || K % KC) return 1;
+  return plan_for(M, N, K, true).splits;
+}
+
+// y float32 [splits, M, N] = x [M, K] W^T, one slice of K each (``splits`` as ptl_tile_gemm_splits says).
+// K a multiple of 64, N of 4, 16-byte aligned rows.
+extern "C" int ptl_tile_gemm_sums(float* y, const void* x, const void* w, int M, int N, int K, long ldx, int splits,
+                                  hipStream_t stream) {
+  if (bad(y, x, w, M, N, K, ldx)) return PTL_ERR_ARG;
+  const Plan p = plan_for(M, N, K, true);
+  if (splits != p.splits) return PTL_ERR_ARG;
+  return run<OUT_SUMS>(p.shape, TileArgs{y, (const bf16_t*)x, (const bf16_t*)w, M, N, K, ldx, p.splits, 0, 0, GluArgs{0, 0.f}},
+                       stream);
+}
+
+// out bfloat16 [M, I] = act(x Wg^T) * (x Wu^T) for W = [Wg; Wu] [2 I, K]. K a multiple of 64, I of 4, 16-byte aligned rows.
+extern "C" int ptl_tile_gate_up(void* out, const void* x, const void* w, int M, int I, int K, long ldx, int act,
+                                float limit, hipStream_t stream) {
+  if (bad(out, x, w, M, I, K, ldx) || !glu_ok(act)) return PTL_ERR_ARG;
+  return run<OUT_GLU>(plan_for(M, 2 * I, K, false).shape,
+                      TileArgs{out, (const bf16_t*)x, (const bf16_t*)w, M, I, K, ldx, 1, 0, 0, GluArgs{act, limit}}, stream);
+}

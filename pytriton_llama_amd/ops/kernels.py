@@ -584,10 +584,7 @@ def sum_add_rmsnorm(partials: torch.Tensor, residual: torch.Tensor, weight: torc
 def gemm_rows_add_rmsnorm_fits(x: torch.Tensor, w: torch.Tensor, blocked: Optional[torch.Tensor],
                                residual: torch.Tensor, norm_weight: torch.Tensor) -> bool:
     N = w.shape[0]
-    return (_rows_x_ok(x, w, blocked, "add_norm") and residual.dtype == torch.bfloat16 and residual.is_cuda
-            and residual.shape == (x.shape[0], N) and residual.is_contiguous()
-            and norm_weight.dtype == torch.float32 and norm_weight.is_cuda and norm_weight.is_contiguous()
-            and norm_weight.numel() == N and N % 8 == 0 and N <= 8192)
+    return _rows_x_ok(x, w, blocked, "add_norm") and _sum_norm_ok(x, N, residual, norm_weight)
 
 
 def gemm_rows_add_rmsnorm(x: torch.Tensor, w: torch.Tensor, blocked: torch.Tensor, residual: torch.Tensor,
@@ -599,6 +596,86 @@ def gemm_rows_add_rmsnorm(x: torch.Tensor, w: torch.Tensor, blocked: torch.Tenso
     M, K = x.shape
     partials = gemm_rows(x, w, blocked, torch.float32, splits=gemm_rows_splits(M, w.shape[0], K))
     return sum_add_rmsnorm(partials, residual, norm_weight, eps)
+
+
+# Rows from which, and up to which, the products of csrc/gemm_tile.hip take a step, against the library's product with the
+# kernel behind it (cold weights, us, one MI355X). A product with the norm behind it, 80 / 285 / 700 rows: output
+# projections 2,048 x 2,048 10.6 / 14.4 / 18.3 against 13.0 / 15.4 / 18.5, 3,072 x 3,072 15.0 / 20.3 / 29.6 against 16.9 / 21.8 /
+# 31.4, 4,096 x 4,096 17.9 / 27.7 / 38.8 against 22.0 / 31.3 / 40.5; at 1,024 rows 21.8 / 38.6 / 51.1 against 22.0 / 37.4 / 49.7.
+# A deep K gains more and longer (2,048 x 8,192, 700 / 1,024 / 1,531 rows: 36 / 48 / 65 against 50 / 56 / 65; 4,096 x 14,336
+# 94 / 121 / 183 against 108 / 138 / 175). Gate-up, 80 / 285 / 532 / 700 rows: 2 x 8,192 x 2,048 20.4 / 30.3 / 41.2 / 56.8
+# against 24.5 / 34.9 / 46.4 / 53.3, 2 x 8,192 x 3,072 27.7 / 43.1 / 60.2 / 81.1 against 31.9 / 47.3 / 64.0 / 71.8; of a larger W the
+# library's large tiles are ahead earlier: 2 x 14,336 x 4,096, 80 / 130 / 200 / 400 rows 54 / 60 / 72 / 117 against 72 / 65 / 71 / 105.
+TILE_MIN_ROWS = 65
+TILE_ROWS_SUMS, TILE_ROWS_SUMS_DEEP = 768, 1088           # ..., where K is at least twice N
+TILE_ROWS_GATE_UP, TILE_ROWS_GATE_UP_LARGE = 576, 160     # ..., where W holds more than TILE_LARGE_W elements
+TILE_LARGE_W = 1 << 26
+
+
+def _tile_x_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether the products of csrc/gemm_tile.hip take x with w [N, K]."""
+    return (x.is_cuda and w.is_cuda and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.dim() == 2
+            and w.dim() == 2 and x.shape[0] > 0 and x.shape[1] % 64 == 0 and w.shape[1] == x.shape[1]
+            and w.shape[0] % 8 == 0 and x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.stride(0) >= x.shape[1]
+            and x.data_ptr() % 16 == 0 and w.is_contiguous() and w.data_ptr() % 16 == 0)
+
+
+def gemm_tile_add_rmsnorm_fits(x: torch.Tensor, w: torch.Tensor, residual: torch.Tensor,
+                               norm_weight: torch.Tensor) -> bool:
+    """Whether ``gemm_tile_add_rmsnorm`` takes the product and is the faster way for it."""
+    M, K = x.shape
+    N = w.shape[0]
+    return (TILE_MIN_ROWS <= M <= (TILE_ROWS_SUMS_DEEP if K >= 2 * N else TILE_ROWS_SUMS) and _tile_x_ok(x, w)
+            and _sum_norm_ok(x, N, residual, norm_weight))
+
+
+def _sum_norm_ok(x: torch.Tensor, N: int, residual: torch.Tensor, norm_weight: torch.Tensor) -> bool:
+    return (residual.dtype == torch.bfloat16 and residual.is_cuda and residual.shape == (x.shape[0], N)
+            and residual.is_contiguous() and norm_weight.dtype == torch.float32 and norm_weight.is_cuda
+            and norm_weight.is_contiguous() and norm_weight.numel() == N and N % 8 == 0 and N <= 8192)
+
+
+def gemm_tile_sums(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """Float32 partial sums [splits, M, N] of x @ w.T over equal slices of K, as many as the plan of
+    csrc/gemm_tile.hip says (for ``sum_add_rmsnorm``)."""
+    if not _tile_x_ok(x, w):
+        raise KernelError("gemm_tile_sums: needs bfloat16 x [M, K] and contiguous w [N, K], K a multiple of 64, N of 8, "
+                          "16-byte aligned rows")
+    M, K = x.shape
+    N = w.shape[0]
+    lib = library.load("gemm_tile")
+    splits = int(lib.ptl_tile_gemm_splits(M, N, K))
+    y = torch.empty((splits, M, N), dtype=torch.float32, device=x.device)
+    _check(lib.ptl_tile_gemm_sums(_ptr(y), _ptr(x), _ptr(w), M, N, K, ctypes.c_long(x.stride(0)), splits, _stream()),
+           "gemm_tile_sums")
+    return y
+
+
+def gemm_tile_add_rmsnorm(x: torch.Tensor, w: torch.Tensor, residual: torch.Tensor, norm_weight: torch.Tensor,
+                          eps: float) -> torch.Tensor:
+    """rmsnorm(x @ w.T + residual) * norm_weight for some hundred rows, ``residual`` replaced by the sum: the product
+    as partial sums over slices of K, then one kernel that adds them up and normalises whole rows."""
+    return sum_add_rmsnorm(gemm_tile_sums(x, w), residual, norm_weight, eps)
+
+
+def gate_up_tile_fits(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether ``gate_up_tile`` takes x and is the faster way for it."""
+    most = TILE_ROWS_GATE_UP_LARGE if w.numel() > TILE_LARGE_W else TILE_ROWS_GATE_UP
+    return TILE_MIN_ROWS <= x.shape[0] <= most and _tile_x_ok(x, w)
+
+
+def gate_up_tile(x: torch.Tensor, w: torch.Tensor, act: int = GLU_SILU, limit: float = 0.0) -> torch.Tensor:
+    """act(x Wg^T) * (x Wu^T) for w = [Wg; Wu] ([2I, K]) in one kernel, for some hundred rows (act as for
+    ``gate_up_silu``; csrc/gemm_tile.hip)."""
+    if not _tile_x_ok(x, w):
+        raise KernelError("gate_up_tile: needs bfloat16 x [M, K] and contiguous w [2 I, K], K a multiple of 64, I of 4, "
+                          "16-byte aligned rows")
+    M, K = x.shape
+    I = w.shape[0] // 2
+    out = torch.empty((M, I), dtype=torch.bfloat16, device=x.device)
+    _check(library.load("gemm_tile").ptl_tile_gate_up(_ptr(out), _ptr(x), _ptr(w), M, I, K, ctypes.c_long(x.stride(0)),
+                                                      int(act), ctypes.c_float(limit), _stream()), "gate_up_tile")
+    return out
 
 
 def gate_up_silu_fits(x: torch.Tensor, w: torch.Tensor, blocked: Optional[torch.Tensor] = None) -> bool:

@@ -61,7 +61,10 @@ class SwiGLU(Part):
             if defer_output:
                 return PendingProduct(a, self.down, self.down_blocked)
             return linear(a, self.down, blocked=self.down_blocked)
-        a = ops.silu_mul(linear(x, self.gate_up, blocked=self.gate_up_blocked), self.act)
+        if ops.gate_up_tile_fits(x, self.gate_up):          # some hundred rows: the same in tiles
+            a = ops.gate_up_tile(x, self.gate_up, self.act)
+        else:
+            a = ops.silu_mul(linear(x, self.gate_up, blocked=self.gate_up_blocked), self.act)
         if defer_output:                    # (the norm that follows picks the kernels by the rows)
             return PendingProduct(a, self.down, self.down_blocked)
         return linear(a, self.down, blocked=self.down_blocked)
@@ -107,7 +110,10 @@ class GatedMLP(Part):
         if ops.gate_up_silu_fits(x, self.gate_up, self.gate_up_blocked):
             a = ops.gate_up_silu(x, self.gate_up, None, self.gate_up_blocked, self.glu, self.limit)
             return linear(a, self.down, blocked=self.down_blocked)
-        a = ops.gated_act(linear(x, self.gate_up, blocked=self.gate_up_blocked), self.act, self.limit)
+        if ops.gate_up_tile_fits(x, self.gate_up):          # some hundred rows: the same in tiles
+            a = ops.gate_up_tile(x, self.gate_up, self.glu, self.limit)
+        else:
+            a = ops.gated_act(linear(x, self.gate_up, blocked=self.gate_up_blocked), self.act, self.limit)
         return linear(a, self.down, blocked=self.down_blocked)
 
 

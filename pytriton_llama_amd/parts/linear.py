@@ -17,7 +17,7 @@ import torch
 
 from .. import ops
 
-LINEAR_LIBRARIES = ("gemm", "gemm_f32", "gemm_rows", "blaslt")
+LINEAR_LIBRARIES = ("gemm", "gemm_f32", "gemm_rows", "gemm_tile", "blaslt")
 SKINNY_ROWS = 8          # rows up to which the skinny kernel takes a bfloat16 product
 SKINNY_ROWS_F32 = 16     # ... when float32 output is wanted (the head)
 

@@ -16,7 +16,7 @@ class RMSNorm(Part):
     call sites lite_llama/models/llama.py:149,160,219). Without a residual the
     input itself is the residual (:181). ``offset``: what is added to the checkpoint's vector
     to give the weight (1.0 for a design that stores its norm weights around zero)."""
-    kernel_libraries = ("norm", "gemm", "gemm_rows", "stream")
+    kernel_libraries = ("norm", "gemm", "gemm_rows", "gemm_tile", "stream")
     takes_pending_product = True
 
     def __init__(self, size: int, eps: float, weight_name: str = "weight", streams: int = 1,
@@ -47,6 +47,10 @@ class RMSNorm(Part):
             if (residual is not None and x.blocked is not None
                     and ops.gemm_rows_add_rmsnorm_fits(x.x, x.w, x.blocked, residual, self.weight)):
                 y = ops.gemm_rows_add_rmsnorm(x.x, x.w, x.blocked, residual, self.weight, self.eps)
+                return y, residual
+            # some hundred rows (a portion of a prompt): the same, in tiles of rows of x and of W
+            if residual is not None and ops.gemm_tile_add_rmsnorm_fits(x.x, x.w, residual, self.weight):
+                y = ops.gemm_tile_add_rmsnorm(x.x, x.w, residual, self.weight, self.eps)
                 return y, residual
             # the few rows of a decode step: the product, the residual sum and the weight in one
             # kernel; the rsqrt factor is left to the part that takes the result

@@ -593,6 +593,59 @@ def test_gemm_rows_add_rmsnorm(ops, mnk):
     torch.testing.assert_close(one.float(), got.float(), atol=2e-2, rtol=2e-2)
 
 
+@pytest.mark.parametrize("mnk", [(1, 8, 64), (65, 2048, 8192), (80, 72, 128), (97, 4096, 2048), (129, 264, 4096),
+                                 (200, 2048, 2048), (285, 2048, 8192), (401, 3072, 3072), (532, 4096, 1536),
+                                 (700, 1032, 576), (1024, 2048, 8192), (1088, 3072, 2048)])
+def test_gemm_tile_add_rmsnorm(ops, mnk):
+    """Products of some hundred rows as partial sums over slices of K: rows of x and of W that are no multiple of a
+    tile, one chunk of K, depths with and without slices, more tiles than the chip holds; against a float64 product
+    (float32 sums of up to 8,192 exact products: 1e-4), and with the norm behind them against the separate kernels."""
+    M, N, K = mnk
+    torch.manual_seed(41)
+    x = torch.randn(M, K + 16, device="cuda").to(torch.bfloat16)[:, :K]          # rows of a wider buffer
+    w = (torch.randn(N, K, device="cuda") / math.sqrt(K)).to(torch.bfloat16)
+    parts = ops.gemm_tile_sums(x, w)
+    assert parts.shape[1:] == (M, N) and K % (64 * parts.shape[0]) == 0
+    torch.testing.assert_close(parts.sum(dim=0), (x.double() @ w.double().T).float(), atol=1e-4, rtol=1e-4)
+    res = torch.randn(M, N, device="cuda").to(torch.bfloat16)
+    nw = (1.0 + 0.2 * torch.randn(N, device="cuda")).float()
+    r1, r2 = res.clone(), res.clone()
+    got = ops.gemm_tile_add_rmsnorm(x, w, r1, nw, 1e-5)
+    want = ops.add_rmsnorm(ops.gemm_nt(x, w), r2, nw, 1e-5)
+    torch.testing.assert_close(r1.float(), r2.float(), atol=2e-2, rtol=2e-2)
+    torch.testing.assert_close(got.float(), want.float(), atol=3e-2, rtol=2e-2)
+    with pytest.raises(ops.KernelError):
+        ops.gemm_tile_sums(x[:, :K - 32], w[:, :K - 32].contiguous())            # K no multiple of a chunk
+    with pytest.raises(ops.KernelError):
+        ops.gemm_tile_sums(x, w[:, 1:])
+
+
+@pytest.mark.parametrize("act", ["silu", "gelu_tanh", "clamped"])
+@pytest.mark.parametrize("mik", [(1, 4, 64), (65, 8192, 2048), (81, 36, 192), (130, 2048, 2048), (200, 8192, 2048),
+                                 (285, 8192, 3072), (400, 1000, 512), (532, 8192, 2048), (576, 14336, 1024)])
+def test_gate_up_tile(ops, mik, act):
+    """Gate and up rows in one tile: columns that are no multiple of a tile, every tile shape the plan takes for
+    these rows, the three activations; against float64 with the two products rounded to bfloat16 (a product on
+    the edge of a rounding may fall to the other side: 2^-8 of it, and the same once more for the result's rounding)."""
+    M, I, K = mik
+    torch.manual_seed(42)
+    x = torch.randn(M, K, device="cuda").to(torch.bfloat16)
+    w = (torch.randn(2 * I, K, device="cuda") / math.sqrt(K) * 2).to(torch.bfloat16)
+    code = {"silu": ops.GLU_SILU, "gelu_tanh": ops.GLU_GELU_TANH, "clamped": ops.GLU_CLAMPED}[act]
+    got = ops.gate_up_tile(x, w, code, 1.5)
+    g, u = (x.double() @ w.double().T).to(torch.bfloat16).double().chunk(2, dim=1)
+    if act == "silu":
+        want = g * torch.sigmoid(g) * u
+    elif act == "gelu_tanh":
+        want = 0.5 * g * (1 + torch.tanh(math.sqrt(2 / math.pi) * (g + 0.044715 * g ** 3))) * u
+    else:
+        g, u = g.clamp(max=1.5), u.clamp(-1.5, 1.5)
+        want = g * torch.sigmoid(1.702 * g) * (u + 1)
+    torch.testing.assert_close(got.double(), want, atol=2e-2, rtol=2e-2)
+    # the activation itself: the hardware's exponential and reciprocal are far below the result's rounding
+    assert (got.double() - want).norm() <= 3e-3 * want.norm()
+
+
 @pytest.mark.parametrize("mik", [(17, 64, 64), (33, 8192, 2048), (64, 352, 160), (128, 1024, 4096), (9, 64, 64),
                                  (16, 8192, 2048), (13, 352, 160), (44, 2048, 512), (48, 96, 64)])
 def test_gate_up_silu_for_tens_of_rows(ops, mik):
