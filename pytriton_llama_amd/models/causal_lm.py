@@ -136,8 +136,12 @@ class CausalLM:
             h = self.embedding.forward(ctx.token_ids, ctx.positions)
         else:
             h = self.embedding.forward(ctx.token_ids)
-        residual = None
+        residual, picked = None, False
         last = len(self.schedule) - 1
+        # Where few rows want logits (a prompt: its last) the last block gives those rows alone, if it can: of the
+        # output projection on everything is row by row. A 2,048-token prompt, 16 layers of the 1B shape: 4.5 % of
+        # the products' time.
+        rows = ctx.logit_rows if 0 < ctx.num_logit_rows < h.shape[0] else None
         for i, call in enumerate(self.schedule):
             cache = storage.view(call.cache_layer, call.writes)
             block = self.blocks[call.block]
@@ -150,12 +154,19 @@ class CausalLM:
             elif (after is not None and getattr(block, "can_defer_output", False)
                     and getattr(after, "takes_pending_product", False)):
                 h, residual = block.forward(h, residual, ctx, cache, defer_output=True)
+            elif i == last and rows is not None and getattr(block, "takes_rows", False):
+                # (the rows of the final norm are picked then, so it may take the last product as well)
+                defer = (getattr(block, "can_defer_output", False)
+                         and getattr(self.final_norm, "takes_pending_product", False))
+                h, residual = block.forward(h, residual, ctx, cache, rows=rows, **({"defer_output": True} if defer else {}))
+                picked = True
             else:
                 h, residual = block.forward(h, residual, ctx, cache)
-        h = as_tensor(h)
+        if not picked:
+            h = as_tensor(h)
         if ctx.num_logit_rows == 0:
             return torch.empty((0, self.vocab_size), dtype=torch.float32, device=h.device)
-        if ctx.num_logit_rows != h.shape[0] or not ctx.logit_rows_are_identity:
+        if not picked and (ctx.num_logit_rows != h.shape[0] or not ctx.logit_rows_are_identity):
             h = h.index_select(0, ctx.logit_rows)
             if residual is not None:
                 residual = residual.index_select(0, ctx.logit_rows)

@@ -234,6 +234,16 @@ def as_tensor(v):
     return v.tensor() if isinstance(v, (PendingProduct, PendingScale, PendingSum, RoutedSum)) else v
 
 
+def pick_rows(v, rows: torch.Tensor):
+    """Rows ``rows`` (int32, on the device) of a tensor or of a product or sum that is not computed yet, which then
+    is one of those rows only."""
+    if isinstance(v, PendingProduct):
+        return PendingProduct(v.x.index_select(0, rows), v.w, v.blocked)
+    if isinstance(v, PendingSum):
+        return PendingSum([(y.index_select(0, rows), f) for y, f in v.terms], v.bias, v.norms)
+    return as_tensor(v).index_select(0, rows)
+
+
 def run_norm(norm, x, residual, consumer=None):
     """norm.forward for an x that may be pending, on behalf of ``consumer`` (the part that gets
     the result; None: someone who wants a tensor)."""
@@ -247,6 +257,8 @@ class Part:
     takes_pending_product = False     # norms, blocks
     takes_pending_scale = False       # mixers, feed-forwards
     can_defer_output = False          # mixers, feed-forwards, blocks
+    takes_rows = False                # blocks: forward(..., rows=) gives those rows only. The mixer runs over all
+                                      # of them (later steps read what it keeps), what is behind it is row by row
     graph_capturable = True           # False: forward waits for the device or reads device data
                                       # on the host; steps of a model with such a part are
                                       # launched kernel by kernel, never replayed as graphs

@@ -4,7 +4,7 @@ from __future__ import annotations
 import torch
 
 from .. import ops
-from .base import ParamSource, Part, PendingSum, as_tensor, place, register_part, run_norm
+from .base import ParamSource, Part, PendingSum, as_tensor, pick_rows, place, register_part, run_norm
 
 
 @register_part("block", "prenorm")
@@ -39,6 +39,7 @@ class PreNormBlock(Part):
         return tuple(dict.fromkeys(lists))
 
     can_defer_output = True
+    takes_rows = True
 
     @property
     def takes_pending_product(self) -> bool:
@@ -54,9 +55,10 @@ class PreNormBlock(Part):
     def graph_capturable(self) -> bool:
         return all(getattr(p, "graph_capturable", True) for p in self.children().values())
 
-    def forward(self, h, residual, ctx, cache, defer_output: bool = False):
+    def forward(self, h, residual, ctx, cache, defer_output: bool = False, rows=None):
         """``h`` may be pending work of the block before (parts/base.py); with ``defer_output``
-        the feed-forward may leave its last product to whoever normalises next."""
+        the feed-forward may leave its last product to whoever normalises next. ``rows``: the rows
+        that are wanted, where not all are."""
         mixer, ffn = self.mixer, self.feed_forward
         h, residual = run_norm(self.input_norm, h, residual, mixer)
         if not getattr(mixer, "takes_pending_scale", False):
@@ -66,6 +68,9 @@ class PreNormBlock(Part):
             h = mixer.forward(h, ctx, cache, defer_output=True)
         else:
             h = mixer.forward(h, ctx, cache)
+        if rows is not None:
+            h = pick_rows(h, rows)
+            residual = residual.index_select(0, rows) if residual is not None else None
         h, residual = run_norm(self.post_norm, h, residual, ffn)
         if not getattr(ffn, "takes_pending_scale", False):
             h = as_tensor(h)
@@ -93,6 +98,7 @@ class SandwichBlock(Part):
     the block that runs next. The block's last kernel then applies it as well and the second
     value it returns, where other blocks carry a residual, is the stream normed for that mixer;
     a block that is handed such a value starts from it instead of norming the stream itself."""
+    takes_rows = True
 
     def __init__(self, pre_mixer_norm: Part, mixer: Part, post_mixer_norm: Part,
                  pre_ffn_norm: Part = None, feed_forward: Part = None, post_ffn_norm: Part = None,
@@ -151,16 +157,19 @@ class SandwichBlock(Part):
         out = pre.forward(copy, None)[0] if pre is not None else None
         return out, copy
 
-    def forward(self, h, residual, ctx, cache):
+    def forward(self, h, residual, ctx, cache, rows=None):
         if h.dtype != torch.float32:
             raise ops.KernelError("a sandwich block runs on a float32 residual stream")
-        stream = h
+        stream, tokens = h, ctx.token_ids
         dtype = self.mixer_dtype()
         if residual is not None:            # the stream, normed for this mixer by the block before
             a = residual
         else:
             a, _ = self._add(stream, None, None, self.norm1, dtype)
         y = self.mixer.forward(a, ctx, cache)
+        if rows is not None:
+            stream, y = stream.index_select(0, rows), pick_rows(y, rows)
+            tokens = tokens.index_select(0, rows) if self.side is not None else tokens
         nxt = self.next_norm if self._fusable(self.next_norm) else None
         want_copy = self.side is not None and dtype != torch.float32
         last_pre = None if self.side is not None else nxt
@@ -171,7 +180,7 @@ class SandwichBlock(Part):
         else:
             ahead, copy = self._add(stream, y, self.norm1b, last_pre, dtype, want_copy)
         if self.side is not None:
-            ahead = self.side.forward(stream, copy if want_copy else stream, ctx.token_ids,
+            ahead = self.side.forward(stream, copy if want_copy else stream, tokens,
                                       nxt.params() if nxt is not None else None, dtype)
         return stream, ahead
 
@@ -202,6 +211,7 @@ class OutputNormBlock(Part):
     stream is the block's ``h`` (float32 [T, hidden], updated in place); what the block returns
     where others carry a residual is that copy, and a block that is handed one starts from it.
     ``last`` (set by the model's builder): nobody reads the copy after this block."""
+    takes_rows = True
 
     def __init__(self, mixer: Part, mixer_norm: Part, feed_forward: Part = None, ffn_norm: Part = None):
         if (feed_forward is None) != (ffn_norm is None):
@@ -252,7 +262,7 @@ class OutputNormBlock(Part):
             _, out = ops.stream_add_rmsnorm(stream, as_tensor(y), norm.weight, norm.eps, None, dtype, copy)
         return out if copy else (stream if want_copy else None)
 
-    def forward(self, h, residual, ctx, cache):
+    def forward(self, h, residual, ctx, cache, rows=None):
         if h.dtype != torch.float32:
             raise ops.KernelError("an output-norm block runs on a float32 residual stream")
         stream, dtype = h, self.norm1.dtype
@@ -260,6 +270,8 @@ class OutputNormBlock(Part):
         if a is None:
             a = stream if dtype == torch.float32 else ops.stream_add_dyt(stream, None, None, None, dtype, True)[1]
         y = self.mixer.forward(a, ctx, cache)
+        if rows is not None:
+            stream, y = stream.index_select(0, rows), pick_rows(y, rows)
         if self.feed_forward is None:
             return stream, self._add(stream, y, self.norm1, dtype, not self.last)
         a = self._add(stream, y, self.norm1, dtype, True)

@@ -118,6 +118,34 @@ def test_a_replayed_portion_gives_the_logits_of_any_one_of_its_rows(cases, dtype
 
 
 @pytest.mark.parametrize("dtype", DTYPES, ids=["fp32", "bf16"])
+@pytest.mark.parametrize("name", ["A", "B", "C"])
+def test_steps_that_want_few_of_their_rows(cases, name, dtype):
+    """Steps of several prompts that want none, one, two (in falling order) or all but one of a prompt's rows: the last
+    block gives those rows alone, in the order asked for, and what it keeps of the other rows is read by the next step."""
+    from pytriton_llama_amd.engine.batch import StepEntry
+    folder, page, seqs, want = cases[name]
+    seqs = dict(list(seqs.items())[:4])
+    runner = load_runner(folder, dtype, page, sum(-(-len(t) // page) for t in seqs.values()))
+    cut = {r: len(t) // 2 for r, t in seqs.items()}
+    first = [[], [cut["r1"] - 1], [cut["r2"] - 1, 0], list(range(1, cut["r3"]))]
+    got = {r: [] for r in seqs}
+    places = {r: [] for r in seqs}
+    for step in (0, 1):
+        wants = first if step == 0 else [[len(t) - cut[r] - 1] for r, t in seqs.items()]
+        entries = [StepEntry(r, t[:cut[r]] if step == 0 else t[cut[r]:], w) for (r, t), w in zip(seqs.items(), wants)]
+        logits = runner.step(entries).float().cpu()
+        assert logits.shape[0] == sum(len(w) for w in wants)
+        for (r, _), w in zip(seqs.items(), wants):
+            got[r].append(logits[:len(w)])
+            logits = logits[len(w):]
+            places[r] += [p + step * cut[r] for p in w]
+    for r, g in got.items():
+        g, plain = torch.cat(g), want[dtype][r]
+        err = float((g - plain[places[r]]).abs().max()) / float(plain.abs().max())
+        assert err <= TOL[dtype], f"config {name} {dtype} {r}: off by {err}"
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=["fp32", "bf16"])
 def test_first_tokens_of_a_sequence(cases, dtype):
     """Positions 0, 1, 2: one token whole, then one by one from an empty cache."""
     folder, page, seqs, want = cases["B"]
