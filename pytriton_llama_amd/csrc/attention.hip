@@ -648,11 +648,13 @@ extern "C" int ptl_attention_decode(void* out, long out_stride, const void* q, l
 // their pairs by length, the longest first, every second turn of the units from the other end: a unit's second
 // workgroup is short where its first is long. Who computes a part is all that changes: a sequence's bits do not
 // depend on the others. From DECODE_ORDER_KEYS keys a split on (of the longest), where some context is a quarter
-// longer or shorter than the first, for 9 to 64 sequences and 2 to 4 splits: with more splits the parts are short and
+// longer or shorter than the first, for 9 to 64 sequences and up to 4 splits: with more splits the parts are short and
 // the order costs 0.5 to 1.5 us (16 sequences, 2 heads of 96, 16 splits: 300 to 3,000 keys 15.0 -> 16.6, 500 each 10.2 ->
 // 11.4); equal contexts keep the order in which a pair's parts lie in the L2 that the second kernel reads them from
 // (48 of 1,000, 8 x 128: 40.9 against 45.0); at 400 keys a split it gains nothing yet (20 of 800 beside 12 empty rows,
-// 8 x 64: 14.5 against 15.8).
+// 8 x 64: 14.5 against 15.8). One split, where there are more workgroups than units, from DECODE_ORDER_KEYS_ONE keys on
+// (of the longest): 64 of 61 to 2,610 keys, 8 kv heads of 64, 47 -> 40, 8 x 128 96 -> 70; 64 of 1,000 to 2,000 42 -> 40 and 82 ->
+// 73; one of 3,000 beside 63 of 100 46 -> 39 and 90 -> 61; at 400 to 600 keys it costs (16.5 -> 19.0, 28.7 -> 29.9).
 // Measured (one MI355X, us with the second kernel; the sequences fastest in brackets): 20 of 130 to 2,900 keys
 // beside 12 empty rows, 8 kv heads of 128, 42 (55); 32 of 300 to 3,000, 8 x 128, 48 (60), 8 x 64, 29 (34); 16 of 300 to
 // 3,000, 8 x 128, 30 (36); 48 of 300 to 3,000, 8 x 128, 68 (86); 32 of 1,000 to 2,000, 8 x 128, 42 (45.5); one of 3,000
@@ -689,6 +691,7 @@ __device__ __forceinline__ void wave_lds_fence() {
 
 #define DECODE_ORDER_SEQS 64       // sequences of an ordered launch (one a lane)
 #define DECODE_ORDER_KEYS 512      // keys a split from which on the order matters
+#define DECODE_ORDER_KEYS_ONE 1024 // ... where there is one split
 
 // A grid of one dimension: workgroups (sequence, kv head, split), the sequences fastest. ORDERED: by length where
 // contexts differ (above); cus: the compute units.
@@ -733,7 +736,7 @@ attn_decode_mfma_kernel(bf16_t* __restrict__ out, long out_stride, const bf16_t*
     const int c = lane < n_seq ? ctx_len[lane] : 0, keys = c > 0 ? walk_of(ex, c) : 0;
     const unsigned long long some = __ballot(keys > 0);
     const int one = some ? __builtin_amdgcn_readlane(keys, __ffsll(some) - 1) : 0;
-    if (__any(keys > DECODE_ORDER_KEYS * num_splits) && __any(keys > 0 && abs(keys - one) > one / 4)) {
+    if (__any(keys > (num_splits == 1 ? DECODE_ORDER_KEYS_ONE : DECODE_ORDER_KEYS * num_splits)) && __any(keys > 0 && abs(keys - one) > one / 4)) {
       // unit u: the workgroups of a sequence's split (one a kv head); turn: the units that all compute units take
       const int u = blockIdx.x / Hkv, turn = max(1, cus / Hkv), first = u / turn * turn;
       const int at = u / turn % 2 ? first + min(turn, n_seq * num_splits - first) - 1 - (u - first) : u;
@@ -943,8 +946,8 @@ attn_decode_mfma_kernel(bf16_t* __restrict__ out, long out_stride, const bf16_t*
   }
 }
 
-static bool decode_ordered(int n_seq, int num_splits) {
-  return num_splits > 1 && num_splits <= 4 && n_seq > 8 && n_seq <= DECODE_ORDER_SEQS;
+static bool decode_ordered(int n_seq, int Hkv, int num_splits) {
+  return num_splits <= 4 && n_seq > 8 && n_seq <= DECODE_ORDER_SEQS && (num_splits > 1 || n_seq * Hkv > compute_units());
 }
 
 template <int NDT, int UNR, bool ORDERED>
@@ -1008,7 +1011,7 @@ extern "C" int ptl_attention_decode_mfma(void* out, long out_stride, const void*
     return PTL_ERR_ARG;
   if (unroll == 0) unroll = 2;
 #define GO(N, U)                                                                                                \
-  (decode_ordered(n_seq, num_splits)                                                                            \
+  (decode_ordered(n_seq, Hkv, num_splits)                                                                            \
        ? launch_decode_mfma<N, U, true>(out, out_stride, q, q_stride, k_cache, v_cache, q_start, ctx_len,       \
                                         block_table, bt_stride, parts, n_seq, Hq, Hkv, page_size, ex, scale,    \
                                         num_splits, stream)                                                     \

@@ -1006,6 +1006,31 @@ def test_attention_decode_mfma_ragged_batch_gives_what_each_gives_alone(ops, n, 
         torch.testing.assert_close(out[r].float().cpu(), want.float(), **tol(torch.bfloat16))
 
 
+@pytest.mark.parametrize("n,Hkv,D", [(33, 8, 64), (64, 8, 64), (64, 5, 128), (56, 8, 96)])
+@pytest.mark.parametrize("longest", [1024, 1025, 3000])
+def test_attention_decode_mfma_one_split_in_order(ops, n, Hkv, D, longest):
+    """More workgroups than compute units and one split: the order by length (from 1,025 keys on) covers every pair, a
+    turn that the kv heads do not fill and a short last turn among them; the bits are those of each sequence alone."""
+    P, pages, Hq = 16, 200, 2 * Hkv
+    g = torch.Generator().manual_seed(n)
+    ctx = [7 * i * i % 400 + 1 for i in range(n)]
+    ctx[n // 3], ctx[2], ctx[n - 1], ctx[5] = longest, longest - 1, longest // 2, 0
+    kc, vc = (torch.randn(pages, Hkv, P, D, generator=g).to(torch.bfloat16).cuda() for _ in range(2))
+    bt = torch.stack([torch.randperm(pages, generator=g) for _ in range(n)]).to(torch.int32).cuda()
+    q = torch.randn(n, Hq, D, generator=g).to(torch.bfloat16).cuda()
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")
+
+    def run(rows):
+        out = torch.full((len(rows), Hq, D), 9.0, dtype=torch.bfloat16, device="cuda")
+        ops.attention_decode(out, q[rows], kc, vc, i32(list(range(len(rows) + 1))), i32([ctx[r] for r in rows]),
+                             bt[rows], len(rows), D ** -0.5, num_splits=1, matrix_cores=True)
+        return out
+    out = run(list(range(n)))
+    assert bool((out[5] == 0).all())
+    for r in range(n):
+        assert torch.equal(out[r], run([r])[0]), f"sequence {r}"
+
+
 @pytest.mark.parametrize("D", [16, 32, 48, 64, 80, 128])
 @pytest.mark.parametrize("heads", [3, 4, 8, 16])
 def test_attention_decode_float32_form_by_head_size(ops, D, heads):
