@@ -9,6 +9,7 @@ from typing import Any, Dict, List, Optional, Sequence, Tuple
 import torch
 
 from ..parts.base import ParamSource, Part, as_tensor, run_norm
+from . import prompt_steps
 
 
 def _numel(shape) -> int:
@@ -142,7 +143,13 @@ class CausalLM:
         # output projection on everything is row by row. A 2,048-token prompt, 16 layers of the 1B shape: 4.5 % of
         # the products' time.
         rows = ctx.logit_rows if 0 < ctx.num_logit_rows < h.shape[0] else None
+        # a step of prompts: all blocks but the last in native code, if they are of the kind that has it
+        done = prompt_steps.run(self, h, ctx, storage)
+        if done is not None:
+            h, residual = done
         for i, call in enumerate(self.schedule):
+            if done is not None and i < last:
+                continue
             cache = storage.view(call.cache_layer, call.writes)
             block = self.blocks[call.block]
             # a block may leave its last product to the norm that comes next, if that norm can

@@ -635,6 +635,11 @@ def _sum_norm_ok(x: torch.Tensor, N: int, residual: torch.Tensor, norm_weight: t
             and norm_weight.is_contiguous() and norm_weight.numel() == N and N % 8 == 0 and N <= 8192)
 
 
+def gemm_tile_splits(M: int, N: int, K: int) -> int:
+    """The slices of K that ``gemm_tile_sums`` leaves partial sums of."""
+    return int(library.load("gemm_tile").ptl_tile_gemm_splits(int(M), int(N), int(K)))
+
+
 def gemm_tile_sums(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """Float32 partial sums [splits, M, N] of x @ w.T over equal slices of K, as many as the plan of
     csrc/gemm_tile.hip says (for ``sum_add_rmsnorm``)."""
@@ -644,7 +649,7 @@ def gemm_tile_sums(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     M, K = x.shape
     N = w.shape[0]
     lib = library.load("gemm_tile")
-    splits = int(lib.ptl_tile_gemm_splits(M, N, K))
+    splits = gemm_tile_splits(M, N, K)
     y = torch.empty((splits, M, N), dtype=torch.float32, device=x.device)
     _check(lib.ptl_tile_gemm_sums(_ptr(y), _ptr(x), _ptr(w), M, N, K, ctypes.c_long(x.stride(0)), splits, _stream()),
            "gemm_tile_sums")

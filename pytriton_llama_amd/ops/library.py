@@ -27,7 +27,7 @@ HIPCC_FLAGS = ["--offload-arch=" + ARCH, "-O3", "-fPIC", "-shared", "-std=c++17"
                "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
 
 KERNEL_LIBRARIES = ("embedding", "norm", "rope", "attention", "attention_prefill", "activation",
-                    "gemm", "gemm_f32", "gemm_rows", "gemm_tile", "blaslt", "sampling", "probe", "stream", "latent", "moe", "prepare",
+                    "gemm", "gemm_f32", "gemm_rows", "gemm_tile", "blaslt", "sampling", "probe", "stream", "latent", "moe", "prepare", "prompt",
                     "recurrent", "selective", "linear_scan")
 # options of single sources. attention_prefill: no value there is a NaN unless an input is, and
 # without the promise every maximum of scores is preceded by instructions that quiet its inputs

@@ -61,7 +61,7 @@ class PagedAttention(Part):
         self.o_blocked: Optional[torch.Tensor] = None
         libs = ("attention", "rope") + LINEAR_LIBRARIES
         if self.head_dim % 32 == 0 and self.head_dim <= 128:
-            libs += ("attention_prefill",)          # the matrix-core kernel for prompt portions
+            libs += ("attention_prefill", "prompt")     # the matrix-core kernel for prompt portions, steps of prompts
         if position is not None:
             libs += tuple(position.kernel_libraries)
         self.kernel_libraries = tuple(dict.fromkeys(libs))

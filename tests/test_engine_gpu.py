@@ -145,6 +145,35 @@ def test_steps_that_want_few_of_their_rows(cases, name, dtype):
         assert err <= TOL[dtype], f"config {name} {dtype} {r}: off by {err}"
 
 
+@pytest.mark.parametrize("lengths", [(40, 25), (40, 24), (70, 45, 1), (129, 3, 64, 100), (300, 280, 7), (400, 390, 311)])
+def test_steps_of_prompts_in_native_code_give_the_bits_of_the_parts(cases, lengths, monkeypatch):
+    """Steps of several prompts: native calls between the attentions (from 65 rows on) launch what the parts launch:
+    equal logits, and equal ones in the next step, which reads the pages; rows where the tile products take all, some
+    and none of the products, with and without a decoding request."""
+    from pytriton_llama_amd.engine.batch import StepEntry
+    from pytriton_llama_amd.models import prompt_steps
+    folder, page = cases["B"][0], cases["B"][1]
+    seqs = random_sequences(tiny("B")[0]["vocab_size"], lengths, seed=9)
+    went = []
+    native = prompt_steps.run
+
+    def run(how):
+        monkeypatch.setattr(prompt_steps, "run", how)
+        runner = load_runner(folder, torch.bfloat16, page, sum(-(-len(t) // page) + 1 for t in seqs.values()))
+        out = []
+        for cut in (slice(0, None), slice(0, 2)):
+            out.append(runner.step([StepEntry(r, t[cut], range(len(t[cut]))) for r, t in seqs.items()]).clone())
+        return out
+
+    def counted(*args):
+        done = native(*args)
+        went.append(done is not None)
+        return done
+    with_native, with_parts = run(counted), run(lambda *args: None)
+    assert went == [sum(lengths) >= 65, False]
+    assert all(torch.equal(a, b) for a, b in zip(with_native, with_parts))
+
+
 @pytest.mark.parametrize("dtype", DTYPES, ids=["fp32", "bf16"])
 def test_first_tokens_of_a_sequence(cases, dtype):
     """Positions 0, 1, 2: one token whole, then one by one from an empty cache."""
