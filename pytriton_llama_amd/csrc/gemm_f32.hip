@@ -65,6 +65,75 @@ __device__ __forceinline__ void few_results(float* __restrict__ y, const float* 
   }
 }
 
+// What becomes of a tile's results. FORM_PLAIN: rows of y. The other two have 8-row tiles of four pairs of rows of W, the
+// first of a pair in row n, the second in row n + 4, and finish the pair: FORM_GLU a gate and its up row, I apart,
+// act(gate) * up; FORM_QKV rows j and j + D / 2 of a head of q | k | v, rotated (pairs, angles and cache pages as
+// rope.hip has them). A decode step of 4 rows at the Llama-3.2-1B shape had a kernel of 4.7 us for either in every layer.
+enum { FORM_PLAIN = 0, FORM_GLU = 1, FORM_QKV = 2 };
+
+struct FewOut {
+  int half;                        // FORM_GLU: I, FORM_QKV: D / 2
+  int act;
+  const int32_t *positions, *slots;          // of the rows of x; slots null: nothing goes into the cache
+  const float* inv_freq;           // null: no rotation
+  float *k_cache, *v_cache;
+  int Hq, Hkv, page_size;
+};
+
+// row of W in place r (0 .. 7) of a tile
+template <int FORM, int ROWS> __device__ __forceinline__ int few_row(const FewOut& o, int tile, int r, int N) {
+  if (FORM == FORM_PLAIN) return min(ROWS * tile + r, N - 1);
+  const int pair = 4 * tile + (r & 3);
+  if (FORM == FORM_GLU) return pair + (r >= 4 ? o.half : 0);
+  const int head = pair / o.half;
+  return head * o.half + pair + (r >= 4 ? o.half : 0);
+}
+
+// The pairs of an 8-row tile from the spans' sums, added up as few_results does.
+template <int FORM>
+__device__ __forceinline__ void pair_results(float* __restrict__ y, const float* sums, int spans, int M, int tile, long ldy,
+                                             const FewOut& o) {
+  for (int i = threadIdx.x; i < 32; i += blockDim.x) {
+    const int n = i & 3, m = i >> 2;
+    if (m >= M) continue;
+    const float *p = sums + m * 4 + n, *p2 = p + 16 * 4;
+    constexpr int ODD = (2 * 16 + 8) * 4;
+    float a = 0.f, b = 0.f;
+    for (int sp = 0; sp < spans; ++sp, p += 256, p2 += 256) {
+      a += p[0] + p[ODD];
+      b += p2[0] + p2[ODD];
+    }
+    const int pair = 4 * tile + n;
+    if (FORM == FORM_GLU) {
+      y[(size_t)m * ldy + pair] = glu_act(o.act, a) * b;
+    } else {
+      const int head = pair / o.half, j = pair - head * o.half, D = 2 * o.half;
+      if (o.inv_freq && head < o.Hq + o.Hkv) {
+        float s, c;
+        sincosf((float)o.positions[m] * o.inv_freq[j], &s, &c);
+        const float x1 = a, x2 = b;
+        a = x1 * c - x2 * s;
+        b = x2 * c + x1 * s;
+      }
+      float* at = nullptr;
+      if (head < o.Hq) {
+        at = y + (size_t)m * ldy + (size_t)head * D;
+      } else {
+        const int slot = o.slots ? o.slots[m] : -1;
+        const bool k = head < o.Hq + o.Hkv;
+        if (slot >= 0) {
+          const int page = slot / o.page_size, off = slot - page * o.page_size, h = head - o.Hq - (k ? 0 : o.Hkv);
+          at = (k ? o.k_cache : o.v_cache) + (((size_t)page * o.Hkv + h) * o.page_size + off) * D;
+        }
+      }
+      if (at) {
+        at[j] = a;
+        at[j + o.half] = b;
+      }
+    }
+  }
+}
+
 template <int ROWS, int MT, int U>
 __global__ void __launch_bounds__(1024)
 gemm_f32_few_kernel(float* __restrict__ y, const float* __restrict__ x, const float* __restrict__ w,
@@ -144,10 +213,11 @@ gemm_f32_few_kernel(float* __restrict__ y, const float* __restrict__ x, const fl
 // is read in the loop: read again for every tile, x comes through the same path from L2 as W does and is as many
 // bytes (128,256 x 2,048, us at 1, 4 and 8 rows: 185, 214, 254; held 161, 171, 177). The next tile's first columns are on their way while a tile's
 // sums are added up, in two buffers, one barrier a tile. SB: load blocks of a span.
-template <int ROWS, int NB, int SB>
+template <int ROWS, int NB, int SB, int FORM>
 __global__ void __launch_bounds__(1024)
 gemm_f32_held_kernel(float* __restrict__ y, const float* __restrict__ x, const float* __restrict__ w,
-                     int M, int N, int K, long ldx, long ldy, int tiles) {
+                     int M, int N, int K, long ldx, long ldy, int tiles, FewOut out) {
+  static_assert(ROWS == 8 || FORM == FORM_PLAIN, "pairs lie in 8-row tiles");
   constexpr int KB = ROWS == 8 ? 32 : 16;        // columns of a block (as above)
   constexpr int H = ROWS == 8 ? 1 : 2;
   constexpr int U = 4, S = NB / U;               // blocks a turn, turns a tile
@@ -168,7 +238,7 @@ gemm_f32_held_kernel(float* __restrict__ y, const float* __restrict__ x, const f
   }
   F4 wa[U], wb[U];
   auto load_w = [&](F4 (&f)[U], int tile, int b0) __attribute__((always_inline)) {
-    const float* wp = w + (size_t)min(ROWS * tile + ln % ROWS, N - 1) * K + kb;
+    const float* wp = w + (size_t)few_row<FORM, ROWS>(out, tile, ln % ROWS, N) * K + kb;
 #pragma unroll
     for (int u = 0; u < U; ++u) f[u].u = KB * (b0 + u) < left ? load_once(wp + KB * (b0 + u)) : zero16();
   };
@@ -200,8 +270,37 @@ gemm_f32_held_kernel(float* __restrict__ y, const float* __restrict__ x, const f
       }
     }
     __syncthreads();
-    few_results<ROWS, 1>(y, sums, nwaves * EACH, M, N, ROWS * tile, ldy);
+    if (FORM == FORM_PLAIN) few_results<ROWS, 1>(y, sums, nwaves * EACH, M, N, ROWS * tile, ldy);
+    else pair_results<FORM>(y, sums, nwaves * EACH, M, tile, ldy, out);
   }
+}
+
+// x in registers, tiles of ``rows`` rows of W: up to 8 rows of x and 8,192 columns, or 16 and 4,096.
+template <int FORM>
+static int launch_held(float* y, const float* x, const float* w, int M, int N, int K, long ldx, long ldy, int rows,
+                       const FewOut& out, hipStream_t st) {
+  const int cus = compute_units();
+  const long blocks = (N + rows - 1) / rows;
+  const int width = span_width(K);
+  // (8 rows: 512 columns a wave where that gives 64 waves a compute unit, else 256)
+  const bool half = rows == 8 && K <= 4096 && blocks * ((K + 511) / 512) < 64L * cus;
+  const int share = rows == 8 && !half ? 512 : 256;
+  const int waves = (K + share - 1) / share;
+  const long resident = (long)cus * (16 / waves);
+  const long walk = (blocks + resident - 1) / resident;
+  const unsigned grid = (unsigned)((blocks + walk - 1) / walk);
+#define HELD(ROWS, NB, SB)                                                                                      \
+  gemm_f32_held_kernel<ROWS, NB, SB, ROWS == 8 ? FORM : FORM_PLAIN>                                             \
+      <<<grid, waves * 64, (size_t)waves * (NB / SB) * 2048, st>>>(y, x, w, M, N, K, ldx, ldy, (int)blocks, out)
+  if (rows == 16 && width == 128) HELD(16, 16, 8);
+  else if (rows == 16) HELD(16, 16, 16);
+  else if (half && width == 128) HELD(8, 8, 4);
+  else if (half) HELD(8, 8, 8);
+  else if (width == 128) HELD(8, 16, 4);
+  else if (width == 256) HELD(8, 16, 8);
+  else HELD(8, 16, 16);
+#undef HELD
+  return ptl_launch_status();
 }
 
 static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
@@ -223,25 +322,7 @@ extern "C" int ptl_gemm_f32_few(float* y, const float* x, const float* w, int M,
   // (16 rows, read again against held: 16,384 x 2,048 43 / 36, 3,072 x 2,048 12.0 / 12.2, 128,256 x 2,048 317 / 230;
   // not where 8-row tiles are taken for more than 8 rows: 2,048 x 2,048 10.4 / 11.3)
   if (rows == 8 ? M <= 8 && K <= 8192 : K <= 4096) {
-    // (8 rows: 512 columns a wave where that gives 64 waves a compute unit, else 256)
-    const bool half = rows == 8 && K <= 4096 && blocks * ((K + 511) / 512) < 64L * cus;
-    const int share = rows == 8 && !half ? 512 : 256;
-    const int waves = (K + share - 1) / share;
-    const long resident = (long)cus * (16 / waves);
-    const long walk = (blocks + resident - 1) / resident;
-    const unsigned grid = (unsigned)((blocks + walk - 1) / walk);
-#define HELD(ROWS, NB, SB)                                                                                      \
-  gemm_f32_held_kernel<ROWS, NB, SB><<<grid, waves * 64, (size_t)waves * (NB / SB) * 2048, st>>>(y, x, w, M, N, K, ldx, \
-                                                                                                 ldy, (int)blocks)
-    if (rows == 16 && width == 128) HELD(16, 16, 8);
-    else if (rows == 16) HELD(16, 16, 16);
-    else if (half && width == 128) HELD(8, 8, 4);
-    else if (half) HELD(8, 8, 8);
-    else if (width == 128) HELD(8, 16, 4);
-    else if (width == 256) HELD(8, 16, 8);
-    else HELD(8, 16, 16);
-#undef HELD
-    return ptl_launch_status();
+    return launch_held<FORM_PLAIN>(y, x, w, M, N, K, ldx, ldy, rows, FewOut{}, st);
   }
 #define GO(ROWS, MT)                                                                                        \
   gemm_f32_few_kernel<ROWS, MT, 8 / MT><<<(unsigned)blocks, spans * 64, (size_t)spans * MT * 1024, st>>>(y, x, w, M, N, K, \
@@ -251,6 +332,33 @@ extern "C" int ptl_gemm_f32_few(float* y, const float* x, const float* w, int M,
   else GO(8, 2);
 #undef GO
   return ptl_launch_status();
+}
+
+static bool pairs_ok(int M, int K, long ldx, const float* x, const float* w) {
+  return M > 0 && M <= 8 && K > 0 && K <= 8192 && K % 4 == 0 && (M == 1 || ldx % 4 == 0) && ldx >= K && aligned16(x) && aligned16(w);
+}
+
+// out [M, I] = act(x Wg^T) * (x Wu^T) for W = [Wg; Wu] [2 I, K]: up to 8 rows, K up to 8,192 in steps of 4, I in steps of 4.
+extern "C" int ptl_gate_up_f32(float* out, const float* x, const float* w, int M, int I, int K, long ldx, int act,
+                               hipStream_t st) {
+  if (!pairs_ok(M, K, ldx, x, w) || I <= 0 || I % 4 || (act != GLU_SILU && act != GLU_GELU_TANH)) return PTL_ERR_ARG;
+  FewOut o{};
+  o.half = I;
+  o.act = act;
+  return launch_held<FORM_GLU>(out, x, w, M, 2 * I, K, ldx, I, 8, o, st);
+}
+
+// q | k | v = x W^T, q and k rotated; q to q_out [M, Hq D], k and v into the cache pages at ``slots`` (null: nowhere).
+// Up to 8 rows, K up to 8,192 in steps of 4, D in steps of 8.
+extern "C" int ptl_qkv_rope_store_f32(float* q_out, const float* x, const float* w, int M, int K, long ldx,
+                                      const int32_t* positions, const float* inv_freq, const int32_t* slots,
+                                      float* k_cache, float* v_cache, int Hq, int Hkv, int D, int page_size,
+                                      hipStream_t st) {
+  if (!pairs_ok(M, K, ldx, x, w) || Hq <= 0 || Hkv <= 0 || D <= 0 || D % 8 || page_size <= 0 || !positions ||
+      (slots && (!k_cache || !v_cache)))
+    return PTL_ERR_ARG;
+  return launch_held<FORM_QKV>(q_out, x, w, M, (Hq + 2 * Hkv) * D, K, ldx, (long)Hq * D, 8,
+                               FewOut{D / 2, 0, positions, slots, inv_freq, k_cache, v_cache, Hq, Hkv, page_size}, st);
 }
 
 // ===========================================================================

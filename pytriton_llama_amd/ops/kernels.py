@@ -248,6 +248,72 @@ def gemm_nt(x: torch.Tensor, w: torch.Tensor, out_dtype: Optional[torch.dtype] =
     return y
 
 
+F32_PAIR_ROWS, F32_PAIR_COLUMNS = 8, 8192      # rows of x and columns up to which pairs of rows of W are finished in the product
+
+
+def _f32_pairs_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
+    return (x.dim() == 2 and 0 < x.shape[0] <= F32_PAIR_ROWS and x.is_cuda and x.dtype == torch.float32
+            and w.is_cuda and w.dtype == torch.float32 and w.dim() == 2 and w.is_contiguous() and w.shape[1] == x.shape[1]
+            and 0 < x.shape[1] <= F32_PAIR_COLUMNS and x.shape[1] % 4 == 0 and x.stride(1) == 1
+            and (x.shape[0] == 1 or (x.stride(0) % 4 == 0 and x.stride(0) >= x.shape[1]))
+            and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
+
+
+def gate_up_f32_fits(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether ``gate_up_f32`` takes x with w = [Wg; Wu]."""
+    return _f32_pairs_ok(x, w) and w.shape[0] % 8 == 0
+
+
+def gate_up_f32(x: torch.Tensor, w: torch.Tensor, act: int = GLU_SILU) -> torch.Tensor:
+    """act(x Wg^T) * (x Wu^T) for w = [Wg; Wu] ([2I, K]) in float32 and one kernel, for at most 8 rows: the bits of
+    ``silu_mul(gemm_nt(x, w), act)`` (csrc/gemm_f32.hip)."""
+    if not gate_up_f32_fits(x, w):
+        raise KernelError("gate_up_f32: needs float32 x [M, K] of at most 8 rows and contiguous w [2 I, K], K a multiple of 4 "
+                          "up to 8,192, I of 4, 16-byte aligned rows")
+    M, K = x.shape
+    out = torch.empty((M, w.shape[0] // 2), dtype=torch.float32, device=x.device)
+    _check(library.load("gemm_f32").ptl_gate_up_f32(_ptr(out), _ptr(x), _ptr(w), M, w.shape[0] // 2, K,
+                                                    ctypes.c_long(x.stride(0) if M > 1 else K), int(act), _stream()),
+           "gate_up_f32")
+    return out
+
+
+def qkv_rope_store_f32_fits(x: torch.Tensor, w: torch.Tensor, head_dim: int) -> bool:
+    """Whether ``qkv_rope_store_f32`` takes x."""
+    return head_dim % 8 == 0 and _f32_pairs_ok(x, w)
+
+
+def qkv_rope_store_f32(x: torch.Tensor, w: torch.Tensor, positions: torch.Tensor, inv_freq: Optional[torch.Tensor],
+                       slots: Optional[torch.Tensor], k_cache: Optional[torch.Tensor], v_cache: Optional[torch.Tensor],
+                       num_heads: int, num_kv_heads: int, head_dim: int, page_size: int) -> torch.Tensor:
+    """``qkv_rope_store`` in float32, for at most 8 rows: the bits of ``gemm_nt`` and ``rope_store``."""
+    M, K = x.shape
+    Hq, Hkv, D = num_heads, num_kv_heads, head_dim
+    if not qkv_rope_store_f32_fits(x, w, D) or w.shape[0] != (Hq + 2 * Hkv) * D:
+        raise KernelError(f"qkv_rope_store_f32: needs float32 x of at most 8 rows, K a multiple of 4 up to 8,192, a head size in "
+                          f"steps of 8, 16-byte aligned rows and a weight of ({Hq} + 2*{Hkv}) * {D} rows")
+    _need_gpu(positions, inv_freq, slots, k_cache, v_cache)
+    _i32(positions, "positions")
+    if positions.numel() != M:
+        raise KernelError("qkv_rope_store_f32: one position per row of x")
+    if inv_freq is not None and (inv_freq.dtype != torch.float32 or inv_freq.numel() != D // 2
+                                 or not inv_freq.is_contiguous()):
+        raise KernelError(f"qkv_rope_store_f32: inv_freq must be float32 [{D // 2}]")
+    if slots is not None:
+        if slots.dtype != torch.int32 or slots.numel() != M or not slots.is_contiguous():
+            raise KernelError("qkv_rope_store_f32: slots must be contiguous int32 [M]")
+        for name, c in (("k_cache", k_cache), ("v_cache", v_cache)):
+            if c is None or c.dim() != 4 or c.shape[1:] != (Hkv, page_size, D) \
+                    or c.dtype != torch.float32 or not c.is_contiguous():
+                raise KernelError(f"qkv_rope_store_f32: {name} must be contiguous float32 "
+                                  f"[pages, {Hkv}, {page_size}, {D}]")
+    q = torch.empty((M, Hq, D), dtype=torch.float32, device=x.device)
+    _check(library.load("gemm_f32").ptl_qkv_rope_store_f32(
+        _ptr(q), _ptr(x), _ptr(w), M, K, ctypes.c_long(x.stride(0) if M > 1 else K), _ptr(positions), _ptr(inv_freq),
+        _ptr(slots), _ptr(k_cache), _ptr(v_cache), Hq, Hkv, D, int(page_size), _stream()), "qkv_rope_store_f32")
+    return q
+
+
 F32_FEW_ROWS = 16          # rows of x up to which the kernel that streams W once takes a float32 product
 
 

@@ -114,11 +114,11 @@ class PagedAttention(Part):
             q = ops.qkv_rope_store(x, self.qkv, ctx.positions, rotary,
                                    group.slots if cache.writable else None, cache.k, cache.v,
                                    Hq, Hkv, D, cache.page_size, scale, blocked=self.qkv_blocked)
-            out = torch.empty((T, Hq, D), dtype=x.dtype, device=x.device)
-            self.attend(out, q, cache, ctx, group)
-            if defer_output:
-                return PendingProduct(out.view(T, Hq * D), self.o, self.o_blocked)
-            return linear(out.view(T, Hq * D), self.o, blocked=self.o_blocked)
+            return self._attended(q, ctx, cache, group, defer_output)
+        if fused and ops.qkv_rope_store_f32_fits(x, self.qkv, D):       # ... in float32
+            q = ops.qkv_rope_store_f32(x, self.qkv, ctx.positions, rotary, group.slots if cache.writable else None,
+                                       cache.k, cache.v, Hq, Hkv, D, cache.page_size)
+            return self._attended(q, ctx, cache, group, defer_output)
         qkv = linear(x, self.qkv, blocked=self.qkv_blocked)
         q = qkv[:, :self.q_size].view(T, Hq, D)
         k = qkv[:, self.q_size:self.q_size + self.kv_size].view(T, Hkv, D)
@@ -131,7 +131,12 @@ class PagedAttention(Part):
         ops.rope_store(q, k, v, ctx.positions, inv_freq,
                        group.slots if cache.writable else None, cache.k, cache.v,
                        cache.page_size)
-        out = torch.empty((T, Hq, D), dtype=x.dtype, device=x.device)
+        return self._attended(q, ctx, cache, group, defer_output)
+
+    def _attended(self, q, ctx, cache, group, defer_output: bool):
+        """The attention of the rotated queries and the output projection."""
+        T, Hq, D = q.shape
+        out = torch.empty((T, Hq, D), dtype=q.dtype, device=q.device)
         self.attend(out, q, cache, ctx, group)
         if defer_output:                    # (the norm that follows picks the kernels by the rows)
             return PendingProduct(out.view(T, Hq * D), self.o, self.o_blocked)

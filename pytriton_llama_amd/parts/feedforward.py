@@ -61,7 +61,9 @@ class SwiGLU(Part):
             if defer_output:
                 return PendingProduct(a, self.down, self.down_blocked)
             return linear(a, self.down, blocked=self.down_blocked)
-        if ops.gate_up_tile_fits(x, self.gate_up):          # some hundred rows: the same in tiles
+        if ops.gate_up_f32_fits(x, self.gate_up):           # ... in float32
+            a = ops.gate_up_f32(x, self.gate_up, self.act)
+        elif ops.gate_up_tile_fits(x, self.gate_up):        # some hundred rows: the same in tiles
             a = ops.gate_up_tile(x, self.gate_up, self.act)
         else:
             a = ops.silu_mul(linear(x, self.gate_up, blocked=self.gate_up_blocked), self.act)

@@ -646,6 +646,49 @@ def test_gate_up_tile(ops, mik, act):
     assert (got.double() - want).norm() <= 3e-3 * want.norm()
 
 
+@pytest.mark.parametrize("mik", [(1, 4, 4), (3, 36, 100), (8, 8192, 2048), (4, 1000, 1028), (5, 512, 8192), (2, 20, 516),
+                                 (7, 2816, 1024)])
+def test_gate_up_f32(ops, mik):
+    """Pairs of gate and up rows finished in the float32 product of few rows: the bits of the product and the
+    activation by themselves, for every number of columns a wave holds."""
+    M, I, K = mik
+    torch.manual_seed(43)
+    x = torch.randn(M, K + 4, device="cuda")[:, :K]
+    w = torch.randn(2 * I, K, device="cuda") / math.sqrt(K)
+    for act in (ops.GLU_SILU, ops.GLU_GELU_TANH):
+        assert torch.equal(ops.gate_up_f32(x, w, act), ops.silu_mul(ops.gemm_nt(x, w), act))
+    assert not ops.gate_up_f32_fits(torch.zeros(9, K, device="cuda"), w)
+    with pytest.raises(ops.KernelError):
+        ops.gate_up_f32(x, w[:-2])
+
+
+@pytest.mark.parametrize("rotated", [True, False])
+@pytest.mark.parametrize("case", [(1, 2, 1, 8, 64), (4, 32, 8, 64, 2048), (8, 3, 3, 128, 516), (5, 5, 1, 40, 4100),
+                                  (3, 8, 2, 16, 8192)])
+def test_qkv_rope_store_f32(ops, case, rotated):
+    """The float32 q | k | v projection of few rows with rotation and cache write: the bits of the three kernels it
+    stands for, in q and in the pages; rows without a slot write nothing."""
+    M, Hq, Hkv, D, K = case
+    torch.manual_seed(44)
+    P, pages = 4, 6
+    x = torch.randn(M, K, device="cuda")
+    w = torch.randn((Hq + 2 * Hkv) * D, K, device="cuda") / math.sqrt(K)
+    pos = torch.randint(0, 9000, (M,), dtype=torch.int32, device="cuda")
+    inv = (10000.0 ** (-torch.arange(0, D, 2).float() / D)).cuda() if rotated else None
+    slots = torch.randperm(P * pages)[:M].to(torch.int32)
+    slots[M // 2] = -1
+    slots = slots.cuda()
+    caches = [torch.full((pages, Hkv, P, D), 7.0, device="cuda") for _ in range(4)]
+    q = ops.qkv_rope_store_f32(x, w, pos, inv, slots, caches[0], caches[1], Hq, Hkv, D, P)
+    y = ops.gemm_nt(x, w).view(M, Hq + 2 * Hkv, D)
+    ops.rope_store(y[:, :Hq], y[:, Hq:Hq + Hkv], y[:, Hq + Hkv:], pos, inv, slots, caches[2], caches[3], P)
+    assert torch.equal(q, y[:, :Hq])
+    assert torch.equal(caches[0], caches[2]) and torch.equal(caches[1], caches[3])
+    assert torch.equal(ops.qkv_rope_store_f32(x, w, pos, inv, None, None, None, Hq, Hkv, D, P), q)
+    with pytest.raises(ops.KernelError):
+        ops.qkv_rope_store_f32(x, w, pos[:0], inv, slots, caches[0], caches[1], Hq, Hkv, D, P)
+
+
 @pytest.mark.parametrize("mik", [(17, 64, 64), (33, 8192, 2048), (64, 352, 160), (128, 1024, 4096), (9, 64, 64),
                                  (16, 8192, 2048), (13, 352, 160), (44, 2048, 512), (48, 96, 64)])
 def test_gate_up_silu_for_tens_of_rows(ops, mik):
