@@ -143,6 +143,7 @@ class CausalLM:
         # output projection on everything is row by row. A 2,048-token prompt, 16 layers of the 1B shape: 4.5 % of
         # the products' time.
         rows = ctx.logit_rows if 0 < ctx.num_logit_rows < h.shape[0] else None
+        every_row = ctx.logit_rows_are_identity and ctx.num_logit_rows == h.shape[0]
         # a step of prompts: all blocks but the last in native code, if they are of the kind that has it
         done = prompt_steps.run(self, h, ctx, storage)
         if done is not None:
@@ -152,8 +153,8 @@ class CausalLM:
                 continue
             cache = storage.view(call.cache_layer, call.writes)
             block = self.blocks[call.block]
-            # a block may leave its last product to the norm that comes next, if that norm can
-            # take it (parts/base.py); the rows for the final norm are picked first, so not there
+            # a block may leave its last product to the norm that comes next, if that norm can take it (parts/base.py),
+            # the last block to the final norm where that one's rows are not picked behind the block
             after = self.blocks[self.schedule[i + 1].block] if i < last else None
             if getattr(block, "takes_next_block", False):
                 # a block whose last kernel also does the first work of the block that runs next
@@ -161,11 +162,13 @@ class CausalLM:
             elif (after is not None and getattr(block, "can_defer_output", False)
                     and getattr(after, "takes_pending_product", False)):
                 h, residual = block.forward(h, residual, ctx, cache, defer_output=True)
-            elif i == last and rows is not None and getattr(block, "takes_rows", False):
-                # (the rows of the final norm are picked then, so it may take the last product as well)
-                defer = (getattr(block, "can_defer_output", False)
-                         and getattr(self.final_norm, "takes_pending_product", False))
-                h, residual = block.forward(h, residual, ctx, cache, rows=rows, **({"defer_output": True} if defer else {}))
+            elif i == last and (every_row or (rows is not None and getattr(block, "takes_rows", False))):
+                # (no rows are picked behind the block then, so the final norm may take its last product as well)
+                more = {"rows": rows} if rows is not None else {}
+                if (getattr(block, "can_defer_output", False)
+                        and getattr(self.final_norm, "takes_pending_product", False)):
+                    more["defer_output"] = True
+                h, residual = block.forward(h, residual, ctx, cache, **more)
                 picked = True
             else:
                 h, residual = block.forward(h, residual, ctx, cache)
