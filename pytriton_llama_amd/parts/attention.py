@@ -165,11 +165,16 @@ class PagedAttention(Part):
         # measured on MI355X (256 compute units): the matrix-core kernel is best with about two
         # workgroups a compute unit, and without splits once the batch brings 1.75 for each
         # (batch 56 with 8 kv heads; at batch 24 to 48 two splits are 2 to 3 % of a step faster
-        # than one); the other one with about four
+        # than one), and with three where there is about one workgroup a unit: in a recorded step 32 rows stand for 17
+        # to 32 requests, and the parts of the rows that are none leave at once (us with two and three at 8 kv heads of
+        # 64 / 128: 20 of 130 to 2,900 keys beside 12 empty rows 27.5 and 22.3 / 43.7 and 34.8, 24 of 300 to 2,000
+        # beside 8 22.7 and 21.2 / 34.2 and 31.8, 32 of 130 to 2,900 29.8 and 27.8 / 46.1 and 47.8, 32 of 2,000 29.7 and
+        # 28.7 / 51.6 and 53.1; not at 48 rows, 33 beside 15 empty ones: 27.7 and 26.2 / 42.3 and 46.4);
+        # the other one with about four
         base = max(1, n_dec * groups)
         cus = ops.compute_units(device)
         if matrix_cores:
-            want = 1 if 4 * base >= 7 * cus else -(-2 * cus // base)
+            want = 1 if 4 * base >= 7 * cus else max(-(-2 * cus // base), 3 if 8 * base <= 9 * cus else 2)
         else:
             want = -(-4 * cus // base)
         return max(1, min(want, -(-span // turn), 64))
