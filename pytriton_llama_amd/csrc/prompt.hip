@@ -25,7 +25,8 @@ struct PtlPromptStep {
   int o_splits, down_splits, gate_up_tile, unused;
   const int32_t *positions, *slots;
   // rows of the step: y (normed) [T, H], residual [T, H], qkv [T, (Hq + 2 Hkv) D], mixed [T, Hq D], a [T, I]; product: the
-  // partial sums, or a product [T, H]; gate_up [T, 2 I] (null where the tile product takes it)
+  // partial sums, or a product [T, H]; gate_up [T, 2 I] (not used where the tile product takes it). qkv, product and
+  // gate_up may be one place: none is read any more when the next of them is written.
   void *y, *residual, *qkv, *mixed, *product, *gate_up, *a;
 };
 

@@ -8,6 +8,7 @@ from typing import Any, Dict, List, Optional, Sequence, Tuple
 
 import torch
 
+from .. import ops
 from ..parts.base import ParamSource, Part, as_tensor, run_norm
 from . import prompt_steps
 
@@ -143,7 +144,9 @@ class CausalLM:
         # output projection on everything is row by row. A 2,048-token prompt, 16 layers of the 1B shape: 4.5 % of
         # the products' time.
         rows = ctx.logit_rows if 0 < ctx.num_logit_rows < h.shape[0] else None
-        every_row = ctx.logit_rows_are_identity and ctx.num_logit_rows == h.shape[0]
+        # (fewer rows than that: the final norm would have the same product by itself)
+        every_row = (ctx.logit_rows_are_identity and ctx.num_logit_rows == h.shape[0]
+                     and h.shape[0] >= ops.ROWS_MIN)
         # a step of prompts: all blocks but the last in native code, if they are of the kind that has it
         done = prompt_steps.run(self, h, ctx, storage)
         if done is not None:

@@ -81,20 +81,21 @@ def run(model, h: torch.Tensor, ctx, storage) -> Optional[Tuple[PendingProduct, 
         return torch.empty((T, n), dtype=torch.bfloat16, device=h.device)
     residual = h
     y = ops.add_rmsnorm(h, None, first.input_norm.weight, first.input_norm.eps)
-    qkv, mixed, a = rows(width), rows(Hq * D), rows(I)
+    mixed, a = rows(Hq * D), rows(I)
     # which kernels take the products: what the parts would choose, asked once for all layers (their shapes are equal)
     norm = first.post_norm.weight
     o_splits = ops.gemm_tile_splits(T, H, Hq * D) if ops.gemm_tile_add_rmsnorm_fits(mixed, mixer.o, residual, norm) else 0
     down_splits = ops.gemm_tile_splits(T, H, I) if ops.gemm_tile_add_rmsnorm_fits(a, ffn.down, residual, norm) else 0
     tile = ops.gate_up_tile_fits(y, ffn.gate_up)
-    product = torch.empty(T * H * max(2 * o_splits, 2 * down_splits, 1), dtype=torch.bfloat16, device=h.device)
-    gate_up = None if tile else rows(2 * I)
+    # q | k | v, a product (or its float32 sums) and gate | up, one after the other in one place: each has been read when
+    # the next is written, so a long step takes no more memory than by the parts
+    wide = torch.empty(T * max(width, H * max(2 * o_splits, 2 * down_splits, 1), 0 if tile else 2 * I),
+                       dtype=torch.bfloat16, device=h.device)
     step = prompt.PromptStep(
         T, H, I, Hq, Hkv, D, page_size, act, o_splits, down_splits, int(tile), 0, ctx.positions.data_ptr(), slots.data_ptr(),
-        y.data_ptr(), residual.data_ptr(), qkv.data_ptr(), mixed.data_ptr(), product.data_ptr(),
-        0 if gate_up is None else gate_up.data_ptr(), a.data_ptr())
+        y.data_ptr(), residual.data_ptr(), wide.data_ptr(), mixed.data_ptr(), wide.data_ptr(), wide.data_ptr(), a.data_ptr())
     table = prompt.entries()
-    q, out = qkv.view(T, Hq + 2 * Hkv, D)[:, :Hq], mixed.view(T, Hq, D)
+    q, out = wide[:T * width].view(T, Hq + 2 * Hkv, D)[:, :Hq], mixed.view(T, Hq, D)
     before = None
     for i, (b, cache) in enumerate(zip(blocks, caches)):
         m, f = b.mixer, b.feed_forward
