@@ -416,8 +416,13 @@ extern "C" int ptl_rows_gate_up_silu(void* out, const void* x, const void* w_blo
 // registers (N % 8 == 0, N <= 8192). The product is rounded to bfloat16 first, as a product
 // stored in bfloat16 would be; the sum with the residual and the statistics are float32, and
 // the norm uses the unrounded sum (lite_llama/kernels/skip_rmsnorm.py:145-152).
+// With a workgroup a row and a row read once, what bounds it is the trip to memory and back of a
+// thread's loads: a thread takes one piece of 8 columns (two above 4,096 columns), so all of a row
+// is asked for at once. us with at most 256 threads and up to four pieces a thread / so: 64 rows of
+// 3,072 in 8 slices 7.9 / 5.8, 64 of 4,096 in 4 6.3 / 4.8, 20 of 3,072 in 8 6.2 / 4.7, 64 of 5,120 in
+// 4 8.3 / 6.5, 300 of 8,192 in 1 10.8 / 8.9, 544 of 3,072 in 4 9.9 / 9.6 (36.8 MB: 3.8 TB/s).
 template <int CH>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(512)
 sum_add_rmsnorm_kernel(bf16_t* __restrict__ y, const float* __restrict__ partials, int splits,
                        bf16_t* __restrict__ residual, const float* __restrict__ w, int M, int N, float eps) {
   __shared__ float scratch[16];
@@ -480,15 +485,13 @@ sum_add_rmsnorm_kernel(bf16_t* __restrict__ y, const float* __restrict__ partial
 extern "C" int ptl_rows_sum_add_rmsnorm(void* y, const float* partials, int splits, void* residual,
                                         const float* w, int M, int N, float eps, hipStream_t stream) {
   if (M <= 0) return PTL_OK;
-  if (N <= 0 || N % 8 || N > 8 * 256 * 4 || splits < 1 || !partials || !residual || !w ||
+  if (N <= 0 || N % 8 || N > 8 * 512 * 2 || splits < 1 || !partials || !residual || !w ||
       ((uintptr_t)y | (uintptr_t)partials | (uintptr_t)residual | (uintptr_t)w) % 16)
     return PTL_ERR_ARG;
   const int nchunk = N / 8;
-  int vt = 64;
-  while (vt < 256 && vt < nchunk) vt <<= 1;
-  const int ch = (nchunk + vt - 1) / vt;
+  const int vt = min((nchunk + 63) / 64 * 64, 512);
 #define GO(C) sum_add_rmsnorm_kernel<C><<<M, vt, 0, stream>>>((bf16_t*)y, partials, splits, (bf16_t*)residual, w, M, N, eps)
-  if (ch <= 1) GO(1); else if (ch == 2) GO(2); else if (ch == 3) GO(3); else GO(4);
+  if (nchunk <= vt) GO(1); else GO(2);
 #undef GO
   return ptl_launch_status();
 }

@@ -593,6 +593,25 @@ def test_gemm_rows_add_rmsnorm(ops, mnk):
     torch.testing.assert_close(one.float(), got.float(), atol=2e-2, rtol=2e-2)
 
 
+@pytest.mark.parametrize("smn", [(1, 3, 8), (3, 2, 512), (4, 5, 520), (8, 64, 2056), (5, 20, 3072), (2, 7, 4096), (4, 3, 4104),
+                                 (4, 64, 5120), (9, 2, 8184), (1, 300, 8192)])
+def test_sum_add_rmsnorm(ops, smn):
+    """Widths around the pieces a thread and the threads a row: the float64 result of the same rounded sums."""
+    S, M, N = smn
+    torch.manual_seed(28)
+    p, res = torch.randn(S, M, N, device="cuda"), torch.randn(M, N, device="cuda").to(torch.bfloat16)
+    nw, eps = torch.randn(N, device="cuda"), 1e-5
+    total = p[0].clone()
+    for s in range(1, S):
+        total += p[s]                                              # float32, in the order of the slices
+    h = total.to(torch.bfloat16).double() + res.double()
+    want = h * torch.rsqrt(h.pow(2).mean(-1, keepdim=True) + eps) * nw.double()
+    got = ops.sum_add_rmsnorm(p, res, nw, eps)
+    assert torch.equal(res, h.float().to(torch.bfloat16))
+    # one rounding to bfloat16 (2^-9 of the value) and the float32 statistics
+    torch.testing.assert_close(got.double(), want, atol=1e-5, rtol=2 ** -8)
+
+
 @pytest.mark.parametrize("mnk", [(1, 8, 64), (65, 2048, 8192), (80, 72, 128), (97, 4096, 2048), (129, 264, 4096),
                                  (200, 2048, 2048), (285, 2048, 8192), (401, 3072, 3072), (532, 4096, 1536),
                                  (700, 1032, 576), (1024, 2048, 8192), (1088, 3072, 2048)])
