@@ -9,7 +9,7 @@ from typing import Any, Dict, List, Optional, Sequence, Tuple
 import torch
 
 from .. import ops
-from ..parts.base import ParamSource, Part, as_tensor, run_norm
+from ..parts.base import ParamSource, Part, as_tensor, run_norm, says
 from . import prompt_steps
 
 
@@ -165,11 +165,10 @@ class CausalLM:
             elif (after is not None and getattr(block, "can_defer_output", False)
                     and getattr(after, "takes_pending_product", False)):
                 h, residual = block.forward(h, residual, ctx, cache, defer_output=True)
-            elif i == last and (every_row or (rows is not None and getattr(block, "takes_rows", False))):
+            elif i == last and (every_row or (rows is not None and says(block, "takes_rows"))):
                 # (no rows are picked behind the block then, so the final norm may take its last product as well)
                 more = {"rows": rows} if rows is not None else {}
-                if (getattr(block, "can_defer_output", False)
-                        and getattr(self.final_norm, "takes_pending_product", False)):
+                if says(block, "can_defer_output") and getattr(self.final_norm, "takes_pending_product", False):
                     more["defer_output"] = True
                 h, residual = block.forward(h, residual, ctx, cache, **more)
                 picked = True

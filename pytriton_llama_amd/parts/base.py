@@ -25,7 +25,11 @@ embedding:       forward(token_ids int32 [T]) -> [T, hidden]; one whose class sa
 head:            forward(x [R, hidden]) -> float32 logits [R, vocab]
 block:           forward(h, residual, ctx, cache) -> (h, residual); may set the flags
                  can_defer_output (forward then takes defer_output=True and may return a
-                 pending h) and takes_pending_product (its h may arrive pending)
+                 pending h), takes_pending_product (its h may arrive pending) and takes_rows
+                 (forward then takes rows=, int32 indices on the device, and returns those rows
+                 only: what the model asks of its last block where few rows want logits. What
+                 such a block has behind its mixer must be row by row; feed-forwards and norms
+                 are, since a step may bring any rows of a sequence)
 
 Work handed on instead of done (optional; a part that knows nothing of it is given tensors)
 ------------------------------------------------------------------------------------------
@@ -226,6 +230,19 @@ class PendingSum:
         if self.bias is not None:
             out = out + self.bias[0] * self.bias[1]
         return out.to(self.terms[0][0].dtype)
+
+
+def says(part, flag: str) -> bool:
+    """Whether ``part`` sets ``flag`` for the ``forward`` it has: a class (or an instance) that brings a forward of its own
+    in place of an inherited one says anew what that forward takes, so a flag from further up does not count."""
+    if not getattr(part, flag, False):
+        return False
+    for named in [getattr(part, "__dict__", {})] + [vars(c) for c in type(part).__mro__]:
+        if flag in named:
+            return True
+        if "forward" in named:
+            return False
+    return False
 
 
 def as_tensor(v):
