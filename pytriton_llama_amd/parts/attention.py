@@ -59,9 +59,9 @@ class PagedAttention(Part):
         self.o: Optional[torch.Tensor] = None
         self.qkv_blocked: Optional[torch.Tensor] = None          # decode copies (make_decode_copies)
         self.o_blocked: Optional[torch.Tensor] = None
-        libs = ("attention", "rope") + LINEAR_LIBRARIES
+        libs = ("attention", "rope", "prompt") + LINEAR_LIBRARIES    # (prompt: steps of prompts, any head size)
         if self.head_dim % 32 == 0 and self.head_dim <= 128:
-            libs += ("attention_prefill", "prompt")     # the matrix-core kernel for prompt portions, steps of prompts
+            libs += ("attention_prefill",)          # the matrix-core kernel for prompt portions
         if position is not None:
             libs += tuple(position.kernel_libraries)
         self.kernel_libraries = tuple(dict.fromkeys(libs))
