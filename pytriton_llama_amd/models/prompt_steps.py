@@ -24,11 +24,15 @@ from ..parts.rotary import RotaryEncoding
 
 
 def _plain(block) -> bool:
+    """Whether the block is the plain decoder's, and what its parts do in such a step is what their classes say: a part
+    whose forward somebody replaced (to watch or to change what goes through it) is asked, not passed by."""
     mixer, ffn = block.mixer, block.feed_forward
     return (type(block) is PreNormBlock and type(mixer) is PagedAttention and type(ffn) is SwiGLU
             and type(block.input_norm) is RMSNorm and type(block.post_norm) is RMSNorm
             and block.input_norm.streams == 1 and block.post_norm.streams == 1
-            and type(mixer.position) is RotaryEncoding)
+            and type(mixer.position) is RotaryEncoding
+            and not any("forward" in vars(p) for p in (block, mixer, ffn, block.input_norm, block.post_norm))
+            and "rotary_inv_freq" not in vars(mixer.position))
 
 
 def _matrix(w, rows: int, cols: int) -> bool:
