@@ -165,16 +165,18 @@ class PagedAttention(Part):
         # measured on MI355X (256 compute units): the matrix-core kernel is best with about two
         # workgroups a compute unit, and without splits once the batch brings 1.75 for each
         # (batch 56 with 8 kv heads; at batch 24 to 48 two splits are 2 to 3 % of a step faster
-        # than one), and with three where there is about one workgroup a unit: in a recorded step 32 rows stand for 17
-        # to 32 requests, and the parts of the rows that are none leave at once (us with two and three at 8 kv heads of
-        # 64 / 128: 20 of 130 to 2,900 keys beside 12 empty rows 27.5 and 22.3 / 43.7 and 34.8, 24 of 300 to 2,000
-        # beside 8 22.7 and 21.2 / 34.2 and 31.8, 32 of 130 to 2,900 29.8 and 27.8 / 46.1 and 47.8, 32 of 2,000 29.7 and
-        # 28.7 / 51.6 and 53.1; not at 48 rows, 33 beside 15 empty ones: 27.7 and 26.2 / 42.3 and 46.4);
-        # the other one with about four
+        # than one); from 513 keys on with three where there is about one workgroup a unit, up to head size 96 (us with
+        # two and three, 32 rows at 8 kv heads, contexts of 130 to 2,900 / 1,000 / 2,000 / 300 keys each; all rows, then 24
+        # beside 8 empty ones, which leave at once and leave their units idle, as in the recorded step that stands for 17
+        # to 32 requests: head size 64 30.0 29.3 / 19.0 18.4 / 30.4 29.5 / 11.7 11.8 and 26.8 24.5 / 17.9 17.6 / 29.1 28.0 /
+        # 11.3 11.7; 96 38.5 36.9 / 25.6 25.0 / 42.8 41.6 / 14.1 14.3 and 35.7 31.8 / 25.1 24.5 / 40.4 38.1 / 13.8 14.1; but
+        # 128 48.6 55.0 / 31.2 33.6 / 53.1 54.3 / 16.1 18.3 and 45.5 42.1 / 28.0 29.9 / 50.7 52.3 / 15.6 17.8. 64 rows at 4 kv
+        # heads, 16 at 16 and 36 at 8 the same way); the other one with about four
         base = max(1, n_dec * groups)
         cus = ops.compute_units(device)
         if matrix_cores:
-            want = 1 if 4 * base >= 7 * cus else max(-(-2 * cus // base), 3 if 8 * base <= 9 * cus else 2)
+            least = 3 if D <= 96 and span > 512 and 8 * base <= 9 * cus else 2
+            want = 1 if 4 * base >= 7 * cus else max(-(-2 * cus // base), least)
         else:
             want = -(-4 * cus // base)
         return max(1, min(want, -(-span // turn), 64))
