@@ -194,15 +194,8 @@ static int launch_generic(void* out, long out_stride, const void* q, long q_stri
   const size_t lds = (size_t)(BM * Dk + BN * (Dk + 1) + BN * Dv + BM * BN) * sizeof(float);
   if (lds > 64 * 1024) {
     // more dynamic LDS than a kernel may ask for without saying so beforehand (wide heads only)
-    static size_t allowed = 0;
-    if (lds > allowed) {
-      if (hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_generic_kernel<T, TO, BN, NJ>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) {
-        (void)hipGetLastError();
-        return PTL_ERR_ARG;
-      }
-      allowed = lds;
-    }
+    static LdsAllowance allowance;
+    if (!allowance.ask(reinterpret_cast<const void*>(&attn_generic_kernel<T, TO, BN, NJ>), lds)) return PTL_ERR_ARG;
   }
   dim3 grid(n_work, Hq);
   attn_generic_kernel<T, TO, BN, NJ><<<grid, 256, lds, stream>>>(

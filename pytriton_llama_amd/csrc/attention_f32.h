@@ -22,9 +22,8 @@
 // 700 tokens, 24 heads of 128 on 8: 146 (897), 16 heads of 16 on 4: 34 (207); 64 rows on 1,500 keys, 8 x 128: 98 (1,451);
 // one token behind 333 to 601 keys of four sequences, 32 heads on 8, head size 64, 32 splits planned: 9.3 (24.9).
 #pragma once
-#include <atomic>
-
 #include "attention.h"
+#include "device.h"
 #include "mfma.h"
 #include "mfma_f32.h"
 
@@ -262,18 +261,9 @@ static int launch_attn_f32(dim3 grid, hipStream_t st, Args... args) {
   const size_t tiles = (size_t)2 * BN * (2 * D + 4) * sizeof(float);
   const size_t merge = (size_t)4 * (NK * 256 + 128) * sizeof(float);
   const size_t bytes = tiles > merge ? tiles : merge;
-  if (bytes > 64 * 1024) {                       // more than a kernel gets unasked: asked for once a device
-    static std::atomic<unsigned long long> asked{0};
-    int dev = 64;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev > 63) dev = 64;
-    if (dev == 64 || !(asked.load(std::memory_order_relaxed) >> dev & 1)) {
-      if (hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_f32_kernel<HPW, NK, BN, DECODE>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) != hipSuccess) {
-        (void)hipGetLastError();
-        return PTL_ERR_ARG;
-      }
-      if (dev < 64) asked.fetch_or(1ull << dev, std::memory_order_relaxed);
-    }
+  if (bytes > 64 * 1024) {                       // more than a kernel gets unasked
+    static LdsAllowance allowance;
+    if (!allowance.ask(reinterpret_cast<const void*>(&attn_f32_kernel<HPW, NK, BN, DECODE>), bytes)) return PTL_ERR_ARG;
   }
   attn_f32_kernel<HPW, NK, BN, DECODE><<<grid, 256, bytes, st>>>(args...);
   return ptl_launch_status();

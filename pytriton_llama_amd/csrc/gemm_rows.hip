@@ -34,6 +34,7 @@
 //     for every load a wave has under way), and no sums cross waves (pairs of tiles that an
 //     epilogue combines, gate with up, meet in LDS once at the end).
 #include "common.h"
+#include "device.h"
 #include "mfma.h"
 
 namespace {
@@ -299,39 +300,13 @@ gemm_rows_kernel(TY* __restrict__ y, const bf16_t* __restrict__ x, const bf16_t*
   }
 }
 
-int compute_units() {
-  constexpr int MAX_DEVICES = 64;
-  static int cached[MAX_DEVICES];
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= MAX_DEVICES) {
-    (void)hipGetLastError();
-    return 256;
-  }
-  if (cached[dev] == 0) {
-    int n = 0;
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) {
-      (void)hipGetLastError();
-      n = 256;
-    }
-    cached[dev] = n;
-  }
-  return cached[dev];
-}
-
 template <int MT, int KC, int DEPTH, int WT, int MODE, typename TY>
 int launch(void* y, const void* x, const void* wb, int M, int N_out, int w_rows, int K, long ldx, long ldy,
            int blocks, int splits, int pair_offset, hipStream_t stream, GluArgs act = {GLU_SILU, 0.f}) {
   const size_t lds = (size_t)NB * MT * 16 * KC * sizeof(bf16_t);
   auto kernel = gemm_rows_kernel<MT, KC, DEPTH, WT, MODE, TY>;
-  static bool raised = false;                  // (per instantiation)
-  if (!raised) {
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                            (int)lds) != hipSuccess) {
-      (void)hipGetLastError();
-      return PTL_ERR_LAUNCH;
-    }
-    raised = true;
-  }
+  static LdsAllowance allowance;
+  if (!allowance.ask(reinterpret_cast<const void*>(kernel), lds)) return PTL_ERR_LAUNCH;
   const int k_per_split = ((K + splits - 1) / splits + 31) / 32 * 32;
   kernel<<<dim3(blocks, splits), (TILES / WT + 1) * 64, lds, stream>>>(
       (TY*)y, (const bf16_t*)x, (const bf16_t*)wb, M, N_out, w_rows, K, ldx, ldy, k_per_split, pair_offset, act);

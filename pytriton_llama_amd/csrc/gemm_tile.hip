@@ -29,8 +29,6 @@
 #include "mfma.h"
 #include "tile_stream.h"
 
-#include <atomic>
-
 namespace {
 
 enum { OUT_SUMS = 0, OUT_GLU = 1 };
@@ -264,15 +262,8 @@ template <int BM, int BN, int WGM, int WGN, int NB, int OCC, int MODE>
 int launch(TileArgs a, hipStream_t stream) {
   const size_t lds = (size_t)NB * (BM + BN) * TILE_ROW;
   auto kernel = gemm_tile_kernel<BM, BN, WGM, WGN, NB, 2, MODE>;
-  static std::atomic<bool> raised{false};      // (per instantiation)
-  if (!raised.load(std::memory_order_relaxed)) {
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                            (int)lds) != hipSuccess) {
-      (void)hipGetLastError();
-      return PTL_ERR_LAUNCH;
-    }
-    raised.store(true, std::memory_order_relaxed);
-  }
+  static LdsAllowance allowance;
+  if (!allowance.ask(reinterpret_cast<const void*>(kernel), lds)) return PTL_ERR_LAUNCH;
   const int cols = MODE == OUT_GLU ? BN / 2 : BN;
   a.tiles_m = (a.M + BM - 1) / BM;
   a.tiles_n = (a.N + cols - 1) / cols;

@@ -41,6 +41,7 @@
 // form the logarithms are summed in double, in the channel form products of decays are taken inside
 // blocks of 16 tokens, so decays that vanish do no harm.
 #include "common.h"
+#include "device.h"
 #include <math.h>
 
 #define MODE_SCALAR 0
@@ -520,15 +521,9 @@ __global__ void __launch_bounds__(256) linear_combine_kernel(LinArgs A) {
 template <int NDT, int MODE, bool FINAL>
 static int launch_chunks(const LinArgs& A, int vec, int n_seqs, hipStream_t st) {
   constexpr size_t lds = chunk_lds_floats<NDT, MODE, FINAL>() * sizeof(float);
-  static bool raised = false;               // (per instantiation)
-  if (lds > 48 * 1024 && !raised) {
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(&linear_chunk_kernel<NDT, MODE, FINAL>),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) {
-      (void)hipGetLastError();
-      return PTL_ERR_LAUNCH;
-    }
-    raised = true;
-  }
+  static LdsAllowance allowance;
+  if (lds > 48 * 1024 && !allowance.ask(reinterpret_cast<const void*>(&linear_chunk_kernel<NDT, MODE, FINAL>), lds))
+    return PTL_ERR_LAUNCH;
   linear_chunk_kernel<NDT, MODE, FINAL><<<dim3((A.Dv + 63) / 64, A.H, n_seqs * A.P), 256, lds, st>>>(A, vec);
   return ptl_launch_status();
 }
