@@ -43,11 +43,13 @@ __device__ __forceinline__ bf16_t to_bf16(float f) {
 }
 __device__ __forceinline__ float rounded(float f) { return (float)(__bf16)f; }
 
-// The activation of a pair. SiLU by the hardware's exponential and reciprocal (1 ulp each, far below the rounding of the
-// result to bfloat16): the matrix cores stand still meanwhile, and with expf and a division 2,048 x 16,384 x 2,048 takes
-// 150 us instead of 136.
+// The activation of a pair, as the other kernels for a gate and its up row have it (glu); TILE_SILU_HW: SiLU by the
+// hardware's exponential and reciprocal, a few units in the last place of float32 in front of the rounding to bfloat16,
+// as silu_mul has it (activation.hip). The matrix cores stand still meanwhile: 2,048 x 16,384 x 2,048 takes 136 us so and
+// 150 with expf and a division. It is the caller who says that it had the one or the other before.
+constexpr int TILE_SILU_HW = 16;
 __device__ __forceinline__ float pair_value(const GluArgs& a, float g, float u) {
-  if (a.act == GLU_SILU)
+  if (a.act == TILE_SILU_HW)
     return g * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * g)) * u;
   return glu(a, g, u);
 }
@@ -308,9 +310,11 @@ extern "C" int ptl_tile_gemm_sums(float* y, const void* x, const void* w, int M,
 }
 
 // out bfloat16 [M, I] = act(x Wg^T) * (x Wu^T) for W = [Wg; Wu] [2 I, K]. K a multiple of 64, I of 4, 16-byte aligned rows.
+// hw_silu != 0: act is SiLU, by the hardware's functions (pair_value).
 extern "C" int ptl_tile_gate_up(void* out, const void* x, const void* w, int M, int I, int K, long ldx, int act,
-                                float limit, hipStream_t stream) {
-  if (bad(out, x, w, M, I, K, ldx) || !glu_ok(act)) return PTL_ERR_ARG;
+                                float limit, int hw_silu, hipStream_t stream) {
+  if (bad(out, x, w, M, I, K, ldx) || !glu_ok(act) || (hw_silu && act != GLU_SILU)) return PTL_ERR_ARG;
+  if (hw_silu) act = TILE_SILU_HW;
   return run<OUT_GLU>(plan_for(M, 2 * I, K, false).shape,
                       TileArgs{out, (const bf16_t*)x, (const bf16_t*)w, M, I, K, ldx, 1, 0, 0, GluArgs{act, limit}}, stream);
 }

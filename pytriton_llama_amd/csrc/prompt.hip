@@ -14,7 +14,7 @@ struct PtlPromptEntries {
   int (*sums)(float*, const void*, const void*, int, int, int, long, int, hipStream_t);
   int (*sum_norm)(void*, const float*, int, void*, const float*, int, int, float, hipStream_t);
   int (*add_norm)(void*, const void*, void*, const float*, int, int, float, int, hipStream_t);
-  int (*gate_up)(void*, const void*, const void*, int, int, int, long, int, float, hipStream_t);
+  int (*gate_up)(void*, const void*, const void*, int, int, int, long, int, float, int, hipStream_t);
   int (*act_mul)(void*, const void*, int, int, int, int, hipStream_t);
 };
 
@@ -59,7 +59,7 @@ extern "C" int ptl_prompt_between(const PtlPromptEntries* e, const PtlPromptStep
   if (before) {
     if ((rc = product_norm(s->mixed, before->o, s->Hq * D, s->o_splits, before->post_norm, before->post_eps))) return rc;
     if (s->gate_up_tile) {
-      if ((rc = e->gate_up(s->a, s->y, before->gate_up, T, s->I, H, H, s->act, 0.f, st))) return rc;
+      if ((rc = e->gate_up(s->a, s->y, before->gate_up, T, s->I, H, H, s->act, 0.f, s->act == GLU_SILU, st))) return rc;
     } else {
       if ((rc = e->product(s->gate_up, s->y, before->gate_up, T, 2 * s->I, H, H, 2 * s->I, PTL_DTYPE_BF16, 1, 0, 0, 0, 0, st)))
         return rc;

@@ -735,9 +735,11 @@ def gate_up_tile_fits(x: torch.Tensor, w: torch.Tensor) -> bool:
     return TILE_MIN_ROWS <= x.shape[0] <= most and _tile_x_ok(x, w)
 
 
-def gate_up_tile(x: torch.Tensor, w: torch.Tensor, act: int = GLU_SILU, limit: float = 0.0) -> torch.Tensor:
+def gate_up_tile(x: torch.Tensor, w: torch.Tensor, act: int = GLU_SILU, limit: float = 0.0,
+                 hw_silu: bool = False) -> torch.Tensor:
     """act(x Wg^T) * (x Wu^T) for w = [Wg; Wu] ([2I, K]) in one kernel, for some hundred rows (act as for
-    ``gate_up_silu``; csrc/gemm_tile.hip)."""
+    ``gate_up_silu``; csrc/gemm_tile.hip). ``hw_silu``: SiLU by the hardware's exponential and reciprocal, for a caller
+    who took it from ``silu_mul`` otherwise, which does that in bfloat16."""
     if not _tile_x_ok(x, w):
         raise KernelError("gate_up_tile: needs bfloat16 x [M, K] and contiguous w [2 I, K], K a multiple of 64, I of 4, "
                           "16-byte aligned rows")
@@ -745,7 +747,8 @@ def gate_up_tile(x: torch.Tensor, w: torch.Tensor, act: int = GLU_SILU, limit: f
     I = w.shape[0] // 2
     out = torch.empty((M, I), dtype=torch.bfloat16, device=x.device)
     _check(library.load("gemm_tile").ptl_tile_gate_up(_ptr(out), _ptr(x), _ptr(w), M, I, K, ctypes.c_long(x.stride(0)),
-                                                      int(act), ctypes.c_float(limit), _stream()), "gate_up_tile")
+                                                      int(act), ctypes.c_float(limit),
+                                                      int(hw_silu and act == GLU_SILU), _stream()), "gate_up_tile")
     return out
 
 

@@ -64,7 +64,7 @@ class SwiGLU(Part):
         if ops.gate_up_f32_fits(x, self.gate_up):           # ... in float32
             a = ops.gate_up_f32(x, self.gate_up, self.act)
         elif ops.gate_up_tile_fits(x, self.gate_up):        # some hundred rows: the same in tiles
-            a = ops.gate_up_tile(x, self.gate_up, self.act)
+            a = ops.gate_up_tile(x, self.gate_up, self.act, hw_silu=True)
         else:
             a = ops.silu_mul(linear(x, self.gate_up, blocked=self.gate_up_blocked), self.act)
         if defer_output:                    # (the norm that follows picks the kernels by the rows)

@@ -11,7 +11,7 @@ def i(*values):
     return [("i", v) for v in values]
 
 
-GATE_UP = ("ptl_tile_gate_up", [P, P, P, *i(285, 8192, 2048), ("l", 2048), ("i", 0), ("f", 0.0), NO])
+GATE_UP = ("ptl_tile_gate_up", [P, P, P, *i(285, 8192, 2048), ("l", 2048), ("i", 0), ("f", 0.0), ("i", 0), NO])
 ROWS = ("ptl_rows_gate_up_silu", [P, P, P, *i(64, 8192, 2048), ("l", 2048), ("i", 0), ("f", 0.0), NO])
 EXTRAS = [*i(0, 0, 0), NO, NO, ("l", 0), ("f", 0.0), ("f", 0.1)]
 

@@ -665,6 +665,24 @@ def test_gate_up_tile(ops, mik, act):
     assert (got.double() - want).norm() <= 3e-3 * want.norm()
 
 
+def test_gate_up_tile_has_the_activation_of_the_kernels_beside_it(ops):
+    """Every finite bfloat16 gate (columns of x that W picks out, so the products are exact): SiLU has the bits of the
+    kernel for up to 64 rows, so a feed-forward's result does not get less exact with the 65th row; with ``hw_silu`` the bits
+    of the separate activation kernel, which takes over from 577 rows on."""
+    gates = torch.arange(-2 ** 15, 2 ** 15, dtype=torch.int32).to(torch.int16).view(torch.bfloat16)
+    gates = gates[gates.isfinite()]
+    x = torch.zeros(gates.numel(), 64, dtype=torch.bfloat16)
+    x[:, 0], x[:, 1] = gates, 1.25
+    w = torch.zeros(128, 64, dtype=torch.bfloat16)
+    w[:64, 0], w[64:, 1] = 1.0, 1.0
+    x, w = x.cuda(), w.cuda()
+    blocked = ops.blocked_weight(w)
+    few = torch.cat([ops.gate_up_silu(part, w, blocked=blocked) for part in x.split(60)])
+    assert torch.equal(ops.gate_up_tile(x, w), few)
+    dense = torch.cat([x[:, :1].expand(-1, 64), x[:, 1:2].expand(-1, 64)], dim=1).contiguous()
+    assert torch.equal(ops.gate_up_tile(x, w, hw_silu=True), ops.silu_mul(dense))
+
+
 @pytest.mark.parametrize("mik", [(1, 4, 4), (3, 36, 100), (8, 8192, 2048), (4, 1000, 1028), (5, 512, 8192), (2, 20, 516),
                                  (7, 2816, 1024)])
 def test_gate_up_f32(ops, mik):
