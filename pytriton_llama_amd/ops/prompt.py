@@ -5,10 +5,8 @@ from __future__ import annotations
 import ctypes
 from typing import Optional
 
-import torch
-
 from . import library
-from .kernels import _check
+from .kernels import _check, _stream
 
 _P, _I, _F = ctypes.c_void_p, ctypes.c_int, ctypes.c_float
 
@@ -20,7 +18,7 @@ ENTRIES = (("blaslt", "ptl_blaslt_gemm_bf16"), ("rope", "ptl_rope_store"), ("gem
 
 class PromptStep(ctypes.Structure):
     _fields_ = ([(n, _I) for n in ("T", "H", "I", "Hq", "Hkv", "D", "page_size", "act", "o_splits", "down_splits",
-                                   "gate_up_tile", "unused")]
+                                   "gate_up_tile", "failed")]
                 + [(n, _P) for n in ("positions", "slots", "y", "residual", "qkv", "mixed", "product", "gate_up", "a")])
 
 
@@ -38,7 +36,8 @@ def entries():
 def prompt_between(table, step: PromptStep, before: Optional[PromptLayer], after: Optional[PromptLayer]) -> None:
     """Launch on torch's current stream what lies between the attentions of two layers; the caller has checked the
     operands and keeps them alive until it returns."""
-    _check(library.load("prompt").ptl_prompt_between(
+    code = library.load("prompt").ptl_prompt_between(
         table, ctypes.byref(step), ctypes.byref(before) if before is not None else None,
-        ctypes.byref(after) if after is not None else None,
-        ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice()))), "prompt_between")
+        ctypes.byref(after) if after is not None else None, _stream())
+    if code:
+        _check(code, f"prompt_between, {ENTRIES[step.failed][1]}" if step.failed >= 0 else "prompt_between")
