@@ -92,7 +92,8 @@ def run(model, h: torch.Tensor, ctx, storage) -> Optional[Tuple[PendingProduct, 
     down_splits = ops.gemm_tile_splits(T, H, I) if ops.gemm_tile_add_rmsnorm_fits(a, ffn.down, residual, norm) else 0
     tile = ops.gate_up_tile_fits(y, ffn.gate_up)
     # q | k | v, a product (or its float32 sums) and gate | up, one after the other in one place: each has been read when
-    # the next is written, so a long step takes no more memory than by the parts
+    # the next is written, so a long step takes no more memory than by the parts, which hold the activation of the block
+    # before where ``mixed`` is held here
     wide = torch.empty(T * max(width, H * max(2 * o_splits, 2 * down_splits, 1), 0 if tile else 2 * I),
                        dtype=torch.bfloat16, device=h.device)
     step = prompt.PromptStep(

@@ -174,6 +174,41 @@ def test_steps_of_prompts_in_native_code_give_the_bits_of_the_parts(cases, lengt
     assert all(torch.equal(a, b) for a, b in zip(with_native, with_parts))
 
 
+@pytest.mark.parametrize("lengths", [(1500, 1571), (400, 301), (200, 40)])
+def test_a_native_step_of_prompts_holds_no_more_memory_than_the_parts(tmp_path, lengths, monkeypatch, gpu_device):
+    """The most that is allocated during a step of two prompts, launched natively and by the parts (where the activation of
+    the block before is held beside the results of the one that runs): rows where the tile products take none, some and all
+    of the products. A kept intermediate of the step would be 0.5 to 6 MB; 64 KB are small tensors."""
+    from pytriton_llama_amd.engine.batch import StepEntry
+    from pytriton_llama_amd.models import prompt_steps
+    from pytriton_llama_amd.weights import write_random_model
+    cfg = dict(tiny("B")[0], hidden_size=512, num_attention_heads=16, num_key_value_heads=4, head_dim=64,
+               intermediate_size=1024, vocab_size=512)
+    write_random_model(cfg, str(tmp_path), seed=4, dtype=torch.bfloat16)
+    seqs = random_sequences(512, lengths, seed=2)
+    native, went, peak, logits = prompt_steps.run, [], [], []
+
+    def counted(*args):
+        done = native(*args)
+        went.append(done is not None)
+        return done
+    for how in (counted, lambda *args: None):
+        monkeypatch.setattr(prompt_steps, "run", how)
+        runner = load_runner(str(tmp_path), torch.bfloat16, 16, 512)
+        for turn in range(2):                   # the first step brings what stays: plans, libraries
+            torch.cuda.synchronize()
+            torch.cuda.reset_peak_memory_stats()
+            held = torch.cuda.memory_allocated()
+            got = runner.step([StepEntry((turn, r), t, [len(t) - 1]) for r, t in seqs.items()])
+            torch.cuda.synchronize()
+            most = torch.cuda.max_memory_allocated() - held
+        peak.append(most)
+        logits.append(got.clone())
+        del runner
+    assert went == [True, True] and torch.equal(*logits)
+    assert peak[0] <= peak[1] + 65536, f"{peak[0]} bytes natively, {peak[1]} by the parts"
+
+
 @pytest.mark.parametrize("dtype", DTYPES, ids=["fp32", "bf16"])
 def test_first_tokens_of_a_sequence(cases, dtype):
     """Positions 0, 1, 2: one token whole, then one by one from an empty cache."""
