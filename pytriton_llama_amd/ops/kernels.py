@@ -738,8 +738,8 @@ def gate_up_tile_fits(x: torch.Tensor, w: torch.Tensor) -> bool:
 def gate_up_tile(x: torch.Tensor, w: torch.Tensor, act: int = GLU_SILU, limit: float = 0.0,
                  hw_silu: bool = False) -> torch.Tensor:
     """act(x Wg^T) * (x Wu^T) for w = [Wg; Wu] ([2I, K]) in one kernel, for some hundred rows (act as for
-    ``gate_up_silu``; csrc/gemm_tile.hip). ``hw_silu``: SiLU by the hardware's exponential and reciprocal, for a caller
-    who took it from ``silu_mul`` otherwise, which does that in bfloat16."""
+    ``gate_up_silu``; csrc/gemm_tile.hip). ``hw_silu``: SiLU as ``silu_mul`` has it, for a caller who took it from there
+    otherwise: by the hardware's exponential and reciprocal for bfloat16 rows of a multiple of 8."""
     if not _tile_x_ok(x, w):
         raise KernelError("gate_up_tile: needs bfloat16 x [M, K] and contiguous w [2 I, K], K a multiple of 64, I of 4, "
                           "16-byte aligned rows")
@@ -748,7 +748,7 @@ def gate_up_tile(x: torch.Tensor, w: torch.Tensor, act: int = GLU_SILU, limit: f
     out = torch.empty((M, I), dtype=torch.bfloat16, device=x.device)
     _check(library.load("gemm_tile").ptl_tile_gate_up(_ptr(out), _ptr(x), _ptr(w), M, I, K, ctypes.c_long(x.stride(0)),
                                                       int(act), ctypes.c_float(limit),
-                                                      int(hw_silu and act == GLU_SILU), _stream()), "gate_up_tile")
+                                                      int(hw_silu and act == GLU_SILU and I % 8 == 0), _stream()), "gate_up_tile")
     return out
 
 
