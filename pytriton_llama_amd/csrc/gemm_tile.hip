@@ -292,10 +292,23 @@ bool bad(const void* y, const void* x, const void* w, int M, int N, int K, long 
 
 }  // namespace
 
+extern "C" int ptl_tile_shapes() { return N_SHAPES; }
+
 // The slices of K that ptl_tile_gemm_sums should leave partial sums of.
 extern "C" int ptl_tile_gemm_splits(int M, int N, int K) {
   if (M <= 0 || N <= 0 || K <= 0 || K % KC) return 1;
   return plan_for(M, N, K, true).splits;
+}
+
+// The products in a tile of the caller's (an index below ptl_tile_shapes()), for tests; the two entries behind it take the
+// plan's. sums != 0: as ptl_tile_gemm_sums, in ``splits`` slices of whole chunks; else as ptl_tile_gate_up (N: I).
+extern "C" int ptl_tile_product(void* y, const void* x, const void* w, int M, int N, int K, long ldx, int sums, int tile,
+                                int splits, int act, float limit, hipStream_t stream) {
+  if (bad(y, x, w, M, N, K, ldx) || splits < 1 || (K / KC) % splits) return PTL_ERR_ARG;
+  TileArgs a{y, (const bf16_t*)x, (const bf16_t*)w, M, N, K, ldx, splits, 0, 0, GluArgs{act, limit}};
+  if (sums) return run<OUT_SUMS>(tile, a, stream);
+  if (splits != 1 || !(glu_ok(act) || act == TILE_SILU_HW)) return PTL_ERR_ARG;
+  return run<OUT_GLU>(tile, a, stream);
 }
 
 // y float32 [splits, M, N] = x [M, K] W^T, one slice of K each (``splits`` as ptl_tile_gemm_splits says).
@@ -305,8 +318,7 @@ extern "C" int ptl_tile_gemm_sums(float* y, const void* x, const void* w, int M,
   if (bad(y, x, w, M, N, K, ldx)) return PTL_ERR_ARG;
   const Plan p = plan_for(M, N, K, true);
   if (splits != p.splits) return PTL_ERR_ARG;
-  return run<OUT_SUMS>(p.shape, TileArgs{y, (const bf16_t*)x, (const bf16_t*)w, M, N, K, ldx, p.splits, 0, 0, GluArgs{0, 0.f}},
-                       stream);
+  return ptl_tile_product(y, x, w, M, N, K, ldx, 1, p.shape, p.splits, GLU_SILU, 0.f, stream);
 }
 
 // out bfloat16 [M, I] = act(x Wg^T) * (x Wu^T) for W = [Wg; Wu] [2 I, K]. K a multiple of 64, I of 4, 16-byte aligned rows.
@@ -314,7 +326,6 @@ extern "C" int ptl_tile_gemm_sums(float* y, const void* x, const void* w, int M,
 extern "C" int ptl_tile_gate_up(void* out, const void* x, const void* w, int M, int I, int K, long ldx, int act,
                                 float limit, int hw_silu, hipStream_t stream) {
   if (bad(out, x, w, M, I, K, ldx) || !glu_ok(act) || (hw_silu && act != GLU_SILU)) return PTL_ERR_ARG;
-  if (hw_silu) act = TILE_SILU_HW;
-  return run<OUT_GLU>(plan_for(M, 2 * I, K, false).shape,
-                      TileArgs{out, (const bf16_t*)x, (const bf16_t*)w, M, I, K, ldx, 1, 0, 0, GluArgs{act, limit}}, stream);
+  return ptl_tile_product(out, x, w, M, I, K, ldx, 0, plan_for(M, 2 * I, K, false).shape, 1, hw_silu ? TILE_SILU_HW : act,
+                          limit, stream);
 }

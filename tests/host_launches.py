@@ -9,6 +9,10 @@ import sys
 
 from pytriton_llama_amd.ops import library
 
+# the tiles of csrc/gemm_tile.hip in their order: rows of x, rows of W, workgroups a compute unit
+TILES = [(64, 64, 2), (64, 128, 1), (128, 64, 1), (96, 128, 1), (128, 128, 1), (160, 128, 1), (192, 128, 1), (128, 192, 1),
+         (96, 256, 1), (112, 256, 1), (128, 256, 1), (144, 256, 1)]
+
 RUNTIME = r"""
 #include <cstdint>
 #include <cstdio>

@@ -174,6 +174,50 @@ def test_steps_of_prompts_in_native_code_give_the_bits_of_the_parts(cases, lengt
     assert all(torch.equal(a, b) for a, b in zip(with_native, with_parts))
 
 
+@pytest.mark.parametrize("heads,kv_heads,head_dim,act", [(16, 4, 64, "silu"), (8, 2, 128, "gelu_tanh"), (16, 4, 80, "silu"),
+                                                         (64, 4, 16, "silu")])
+def test_native_steps_of_prompts_where_products_come_in_slices(tmp_path, heads, kv_heads, head_dim, act, monkeypatch, gpu_device):
+    """As above, at widths whose output and down projections come as several float32 slices, a different number of each, in
+    the place that q | k | v and gate | up share with them: numbers of rows with eight, four and two slices, and both sides of
+    where a product goes to the library (576, 768 and 1,088 rows); head sizes of the matrix-core and of the vector attention."""
+    from pytriton_llama_amd import ops
+    from pytriton_llama_amd.engine.batch import StepEntry
+    from pytriton_llama_amd.models import prompt_steps
+    from pytriton_llama_amd.weights import write_random_model
+    H, I = 1024, 4096
+    cfg = dict(tiny("B")[0], hidden_size=H, num_attention_heads=heads, num_key_value_heads=kv_heads, head_dim=head_dim,
+               intermediate_size=I, vocab_size=512)
+    write_random_model(cfg, str(tmp_path), seed=6, dtype=torch.bfloat16, std=0.03)
+    runner = load_runner(str(tmp_path), torch.bfloat16, 16, 256)
+    assert {prompt_steps._plain(b) for b in runner.model.blocks} == {True}
+    for b in runner.model.blocks:
+        b.feed_forward.act = ops.GLU_GELU_TANH if act == "gelu_tanh" else ops.GLU_SILU
+    native, went = prompt_steps.run, []
+
+    def counted(*args):
+        done = native(*args)
+        went.append(done is not None)
+        return done
+    slices = set()
+    for rows in (65, 130, 285, 532, 576, 577, 768, 769, 1088, 1089):
+        o, down = ops.gemm_tile_splits(rows, H, heads * head_dim), ops.gemm_tile_splits(rows, H, I)
+        slices |= {("o", o), ("down", down)} if rows <= 768 else {("down", down)} if rows <= 1088 else set()
+        seqs = random_sequences(512, (rows - rows // 3, rows // 3), seed=rows)
+        out = []
+        for how in (counted, lambda *args: None):
+            monkeypatch.setattr(prompt_steps, "run", how)
+            out.append([])
+            for cut in (slice(0, None), slice(0, 2)):           # the second step reads the pages that the first wrote
+                entries = [StepEntry((rows, r), t[cut], range(len(t[cut]))) for r, t in seqs.items()]
+                out[-1].append(runner.step(entries).clone())
+            for r in seqs:
+                runner.end((rows, r))
+        assert all(torch.equal(a, b) for a, b in zip(*out)), f"{rows} rows"
+        assert bool(torch.isfinite(out[0][0]).all()) and float(out[0][0].std()) > 0.01
+    assert went == [True, False] * 10
+    assert {("o", 2), ("down", 8), ("down", 4), ("down", 2)} <= slices
+
+
 @pytest.mark.parametrize("lengths", [(1500, 1571), (400, 301), (200, 40)])
 def test_a_native_step_of_prompts_holds_no_more_memory_than_the_parts(tmp_path, lengths, monkeypatch, gpu_device):
     """The most that is allocated during a step of two prompts, launched natively and by the parts (where the activation of

@@ -1,7 +1,7 @@
 """The launchers of the kernel libraries, called without a GPU (host_launches.py)."""
 import pytest
 
-from host_launches import run
+from host_launches import TILES, run
 
 P = ("p", 1 << 20)                     # an aligned address that nothing reads
 NO = ("p", 0)
@@ -44,3 +44,42 @@ def test_a_larger_size_is_asked_for_after_a_smaller_one(tmp_path):
     took = run(tmp_path, "attention", [(d, *generic(h, 1)) for d in (0, 1) for h in (300, 640, 300, 576)])
     assert [t["code"] for t in took] == [0] * 8
     assert len({t["launches"][0]["kernel"] for t in took}) == 1
+
+
+def tile_of(launch):
+    """(rows of x, rows of W) of a launched tile product, from the kernel's template arguments."""
+    inner = launch["kernel"].split("gemm_tile_kernelI")[1]
+    return tuple(int(v) for v in inner.split("Li")[1:3] for v in [v.rstrip("E")])
+
+
+def product(M, N, K, sums, tile, splits):
+    return ("ptl_tile_product", [P, P, P, *i(M, N, K), ("l", K), *i(sums, tile, splits, 0), ("f", 0.0), NO])
+
+
+@pytest.mark.parametrize("sums", [1, 0])
+def test_every_tile_of_the_tile_products(tmp_path, sums):
+    """An index launches its own tile, with no more workgroups than tiles or than the chip holds; refused: an index that
+    is none, slices that are no whole chunks, slices of a gate-up product."""
+    bad = [product(100, 512, 512, sums, len(TILES), 1), product(100, 512, 512, sums, -1, 1),
+           product(100, 512, 512, sums, 0, 0), product(100, 512, 512, sums, 0, 3 if sums else 2)]
+    good = [product(M, N, 512, sums, t, 4 if sums else 1) for t in range(len(TILES)) for M, N in ((65, 132), (1000, 16384))]
+    took = run(tmp_path, "gemm_tile", [(0, *c) for c in [("ptl_tile_shapes", [])] + bad + good])
+    assert took[0]["code"] == len(TILES)
+    assert all(t == {"code": -1, "launches": []} for t in took[1:5])
+    for n, t in enumerate(took[5:]):
+        rows, cols, places = TILES[n // 2]
+        M, N = ((65, 132), (1000, 16384))[n % 2]
+        tiles = -(-M // rows) * -(-N // (cols if sums else cols // 2)) * (4 if sums else 1)
+        assert t["code"] == 0 and len(t["launches"]) == 1 and tile_of(t["launches"][0]) == (rows, cols)
+        assert t["launches"][0]["grid"] == [min(tiles, 256 * places), 1, 1]
+
+
+def test_products_of_every_number_of_rows_launch_a_tile(tmp_path):
+    """Gate-up over the rows it takes at the 1B, 3B and 8B widths: which tiles come up, so that a refit of the plan's times
+    that no longer uses one, or uses it elsewhere, shows here."""
+    calls = [("ptl_tile_gate_up", [P, P, P, *i(M, I, K), ("l", K), ("i", 0), ("f", 0.0), ("i", 1), NO])
+             for I, K, most in ((8192, 2048, 576), (8192, 3072, 576), (14336, 4096, 160)) for M in range(65, most + 1, 7)]
+    took = run(tmp_path, "gemm_tile", [(0, *c) for c in calls])
+    assert all(t["code"] == 0 and len(t["launches"]) == 1 for t in took)
+    used = {tile_of(t["launches"][0]) for t in took}
+    assert used <= {t[:2] for t in TILES} and len(used) >= 6, used

@@ -6,6 +6,7 @@ import pytest
 import torch
 
 import plain_llama
+from host_launches import TILES
 
 pytestmark = pytest.mark.gpu
 
@@ -616,8 +617,9 @@ def test_sum_add_rmsnorm(ops, smn):
                                  (200, 2048, 2048), (285, 2048, 8192), (401, 3072, 3072), (532, 4096, 1536),
                                  (700, 1032, 576), (1024, 2048, 8192), (1088, 3072, 2048)])
 def test_gemm_tile_add_rmsnorm(ops, mnk):
-    """Products of some hundred rows as partial sums over slices of K: rows of x and of W that are no multiple of a
-    tile, one chunk of K, depths with and without slices, more tiles than the chip holds; against a float64 product
+    """Products of some hundred rows as partial sums over slices of K, in the tiles the plan takes for them (six of the
+    twelve; test_every_tile runs all): rows of x and of W that are no multiple of a tile, one chunk of K, depths with and
+    without slices; against a float64 product
     (float32 sums of up to 8,192 exact products: 1e-4), and with the norm behind them against the separate kernels."""
     M, N, K = mnk
     torch.manual_seed(41)
@@ -643,8 +645,8 @@ def test_gemm_tile_add_rmsnorm(ops, mnk):
 @pytest.mark.parametrize("mik", [(1, 4, 64), (65, 8192, 2048), (81, 36, 192), (130, 2048, 2048), (200, 8192, 2048),
                                  (285, 8192, 3072), (400, 1000, 512), (532, 8192, 2048), (576, 14336, 1024)])
 def test_gate_up_tile(ops, mik, act):
-    """Gate and up rows in one tile: columns that are no multiple of a tile, every tile shape the plan takes for
-    these rows, the three activations; against float64 with the two products rounded to bfloat16 (a product on
+    """Gate and up rows in one tile, the one the plan takes for these rows (five of the twelve come up; test_every_tile
+    runs all): columns that are no multiple of a tile, the three activations; against float64 with the two products rounded to bfloat16 (a product on
     the edge of a rounding may fall to the other side: 2^-8 of it, and the same once more for the result's rounding)."""
     M, I, K = mik
     torch.manual_seed(42)
@@ -663,6 +665,42 @@ def test_gate_up_tile(ops, mik, act):
     torch.testing.assert_close(got.double(), want, atol=2e-2, rtol=2e-2)
     # the activation itself: the hardware's exponential and reciprocal are far below the result's rounding
     assert (got.double() - want).norm() <= 3e-3 * want.norm()
+
+
+@pytest.mark.parametrize("sums", [True, False], ids=["sums", "gate_up"])
+@pytest.mark.parametrize("tile", range(len(TILES)), ids=["x".join(map(str, t[:2])) for t in TILES])
+def test_every_tile(ops, tile, sums):
+    """Each tile by its index: one chunk of K with a remainder of rows and columns, slices of one chunk, more tiles than the
+    chip holds (with slices, for the sums). Small whole numbers, so every product is exact in whatever order it is added
+    up and is compared for equality; the activation is SiLU of two exact products (float32, rounded)."""
+    import ctypes
+    rows, cols, places = TILES[tile]
+    cols = cols if sums else cols // 2
+    lib = ops.library.load("gemm_tile")
+    ptr = lambda t: ctypes.c_void_p(t.data_ptr())
+    g = torch.Generator(device="cuda").manual_seed(tile)
+    wide = -(-(places * ops.compute_units("cuda") + 1) // (4 * (4 if sums else 1)))      # tiles along W for more than all places
+    for M, N, K, splits in ((rows + 3, cols - 4, 64, 1), (2 * rows - 5, 2 * cols + 12, 192, 3 if sums else 1),
+                            (3 * rows + 1, (wide - 1) * cols + 4, 512, 4 if sums else 1)):
+        x = torch.randint(-3, 4, (M, K), generator=g, device="cuda").to(torch.bfloat16)
+        w = torch.randint(-3, 4, (N if sums else 2 * N, K), generator=g, device="cuda").to(torch.bfloat16)
+        if not sums:
+            x, w = x / 8, w / 8                              # (gates of some units: neither 0 nor 1 after the sigmoid)
+        want = x.double() @ w.double().T
+        y = torch.full((splits, M, N), float("nan"), device="cuda", dtype=torch.float32 if sums else torch.bfloat16)
+        code = lib.ptl_tile_product(ptr(y), ptr(x), ptr(w), M, N, K, ctypes.c_long(K), int(sums), tile, splits, 0,
+                                    ctypes.c_float(0.0), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+        assert code == 0
+        if sums:
+            at = [slice(s * (K // splits), (s + 1) * (K // splits)) for s in range(splits)]
+            want = torch.stack([x[:, a].double() @ w[:, a].double().T for a in at])
+            assert torch.equal(y.double(), want), f"{M} x {N} x {K}"
+        else:
+            gate, up = want.to(torch.bfloat16).float().chunk(2, dim=1)
+            assert N % 8                            # (silu_mul: the kernel with expf and a division)
+            assert torch.equal(y[0], ops.silu_mul(want.to(torch.bfloat16))), f"{M} x {N} x {K}"
+            exact = gate.double() * torch.sigmoid(gate.double()) * up.double()
+            torch.testing.assert_close(y[0].double(), exact, atol=1e-30, rtol=2 ** -8)
 
 
 def test_gate_up_tile_has_the_activation_of_the_kernels_beside_it(ops):
