@@ -665,17 +665,41 @@ def gemm_rows_add_rmsnorm(x: torch.Tensor, w: torch.Tensor, blocked: torch.Tenso
 
 
 # Rows from which, and up to which, the products of csrc/gemm_tile.hip take a step, against the library's product with the
-# kernel behind it (cold weights, us, one MI355X). A product with the norm behind it, 80 / 285 / 700 rows: output
-# projections 2,048 x 2,048 10.6 / 14.4 / 18.3 against 13.0 / 15.4 / 18.5, 3,072 x 3,072 15.0 / 20.3 / 29.6 against 16.9 / 21.8 /
-# 31.4, 4,096 x 4,096 17.9 / 27.7 / 38.8 against 22.0 / 31.3 / 40.5; at 1,024 rows 21.8 / 38.6 / 51.1 against 22.0 / 37.4 / 49.7.
-# A deep K gains more and longer (2,048 x 8,192, 700 / 1,024 / 1,531 rows: 36 / 48 / 65 against 50 / 56 / 65; 4,096 x 14,336
-# 94 / 121 / 183 against 108 / 138 / 175). Gate-up, 80 / 285 / 532 / 700 rows: 2 x 8,192 x 2,048 20.4 / 30.3 / 41.2 / 56.8
-# against 24.5 / 34.9 / 46.4 / 53.3, 2 x 8,192 x 3,072 27.7 / 43.1 / 60.2 / 81.1 against 31.9 / 47.3 / 64.0 / 71.8; of a larger W the
-# library's large tiles are ahead earlier: 2 x 14,336 x 4,096, 80 / 130 / 200 / 400 rows 54 / 60 / 72 / 117 against 72 / 65 / 71 / 105.
+# kernel behind it (its first proposal, which steps launched kernel by kernel run). Measured inside a step of two prompts
+# of a model of 4 to 14 layers, one of the layer's three products at a time given to the library: by themselves, one
+# after the other, the library's kernels are faster than in a step (2,048 x 2,048 at 284 rows 16.4 us against the tile's 17.7,
+# level in a step). Below: what a layer of the step takes more (+) or less (-) with the tile, us, one MI355X.
+# A product with the norm behind it. A deep K gains most: 2,048 x 8,192 at 96 / 277 / 576 / 768 rows -6.1 / -9.1 / -15 / -8.4,
+# 3,072 x 8,192 -17 / -3.5 / -11 / -14, 4,096 x 14,336 -35 / -27 / -41 / -13, 768 x 2,048 -3.4 / -3.5 / -2.3 / -1.4; 5,120 x 13,824
+# at 900 / 1,024 -12 / +29 and 8,192 x 28,672 by itself at 560 / 640 253 / 326 against 256 / 265, so the bound falls with N.
+# Of a K below 2 N less is left to cut into slices: 2,048 x 2,048 at 96 / 277 / 320 / 360 / 512 / 576 / 768 -3.6 / -0.4 / +1.4 /
+# -3.1 / +0.6 / +1.3 / +1.6, 3,072 x 3,072 at 96 / 277 / 448 / 512 / 560 / 640 / 768 -5.0 / -1.5 / -3.3 / +3.8 / -1.4 / +3.2 /
+# -4.4, 1,536 x 1,536 at 277 / 448 / 768 -0.5 / +2.1 / -0.8, 4,096 x 4,096 at 277 / 576 / 640 / 768 -4.2 / -6.2 / -5.5 / +5.9, 5,120 x 5,120 at 448 / 512 /
+# 532 -5.4 / -5.1 / +6.2, 1,024 x 1,024 at 277 / 576 / 768 -3.3 / -1.7 / -1.1.
 TILE_MIN_ROWS = 65
-TILE_ROWS_SUMS, TILE_ROWS_SUMS_DEEP = 768, 1088           # ..., where K is at least twice N
-TILE_ROWS_GATE_UP, TILE_ROWS_GATE_UP_LARGE = 576, 160     # ..., where W holds more than TILE_LARGE_W elements
-TILE_LARGE_W = 1 << 26
+
+
+def tile_most_rows_sums(N: int, K: int) -> int:
+    """Rows up to which ``gemm_tile_add_rmsnorm`` is the faster way for w [N, K]."""
+    if K >= 2 * N:
+        return min(1088 if K >= 3072 else 768, (17 << 18) // max(N, 1))
+    if K < 4096:
+        return 768
+    return 640 if N <= 4096 else 512
+
+
+# Gate-up with its activation: up to 576 rows of a small w, 448 of one up to 54 M elements, 96 of a larger one, and as
+# long as the largest tiles (144 rows of x, 256 of w) all lie on the chip at once. 2 x 4,096 x 1,024 at 96 / 277 / 576 rows -6.7 /
+# -4.5 / -5.6; 2 x 5,632 x 2,048 at 277 / 512 / 576 -4.6 / -3.6 / +4.4; 2 x 8,192 x 2,048 at 96 / 160 / 277 / 448 / 480 / 512 -2.0 /
+# -5.0 / -1.7 / +0.2 / +1.3 / +2.7; 2 x 8,192 x 3,072 at 256 / 448 / 512 / 576 -3.5 / -1.0 / +0.8 / +1.5; 2 x 8,960 x 1,536 (70 tiles
+# along w) at 256 / 400 / 448 / 512 -4.4 / +0.5 / +5.9 / +9.4; 2 x 10,240 x 2,560 (80) at 128 / 256 / 420 / 448 +4.5 / -5.7 / -7.5 /
+# +11; 2 x 14,336 x 2,048 (112) at 96 / 256 / 300 -1.7 / +1.0 / +5.9; 2 x 14,336 x 4,096 at 96 / 128 / 160 / 300 -3.4 / +1.4 /
+# +2.2 / +14; 2 x 13,824 x 5,120 at 65 / 96 / 128 / 160 -3.1 / +4.0 / +5.6 / +5.3.
+def tile_most_rows_gate_up(rows_w: int, K: int, units: int) -> int:
+    """Rows up to which ``gate_up_tile`` is the faster way for w [rows_w, K] on a chip of ``units`` compute units."""
+    size = rows_w * K
+    most = 576 if size <= 3 << 23 else 448 if size <= 13 << 22 else 96
+    return min(most, 144 * (units // max(1, -(-rows_w // 256))))
 
 
 def _tile_x_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
@@ -691,7 +715,7 @@ def gemm_tile_add_rmsnorm_fits(x: torch.Tensor, w: torch.Tensor, residual: torch
     """Whether ``gemm_tile_add_rmsnorm`` takes the product and is the faster way for it."""
     M, K = x.shape
     N = w.shape[0]
-    return (TILE_MIN_ROWS <= M <= (TILE_ROWS_SUMS_DEEP if K >= 2 * N else TILE_ROWS_SUMS) and _tile_x_ok(x, w)
+    return (TILE_MIN_ROWS <= M <= tile_most_rows_sums(N, K) and _tile_x_ok(x, w)
             and _sum_norm_ok(x, N, residual, norm_weight))
 
 
@@ -731,8 +755,8 @@ def gemm_tile_add_rmsnorm(x: torch.Tensor, w: torch.Tensor, residual: torch.Tens
 
 def gate_up_tile_fits(x: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether ``gate_up_tile`` takes x and is the faster way for it."""
-    most = TILE_ROWS_GATE_UP_LARGE if w.numel() > TILE_LARGE_W else TILE_ROWS_GATE_UP
-    return TILE_MIN_ROWS <= x.shape[0] <= most and _tile_x_ok(x, w)
+    return (x.shape[0] >= TILE_MIN_ROWS and _tile_x_ok(x, w)
+            and x.shape[0] <= tile_most_rows_gate_up(w.shape[0], w.shape[1], compute_units(x.device)))
 
 
 def gate_up_tile(x: torch.Tensor, w: torch.Tensor, act: int = GLU_SILU, limit: float = 0.0,
