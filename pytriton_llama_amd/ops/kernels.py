@@ -722,7 +722,8 @@ def gemm_tile_add_rmsnorm_fits(x: torch.Tensor, w: torch.Tensor, residual: torch
 def _sum_norm_ok(x: torch.Tensor, N: int, residual: torch.Tensor, norm_weight: torch.Tensor) -> bool:
     return (residual.dtype == torch.bfloat16 and residual.is_cuda and residual.shape == (x.shape[0], N)
             and residual.is_contiguous() and norm_weight.dtype == torch.float32 and norm_weight.is_cuda
-            and norm_weight.is_contiguous() and norm_weight.numel() == N and N % 8 == 0 and N <= 8192)
+            and norm_weight.is_contiguous() and norm_weight.numel() == N and N % 8 == 0 and N <= 8192
+            and (residual.data_ptr() | norm_weight.data_ptr()) % 16 == 0)
 
 
 def gemm_tile_splits(M: int, N: int, K: int) -> int:

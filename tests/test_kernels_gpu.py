@@ -641,6 +641,27 @@ def test_gemm_tile_add_rmsnorm(ops, mnk):
         ops.gemm_tile_sums(x, w[:, 1:])
 
 
+@pytest.mark.parametrize("rows", [20, 64, 70, 300])
+@pytest.mark.parametrize("shift", [(4, 0), (0, 1), (4, 1), (0, 0)], ids=["residual", "weight", "both", "aligned"])
+def test_a_norm_behind_a_product_with_rows_that_are_not_aligned(ops, rows, shift):
+    """A residual that begins 8 bytes into a buffer (an embedding's own), a norm weight 4 bytes into one (a checkpoint held
+    as one flat buffer): kernels that read 16 bytes at a time leave them to the others."""
+    from pytriton_llama_amd.parts.base import PendingProduct
+    from pytriton_llama_amd.parts.norm import RMSNorm
+    N, K = 512, 1024
+    torch.manual_seed(46)
+    x = torch.randn(rows, K, device="cuda").to(torch.bfloat16)
+    w = (torch.randn(N, K, device="cuda") / math.sqrt(K)).to(torch.bfloat16)
+    res = torch.randn(rows * N + 8, device="cuda").to(torch.bfloat16)[shift[0]:shift[0] + rows * N].view(rows, N)
+    norm = RMSNorm(N, 1e-5)
+    norm.weight = (1.0 + 0.2 * torch.randn(N + 4, device="cuda"))[shift[1]:shift[1] + N]
+    h = (x.double() @ w.double().T).to(torch.bfloat16).double() + res.double()
+    want = h * torch.rsqrt(h.pow(2).mean(-1, keepdim=True) + 1e-5) * norm.weight.double()
+    got, out = norm.forward(PendingProduct(x, w, ops.blocked_weight(w)), res)
+    torch.testing.assert_close(got.double(), want, atol=2e-2, rtol=2e-2)
+    torch.testing.assert_close(out.double(), h, atol=2e-2, rtol=2e-2)
+
+
 @pytest.mark.parametrize("act", ["silu", "gelu_tanh", "clamped"])
 @pytest.mark.parametrize("mik", [(1, 4, 64), (65, 8192, 2048), (81, 36, 192), (130, 2048, 2048), (200, 8192, 2048),
                                  (285, 8192, 3072), (400, 1000, 512), (532, 8192, 2048), (576, 14336, 1024)])
