@@ -19,7 +19,8 @@
 // 128 x 256, 85 for 128 x 128, against 103 and 67); a seventh wave that touches W 6 to 16 chunks ahead (10 to 35 % slower);
 // rows of x and W padded by 64 or 128 columns (level).
 //
-// Measured (one MI355X, cold weights, us; the library's product and the kernel behind it in brackets): down projection with
+// Measured (one MI355X, cold weights, us, a product over and over, which flatters the library against a step, where it shares
+// the caches with others: ops/kernels.py has the times in a step; the library's product and the kernel behind it in brackets): down projection with
 // sum, residual and norm, 2,048 x 8,192, 80 / 285 / 532 / 1,024 rows: 16.5 / 26.4 / 32.0 / 47.5 (25.3 / 37.0 / 49.0 / 56.0);
 // 3,072 x 8,192 22.7 / 35.0 / 43.3 / 64.4 (44.0 / 40.1 / 56.3 / 71.7); 4,096 x 14,336 34.3 / 54.4 / 75.7 / 121 (49.9 / 85.2 /
 // 119 / 138); output projection, 2,048 x 2,048 10.6 / 14.4 / 17.3 / 21.8 (13.0 / 15.4 / 17.5 / 22.0). Gate-up with SiLU-multiply,

@@ -1,7 +1,6 @@
-// Rows of two matrices on their way through LDS, for products in which both are multiplied from there (gemm_tile.hip in
-// bfloat16, gemm_f32.hip in float32).
+// Rows of two matrices on their way through LDS, for products in which both are multiplied from there (gemm_tile.hip).
 //
-// A chunk is 128 bytes of every row of a tile (64 columns of bfloat16, 32 of float32). Chunks lie in NB buffers; waves
+// A chunk is 128 bytes of every row of a tile (64 columns of bfloat16). Chunks lie in NB buffers; waves
 // that do nothing else bring them, with loads that go from global memory to LDS without a register, NB - 1
 // chunks ahead of the waves that multiply, and run on into the workgroup's next tile while the others store the results
 // of this one. Two reasons for waves of their own. A weight comes from HBM, some 2 us away under load: a workgroup that loaded the
@@ -34,9 +33,6 @@ template <int N> __device__ __forceinline__ void tile_wait_loads_but() {
 
 // s_waitcnt lgkmcnt(0): what the wave has read from LDS is in its registers
 __device__ __forceinline__ void tile_wait_lds() { __builtin_amdgcn_s_waitcnt(0xC07F); }
-
-// byte offset of the 16-byte piece of a row of a chunk
-__device__ __forceinline__ int tile_piece(int row, int piece) { return row * TILE_ROW + 16 * (piece ^ (row & 7)); }
 
 // What a loading wave does (``me``: which of the PW): ``tiles`` tiles of ROWS rows one after the other, ``chunks`` chunks
 // each. rows(i, r): where row r of the workgroup's i-th tile begins (a valid row for every r < ROWS), in bytes, at

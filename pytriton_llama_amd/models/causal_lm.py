@@ -141,8 +141,8 @@ class CausalLM:
         residual, picked = None, False
         last = len(self.schedule) - 1
         # Where few rows want logits (a prompt: its last) the last block gives those rows alone, if it can: of the
-        # output projection on everything is row by row. A 2,048-token prompt, 16 layers of the 1B shape: 4.5 % of
-        # the products' time.
+        # output projection on everything is row by row. A 2,048-token prompt, 16 layers of the 1B shape: 5.6 % of
+        # the layers' operations, 205 us of 3,850 in the products.
         rows = ctx.logit_rows if 0 < ctx.num_logit_rows < h.shape[0] else None
         # (fewer rows than that: the final norm would have the same product by itself)
         every_row = (ctx.logit_rows_are_identity and ctx.num_logit_rows == h.shape[0]

@@ -5,7 +5,8 @@ kernels than they take to run (csrc/prompt.hip). ``run`` goes over the blocks of
 and the mixer's own attention a block where they are the plain decoder's (RMSNorm, attention with rotary positions over
 pages, SwiGLU, bfloat16): the same kernels in the same order with the same operands as the parts launch, so the same bits.
 Everything else stays with the parts, and so does the last block, which may give some rows only. Eight prompts of 277
-tokens in all at the 1B shape: 2.29 -> 1.73 ms, what the kernels take.
+tokens in all at the 1B shape: 2.29 -> 1.69 ms in a row of steps, what the kernels take (one from idle takes 2.24: the host
+issues it in 1.4 to 1.5).
 """
 from __future__ import annotations
 
