@@ -1,23 +1,21 @@
-// y = x W^T in float32 on the matrix cores: row-major x [M, K] (row stride ldx) and W [N, K],
-// float32 products and sums (v_mfma_f32_16x16x4_f32 multiplies and adds in float32, so this is the same
-// true 32-bit arithmetic as the vector-FMA kernel of gemm.hip, in another order).
+// y = x W^T in float32 on the matrix cores: row-major x [M, K] (row stride ldx) and W [N, K]; both are split into three
+// bfloat16 parts, whose products are exact, and the sums are float32 (split_f32.h).
 //
 // All kernels need K % 4 == 0 and 16-byte aligned rows of x and W; everything else stays with the
 // vector-FMA kernel.
 //
 // One order of sums. The bits of a result do not depend on the other rows of x, nor on how many there are, so
 // that a request's float32 results are the same alone and in a batch: all kernels add the products of a result
-// in an order that K alone fixes. The columns are cut into spans of span_width(K) (at most 16). A span's sum is
-// that of its even plus that of its odd blocks of 16 columns; either starts from zero and takes its blocks one
-// after the other, four matrix instructions a block, of which number s multiplies columns 3 - s, 7 - s, 11 - s and
-// 15 - s (a lane loads four consecutive columns at once and hands them to the four instructions). The spans'
-// sums are added in order. Which wave, workgroup or lane computes a span is free. (Measured, in us, against
-// kernels whose order followed M: level at up to 8 rows; 64 x 2,048 x 2,048 19.0 -> 15.0, 700 x 2,048 x 2,048 76 -> 80,
-// 300 x 4,096 x 4,096 116 -> 128, 17 x 16 x 2,048 8.9 -> 10.9; a prompt of 700 tokens and a decode step of four rows at
-// the Llama-3.2-1B shape are level, their errors against 64 bits 1.1e-6 -> 4.1e-7 and 4.5e-7 -> 3.9e-7.)
+// in an order that K alone fixes. The columns are cut into spans of span_width(K) (at most 16), a span into blocks of 32
+// columns. A block's sum starts from zero and takes six matrix instructions; a span's starts from zero and takes its
+// blocks' one after the other; the spans' sums are added in order. Which wave, workgroup or lane computes a span is free.
+// (Measured against the float32 matrix instructions, which add four columns at a time, with sums of even and odd blocks of
+// 16 columns: errors against 64 bits, relative to the result, 2.1e-7 -> 1.0e-7 at K 2,048 and 3.0e-7 -> 1.5e-7 at 8,192;
+// of a 700-token prompt's logits at the Llama-3.2-1B shape 4.2e-7 -> 3.9e-7.)
 #include "common.h"
 #include "device.h"
-#include "mfma_f32.h"
+#include "split_f32.h"
+#include "tile_stream.h"
 
 // columns of a span: 256, doubled until there are no more than 16; 128 of short sums, which have few spans to share
 __host__ __device__ static inline int span_width(int K) {
@@ -27,40 +25,37 @@ __host__ __device__ static inline int span_width(int K) {
 }
 
 // ===========================================================================
-// Few rows of x (M <= 16, a decode step): bound by reading W once. A workgroup owns ROWS rows of W;
-// its waves take the spans, every wave keeps up to 16 KB of W under way (two sets of U
-// loads of 1 KB), and the spans' sums meet in LDS. v_mfma_f32_16x16x4_f32: lane l (ln = l % 16,
-// lg = l / 16) holds A[ln][k = lg] and B[k = lg][ln] and gets D[4 lg + i][ln].
+// Few rows of x (M <= 16, a decode step): bound by reading W once, and next to that by the instructions that split W and
+// x, 52 and 44 for the 2 KB of W that a wave multiplies at a time. A workgroup owns ROWS rows of W; its waves take the spans, and the
+// spans' sums meet in LDS.
 //
-// ROWS 16: A is 16 rows of W x 16 columns, a load instruction reads 64 bytes of each row; B the same
-// columns of 16 rows of x, from L2. Even and odd blocks have sums of their own.
-// ROWS 8: with at most 8 rows of x half of such a tile would be empty, so the tile holds two blocks of
-// 16 columns of the same 8 rows (lanes ln < 8 the even block, ln >= 8 the odd one), of W and of x
-// alike. The products that matter are then D[n < 8][m < 8] and D[n >= 8][m >= 8], the sums of the even and
-// of the odd blocks, and every load instruction, of W and of x, still brings 1 KB that is used. It gives twice
+// ROWS 16: A is 16 rows of W x a block of 32 columns, two load instructions that read 64 bytes of each row; B the same
+// columns of 16 rows of x, from L2.
+// ROWS 8: with at most 8 rows of x half of such a tile would be empty, so the tile holds two blocks of the same 8 rows
+// (lanes ln < 8 the first, ln >= 8 the second), of W and of x alike. The products that matter are then D[n < 8][m < 8]
+// and D[n >= 8][m >= 8], and every load instruction, of W and of x, still brings 1 KB that is used. It gives twice
 // the workgroups. MT tiles of 8 rows of x share the loads of W.
 //
 // gemm_f32_few_kernel reads x again for every tile and takes the sums of any length;
 // gemm_f32_held_kernel keeps x in registers and walks several tiles.
 //
-// Measured (one MI355X, cold weights, us at 4 rows; in brackets the vector-FMA kernel that ran first and
-// gemm_f32_few_kernel): 16,384 x 2,048 26 = 5.2 TB/s (240, 33), 2,048 x 8,192 17 = 4.0 TB/s (922, 18.5),
-// 128,256 x 2,048 171 = 6.1 TB/s (643, 214), 2,048 x 2,048 6.7 (209), 64 x 256 3.6 (25); a decode step of 4 rows at
-// the Llama-3.2-1B shape 1.57 ms (28.2).
+// Measured (one MI355X, cold weights, us at 4 and 16 rows; in brackets on the float32 matrix instructions): 16,384 x 2,048 26.3
+// = 5.1 TB/s, 33.5 (25.8, 34.0), 2,048 x 8,192 18.5 = 3.6 TB/s, 27.7 (16.8, 29.9), 128,256 x 2,048 168 = 6.3 TB/s, 214
+// (166, 228), 2,048 x 2,048 8.8, 10.0 (8.9, 10.2); the product of a decode step of 4 rows at the Llama-3.2-1B shape together 1 % more.
 // ===========================================================================
 
 // A tile's results from the spans' sums in LDS ([span][MT][64 lanes][4], lane and element as in D; of 8-row tiles
 // the two halves).
 template <int ROWS, int MT>
-__device__ __forceinline__ void few_results(float* __restrict__ y, const float* sums, int spans, int M, int N, int n0,
-                                            long ldy) {
+__device__ __forceinline__ void few_results(float* __restrict__ y, const float* __restrict__ x, const float* __restrict__ w,
+                                            const float* sums, int spans, int M, int N, int K, int n0, long ldx, long ldy) {
   for (int i = threadIdx.x; i < ROWS * ROWS * MT; i += blockDim.x) {
     const int n = i % ROWS, m = i / ROWS, t = m / ROWS, j = m % ROWS;
     if (m >= M || n0 + n >= N) continue;
     const float* p = sums + t * 256 + ((n >> 2) * 16 + j) * 4 + (n & 3);
-    constexpr int ODD = (2 * 16 + 8) * 4;          // from D[n][j] to D[n + 8][j + 8]
     float s = 0.f;
-    for (int sp = 0; sp < spans; ++sp, p += MT * 256) s += ROWS == 8 ? p[0] + p[ODD] : p[0];
+    for (int sp = 0; sp < spans; ++sp, p += MT * 256) s += p[0];
+    if (!is_finite(s)) s = plain_dot(x + (size_t)m * ldx, w + (size_t)(n0 + n) * K, K);
     y[(size_t)m * ldy + n0 + n] = s;
   }
 }
@@ -91,18 +86,20 @@ template <int FORM, int ROWS> __device__ __forceinline__ int few_row(const FewOu
 
 // The pairs of an 8-row tile from the spans' sums, added up as few_results does.
 template <int FORM>
-__device__ __forceinline__ void pair_results(float* __restrict__ y, const float* sums, int spans, int M, int tile, long ldy,
+__device__ __forceinline__ void pair_results(float* __restrict__ y, const float* __restrict__ x, const float* __restrict__ w,
+                                             const float* sums, int spans, int M, int N, int K, int tile, long ldx, long ldy,
                                              const FewOut& o) {
   for (int i = threadIdx.x; i < 32; i += blockDim.x) {
     const int n = i & 3, m = i >> 2;
     if (m >= M) continue;
     const float *p = sums + m * 4 + n, *p2 = p + 16 * 4;
-    constexpr int ODD = (2 * 16 + 8) * 4;
     float a = 0.f, b = 0.f;
     for (int sp = 0; sp < spans; ++sp, p += 256, p2 += 256) {
-      a += p[0] + p[ODD];
-      b += p2[0] + p2[ODD];
+      a += p[0];
+      b += p2[0];
     }
+    if (!is_finite(a)) a = plain_dot(x + (size_t)m * ldx, w + (size_t)few_row<FORM, 8>(o, tile, n, N) * K, K);
+    if (!is_finite(b)) b = plain_dot(x + (size_t)m * ldx, w + (size_t)few_row<FORM, 8>(o, tile, n + 4, N) * K, K);
     const int pair = 4 * tile + n;
     if (FORM == FORM_GLU) {
       y[(size_t)m * ldy + pair] = glu_act(o.act, a) * b;
@@ -134,78 +131,114 @@ __device__ __forceinline__ void pair_results(float* __restrict__ y, const float*
   }
 }
 
-template <int ROWS, int MT, int U>
+// Where a lane's columns of x begin, and the column from there of load u: two loads make the eight columns a lane has of
+// a fragment, of 16-row tiles one block, of 8-row tiles two, the first in the lanes ln < 8.
+template <int ROWS> __device__ __forceinline__ int few_first(int ln, int lg) { return 4 * lg + (ROWS == 8 ? 32 * (ln >> 3) : 0); }
+template <int ROWS> __host__ __device__ constexpr int few_column(int u) { return (ROWS == 8 ? 64 : 32) * (u / 2) + 16 * (u % 2); }
+
+// The same of W. In 8-row tiles a load takes whole 128-byte lines, a block of all 8 rows (with the columns of x, half of
+// two blocks, it is 15 % slower: 128,256 x 2,048 164 -> 195 us): its second half comes to the lanes ln >= 8,
+// and few_pair hands the halves over.
+template <int ROWS> __device__ __forceinline__ int few_first_w(int ln, int lg) { return 4 * lg + (ROWS == 8 ? 16 * (ln >> 3) : 0); }
+template <int ROWS> __host__ __device__ constexpr int few_column_w(int u) { return (ROWS == 8 ? 32 : 16) * u; }
+
+// the lower (upper) half of every 16 lanes from ``here``, the other from the lanes 8 away of ``there``
+template <bool LOWER> __device__ __forceinline__ uint32_t half_of(uint32_t here, uint32_t there) {
+  return (uint32_t)__builtin_amdgcn_update_dpp((int)here, (int)there, 0x128, 0xf, LOWER ? 0xc : 0x3, false);
+}
+template <int ROWS> __device__ __forceinline__ Split few_pair(const F4& a, const F4& b) {
+  if (ROWS == 16) return split8(a, b);
+  F4 first, second;
+  first.u = make_uint4(half_of<true>(a.u.x, b.u.x), half_of<true>(a.u.y, b.u.y), half_of<true>(a.u.z, b.u.z),
+                       half_of<true>(a.u.w, b.u.w));
+  second.u = make_uint4(half_of<false>(b.u.x, a.u.x), half_of<false>(b.u.y, a.u.y), half_of<false>(b.u.z, a.u.z),
+                        half_of<false>(b.u.w, a.u.w));
+  return split8(first, second);
+}
+
+// acc += a fragment's products. Of 8-row tiles D[n < 8][m < 8] is the sum of the fragment's first block and
+// D[n >= 8][m >= 8], 40 lanes on, that of the second: added one after the other, in the lanes of the first.
+template <int ROWS> __device__ __forceinline__ void few_add(f32x4_t& acc, const Split& w, const Split& x) {
+  const f32x4_t t = split_dot(w, x);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) acc[i] += t[i];
+  if (ROWS == 8) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const auto other = __builtin_amdgcn_permlane32_swap(__float_as_uint(t[i]), __float_as_uint(t[i]), false, false);
+      acc[i] += __uint_as_float(__builtin_amdgcn_update_dpp(0, other[1], 0x128, 0xf, 0xf, true));   // (rotate by 8 of 16)
+    }
+  }
+}
+
+// R fragments of W and of x are under way, and come in the order in which they are used. (x asked for first and split while
+// W is on its way: 2,048 x 8,192 18.4 -> 20.7.)
+template <int ROWS, int MT, int R, int FORM>
 __global__ void __launch_bounds__(1024)
 gemm_f32_few_kernel(float* __restrict__ y, const float* __restrict__ x, const float* __restrict__ w,
-                    int M, int N, int K, long ldx, long ldy, int width) {
+                    int M, int N, int K, long ldx, long ldy, int width, FewOut out) {
   extern __shared__ float red[];                 // [waves][MT][64][4]: a wave a span
   static_assert((ROWS == 16 && MT == 1) || ROWS == 8, "rows of W a tile");
-  constexpr int KB = ROWS == 8 ? 32 : 16;        // columns of W that one load instruction covers
-  constexpr int H = ROWS == 8 ? 1 : 2;           // sums a lane keeps of a tile
+  static_assert(FORM == FORM_PLAIN || (ROWS == 8 && MT == 1), "pairs lie in 8-row tiles, of up to 8 rows of x");
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, ln = lane & 15, lg = lane >> 4;
-  const int n0 = blockIdx.x * ROWS;
-  const int koff = 4 * lg + (ROWS == 8 ? 16 * (ln >> 3) : 0);
-  const float* wp = w + (size_t)min(n0 + ln % ROWS, N - 1) * K + koff;
+  const int kb = wave * width, ke = min(K, kb + width);
+  const int kx = kb + few_first<ROWS>(ln, lg), kw = kb + few_first_w<ROWS>(ln, lg);
+  const float* wp = w + (size_t)few_row<FORM, ROWS>(out, blockIdx.x, ln % ROWS, N) * K + kw;
   const float* xp[MT];
-  bool xok[MT];
+  int x_end[MT];                                 // (0: no row of x)
 #pragma unroll
   for (int t = 0; t < MT; ++t) {
     const int m = ROWS * t + ln % ROWS;
-    xok[t] = m < M;
-    xp[t] = x + (size_t)min(m, M - 1) * ldx + koff;
+    x_end[t] = m < M ? ke : 0;
+    xp[t] = x + (size_t)min(m, M - 1) * ldx + kx;
   }
-  f32x4_t acc[MT][H];
+  f32x4_t acc[MT];
 #pragma unroll
-  for (int t = 0; t < MT; ++t)
+  for (int t = 0; t < MT; ++t) acc[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  constexpr int FB = few_column<ROWS>(2);        // columns of a fragment
+  F4 wr[R][2], xr[R][MT][2];
+  auto load_w = [&](int r, int k) __attribute__((always_inline)) {     // k: from kb on
 #pragma unroll
-    for (int h = 0; h < H; ++h) acc[t][h] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  const int kb = wave * width;
-  const int ke = min(K, kb + width);
-  // two sets of weight registers: the next U blocks are under way while these are multiplied
-  F4 wa[U], wb[U];
-  auto load_w = [&](F4 (&f)[U], int k) {
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const bool ok = k + KB * u + koff < ke;
-      f[u].u = ok ? load_once(wp + k + KB * u) : zero16();
+    for (int u = 0; u < 2; ++u) {
+      const int at = k + few_column_w<ROWS>(u);
+      wr[r][u].u = kw + at < ke ? load_once(wp + at) : zero16();
     }
   };
-  auto multiply = [&](const F4 (&f)[U], int k) {
-    F4 xf[MT][U];
+  auto load_x = [&](int r, int k) __attribute__((always_inline)) {
 #pragma unroll
-    for (int u = 0; u < U; ++u)
+    for (int t = 0; t < MT; ++t)
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const int at = k + few_column<ROWS>(u);
+        xr[r][t][u].u = kx + at < x_end[t] ? load16(xp[t] + at) : zero16();
+      }
+  };
+  const int fragments = max(0, (ke - kb + FB - 1) / FB);
+  auto load = [&](int r, int f) __attribute__((always_inline)) {
+    load_w(r, FB * f);
+    load_x(r, FB * f);
+  };
+#pragma unroll
+  for (int r = 0; r < R; ++r) load(r, r);
+  for (int f = 0; f < fragments; f += R) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      if (f + r >= fragments) break;
+      const Split s = few_pair<ROWS>(wr[r][0], wr[r][1]);
 #pragma unroll
       for (int t = 0; t < MT; ++t) {
-        const bool ok = xok[t] && k + KB * u + koff < ke;
-        xf[t][u].u = ok ? load16(xp[t] + k + KB * u) : zero16();
+        few_add<ROWS>(acc[t], s, split8(xr[r][t][0], xr[r][t][1]));
+        // (one fragment's parts at a time: there are no registers for more)
+        asm volatile("" : "+v"(acc[t]));
       }
-#pragma unroll
-    for (int u = 0; u < U; ++u)
-#pragma unroll
-      for (int s = 0; s < 4; ++s)
-#pragma unroll
-        for (int t = 0; t < MT; ++t)
-          acc[t][u % H] = __builtin_amdgcn_mfma_f32_16x16x4f32(f[u].f[3 - s], xf[t][u].f[3 - s], acc[t][u % H], 0, 0, 0);
-  };
-  if (kb < ke) load_w(wa, kb);
-  for (int k = kb; k < ke; k += 2 * KB * U) {
-    const int k1 = k + KB * U, k2 = k + 2 * KB * U;
-    if (k1 < ke) load_w(wb, k1);
-    multiply(wa, k);
-    if (k1 >= ke) break;
-    if (k2 < ke) load_w(wa, k2);
-    multiply(wb, k1);
+      if (f + r + R < fragments) load(r, f + r + R);
+    }
   }
 #pragma unroll
-  for (int t = 0; t < MT; ++t) {
-    f32x4_t s = acc[t][0];
-    if (H == 2)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) s[i] += acc[t][H - 1][i];
-    *reinterpret_cast<f32x4_t*>(red + (((size_t)wave * MT + t) * 64 + lane) * 4) = s;
-  }
+  for (int t = 0; t < MT; ++t) *reinterpret_cast<f32x4_t*>(red + (((size_t)wave * MT + t) * 64 + lane) * 4) = acc[t];
   __syncthreads();
-  few_results<ROWS, MT>(y, red, blockDim.x >> 6, M, N, n0, ldy);
+  if (FORM == FORM_PLAIN) few_results<ROWS, MT>(y, x, w, red, blockDim.x >> 6, M, N, K, blockIdx.x * ROWS, ldx, ldy);
+  else pair_results<FORM>(y, x, w, red, blockDim.x >> 6, M, N, K, blockIdx.x, ldx, ldy, out);
 }
 
 // Up to 8 rows (16 of 16-row tiles) with a wave's share of the columns in registers: x [ROWS, KB NB] of every wave
@@ -213,81 +246,102 @@ gemm_f32_few_kernel(float* __restrict__ y, const float* __restrict__ x, const fl
 // is read in the loop: read again for every tile, x comes through the same path from L2 as W does and is as many
 // bytes (128,256 x 2,048, us at 1, 4 and 8 rows: 185, 214, 254; held 161, 171, 177). The next tile's first columns are on their way while a tile's
 // sums are added up, in two buffers, one barrier a tile. SB: load blocks of a span.
+#define RING 2
 template <int ROWS, int NB, int SB, int FORM>
 __global__ void __launch_bounds__(1024)
 gemm_f32_held_kernel(float* __restrict__ y, const float* __restrict__ x, const float* __restrict__ w,
                      int M, int N, int K, long ldx, long ldy, int tiles, FewOut out) {
   static_assert(ROWS == 8 || FORM == FORM_PLAIN, "pairs lie in 8-row tiles");
-  constexpr int KB = ROWS == 8 ? 32 : 16;        // columns of a block (as above)
-  constexpr int H = ROWS == 8 ? 1 : 2;
-  constexpr int U = 4, S = NB / U;               // blocks a turn, turns a tile
+  constexpr int KB = ROWS == 8 ? 32 : 16;        // columns of a load, of all lanes
+  constexpr int F = NB / 2, R = NB > 8 ? RING : 4;   // fragments (two loads) a tile, and under way
   constexpr int EACH = NB / SB;                  // spans of a wave
-  static_assert(S % 2 == 0, "the two sets of registers change places an even number of times a tile");
-  static_assert(NB % SB == 0 && SB % U == 0, "a turn does not cross a span's end, a wave's share ends with a span");
+  static_assert(F % R == 0, "a tile's fragments come into the same registers as the last tile's");
+  static_assert(NB % SB == 0 && SB % 2 == 0, "a wave's share ends with a span, a span with a fragment");
   extern __shared__ float red[];                 // [2][waves][EACH][64][4]
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, ln = lane & 15, lg = lane >> 4;
   const int nwaves = blockDim.x >> 6;
-  const int kb = KB * NB * wave + 4 * lg + (ROWS == 8 ? 16 * (ln >> 3) : 0);
-  const int left = K - kb;                       // this lane's columns of block b are there if KB b < left
+  const int kb = KB * NB * wave + few_first<ROWS>(ln, lg), kw = KB * NB * wave + few_first_w<ROWS>(ln, lg);
+  const int left = K - kb, left_w = K - kw;      // this lane's columns of load b are there if few_column(b) < left
   F4 xf[NB];
   {
     const float* xp = x + (size_t)min(ln % ROWS, M - 1) * ldx + kb;
     const bool row = ln % ROWS < M;
 #pragma unroll
-    for (int b = 0; b < NB; ++b) xf[b].u = row && KB * b < left ? load16(xp + KB * b) : zero16();
+    for (int b = 0; b < NB; ++b) xf[b].u = row && few_column<ROWS>(b) < left ? load16(xp + few_column<ROWS>(b)) : zero16();
   }
-  F4 wa[U], wb[U];
-  auto load_w = [&](F4 (&f)[U], int tile, int b0) __attribute__((always_inline)) {
-    const float* wp = w + (size_t)few_row<FORM, ROWS>(out, tile, ln % ROWS, N) * K + kb;
+  F4 ring[R][2];
+  const float* wp = w + (size_t)few_row<FORM, ROWS>(out, blockIdx.x, ln % ROWS, N) * K + kw;
+  auto load_w = [&](F4 (&to)[2], int f) __attribute__((always_inline)) {
 #pragma unroll
-    for (int u = 0; u < U; ++u) f[u].u = KB * (b0 + u) < left ? load_once(wp + KB * (b0 + u)) : zero16();
+    for (int u = 0; u < 2; ++u) {
+      const int at = few_column_w<ROWS>(2 * f + u);
+      to[u].u = at < left_w ? load_once(wp + at) : zero16();
+    }
   };
-  load_w(wa, blockIdx.x, 0);
+#pragma unroll
+  for (int f = 0; f < R; ++f) load_w(ring[f], f);
   int at = 0;
   for (int tile = blockIdx.x; tile < tiles; tile += gridDim.x, at ^= 1) {
     float* const sums = red + at * nwaves * EACH * 256;
-    f32x4_t acc[H];
+    const bool more = tile + (int)gridDim.x < tiles;
+    f32x4_t acc = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int h = 0; h < H; ++h) acc[h] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    for (int f = 0; f < F; ++f) {
+      Split s = few_pair<ROWS>(ring[f % R][0], ring[f % R][1]);
+      // (the parts take other registers: the next loads go to those that have become free)
+      asm volatile("" : "+v"(s.h.u.x), "+v"(s.h.u.y), "+v"(s.h.u.z), "+v"(s.h.u.w), "+v"(s.m.u.x), "+v"(s.m.u.y),
+                   "+v"(s.m.u.z), "+v"(s.m.u.w), "+v"(s.l.u.x), "+v"(s.l.u.y), "+v"(s.l.u.z), "+v"(s.l.u.w));
+      if (f + R < F) {
+        load_w(ring[f % R], f + R);
+      } else {
+        if (f + R == F) wp = w + (size_t)few_row<FORM, ROWS>(out, min(tile + (int)gridDim.x, tiles - 1), ln % ROWS, N) * K + kw;
+        if (more) load_w(ring[f % R], f + R - F);
+      }
+      // (x is split anew for every tile, and here: kept, or done at once, the parts of NB > 8 loads would not fit into the
+      // registers)
+      if (NB > 8)
 #pragma unroll
-    for (int s = 0; s < S; ++s) {
-      F4 (&cur)[U] = s % 2 ? wb : wa;
-      F4 (&next)[U] = s % 2 ? wa : wb;
-      if (s + 1 < S) load_w(next, tile, U * (s + 1));
-      else if (tile + (int)gridDim.x < tiles) load_w(next, tile + gridDim.x, 0);
-#pragma unroll
-      for (int u = 0; u < U; ++u)
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          acc[u % H] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur[u].f[3 - i], xf[U * s + u].f[3 - i], acc[u % H], 0, 0, 0);
-      if ((s + 1) * U % SB == 0) {               // the end of a span
-        if (H == 2)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) acc[0][i] += acc[H - 1][i];
-        *reinterpret_cast<f32x4_t*>(sums + ((wave * EACH + s * U / SB) * 64 + lane) * 4) = acc[0];
-#pragma unroll
-        for (int h = 0; h < H; ++h) acc[h] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        for (int u = 2 * f; u < 2 * f + 2; ++u)
+          asm volatile("" : "+v"(xf[u].u.x), "+v"(xf[u].u.y), "+v"(xf[u].u.z), "+v"(xf[u].u.w));
+      few_add<ROWS>(acc, s, split8(xf[2 * f], xf[2 * f + 1]));
+      if (NB > 8) asm volatile("" : "+v"(acc));
+      if ((2 * f + 2) % SB == 0) {               // the end of a span
+        *reinterpret_cast<f32x4_t*>(sums + ((wave * EACH + 2 * f / SB) * 64 + lane) * 4) = acc;
+        acc = f32x4_t{0.f, 0.f, 0.f, 0.f};
       }
     }
-    __syncthreads();
-    if (FORM == FORM_PLAIN) few_results<ROWS, 1>(y, sums, nwaves * EACH, M, N, ROWS * tile, ldy);
-    else pair_results<FORM>(y, sums, nwaves * EACH, M, tile, ldy, out);
+    tile_wait_lds();
+    tile_meet();                                 // (the loads of the next tile stay under way)
+    if (FORM == FORM_PLAIN) few_results<ROWS, 1>(y, x, w, sums, nwaves * EACH, M, N, K, ROWS * tile, ldx, ldy);
+    else pair_results<FORM>(y, x, w, sums, nwaves * EACH, M, N, K, tile, ldx, ldy, out);
   }
 }
 
-// x in registers, tiles of ``rows`` rows of W: up to 8 rows of x and 8,192 columns, or 16 and 4,096.
+// Tiles of ``rows`` rows of W, x held in registers (up to 8 rows and 8,192 columns, or 16 and 4,096) where a workgroup
+// walks several of them; where every workgroup has one, x is read no more often by the other kernel, which has twice as many
+// loads of W under way (2,048 x 8,192, 4 rows, 19.1 us held, 18.4 so).
 template <int FORM>
-static int launch_held(float* y, const float* x, const float* w, int M, int N, int K, long ldx, long ldy, int rows,
-                       const FewOut& out, hipStream_t st) {
+static int launch_few(float* y, const float* x, const float* w, int M, int N, int K, long ldx, long ldy, int rows,
+                      const FewOut& out, hipStream_t st) {
   const int cus = compute_units();
   const long blocks = (N + rows - 1) / rows;
-  const int width = span_width(K);
-  // (8 rows: 512 columns a wave where that gives 64 waves a compute unit, else 256)
-  const bool half = rows == 8 && K <= 4096 && blocks * ((K + 511) / 512) < 64L * cus;
+  const int width = span_width(K), spans = (K + width - 1) / width;
+  const bool half = rows == 8 && K <= 4096;      // (256 columns a wave)
   const int share = rows == 8 && !half ? 512 : 256;
   const int waves = (K + share - 1) / share;
-  const long resident = (long)cus * (16 / waves);
-  const long walk = (blocks + resident - 1) / resident;
+  const bool holds = rows == 8 ? M <= 8 && K <= 8192 : K <= 4096;
+  const long resident = holds ? (long)cus * (16 / waves) : 0;
+  const long walk = holds ? (blocks + resident - 1) / resident : 1;
+#define GO(ROWS, MT, FORM)                                                                                            \
+  gemm_f32_few_kernel<ROWS, MT, 4 / MT, FORM><<<(unsigned)blocks, spans * 64, (size_t)spans * MT * 1024, st>>>(       \
+      y, x, w, M, N, K, ldx, ldy, width, out)
+  if (!holds || (rows == 8 && walk == 1)) {
+    if (rows == 16) GO(16, 1, FORM_PLAIN);
+    else if (M <= 8) GO(8, 1, FORM);
+    else GO(8, 2, FORM_PLAIN);
+    return ptl_launch_status();
+  }
+#undef GO
   const unsigned grid = (unsigned)((blocks + walk - 1) / walk);
 #define HELD(ROWS, NB, SB)                                                                                      \
   gemm_f32_held_kernel<ROWS, NB, SB, ROWS == 8 ? FORM : FORM_PLAIN>                                             \
@@ -296,8 +350,6 @@ static int launch_held(float* y, const float* x, const float* w, int M, int N, i
   else if (rows == 16) HELD(16, 16, 16);
   else if (half && width == 128) HELD(8, 8, 4);
   else if (half) HELD(8, 8, 8);
-  else if (width == 128) HELD(8, 16, 4);
-  else if (width == 256) HELD(8, 16, 8);
   else HELD(8, 16, 16);
 #undef HELD
   return ptl_launch_status();
@@ -316,22 +368,8 @@ extern "C" int ptl_gemm_f32_few(float* y, const float* x, const float* w, int M,
   // 11.9, 16,384 x 2,048 54.6 / 39.9). At 32 rows gemm_f32_few_kernel is slower than the tiles below at every size.
   const int cus = compute_units();
   const int rows = M <= 8 || (N + 15) / 16 * 3 < 2L * cus ? 8 : 16;
-  const long blocks = (N + rows - 1) / rows;
-  const int width = span_width(K), spans = (K + width - 1) / width;
-  // x in registers where it fits, up to 512 columns a wave of 8 rows or 256 of 16, 16 waves a compute unit
-  // (16 rows, read again against held: 16,384 x 2,048 43 / 36, 3,072 x 2,048 12.0 / 12.2, 128,256 x 2,048 317 / 230;
-  // not where 8-row tiles are taken for more than 8 rows: 2,048 x 2,048 10.4 / 11.3)
-  if (rows == 8 ? M <= 8 && K <= 8192 : K <= 4096) {
-    return launch_held<FORM_PLAIN>(y, x, w, M, N, K, ldx, ldy, rows, FewOut{}, st);
-  }
-#define GO(ROWS, MT)                                                                                        \
-  gemm_f32_few_kernel<ROWS, MT, 8 / MT><<<(unsigned)blocks, spans * 64, (size_t)spans * MT * 1024, st>>>(y, x, w, M, N, K, \
-                                                                                                       ldx, ldy, width)
-  if (rows == 16) GO(16, 1);
-  else if (M <= 8) GO(8, 1);
-  else GO(8, 2);
-#undef GO
-  return ptl_launch_status();
+  // (16 rows, read again against held: 16,384 x 2,048 43 / 36, 128,256 x 2,048 317 / 230)
+  return launch_few<FORM_PLAIN>(y, x, w, M, N, K, ldx, ldy, rows, FewOut{}, st);
 }
 
 static bool pairs_ok(int M, int K, long ldx, const float* x, const float* w) {
@@ -345,7 +383,7 @@ extern "C" int ptl_gate_up_f32(float* out, const float* x, const float* w, int M
   FewOut o{};
   o.half = I;
   o.act = act;
-  return launch_held<FORM_GLU>(out, x, w, M, 2 * I, K, ldx, I, 8, o, st);
+  return launch_few<FORM_GLU>(out, x, w, M, 2 * I, K, ldx, I, 8, o, st);
 }
 
 // q | k | v = x W^T, q and k rotated; q to q_out [M, Hq D], k and v into the cache pages at ``slots`` (null: nowhere).
@@ -357,77 +395,58 @@ extern "C" int ptl_qkv_rope_store_f32(float* q_out, const float* x, const float*
   if (!pairs_ok(M, K, ldx, x, w) || Hq <= 0 || Hkv <= 0 || D <= 0 || D % 8 || page_size <= 0 || !positions ||
       (slots && (!k_cache || !v_cache)))
     return PTL_ERR_ARG;
-  return launch_held<FORM_QKV>(q_out, x, w, M, (Hq + 2 * Hkv) * D, K, ldx, (long)Hq * D, 8,
+  return launch_few<FORM_QKV>(q_out, x, w, M, (Hq + 2 * Hkv) * D, K, ldx, (long)Hq * D, 8,
                                FewOut{D / 2, 0, positions, slots, inv_freq, k_cache, v_cache, Hq, Hkv, page_size}, st);
 }
 
 // ===========================================================================
-// Many rows of x (a prompt portion): tiles of 64 rows of W x 64 rows of x a workgroup of four waves, each 32 x 32,
-// F32_BK columns of K at a time through LDS, two buffers: the next tile is on its way from memory to registers
-// while this one is multiplied, one barrier a tile. For 16 columns a wave reads four 16-byte fragments a lane and
-// issues 16 matrix instructions of 32 clocks each (mfma_f32.h), so the matrix cores bound it. A wave keeps its
-// results three times, the sums of the even blocks, of the odd blocks and of the spans so far; at the end of a
-// span the first two are added to the third. (Tiles of 128 x 64 and 128 x 128, M 17 to 2,048, N 1,536 to 28,672: at
-// most 5 % faster anywhere, up to 40 % slower.)
+// Many rows of x (a prompt portion), both forms with the order of sums of the kernels above. Where K is a multiple of
+// 32, gemm_f32_stream_kernel: a first kernel splits x into its parts, and waves that do nothing else bring them and W through
+// LDS (tile_stream.h); else gemm_f32_tile_kernel (split_f32.h).
 //
-// A grid of few tiles is cut along K as well (blockIdx.y, a number of spans each): the spans' sums go to a
-// workspace [spans, M, N] and a second kernel adds them in order.
+// A grid of few tiles is cut along K as well (a number of spans a workgroup): the spans' sums go to a workspace
+// [spans, M, N] and another kernel adds them in order.
 //
-// Measured (one MI355X, us; the vector-FMA kernel that ran before in brackets): 700 x 16,384 x 2,048 432 =
-// 109 TFLOP/s (1,386), 700 x 2,048 x 8,192 237 (1,251), 700 x 3,072 x 2,048 115 (370), 64 x 2,048 x 8,192 30.5 (963),
-// 17 x 2,048 x 2,048 13.5 (228). Relative error against 64 bits of a 700-token prompt's logits at the Llama-3.2-1B shape
-// 4.1e-7 (1.5e-6).
+// Measured (one MI355X, cold weights, us, with the kernel that splits x; in brackets tiles of 64 x 64 on the float32 matrix
+// instructions, which ran before): 700 x 16,384 x 2,048 240 = 196 TFLOP/s (472), 700 x 2,048 x 8,192 146 (237), 700 x 3,072 x
+// 2,048 77 (110), 483 x 4,096 x 2,048 57 (94), 64 x 2,048 x 8,192 27 (30), 17 x 2,048 x 2,048 13.5 (13.1); 300 x 200 x 96 in
+// either form 12 (8.6).
 // ===========================================================================
-#define F32_TILE 64
-// (two workgroups a unit asked for: without it the sums go to accumulation registers and the occupancy falls)
+
+// K not a multiple of 32 (700 x 16,384 x 2,048 320 us in this form).
+template <int TA, int TC, bool PARTS>
 __global__ void __launch_bounds__(256, 2)
 gemm_f32_tile_kernel(float* __restrict__ y, const float* __restrict__ x, const float* __restrict__ w,
                      int M, int N, int K, long ldx, long ldy, int tiles_m, int tiles, int width, int k_per_split,
                      float* __restrict__ parts) {
-  constexpr int T = 2;                           // 16 x 16 results of a wave along each side
-  constexpr int L = F32_TILE / 32;               // 16-byte pieces of W and of x a thread loads, of rows 32 apart
-  __shared__ uint4 ws[2][F32_TILE * 8];
-  __shared__ uint4 xs[2][F32_TILE * 8];
+  constexpr int TN = 64 * TA, TM = 16 * TC, EACH = SplitX<TC>::EACH;
+  __shared__ uint4 lds[SplitX<TC>::LDS];
   // Workgroups go to the eight XCDs in turn: each gets a run of tiles, neighbours in the run share
   // rows of W, so that W comes into one L2 once.
   const int per_xcd = (tiles + 7) / 8;
   const int tile = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
   if (tile >= tiles || (int)(blockIdx.x >> 3) >= per_xcd) return;
-  const int n0 = tile / tiles_m * F32_TILE, m0 = tile % tiles_m * F32_TILE;
+  const int n0 = tile / tiles_m * TN, m0 = tile % tiles_m * TM;
   const int kb = blockIdx.y * k_per_split, ke = min(K, kb + k_per_split);
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, ln = lane & 15, lg = lane >> 4;
-  const int wn = 32 * (wave & 1), wm = 32 * (wave >> 1);
-  const int piece = tid & 7, row = tid >> 3;
-  const float* wp[L];
-  const float* xp[L];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, ln = lane & 15, lg = lane >> 4;
+  const int wn = n0 + 16 * TA * wave;
+  const float* wp[TA];
+  const float* xp[EACH];
 #pragma unroll
-  for (int i = 0; i < L; ++i) wp[i] = w + (size_t)min(n0 + row + 32 * i, N - 1) * K + 4 * piece;
+  for (int a = 0; a < TA; ++a) wp[a] = w + (size_t)min(wn + 16 * a + ln, N - 1) * K;
 #pragma unroll
-  for (int i = 0; i < L; ++i) xp[i] = x + (size_t)min(m0 + row + 32 * i, M - 1) * ldx + 4 * piece;
-  uint4 wr[L], xr[L];
-  auto fetch = [&](int k) {
-    const bool ok = k + 4 * piece < ke;
-#pragma unroll
-    for (int i = 0; i < L; ++i) wr[i] = ok ? load16(wp[i] + k) : zero16();
-#pragma unroll
-    for (int i = 0; i < L; ++i) xr[i] = ok ? load16(xp[i] + k) : zero16();
-  };
-  auto put = [&](int b) {
-#pragma unroll
-    for (int i = 0; i < L; ++i) ws[b][f32_piece(row + 32 * i, piece)] = wr[i];
-#pragma unroll
-    for (int i = 0; i < L; ++i) xs[b][f32_piece(row + 32 * i, piece)] = xr[i];
-  };
+  for (int i = 0; i < EACH; ++i) xp[i] = x + (size_t)min(m0 + (int)(threadIdx.x >> 2) + 64 * i, M - 1) * ldx;
   // results [M, N] of row stride ld, from D[n = 4 lg + i][m = ln] of every 16 x 16 tile
-  auto store = [&](float* to, long ld, const f32x4_t (&v)[T][T]) {
+  auto store = [&](float* to, long ld, const f32x4_t (&v)[TA][TC]) __attribute__((always_inline)) {
     const bool four = (N & 3) == 0 && (ld & 3) == 0 && (reinterpret_cast<uintptr_t>(to) & 15) == 0;
+    bool finite = true;
 #pragma unroll
-    for (int c = 0; c < T; ++c) {
-      const int m = m0 + wm + 16 * c + ln;
+    for (int c = 0; c < TC; ++c) {
+      const int m = m0 + 16 * c + ln;
       if (m >= M) continue;
 #pragma unroll
-      for (int a = 0; a < T; ++a) {
-        const int n = n0 + wn + 16 * a + 4 * lg;
+      for (int a = 0; a < TA; ++a) {
+        const int n = wn + 16 * a + 4 * lg;
         float* at = to + (size_t)m * ld + n;
         if (four) {
           if (n < N) *reinterpret_cast<f32x4_t*>(at) = v[a][c];
@@ -436,44 +455,49 @@ gemm_f32_tile_kernel(float* __restrict__ y, const float* __restrict__ x, const f
           for (int i = 0; i < 4; ++i)
             if (n + i < N) at[i] = v[a][c][i];
         }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) finite = finite && is_finite(v[a][c][i]);
       }
     }
+    return finite;
   };
-  f32x4_t acc[2][T][T], sum[T][T];           // acc: of the span's even and of its odd blocks
+  f32x4_t acc[TA][TC], sum[TA][TC];              // of the span, of the spans so far
 #pragma unroll
-  for (int a = 0; a < T; ++a)
+  for (int a = 0; a < TA; ++a)
 #pragma unroll
-    for (int c = 0; c < T; ++c) acc[0][a][c] = acc[1][a][c] = sum[a][c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  fetch(kb);
-  put(0);
-  __syncthreads();
-  int buf = 0;
-  for (int k = kb; k < ke; k += F32_BK, buf ^= 1) {
-    const bool more = k + F32_BK < ke;
-    if (more) fetch(k + F32_BK);
-    f32_multiply16<T, T>(acc, ws[buf], xs[buf], wn, wm, lane);
-    if (!more || (k + F32_BK) % width == 0) {    // the end of a span
+    for (int c = 0; c < TC; ++c) acc[a][c] = sum[a][c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  split_tile<TA, TC>(lds, wp, xp, kb, ke, width, acc, [&](int k) __attribute__((always_inline)) {
+    if (PARTS) {
+      store(parts + (size_t)(k / width) * M * N, N, acc);
+    } else {
 #pragma unroll
-      for (int a = 0; a < T; ++a)
+      for (int a = 0; a < TA; ++a)
 #pragma unroll
-        for (int c = 0; c < T; ++c) {
+        for (int c = 0; c < TC; ++c)
 #pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const float s = acc[0][a][c][i] + acc[1][a][c][i];
-            sum[a][c][i] = parts ? s : sum[a][c][i] + s;
-          }
-          acc[0][a][c] = acc[1][a][c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-        }
-      if (parts) store(parts + (size_t)(k / width) * M * N, N, sum);
+          for (int i = 0; i < 4; ++i) sum[a][c][i] += acc[a][c][i];
     }
-    if (more) put(buf ^ 1);
-    __syncthreads();
+#pragma unroll
+    for (int a = 0; a < TA; ++a)
+#pragma unroll
+      for (int c = 0; c < TC; ++c) acc[a][c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  });
+  if (!PARTS && !store(y, ldy, sum)) {
+    // (a thread's own results, as it stored them)
+#pragma unroll 1
+    for (int c = 0; c < TC; ++c)
+#pragma unroll 1
+      for (int a = 0; a < 4 * TA; ++a) {
+        const int m = m0 + 16 * c + ln, n = wn + 16 * (a >> 2) + 4 * lg + (a & 3);
+        if (m < M && n < N && !is_finite(y[(size_t)m * ldy + n]))
+          y[(size_t)m * ldy + n] = plain_dot(x + (size_t)m * ldx, w + (size_t)n * K, K);
+      }
   }
-  if (!parts) store(y, ldy, sum);
 }
 
 __global__ void __launch_bounds__(256)
-gemm_f32_sum_kernel(float* __restrict__ y, const float* __restrict__ parts, int spans, int M, int N, long ldy) {
+gemm_f32_sum_kernel(float* __restrict__ y, const float* __restrict__ parts, int spans, const float* __restrict__ x,
+                    const float* __restrict__ w, int M, int N, int K, long ldx, long ldy) {
   const long total = (long)M * N;
   if ((N & 3) == 0 && (ldy & 3) == 0 && (reinterpret_cast<uintptr_t>(y) & 15) == 0) {
     const long i = ((long)blockIdx.x * 256 + threadIdx.x) * 4;
@@ -484,7 +508,12 @@ gemm_f32_sum_kernel(float* __restrict__ y, const float* __restrict__ parts, int 
       const float4 v = *reinterpret_cast<const float4*>(parts + (size_t)p * total + i);
       s.x += v.x; s.y += v.y; s.z += v.z; s.w += v.w;
     }
-    *reinterpret_cast<float4*>(y + i / N * ldy + i % N) = s;
+    const long m = i / N, n = i % N;
+    float f[4] = {s.x, s.y, s.z, s.w};
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (!is_finite(f[j])) f[j] = plain_dot(x + m * ldx, w + (n + j) * K, K);
+    *reinterpret_cast<float4*>(y + m * ldy + n) = make_float4(f[0], f[1], f[2], f[3]);
     return;
   }
   for (int j = 0; j < 4; ++j) {
@@ -492,60 +521,374 @@ gemm_f32_sum_kernel(float* __restrict__ y, const float* __restrict__ parts, int 
     if (i >= total) return;
     float s = 0.f;
     for (int p = 0; p < spans; ++p) s += parts[(size_t)p * total + i];
+    if (!is_finite(s)) s = plain_dot(x + i / N * ldx, w + i % N * K, K);
     y[i / N * ldy + i % N] = s;
   }
 }
 
-// Columns that a workgroup takes (a number of spans; all: no second kernel): what a count of the work says is done
-// first. The waves of a workgroup take the four SIMDs of a compute unit, so what counts is the fullest unit: r
-// workgroups, one after the other, at 0.5 TFLOP/s (128 TFLOP/s on 256 units), each with about two
-// steps of F32_BK lost at its start and end; less than three at a time on a unit leave gaps (one alone
-// takes 1.6 times as long). Cuts cost the second kernel and the traffic of the spans' sums, however many they are.
-// Against a sweep of all numbers of cuts (M 17 to 700, N 16 to 28,672, K 512 to 14,336; one MI355X) the plan is
-// within 6 % of the fastest; without cuts 64 x 2,048 x 8,192 takes 140 instead of 31.
-static int columns_a_split(int M, int N, int K) {
-  const int cus = compute_units();
-  const int width = span_width(K), spans = (K + width - 1) / width;
-  const long tiles = (long)((N + F32_TILE - 1) / F32_TILE) * ((M + F32_TILE - 1) / F32_TILE);
-  int best = spans * width;
-  double least = 1e30;
-  for (int splits = 1; splits <= spans; ++splits) {
-    const int per = (spans + splits - 1) / splits * width;
-    if ((long)per * (splits - 1) >= K) continue;
-    const double one = 2.0 * F32_TILE * F32_TILE * (min(per, K) + 2 * F32_BK) / 0.5e12;
-    const double r = (double)((tiles * splits + cus - 1) / cus);
-    double t = one * (r < 4 ? 0.8 * (r + 1) : r + 0.3);
-    if (splits > 1) t += 4e-6 + 4.0 * M * N * (spans + 1) / 6e12;
-    if (t < least) {
-      least = t;
-      best = per;
+// The parts of x for gemm_f32_stream_kernel: [blocks of 32 columns][rows: h | m, 128 bytes][pairs of rows: l | l, 128 bytes],
+// rows of 128 bytes as tile_stream.h has them. One thread eight columns.
+__host__ __device__ static inline size_t split_rows_bytes(int Mp) { return (size_t)Mp * 192; }
+
+__global__ void __launch_bounds__(256)
+split_rows_kernel(unsigned char* __restrict__ out, const float* __restrict__ x, int M, int K, long ldx, int Mp) {
+  const int lg = threadIdx.x & 3, row = blockIdx.x * 64 + (threadIdx.x >> 2), b = blockIdx.y;
+  if (row >= M) return;
+  const float* p = x + (size_t)row * ldx + 32 * b + 4 * lg;
+  F4 u, v;
+  u.u = load16(p);
+  v.u = load16(p + 16);
+  const Split s = split8(u, v);
+  unsigned char* at = out + split_rows_bytes(Mp) * b;
+  *reinterpret_cast<uint4*>(at + (size_t)row * 128 + 16 * lg) = s.h.u;
+  *reinterpret_cast<uint4*>(at + (size_t)row * 128 + 64 + 16 * lg) = s.m.u;
+  *reinterpret_cast<uint4*>(at + (size_t)Mp * 128 + (size_t)row * 64 + 16 * lg) = s.l.u;
+}
+
+struct StreamArgs {
+  float *y, *parts;               // parts: of the spans, where K is cut
+  const float *x, *w;
+  const unsigned char* xs;
+  int M, N, K, Mp;
+  long ldx, ldy;
+  int tiles_m, tiles_n, splits, per, width;
+};
+
+// Tiles of BM rows of x and BN of W; four waves multiply, each all rows of x and a quarter of W's, PW bring the operands, a block
+// of 32 columns at a time into one of NB buffers. W lies in LDS as it is in memory and is split by the wave that
+// wants it, a block ahead, between the products of the block before: 11 instructions for a pair of
+// numbers, where every matrix instruction leaves room for about one. The sums of a 16 x 16 tile are added
+// while the next tile's are on their way. What bounds it: a block of 128 x 128 takes 0.98 us a workgroup where 96 matrix instructions
+// of 18 clocks take 0.72, and 1.23 with all compute units at work, 40 KB from L2 each. (Without the
+// order by hand the compiler moves the splitting and the sums behind all products of the block: 1.11 us; with two
+// loading waves 700 x 16,384 x 2,048 takes 284 us, with four 240; x split by every workgroup 308 at best.)
+template <int BM, int BN, int NB, int PW, bool PARTS>
+__global__ void __launch_bounds__(64 * (4 + PW))
+gemm_f32_stream_kernel(const StreamArgs a) {
+  constexpr int TM = BM / 16, TN = BN / 64;
+  constexpr int ROWS = BN + BM + BM / 2, CHUNK = ROWS * TILE_ROW;
+  extern __shared__ __align__(16) unsigned char lds[];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  const int M = a.M, N = a.N, K = a.K;
+  const int total = a.tiles_m * a.tiles_n * a.splits, G = gridDim.x;
+  const int run = G >> 3, rest = G & 7, xcd = blockIdx.x & 7;
+  const int first_tile = xcd * run + min(xcd, rest) + (blockIdx.x >> 3);
+  const int my_tiles = (total - first_tile + G - 1) / G;
+  auto place = [&](int t, int& m0, int& n0, int& kb, int& chunks) __attribute__((always_inline)) {
+    const int each = a.tiles_m * a.tiles_n, split = t / each, u = t - split * each;
+    const int tn = u / a.tiles_m;
+    n0 = tn * BN;
+    m0 = (u - tn * a.tiles_m) * BM;
+    kb = split * a.per;
+    chunks = (min(K, kb + a.per) - kb) / SPLIT_BK;
+  };
+
+  if (wave >= 4) {
+    constexpr int LI = ROWS / 8 / PW;
+    static_assert(ROWS % (8 * PW) == 0 && (NB - 2) * LI < 64, "loads are counted in six bits");
+    const int lrow = lane >> 3, lpiece = (lane & 7) ^ lrow, first = (wave - 4) * LI;
+    const char* src[LI];
+    const long xstep = (long)split_rows_bytes(a.Mp);
+    int all = 0, m0, n0, kb, chunks;
+    for (int n = 0; n < my_tiles; ++n) { place(first_tile + n * G, m0, n0, kb, chunks); all += chunks; }
+    int next = 0, next_tile = 0, left = 0, slot = 0;
+    auto fetch = [&]() __attribute__((always_inline)) {
+      if (left == 0) {
+        place(first_tile + next_tile * G, m0, n0, kb, left);
+        ++next_tile;
+        const unsigned char* xb = a.xs + (size_t)(kb / SPLIT_BK) * xstep;
+#pragma unroll
+        for (int i = 0; i < LI; ++i) {
+          const int r = 8 * (first + i) + lrow;
+          const char* p;
+          if (8 * (first + i) < BN) p = reinterpret_cast<const char*>(a.w + (size_t)min(n0 + r, N - 1) * K + kb);
+          else if (8 * (first + i) < BN + BM) p = reinterpret_cast<const char*>(xb + (size_t)(m0 + r - BN) * 128);
+          else p = reinterpret_cast<const char*>(xb + (size_t)a.Mp * 128 + (size_t)(m0 / 2 + r - BN - BM) * 128);
+          src[i] = p + 16 * lpiece;
+        }
+      }
+      unsigned char* dst = lds + (size_t)slot * CHUNK + 1024 * first;
+#pragma unroll
+      for (int i = 0; i < LI; ++i) {
+        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src[i],
+                                         (__attribute__((address_space(3))) void*)(dst + 1024 * i), 16, 0, 0);
+        src[i] += 8 * (first + i) < BN ? (long)TILE_ROW : xstep;
+      }
+      ++next;
+      --left;
+      slot = slot + 1 == NB ? 0 : slot + 1;
+    };
+    for (int c = 0; c < NB - 1; ++c)
+      if (next < all) fetch();
+    for (int c = 0; c < all; ++c) {
+      // chunks c and c + 1 have landed when at most the chunks after them are still under way
+      switch (max(0, min(NB - 3, all - 2 - c))) {
+        case 0: tile_wait_loads_but<0>(); break;
+        case 1: tile_wait_loads_but<LI>(); break;
+        default: tile_wait_loads_but<(NB > 4 ? 2 * LI : 0)>(); break;
+      }
+      tile_meet();                               // chunk c - 1 has been read
+      if (next < all) fetch();
+    }
+    return;
+  }
+
+  const int ln = lane & 15, lg = lane >> 4;
+  const int p0 = 16 * (lg ^ (ln & 7)), p1 = 16 * ((4 + lg) ^ (ln & 7));
+  const int w_at = (wave * 16 * TN + ln) * TILE_ROW, x_at = (BN + ln) * TILE_ROW;
+  const int l_at = (BN + BM + (ln >> 1)) * TILE_ROW + 16 * ((4 * (ln & 1) + lg) ^ ((ln >> 1) & 7));
+  f32x4_t acc[TN][TM], sum[TN][TM];
+  Split wa[TN], wb[TN];
+  F4 wr[TN][2];
+  Split x[2];
+  auto read_x = [&](Split& to, const unsigned char* at, int i) __attribute__((always_inline)) {
+    to.h.u = load16(at + x_at + i * 16 * TILE_ROW + p0);
+    to.m.u = load16(at + x_at + i * 16 * TILE_ROW + p1);
+    to.l.u = load16(at + l_at + i * 8 * TILE_ROW);
+  };
+  auto read_w = [&](const unsigned char* at) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      wr[j][0].u = load16(at + w_at + j * 16 * TILE_ROW + p0);
+      wr[j][1].u = load16(at + w_at + j * 16 * TILE_ROW + p1);
+    }
+  };
+  auto split_pair = [&](Split (&wn)[TN], int q) __attribute__((always_inline)) {        // q: 0 .. 4 TN - 1
+    const int j = q >> 2, e = q & 3;
+    const F4& f = wr[j][e >> 1];
+    uint32_t h, m, l;
+    split2(f.f[2 * (e & 1)], f.f[2 * (e & 1) + 1], h, m, l);
+    (&wn[j].h.u.x)[e] = h;
+    (&wn[j].m.u.x)[e] = m;
+    (&wn[j].l.u.x)[e] = l;
+  };
+  int slot = 0;
+  bool first = true;
+  for (int n = 0; n < my_tiles; ++n) {
+    int m0, n0, kb, chunks;
+    place(first_tile + n * G, m0, n0, kb, chunks);
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int i = 0; i < TM; ++i) acc[j][i] = sum[j][i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    auto store = [&](float* to, long ld, const f32x4_t (&v)[TN][TM]) __attribute__((always_inline)) {
+      const bool four = (N & 3) == 0 && (ld & 3) == 0 && (reinterpret_cast<uintptr_t>(to) & 15) == 0;
+      bool finite = true;
+#pragma unroll
+      for (int i = 0; i < TM; ++i) {
+        const int m = m0 + 16 * i + ln;
+        if (m >= M) continue;
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+          const int c = n0 + 16 * TN * wave + 16 * j + 4 * lg;
+          float* at = to + (size_t)m * ld + c;
+          if (four) {
+            if (c < N) *reinterpret_cast<f32x4_t*>(at) = v[j][i];
+          } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              if (c + e < N) at[e] = v[j][i][e];
+          }
+#pragma unroll
+          for (int e = 0; e < 4; ++e) finite = finite && is_finite(v[j][i][e]);
+        }
+      }
+      return finite;
+    };
+    // one chunk; its weights' parts are in ws, those of the next go to wn
+    auto chunk = [&](int c, Split (&ws)[TN], Split (&wn)[TN]) __attribute__((always_inline)) {
+      tile_meet();
+      const unsigned char* at = lds + (size_t)slot * CHUNK;
+      slot = slot + 1 == NB ? 0 : slot + 1;
+      const unsigned char* after = lds + (size_t)slot * CHUNK;
+      if (first) {
+        read_w(at);
+#pragma unroll
+        for (int q = 0; q < 4 * TN; ++q) split_pair(ws, q);
+        first = false;
+      }
+      read_x(x[0], at, 0);
+      read_w(after);                             // (behind the last chunk: what is there is not used)
+      f32x4_t t[2][TN];
+#pragma unroll
+      for (int i = 0; i < TM; ++i) {
+        __builtin_amdgcn_sched_barrier(0);
+        if (i + 1 < TM) read_x(x[(i + 1) & 1], at, i + 1);
+#pragma unroll
+        for (int j = 0; j < TN; ++j) t[i & 1][j] = split_dot(ws[j], x[i & 1]);
+        if (i > 0)
+#pragma unroll
+          for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[j][i - 1][e] += t[(i - 1) & 1][j][e];
+#pragma unroll
+        for (int q = 4 * TN * i / TM; q < 4 * TN * (i + 1) / TM; ++q) split_pair(wn, q);
+        // (sums and parts are wanted here, between the products: the compiler would put them all behind the loop)
+        if (i > 0)
+#pragma unroll
+          for (int j = 0; j < TN; ++j) asm volatile("" : "+v"(acc[j][i - 1]));
+#pragma unroll
+        for (int q = 4 * TN * i / TM; q < 4 * TN * (i + 1) / TM; ++q)
+          asm volatile("" : "+v"((&wn[q >> 2].h.u.x)[q & 3]), "+v"((&wn[q >> 2].m.u.x)[q & 3]), "+v"((&wn[q >> 2].l.u.x)[q & 3]));
+#pragma unroll
+        for (int g = 0; g < 6 * TN; ++g) {
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+          if (g < 3) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[j][TM - 1][e] += t[(TM - 1) & 1][j][e];
+      if (c + 1 == chunks || (kb + (c + 1) * SPLIT_BK) % a.width == 0) {
+        if (PARTS) store(a.parts + (size_t)((kb + c * SPLIT_BK) / a.width) * M * N, N, acc);
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+          for (int i = 0; i < TM; ++i) {
+            if (!PARTS)
+#pragma unroll
+              for (int e = 0; e < 4; ++e) sum[j][i][e] += acc[j][i][e];
+            acc[j][i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+          }
+      }
+      tile_wait_lds();
+    };
+    for (int c = 0; c < chunks; c += 2) {
+      chunk(c, wa, wb);
+      if (c + 1 < chunks) {
+        chunk(c + 1, wb, wa);
+      } else {
+#pragma unroll
+        for (int j = 0; j < TN; ++j) wa[j] = wb[j];
+      }
+    }
+    if (!PARTS && !store(a.y, a.ldy, sum)) {
+#pragma unroll 1
+      for (int i = 0; i < TM; ++i)
+#pragma unroll 1
+        for (int e = 0; e < 4 * TN; ++e) {
+          const int m = m0 + 16 * i + ln, c = n0 + 16 * TN * wave + 16 * (e >> 2) + 4 * lg + (e & 3);
+          if (m < M && c < N && !is_finite(a.y[(size_t)m * a.ldy + c]))
+            a.y[(size_t)m * a.ldy + c] = plain_dot(a.x + (size_t)m * a.ldx, a.w + (size_t)c * K, K);
+        }
     }
   }
+}
+
+// The tiles there are: rows of x and of W, buffers, workgroups a compute unit, and what one takes, in us: R rounds of
+// workgroups with c blocks of 32 columns each, of which a share f of the chip's places is taken, take
+// R (c (block + full f) + 2). The last one is gemm_f32_tile_kernel's.
+#define STREAM_TILES(T)                       \
+  T(128, 128, 4, 1, 0.98f, 0.27f)             \
+  T(64, 128, 5, 1, 0.65f, 0.08f)              \
+  T(64, 64, 4, 2, 0.44f, 0.33f)
+constexpr int LOADERS = 4;
+
+struct TilePlan {
+  int tile;                                      // of STREAM_TILES, or -1: gemm_f32_tile_kernel
+  int bm, bn;                                    // rows of x and of W a tile
+  int per;                                       // columns a workgroup
+  int per_cu;
+};
+
+static TilePlan tile_plan(int M, int N, int K) {
+  const int cus = compute_units();
+  const int width = span_width(K), spans = (K + width - 1) / width;
+  TilePlan best{};
+  double least = 1e30;
+  auto offer = [&](int tile, int bm, int bn, int per_cu, float block, float full) {
+    const long tiles = (long)((N + bn - 1) / bn) * ((M + bm - 1) / bm);
+    for (int splits = 1; splits <= spans; ++splits) {
+      const int per = (spans + splits - 1) / splits * width;
+      if ((long)per * (splits - 1) >= K) continue;
+      const long places = (long)cus * per_cu, all = tiles * splits, rounds = (all + places - 1) / places;
+      const double c = (min(per, K) + SPLIT_BK - 1) / SPLIT_BK;
+      double t = rounds * (c * (block + full * (double)all / (rounds * places)) + 2.0);
+      if (splits > 1) t += 4.0 + 4.0 * M * N * (spans + 1) / 6e6;
+      if (t < least) {
+        least = t;
+        best = {tile, bm, bn, per, per_cu};
+      }
+    }
+  };
+  if (K % SPLIT_BK == 0) {
+    int n = 0;
+#define T(BM, BN, NB, CU, BLOCK, FULL) offer(n++, BM, BN, CU, BLOCK, FULL);
+    STREAM_TILES(T)
+#undef T
+  } else {
+    offer(-1, 64, 64, 4, 1.3f, 0.35f);
+  }
   return best;
+}
+
+static int padded_rows(int M) { return (M + 127) / 128 * 128; }
+
+// floats of the parts of x
+static long split_rows_floats(const TilePlan& plan, int M, int K) {
+  return plan.tile < 0 ? 0 : (long)(split_rows_bytes(padded_rows(M)) / 4) * (K / SPLIT_BK);
+}
+
+template <int BM, int BN, int NB, bool PARTS> static int launch_stream(const StreamArgs& a, int per_cu, hipStream_t st) {
+  constexpr size_t lds = (size_t)NB * (BN + BM + BM / 2) * TILE_ROW;
+  static LdsAllowance allowance;
+  if (!allowance.ask((const void*)gemm_f32_stream_kernel<BM, BN, NB, LOADERS, PARTS>, lds)) return PTL_ERR_LAUNCH;
+  const long tiles = (long)a.tiles_m * a.tiles_n * a.splits;
+  const unsigned grid = (unsigned)min(tiles, (long)compute_units() * per_cu);
+  gemm_f32_stream_kernel<BM, BN, NB, LOADERS, PARTS><<<grid, 64 * (4 + LOADERS), lds, st>>>(a);
+  return ptl_launch_status();
+}
+
+// work: split_rows_floats, then the spans' sums if K is cut
+static int launch_tiles(float* y, const float* x, const float* w, int M, int N, int K, long ldx, long ldy,
+                        const TilePlan& plan, float* work, hipStream_t st) {
+  const int width = span_width(K), spans = (K + width - 1) / width;
+  const int tiles_m = (M + plan.bm - 1) / plan.bm, tiles_n = (N + plan.bn - 1) / plan.bn;
+  const int splits = (K + plan.per - 1) / plan.per;
+  if ((long)tiles_m * tiles_n * splits > 0x3fffffff) return PTL_ERR_ARG;
+  float* parts = splits > 1 ? work + split_rows_floats(plan, M, K) : nullptr;
+  if (plan.tile < 0) {
+    const long tiles = (long)tiles_m * tiles_n;
+    const dim3 grid((unsigned)((tiles + 7) / 8 * 8), splits);
+    (parts ? gemm_f32_tile_kernel<1, 4, true> : gemm_f32_tile_kernel<1, 4, false>)<<<grid, 256, 0, st>>>(
+        y, x, w, M, N, K, ldx, ldy, tiles_m, (int)tiles, width, plan.per, parts);
+  } else {
+    const int Mp = padded_rows(M);
+    unsigned char* xs = reinterpret_cast<unsigned char*>(work);
+    split_rows_kernel<<<dim3((M + 63) / 64, K / SPLIT_BK), 256, 0, st>>>(xs, x, M, K, ldx, Mp);
+    const StreamArgs a{y, parts, x, w, xs, M, N, K, Mp, ldx, ldy, tiles_m, tiles_n, splits, plan.per, width};
+    int rc = PTL_ERR_ARG, n = 0;
+#define T(BM, BN, NB, CU, BLOCK, FULL)                                                                   \
+  if (plan.tile == n++)                                                                                  \
+    rc = parts ? launch_stream<BM, BN, NB, true>(a, CU, st) : launch_stream<BM, BN, NB, false>(a, CU, st);
+    STREAM_TILES(T)
+#undef T
+    if (rc != PTL_OK) return rc;
+  }
+  if (parts)
+    gemm_f32_sum_kernel<<<(unsigned)(((long)M * N + 1023) / 1024), 256, 0, st>>>(y, parts, spans, x, w, M, N, K, ldx, ldy);
+  return ptl_launch_status();
 }
 
 // floats of workspace ptl_gemm_f32 wants for these sizes (0: none)
 extern "C" long ptl_gemm_f32_workspace(int M, int N, int K) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
+  const TilePlan plan = tile_plan(M, N, K);
   const int width = span_width(K);
-  return columns_a_split(M, N, K) < K ? (long)((K + width - 1) / width) * M * N : 0;
+  return split_rows_floats(plan, M, K) + (plan.per < K ? (long)((K + width - 1) / width) * M * N : 0);
 }
 
-// K % 4 == 0, ldx % 4 == 0, x and w 16-byte aligned. ``parts``: workspace of ptl_gemm_f32_workspace(M, N, K)
+// K % 4 == 0, ldx % 4 == 0, x and w 16-byte aligned. ``work``: workspace of ptl_gemm_f32_workspace(M, N, K)
 // floats, 16-byte aligned (null where that is 0).
 extern "C" int ptl_gemm_f32(float* y, const float* x, const float* w, int M, int N, int K, long ldx, long ldy,
-                            float* parts, hipStream_t st) {
+                            float* work, hipStream_t st) {
   if (M <= 0 || N <= 0) return PTL_OK;
   if (K <= 0 || K % 4 || (M > 1 && ldx % 4) || ldx < K || ldy < N || !aligned16(x) || !aligned16(w)) return PTL_ERR_ARG;
-  const int width = span_width(K), per = columns_a_split(M, N, K);
-  const bool cut = per < K;
-  if (cut && (parts == nullptr || !aligned16(parts))) return PTL_ERR_ARG;
-  const int tiles_m = (M + F32_TILE - 1) / F32_TILE;
-  const long tiles = (long)((N + F32_TILE - 1) / F32_TILE) * tiles_m;
-  if (tiles > 0x3fffffff) return PTL_ERR_ARG;
-  gemm_f32_tile_kernel<<<dim3((unsigned)((tiles + 7) / 8 * 8), (K + per - 1) / per), 256, 0, st>>>(
-      y, x, w, M, N, K, ldx, ldy, tiles_m, (int)tiles, width, per, cut ? parts : nullptr);
-  if (cut)
-    gemm_f32_sum_kernel<<<(unsigned)(((long)M * N + 1023) / 1024), 256, 0, st>>>(y, parts, (K + width - 1) / width, M, N, ldy);
-  return ptl_launch_status();
+  const TilePlan plan = tile_plan(M, N, K);
+  if ((plan.tile >= 0 || plan.per < K) && (work == nullptr || !aligned16(work))) return PTL_ERR_ARG;
+  return launch_tiles(y, x, w, M, N, K, ldx, ldy, plan, work, st);
 }

@@ -31,7 +31,7 @@
 // g' * sigmoid(1.702 g') * (u' + 1). Without a gate: 2: relu(u)^2.
 #include "common.h"
 #include "mfma.h"
-#include "mfma_f32.h"
+#include "split_f32.h"
 #include <math.h>
 
 #define MOE_TM 64
@@ -465,11 +465,10 @@ moe_gemm_kernel(T* __restrict__ out, long ldo, const T* __restrict__ x, long ldx
   }
 }
 
-// The same products in float32 on the matrix cores (K % 4 == 0, aligned rows): 64 sorted rows x 64
-// result columns a workgroup of four waves, each 32 x 32 of every product, F32_BK columns of K at a time
-// through LDS (mfma_f32.h), two buffers, the next step on its way to registers while this one is
-// multiplied. The gate and the up row of a result meet in one lane. 966 pairs of 16 experts of 2,048 x
-// 2,048 (one MI355X, us; the vector form in brackets): gate|up 251 (691), down 139 (419).
+// The same products in float32 on the matrix cores (K % 4 == 0, aligned rows; split_f32.h): 64 sorted rows x 64
+// result columns a workgroup of four waves, a wave all rows and 16 columns of every product, so that the gate and the up row
+// of a result meet in one lane. 966 pairs of 16 experts of 2,048 x 2,048 (one MI355X, us; on the float32 matrix
+// instructions and in the vector form in brackets): gate|up 190 (231, 691), down 107 (130, 419).
 template <int MODE>
 __global__ void __launch_bounds__(256)
 moe_gemm_f32_kernel(float* __restrict__ out, long ldo, const float* __restrict__ x, long ldx, const float* __restrict__ w,
@@ -478,73 +477,46 @@ moe_gemm_f32_kernel(float* __restrict__ out, long ldo, const float* __restrict__
                     const float* __restrict__ wgt, int top, int N, int K, int act, float limit) {
   constexpr bool GATE_UP = MODE == MODE_GATE_UP;
   constexpr bool GATHER = MODE != MODE_DOWN;
-  constexpr int G = GATE_UP ? 2 : 1;
+  constexpr int G = GATE_UP ? 2 : 1, TC = MOE_TM / 16;
+  static_assert(MOE_TM == 64, "a piece of x a thread");
+  __shared__ uint4 lds[SplitX<TC>::LDS];
   const int e = tile_expert[blockIdx.y];
   if (e < 0) return;
-  __shared__ uint4 ws[2][64 * G * 8];
-  __shared__ uint4 xs[2][64 * 8];
   const int row0 = tile_row0[blockIdx.y];
   const int rows = min(MOE_TM, expert_end[e] - row0);
-  const int n0 = blockIdx.x * 64;
   w += (size_t)e * G * N * K;
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int piece = tid & 7, row = tid >> 3;     // of a step's 16-byte pieces, those of rows row + 32 i
-  const float* wp[2 * G];
-  const float* xp[2];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, ln = lane & 15, lg = lane >> 4;
+  const int n0 = blockIdx.x * 64 + 16 * wave;
+  auto x_row = [&](int m) { return x + (size_t)(GATHER ? sorted[row0 + m] / top : row0 + m) * ldx; };
+  const float* wp[G];
 #pragma unroll
-  for (int i = 0; i < 2 * G; ++i)
-    wp[i] = w + ((size_t)(i >> 1) * N + min(n0 + row + 32 * (i & 1), N - 1)) * K + 4 * piece;
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    // (a row past the tile's end repeats the last: its results are not stored)
-    const int at = row0 + min(row + 32 * i, rows - 1);
-    xp[i] = x + (size_t)(GATHER ? sorted[at] / top : at) * ldx + 4 * piece;
-  }
-  uint4 wr[2 * G], xr[2];
-  auto fetch = [&](int k) {
-    const bool ok = k + 4 * piece < K;
-#pragma unroll
-    for (int i = 0; i < 2 * G; ++i) wr[i] = ok ? load16(wp[i] + k) : zero16();
-#pragma unroll
-    for (int i = 0; i < 2; ++i) xr[i] = ok ? load16(xp[i] + k) : zero16();
-  };
-  auto put = [&](int b) {
-#pragma unroll
-    for (int i = 0; i < 2 * G; ++i) ws[b][f32_piece(row + 32 * i, piece)] = wr[i];
-#pragma unroll
-    for (int i = 0; i < 2; ++i) xs[b][f32_piece(row + 32 * i, piece)] = xr[i];
-  };
-  f32x16_t acc[G][1];
+  for (int g = 0; g < G; ++g) wp[g] = w + ((size_t)g * N + min(n0 + ln, N - 1)) * K;
+  // (a row past the tile's end repeats the last: its results are not stored)
+  const float* const xp[1] = {x_row(min((int)threadIdx.x >> 2, rows - 1))};
+  f32x4_t acc[G][TC];
 #pragma unroll
   for (int g = 0; g < G; ++g)
 #pragma unroll
-    for (int i = 0; i < 16; ++i) acc[g][0][i] = 0.f;
-  const int cn = 32 * (wave & 1), cm = 32 * (wave >> 1);
-  int wrow[G];
+    for (int c = 0; c < TC; ++c) acc[g][c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  split_tile<G, TC>(lds, wp, xp, 0, K, (K + SPLIT_BK - 1) / SPLIT_BK * SPLIT_BK, acc, [](int) {});
 #pragma unroll
-  for (int g = 0; g < G; ++g) wrow[g] = 64 * g + cn;
-  const int xrow[1] = {cm};
-  fetch(0);
-  put(0);
-  __syncthreads();
-  int buf = 0;
-  for (int k = 0; k < K; k += F32_BK, buf ^= 1) {
-    const bool more = k + F32_BK < K;
-    if (more) fetch(k + F32_BK);
-    f32_multiply<G, 1>(acc, ws[buf], xs[buf], wrow, xrow, lane);
-    if (more) put(buf ^ 1);
-    __syncthreads();
-  }
-  const int m = cm + (lane & 31), lh = lane >> 5;
-  if (m >= rows) return;
-  const float f = GATHER && wgt ? wgt[sorted[row0 + m]] : 1.f;
-  float* orow = out + (size_t)(row0 + m) * ldo;
+  for (int c = 0; c < TC; ++c) {
+    const int m = 16 * c + ln;
+    if (m >= rows) continue;
+    const float f = GATHER && wgt ? wgt[sorted[row0 + m]] : 1.f;
+    float* orow = out + (size_t)(row0 + m) * ldo;
 #pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    const int n = n0 + cn + 8 * (i >> 2) + 4 * lh + (i & 3);
-    if (n >= N) continue;
-    orow[n] = GATE_UP ? gated_act(act, acc[0][0][i] * f, acc[G - 1][0][i] * f, limit)
-                      : (MODE == MODE_UP ? unary_act(act, acc[0][0][i] * f) : acc[0][0][i]);
+    for (int i = 0; i < 4; ++i) {
+      const int n = n0 + 4 * lg + i;
+      if (n >= N) continue;
+      float v[G];
+#pragma unroll
+      for (int g = 0; g < G; ++g) {
+        v[g] = acc[g][c][i];
+        if (!is_finite(v[g])) v[g] = plain_dot(x_row(m), w + ((size_t)g * N + n) * K, K);
+      }
+      orow[n] = GATE_UP ? gated_act(act, v[0] * f, v[G - 1] * f, limit) : (MODE == MODE_UP ? unary_act(act, v[0] * f) : v[0]);
+    }
   }
 }
 

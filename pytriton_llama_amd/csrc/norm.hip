@@ -105,6 +105,42 @@ add_rmsnorm_bf16_vec_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x
   }
 }
 
+// float32 rows whose width is a multiple of 4: a thread CH pieces of 16 bytes, one up to 4,096 columns; residual and
+// weight are asked for with x. At a few rows it is the trip to memory and the two meetings of the waves that count (4 rows
+// of 2,048: 4.65 us, one number at a time through LDS 5.1).
+template <int CH>
+__global__ void __launch_bounds__(1024)
+add_rmsnorm_f32_vec_kernel(float* __restrict__ y, const float* __restrict__ x, float* __restrict__ residual,
+                           const float* __restrict__ w, int H, float eps, int has_residual) {
+  __shared__ float scratch[16];
+  const size_t base = (size_t)blockIdx.x * H;
+  float4 v[CH], g[CH];
+  float ss = 0.f;
+#pragma unroll
+  for (int c = 0; c < CH; ++c) {
+    const int i = 4 * (threadIdx.x + c * blockDim.x);
+    if (i >= H) continue;
+    float4 a = *reinterpret_cast<const float4*>(x + base + i);
+    g[c] = *reinterpret_cast<const float4*>(w + i);
+    if (has_residual) {
+      const float4 r = *reinterpret_cast<const float4*>(residual + base + i);
+      a = make_float4(a.x + r.x, a.y + r.y, a.z + r.z, a.w + r.w);
+      *reinterpret_cast<float4*>(residual + base + i) = a;
+    }
+    v[c] = a;
+    ss += (a.x * a.x + a.y * a.y) + (a.z * a.z + a.w * a.w);
+  }
+  ss = block_sum(ss, scratch);
+  const float rr = 1.0f / sqrtf(ss / (float)H + eps);
+#pragma unroll
+  for (int c = 0; c < CH; ++c) {
+    const int i = 4 * (threadIdx.x + c * blockDim.x);
+    if (i < H)
+      *reinterpret_cast<float4*>(y + base + i) =
+          make_float4(v[c].x * rr * g[c].x, v[c].y * rr * g[c].y, v[c].z * rr * g[c].z, v[c].w * rr * g[c].w);
+  }
+}
+
 extern "C" int ptl_add_rmsnorm(void* y, const void* x, void* residual, const float* w,
                                int T_, int H, float eps, int dtype, hipStream_t stream) {
   if (T_ <= 0) return PTL_OK;
@@ -118,6 +154,16 @@ extern "C" int ptl_add_rmsnorm(void* y, const void* x, void* residual, const flo
     const int has = residual != nullptr;
 #define GO(C) add_rmsnorm_bf16_vec_kernel<C><<<T_, vt, 0, stream>>>(                              \
       (bf16_t*)y, (const bf16_t*)x, (bf16_t*)residual, w, H, eps, has)
+    if (ch <= 1) GO(1); else if (ch == 2) GO(2); else if (ch == 3) GO(3); else GO(4);
+#undef GO
+    return ptl_launch_status();
+  }
+  if (dtype == PTL_DTYPE_F32 && H % 4 == 0 && H <= 4 * 1024 * 4 &&
+      ((uintptr_t)x | (uintptr_t)y | (uintptr_t)residual | (uintptr_t)w) % 16 == 0) {
+    const int pieces = H / 4, threads = pieces >= 1024 ? 1024 : (pieces + 63) / 64 * 64, ch = (pieces + threads - 1) / threads;
+    const int has = residual != nullptr;
+#define GO(C) add_rmsnorm_f32_vec_kernel<C><<<T_, threads, 0, stream>>>(                              \
+      (float*)y, (const float*)x, (float*)residual, w, H, eps, has)
     if (ch <= 1) GO(1); else if (ch == 2) GO(2); else if (ch == 3) GO(3); else GO(4);
 #undef GO
     return ptl_launch_status();

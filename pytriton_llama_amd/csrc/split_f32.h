@@ -1,0 +1,194 @@
+// float32 products on the bfloat16 matrix cores, which do sixteen times the work of the float32 ones in the same time.
+//
+// A float32 number has 24 significant bits, a bfloat16 one 8, with the same exponents: x = h + m + l, h = x rounded to
+// bfloat16, m = x - h rounded, l = x - h - m, and nothing is lost (h takes 8 bits, what is left of the 24 has 16 and a
+// sign, m takes 8 of them, l the other 8). A product of two numbers is then nine products, each exact in float32 (8 x 8
+// bits); the three smallest, m l, l m and l l, are at most 2^-23 of the whole and typically 2^-26, less than the 2^-24 that one
+// addition in float32 rounds off, and are left out. (The splitting of float32 into three bfloat16 parts: Henry, Tang and
+// Heinecke, "Leveraging the bfloat16 Artificial Intelligence Datatype For Higher-Precision Computations", 2019.)
+// The six that are kept are added by the matrix cores from the smallest up, over a block of 32 columns; the blocks' sums
+// are added to the result by vector instructions. A float32 matrix instruction rounds its sum every four columns, this one
+// every 32.
+//
+// What is lost: the last part of numbers below 2^-110 may be too small for bfloat16.
+//
+// What is not finite: inf - inf in the split makes a NaN of every sum that an infinite (or nearly infinite) number enters.
+// Whoever stores a result that is not finite works it out again by plain_dot.
+//
+// v_mfma_f32_16x16x32_bf16: lane l (ln = l % 16, lg = l / 16) holds eight columns of A[ln] and of B[ln] and gets
+// D[4 lg + i][ln]. Which columns a lane group holds is free as long as A and B agree: here 4 lg .. + 3 and 16 + 4 lg .. + 3,
+// which are two loads of 16 bytes that read whole 64-byte pieces of a row.
+#pragma once
+#include <hip/hip_runtime.h>
+
+#include "common.h"
+#include "mfma.h"
+#include "mfma_f32.h"
+
+#define SPLIT_BK 32                    // columns of a block
+
+typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+typedef float f32x2_t __attribute__((ext_vector_type(2)));
+
+struct Split {
+  Frag8 h, m, l;
+};
+
+// two numbers rounded to bfloat16, the first in the low half
+__device__ __forceinline__ uint32_t two_bf16(float a, float b) {
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2_t{a, b}), bf16x2_t));
+}
+
+__device__ __forceinline__ void split2(float a, float b, uint32_t& h, uint32_t& m, uint32_t& l) {
+  h = two_bf16(a, b);
+  a -= __uint_as_float(h << 16);
+  b -= __uint_as_float(h & 0xffff0000u);
+  m = two_bf16(a, b);
+  a -= __uint_as_float(m << 16);
+  b -= __uint_as_float(m & 0xffff0000u);
+  l = two_bf16(a, b);
+}
+
+__device__ __forceinline__ Split split8(const F4& a, const F4& b) {
+  Split s;
+  split2(a.f[0], a.f[1], s.h.u.x, s.m.u.x, s.l.u.x);
+  split2(a.f[2], a.f[3], s.h.u.y, s.m.u.y, s.l.u.y);
+  split2(b.f[0], b.f[1], s.h.u.z, s.m.u.z, s.l.u.z);
+  split2(b.f[2], b.f[3], s.h.u.w, s.m.u.w, s.l.u.w);
+  return s;
+}
+
+// step 0 .. 5 of a block's products: which parts of A and of B, from the smallest up
+template <int STEP> __device__ __forceinline__ f32x4_t split_step(const Split& a, const Split& b, f32x4_t t) {
+  const Frag8& p = STEP == 0 ? a.l : STEP == 2 || STEP == 3 ? a.m : a.h;
+  const Frag8& q = STEP == 1 ? b.l : STEP == 2 || STEP == 4 ? b.m : b.h;
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(p.v, q.v, t, 0, 0, 0);
+}
+
+__device__ __forceinline__ f32x4_t split_dot(const Split& a, const Split& b) {
+  f32x4_t t = {0.f, 0.f, 0.f, 0.f};
+  t = split_step<0>(a, b, t);
+  t = split_step<1>(a, b, t);
+  t = split_step<2>(a, b, t);
+  t = split_step<3>(a, b, t);
+  t = split_step<4>(a, b, t);
+  return split_step<5>(a, b, t);
+}
+
+__device__ __forceinline__ bool is_finite(float v) { return (__float_as_uint(v) & 0x7f800000u) != 0x7f800000u; }
+
+// The sum of K products in float32, one after the other.
+__device__ __forceinline__ float plain_dot(const float* __restrict__ a, const float* __restrict__ b, int K) {
+  float s = 0.f;
+#pragma unroll 1
+  for (int k = 0; k < K; ++k) s = fmaf(a[k], b[k], s);
+  return s;
+}
+
+// Tiles of 64 TA rows of W (or TA times 64 rows of different matrices) x 16 TC rows of x, a workgroup of four waves. A wave
+// takes 16 TA rows of W, which no other wave wants, straight from memory into registers and splits them there, and all rows
+// of x, which all waves want: split once, they lie in LDS as three matrices of bfloat16, two buffers of a block of 32 columns.
+// Memory is two blocks ahead of the products in registers, LDS one; one barrier a block.
+//
+// In LDS a row's part is four 16-byte pieces, piece lg what lane group lg multiplies; they are permuted by (row / 2) % 4, so
+// that eight neighbouring lanes touch every bank once, writing along a row and reading down a column of pieces.
+template <int TC> struct SplitX {
+  static constexpr int ROWS = 16 * TC;
+  static constexpr int EACH = (4 * ROWS + 255) / 256;      // pieces of a block a thread brings: of rows 64 apart
+  static constexpr int PIECES = 4 * ROWS;                  // of one part of a block
+  static constexpr int LDS = 2 * 3 * PIECES;               // uint4
+};
+
+__device__ __forceinline__ int split_piece(int row, int lg) { return 4 * row + (lg ^ ((row >> 1) & 3)); }
+
+// wp[a]: this lane's row of W (ln) of the wave's a-th 16, xp[i]: row threadIdx.x / 4 + 64 i of x; both at column 0. Columns
+// kb .. ke, kb a multiple of the block. done(k, acc): called when the sums of a span are complete, k one past its last block's
+// first column; it has to leave zeros. ``width``: columns of a span, a multiple of the block.
+template <int TA, int TC, typename Done>
+__device__ __forceinline__ void split_tile(uint4* __restrict__ lds, const float* const (&wp)[TA],
+                                           const float* const (&xp)[SplitX<TC>::EACH], int kb, int ke, int width,
+                                           f32x4_t (&acc)[TA][TC], Done done) {
+  constexpr int EACH = SplitX<TC>::EACH, PIECES = SplitX<TC>::PIECES;
+  const int tid = threadIdx.x, lane = tid & 63, ln = lane & 15, lg = lane >> 4;
+  const int xrow = tid >> 2, xlg = tid & 3;
+  const bool brings = SplitX<TC>::ROWS >= 64 || xrow < SplitX<TC>::ROWS;      // (of fewer rows not every thread)
+  F4 wr[TA][2], xr[EACH][2];
+  auto fetch = [&](int k) __attribute__((always_inline)) {
+    const bool whole = k + SPLIT_BK <= ke;                 // (of the workgroup: no branch around every load)
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int kw = k + 16 * h + 4 * lg, kx = k + 16 * h + 4 * xlg;
+      if (whole) {
+#pragma unroll
+        for (int a = 0; a < TA; ++a) wr[a][h].u = load16(wp[a] + kw);
+#pragma unroll
+        for (int i = 0; i < EACH; ++i) xr[i][h].u = load16(xp[i] + kx);
+      } else {
+#pragma unroll
+        for (int a = 0; a < TA; ++a) wr[a][h].u = kw < ke ? load16(wp[a] + kw) : zero16();
+#pragma unroll
+        for (int i = 0; i < EACH; ++i) xr[i][h].u = kx < ke ? load16(xp[i] + kx) : zero16();
+      }
+    }
+  };
+  Split ws[TA];
+  auto put = [&](int b) __attribute__((always_inline)) {
+#pragma unroll
+    for (int a = 0; a < TA; ++a) ws[a] = split8(wr[a][0], wr[a][1]);
+#pragma unroll
+    for (int i = 0; i < EACH; ++i) {
+      const Split s = split8(xr[i][0], xr[i][1]);
+      uint4* at = lds + b * 3 * PIECES + split_piece(xrow + 64 * i, xlg);
+      if (brings) {
+        at[0] = s.h.u;
+        at[PIECES] = s.m.u;
+        at[2 * PIECES] = s.l.u;
+      }
+    }
+  };
+  auto meet = [&]() __attribute__((always_inline)) {       // LDS is written and read; loads from memory stay under way
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0xC07F);
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+  fetch(kb);
+  put(0);
+  if (kb + SPLIT_BK < ke) fetch(kb + SPLIT_BK);
+  meet();
+  int buf = 0;
+  for (int k = kb; k < ke; k += SPLIT_BK, buf ^= 1) {
+    const uint4* xs = lds + buf * 3 * PIECES;
+    Split x[2];                                            // of 16 rows, and of the next
+    auto read = [&](Split& to, int c) __attribute__((always_inline)) {
+      const uint4* at = xs + split_piece(16 * c + ln, lg);
+      to.h.u = at[0];
+      to.m.u = at[PIECES];
+      to.l.u = at[2 * PIECES];
+    };
+    read(x[0], 0);
+#pragma unroll
+    for (int c = 0; c < TC; ++c) {
+      if (c + 1 < TC) read(x[(c + 1) & 1], c + 1);
+      f32x4_t t[TA];
+#pragma unroll
+      for (int a = 0; a < TA; ++a) t[a] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#define STEP(S) _Pragma("unroll") for (int a = 0; a < TA; ++a) t[a] = split_step<S>(ws[a], x[c & 1], t[a]);
+      STEP(0) STEP(1) STEP(2) STEP(3) STEP(4) STEP(5)
+#undef STEP
+#pragma unroll
+      for (int a = 0; a < TA; ++a)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[a][c][i] += t[a][i];
+      __builtin_amdgcn_sched_barrier(0);                   // (or all of x is read at once, into registers that are not there)
+    }
+    const bool more = k + SPLIT_BK < ke;
+    if (!more || (k + SPLIT_BK) % width == 0) done(k);
+    if (more) {
+      put(buf ^ 1);
+      __builtin_amdgcn_sched_barrier(0);                   // (the loads take the registers that have just become free)
+      if (k + 2 * SPLIT_BK < ke) fetch(k + 2 * SPLIT_BK);
+    }
+    meet();
+  }
+}

@@ -157,6 +157,47 @@ def test_gemm_f32_same_bits_alone_and_in_a_batch(ops, nk):
             assert torch.equal(ops.gemm_nt(x[first:first + M], w), want[first:first + M]), (M, first)
 
 
+@pytest.mark.parametrize("mnk", [
+    # the tiles of many rows: one and just over one of every size, an odd and an even number of blocks of 32 columns, one block,
+    # cuts along K with a short last one, N of no whole 16-byte piece, more tiles than the compute units hold at a time
+    (64, 64, 32), (65, 130, 96), (127, 127, 4128), (128, 128, 2080), (129, 257, 64), (300, 66, 8224), (20, 2051, 544),
+    (515, 9001, 160), (1500, 4100, 128)])
+def test_gemm_f32_streamed_tiles(ops, mnk):
+    """Within the bound of test_gemm_f32_matrix_cores, and what is infinite or too large for the bfloat16 parts as the
+    float32 sums have it: in every form of the products."""
+    test_gemm_f32_matrix_cores(ops, mnk)
+    M, N, K = mnk
+    torch.manual_seed(47)
+    x, w = torch.randn(M, K, device="cuda"), torch.randn(N, K, device="cuda")
+    x[M - 1, K // 2] = float("-inf")
+    x[0, 0] = 3.4e38                       # rounds to infinity in bfloat16
+    w[:, 0] *= 1e-3
+    want = x.double() @ w.double().T
+    for rows in {1, min(9, M - 1), M - 1}:
+        y = ops.gemm_nt(x[M - rows:], w)
+        assert torch.equal(y[-1].double(), want[-1])                 # all infinite
+        y = ops.gemm_nt(x[:rows], w).double()
+        bound = (K + 1) * 2.0 ** -24 * (x[:rows].double().abs() @ w.double().abs().T)
+        assert ((y - want[:rows]).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("width", [4, 252, 260, 4096, 4100, 12292, 16384, 16388, 2050])
+def test_add_rmsnorm_f32_widths(ops, width):
+    """Every number of pieces a thread, a last piece alone in its wave, rows beyond the kernel with registers; and rows of
+    any alignment."""
+    torch.manual_seed(48)
+    x, r = torch.randn(3, width, device="cuda"), torch.randn(3, width, device="cuda")
+    w = 1 + 0.1 * torch.randn(width, device="cuda")
+    odd = torch.empty(3 * width + 1, device="cuda")[1:].view(3, width)
+    for a in (x, odd.copy_(x)):
+        res = r.clone()
+        y = ops.add_rmsnorm(a, res, w, 1e-5)
+        s = a.double() + r.double()
+        want = s / torch.sqrt((s * s).mean(-1, keepdim=True) + 1e-5) * w.double()
+        assert torch.equal(res, a + r)
+        torch.testing.assert_close(y.double(), want, atol=1e-5, rtol=1e-5)
+
+
 @pytest.mark.parametrize("sizes", [(1, 36, 8, 3, 2), (70, 132, 66, 2, 1), (200, 64, 130, 5, 2), (9, 30, 20, 4, 2)],
                          ids=["one_row", "65_rows_an_expert", "edges", "unaligned"])
 @pytest.mark.parametrize("gated", [True, False])
