@@ -470,7 +470,7 @@ moe_gemm_kernel(T* __restrict__ out, long ldo, const T* __restrict__ x, long ldx
 // of a result meet in one lane. 966 pairs of 16 experts of 2,048 x 2,048 (one MI355X, us; on the float32 matrix
 // instructions and in the vector form in brackets): gate|up 190 (231, 691), down 107 (130, 419).
 template <int MODE>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(256, 3)
 moe_gemm_f32_kernel(float* __restrict__ out, long ldo, const float* __restrict__ x, long ldx, const float* __restrict__ w,
                     const int32_t* __restrict__ tile_expert, const int32_t* __restrict__ tile_row0,
                     const int32_t* __restrict__ expert_end, const int32_t* __restrict__ sorted,
@@ -498,7 +498,8 @@ moe_gemm_f32_kernel(float* __restrict__ out, long ldo, const float* __restrict__
   for (int g = 0; g < G; ++g)
 #pragma unroll
     for (int c = 0; c < TC; ++c) acc[g][c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  split_tile<G, TC>(lds, wp, xp, 0, K, (K + SPLIT_BK - 1) / SPLIT_BK * SPLIT_BK, acc, [](int) {});
+  split_tile<G, TC>(lds, wp, xp, 0, K, (K + SPLIT_BK - 1) / SPLIT_BK * SPLIT_BK, acc, [](int) {},
+                    (rows + 15) / 16);
 #pragma unroll
   for (int c = 0; c < TC; ++c) {
     const int m = 16 * c + ln;

@@ -88,13 +88,14 @@ __device__ __forceinline__ float plain_dot(const float* __restrict__ a, const fl
 // Tiles of 64 TA rows of W (or TA times 64 rows of different matrices) x 16 TC rows of x, a workgroup of four waves. A wave
 // takes 16 TA rows of W, which no other wave wants, straight from memory into registers and splits them there, and all rows
 // of x, which all waves want: split once, they lie in LDS as three matrices of bfloat16, two buffers of a block of 32 columns.
-// Memory is two blocks ahead of the products in registers, LDS one; one barrier a block.
+// Memory is three blocks ahead of the products, in registers, LDS one; one barrier a block.
 //
 // In LDS a row's part is four 16-byte pieces, piece lg what lane group lg multiplies; they are permuted by (row / 2) % 4, so
 // that eight neighbouring lanes touch every bank once, writing along a row and reading down a column of pieces.
 template <int TC> struct SplitX {
   static constexpr int ROWS = 16 * TC;
-  static constexpr int EACH = (4 * ROWS + 255) / 256;      // pieces of a block a thread brings: of rows 64 apart
+  static_assert(ROWS % 64 == 0, "every thread brings as much");
+  static constexpr int EACH = ROWS / 64;                   // pieces of a block a thread brings: of rows 64 apart
   static constexpr int PIECES = 4 * ROWS;                  // of one part of a block
   static constexpr int LDS = 2 * 3 * PIECES;               // uint4
 };
@@ -103,47 +104,49 @@ __device__ __forceinline__ int split_piece(int row, int lg) { return 4 * row + (
 
 // wp[a]: this lane's row of W (ln) of the wave's a-th 16, xp[i]: row threadIdx.x / 4 + 64 i of x; both at column 0. Columns
 // kb .. ke, kb a multiple of the block. done(k, acc): called when the sums of a span are complete, k one past its last block's
-// first column; it has to leave zeros. ``width``: columns of a span, a multiple of the block.
+// first column; it has to leave zeros. ``width``: columns of a span, a multiple of the block. ``groups``: of the TC 16 rows of x those that
+// are wanted, the first ones (of the workgroup).
 template <int TA, int TC, typename Done>
 __device__ __forceinline__ void split_tile(uint4* __restrict__ lds, const float* const (&wp)[TA],
                                            const float* const (&xp)[SplitX<TC>::EACH], int kb, int ke, int width,
-                                           f32x4_t (&acc)[TA][TC], Done done) {
+                                           f32x4_t (&acc)[TA][TC], Done done, int groups = TC) {
   constexpr int EACH = SplitX<TC>::EACH, PIECES = SplitX<TC>::PIECES;
   const int tid = threadIdx.x, lane = tid & 63, ln = lane & 15, lg = lane >> 4;
   const int xrow = tid >> 2, xlg = tid & 3;
-  const bool brings = SplitX<TC>::ROWS >= 64 || xrow < SplitX<TC>::ROWS;      // (of fewer rows not every thread)
-  F4 wr[TA][2], xr[EACH][2];
-  auto fetch = [&](int k) __attribute__((always_inline)) {
-    const bool whole = k + SPLIT_BK <= ke;                 // (of the workgroup: no branch around every load)
+  F4 wr[2][TA][2], xr[2][EACH][2];
+  // (no branches here: behind one the compiler does not know how many loads are under way, and waits for all)
+  auto fetch = [&](int r, int k) __attribute__((always_inline)) {
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      const int kw = k + 16 * h + 4 * lg, kx = k + 16 * h + 4 * xlg;
-      if (whole) {
+      const int kw = min(k + 16 * h + 4 * lg, ke - 4), kx = min(k + 16 * h + 4 * xlg, ke - 4);
 #pragma unroll
-        for (int a = 0; a < TA; ++a) wr[a][h].u = load16(wp[a] + kw);
+      for (int a = 0; a < TA; ++a) wr[r][a][h].u = load16(wp[a] + kw);
 #pragma unroll
-        for (int i = 0; i < EACH; ++i) xr[i][h].u = load16(xp[i] + kx);
-      } else {
-#pragma unroll
-        for (int a = 0; a < TA; ++a) wr[a][h].u = kw < ke ? load16(wp[a] + kw) : zero16();
-#pragma unroll
-        for (int i = 0; i < EACH; ++i) xr[i][h].u = kx < ke ? load16(xp[i] + kx) : zero16();
-      }
+      for (int i = 0; i < EACH; ++i) xr[r][i][h].u = load16(xp[i] + kx);
     }
   };
   Split ws[TA];
-  auto put = [&](int b) __attribute__((always_inline)) {
+  auto put = [&](int r, int k, int b) __attribute__((always_inline)) {
+    if (k + SPLIT_BK > ke) {                               // columns past the end are zeros in both
 #pragma unroll
-    for (int a = 0; a < TA; ++a) ws[a] = split8(wr[a][0], wr[a][1]);
+      for (int h = 0; h < 2; ++h) {
+#pragma unroll
+        for (int a = 0; a < TA; ++a)
+          if (k + 16 * h + 4 * lg >= ke) wr[r][a][h].u = zero16();
+#pragma unroll
+        for (int i = 0; i < EACH; ++i)
+          if (k + 16 * h + 4 * xlg >= ke) xr[r][i][h].u = zero16();
+      }
+    }
+#pragma unroll
+    for (int a = 0; a < TA; ++a) ws[a] = split8(wr[r][a][0], wr[r][a][1]);
 #pragma unroll
     for (int i = 0; i < EACH; ++i) {
-      const Split s = split8(xr[i][0], xr[i][1]);
+      const Split s = split8(xr[r][i][0], xr[r][i][1]);
       uint4* at = lds + b * 3 * PIECES + split_piece(xrow + 64 * i, xlg);
-      if (brings) {
-        at[0] = s.h.u;
-        at[PIECES] = s.m.u;
-        at[2 * PIECES] = s.l.u;
-      }
+      at[0] = s.h.u;
+      at[PIECES] = s.m.u;
+      at[2 * PIECES] = s.l.u;
     }
   };
   auto meet = [&]() __attribute__((always_inline)) {       // LDS is written and read; loads from memory stay under way
@@ -152,13 +155,15 @@ __device__ __forceinline__ void split_tile(uint4* __restrict__ lds, const float*
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
   };
-  fetch(kb);
-  put(0);
-  if (kb + SPLIT_BK < ke) fetch(kb + SPLIT_BK);
+  fetch(0, kb);
+  fetch(1, kb + SPLIT_BK);
+  put(0, kb, 0);
+  __builtin_amdgcn_sched_barrier(0);
+  fetch(0, kb + 2 * SPLIT_BK);
   meet();
-  int buf = 0;
-  for (int k = kb; k < ke; k += SPLIT_BK, buf ^= 1) {
-    const uint4* xs = lds + buf * 3 * PIECES;
+  // the block at k from buffer b; that behind it is in registers 1 - b
+  auto block = [&](int k, int b) __attribute__((always_inline)) {
+    const uint4* xs = lds + b * 3 * PIECES;
     Split x[2];                                            // of 16 rows, and of the next
     auto read = [&](Split& to, int c) __attribute__((always_inline)) {
       const uint4* at = xs + split_piece(16 * c + ln, lg);
@@ -169,6 +174,7 @@ __device__ __forceinline__ void split_tile(uint4* __restrict__ lds, const float*
     read(x[0], 0);
 #pragma unroll
     for (int c = 0; c < TC; ++c) {
+      if (c >= groups) break;
       if (c + 1 < TC) read(x[(c + 1) & 1], c + 1);
       f32x4_t t[TA];
 #pragma unroll
@@ -182,13 +188,14 @@ __device__ __forceinline__ void split_tile(uint4* __restrict__ lds, const float*
         for (int i = 0; i < 4; ++i) acc[a][c][i] += t[a][i];
       __builtin_amdgcn_sched_barrier(0);                   // (or all of x is read at once, into registers that are not there)
     }
-    const bool more = k + SPLIT_BK < ke;
-    if (!more || (k + SPLIT_BK) % width == 0) done(k);
-    if (more) {
-      put(buf ^ 1);
-      __builtin_amdgcn_sched_barrier(0);                   // (the loads take the registers that have just become free)
-      if (k + 2 * SPLIT_BK < ke) fetch(k + 2 * SPLIT_BK);
-    }
+    if (k + SPLIT_BK >= ke || (k + SPLIT_BK) % width == 0) done(k);
+    put(1 - b, k + SPLIT_BK, 1 - b);                       // (behind the last block: zeros that nobody reads)
+    __builtin_amdgcn_sched_barrier(0);                     // (the loads take the registers that have just become free)
+    fetch(1 - b, k + 3 * SPLIT_BK);
     meet();
+  };
+  for (int k = kb; k < ke; k += 2 * SPLIT_BK) {
+    block(k, 0);
+    if (k + SPLIT_BK < ke) block(k + SPLIT_BK, 1);
   }
 }
