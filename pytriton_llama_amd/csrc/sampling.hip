@@ -19,6 +19,7 @@
 #include "common.h"
 #include "no_alloc.h"
 #include <math.h>
+#include <string.h>
 #include <mutex>
 
 // Two passes so that a row of vocabulary size is read by many workgroups: every
@@ -522,7 +523,11 @@ extern "C" int ptl_sample_top_p(int32_t* out, float* work, int want_probs, const
 // One workgroup reads a row of 128k logits at a small part of what the chip can deliver, and
 // the kernel above passes over the row seven times. Here a row is cut into chunks of 4096
 // logits, a workgroup a chunk, and the passes become kernels:
-//   (1) minmax:  every chunk's largest and smallest finite logit;
+//   (1) scan:    every chunk's largest and smallest finite logit, its sum of exp(x/T - chunk max), and the tokens that the
+//                nucleus can be made of (below);
+//       small:   one workgroup a row draws the token from these, if there are few, and the kernels that
+//                follow leave at once: a model's logits are peaked, and 64 rows of 128,256 have some 300
+//                candidates each. Not for rows with top_p 1 and not if the probabilities are asked for;
 //   (2) hist:    the chunk's sum of e = exp(x/T - max) and its histogram of that mass over 2048
 //                buckets of x, equally wide, from the row's max down to its min (at most 32 T
 //                below the max; what lies further goes to the last bucket). The histogram is
@@ -541,8 +546,9 @@ extern "C" int ptl_sample_top_p(int32_t* out, float* work, int want_probs, const
 // A token is kept iff it lies in a bucket above the crossing one, or in it and above the edge;
 // equal logits are kept or dropped together. e is worked out again from x wherever it is wanted
 // (one multiplication, one exp2, the same bits): keeping it would be a write and a read of the
-// whole row. 64 rows of 128,256 logits (one MI355X): 66 us for the five kernels, 12 to 17 for each of the
-// three passes over the logits; 97 us with e kept, the crossing found by every workgroup of the gather
+// whole row. 64 rows of 128,256 logits (one MI355X): 66 us for the five kernels without small, 12 to 17 for each of the
+// three passes over the logits, of which peaked rows take one: scan 13.6, small 12.6, the others 2 to 3 each, 35 us
+// in all (rows with too many candidates 71); 97 us with e kept, the crossing found by every workgroup of the gather
 // kernel and the last bucket in LDS. If a chunk has more than 256 tokens in the crossing
 // bucket, or the row more than 4096 (many equal logits), the draw kernel bisects over the whole
 // row instead: slower, same result. Everything is added in a fixed order: the same logits,
@@ -563,7 +569,7 @@ struct SwRow {
   int32_t *ccount, *seg_i;
 };
 __host__ __device__ static inline size_t sw_row_words(int S) {
-  return (size_t)5 * S + (size_t)S * SW_BUCKETS + (size_t)2 * S * SW_SEG + 8;
+  return (size_t)5 * S + (size_t)S * SW_BUCKETS + (size_t)2 * S * SW_SEG + 12;
 }
 __device__ __forceinline__ SwRow sw_row(float* ws, int r, int S) {
   float* p = ws + (size_t)r * sw_row_words(S);
@@ -577,7 +583,8 @@ __device__ __forceinline__ SwRow sw_row(float* ws, int r, int S) {
   w.seg_x = p; p += (size_t)S * SW_SEG;
   w.seg_i = reinterpret_cast<int32_t*>(p); p += (size_t)S * SW_SEG;
   w.result = p;        // [0] edge key (bits), [1] crossing bucket (bits), [2] kept mass, [3] mass before
-                       // the crossing bucket, [4] row max, [5] buckets per unit of x, [6] sum of e
+                       // the crossing bucket, [4] row max, [5] buckets per unit of x, [6] sum of e,
+                       // [7] not 0: the token is drawn, [8] temperature, [9] top_p, [10] u
   return w;
 }
 
@@ -620,35 +627,156 @@ __device__ __forceinline__ bool sw_kept(float x, const SwScale& s, int cross, ui
   return b < cross || (b == cross && sw_key(x) > edge);
 }
 
-__global__ void __launch_bounds__(SW_THREADS)
-sw_minmax_kernel(float* __restrict__ ws, const float* __restrict__ logits, int V, long stride, int S) {
-  __shared__ float scratch[16];
-  const int r = blockIdx.y, c = blockIdx.x;
-  const SwRow w = sw_row(ws, r, S);
-  const float* row = logits + (size_t)r * stride;
-  const int lo = c * SW_CHUNK;
-  float mx = -INFINITY, mn = INFINITY;
-#pragma unroll
-  for (int j = 0; j < SW_PER; ++j) {
-    const int i = lo + j * SW_THREADS + threadIdx.x;
-    const float x = i < V ? sw_clean(row[i]) : -INFINITY;
-    mx = fmaxf(mx, x);
-    if (x > -INFINITY) mn = fminf(mn, x);
+// Parameters of the rows of a launch: in device memory, or by value from the host (a copy to the device would be a pinned
+// allocation, a transfer and its place in the stream for 12 bytes a row).
+#define SW_GROUP 64
+struct SwParams {
+  const float *temperature, *top_p, *uniform;      // null: by value
+  float value[SW_GROUP][3];
+};
+__device__ __forceinline__ void sw_params(const SwParams& p, int r, int row0, float& t, float& top, float& u) {
+  if (p.temperature) {
+    t = p.temperature[row0 + r];
+    top = p.top_p[row0 + r];
+    u = p.uniform[row0 + r];
+  } else {
+    t = p.value[r][0];
+    top = p.value[r][1];
+    u = p.value[r][2];
   }
-  mx = block_max(mx, scratch);
-  mn = -block_max(-mn, scratch);
-  if (threadIdx.x == 0) { w.cmax[c] = mx; w.cmin[c] = mn; }
+}
+
+// The larger of two numbers each over the block; scratch holds 16 floats.
+__device__ __forceinline__ void block_max2(float& a, float& b, float* scratch) {
+  a = wave_max(a);
+  b = wave_max(b);
+  const int wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
+  __syncthreads();
+  if ((threadIdx.x & 63) == 0) { scratch[wave] = a; scratch[8 + wave] = b; }
+  __syncthreads();
+  a = scratch[0];
+  b = scratch[8];
+  for (int i = 1; i < nw; ++i) { a = fmaxf(a, scratch[i]); b = fmaxf(b, scratch[8 + i]); }
+}
+
+// A chunk's largest and smallest finite logit and, if ``candidates``, what the row's nucleus can be made of (a token left out
+// has all of a mass above top_p before it). With e = exp(x/T - chunk max), z_c the chunk's sum, z the row's: tokens
+// whose e is below (1 - top_p) z / V have together less than (1 - top_p) z, so the cumulative mass passes top_p above
+// them; z_c is at most z in the same units, and half of that bound leaves room for rounding. Candidates go on in the
+// order of the vocabulary: a thread has four consecutive tokens of each quarter of the chunk, and one scan counts all four quarters.
+__global__ void __launch_bounds__(SW_THREADS)
+sw_scan_kernel(float* __restrict__ ws, const float* __restrict__ logits, int V, long stride, int S, int row0, int candidates,
+               const SwParams params) {
+  constexpr int Q = SW_PER / 4;
+  static_assert(Q == 4, "four counts of 16 bits");
+  __shared__ float scratch[17];
+  __shared__ unsigned long long counts[SW_THREADS / 64];
+  const int r = blockIdx.y, c = blockIdx.x, tid = threadIdx.x;
+  const SwRow w = sw_row(ws, row0 + r, S);
+  float T, top_p, u;
+  sw_params(params, r, row0, T, top_p, u);
+  const float* row = logits + (size_t)(row0 + r) * stride;
+  const int lo = c * SW_CHUNK;
+  float x[Q][4];
+  const bool whole = lo + SW_CHUNK <= V && (reinterpret_cast<uintptr_t>(row) & 15) == 0;
+#pragma unroll
+  for (int q = 0; q < Q; ++q) {
+    const int i = lo + 4 * (q * SW_THREADS + tid);
+    if (whole) {
+      const float4 v = *reinterpret_cast<const float4*>(row + i);
+      x[q][0] = v.x; x[q][1] = v.y; x[q][2] = v.z; x[q][3] = v.w;
+    } else {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) x[q][k] = i + k < V ? row[i + k] : -INFINITY;
+    }
+  }
+  float mx = -INFINITY, neg = -INFINITY;
+#pragma unroll
+  for (int q = 0; q < Q; ++q)
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      x[q][k] = sw_clean(x[q][k]);
+      mx = fmaxf(mx, x[q][k]);
+      if (x[q][k] > -INFINITY) neg = fmaxf(neg, -x[q][k]);
+    }
+  block_max2(mx, neg, scratch);
+  if (tid == 0) {
+    w.cmax[c] = mx;
+    w.cmin[c] = -neg;
+    if (c == 0) {
+      w.result[7] = 0.f;
+      w.result[8] = T;
+      w.result[9] = top_p;
+      w.result[10] = u;
+    }
+  }
+  if (!candidates) return;
+  if (!(top_p < 1.0f)) {                       // every token is kept: the other kernels
+    if (tid == 0) w.ccount[c] = SW_SEG + 1;
+    return;
+  }
+  const float scale = 1.4426950408889634f / T, mc = mx * scale;
+  float e[Q][4], z = 0.f;
+#pragma unroll
+  for (int q = 0; q < Q; ++q)
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      e[q][k] = mx > -INFINITY ? __builtin_amdgcn_exp2f(fmaf(x[q][k], scale, -mc)) : 0.f;
+      z += e[q][k];
+    }
+  z = block_sum(z, scratch);
+  const float least = 0.5f * (1.0f - top_p) * z / (float)V;
+  unsigned long long mine = 0ull;
+#pragma unroll
+  for (int q = 0; q < Q; ++q)
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      if (e[q][k] > 0.f && e[q][k] >= least) mine += 1ull << (16 * q);
+  unsigned long long upto = mine;
+  const int lane = tid & 63, wave = tid >> 6;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const unsigned long long n = __shfl_up(upto, o, 64);
+    if (lane >= o) upto += n;
+  }
+  if (lane == 63) counts[wave] = upto;
+  __syncthreads();
+  unsigned long long before = upto - mine, all = 0ull;
+#pragma unroll
+  for (int i = 0; i < SW_THREADS / 64; ++i) {
+    if (i < wave) before += counts[i];
+    all += counts[i];
+  }
+  int first = 0;
+#pragma unroll
+  for (int q = 0; q < Q; ++q) {
+    int at = first + (int)((before >> (16 * q)) & 0xffff);
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      if (e[q][k] > 0.f && e[q][k] >= least) {
+        if (at < SW_SEG) {
+          w.seg_x[(size_t)c * SW_SEG + at] = x[q][k];
+          w.seg_i[(size_t)c * SW_SEG + at] = lo + 4 * (q * SW_THREADS + tid) + k;
+        }
+        ++at;
+      }
+    first += (int)((all >> (16 * q)) & 0xffff);
+  }
+  if (tid == 0) {
+    w.csum[c] = z;
+    w.ccount[c] = first;
+  }
 }
 
 __global__ void __launch_bounds__(SW_THREADS)
-sw_hist_kernel(float* __restrict__ ws, const float* __restrict__ logits, int V, long stride, int S,
-               const float* __restrict__ temperature) {
+sw_hist_kernel(float* __restrict__ ws, const float* __restrict__ logits, int V, long stride, int S) {
   __shared__ unsigned long long hist[SW_BUCKETS];
   __shared__ float scratch[16];
   const int r = blockIdx.y, c = blockIdx.x;
   const SwRow w = sw_row(ws, r, S);
+  if (w.result[7] != 0.f) return;
   const float* row = logits + (size_t)r * stride;
-  const SwScale s = sw_scale(w, S, temperature[r], false);
+  const SwScale s = sw_scale(w, S, w.result[8], false);
   for (int b = threadIdx.x; b < SW_BUCKETS; b += SW_THREADS) hist[b] = 0ull;
   __syncthreads();
   const int lo = c * SW_CHUNK;
@@ -682,11 +810,12 @@ sw_hist_kernel(float* __restrict__ ws, const float* __restrict__ logits, int V, 
 }
 
 // The bucket in which the mass, most likely tokens first, passes tp, and the mass before it;
-// SW_BUCKETS if it never does (everything is kept). The first SW_THREADS threads work, every
+// BUCKETS if it never does (everything is kept). The first SW_THREADS threads work, every
 // thread of the block must call (barriers). tmp: 8 floats and 2 ints of LDS.
+template <int BUCKETS>
 __device__ __forceinline__ void sw_crossing(const float* tot, float tp, float* tmp, int* itmp, int* cross,
                                             float* before) {
-  constexpr int PER = SW_BUCKETS / SW_THREADS;
+  constexpr int PER = BUCKETS / SW_THREADS;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const bool works = tid < SW_THREADS;
   float v[PER], mine = 0.f;
@@ -702,48 +831,49 @@ __device__ __forceinline__ void sw_crossing(const float* tot, float tp, float* t
       if (lane >= o) inc += n;
     }
   }
-  if (tid == 0) { itmp[0] = SW_BUCKETS; }
+  if (tid == 0) { itmp[0] = BUCKETS; }
   if (works && lane == 63) tmp[wave] = inc;
   __syncthreads();
   float run = 0.f;
   if (works) {
     for (int i = 0; i < wave; ++i) run += tmp[i];
     run += inc - mine;                     // mass before this thread's buckets
-    int first = SW_BUCKETS;
+    int first = BUCKETS;
     float r2 = run;
 #pragma unroll
     for (int j = 0; j < PER; ++j) {
-      if (first == SW_BUCKETS && r2 + v[j] > tp) first = tid * PER + j;
-      if (first == SW_BUCKETS) r2 += v[j];
+      if (first == BUCKETS && r2 + v[j] > tp) first = tid * PER + j;
+      if (first == BUCKETS) r2 += v[j];
     }
-    if (first < SW_BUCKETS) atomicMin(&itmp[0], first);
+    if (first < BUCKETS) atomicMin(&itmp[0], first);
   }
   __syncthreads();
   const int cb = itmp[0];
-  if (works && cb < SW_BUCKETS && cb / PER == tid) {
+  if (works && cb < BUCKETS && cb / PER == tid) {
     float r2 = run;
     for (int j = 0; j < cb - tid * PER; ++j) r2 += v[j];
     tmp[4] = r2;
   }
   __syncthreads();
   *cross = cb;
-  *before = cb < SW_BUCKETS ? tmp[4] : 0.f;
+  *before = cb < BUCKETS ? tmp[4] : 0.f;
 }
 
 // One workgroup a row; a thread adds two buckets, eight chunks' loads under way, in chunk order.
 #define SW_COMBINE_THREADS (SW_BUCKETS / 2)
 __global__ void __launch_bounds__(SW_COMBINE_THREADS)
-sw_combine_kernel(float* __restrict__ ws, int S, const float* __restrict__ temperature,
-                  const float* __restrict__ top_p) {
+sw_combine_kernel(float* __restrict__ ws, int S) {
   __shared__ float tot[SW_BUCKETS];
   __shared__ float tmp[17];
   __shared__ int itmp[2];
   const int r = blockIdx.x;
   const SwRow w = sw_row(ws, r, S);
-  const SwScale s = sw_scale(w, S, temperature[r], true);
+  if (w.result[7] != 0.f) return;
+  const float top_p = w.result[9];
+  const SwScale s = sw_scale(w, S, w.result[8], true);
   int cross = SW_BUCKETS;
   float before = 0.f;
-  if (top_p[r] < 1.0f) {
+  if (top_p < 1.0f) {
     float2 t = make_float2(0.f, 0.f);
     const float* mine = w.hist + 2 * threadIdx.x;
     for (int c0 = 0; c0 < S; c0 += 8) {
@@ -763,7 +893,7 @@ sw_combine_kernel(float* __restrict__ ws, int S, const float* __restrict__ tempe
     tot[2 * threadIdx.x] = t.x;
     tot[2 * threadIdx.x + 1] = t.y;
     __syncthreads();
-    sw_crossing(tot, top_p[r] * s.z, tmp, itmp, &cross, &before);
+    sw_crossing<SW_BUCKETS>(tot, top_p * s.z, tmp, itmp, &cross, &before);
   }
   if (threadIdx.x == 0) {
     w.result[1] = __int_as_float(cross);
@@ -787,14 +917,14 @@ __device__ __forceinline__ SwScale sw_found(const SwRow& w, float T, int* cross)
 }
 
 __global__ void __launch_bounds__(SW_THREADS)
-sw_gather_kernel(float* __restrict__ ws, const float* __restrict__ logits, int V, long stride, int S,
-                 const float* __restrict__ temperature) {
+sw_gather_kernel(float* __restrict__ ws, const float* __restrict__ logits, int V, long stride, int S) {
   __shared__ float tmp[17];
   const int r = blockIdx.y, c = blockIdx.x;
   const SwRow w = sw_row(ws, r, S);
+  if (w.result[7] != 0.f) return;
   const float* row = logits + (size_t)r * stride;
   int cross;
-  const SwScale s = sw_found(w, temperature[r], &cross);
+  const SwScale s = sw_found(w, w.result[8], &cross);
   const int lo = c * SW_CHUNK;
   float x[SW_PER];
 #pragma unroll
@@ -844,11 +974,194 @@ __device__ __forceinline__ float wave_inclusive_scan(float v) {
   return v;
 }
 
+// The edge of the nucleus among the n tokens of the crossing bucket, in LDS (kept: key > edge): the mass of all larger ones,
+// added in list order, and what lies ``before`` the bucket is at most tp. A block of SW_THREADS; vote_key and vote_low: 4 words of LDS.
+__device__ __forceinline__ uint32_t sw_edge(const float* list_x, const float* list_e, int n, float before, float tp,
+                                            uint32_t* vote_key, int* vote_low) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  uint32_t lo = 0u, hi = 0xffffffffu, edge;
+  if (n <= SW_THREADS) {
+    // Few tokens: every one of them asks directly whether it is kept (the mass of the
+    // tokens above it, added in list order, and what lies before the bucket); the edge is
+    // the smallest kept key, less one.
+    uint32_t lowest = 0xffffffffu;
+    for (int i = tid; i < n; i += SW_THREADS) {
+      const uint32_t k = sw_key(list_x[i]);
+      float mass = 0.f;
+      for (int j = 0; j < n; ++j) mass += sw_key(list_x[j]) > k ? list_e[j] : 0.f;
+      if (mass + before <= tp) lowest = min(lowest, k);
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) lowest = min(lowest, (uint32_t)__shfl_xor((int)lowest, o, 64));
+    if (lane == 0) vote_key[wave] = lowest;
+    __syncthreads();
+    lowest = min(min(vote_key[0], vote_key[1]), min(vote_key[2], vote_key[3]));
+    edge = lowest - 1u;                // (no token kept: 0xfffffffe, nothing in the bucket passes)
+    if (lowest == 0xffffffffu) edge = 0xffffffffu;
+  } else {
+    // The edge lies between the list's smallest key (less one: everything above it is the
+    // whole list) and its largest (nothing above it). Four waves try four keys a round.
+    uint32_t kmin = 0xffffffffu, kmax = 0u;
+    for (int i = lane; i < n; i += 64) {
+      const uint32_t k = sw_key(list_x[i]);
+      kmin = min(kmin, k);
+      kmax = max(kmax, k);
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+      kmin = min(kmin, (uint32_t)__shfl_xor((int)kmin, o, 64));
+      kmax = max(kmax, (uint32_t)__shfl_xor((int)kmax, o, 64));
+    }
+    lo = kmin - 1u;
+    hi = kmax;
+    while (hi - lo > 1u) {
+      // gap keys lie strictly between lo and hi; wave v tries one of them: all of them
+      // when there are at most four, else four spread evenly
+      const uint32_t gap = hi - lo - 1u;
+      const bool mine = gap > 4u || (uint32_t)wave < gap;
+      const uint32_t mid = gap > 4u
+          ? lo + 1u + (uint32_t)(((unsigned long long)gap * (uint32_t)(wave + 1)) / 5u)
+          : lo + 1u + (uint32_t)wave;
+      float mass = 0.f;
+      if (mine) {
+        for (int i = lane; i < n; i += 64) mass += sw_key(list_x[i]) > mid ? list_e[i] : 0.f;
+        mass = wave_sum(mass) + before;
+      }
+      __syncthreads();
+      if (lane == 0) { vote_key[wave] = mine ? mid : 0u; vote_low[wave] = !mine ? -1 : (mass > tp ? 1 : 0); }
+      __syncthreads();
+      uint32_t nlo = lo, nhi = hi;
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        if (vote_low[v] == 1) nlo = max(nlo, vote_key[v]);
+        if (vote_low[v] == 0) nhi = min(nhi, vote_key[v]);
+      }
+      lo = nlo; hi = nhi;
+    }
+    edge = lo;
+  }
+  return edge;
+}
+
+// The token of a row from its candidates alone, if there are few: what the kernels from hist to draw do, by one workgroup in
+// LDS. Rows with more, or with more than SW_SMALL_LIST tokens in the crossing bucket, are left to those kernels, which leave at
+// once from a row that is done.
+#define SW_SMALL 4096
+#define SW_SMALL_BUCKETS 1024
+#define SW_SMALL_LIST 1024
+__global__ void __launch_bounds__(SW_THREADS)
+sw_small_kernel(int32_t* __restrict__ out, float* __restrict__ ws, int S, int row0) {
+  __shared__ float tmp[17];
+  __shared__ int itmp[2];
+  __shared__ float cand[SW_SMALL];
+  __shared__ int32_t token[SW_SMALL];
+  __shared__ unsigned long long hist[SW_SMALL_BUCKETS];
+  __shared__ float list_x[SW_SMALL_LIST], list_e[SW_SMALL_LIST];
+  __shared__ int seg_at[65];
+  __shared__ uint32_t vote_key[4];
+  __shared__ int vote_low[4], choice_s, last_kept;
+  float* const tot = list_x;               // (the buckets' sums are read before the list is made)
+  static_assert(SW_SMALL_LIST >= SW_SMALL_BUCKETS, "one place for both");
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = row0 + blockIdx.x;
+  const SwRow w = sw_row(ws, r, S);
+  const float T = w.result[8], top_p = w.result[9], u = w.result[10];
+  const int count = lane < S ? w.ccount[lane] : 0;
+  const float cmax = lane < S ? w.cmax[lane] : -INFINITY, csum = lane < S ? w.csum[lane] : 0.f;
+  SwScale s = sw_scale(w, S, T, false);
+  s.inv_w *= (float)SW_SMALL_BUCKETS / SW_BUCKETS;
+  if (__any(count > SW_SEG) || !(s.mx > -INFINITY)) return;
+  s.z = wave_sum(csum > 0.f ? csum * __builtin_amdgcn_exp2f((cmax - s.mx) * s.c) : 0.f);
+  const int upto = (int)wave_inclusive_scan((float)count);            // (small integers: exact)
+  const int n = __shfl(upto, 63, 64);
+  if (n > SW_SMALL) return;
+  if (wave == 0 && lane < S) { seg_at[lane] = upto - count; seg_at[lane + 1] = upto; }
+  for (int b = tid; b < SW_SMALL_BUCKETS; b += SW_THREADS) hist[b] = 0ull;
+  if (tid == 0) { choice_s = -1; last_kept = -1; }
+  __syncthreads();
+  auto bucket = [&](float x) {
+    return (int)fminf(fmaxf((s.mx - x) * s.inv_w, 0.f), (float)(SW_SMALL_BUCKETS - 1));
+  };
+  for (int c = tid >> 3; c < S; c += SW_THREADS / 8) {                // eight threads a chunk
+    const int base = seg_at[c], k = seg_at[c + 1] - base;
+    for (int j0 = tid & 7; j0 < k; j0 += 8 * 4) {                     // four loads of each under way
+      float x[4];
+      int32_t at[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int j = min(j0 + 8 * q, k - 1);
+        x[q] = w.seg_x[(size_t)c * SW_SEG + j];
+        at[q] = w.seg_i[(size_t)c * SW_SEG + j];
+      }
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int j = j0 + 8 * q;
+        if (j >= k) continue;
+        cand[base + j] = x[q];
+        token[base + j] = at[q];
+        atomicAdd(&hist[bucket(x[q])], (unsigned long long)(sw_exp(x[q], s) * SW_FIXED + 0.5f));
+      }
+    }
+  }
+  __syncthreads();
+  for (int b = tid; b < SW_SMALL_BUCKETS; b += SW_THREADS) tot[b] = (float)hist[b] * (1.0f / SW_FIXED);
+  __syncthreads();
+  const float tp = top_p * s.z;
+  int cross;
+  float before;
+  sw_crossing<SW_SMALL_BUCKETS>(tot, tp, tmp, itmp, &cross, &before);
+  if (cross >= SW_SMALL_BUCKETS) return;   // (rounding, with top_p next to 1)
+  // a thread has consecutive candidates from here on
+  const int per = (n + SW_THREADS - 1) / SW_THREADS, a = min(n, per * tid), b = min(n, a + per);
+  int mine = 0;
+  for (int i = a; i < b; ++i) mine += bucket(cand[i]) == cross ? 1 : 0;
+  float in_bucket;
+  int at = (int)block_exclusive_scan((float)mine, tmp, &in_bucket);
+  if (in_bucket > (float)SW_SMALL_LIST) return;
+  for (int i = a; i < b; ++i)
+    if (bucket(cand[i]) == cross) {
+      list_x[at] = cand[i];
+      list_e[at++] = sw_exp(cand[i], s);
+    }
+  __syncthreads();
+  uint32_t edge = sw_edge(list_x, list_e, (int)in_bucket, before, tp, vote_key, vote_low);
+  // the most likely token is always kept: nothing lies before it
+  if (cross == 0 && edge >= sw_key(s.mx)) edge = sw_key(s.mx) - 1u;
+  auto kept = [&](float x) {
+    const int k = bucket(x);
+    return k < cross || (k == cross && sw_key(x) > edge);
+  };
+  float mass = 0.f;
+  int my_last = -1;
+  for (int i = a; i < b; ++i)
+    if (kept(cand[i])) {
+      mass += sw_exp(cand[i], s);
+      my_last = i;
+    }
+  float total;
+  const float run = block_exclusive_scan(mass, tmp, &total);
+  const float target = u * total;
+  if (mass > 0.f && run <= target && target < run + mass) {
+    int choice = my_last;
+    float sum = run;
+    for (int i = a; i < b; ++i)
+      if (kept(cand[i])) {
+        sum += sw_exp(cand[i], s);
+        if (sum > target) { choice = i; break; }
+      }
+    choice_s = choice;
+  }
+  if (my_last >= 0) atomicMax(&last_kept, my_last);
+  __syncthreads();
+  // rounding may leave the target past the last kept token: take that token
+  if (tid == 0) {
+    out[r] = token[choice_s >= 0 ? choice_s : last_kept];
+    w.result[7] = 1.f;
+  }
+}
+
 __global__ void __launch_bounds__(SW_THREADS)
 sw_draw_kernel(int32_t* __restrict__ out, float* __restrict__ ws, const float* __restrict__ logits, int V,
-               long stride, int S,
-               const float* __restrict__ temperature, const float* __restrict__ top_p,
-               const float* __restrict__ uniform) {
+               long stride, int S) {
   __shared__ float tmp[17];
   __shared__ float list_x[SW_LIST], list_e[SW_LIST];
   __shared__ int seg_at[65];
@@ -860,9 +1173,10 @@ sw_draw_kernel(int32_t* __restrict__ out, float* __restrict__ ws, const float* _
   const SwRow w = sw_row(ws, r, S);
   const float* row = logits + (size_t)r * stride;
   int cross;
-  const SwScale s = sw_found(w, temperature[r], &cross);
+  if (w.result[7] != 0.f) return;
+  const SwScale s = sw_found(w, w.result[8], &cross);
   const float before = w.result[3];
-  const float tp = top_p[r] * s.z;
+  const float tp = w.result[9] * s.z, uniform = w.result[10];
   const int my_count = lane < S ? w.ccount[lane] : 0;
   const float my_sure = lane < S ? w.ckept[lane] : 0.f;
   if (tid == 0) { last_kept = -1; choice_s = -1; }
@@ -890,66 +1204,7 @@ sw_draw_kernel(int32_t* __restrict__ out, float* __restrict__ ws, const float* _
         }
       }
       __syncthreads();
-      if (n <= SW_THREADS) {
-        // Few tokens: every one of them asks directly whether it is kept (the mass of the
-        // tokens above it, added in list order, and what lies before the bucket); the edge is
-        // the smallest kept key, less one.
-        uint32_t lowest = 0xffffffffu;
-        for (int i = tid; i < n; i += SW_THREADS) {
-          const uint32_t k = sw_key(list_x[i]);
-          float mass = 0.f;
-          for (int j = 0; j < n; ++j) mass += sw_key(list_x[j]) > k ? list_e[j] : 0.f;
-          if (mass + before <= tp) lowest = min(lowest, k);
-        }
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) lowest = min(lowest, (uint32_t)__shfl_xor((int)lowest, o, 64));
-        if (lane == 0) vote_key[wave] = lowest;
-        __syncthreads();
-        lowest = min(min(vote_key[0], vote_key[1]), min(vote_key[2], vote_key[3]));
-        edge = lowest - 1u;                // (no token kept: 0xfffffffe, nothing in the bucket passes)
-        if (lowest == 0xffffffffu) edge = 0xffffffffu;
-      } else {
-        // The edge lies between the list's smallest key (less one: everything above it is the
-        // whole list) and its largest (nothing above it). Four waves try four keys a round.
-        uint32_t kmin = 0xffffffffu, kmax = 0u;
-        for (int i = lane; i < n; i += 64) {
-          const uint32_t k = sw_key(list_x[i]);
-          kmin = min(kmin, k);
-          kmax = max(kmax, k);
-        }
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) {
-          kmin = min(kmin, (uint32_t)__shfl_xor((int)kmin, o, 64));
-          kmax = max(kmax, (uint32_t)__shfl_xor((int)kmax, o, 64));
-        }
-        lo = kmin - 1u;
-        hi = kmax;
-        while (hi - lo > 1u) {
-          // gap keys lie strictly between lo and hi; wave v tries one of them: all of them
-          // when there are at most four, else four spread evenly
-          const uint32_t gap = hi - lo - 1u;
-          const bool mine = gap > 4u || (uint32_t)wave < gap;
-          const uint32_t mid = gap > 4u
-              ? lo + 1u + (uint32_t)(((unsigned long long)gap * (uint32_t)(wave + 1)) / 5u)
-              : lo + 1u + (uint32_t)wave;
-          float mass = 0.f;
-          if (mine) {
-            for (int i = lane; i < n; i += 64) mass += sw_key(list_x[i]) > mid ? list_e[i] : 0.f;
-            mass = wave_sum(mass) + before;
-          }
-          __syncthreads();
-          if (lane == 0) { vote_key[wave] = mine ? mid : 0u; vote_low[wave] = !mine ? -1 : (mass > tp ? 1 : 0); }
-          __syncthreads();
-          uint32_t nlo = lo, nhi = hi;
-#pragma unroll
-          for (int v = 0; v < 4; ++v) {
-            if (vote_low[v] == 1) nlo = max(nlo, vote_key[v]);
-            if (vote_low[v] == 0) nhi = min(nhi, vote_key[v]);
-          }
-          lo = nlo; hi = nhi;
-        }
-        edge = lo;
-      }
+      edge = sw_edge(list_x, list_e, n, before, tp, vote_key, vote_low);
     } else {                               // too many tokens in one bucket: bisect over the whole row
       while (hi - lo > 1u) {
         const uint32_t mid = lo + ((hi - lo) >> 1);
@@ -987,7 +1242,7 @@ sw_draw_kernel(int32_t* __restrict__ out, float* __restrict__ ws, const float* _
     const float mass = my_sure + extra;
     const float upto = wave_inclusive_scan(mass);
     const float kept = __shfl(upto, 63, 64);
-    const float target = uniform[r] * kept;
+    const float target = uniform * kept;
     const unsigned long long holds = __ballot(mass > 0.f && upto > target);
     const unsigned long long any = __ballot(mass > 0.f);
     if (lane == 0) {
@@ -1008,7 +1263,7 @@ sw_draw_kernel(int32_t* __restrict__ out, float* __restrict__ ws, const float* _
   __syncthreads();
   // walk the chunk that holds the target: sixteen consecutive tokens a thread
   const int c0 = pick_chunk * SW_CHUNK;
-  const float target = uniform[r] * kept_s - pick_before;
+  const float target = uniform * kept_s - pick_before;
   float xv[SW_PER], v[SW_PER], mine = 0.f;
   int my_last = -1;
 #pragma unroll
@@ -1047,13 +1302,13 @@ sw_draw_kernel(int32_t* __restrict__ out, float* __restrict__ ws, const float* _
 
 __global__ void __launch_bounds__(SW_THREADS)
 sw_probs_kernel(float* __restrict__ ws, float* __restrict__ work, const float* __restrict__ logits,
-                int V, long stride, int S, const float* __restrict__ temperature) {
+                int V, long stride, int S) {
   const int r = blockIdx.y, c = blockIdx.x;
   const SwRow w = sw_row(ws, r, S);
   const float* row = logits + (size_t)r * stride;
   float* ex = work + (size_t)r * V;
   int cross;
-  const SwScale s = sw_found(w, temperature[r], &cross);
+  const SwScale s = sw_found(w, w.result[8], &cross);
   const uint32_t edge = __float_as_uint(w.result[0]);
   const float inv_kept = 1.0f / w.result[2];
 #pragma unroll
@@ -1071,6 +1326,26 @@ extern "C" size_t ptl_sample_top_p_wide_workspace(int R, int V) {
   return (size_t)R * sw_row_words(S) * sizeof(float);
 }
 
+static int sample_wide(int32_t* out, float* work, int want_probs, const float* logits, int R, int V, long stride,
+                       const SwParams& params, const float* values, float* ws, hipStream_t stream) {
+  const int S = (V + SW_CHUNK - 1) / SW_CHUNK;
+  const dim3 chunks(S, R);
+  for (int row0 = 0; row0 < R; row0 += SW_GROUP) {
+    const int rows = R - row0 < SW_GROUP ? R - row0 : SW_GROUP;
+    SwParams p = params;
+    if (values) memcpy(p.value, values + (size_t)3 * row0, (size_t)rows * 3 * sizeof(float));
+    sw_scan_kernel<<<dim3(S, rows), SW_THREADS, 0, stream>>>(ws, logits, V, stride, S, row0, !want_probs, p);
+  }
+  // (with the probabilities of all tokens the nucleus is wanted in the form that the last kernel reads)
+  if (!want_probs) sw_small_kernel<<<R, SW_THREADS, 0, stream>>>(out, ws, S, 0);
+  sw_hist_kernel<<<chunks, SW_THREADS, 0, stream>>>(ws, logits, V, stride, S);
+  sw_combine_kernel<<<R, SW_COMBINE_THREADS, 0, stream>>>(ws, S);
+  sw_gather_kernel<<<chunks, SW_THREADS, 0, stream>>>(ws, logits, V, stride, S);
+  sw_draw_kernel<<<R, SW_THREADS, 0, stream>>>(out, ws, logits, V, stride, S);
+  if (want_probs) sw_probs_kernel<<<chunks, SW_THREADS, 0, stream>>>(ws, work, logits, V, stride, S);
+  return ptl_launch_status();
+}
+
 // As ptl_sample_top_p (work: only for the probabilities, if wanted); ws:
 // ptl_sample_top_p_wide_workspace(R, V) bytes, 16-byte aligned.
 // Rows of up to 64 chunks (262,144 logits).
@@ -1080,16 +1355,84 @@ extern "C" int ptl_sample_top_p_wide(int32_t* out, float* work, int want_probs, 
                                      hipStream_t stream) {
   if (R <= 0) return PTL_OK;
   const int S = (V + SW_CHUNK - 1) / SW_CHUNK;
-  if (V <= 0 || stride < V || (want_probs && !work) || !ws || S > 64 || R > 65535) return PTL_ERR_ARG;
-  const dim3 chunks(S, R);
-  sw_minmax_kernel<<<chunks, SW_THREADS, 0, stream>>>(ws, logits, V, stride, S);
-  sw_hist_kernel<<<chunks, SW_THREADS, 0, stream>>>(ws, logits, V, stride, S, temperature);
-  sw_combine_kernel<<<R, SW_COMBINE_THREADS, 0, stream>>>(ws, S, temperature, top_p);
-  sw_gather_kernel<<<chunks, SW_THREADS, 0, stream>>>(ws, logits, V, stride, S, temperature);
-  sw_draw_kernel<<<R, SW_THREADS, 0, stream>>>(out, ws, logits, V, stride, S, temperature, top_p, uniform);
-  if (want_probs)
-    sw_probs_kernel<<<chunks, SW_THREADS, 0, stream>>>(ws, work, logits, V, stride, S, temperature);
-  return ptl_launch_status();
+  if (V <= 0 || stride < V || (want_probs && !work) || !ws || S > 64 || R > 65535 || !temperature || !top_p || !uniform)
+    return PTL_ERR_ARG;
+  SwParams params{};
+  params.temperature = temperature;
+  params.top_p = top_p;
+  params.uniform = uniform;
+  return sample_wide(out, work, want_probs, logits, R, V, stride, params, nullptr, ws, stream);
+}
+
+// BLAKE2b (RFC 7693) without a key, the first 8 bytes of a digest of that length as a little-endian number.
+static uint64_t blake2b_8(const uint8_t* text, size_t length) {
+  static const uint64_t iv[8] = {0x6a09e667f3bcc908ull, 0xbb67ae8584caa73bull, 0x3c6ef372fe94f82bull, 0xa54ff53a5f1d36f1ull,
+                                 0x510e527fade682d1ull, 0x9b05688c2b3e6c1full, 0x1f83d9abfb41bd6bull, 0x5be0cd19137e2179ull};
+  static constexpr uint8_t sigma[10][16] = {
+      {0, 1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15}, {14, 10, 4, 8, 9, 15, 13, 6, 1, 12, 0, 2, 11, 7, 5, 3},
+      {11, 8, 12, 0, 5, 2, 15, 13, 10, 14, 3, 6, 7, 1, 9, 4}, {7, 9, 3, 1, 13, 12, 11, 14, 2, 6, 5, 10, 4, 0, 15, 8},
+      {9, 0, 5, 7, 2, 4, 10, 15, 14, 1, 11, 12, 6, 8, 3, 13}, {2, 12, 6, 10, 0, 11, 8, 3, 4, 13, 7, 5, 15, 14, 1, 9},
+      {12, 5, 1, 15, 14, 13, 4, 10, 0, 7, 6, 3, 9, 2, 8, 11}, {13, 11, 7, 14, 12, 1, 3, 9, 5, 0, 15, 4, 8, 6, 2, 10},
+      {6, 15, 14, 9, 11, 3, 0, 8, 12, 2, 13, 7, 1, 4, 10, 5}, {10, 2, 8, 4, 7, 6, 1, 5, 15, 11, 9, 14, 3, 12, 13, 0}};
+  uint64_t h[8];
+  memcpy(h, iv, sizeof(h));
+  h[0] ^= 0x01010000ull ^ 8ull;
+  size_t done = 0;
+  do {
+    const size_t n = length - done < 128 ? length - done : 128;
+    uint64_t m[16] = {};
+    memcpy(m, text + done, n);                   // (this host is little-endian too)
+    done += n;
+    uint64_t v[16];
+    memcpy(v, h, sizeof(h));
+    memcpy(v + 8, iv, sizeof(iv));
+    v[12] ^= done;
+    if (done == length) v[14] = ~v[14];
+    auto mix = [&](int a, int b, int c, int d, uint64_t x, uint64_t y) {
+      auto turn = [](uint64_t w, int k) { return (w >> k) | (w << (64 - k)); };
+      v[a] += v[b] + x;
+      v[d] = turn(v[d] ^ v[a], 32);
+      v[c] += v[d];
+      v[b] = turn(v[b] ^ v[c], 24);
+      v[a] += v[b] + y;
+      v[d] = turn(v[d] ^ v[a], 16);
+      v[c] += v[d];
+      v[b] = turn(v[b] ^ v[c], 63);
+    };
+#pragma unroll                                   // (the places of the words are known then: half the time)
+    for (int round = 0; round < 12; ++round) {
+      const uint8_t* at = sigma[round % 10];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) mix(i, 4 + i, 8 + i, 12 + i, m[at[2 * i]], m[at[2 * i + 1]]);
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        mix(i, 4 + (i + 1) % 4, 8 + (i + 2) % 4, 12 + (i + 3) % 4, m[at[8 + 2 * i]], m[at[9 + 2 * i]]);
+    }
+    for (int i = 0; i < 8; ++i) h[i] ^= v[i] ^ v[8 + i];
+  } while (done < length);
+  return h[0];
+}
+
+// values[i][2] = a number in [0, 1) that depends on text i alone (texts one after the other, ends[i]: where the i-th ends)
+extern "C" int ptl_uniforms(float* values, const uint8_t* texts, const int32_t* ends, int n) {
+  int at = 0;
+  for (int i = 0; i < n; ++i) {
+    if (ends[i] < at) return PTL_ERR_ARG;
+    values[3 * (size_t)i + 2] = (float)((double)(blake2b_8(texts + at, (size_t)(ends[i] - at)) >> 11) * (1.0 / 9007199254740992.0));
+    at = ends[i];
+  }
+  return PTL_OK;
+}
+
+// The same without probabilities, temperature, top_p and u of every row in host memory ([R][3]); they are in the launch when
+// the call returns. With texts u is made here (ptl_uniforms).
+extern "C" int ptl_sample_top_p_rows(int32_t* out, const float* logits, int R, int V, long stride, float* values,
+                                     const uint8_t* texts, const int32_t* ends, float* ws, hipStream_t stream) {
+  if (R <= 0) return PTL_OK;
+  const int S = (V + SW_CHUNK - 1) / SW_CHUNK;
+  if (V <= 0 || stride < V || !ws || S > 64 || R > 65535 || !values || (texts && !ends)) return PTL_ERR_ARG;
+  if (texts && ptl_uniforms(values, texts, ends, R) != PTL_OK) return PTL_ERR_ARG;
+  return sample_wide(out, nullptr, 0, logits, R, V, stride, SwParams{}, values, ws, stream);
 }
 
 // ptl_token_logprob: out[r] = log_softmax(logits[r])[tokens[r]], the log-probability the

@@ -6,9 +6,11 @@ raises.
 """
 from __future__ import annotations
 
+import array
 import contextlib
 import ctypes
 import functools
+import itertools
 from typing import Optional
 
 import torch
@@ -1141,6 +1143,13 @@ SAMPLE_WIDE_FROM = 16384      # rows at least this long are sampled by many work
 SAMPLE_WIDE_UP_TO = 64 * 4096
 
 
+def _sample_words(R: int, V: int) -> int:
+    """float32 words of workspace the many-workgroup form takes."""
+    fn = library.load("sampling").ptl_sample_top_p_wide_workspace
+    fn.restype = ctypes.c_size_t
+    return fn(R, V) // 4
+
+
 def sample_top_p(logits: torch.Tensor, temperature: torch.Tensor, top_p: torch.Tensor,
                  uniform: torch.Tensor, return_probs: bool = False, wide: Optional[bool] = None):
     """One token per row from the nucleus of softmax(logits / temperature).
@@ -1164,9 +1173,7 @@ def sample_top_p(logits: torch.Tensor, temperature: torch.Tensor, top_p: torch.T
              else None)
     lib = library.load("sampling")
     if wide:
-        lib.ptl_sample_top_p_wide_workspace.restype = ctypes.c_size_t
-        nbytes = int(lib.ptl_sample_top_p_wide_workspace(R, V))
-        ws = torch.empty((nbytes // 4,), dtype=torch.float32, device=logits.device)
+        ws = torch.empty((_sample_words(R, V),), dtype=torch.float32, device=logits.device)
         _check(lib.ptl_sample_top_p_wide(_ptr(out), _ptr(probs), int(return_probs), _ptr(logits), R, V,
                                          ctypes.c_long(logits.stride(0)), _ptr(temperature),
                                          _ptr(top_p), _ptr(uniform), _ptr(ws), _stream()),
@@ -1176,6 +1183,34 @@ def sample_top_p(logits: torch.Tensor, temperature: torch.Tensor, top_p: torch.T
                                     ctypes.c_long(logits.stride(0)), _ptr(temperature), _ptr(top_p),
                                     _ptr(uniform), _stream()), "sample_top_p")
     return (out, probs) if return_probs else out
+
+
+def sample_rows_fits(logits: torch.Tensor) -> bool:
+    """Whether ``sample_rows`` takes these logits: rows that many workgroups share."""
+    return (logits.is_cuda and logits.dtype == torch.float32 and logits.dim() == 2 and logits.stride(1) == 1
+            and SAMPLE_WIDE_FROM <= logits.shape[1] <= SAMPLE_WIDE_UP_TO)
+
+
+def sample_rows(logits: torch.Tensor, params, texts) -> torch.Tensor:
+    """As ``sample_top_p``, with what the host knows handed over in the launch itself: ``params`` (temperature, top_p, 0.0)
+    of every row, one after the other; ``texts``: a string a row, of which u is made (``sampling.uniform_for``)."""
+    if not sample_rows_fits(logits):
+        raise KernelError("sample_rows: logits must be float32 [R, V] on the GPU with dense rows of vocabulary size")
+    R, V = logits.shape
+    if len(texts) != R or len(params) != 3 * R:
+        raise KernelError(f"sample_rows: three parameters and a text for each of {R} rows")
+    values = array.array("f", params)
+    joined = "".join(texts).encode()
+    ends = array.array("i", itertools.accumulate(map(len, texts)))
+    if ends and ends[-1] != len(joined):          # (a character of more than one byte)
+        ends = array.array("i", itertools.accumulate(len(t.encode()) for t in texts))
+    lib = library.load("sampling")
+    out = torch.empty((R,), dtype=torch.int32, device=logits.device)
+    ws = torch.empty((_sample_words(R, V),), dtype=torch.float32, device=logits.device)
+    _check(lib.ptl_sample_top_p_rows(_ptr(out), _ptr(logits), R, V, ctypes.c_long(logits.stride(0)),
+                                     ctypes.c_void_p(values.buffer_info()[0]), joined, ctypes.c_void_p(ends.buffer_info()[0]),
+                                     _ptr(ws), _stream()), "sample_rows")
+    return out
 
 
 LOGPROB_ONE_UP_TO = 32768     # rows up to this long: a workgroup a row (longer ones: many, and a second kernel)

@@ -1666,6 +1666,35 @@ def test_sample_top_p_one_and_many_workgroups_a_row_agree(ops, V):
         assert float((prw[r].double().cpu() - want).abs().sum()) < 1e-3
 
 
+@pytest.mark.parametrize("rows,V", [(1, 16384), (70, 20001), (64, 32000), (3, 128256)])
+def test_sample_rows(ops, rows, V):
+    """Tokens from parameters in the launch and numbers made of texts: those of ``sample_top_p`` with the same numbers, and, where
+    a row's candidates alone decide (peaked rows), where they are too many (flat ones, equal logits) and where all tokens
+    are kept, a token of the nucleus that the other kernels find, at the same place of its cumulative distribution."""
+    from pytriton_llama_amd.sampling.sampler import uniform_for, uniform_text
+    g = torch.Generator().manual_seed(V)
+    logits = torch.randn(rows, V + 3, generator=g)
+    kinds = [4.0, 0.02, 2.0, 0.7, 30.0, 1.0]
+    for r in range(rows):
+        logits[r] *= kinds[r % 6]
+        if r % 6 == 5:
+            logits[r] = logits[r].round()                     # many equal logits
+    logits = logits.cuda()[:, :V]                             # rows of any alignment
+    params = [(0.6 + 0.1 * (r % 5), (0.9, 0.95, 0.5, 1.0, 0.999999)[r % 5], 0.0) for r in range(rows)]
+    texts = [uniform_text(9, ("chat é", r), 7) for r in range(rows)]
+    got = ops.sample_rows(logits, [v for p in params for v in p], texts)
+    t, p = (torch.tensor([q[i] for q in params]).cuda() for i in (0, 1))
+    u = torch.tensor([uniform_for(9, ("chat é", r), 7) for r in range(rows)]).cuda()
+    assert torch.equal(got, ops.sample_top_p(logits, t, p, u))
+    tok, probs = ops.sample_top_p(logits, t, p, u, return_probs=True)
+    for r in range(rows):
+        cdf = torch.cumsum(probs[r].double(), 0)
+        assert probs[r, int(got[r])] > 0
+        assert int(got[r]) == int(tok[r]) or abs(float(cdf[int(got[r])] - cdf[int(tok[r])])) < 1e-4, r
+    with pytest.raises(ops.KernelError):
+        ops.sample_rows(logits, [0.6, 0.9, 0.0] * rows, texts[1:])
+
+
 @pytest.mark.parametrize("wide", [False, True], ids=["one_workgroup", "many_workgroups"])
 def test_sample_top_p_nearly_flat_row_and_signed_zeros(ops, wide):
     """A nearly flat row with a top_p that admits two tokens keeps exactly those two (the most

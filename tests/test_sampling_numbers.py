@@ -1,0 +1,26 @@
+"""The random numbers of sampled requests, worked out by the kernel library's host code, against Python's."""
+import array
+import ctypes
+import itertools
+
+import pytest
+
+import pytriton_llama_amd.engine  # noqa: F401
+from pytriton_llama_amd.ops import library
+from pytriton_llama_amd.sampling.sampler import uniform_for, uniform_text
+
+
+@pytest.mark.parametrize("ids", [
+    [0, 1, 2 ** 70, -5], ["a", "", "é€", "x" * 119, "x" * 120, "x" * 121, "y" * 300], [("chat", 3), None, 2.5, b"z"]],
+    ids=["numbers", "texts", "others"])
+def test_uniform_numbers_of_the_library(ids):
+    """One block of the hash, its edges and several; ids of any kind."""
+    for seed, step in [(0, 0), (123456789, 4095)]:
+        texts = [uniform_text(seed, i, step).encode() for i in ids]
+        values = array.array("f", [7.0] * (3 * len(ids)))
+        ends = array.array("i", itertools.accumulate(map(len, texts)))
+        rc = library.load("sampling").ptl_uniforms(ctypes.c_void_p(values.buffer_info()[0]), b"".join(texts),
+                                                   ctypes.c_void_p(ends.buffer_info()[0]), len(ids))
+        assert rc == 0
+        want = array.array("f", [uniform_for(seed, i, step) for i in ids])
+        assert values[2::3] == want and set(values[0::3]) == set(values[1::3]) == {7.0}
