@@ -476,10 +476,9 @@ attn_decode_kernel(TO* __restrict__ out, long out_stride, const T* __restrict__ 
 
 template <typename T>
 __global__ void __launch_bounds__(64)
-attn_decode_merge_kernel(T* __restrict__ out, long out_stride, const int32_t* __restrict__ q_start,
-                         const float* __restrict__ part_acc, const float* __restrict__ part_ml,
-                         int Hq, int D, int num_splits, AttnExtras ex, const int32_t* __restrict__ ctx_len = nullptr,
-                         int tile = 0) {
+attn_decode_merge_kernel(const float* __restrict__ part_acc, const float* __restrict__ part_ml,
+                         const int32_t* __restrict__ ctx_len, int Hq, int D, int num_splits, int tile,
+                         const int32_t* __restrict__ q_start, T* __restrict__ out, long out_stride, AttnExtras ex) {
   // tile (0: every split left a part): keys a split is a multiple of; splits without keys left none, and a
   // sequence that one split answered for is done.
   // one wave per (sequence, head): lanes take the splits' (max, denominator) side by side,
@@ -551,8 +550,8 @@ static int launch_decode(void* out, long out_stride, const void* q, long q_strid
   if (hipGetLastError() != hipSuccess) return PTL_ERR_LAUNCH;
   if (num_splits > 1) {
     dim3 mgrid(n_seq, Hq);
-    attn_decode_merge_kernel<TO><<<mgrid, 64, 0, stream>>>((TO*)out, out_stride, q_start, part_acc,
-                                                          part_ml, Hq, Dv, num_splits, ex);
+    attn_decode_merge_kernel<TO><<<mgrid, 64, 0, stream>>>(part_acc, part_ml, nullptr, Hq, Dv, num_splits, 0, q_start,
+                                                          (TO*)out, out_stride, ex);
   }
   return ptl_launch_status();
 }
@@ -583,8 +582,8 @@ extern "C" int ptl_attention_decode_kv(void* out, long out_stride, int out_f32, 
                                         SplitArgs{part_acc, part_ml, num_splits}, n_seq, Hq, Hkv, Dk, Dv, page_size, ex,
                                         scale, stream);
     if (rc != PTL_OK || num_splits == 1) return rc;
-    attn_decode_merge_kernel<float><<<dim3(n_seq, Hq), 64, 0, stream>>>((float*)out, out_stride, q_start, part_acc, part_ml, Hq,
-                                                                       Dv, num_splits, ex, ctx_len, AF_DECODE_TILE);
+    attn_decode_merge_kernel<float><<<dim3(n_seq, Hq), 64, 0, stream>>>(part_acc, part_ml, ctx_len, Hq, Dv, num_splits,
+                                                                       AF_DECODE_TILE, q_start, (float*)out, out_stride, ex);
     return ptl_launch_status();
   }
   const int chunks = (Dk > Dv ? Dk : Dv) / 16;
@@ -694,13 +693,12 @@ __device__ __forceinline__ void wave_lds_fence() {
 // pair that has several, and their (max, denominator).
 template <int NDT, int UNR, bool ORDERED, bool KEPT, bool CAP>
 __global__ void __launch_bounds__(256, NDT <= 2 ? 3 : 2)
-attn_decode_mfma_kernel(bf16_t* __restrict__ out, long out_stride, const bf16_t* __restrict__ q,
-                        long q_stride, const bf16_t* __restrict__ k_cache,
-                        const bf16_t* __restrict__ v_cache, const int32_t* __restrict__ q_start,
-                        const int32_t* __restrict__ ctx_len, const int32_t* __restrict__ block_table,
-                        int bt_stride, float* __restrict__ part_acc, float* __restrict__ part_ml, int n_seq, int Hq, int Hkv,
-                        int page_size, int page_shift, AttnExtras ex, float scale_log2, float cap_in, int num_splits,
-                        int cus) {
+attn_decode_mfma_kernel(const int32_t* __restrict__ ctx_len, const int32_t* __restrict__ block_table,
+                        const bf16_t* __restrict__ k_cache, const bf16_t* __restrict__ v_cache, int n_seq, int Hkv,
+                        int num_splits, int bt_stride, int page_size, int page_shift, const bf16_t* __restrict__ q, long q_stride,
+                        int Hq, int cus, bf16_t* __restrict__ out, long out_stride, const int32_t* __restrict__ q_start,
+                        float* __restrict__ part_acc, float* __restrict__ part_ml, AttnExtras ex, float scale_log2,
+                        float cap_in) {
   constexpr int D = 32 * NDT;
   constexpr int NT = 2 * NDT;             // 16-wide tiles of the head dimension
   constexpr int WAVES = 4;
@@ -963,9 +961,9 @@ static int launch_decode_mfma(void* out, long out_stride, const void* q, long q_
   const float scale_log2 = (cap ? ex.softcap : scale) * log2e, cap_in = cap ? 2.0f * log2e * scale / ex.softcap : 0.f;
 #define GO(KEPT, CAP)                                                                                              \
   attn_decode_mfma_kernel<NDT, UNR, ORDERED, KEPT, CAP><<<(unsigned)groups, 64 * WAVES, lds, stream>>>(            \
-      (bf16_t*)out, out_stride, (const bf16_t*)q, q_stride, (const bf16_t*)k_cache, (const bf16_t*)v_cache, q_start, \
-      ctx_len, block_table, bt_stride, parts, part_ml, n_seq, Hq, Hkv, page_size, page_shift, ex, scale_log2, cap_in, \
-      num_splits, compute_units())
+      ctx_len, block_table, (const bf16_t*)k_cache, (const bf16_t*)v_cache, n_seq, Hkv, num_splits, bt_stride, page_size, \
+      page_shift, (const bf16_t*)q, q_stride, Hq, compute_units(), (bf16_t*)out, out_stride, q_start, parts, part_ml, ex, \
+      scale_log2, cap_in)
   if (kept) {
     if (cap) GO(true, true); else GO(true, false);
   } else {
@@ -975,7 +973,7 @@ static int launch_decode_mfma(void* out, long out_stride, const void* q, long q_
   if (hipGetLastError() != hipSuccess) return PTL_ERR_LAUNCH;
   if (num_splits > 1)
     attn_decode_merge_kernel<bf16_t><<<dim3(n_seq, Hq), 64, 0, stream>>>(
-        (bf16_t*)out, out_stride, q_start, parts, part_ml, Hq, D, num_splits, ex, ctx_len, TILE);
+        parts, part_ml, ctx_len, Hq, D, num_splits, TILE, q_start, (bf16_t*)out, out_stride, ex);
   return ptl_launch_status();
 }
 

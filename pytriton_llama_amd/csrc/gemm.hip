@@ -189,7 +189,7 @@ struct GroupArgs {
 template <int MT, int U, int ROWS, typename TY, bool ADD_NORM = false, int XR = 16, bool BLOCKED = false>
 __global__ void __launch_bounds__(1024)
 gemm_skinny_kernel(TY* __restrict__ y, const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
-                   int M, int N, int K, long ldx, long ldy, int k_per_wave, AddNormArgs an, GroupArgs gr) {
+                   int N, int K, int k_per_wave, int M, long ldx, long ldy, AddNormArgs an, GroupArgs gr) {
   extern __shared__ float red[];                 // [waves][MT][64][4]
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, ln = lane & 15, lg = lane >> 4;
   const int nwaves = blockDim.x >> 6;
@@ -366,7 +366,7 @@ static int launch_skinny_rows(void* y, const void* x, const void* w, int M, int 
   const int xr = MT == 1 ? gs_rows_of(M) : 16;
 #define GO1(TY, AN, XR, BL, args)                                                                    \
   gemm_skinny_kernel<(XR == 16 ? MT : 1), U, ROWS, TY, AN, XR, BL><<<blocks, waves * 64, lds, stream>>>( \
-      (TY*)y, (const bf16_t*)x, (const bf16_t*)w, M, N, K, ldx, ldy, k_per_wave, args, gr)
+      (TY*)y, (const bf16_t*)x, (const bf16_t*)w, N, K, k_per_wave, M, ldx, ldy, args, gr)
 #define GO(TY, AN, XR, args)                                                                         \
   if (blocked) GO1(TY, AN, XR, true, args); else GO1(TY, AN, XR, false, args)
 #define BY_ROWS(TY, AN, args)                                                                        \
@@ -499,8 +499,8 @@ struct RowScaleArgs {
 template <int MODE, int U, int ROWS, int XR, bool BLOCKED>
 __global__ void __launch_bounds__(1024)
 gemm_pair_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
-                 int M, int N_out, int K, long ldx, long ldy, int k_per_wave, int pair_offset,
-                 int tiles_per_group, int group_rows, RopeStoreArgs rs, RowScaleArgs sc, GluArgs act) {
+                 long ldx, int K, int k_per_wave, int pair_offset, int tiles_per_group, int group_rows, int M, int N_out,
+                 long ldy, RopeStoreArgs rs, RowScaleArgs sc, GluArgs act) {
   extern __shared__ float red[];                 // [waves][2][64][4]
   __shared__ float row_factor[16];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, ln = lane & 15, lg = lane >> 4;
@@ -686,7 +686,7 @@ extern "C" int ptl_gate_up_silu_bf16(void* out, const void* x, const void* w, in
   RopeStoreArgs none = {};
 #define GO1(XR, BL)                                                                                   \
   gemm_pair_kernel<PAIR_SILU, 8, 16, XR, BL><<<blocks, waves * 64, lds, stream>>>(                    \
-      (bf16_t*)out, (const bf16_t*)x, (const bf16_t*)w, M, I, K, ldx, I, k_per_wave, I, blocks, 0, none, sc, GluArgs{act, limit})
+      (bf16_t*)out, (const bf16_t*)x, (const bf16_t*)w, ldx, K, k_per_wave, I, blocks, 0, M, I, I, none, sc, GluArgs{act, limit})
 #define GO(XR) if (w_blocked) GO1(XR, true); else GO1(XR, false)
   switch (gs_rows_of(M)) {
     case 4: GO(4); break;
@@ -721,8 +721,8 @@ extern "C" int ptl_qkv_rope_store_bf16(void* q_out, long ldq, const void* x, con
   RopeStoreArgs rs = {positions, inv_freq, slots, (bf16_t*)k_cache, (bf16_t*)v_cache, Hq, Hkv, D, page_size};
 #define GO1(ROWS, XR, BL)                                                                             \
   gemm_pair_kernel<PAIR_ROPE, 8, ROWS, XR, BL><<<blocks, waves * 64, lds, stream>>>(                  \
-      (bf16_t*)q_out, (const bf16_t*)x, (const bf16_t*)w, M, Hq * D, K, ldx, ldq, k_per_wave, D / 2,  \
-      tiles, D, rs, sc, GluArgs{})
+      (bf16_t*)q_out, (const bf16_t*)x, (const bf16_t*)w, ldx, K, k_per_wave, D / 2, tiles, D, M,      \
+      Hq * D, ldq, rs, sc, GluArgs{})
 #define GO(ROWS, XR) if (w_blocked) GO1(ROWS, XR, true); else GO1(ROWS, XR, false)
 #define BY_ROWS(ROWS)                                                                                 \
   switch (gs_rows_of(M)) {                                                                            \

@@ -22,9 +22,14 @@ from typing import Dict, Iterable, List
 CSRC_DIR = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "csrc")
 BUILD_DIR = os.path.join(CSRC_DIR, "_build")
 ARCH = "gfx950"
-# packed float32 instructions are switched off for every kernel of this package
+# packed float32 instructions are switched off for every kernel of this package. The first 14 words of a kernel's arguments
+# (up to the first struct) come in registers with the wave, not by a load from memory that the first addresses wait for: a decode step is
+# a chain of some hundred kernels of 4 to 15 us, and 0.6 to 1.4 % of it (batch 8 of the Llama-3.2-1B shape 984 -> 976 us, batch 64
+# 1,840 -> 1,814, float32 1,465 -> 1,445). The kernels of such a step name first what the first loads need (with the
+# widths of a product's share behind the 14 words, batch 1 and 8 were level or slower).
 HIPCC_FLAGS = ["--offload-arch=" + ARCH, "-O3", "-fPIC", "-shared", "-std=c++17",
-               "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
+               "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+               "-mllvm", "-amdgpu-kernarg-preload-count=16"]
 
 KERNEL_LIBRARIES = ("embedding", "norm", "rope", "attention", "attention_prefill", "activation",
                     "gemm", "gemm_f32", "gemm_rows", "gemm_tile", "blaslt", "sampling", "probe", "stream", "latent", "moe", "prepare", "prompt",
