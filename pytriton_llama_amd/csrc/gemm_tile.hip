@@ -9,7 +9,7 @@
 // The reference runs these products through cuBLAS and the rest as kernels of their own
 // (lite_llama/models/llama.py:107-120, lite_llama/kernels/swiglu.py, skip_rmsnorm.py).
 //
-// Four waves multiply, each a part of the tile, and two bring the operands through LDS (tile_stream.h). What bounds it: with
+// Four waves multiply, each a part of the tile, and four bring the operands through LDS (tile_stream.h). What bounds it: with
 // few workgroups the latency of W on its way from HBM (a chunk a compute unit and 0.35 to 0.7 us, of which the matrix
 // instructions take 0.06 to 0.5), with all compute units at work what they read from L2, 11 to 16 TB/s. LDS is next: a
 // wave of 64 x 64 reads as many bytes as LDS gives in the time of its products, hence parts of 64 x 128 and 144 x 64 in the
@@ -225,6 +225,8 @@ gemm_tile_kernel(const TileArgs a) {
   T(128, 256, 2, 2, 3, 1, 0.59f, 0.35f, 7.3f)        \
   T(144, 256, 1, 4, 3, 1, 0.67f, 0.27f, 7.6f)
 
+constexpr int LOADERS = 4;                       // loading waves (with two of them 1 to 4 % slower: tile_stream.h)
+
 struct Shape {
   int rows, cols, per_unit;
   float chunk, full, tile;
@@ -264,7 +266,7 @@ Plan plan_for(int M, int rows_w, int K, bool sums) {
 template <int BM, int BN, int WGM, int WGN, int NB, int OCC, int MODE>
 int launch(TileArgs a, hipStream_t stream) {
   const size_t lds = (size_t)NB * (BM + BN) * TILE_ROW;
-  auto kernel = gemm_tile_kernel<BM, BN, WGM, WGN, NB, 2, MODE>;
+  auto kernel = gemm_tile_kernel<BM, BN, WGM, WGN, NB, LOADERS, MODE>;
   static LdsAllowance allowance;
   if (!allowance.ask(reinterpret_cast<const void*>(kernel), lds)) return PTL_ERR_LAUNCH;
   const int cols = MODE == OUT_GLU ? BN / 2 : BN;
@@ -272,7 +274,7 @@ int launch(TileArgs a, hipStream_t stream) {
   a.tiles_n = (a.N + cols - 1) / cols;
   const long total = (long)a.tiles_m * a.tiles_n * a.splits, most = (long)OCC * compute_units();
   if (total > 0x3fffffff) return PTL_ERR_ARG;
-  kernel<<<(unsigned)(total < most ? total : most), 64 * (WGM * WGN + 2), lds, stream>>>(a);
+  kernel<<<(unsigned)(total < most ? total : most), 64 * (WGM * WGN + LOADERS), lds, stream>>>(a);
   return ptl_launch_status();
 }
 

@@ -11,7 +11,9 @@
 // A load instruction fills 8 rows of 128 bytes, lane l the l-th 16 bytes: row l / 8, place l % 8, which holds the row's
 // piece (l % 8) ^ (row % 8). A fragment read (16 neighbouring rows, the same piece, at piece ^ (row % 8)) then meets no bank
 // twice (counted: no conflicts). One such wave issues a load every 66 to 83 clocks, 12 to 15 bytes a clock of the 50
-// that a compute unit takes from L2: hence two of them.
+// that a compute unit takes from L2: hence four of them, one beside every wave that multiplies (gemm_tile.hip, us with two
+// and with four: 277 x 16,384 x 2,048 28.7 / 27.8, 277 x 2,048 x 8,192 19.2 / 18.6, 532 x 16,384 x 3,072 56.1 / 54.2, 1,000 x 16,384 x
+// 2,048 71.2 / 69.4; a group of 8 rows more for some of them where four do not share a tile's evenly).
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -34,14 +36,11 @@ template <int N> __device__ __forceinline__ void tile_wait_loads_but() {
 // s_waitcnt lgkmcnt(0): what the wave has read from LDS is in its registers
 __device__ __forceinline__ void tile_wait_lds() { __builtin_amdgcn_s_waitcnt(0xC07F); }
 
-// What a loading wave does (``me``: which of the PW): ``tiles`` tiles of ROWS rows one after the other, ``chunks`` chunks
-// each. rows(i, r): where row r of the workgroup's i-th tile begins (a valid row for every r < ROWS), in bytes, at
-// the first column the tile takes. The other waves call tile_meet() once a chunk before they read it, in the same order.
-template <int ROWS, int NB, int PW, typename Rows>
-__device__ __forceinline__ void tile_bring(unsigned char* lds, int me, int lane, int tiles, int chunks, Rows rows) {
-  constexpr int LI = ROWS / 8 / PW;              // load instructions a chunk
-  static_assert(ROWS % (8 * PW) == 0 && NB >= 3 && NB <= 5 && (NB - 2) * LI < 64, "loads are counted in six bits");
-  const int lrow = lane >> 3, lpiece = (lane & 7) ^ lrow, first = me * LI;
+// What a loading wave does that brings LI groups of 8 rows, from the ``first`` on.
+template <int ROWS, int NB, int LI, typename Rows>
+__device__ __forceinline__ void tile_bring_groups(unsigned char* lds, int first, int lane, int tiles, int chunks, Rows rows) {
+  static_assert(NB >= 3 && NB <= 5 && (NB - 2) * LI < 64, "loads are counted in six bits");
+  const int lrow = lane >> 3, lpiece = (lane & 7) ^ lrow;
   const char* src[LI];
   int next = 0, next_tile = 0, next_chunk = 0, slot = 0;
   const int all = tiles * chunks;
@@ -74,6 +73,17 @@ __device__ __forceinline__ void tile_bring(unsigned char* lds, int me, int lane,
     tile_meet();                                 // chunk c is there; chunk c - 1 has been read
     if (next < all) fetch();
   }
+}
+
+// What a loading wave does (``me``: which of the PW): ``tiles`` tiles of ROWS rows one after the other, ``chunks`` chunks
+// each. rows(i, r): where row r of the workgroup's i-th tile begins (a valid row for every r < ROWS), in bytes, at
+// the first column the tile takes. The other waves call tile_meet() once a chunk before they read it, in the same order.
+template <int ROWS, int NB, int PW, typename Rows>
+__device__ __forceinline__ void tile_bring(unsigned char* lds, int me, int lane, int tiles, int chunks, Rows rows) {
+  static_assert(ROWS % 8 == 0 && ROWS / 8 >= PW, "groups of 8 rows");
+  constexpr int EACH = ROWS / 8 / PW, MORE = ROWS / 8 % PW;    // (the first MORE waves bring one more)
+  if (MORE > 0 && me < MORE) tile_bring_groups<ROWS, NB, EACH + 1>(lds, me * (EACH + 1), lane, tiles, chunks, rows);
+  else tile_bring_groups<ROWS, NB, EACH>(lds, me * EACH + MORE, lane, tiles, chunks, rows);
 }
 
 // The order of a stage of R reads from LDS (for the next stage) and P matrix instructions: the reads one at a time
