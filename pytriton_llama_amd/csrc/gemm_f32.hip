@@ -552,7 +552,14 @@ struct StreamArgs {
   int M, N, K, Mp;
   long ldx, ldy;
   int tiles_m, tiles_n, splits, per, width;
+  int act;
 };
+
+// What becomes of a tile's sums: y; parts, the sums of every span by itself; or, for W = [Wg; Wu] with N rows each, act(gate) * up,
+// the rows of a wave being 16 of Wg and the same 16 of Wu: the two are finished where they are, where the product of 700 rows and
+// 2 x 8,192 of 2,048 columns wrote 46 MB for a kernel of 16 us that read them again (with it 9.33, so 9.11 ms for such a prompt
+// through 16 layers).
+enum { STREAM_Y = 0, STREAM_PARTS = 1, STREAM_GLU = 2 };
 
 // Tiles of BM rows of x and BN of W; four waves multiply, each all rows of x and a quarter of W's, PW bring the operands, a block
 // of 32 columns at a time into one of NB buffers. W lies in LDS as it is in memory and is split by the wave that
@@ -562,9 +569,12 @@ struct StreamArgs {
 // of 18 clocks take 0.72, and 1.23 with all compute units at work, 40 KB from L2 each. (Without the
 // order by hand the compiler moves the splitting and the sums behind all products of the block: 1.11 us; with two
 // loading waves 700 x 16,384 x 2,048 takes 284 us, with four 240; x split by every workgroup 308 at best.)
-template <int BM, int BN, int NB, int PW, bool PARTS>
+template <int BM, int BN, int NB, int PW, int MODE>
 __global__ void __launch_bounds__(64 * (4 + PW))
 gemm_f32_stream_kernel(const StreamArgs a) {
+  constexpr bool PARTS = MODE == STREAM_PARTS, GLU = MODE == STREAM_GLU;
+  constexpr int COLS = GLU ? BN / 2 : BN;        // columns of y a tile gives
+  static_assert(!GLU || BN == 128, "a wave has 16 rows of either");
   constexpr int TM = BM / 16, TN = BN / 64;
   constexpr int ROWS = BN + BM + BM / 2, CHUNK = ROWS * TILE_ROW;
   extern __shared__ __align__(16) unsigned char lds[];
@@ -578,7 +588,7 @@ gemm_f32_stream_kernel(const StreamArgs a) {
   auto place = [&](int t, int& m0, int& n0, int& kb, int& chunks) __attribute__((always_inline)) {
     const int each = a.tiles_m * a.tiles_n, split = t / each, u = t - split * each;
     const int tn = u / a.tiles_m;
-    n0 = tn * BN;
+    n0 = tn * COLS;
     m0 = (u - tn * a.tiles_m) * BM;
     kb = split * a.per;
     chunks = (min(K, kb + a.per) - kb) / SPLIT_BK;
@@ -602,7 +612,10 @@ gemm_f32_stream_kernel(const StreamArgs a) {
         for (int i = 0; i < LI; ++i) {
           const int r = 8 * (first + i) + lrow;
           const char* p;
-          if (8 * (first + i) < BN) p = reinterpret_cast<const char*>(a.w + (size_t)min(n0 + r, N - 1) * K + kb);
+          if (8 * (first + i) < BN) {
+            const int row = GLU ? min(n0 + 16 * (r >> 5) + (r & 15), N - 1) + (r & 16 ? N : 0) : min(n0 + r, N - 1);
+            p = reinterpret_cast<const char*>(a.w + (size_t)row * K + kb);
+          }
           else if (8 * (first + i) < BN + BM) p = reinterpret_cast<const char*>(xb + (size_t)(m0 + r - BN) * 128);
           else p = reinterpret_cast<const char*>(xb + (size_t)a.Mp * 128 + (size_t)(m0 / 2 + r - BN - BM) * 128);
           src[i] = p + 16 * lpiece;
@@ -766,7 +779,41 @@ gemm_f32_stream_kernel(const StreamArgs a) {
         for (int j = 0; j < TN; ++j) wa[j] = wb[j];
       }
     }
-    if (!PARTS && !store(a.y, a.ldy, sum)) {
+    if (GLU) {
+      // (plain_dot written out for each of the 64 sums cost 4 us a tile in code alone: which of them want it is noted first)
+      const int c = n0 + 16 * wave + 4 * lg;     // (N is a multiple of 4)
+      unsigned odd[2] = {0, 0};
+#pragma unroll
+      for (int i = 0; i < TM; ++i) {
+        const int m = m0 + 16 * i + ln;
+        if (m >= M || c >= N) continue;
+        f32x4_t out;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          out[e] = glu_act(a.act, sum[0][i][e]) * sum[TN - 1][i][e];
+          odd[0] |= is_finite(sum[0][i][e]) ? 0u : 1u << (4 * i + e);
+          odd[1] |= is_finite(sum[TN - 1][i][e]) ? 0u : 1u << (4 * i + e);
+        }
+        *reinterpret_cast<f32x4_t*>(a.y + (size_t)m * a.ldy + c) = out;
+      }
+      for (unsigned left = odd[0] | odd[1]; left; left &= left - 1) {
+        const int k = __builtin_ctz(left);
+        const size_t m = m0 + 16 * (k >> 2) + ln, col = c + (k & 3);
+        float g = 0.f, u = 0.f;
+#pragma unroll
+        for (int q = 0; q < 4 * TM; ++q) {
+          g = q == k ? sum[0][q >> 2][q & 3] : g;
+          u = q == k ? sum[TN - 1][q >> 2][q & 3] : u;
+        }
+#pragma unroll 1
+        for (int side = 0; side < 2; ++side) {
+          if (!(odd[side] >> k & 1)) continue;
+          const float v = plain_dot(a.x + m * a.ldx, a.w + (side * (size_t)N + col) * K, K);
+          if (side) u = v; else g = v;
+        }
+        a.y[m * a.ldy + col] = glu_act(a.act, g) * u;
+      }
+    } else if (!PARTS && !store(a.y, a.ldy, sum)) {
 #pragma unroll 1
       for (int i = 0; i < TM; ++i)
 #pragma unroll 1
@@ -793,16 +840,19 @@ struct TilePlan {
   int bm, bn;                                    // rows of x and of W a tile
   int per;                                       // columns a workgroup
   int per_cu;
+  float us;
 };
 
-static TilePlan tile_plan(int M, int N, int K) {
+// pairs: W is [Wg; Wu] and the pairs are finished in the tile, for which K is not cut
+static TilePlan tile_plan(int M, int N, int K, bool pairs = false) {
   const int cus = compute_units();
   const int width = span_width(K), spans = (K + width - 1) / width;
   TilePlan best{};
   double least = 1e30;
   auto offer = [&](int tile, int bm, int bn, int per_cu, float block, float full) {
     const long tiles = (long)((N + bn - 1) / bn) * ((M + bm - 1) / bm);
-    for (int splits = 1; splits <= spans; ++splits) {
+    if (pairs && bn != 128) return;
+    for (int splits = 1; splits <= (pairs ? 1 : spans); ++splits) {
       const int per = (spans + splits - 1) / splits * width;
       if ((long)per * (splits - 1) >= K) continue;
       const long places = (long)cus * per_cu, all = tiles * splits, rounds = (all + places - 1) / places;
@@ -811,7 +861,7 @@ static TilePlan tile_plan(int M, int N, int K) {
       if (splits > 1) t += 4.0 + 4.0 * M * N * (spans + 1) / 6e6;
       if (t < least) {
         least = t;
-        best = {tile, bm, bn, per, per_cu};
+        best = {tile, bm, bn, per, per_cu, (float)t};
       }
     }
   };
@@ -833,13 +883,13 @@ static long split_rows_floats(const TilePlan& plan, int M, int K) {
   return plan.tile < 0 ? 0 : (long)(split_rows_bytes(padded_rows(M)) / 4) * (K / SPLIT_BK);
 }
 
-template <int BM, int BN, int NB, bool PARTS> static int launch_stream(const StreamArgs& a, int per_cu, hipStream_t st) {
+template <int BM, int BN, int NB, int MODE> static int launch_stream(const StreamArgs& a, int per_cu, hipStream_t st) {
   constexpr size_t lds = (size_t)NB * (BN + BM + BM / 2) * TILE_ROW;
   static LdsAllowance allowance;
-  if (!allowance.ask((const void*)gemm_f32_stream_kernel<BM, BN, NB, LOADERS, PARTS>, lds)) return PTL_ERR_LAUNCH;
+  if (!allowance.ask((const void*)gemm_f32_stream_kernel<BM, BN, NB, LOADERS, MODE>, lds)) return PTL_ERR_LAUNCH;
   const long tiles = (long)a.tiles_m * a.tiles_n * a.splits;
   const unsigned grid = (unsigned)min(tiles, (long)compute_units() * per_cu);
-  gemm_f32_stream_kernel<BM, BN, NB, LOADERS, PARTS><<<grid, 64 * (4 + LOADERS), lds, st>>>(a);
+  gemm_f32_stream_kernel<BM, BN, NB, LOADERS, MODE><<<grid, 64 * (4 + LOADERS), lds, st>>>(a);
   return ptl_launch_status();
 }
 
@@ -860,11 +910,11 @@ static int launch_tiles(float* y, const float* x, const float* w, int M, int N, 
     const int Mp = padded_rows(M);
     unsigned char* xs = reinterpret_cast<unsigned char*>(work);
     split_rows_kernel<<<dim3((M + 63) / 64, K / SPLIT_BK), 256, 0, st>>>(xs, x, M, K, ldx, Mp);
-    const StreamArgs a{y, parts, x, w, xs, M, N, K, Mp, ldx, ldy, tiles_m, tiles_n, splits, plan.per, width};
+    const StreamArgs a{y, parts, x, w, xs, M, N, K, Mp, ldx, ldy, tiles_m, tiles_n, splits, plan.per, width, 0};
     int rc = PTL_ERR_ARG, n = 0;
 #define T(BM, BN, NB, CU, BLOCK, FULL)                                                                   \
   if (plan.tile == n++)                                                                                  \
-    rc = parts ? launch_stream<BM, BN, NB, true>(a, CU, st) : launch_stream<BM, BN, NB, false>(a, CU, st);
+    rc = parts ? launch_stream<BM, BN, NB, STREAM_PARTS>(a, CU, st) : launch_stream<BM, BN, NB, STREAM_Y>(a, CU, st);
     STREAM_TILES(T)
 #undef T
     if (rc != PTL_OK) return rc;
@@ -891,4 +941,34 @@ extern "C" int ptl_gemm_f32(float* y, const float* x, const float* w, int M, int
   const TilePlan plan = tile_plan(M, N, K);
   if ((plan.tile >= 0 || plan.per < K) && (work == nullptr || !aligned16(work))) return PTL_ERR_ARG;
   return launch_tiles(y, x, w, M, N, K, ldx, ldy, plan, work, st);
+}
+
+// Whether ptl_gate_up_f32_tiles is the faster way for M rows of x and W = [Wg; Wu] [2 I, K]: what the plans say, the activation's
+// kernel taking 3 us and its 12 bytes a result at 5 TB/s (700 rows, 2 x 8,192 x 2,048: 15 to 16 us).
+extern "C" int ptl_gate_up_f32_tiles_fits(int M, int I, int K) {
+  if (M <= 0 || I <= 0 || I % 4 || K <= 0 || K % SPLIT_BK) return 0;
+  return tile_plan(M, 2 * I, K, true).us <= tile_plan(M, 2 * I, K).us + 3.0f + 12.0f * M * I / 5e6f;
+}
+
+// floats of workspace it wants
+extern "C" long ptl_gate_up_f32_tiles_workspace(int M, int I, int K) {
+  return M <= 0 || I <= 0 || K <= 0 ? 0 : split_rows_floats(tile_plan(M, 2 * I, K, true), M, K);
+}
+
+// out [M, I] = act(x Wg^T) * (x Wu^T), the bits of the product and the activation by themselves. K % 32 == 0, I % 4 == 0, ldx % 4
+// == 0, 16-byte aligned rows and workspace.
+extern "C" int ptl_gate_up_f32_tiles(float* out, const float* x, const float* w, int M, int I, int K, long ldx, int act,
+                                     float* work, hipStream_t st) {
+  if (M <= 0) return PTL_OK;
+  if (I <= 0 || I % 4 || K <= 0 || K % SPLIT_BK || (M > 1 && ldx % 4) || ldx < K || !aligned16(out) || !aligned16(x) ||
+      !aligned16(w) || !work || !aligned16(work) || (act != GLU_SILU && act != GLU_GELU_TANH))
+    return PTL_ERR_ARG;
+  const TilePlan plan = tile_plan(M, 2 * I, K, true);
+  const int tiles_m = (M + plan.bm - 1) / plan.bm, tiles_n = (I + 63) / 64, Mp = padded_rows(M);
+  if ((long)tiles_m * tiles_n > 0x3fffffff) return PTL_ERR_ARG;
+  unsigned char* xs = reinterpret_cast<unsigned char*>(work);
+  split_rows_kernel<<<dim3((M + 63) / 64, K / SPLIT_BK), 256, 0, st>>>(xs, x, M, K, ldx, Mp);
+  const StreamArgs a{out, nullptr, x, w, xs, M, I, K, Mp, ldx, I, tiles_m, tiles_n, 1, K, span_width(K), act};
+  if (plan.bm == 128) return launch_stream<128, 128, 4, STREAM_GLU>(a, 1, st);
+  return launch_stream<64, 128, 5, STREAM_GLU>(a, 1, st);
 }

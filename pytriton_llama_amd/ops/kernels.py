@@ -280,6 +280,32 @@ def gate_up_f32(x: torch.Tensor, w: torch.Tensor, act: int = GLU_SILU) -> torch.
     return out
 
 
+def gate_up_f32_tiles_fits(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether ``gate_up_f32_tiles`` takes x with w = [Wg; Wu] and is the faster way for it: a prompt's rows."""
+    if not (x.dim() == 2 and x.shape[0] > F32_FEW_ROWS and x.is_cuda and x.dtype == torch.float32 and w.is_cuda
+            and w.dtype == torch.float32 and w.dim() == 2 and w.is_contiguous() and w.shape[1] == x.shape[1]
+            and x.shape[1] % 32 == 0 and x.shape[1] > 0 and w.shape[0] % 8 == 0 and w.shape[0] > 0 and x.stride(1) == 1
+            and x.stride(0) % 4 == 0 and x.stride(0) >= x.shape[1] and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0):
+        return False
+    return bool(library.load("gemm_f32").ptl_gate_up_f32_tiles_fits(x.shape[0], w.shape[0] // 2, x.shape[1]))
+
+
+def gate_up_f32_tiles(x: torch.Tensor, w: torch.Tensor, act: int = GLU_SILU) -> torch.Tensor:
+    """As ``gate_up_f32`` for a prompt's rows: the bits of ``silu_mul(gemm_nt(x, w), act)``, whose [M, 2 I] product is never
+    stored (csrc/gemm_f32.hip)."""
+    if not gate_up_f32_tiles_fits(x, w):
+        raise KernelError("gate_up_f32_tiles: needs float32 x [M, K] of more than 16 rows and contiguous w [2 I, K], K a multiple "
+                          "of 32, I of 4, 16-byte aligned rows, and sizes for which it is the faster way")
+    (M, K), I = x.shape, w.shape[0] // 2
+    lib = library.load("gemm_f32")
+    lib.ptl_gate_up_f32_tiles_workspace.restype = ctypes.c_long
+    work = torch.empty(lib.ptl_gate_up_f32_tiles_workspace(M, I, K), dtype=torch.float32, device=x.device)
+    out = torch.empty((M, I), dtype=torch.float32, device=x.device)
+    _check(lib.ptl_gate_up_f32_tiles(_ptr(out), _ptr(x), _ptr(w), M, I, K, ctypes.c_long(x.stride(0)), int(act), _ptr(work),
+                                     _stream()), "gate_up_f32_tiles")
+    return out
+
+
 def qkv_rope_store_f32_fits(x: torch.Tensor, w: torch.Tensor, head_dim: int) -> bool:
     """Whether ``qkv_rope_store_f32`` takes x."""
     return head_dim % 8 == 0 and _f32_pairs_ok(x, w)

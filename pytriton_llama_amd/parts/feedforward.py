@@ -63,6 +63,8 @@ class SwiGLU(Part):
             return linear(a, self.down, blocked=self.down_blocked)
         if ops.gate_up_f32_fits(x, self.gate_up):           # ... in float32
             a = ops.gate_up_f32(x, self.gate_up, self.act)
+        elif ops.gate_up_f32_tiles_fits(x, self.gate_up):   # ... and of a prompt in float32
+            a = ops.gate_up_f32_tiles(x, self.gate_up, self.act)
         elif ops.gate_up_tile_fits(x, self.gate_up):        # some hundred rows: the same in tiles
             a = ops.gate_up_tile(x, self.gate_up, self.act, hw_silu=True)
         else:

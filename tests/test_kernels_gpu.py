@@ -800,6 +800,23 @@ def test_gate_up_f32(ops, mik):
         ops.gate_up_f32(x, w[:-2])
 
 
+@pytest.mark.parametrize("mik", [(700, 8192, 2048), (17, 4096, 64), (128, 20, 96), (129, 68, 64), (301, 2816, 1024),
+                                 (1030, 1028, 1024), (64, 12000, 32)])
+def test_gate_up_f32_tiles(ops, mik):
+    """A prompt's gate-up product with its activation, in either tile and where a tile has columns past the end: the bits of
+    the product and the activation by themselves, also of what is not finite."""
+    M, I, K = mik
+    torch.manual_seed(49)
+    x = torch.randn(M, K + 4, device="cuda")[:, :K]
+    w = torch.randn(2 * I, K, device="cuda") / math.sqrt(K)
+    x[M - 1, K - 1] = float("inf")
+    w[I - 1, 0] = 3.4e38
+    for act in (ops.GLU_SILU, ops.GLU_GELU_TANH):
+        got, want = ops.gate_up_f32_tiles(x, w, act), ops.silu_mul(ops.gemm_nt(x, w), act)
+        assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.nan_to_num(7.0), want.nan_to_num(7.0))
+    assert not ops.gate_up_f32_tiles_fits(x[:16], w) and not ops.gate_up_f32_tiles_fits(x[:, :K - 4], w[:, :K - 4].contiguous())
+
+
 @pytest.mark.parametrize("rotated", [True, False])
 @pytest.mark.parametrize("case", [(1, 2, 1, 8, 64), (4, 32, 8, 64, 2048), (8, 3, 3, 128, 516), (5, 5, 1, 40, 4100),
                                   (3, 8, 2, 16, 8192)])
