@@ -468,7 +468,9 @@ moe_gemm_kernel(T* __restrict__ out, long ldo, const T* __restrict__ x, long ldx
 // The same products in float32 on the matrix cores (K % 4 == 0, aligned rows; split_f32.h): 64 sorted rows x 64
 // result columns a workgroup of four waves, a wave all rows and 16 columns of every product, so that the gate and the up row
 // of a result meet in one lane. 966 pairs of 16 experts of 2,048 x 2,048 (one MI355X, us; on the float32 matrix
-// instructions and in the vector form in brackets): gate|up 190 (231, 691), down 107 (130, 419).
+// instructions and in the vector form in brackets): gate|up 176 (231, 691), down 91 (130, 419): 805 MB of weights in all at
+// 3 TB/s, those of an expert with more than 64 rows twice. Loading waves that bring them through LDS are slower (320 to 366 us for
+// both and the kernels around them, 293 to 301 so).
 template <int MODE>
 __global__ void __launch_bounds__(256, 3)
 moe_gemm_f32_kernel(float* __restrict__ out, long ldo, const float* __restrict__ x, long ldx, const float* __restrict__ w,

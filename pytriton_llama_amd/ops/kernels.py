@@ -208,8 +208,8 @@ def rope_store(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, positions: tor
 
 def gemm_nt(x: torch.Tensor, w: torch.Tensor, out_dtype: Optional[torch.dtype] = None,
             out: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """y = x @ w.T with float32 accumulation: float32 operands with 16-byte aligned rows through the
-    32-bit matrix instructions (csrc/gemm_f32.hip), everything else through the vector-FMA kernel;
+    """y = x @ w.T with float32 accumulation: float32 operands with 16-byte aligned rows as three exact
+    bfloat16 parts each on the matrix cores (csrc/gemm_f32.hip), everything else through the vector-FMA kernel;
     in both the bits of a row of y do not depend on the other rows of x, nor on how many there are.
     x [M, K] (rows may be strided), w [N, K] contiguous, same dtype."""
     _need_gpu(x, w)
