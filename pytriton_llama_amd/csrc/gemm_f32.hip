@@ -49,14 +49,19 @@ __host__ __device__ static inline int span_width(int K) {
 template <int ROWS, int MT>
 __device__ __forceinline__ void few_results(float* __restrict__ y, const float* __restrict__ x, const float* __restrict__ w,
                                             const float* sums, int spans, int M, int N, int K, int n0, long ldx, long ldy) {
+  static_assert(ROWS * ROWS * MT % 64 == 0, "whole waves");
   for (int i = threadIdx.x; i < ROWS * ROWS * MT; i += blockDim.x) {
     const int n = i % ROWS, m = i / ROWS, t = m / ROWS, j = m % ROWS;
-    if (m >= M || n0 + n >= N) continue;
+    const bool there = m < M && n0 + n < N;
     const float* p = sums + t * 256 + ((n >> 2) * 16 + j) * 4 + (n & 3);
     float s = 0.f;
     for (int sp = 0; sp < spans; ++sp, p += MT * 256) s += p[0];
-    if (!is_finite(s)) s = plain_dot(x + (size_t)m * ldx, w + (size_t)(n0 + n) * K, K);
-    y[(size_t)m * ldy + n0 + n] = s;
+    const bool odd = there && !is_finite(s);
+    if (__builtin_expect(__any(odd), 0)) {
+      bool nan_x = false;
+      s = plain_dots<1>(s, odd, x + (size_t)m * ldx, w + (size_t)(n0 + n) * K, K, nan_x);
+    }
+    if (there) y[(size_t)m * ldy + n0 + n] = s;
   }
 }
 
@@ -89,17 +94,28 @@ template <int FORM>
 __device__ __forceinline__ void pair_results(float* __restrict__ y, const float* __restrict__ x, const float* __restrict__ w,
                                              const float* sums, int spans, int M, int N, int K, int tile, long ldx, long ldy,
                                              const FewOut& o) {
-  for (int i = threadIdx.x; i < 32; i += blockDim.x) {
-    const int n = i & 3, m = i >> 2;
-    if (m >= M) continue;
+  int tid = threadIdx.x;
+  asm volatile("" : "+v"(tid));                  // (what follows of it is worked out here, for every tile: see plain_dots)
+  if (tid < 64) {                                // (the first wave, half of it with a pair each)
+    const int n = tid & 3, m = (tid >> 2) & 7;
+    const bool there = tid < 32 && m < M;
     const float *p = sums + m * 4 + n, *p2 = p + 16 * 4;
     float a = 0.f, b = 0.f;
     for (int sp = 0; sp < spans; ++sp, p += 256, p2 += 256) {
       a += p[0];
       b += p2[0];
     }
-    if (!is_finite(a)) a = plain_dot(x + (size_t)m * ldx, w + (size_t)few_row<FORM, 8>(o, tile, n, N) * K, K);
-    if (!is_finite(b)) b = plain_dot(x + (size_t)m * ldx, w + (size_t)few_row<FORM, 8>(o, tile, n + 4, N) * K, K);
+    if (__builtin_expect(__any(there && !(is_finite(a) && is_finite(b))), 0)) {
+      bool nan_x = false;
+#pragma unroll 1
+      for (int side = 0; side < 2; ++side) {
+        const float v = side ? b : a;
+        const float again = plain_dots<1>(v, there && !is_finite(v), x + (size_t)m * ldx,
+                                       w + (size_t)few_row<FORM, 8>(o, tile, n + 4 * side, N) * K, K, nan_x);
+        if (side) b = again; else a = again;
+      }
+    }
+    if (!there) return;
     const int pair = 4 * tile + n;
     if (FORM == FORM_GLU) {
       y[(size_t)m * ldy + pair] = glu_act(o.act, a) * b;
@@ -413,6 +429,33 @@ extern "C" int ptl_qkv_rope_store_f32(float* q_out, const float* x, const float*
 // either form 12 (8.6).
 // ===========================================================================
 
+// The results of a wave's tile that are not finite, made again: it has stored TM groups of 16 rows of x, from m0 on, and TN4
+// results a lane and group, of rows n0 + 16 (e / 4) + 4 lg + e % 4 of W; bit i of odd: one of this lane's results in group i.
+template <int TN4, int TM>
+__device__ __forceinline__ void tile_again(float* __restrict__ y, long ldy, unsigned odd, int m0, int n0, int M, int N,
+                                           const float* __restrict__ x, long ldx, const float* __restrict__ w, int K) {
+  const int lane = threadIdx.x & 63, ln = lane & 15, lg = lane >> 4;
+  if (__builtin_expect(!__any(odd), 1)) return;
+#pragma unroll 1
+  for (int i = 0; i < TM; ++i) {
+    if (!__any(odd >> i & 1)) continue;
+    const int m = m0 + 16 * i + ln;
+    const float* xr = x + (size_t)min(m, M - 1) * ldx;
+    bool nan_x = false;
+#pragma unroll 1
+    for (int e = 0; e < TN4; ++e) {
+      const int n = n0 + 16 * (e >> 2) + 4 * lg + (e & 3);
+      const bool there = m < M && n < N && (odd >> i & 1);
+      float* at = y + (size_t)m * ldy + n;
+      const float v = there ? *at : 0.f;         // (as this lane has stored it)
+      const bool again = there && !is_finite(v);
+      if (!__any(again)) continue;
+      const float s = plain_dots(v, again, xr, w + (size_t)min(n, N - 1) * K, K, nan_x);
+      if (again) *at = s;
+    }
+  }
+}
+
 // K not a multiple of 32 (700 x 16,384 x 2,048 320 us in this form).
 template <int TA, int TC, bool PARTS>
 __global__ void __launch_bounds__(256, 2)
@@ -439,7 +482,7 @@ gemm_f32_tile_kernel(float* __restrict__ y, const float* __restrict__ x, const f
   // results [M, N] of row stride ld, from D[n = 4 lg + i][m = ln] of every 16 x 16 tile
   auto store = [&](float* to, long ld, const f32x4_t (&v)[TA][TC]) __attribute__((always_inline)) {
     const bool four = (N & 3) == 0 && (ld & 3) == 0 && (reinterpret_cast<uintptr_t>(to) & 15) == 0;
-    bool finite = true;
+    unsigned odd = 0;                            // groups of 16 rows of x with a result that is not finite
 #pragma unroll
     for (int c = 0; c < TC; ++c) {
       const int m = m0 + 16 * c + ln;
@@ -456,10 +499,10 @@ gemm_f32_tile_kernel(float* __restrict__ y, const float* __restrict__ x, const f
             if (n + i < N) at[i] = v[a][c][i];
         }
 #pragma unroll
-        for (int i = 0; i < 4; ++i) finite = finite && is_finite(v[a][c][i]);
+        for (int i = 0; i < 4; ++i) odd |= is_finite(v[a][c][i]) ? 0u : 1u << c;
       }
     }
-    return finite;
+    return odd;
   };
   f32x4_t acc[TA][TC], sum[TA][TC];              // of the span, of the spans so far
 #pragma unroll
@@ -482,47 +525,51 @@ gemm_f32_tile_kernel(float* __restrict__ y, const float* __restrict__ x, const f
 #pragma unroll
       for (int c = 0; c < TC; ++c) acc[a][c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   });
-  if (!PARTS && !store(y, ldy, sum)) {
-    // (a thread's own results, as it stored them)
-#pragma unroll 1
-    for (int c = 0; c < TC; ++c)
-#pragma unroll 1
-      for (int a = 0; a < 4 * TA; ++a) {
-        const int m = m0 + 16 * c + ln, n = wn + 16 * (a >> 2) + 4 * lg + (a & 3);
-        if (m < M && n < N && !is_finite(y[(size_t)m * ldy + n]))
-          y[(size_t)m * ldy + n] = plain_dot(x + (size_t)m * ldx, w + (size_t)n * K, K);
-      }
-  }
+  if (!PARTS) tile_again<4 * TA, TC>(y, ldy, store(y, ldy, sum), m0, wn, M, N, x, ldx, w, K);
 }
 
 __global__ void __launch_bounds__(256)
 gemm_f32_sum_kernel(float* __restrict__ y, const float* __restrict__ parts, int spans, const float* __restrict__ x,
                     const float* __restrict__ w, int M, int N, int K, long ldx, long ldy) {
   const long total = (long)M * N;
-  if ((N & 3) == 0 && (ldy & 3) == 0 && (reinterpret_cast<uintptr_t>(y) & 15) == 0) {
-    const long i = ((long)blockIdx.x * 256 + threadIdx.x) * 4;
-    if (i >= total) return;
-    float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
+  const bool four = (N & 3) == 0 && (ldy & 3) == 0 && (reinterpret_cast<uintptr_t>(y) & 15) == 0;
+  const long first = four ? ((long)blockIdx.x * 256 + threadIdx.x) * 4 : (long)blockIdx.x * 1024 + threadIdx.x;
+  const int step = four ? 1 : 256;               // a thread has four results, ``step`` apart
+  f32x4_t s = {0.f, 0.f, 0.f, 0.f};
+  if (four) {
+    if (first < total)
 #pragma unroll 4
-    for (int p = 0; p < spans; ++p) {
-      const float4 v = *reinterpret_cast<const float4*>(parts + (size_t)p * total + i);
-      s.x += v.x; s.y += v.y; s.z += v.z; s.w += v.w;
-    }
-    const long m = i / N, n = i % N;
-    float f[4] = {s.x, s.y, s.z, s.w};
+      for (int p = 0; p < spans; ++p) s += *reinterpret_cast<const f32x4_t*>(parts + (size_t)p * total + first);
+  } else {
 #pragma unroll
     for (int j = 0; j < 4; ++j)
-      if (!is_finite(f[j])) f[j] = plain_dot(x + m * ldx, w + (n + j) * K, K);
-    *reinterpret_cast<float4*>(y + m * ldy + n) = make_float4(f[0], f[1], f[2], f[3]);
-    return;
+      if (first + j * step < total)
+        for (int p = 0; p < spans; ++p) s[j] += parts[(size_t)p * total + first + j * step];
   }
-  for (int j = 0; j < 4; ++j) {
-    const long i = (long)blockIdx.x * 1024 + j * 256 + threadIdx.x;
-    if (i >= total) return;
-    float s = 0.f;
-    for (int p = 0; p < spans; ++p) s += parts[(size_t)p * total + i];
-    if (!is_finite(s)) s = plain_dot(x + i / N * ldx, w + i % N * K, K);
-    y[i / N * ldy + i % N] = s;
+  if (__builtin_expect(__any(!(is_finite(s[0]) && is_finite(s[1]) && is_finite(s[2]) && is_finite(s[3]))), 0)) {
+    bool nan_x = false;
+    long last = -1;
+#pragma unroll 1
+    for (int j = 0; j < 4; ++j) {
+      const long i = first + j * step;
+      const float v = j == 0 ? s[0] : j == 1 ? s[1] : j == 2 ? s[2] : s[3];
+      const bool odd = i < total && !is_finite(v);
+      const long m = odd ? i / N : 0, n = odd ? i % N : 0;
+      if (m != last) nan_x = false;
+      last = m;
+      const float again = plain_dots(v, odd, x + m * ldx, w + n * K, K, nan_x);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) s[e] = e == j ? again : s[e];
+    }
+  }
+  if (four) {
+    if (first < total) *reinterpret_cast<f32x4_t*>(y + first / N * ldy + first % N) = s;
+  } else {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const long i = first + j * step;
+      if (i < total) y[i / N * ldy + i % N] = s[j];
+    }
   }
 }
 
@@ -687,7 +734,7 @@ gemm_f32_stream_kernel(const StreamArgs a) {
       for (int i = 0; i < TM; ++i) acc[j][i] = sum[j][i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     auto store = [&](float* to, long ld, const f32x4_t (&v)[TN][TM]) __attribute__((always_inline)) {
       const bool four = (N & 3) == 0 && (ld & 3) == 0 && (reinterpret_cast<uintptr_t>(to) & 15) == 0;
-      bool finite = true;
+      unsigned odd = 0;                          // groups of 16 rows of x with a result that is not finite
 #pragma unroll
       for (int i = 0; i < TM; ++i) {
         const int m = m0 + 16 * i + ln;
@@ -704,10 +751,10 @@ gemm_f32_stream_kernel(const StreamArgs a) {
               if (c + e < N) at[e] = v[j][i][e];
           }
 #pragma unroll
-          for (int e = 0; e < 4; ++e) finite = finite && is_finite(v[j][i][e]);
+          for (int e = 0; e < 4; ++e) odd |= is_finite(v[j][i][e]) ? 0u : 1u << i;
         }
       }
-      return finite;
+      return odd;
     };
     // one chunk; its weights' parts are in ws, those of the next go to wn
     auto chunk = [&](int c, Split (&ws)[TN], Split (&wn)[TN]) __attribute__((always_inline)) {
@@ -780,7 +827,7 @@ gemm_f32_stream_kernel(const StreamArgs a) {
       }
     }
     if (GLU) {
-      // (plain_dot written out for each of the 64 sums cost 4 us a tile in code alone: which of them want it is noted first)
+      // (the sums made again in one place, for each of the 64: written out for each they cost 4 us a tile in code alone)
       const int c = n0 + 16 * wave + 4 * lg;     // (N is a multiple of 4)
       unsigned odd[2] = {0, 0};
 #pragma unroll
@@ -796,32 +843,31 @@ gemm_f32_stream_kernel(const StreamArgs a) {
         }
         *reinterpret_cast<f32x4_t*>(a.y + (size_t)m * a.ldy + c) = out;
       }
-      for (unsigned left = odd[0] | odd[1]; left; left &= left - 1) {
-        const int k = __builtin_ctz(left);
-        const size_t m = m0 + 16 * (k >> 2) + ln, col = c + (k & 3);
-        float g = 0.f, u = 0.f;
+      if (__builtin_expect(__any(odd[0] | odd[1]), 0)) {
+        bool nan_x = false;
+#pragma unroll 1
+        for (int k = 0; k < 4 * TM; ++k) {
+          if (k % 4 == 0) nan_x = false;         // (other rows of x)
+          const bool again = (odd[0] | odd[1]) >> k & 1;
+          if (!__any(again)) continue;
+          const size_t m = min(m0 + 16 * (k >> 2) + ln, M - 1), col = min(c, N - 4) + (k & 3);
+          float g = 0.f, u = 0.f;
 #pragma unroll
-        for (int q = 0; q < 4 * TM; ++q) {
-          g = q == k ? sum[0][q >> 2][q & 3] : g;
-          u = q == k ? sum[TN - 1][q >> 2][q & 3] : u;
-        }
+          for (int q = 0; q < 4 * TM; ++q) {
+            g = q == k ? sum[0][q >> 2][q & 3] : g;
+            u = q == k ? sum[TN - 1][q >> 2][q & 3] : u;
+          }
 #pragma unroll 1
-        for (int side = 0; side < 2; ++side) {
-          if (!(odd[side] >> k & 1)) continue;
-          const float v = plain_dot(a.x + m * a.ldx, a.w + (side * (size_t)N + col) * K, K);
-          if (side) u = v; else g = v;
+          for (int side = 0; side < 2; ++side) {
+            const float v = plain_dots(side ? u : g, odd[side] >> k & 1, a.x + m * a.ldx,
+                                       a.w + (side * (size_t)N + col) * K, K, nan_x);
+            if (side) u = v; else g = v;
+          }
+          if (again) a.y[m * a.ldy + col] = glu_act(a.act, g) * u;
         }
-        a.y[m * a.ldy + col] = glu_act(a.act, g) * u;
       }
-    } else if (!PARTS && !store(a.y, a.ldy, sum)) {
-#pragma unroll 1
-      for (int i = 0; i < TM; ++i)
-#pragma unroll 1
-        for (int e = 0; e < 4 * TN; ++e) {
-          const int m = m0 + 16 * i + ln, c = n0 + 16 * TN * wave + 16 * (e >> 2) + 4 * lg + (e & 3);
-          if (m < M && c < N && !is_finite(a.y[(size_t)m * a.ldy + c]))
-            a.y[(size_t)m * a.ldy + c] = plain_dot(a.x + (size_t)m * a.ldx, a.w + (size_t)c * K, K);
-        }
+    } else if (!PARTS) {
+      tile_again<4 * TN, TM>(a.y, a.ldy, store(a.y, a.ldy, sum), m0, n0 + 16 * TN * wave, M, N, a.x, a.ldx, a.w, K);
     }
   }
 }

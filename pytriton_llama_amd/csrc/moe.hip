@@ -502,6 +502,10 @@ moe_gemm_f32_kernel(float* __restrict__ out, long ldo, const float* __restrict__
     for (int c = 0; c < TC; ++c) acc[g][c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   split_tile<G, TC>(lds, wp, xp, 0, K, (K + SPLIT_BK - 1) / SPLIT_BK * SPLIT_BK, acc, [](int) {},
                     (rows + 15) / 16);
+  auto result = [&](const float (&v)[G], float f) __attribute__((always_inline)) {
+    return GATE_UP ? gated_act(act, v[0] * f, v[G - 1] * f, limit) : (MODE == MODE_UP ? unary_act(act, v[0] * f) : v[0]);
+  };
+  unsigned odd[G] = {};                                    // sums that are not finite, by place
 #pragma unroll
   for (int c = 0; c < TC; ++c) {
     const int m = 16 * c + ln;
@@ -516,10 +520,33 @@ moe_gemm_f32_kernel(float* __restrict__ out, long ldo, const float* __restrict__
 #pragma unroll
       for (int g = 0; g < G; ++g) {
         v[g] = acc[g][c][i];
-        if (!is_finite(v[g])) v[g] = plain_dot(x_row(m), w + ((size_t)g * N + n) * K, K);
+        odd[g] |= is_finite(v[g]) ? 0u : 1u << (4 * c + i);
       }
-      orow[n] = GATE_UP ? gated_act(act, v[0] * f, v[G - 1] * f, limit) : (MODE == MODE_UP ? unary_act(act, v[0] * f) : v[0]);
+      orow[n] = result(v, f);
     }
+  }
+  if (__builtin_expect(!__any(odd[0] | odd[G - 1]), 1)) return;
+  bool nan_x = false;
+#pragma unroll 1
+  for (int k = 0; k < 4 * TC; ++k) {
+    if (k % 4 == 0) nan_x = false;                         // (other rows of x)
+    const bool again = (odd[0] | odd[G - 1]) >> k & 1;
+    if (!__any(again)) continue;
+    const int m = min(16 * (k >> 2) + ln, rows - 1), n = min(n0 + 4 * lg + (k & 3), N - 1);
+    float v[G];
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      v[g] = 0.f;
+#pragma unroll
+      for (int q = 0; q < 4 * TC; ++q) v[g] = q == k ? acc[g][q >> 2][q & 3] : v[g];
+    }
+#pragma unroll 1
+    for (int g = 0; g < G; ++g) {
+      const float s = plain_dots<1>(g ? v[G - 1] : v[0], (g ? odd[G - 1] : odd[0]) >> k & 1, x_row(m),
+                                    w + ((size_t)g * N + n) * K, K, nan_x);
+      if (g) v[G - 1] = s; else v[0] = s;
+    }
+    if (again) out[(size_t)(row0 + m) * ldo + n] = result(v, GATHER && wgt ? wgt[sorted[row0 + m]] : 1.f);
   }
 }
 

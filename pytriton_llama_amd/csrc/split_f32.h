@@ -13,7 +13,7 @@
 // What is lost: the last part of numbers below 2^-110 may be too small for bfloat16.
 //
 // What is not finite: inf - inf in the split makes a NaN of every sum that an infinite (or nearly infinite) number enters.
-// Whoever stores a result that is not finite works it out again by plain_dot.
+// A result that is not finite is worked out again by plain_dots.
 //
 // v_mfma_f32_16x16x32_bf16: lane l (ln = l % 16, lg = l / 16) holds eight columns of A[ln] and of B[ln] and gets
 // D[4 lg + i][ln]. Which columns a lane group holds is free as long as A and B agree: here 4 lg .. + 3 and 16 + 4 lg .. + 3,
@@ -77,12 +77,73 @@ __device__ __forceinline__ f32x4_t split_dot(const Split& a, const Split& b) {
 
 __device__ __forceinline__ bool is_finite(float v) { return (__float_as_uint(v) & 0x7f800000u) != 0x7f800000u; }
 
-// The sum of K products in float32, one after the other.
-__device__ __forceinline__ float plain_dot(const float* __restrict__ a, const float* __restrict__ b, int K) {
-  float s = 0.f;
+// The sums of products that the lanes with ``want`` have of their row of x and their row of W (K columns in steps of 4, 16-byte
+// aligned), in float32; the other lanes keep v. The whole wave calls, and makes one sum after the other: a lane takes every
+// 64th 16-byte piece of the rows (EACH of them under way, which the bits do not depend on), and the lanes' sums meet in a butterfly, so that the bits depend on the two rows alone. A
+// row with a NaN in it is found with the first of its sums and gives NaN to all others that want it; nan_x keeps that of this
+// lane's row of x for the caller's next call. Where such a sum is wanted is rare, and its cost has to be bounded: a NaN in
+// one request's row reaches every result of that row in all products that follow. (One MI355X, us, 300 x 2,048 x 2,048 with a NaN,
+// with an infinity in one row of x, and without: 46, 734, 43; 4 x 16,384 x 2,048 42, 188, 34. By the lane that
+// owns the result, one column after the other: 1,133 and 705 with either. An infinity costs a sum of 2 to 3 us for every result of its row.)
+template <int EACH = 2> __device__ __forceinline__ float plain_dots(float v, bool want, const float* x, const float* w, int K, bool& nan_x) {
+  // (The lane and the NaN are made of a zero that the compiler does not know: worked out ahead of the loop around such a call
+  // they take registers that a kernel with loads under way does not have, and their way back from memory waits for those
+  // loads: gate-up of one row 28.4 -> 32.9 us.)
+  unsigned zero = 0;
+  asm volatile("" : "+s"(zero));
+  const int lane = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, zero));
+  const float nan = __uint_as_float(0x7fc00000u + zero);
+  if (want && nan_x) {
+    v = nan;
+    want = false;
+  }
+  for (unsigned long long left = __ballot(want); left; left = __ballot(want)) {
+    const int owner = __builtin_ctzll(left);
+    auto of_owner = [&](const float* p) __attribute__((always_inline)) {
+      const uint64_t b = reinterpret_cast<uint64_t>(p);
+      const uint32_t lo = __builtin_amdgcn_readlane((int)b, owner), hi = __builtin_amdgcn_readlane((int)(b >> 32), owner);
+      return reinterpret_cast<const float*>((uint64_t)hi << 32 | lo);
+    };
+    const float *xr = of_owner(x), *wr = of_owner(w);
+    float s = 0.f;
+    bool nan_in_x = false, nan_in_w = false;
 #pragma unroll 1
-  for (int k = 0; k < K; ++k) s = fmaf(a[k], b[k], s);
-  return s;
+    for (int k0 = 0; k0 < K; k0 += 256 * EACH) {
+      F4 a[EACH], b[EACH];
+#pragma unroll
+      for (int h = 0; h < EACH; ++h) {
+        const int k = k0 + 256 * h + 4 * lane;
+        a[h].u = k < K ? load16(xr + k) : zero16();
+        b[h].u = k < K ? load16(wr + k) : zero16();
+      }
+#pragma unroll
+      for (int h = 0; h < EACH; ++h)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          nan_in_x = nan_in_x || a[h].f[i] != a[h].f[i];
+          nan_in_w = nan_in_w || b[h].f[i] != b[h].f[i];
+          s = fmaf(a[h].f[i], b[h].f[i], s);
+        }
+      if (__any(s != s)) break;                  // (no later product makes a number of it)
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1)
+      s += __int_as_float(__builtin_amdgcn_ds_bpermute(4 * (lane ^ o), __float_as_int(s)));
+    if (lane == owner) {
+      v = s;
+      want = false;
+    }
+    if (__any(nan_in_x) && x == xr) {
+      nan_x = true;
+      if (want) v = nan;
+      want = false;
+    }
+    if (__any(nan_in_w) && w == wr) {
+      if (want) v = nan;
+      want = false;
+    }
+  }
+  return v;
 }
 
 // Tiles of 64 TA rows of W (or TA times 64 rows of different matrices) x 16 TC rows of x, a workgroup of four waves. A wave

@@ -181,6 +181,101 @@ def test_gemm_f32_streamed_tiles(ops, mnk):
         assert ((y - want[:rows]).abs() <= bound).all()
 
 
+def _gpu_us(fn, times=5):
+    """The fastest of some calls, in us."""
+    fn()
+    best = math.inf
+    for _ in range(times):
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        a.record()
+        fn()
+        b.record()
+        b.synchronize()
+        best = min(best, 1e3 * a.elapsed_time(b))
+    return best
+
+
+@pytest.mark.parametrize("mnk", [(4, 16384, 2048), (8, 2048, 8192), (16, 3072, 2048), (64, 2048, 2048), (300, 4096, 1024),
+                                 (260, 2500, 1028)])
+def test_gemm_f32_with_a_nan_is_not_slow(ops, mnk):
+    """A NaN in one row of x makes every result of the row one; the product takes about as long as without it (four times
+    as long is allowed here; sums made again by single lanes took twenty to fifty times)."""
+    M, N, K = mnk
+    torch.manual_seed(51)
+    x, w = torch.randn(M, K, device="cuda"), torch.randn(N, K, device="cuda")
+    out = torch.empty(M, N, device="cuda")
+    without = _gpu_us(lambda: ops.gemm_nt(x, w, out=out))
+    want = out.clone()
+    x[M // 2, K // 2] = float("nan")
+    assert _gpu_us(lambda: ops.gemm_nt(x, w, out=out)) < 4 * without + 20
+    assert out[M // 2].isnan().all()
+    keep = [m for m in range(M) if m != M // 2]
+    assert torch.equal(out[keep], want[keep])
+
+
+def _odd_operands(x, w):
+    """Puts in x and w what the bfloat16 parts do not take: an infinity, a number that rounds to infinity, a NaN in a row of
+    either, each with rows of the other kind."""
+    M, K = x.shape
+    w[:, 0] *= 1e-3                                          # (3.4e38 times up to 5e-3: within float32)
+    x[:, 2] *= 1e-3
+    x[0, 0] = 3.4e38
+    if M > 1:
+        x[1, K // 2] = float("-inf")
+    if M > 2:
+        x[2, K - 1] = float("nan")
+    w[1, K - 1] = float("inf")
+    w[2, 1] = float("nan")
+    w[3, 2] = 3.4e38
+
+
+def _same(got, want):
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.nan_to_num(7.0), want.nan_to_num(7.0))
+
+
+@pytest.mark.parametrize("nk", [(16, 4), (70, 388), (3073, 2052), (2048, 2048), (2100, 8192), (515, 12292), (9001, 1024)])
+def test_gemm_f32_what_is_not_finite(ops, nk):
+    """Infinities, NaN and numbers that round to infinity give what sums of float32 products give, within the bound of
+    test_gemm_f32_matrix_cores where that is finite, and the same bits whatever the number of rows."""
+    N, K = nk
+    torch.manual_seed(52)
+    x, w = torch.randn(700, K, device="cuda"), torch.randn(N, K, device="cuda")
+    _odd_operands(x, w)
+    got = ops.gemm_nt(x, w)
+    want = x.double() @ w.double().T
+    finite = want.abs() < 3e38
+    assert (finite | want.isnan() | want.isinf()).all()
+    _same(torch.where(finite, 0.0, got.double()), torch.where(finite, 0.0, want))
+    bound = (K + 1) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)
+    assert (((got.double() - want).abs() <= bound) | ~finite).all()
+    for M in (1, 3, 8, 9, 16, 17, 64, 130, 300):
+        _same(ops.gemm_nt(x[:M], w), got[:M])
+
+
+@pytest.mark.parametrize("K", [64, 2048, 4100, 8192])
+def test_f32_pairs_of_what_is_not_finite(ops, K):
+    """The forms of few rows that finish pairs of sums (gate-up, q | k | v): the bits of the kernels that they stand for."""
+    torch.manual_seed(53)
+    for M in (1, 3, 8):
+        x, w = torch.randn(M, K, device="cuda"), torch.randn(2 * 4100, K, device="cuda")
+        _odd_operands(x, w)
+        w[4100] = w[1].flip(0)                               # (the other half of a pair)
+        for act in (ops.GLU_SILU, ops.GLU_GELU_TANH):
+            _same(ops.gate_up_f32(x, w, act), ops.silu_mul(ops.gemm_nt(x, w), act))
+        Hq, Hkv, D, P = 6, 2, 16, 4
+        w = w[:(Hq + 2 * Hkv) * D].contiguous()
+        w[(Hq + Hkv) * D + 1, 0] = float("inf")
+        pos, slots = (torch.arange(M, dtype=torch.int32, device="cuda") for _ in range(2))
+        inv = (10000.0 ** (-torch.arange(0, D, 2).float() / D)).cuda()
+        caches = [torch.zeros((3, Hkv, P, D), device="cuda") for _ in range(4)]
+        q = ops.qkv_rope_store_f32(x, w, pos, inv, slots, caches[0], caches[1], Hq, Hkv, D, P)
+        y = ops.gemm_nt(x, w).view(M, Hq + 2 * Hkv, D)
+        ops.rope_store(y[:, :Hq], y[:, Hq:Hq + Hkv], y[:, Hq + Hkv:], pos, inv, slots, caches[2], caches[3], P)
+        _same(q, y[:, :Hq])
+        _same(caches[0], caches[2])
+        _same(caches[1], caches[3])
+
+
 @pytest.mark.parametrize("width", [4, 252, 260, 4096, 4100, 12292, 16384, 16388, 2050])
 def test_add_rmsnorm_f32_widths(ops, width):
     """Every number of pieces a thread, a last piece alone in its wave, rows beyond the kernel with registers; and rows of
@@ -229,6 +324,43 @@ def test_moe_f32_matrix_cores(ops, sizes, gated):
         want += wgt[:, c:c + 1] * torch.bmm(w2, h[:, :, None].contiguous())[:, :, 0]
         bound += wgt[:, c:c + 1] * torch.bmm(w2.abs(), (e + (I + 8) * u * h.abs())[:, :, None].contiguous())[:, :, 0]
     assert ((got.double() - want).abs() <= bound * 1.01).all()
+
+
+@pytest.mark.parametrize("gated", [True, False])
+def test_moe_f32_what_is_not_finite(ops, gated):
+    """Routed experts with infinities, NaN and numbers that round to infinity in bfloat16: what the vector kernel (operands
+    that are not 16-byte aligned) gives, in both products; and a NaN in one row costs little time."""
+    T, K, I, E, top = 70, 1024, 512, 8, 2
+    torch.manual_seed(54)
+    G = 2 if gated else 1
+    x = torch.randn(T, K, device="cuda")
+    gu = torch.randn(E, G * I, K, device="cuda") / math.sqrt(K)
+    down = torch.randn(E, K, I, device="cuda") / math.sqrt(I)
+    r = ops.moe_route(torch.randn(T, E, device="cuda"), E, top)
+    act = 0 if gated else ops.ACT_RELU2
+    without = _gpu_us(lambda: ops.moe_experts(x, r, gu, down, act, 0.0, False))
+    x[5, K // 2] = float("nan")
+    assert _gpu_us(lambda: ops.moe_experts(x, r, gu, down, act, 0.0, False)) < 4 * without + 20
+    x[0, 0] = 3.4e38
+    gu[:, :, 0] *= 1e-32                                      # (sums of some 1e5, whose square is far from float32's end)
+    x[1, 7] = float("inf")
+    gu[0, 1, 3], gu[1, G * I - 2, 4] = float("-inf"), float("nan")
+    gu[2, 0] *= 1e-3                                          # (a result below 1, times 3.4e38)
+    down[2, 3, 0] = 3.4e38
+    down[3, 1, 5], down[3, 2, 6] = float("inf"), float("nan")
+
+    def unaligned(t):
+        return torch.empty(t.numel() + 1, device="cuda")[1:].view(t.shape).copy_(t)
+
+    got = ops.moe_experts(x, r, gu, down, act, 0.0, False)
+    want = ops.moe_experts(unaligned(x), r, unaligned(gu), unaligned(down), act, 0.0, False)
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())
+    assert torch.equal(got.isinf() & (got > 0), want.isinf() & (want > 0))
+    finite = got.isfinite()
+    assert 0.3 < finite.float().mean() < 1
+    # sums of the same products in another order, in either product: a part of 2 (K + I) 2^-24 of a row's largest result at most
+    scale = want.where(finite, 0.0).abs().amax(1, keepdim=True)
+    assert (((got - want).abs() <= 2 * (K + I) * 2.0 ** -24 * scale) | ~finite).all()
 
 
 @pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float32], ids=["to_bf16", "to_fp32"])
