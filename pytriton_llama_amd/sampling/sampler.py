@@ -3,12 +3,14 @@ from __future__ import annotations
 
 import hashlib
 import struct
-from typing import List, Optional, Sequence
+from typing import TYPE_CHECKING, List, Optional, Sequence
 
 import torch
 
 from .. import ops
-from ..engine.request import Request
+
+if TYPE_CHECKING:                    # (the engine imports this package)
+    from ..engine.request import Request
 
 
 def uniform_text(seed: int, request_seed, step: int) -> str:

@@ -2,10 +2,11 @@
 import array
 import ctypes
 import itertools
+import subprocess
+import sys
 
 import pytest
 
-import pytriton_llama_amd.engine  # noqa: F401
 from pytriton_llama_amd.ops import library
 from pytriton_llama_amd.sampling.sampler import uniform_for, uniform_text
 
@@ -24,3 +25,9 @@ def test_uniform_numbers_of_the_library(ids):
         assert rc == 0
         want = array.array("f", [uniform_for(seed, i, step) for i in ids])
         assert values[2::3] == want and set(values[0::3]) == set(values[1::3]) == {7.0}
+
+
+@pytest.mark.parametrize("package", ["sampling", "engine", "cache", "models", "parts", "ops", "weights", "config"])
+def test_packages_can_be_imported_first(package):
+    """Each in an interpreter of its own: none needs another to be imported before it."""
+    subprocess.run([sys.executable, "-c", f"import pytriton_llama_amd.{package}"], check=True, timeout=300)
