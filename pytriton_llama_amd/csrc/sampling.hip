@@ -715,13 +715,15 @@ sw_scan_kernel(float* __restrict__ ws, const float* __restrict__ logits, int V, 
     if (tid == 0) w.ccount[c] = SW_SEG + 1;
     return;
   }
-  const float scale = 1.4426950408889634f / T, mc = mx * scale;
+  // (as (x - max) c: with x c - (max c), one rounding of the product, a chunk's sum is off by 2^(2^-24 max c), 1 % where the largest
+  // logit is 3e5 temperatures, and every chunk's by another factor)
+  const float scale = 1.4426950408889634f / T;
   float e[Q][4], z = 0.f;
 #pragma unroll
   for (int q = 0; q < Q; ++q)
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-      e[q][k] = mx > -INFINITY ? __builtin_amdgcn_exp2f(fmaf(x[q][k], scale, -mc)) : 0.f;
+      e[q][k] = mx > -INFINITY ? __builtin_amdgcn_exp2f((x[q][k] - mx) * scale) : 0.f;
       z += e[q][k];
     }
   z = block_sum(z, scratch);
@@ -1070,7 +1072,8 @@ sw_small_kernel(int32_t* __restrict__ out, float* __restrict__ ws, int S, int ro
   SwScale s = sw_scale(w, S, T, false);
   s.inv_w *= (float)SW_SMALL_BUCKETS / SW_BUCKETS;
   if (__any(count > SW_SEG) || !(s.mx > -INFINITY)) return;
-  s.z = wave_sum(csum > 0.f ? csum * __builtin_amdgcn_exp2f((cmax - s.mx) * s.c) : 0.f);
+  auto exp_of = [&](float x) { return __builtin_amdgcn_exp2f((x - s.mx) * s.c); };   // (as the chunks' sums have it)
+  s.z = wave_sum(csum > 0.f ? csum * exp_of(cmax) : 0.f);
   const int upto = (int)wave_inclusive_scan((float)count);            // (small integers: exact)
   const int n = __shfl(upto, 63, 64);
   if (n > SW_SMALL) return;
@@ -1098,7 +1101,7 @@ sw_small_kernel(int32_t* __restrict__ out, float* __restrict__ ws, int S, int ro
         if (j >= k) continue;
         cand[base + j] = x[q];
         token[base + j] = at[q];
-        atomicAdd(&hist[bucket(x[q])], (unsigned long long)(sw_exp(x[q], s) * SW_FIXED + 0.5f));
+        atomicAdd(&hist[bucket(x[q])], (unsigned long long)(exp_of(x[q]) * SW_FIXED + 0.5f));
       }
     }
   }
@@ -1120,7 +1123,7 @@ sw_small_kernel(int32_t* __restrict__ out, float* __restrict__ ws, int S, int ro
   for (int i = a; i < b; ++i)
     if (bucket(cand[i]) == cross) {
       list_x[at] = cand[i];
-      list_e[at++] = sw_exp(cand[i], s);
+      list_e[at++] = exp_of(cand[i]);
     }
   __syncthreads();
   uint32_t edge = sw_edge(list_x, list_e, (int)in_bucket, before, tp, vote_key, vote_low);
@@ -1134,7 +1137,7 @@ sw_small_kernel(int32_t* __restrict__ out, float* __restrict__ ws, int S, int ro
   int my_last = -1;
   for (int i = a; i < b; ++i)
     if (kept(cand[i])) {
-      mass += sw_exp(cand[i], s);
+      mass += exp_of(cand[i]);
       my_last = i;
     }
   float total;
@@ -1145,7 +1148,7 @@ sw_small_kernel(int32_t* __restrict__ out, float* __restrict__ ws, int S, int ro
     float sum = run;
     for (int i = a; i < b; ++i)
       if (kept(cand[i])) {
-        sum += sw_exp(cand[i], s);
+        sum += exp_of(cand[i]);
         if (sum > target) { choice = i; break; }
       }
     choice_s = choice;

@@ -1844,6 +1844,25 @@ def test_sample_rows(ops, rows, V):
         ops.sample_rows(logits, [0.6, 0.9, 0.0] * rows, texts[1:])
 
 
+@pytest.mark.parametrize("temperature,share", [(1e-4, 3e-3), (1e-3, 3e-4), (1e-5, 3e-2)])
+def test_sample_edge_at_low_temperature(ops, temperature, share):
+    """Two tokens with 0.7 and 0.3 of the mass and top_p a ``share`` of 0.7 above and below it: the second one belongs to the nucleus
+    above only, whatever the largest logit is (largest logit over temperature times log2(e): off by up to 2^-25 of itself where it is
+    rounded, 1 % of the mass at 25 and 1e-4)."""
+    R, V = 64, 16384
+    gap = temperature * math.log(0.7 / 0.3)
+    logits = torch.randn(R, V, generator=torch.Generator().manual_seed(50)) - 50.0        # (few candidates in every chunk)
+    logits[:, 100] = torch.linspace(20.0, 31.0, R)
+    logits[:, 9000] = logits[:, 100] - gap                    # (in another chunk)
+    d = (logits[:, 100].double() - logits[:, 9000].double()) / temperature
+    first = 1.0 / (1.0 + torch.exp(-d))                       # of the logits as float32 has them
+    t = torch.full((R,), temperature).cuda()
+    u = torch.full((R,), 0.9999).cuda()
+    for sign, token in ((-1, 100), (1, 9000)):
+        p = (first * (1 + sign * share)).float().cuda()
+        assert ops.sample_top_p(logits.cuda(), t, p, u).tolist() == [token] * R, sign
+
+
 @pytest.mark.parametrize("wide", [False, True], ids=["one_workgroup", "many_workgroups"])
 def test_sample_top_p_nearly_flat_row_and_signed_zeros(ops, wide):
     """A nearly flat row with a top_p that admits two tokens keeps exactly those two (the most
