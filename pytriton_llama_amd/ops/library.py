@@ -3,8 +3,8 @@
 Each source ``csrc/<name>.hip`` becomes ``csrc/_build/libptl_<name>.so`` (gfx950
 only) and is loaded with ctypes; its functions are plain ``extern "C"`` entry
 points that take device pointers and a stream. A library is compiled when it is
-missing or older than its sources, which is how a fresh checkout builds what a
-model needs at its first call. There is no other backend: when a library cannot
+missing, older than its sources or built with other options than these, which is how a
+fresh checkout builds what a model needs at its first call. There is no other backend: when a library cannot
 be built or loaded the op raises.
 """
 from __future__ import annotations
@@ -93,9 +93,25 @@ def _headers() -> List[str]:
     return [os.path.join(CSRC_DIR, f) for f in os.listdir(CSRC_DIR) if f.endswith(".h")]
 
 
+def _options(name: str) -> str:
+    """What the file beside a library says of how it was compiled: the options, without the compiler's and the sources' places
+    (a checkout may be built in one and used in another)."""
+    return " ".join(HIPCC_FLAGS + EXTRA_FLAGS.get(name, []) + LINK_FLAGS.get(name, [])) + "\n"
+
+
+def _options_path(lib: str) -> str:
+    return os.path.splitext(lib)[0] + ".options"
+
+
 def is_stale(name: str) -> bool:
     lib = library_path(name)
     if not os.path.isfile(lib):
+        return True
+    try:
+        with open(_options_path(lib), encoding="utf-8") as f:
+            if f.read() != _options(name):
+                return True
+    except OSError:                        # (nobody knows how it was compiled)
         return True
     t = os.path.getmtime(lib)
     return any(os.path.getmtime(p) > t for p in [source_path(name)] + _headers())
@@ -144,6 +160,9 @@ def build(names: Iterable[str] = KERNEL_LIBRARIES, force: bool = False, verbose:
                     os.remove(tmp)
             else:
                 os.replace(tmp, final)
+                with open(tmp, "w", encoding="utf-8") as f:
+                    f.write(_options(n))
+                os.replace(tmp, _options_path(final))
                 if verbose:
                     print(f"[pytriton_llama_amd] built {n} ({time.time() - t0:.1f}s)",
                           file=sys.stderr, flush=True)

@@ -43,3 +43,31 @@ def test_a_failed_compile_names_the_source_and_shows_the_messages(tmp_path, monk
         library.build(["norm"], force=True, verbose=False)
     assert "norm.hip failed to compile" in str(e.value) and "no such thing" in str(e.value)
     assert not [f for f in os.listdir(tmp_path) if f.startswith("libptl_")]
+
+
+def test_a_library_built_with_other_options_is_built_again(tmp_path, monkeypatch):
+    """A library counts as current only if it was compiled with the options of today, and a source newer than it still
+    makes it stale."""
+    cc = _fake_compiler(tmp_path / "cc", _output_of('printf lib > "$out"\n'))
+    monkeypatch.setenv("HIPCC", cc)
+    monkeypatch.setattr(library, "BUILD_DIR", str(tmp_path))
+    monkeypatch.setattr(library, "_build_dir_cache", str(tmp_path))
+    assert library.is_stale("norm")
+    library.build(["norm", "blaslt"], verbose=False)
+    assert not library.is_stale("norm") and not library.is_stale("blaslt")
+    with monkeypatch.context() as m:
+        m.setattr(library, "HIPCC_FLAGS", library.HIPCC_FLAGS + ["-DOTHER=1"])
+        assert library.is_stale("norm")
+        library.build(["norm"], verbose=False)
+        assert not library.is_stale("norm")
+    assert library.is_stale("norm")
+    with monkeypatch.context() as m:
+        m.setattr(library, "LINK_FLAGS", {})
+        assert library.is_stale("blaslt")
+    assert not library.is_stale("blaslt")
+    os.remove(tmp_path / "libptl_blaslt.options")
+    assert library.is_stale("blaslt")
+    library.build(["norm", "blaslt"], verbose=False)
+    os.utime(tmp_path / "libptl_norm.so", (1, 1))
+    assert library.is_stale("norm") and not library.is_stale("blaslt")
+    assert not [f for f in os.listdir(tmp_path) if ".tmp" in f]
