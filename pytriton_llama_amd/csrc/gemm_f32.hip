@@ -418,15 +418,14 @@ extern "C" int ptl_qkv_rope_store_f32(float* q_out, const float* x, const float*
 // ===========================================================================
 // Many rows of x (a prompt portion), both forms with the order of sums of the kernels above. Where K is a multiple of
 // 32, gemm_f32_stream_kernel: a first kernel splits x into its parts, and waves that do nothing else bring them and W through
-// LDS (tile_stream.h); else gemm_f32_tile_kernel (split_f32.h).
+// LDS (tile_stream.h); else, and for small products, gemm_f32_tile_kernel (split_f32.h), which splits x itself.
 //
 // A grid of few tiles is cut along K as well (a number of spans a workgroup): the spans' sums go to a workspace
 // [spans, M, N] and another kernel adds them in order.
 //
 // Measured (one MI355X, cold weights, us, with the kernel that splits x; in brackets tiles of 64 x 64 on the float32 matrix
 // instructions, which ran before): 700 x 16,384 x 2,048 240 = 196 TFLOP/s (472), 700 x 2,048 x 8,192 146 (237), 700 x 3,072 x
-// 2,048 77 (110), 483 x 4,096 x 2,048 57 (94), 64 x 2,048 x 8,192 27 (30), 17 x 2,048 x 2,048 13.5 (13.1); 300 x 200 x 96 in
-// either form 12 (8.6).
+// 2,048 77 (110), 483 x 4,096 x 2,048 57 (94), 64 x 2,048 x 8,192 27 (30), 17 x 2,048 x 2,048 13.5 (13.1).
 // ===========================================================================
 
 // The results of a wave's tile that are not finite, made again: it has stored TM groups of 16 rows of x, from m0 on, and TN4
@@ -456,7 +455,7 @@ __device__ __forceinline__ void tile_again(float* __restrict__ y, long ldy, unsi
   }
 }
 
-// K not a multiple of 32 (700 x 16,384 x 2,048 320 us in this form).
+// K not a multiple of 32, or small products: tile_plan (700 x 16,384 x 2,048 320 us in this form).
 template <int TA, int TC, bool PARTS>
 __global__ void __launch_bounds__(256, 2)
 gemm_f32_tile_kernel(float* __restrict__ y, const float* __restrict__ x, const float* __restrict__ w,
@@ -881,8 +880,10 @@ gemm_f32_stream_kernel(const StreamArgs a) {
   T(64, 64, 4, 2, 0.44f, 0.33f)
 constexpr int LOADERS = 4;
 
+constexpr int N_STREAMS = 3;
+
 struct TilePlan {
-  int tile;                                      // of STREAM_TILES, or -1: gemm_f32_tile_kernel
+  int tile;                                      // of STREAM_TILES, or N_STREAMS: gemm_f32_tile_kernel
   int bm, bn;                                    // rows of x and of W a tile
   int per;                                       // columns a workgroup
   int per_cu;
@@ -916,8 +917,16 @@ static TilePlan tile_plan(int M, int N, int K, bool pairs = false) {
 #define T(BM, BN, NB, CU, BLOCK, FULL) offer(n++, BM, BN, CU, BLOCK, FULL);
     STREAM_TILES(T)
 #undef T
+    // Spans of four blocks and a grid that lies on the chip at once with one span a workgroup: there the kernel that splits x
+    // costs more than its parts save (one MI355X, us, this form against the best of the others: 300 x 200 x 96 5.8 / 7.1, 17 x 256 x
+    // 512 8.1 / 9.0, 300 x 512 x 512 9.4 / 10.9, 128 x 1,024 x 1,024 10.9 / 12.3, 100 x 3,072 x 768 16.1 / 16.3, 130 x 16,384 x 128
+    // 11.8 / 13.9). Not with more of it, 130 x 4,096 x 512 17.2 / 13.3, 64 x 7,000 x 1,024 22.4 / 20.8, 700 x 16,384 x 128 32 / 29,
+    // and not with longer spans, where neither is ahead, 17 x 2,048 x 2,048 13.3 / 12.9, 64 x 3,072 x 2,048 17.5 / 18.8.
+    const long tiles = (long)((N + 63) / 64) * ((M + 63) / 64);
+    if (!pairs && width == 128 && 2 * tiles * spans <= (spans > 1 ? 5L : 8L) * cus)
+      best = {N_STREAMS, 64, 64, width, 4, best.us - 1.5f};
   } else {
-    offer(-1, 64, 64, 4, 1.3f, 0.35f);
+    offer(N_STREAMS, 64, 64, 4, 1.3f, 0.35f);
   }
   return best;
 }
@@ -926,7 +935,7 @@ static int padded_rows(int M) { return (M + 127) / 128 * 128; }
 
 // floats of the parts of x
 static long split_rows_floats(const TilePlan& plan, int M, int K) {
-  return plan.tile < 0 ? 0 : (long)(split_rows_bytes(padded_rows(M)) / 4) * (K / SPLIT_BK);
+  return plan.tile == N_STREAMS ? 0 : (long)(split_rows_bytes(padded_rows(M)) / 4) * (K / SPLIT_BK);
 }
 
 template <int BM, int BN, int NB, int MODE> static int launch_stream(const StreamArgs& a, int per_cu, hipStream_t st) {
@@ -947,7 +956,7 @@ static int launch_tiles(float* y, const float* x, const float* w, int M, int N, 
   const int splits = (K + plan.per - 1) / plan.per;
   if ((long)tiles_m * tiles_n * splits > 0x3fffffff) return PTL_ERR_ARG;
   float* parts = splits > 1 ? work + split_rows_floats(plan, M, K) : nullptr;
-  if (plan.tile < 0) {
+  if (plan.tile == N_STREAMS) {
     const long tiles = (long)tiles_m * tiles_n;
     const dim3 grid((unsigned)((tiles + 7) / 8 * 8), splits);
     (parts ? gemm_f32_tile_kernel<1, 4, true> : gemm_f32_tile_kernel<1, 4, false>)<<<grid, 256, 0, st>>>(
@@ -970,12 +979,14 @@ static int launch_tiles(float* y, const float* x, const float* w, int M, int N, 
   return ptl_launch_status();
 }
 
-// floats of workspace ptl_gemm_f32 wants for these sizes (0: none)
-extern "C" long ptl_gemm_f32_workspace(int M, int N, int K) {
-  if (M <= 0 || N <= 0 || K <= 0) return 0;
-  const TilePlan plan = tile_plan(M, N, K);
+static long workspace_floats(const TilePlan& plan, int M, int N, int K) {
   const int width = span_width(K);
   return split_rows_floats(plan, M, K) + (plan.per < K ? (long)((K + width - 1) / width) * M * N : 0);
+}
+
+// floats of workspace ptl_gemm_f32 wants for these sizes (0: none)
+extern "C" long ptl_gemm_f32_workspace(int M, int N, int K) {
+  return M <= 0 || N <= 0 || K <= 0 ? 0 : workspace_floats(tile_plan(M, N, K), M, N, K);
 }
 
 // K % 4 == 0, ldx % 4 == 0, x and w 16-byte aligned. ``work``: workspace of ptl_gemm_f32_workspace(M, N, K)
@@ -985,7 +996,40 @@ extern "C" int ptl_gemm_f32(float* y, const float* x, const float* w, int M, int
   if (M <= 0 || N <= 0) return PTL_OK;
   if (K <= 0 || K % 4 || (M > 1 && ldx % 4) || ldx < K || ldy < N || !aligned16(x) || !aligned16(w)) return PTL_ERR_ARG;
   const TilePlan plan = tile_plan(M, N, K);
-  if ((plan.tile >= 0 || plan.per < K) && (work == nullptr || !aligned16(work))) return PTL_ERR_ARG;
+  if (workspace_floats(plan, M, N, K) > 0 && (work == nullptr || !aligned16(work))) return PTL_ERR_ARG;
+  return launch_tiles(y, x, w, M, N, K, ldx, ldy, plan, work, st);
+}
+
+// The plan with tile number ``tile`` and the spans in ``splits`` parts; false if there is none.
+static bool plan_with(int M, int N, int K, int tile, int splits, TilePlan& plan) {
+  const int width = span_width(K), spans = (K + width - 1) / width;
+  if (M <= 0 || N <= 0 || K <= 0 || K % 4 || splits < 1 || splits > spans || tile < 0 || tile > N_STREAMS ||
+      (tile < N_STREAMS && K % SPLIT_BK))
+    return false;
+  static const int sizes[][3] = {
+#define T(BM, BN, NB, CU, BLOCK, FULL) {BM, BN, CU},
+      STREAM_TILES(T)
+#undef T
+      {64, 64, 4}};
+  static_assert(sizeof(sizes) / sizeof(sizes[0]) == N_STREAMS + 1, "");
+  const int per = (spans + splits - 1) / splits * width;
+  if ((long)per * (splits - 1) >= K) return false;
+  plan = {tile, sizes[tile][0], sizes[tile][1], per, sizes[tile][2], 0.f};
+  return true;
+}
+
+// ptl_gemm_f32 by a tile of its own choice, and what it wants (-1: there is no such plan)
+extern "C" long ptl_gemm_f32_tiles_workspace(int M, int N, int K, int tile, int splits) {
+  TilePlan plan;
+  return plan_with(M, N, K, tile, splits, plan) ? workspace_floats(plan, M, N, K) : -1;
+}
+
+extern "C" int ptl_gemm_f32_tiles(float* y, const float* x, const float* w, int M, int N, int K, long ldx, long ldy, int tile,
+                                  int splits, float* work, hipStream_t st) {
+  TilePlan plan;
+  if (!plan_with(M, N, K, tile, splits, plan) || (M > 1 && ldx % 4) || ldx < K || ldy < N || !aligned16(x) || !aligned16(w) ||
+      (workspace_floats(plan, M, N, K) > 0 && (work == nullptr || !aligned16(work))))
+    return PTL_ERR_ARG;
   return launch_tiles(y, x, w, M, N, K, ldx, ldy, plan, work, st);
 }
 

@@ -83,3 +83,21 @@ def test_products_of_every_number_of_rows_launch_a_tile(tmp_path):
     assert all(t["code"] == 0 and len(t["launches"]) == 1 for t in took)
     used = {tile_of(t["launches"][0]) for t in took}
     assert used <= {t[:2] for t in TILES} and len(used) >= 6, used
+
+
+@pytest.mark.parametrize("M,N,K,parts", [(300, 200, 96, False), (17, 64, 32, False), (300, 512, 512, False), (128, 1024, 1024, False),
+                                         (130, 16384, 128, False), (300, 200, 100, False), (130, 4096, 512, True),
+                                         (64, 7000, 1024, True), (700, 16384, 128, True), (17, 2048, 2048, True), (300, 200, 1056, True)])
+def test_small_f32_products_have_no_kernel_that_splits_x(tmp_path, M, N, K, parts):
+    """Small products of more than 16 rows of float32 are one kernel, and the sum of the spans' where K is cut; others have the
+    parts of x made first. Both want the workspace they say."""
+    took = run(tmp_path, "gemm_f32", [(0, "ptl_gemm_f32_workspace", i(M, N, K)),
+                                      (0, "ptl_gemm_f32", [P, P, P, *i(M, N, K), ("l", K), ("l", N), P, NO]),
+                                      (0, "ptl_gemm_f32", [P, P, P, *i(M, N, K), ("l", K), ("l", N), NO, NO])])
+    kernels = [k["kernel"] for k in took[1]["launches"]]
+    assert took[1]["code"] == 0
+    assert any("split_rows_kernel" in k for k in kernels) == parts
+    assert any("gemm_f32_stream_kernel" in k for k in kernels) == parts and any("gemm_f32_tile_kernel" in k for k in kernels) != parts
+    wants = took[0]["code"] != 0
+    assert wants == (parts or any("gemm_f32_sum_kernel" in k for k in kernels))
+    assert took[2] == ({"code": -1, "launches": []} if wants else took[1])

@@ -158,13 +158,13 @@ def test_gemm_f32_same_bits_alone_and_in_a_batch(ops, nk):
 
 
 @pytest.mark.parametrize("mnk", [
-    # the tiles of many rows: one and just over one of every size, an odd and an even number of blocks of 32 columns, one block,
-    # cuts along K with a short last one, N of no whole 16-byte piece, more tiles than the compute units hold at a time
+    # many rows: an odd and an even number of blocks of 32 columns, one block, cuts along K with a short last one, N of no
+    # whole 16-byte piece, more tiles than the compute units hold at a time
     (64, 64, 32), (65, 130, 96), (127, 127, 4128), (128, 128, 2080), (129, 257, 64), (300, 66, 8224), (20, 2051, 544),
     (515, 9001, 160), (1500, 4100, 128)])
 def test_gemm_f32_streamed_tiles(ops, mnk):
     """Within the bound of test_gemm_f32_matrix_cores, and what is infinite or too large for the bfloat16 parts as the
-    float32 sums have it: in every form of the products."""
+    float32 sums have it, with the plan's choice of tiles for so many rows and with few rows."""
     test_gemm_f32_matrix_cores(ops, mnk)
     M, N, K = mnk
     torch.manual_seed(47)
@@ -179,6 +179,52 @@ def test_gemm_f32_streamed_tiles(ops, mnk):
         y = ops.gemm_nt(x[:rows], w).double()
         bound = (K + 1) * 2.0 ** -24 * (x[:rows].double().abs() @ w.double().abs().T)
         assert ((y - want[:rows]).abs() <= bound).all()
+
+
+F32_TILES = [(128, 128), (64, 128), (64, 64), (64, 64)]      # rows of x and of W; the last one splits x itself
+
+
+def _f32_tiles(ops, x, w, tile, splits, out=None):
+    """x @ w.T by a tile of csrc/gemm_f32.hip's, the spans of K in ``splits`` parts; None where there is no such plan."""
+    import ctypes
+    (M, K), N = x.shape, w.shape[0]
+    lib = ops.library.load("gemm_f32")
+    lib.ptl_gemm_f32_tiles_workspace.restype = ctypes.c_long
+    floats = lib.ptl_gemm_f32_tiles_workspace(M, N, K, tile, splits)
+    if floats < 0:
+        return None
+    ptr = lambda t: ctypes.c_void_p(t.data_ptr())
+    work = torch.full((max(floats, 4),), float("nan"), device="cuda")
+    y = torch.empty((M, N), device="cuda") if out is None else out
+    code = lib.ptl_gemm_f32_tiles(ptr(y), ptr(x), ptr(w), M, N, K, ctypes.c_long(x.stride(0)), ctypes.c_long(y.stride(0)), tile, splits,
+                                  ptr(work), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    assert code == 0
+    return y
+
+
+@pytest.mark.parametrize("tile", range(4), ids=["128x128", "64x128", "64x64", "64x64_splits_x"])
+@pytest.mark.parametrize("K", [32, 96, 1312, 2048, 4128, 2052])
+def test_every_f32_tile(ops, tile, K):
+    """Each tile by its index, whole and with K cut, with rows and columns one below, at and one above a tile's and more tiles than
+    the chip holds: the bits of the kernels for few rows (which test_gemm_f32_matrix_cores compares with 64 bits), where operands are infinite or NaN too, and nothing past the rows' ends."""
+    bm, bn = F32_TILES[tile]
+    torch.manual_seed(K)
+    wide = 2 * ops.compute_units("cuda") * bn + 8 if K == 96 else 0
+    for M, N in ((17, bn), (bm - 1, bn + 1), (bm, bn - 1), (bm + 1, 2 * bn + 4), (2 * bm, 5)) + (((bm + 3, wide),) if wide else ()):
+        x, w = torch.randn(M, K + 4, device="cuda")[:, :K], torch.randn(N, K, device="cuda")
+        for odd in (False, True):
+            if odd:
+                x = x.contiguous()
+                _odd_operands(x, w)
+            want = torch.cat([ops.gemm_nt(x[m:m + 8], w) for m in range(0, M, 8)])
+            for splits in (1, 2, 5):
+                out = torch.full((M, N + 3), 7.0, device="cuda")
+                if _f32_tiles(ops, x, w, tile, splits, out[:, :N]) is None:
+                    assert splits > 1 or (tile < 3 and K % 32)
+                    continue
+                _same(out[:, :N].contiguous(), want)
+                assert (out[:, N:] == 7.0).all()
+    assert _f32_tiles(ops, torch.zeros(17, 64, device="cuda"), torch.zeros(8, 64, device="cuda"), 4, 1) is None
 
 
 def _gpu_us(fn, times=5):
