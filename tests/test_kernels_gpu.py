@@ -206,7 +206,8 @@ def _f32_tiles(ops, x, w, tile, splits, out=None):
 @pytest.mark.parametrize("K", [32, 96, 1312, 2048, 4128, 2052])
 def test_every_f32_tile(ops, tile, K):
     """Each tile by its index, whole and with K cut, with rows and columns one below, at and one above a tile's and more tiles than
-    the chip holds: the bits of the kernels for few rows (which test_gemm_f32_matrix_cores compares with 64 bits), where operands are infinite or NaN too, and nothing past the rows' ends."""
+    the chip holds: the bits of the kernels for few rows (which test_gemm_f32_matrix_cores and test_f32_low_parts compare with
+    64 bits), where operands are infinite or NaN too, and nothing past the rows' ends."""
     bm, bn = F32_TILES[tile]
     torch.manual_seed(K)
     wide = 2 * ops.compute_units("cuda") * bn + 8 if K == 96 else 0
@@ -225,6 +226,87 @@ def test_every_f32_tile(ops, tile, K):
                 _same(out[:, :N].contiguous(), want)
                 assert (out[:, N:] == 7.0).all()
     assert _f32_tiles(ops, torch.zeros(17, 64, device="cuda"), torch.zeros(8, 64, device="cuda"), 4, 1) is None
+
+
+def _low_parts(rows, K, seed):
+    """Positive numbers (1 + m + l) 2^e whose three bfloat16 parts are 2^e, m 2^e and l 2^e with m in [2^-9, 2^-8), l in [2^-18,
+    2^-17): what a sum misses without one of the parts adds up, it does not cancel."""
+    g = torch.Generator().manual_seed(seed)
+    m = torch.randint(128, 256, (rows, K), generator=g).double() * 2.0 ** -16
+    l = torch.randint(32, 64, (rows, K), generator=g).double() * 2.0 ** -23
+    v = (1 + m + l) * 2.0 ** torch.randint(-2, 3, (rows, K), generator=g).double()
+    assert torch.equal(v.float().double(), v)
+    return v.float().cuda()
+
+
+def _f32_sum_bound(K, width):
+    """What a sum of K positive products is off by, in 2^-24 of it: 2 sqrt(n) for n additions that round (six standard deviations of
+    independent roundings of partial sums that grow evenly), those of the blocks of a span and those of the spans; 2 for the
+    products that are left out, 12 for the six matrix instructions of a block, should they truncate. Without h l or l h it
+    would be off by 90 and more, without m m by 64 and more."""
+    return 2 * math.sqrt(min(K, width) / 32) + 2 * math.sqrt(math.ceil(K / width)) + 14
+
+
+def _span_width(K):
+    width = 128 if K <= 1024 else 256
+    while -(-K // width) > 16:
+        width *= 2
+    return width
+
+
+@pytest.mark.parametrize("K", [512, 1024, 2048, 2052, 8192])
+def test_f32_low_parts(ops, K):
+    """All parts of the operands count in every kernel, over the whole of K: a bound that does not grow with K as the worst case
+    of test_gemm_f32_matrix_cores does."""
+    bound = _f32_sum_bound(K, _span_width(K)) * 2.0 ** -24
+    for M, N in ((4, 70), (8, 5000), (4, 17001), (12, 70), (12, 9001), (70, 140), (300, 2100)):
+        x, w = _low_parts(M, K, 1), _low_parts(N, K, 2)
+        want = x.double() @ w.double().T
+        forms = {"plan": ops.gemm_nt(x, w)}
+        if M > 16:
+            forms.update({(t, s): _f32_tiles(ops, x, w, t, s) for t in range(4) for s in (1, 3)})
+        for form, y in forms.items():
+            if y is not None:
+                off = float(((y.double() - want).abs() / want).max())
+                assert off <= bound, f"{M} x {N}, {form}: {off * 2 ** 24:.1f} of {bound * 2 ** 24:.1f}"
+
+
+@pytest.mark.parametrize("sizes", [(70, 1024, 512, 3, 1), (130, 1028, 1028, 4, 2)], ids=["whole_blocks", "part_of_a_block"])
+def test_moe_f32_low_parts(ops, sizes):
+    """The same of the routed experts: the first product's error counts twice in relu(u)^2, the second's once."""
+    T, K, I, E, top = sizes
+    x = _low_parts(T, K, 3)
+    up, down = _low_parts(E * I, K, 4).view(E, I, K) / 1024, _low_parts(E * K, I, 5).view(E, K, I) / 1024
+    r = ops.moe_route(torch.randn(T, E, device="cuda"), E, top)
+    got = ops.moe_experts(x, r, up, down, ops.ACT_RELU2, 0.0, False)
+    idx, wgt = r.idx.view(T, top).long().cpu(), r.wgt.view(T, top).double()
+    want = torch.zeros(T, K, dtype=torch.float64, device="cuda")
+    for e in range(E):
+        h = (x.double() @ up[e].double().T) ** 2 @ down[e].double().T
+        for c in range(top):
+            rows = (idx[:, c] == e).nonzero()[:, 0].cuda()
+            want[rows] += wgt[rows, c:c + 1] * h[rows]
+    off = float(((got.double() - want).abs() / want).max()) * 2 ** 24
+    bound = 2 * _f32_sum_bound(K, K) + _f32_sum_bound(I, I) + 8      # (8: the square, the weights and the sum over experts)
+    assert off <= bound, f"{off:.1f} of {bound:.1f}"
+
+
+@pytest.mark.parametrize("mn", [(4, 100), (4, 17000), (12, 5000), (70, 300)])
+def test_gemm_f32_small_numbers(ops, mn):
+    """Powers of two change nothing for numbers from 2^-110 on, times numbers around one. Below, the parts that are too small for
+    bfloat16 are lost, less than 2^-126 of a number each, and products that small in the matrix cores."""
+    M, N = mn
+    K = 2048
+    x, w = _low_parts(M, K, 6), _low_parts(N, K, 7)
+    y = ops.gemm_nt(x, w)
+    assert torch.equal(ops.gemm_nt(x * 2.0 ** -108, w), y * 2.0 ** -108)      # (the smallest of x are 2^-2)
+    for power in (-112, -118, -124):
+        small = x.double() * 2.0 ** power
+        got = ops.gemm_nt(small.float(), w).double()
+        rounded = small.float().double()
+        want = rounded @ w.double().T
+        lost = 2.0 ** -125 * (w.double().sum(1) + K)
+        assert ((got - want).abs() <= lost[None] + (K + 1) * 2.0 ** -24 * want.abs()).all(), power
 
 
 def _gpu_us(fn, times=5):
@@ -1859,6 +1941,30 @@ def test_sample_top_p_one_and_many_workgroups_a_row_agree(ops, V):
     for r in (0, 2, 4):                                       # against the plain rule
         want = plain_llama.top_p_probs(torch.nan_to_num(logits[r], nan=float("-inf")), float(t[r]), float(p[r]))
         assert float((prw[r].double().cpu() - want).abs().sum()) < 1e-3
+
+
+def test_sampler_at_vocabulary_size(ops):
+    """A request draws the same tokens alone, with others and beside a greedy one, with and without a seed of its own, with
+    tokens on their way or in its list, and on the host too."""
+    from pytriton_llama_amd.engine.request import Request, SamplingParams
+    from pytriton_llama_amd.sampling import Sampler
+    V, R = 32000, 7
+    logits = (2 * torch.randn(R + 1, V, generator=torch.Generator().manual_seed(60))).cuda()
+    params = [SamplingParams(temperature=0.7 + 0.1 * i, top_p=(0.9, 1.0, 0.95)[i % 3], seed=(None, 5, 6)[i % 3]) for i in range(R)]
+    requests = [Request(("chat é", i), [1, 2], p, output=[3] * (i % 4)) for i, p in enumerate(params)]
+    greedy = Request("greedy", [1], SamplingParams(temperature=0.0))
+    sampler = Sampler(seed=8)
+    for ahead in (0, 2):
+        host = torch.full((R + 1,), -1, dtype=torch.int32).pin_memory()
+        together = sampler.sample_device(logits[:R], requests, ahead, host).tolist()
+        assert host.tolist() == together + [-1]                 # (tolist has waited for the stream)
+        assert together == [int(sampler.sample_device(logits[i:i + 1], [r], ahead)) for i, r in enumerate(requests)]
+        beside = sampler.sample_device(logits, requests + [greedy], ahead, host).tolist()
+        assert host.tolist() == beside
+        assert beside == together + [int(logits[R].argmax())]
+        later = [Request(r.id, r.prompt, r.params, output=r.output + [4] * ahead) for r in requests]
+        assert sampler.sample_device(logits[:R], later).tolist() == together
+    assert len({tuple(sampler.sample_device(logits[:R], requests, a).tolist()) for a in range(4)}) == 4
 
 
 @pytest.mark.parametrize("rows,V", [(1, 16384), (70, 20001), (64, 32000), (3, 128256)])
