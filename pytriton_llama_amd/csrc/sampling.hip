@@ -1052,7 +1052,7 @@ __device__ __forceinline__ uint32_t sw_edge(const float* list_x, const float* li
 #define SW_SMALL_BUCKETS 1024
 #define SW_SMALL_LIST 1024
 __global__ void __launch_bounds__(SW_THREADS)
-sw_small_kernel(int32_t* __restrict__ out, float* __restrict__ ws, int S, int row0) {
+sw_small_kernel(int32_t* __restrict__ out, float* __restrict__ ws, int S) {
   __shared__ float tmp[17];
   __shared__ int itmp[2];
   __shared__ float cand[SW_SMALL];
@@ -1064,7 +1064,7 @@ sw_small_kernel(int32_t* __restrict__ out, float* __restrict__ ws, int S, int ro
   __shared__ int vote_low[4], choice_s, last_kept;
   float* const tot = list_x;               // (the buckets' sums are read before the list is made)
   static_assert(SW_SMALL_LIST >= SW_SMALL_BUCKETS, "one place for both");
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = row0 + blockIdx.x;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = blockIdx.x;
   const SwRow w = sw_row(ws, r, S);
   const float T = w.result[8], top_p = w.result[9], u = w.result[10];
   const int count = lane < S ? w.ccount[lane] : 0;
@@ -1340,7 +1340,7 @@ static int sample_wide(int32_t* out, float* work, int want_probs, const float* l
     sw_scan_kernel<<<dim3(S, rows), SW_THREADS, 0, stream>>>(ws, logits, V, stride, S, row0, !want_probs, p);
   }
   // (with the probabilities of all tokens the nucleus is wanted in the form that the last kernel reads)
-  if (!want_probs) sw_small_kernel<<<R, SW_THREADS, 0, stream>>>(out, ws, S, 0);
+  if (!want_probs) sw_small_kernel<<<R, SW_THREADS, 0, stream>>>(out, ws, S);
   sw_hist_kernel<<<chunks, SW_THREADS, 0, stream>>>(ws, logits, V, stride, S);
   sw_combine_kernel<<<R, SW_COMBINE_THREADS, 0, stream>>>(ws, S);
   sw_gather_kernel<<<chunks, SW_THREADS, 0, stream>>>(ws, logits, V, stride, S);
@@ -1427,14 +1427,14 @@ extern "C" int ptl_uniforms(float* values, const uint8_t* texts, const int32_t* 
   return PTL_OK;
 }
 
-// The same without probabilities, temperature, top_p and u of every row in host memory ([R][3]); they are in the launch when
-// the call returns. With texts u is made here (ptl_uniforms).
+// The same without probabilities, temperature and top_p of every row in host memory ([R][3], the third made here of the row's
+// text: ptl_uniforms); they are in the launch when the call returns.
 extern "C" int ptl_sample_top_p_rows(int32_t* out, const float* logits, int R, int V, long stride, float* values,
                                      const uint8_t* texts, const int32_t* ends, float* ws, hipStream_t stream) {
   if (R <= 0) return PTL_OK;
   const int S = (V + SW_CHUNK - 1) / SW_CHUNK;
-  if (V <= 0 || stride < V || !ws || S > 64 || R > 65535 || !values || (texts && !ends)) return PTL_ERR_ARG;
-  if (texts && ptl_uniforms(values, texts, ends, R) != PTL_OK) return PTL_ERR_ARG;
+  if (V <= 0 || stride < V || !ws || S > 64 || R > 65535 || !values || !texts || !ends) return PTL_ERR_ARG;
+  if (ptl_uniforms(values, texts, ends, R) != PTL_OK) return PTL_ERR_ARG;
   return sample_wide(out, nullptr, 0, logits, R, V, stride, SwParams{}, values, ws, stream);
 }
 
