@@ -19,12 +19,12 @@
 // 128 x 256, 85 for 128 x 128, against 103 and 67); a seventh wave that touches W 6 to 16 chunks ahead (10 to 35 % slower);
 // rows of x and W padded by 64 or 128 columns (level).
 //
-// Measured (one MI355X, cold weights, us, a product over and over, which flatters the library against a step, where it shares
+// Measured (one MI355X, cold weights, us, a product over and over in a recorded graph, which flatters the library against a step, where it shares
 // the caches with others: ops/kernels.py has the times in a step; the library's product and the kernel behind it in brackets): down projection with
-// sum, residual and norm, 2,048 x 8,192, 80 / 285 / 532 / 1,024 rows: 16.5 / 26.4 / 32.0 / 47.5 (25.3 / 37.0 / 49.0 / 56.0);
-// 3,072 x 8,192 22.7 / 35.0 / 43.3 / 64.4 (44.0 / 40.1 / 56.3 / 71.7); 4,096 x 14,336 34.3 / 54.4 / 75.7 / 121 (49.9 / 85.2 /
-// 119 / 138); output projection, 2,048 x 2,048 10.6 / 14.4 / 17.3 / 21.8 (13.0 / 15.4 / 17.5 / 22.0). Gate-up with SiLU-multiply,
-// 2 x 8,192 x 2,048, 80 / 285 / 532 / 700 rows: 20.4 / 30.3 / 41.2 / 56.8 (24.5 / 34.9 / 46.4 / 53.3).
+// sum, residual and norm, 2,048 x 8,192, 80 / 285 / 532 / 1,024 rows: 17.6 / 27.0 / 32.6 / 50.6 (24.6 / 36.2 / 47.8 / 55.2);
+// 3,072 x 8,192 20.8 / 34.8 / 44.2 / 63.2 (43.8 / 38.5 / 54.8 / 72.5); 4,096 x 14,336 32.1 / 52.7 / 74.2 / 120 (47.4 / 83.2 /
+// 120 / 139); output projection, 2,048 x 2,048 10.0 / 16.1 / 18.5 / 21.1 (11.5 / 14.1 / 17.1 / 21.3). Gate-up with SiLU-multiply,
+// 2 x 8,192 x 2,048, 80 / 285 / 532 / 700 rows: 20.5 / 29.6 / 40.7 / 54.3 (22.4 / 34.2 / 47.3 / 53.5).
 #include "common.h"
 #include "device.h"
 #include "mfma.h"
@@ -209,8 +209,9 @@ gemm_tile_kernel(const TileArgs a) {
 // The tiles there are: rows of x and of W, waves along either, buffers, workgroups a compute unit (LDS), and what one
 // takes, in us: r rounds of workgroups with c chunks each, of which a share f of the chip's places is taken, take
 // r (c (chunk + full f) + tile). Fitted to 12 shapes of W (2,048 to 28,672 rows, 2,048 to 14,336 columns), 80 to 2,048 rows and
-// 1 to 8 slices; 6 to 14 % (root mean square) from the measured times, and the plan chosen by it is 1 % slower on average
-// than the fastest, 11 % at worst.
+// 1 to 8 slices with two loading waves. Against the times with four (11 shapes, 80 to 1,024 rows, recorded): 15 to 22 % off
+// (root mean square, each tile's by much the same, which does not change the choice); the plan chosen by it is 1.7 % slower on
+// average than the fastest, 8.5 % at worst.
 #define TILES(T)                                     \
   T(64, 64, 2, 2, 5, 2, 0.17f, 0.30f, 1.4f)          \
   T(64, 128, 2, 2, 5, 1, 0.30f, 0.08f, 1.9f)         \

@@ -10,7 +10,9 @@
 // are added to the result by vector instructions. A float32 matrix instruction rounds its sum every four columns, this one
 // every 32.
 //
-// What is lost: the last part of numbers below 2^-110 may be too small for bfloat16.
+// What is lost: the last bits of numbers below 2^-110 are too small for bfloat16, and products below 2^-126 for the matrix cores. Sums of
+// 2,048 products with numbers around one, error in 2^-24 of the sum of magnitudes: 4 for numbers of about 2^-114 as for large ones, 6 for
+// 2^-116, 8 to 14 for 2^-118, 30 to 80 for 2^-120; at most 2.8 times 2^-126 in all.
 //
 // What is not finite: inf - inf in the split makes a NaN of every sum that an infinite (or nearly infinite) number enters.
 // A result that is not finite is worked out again by plain_dots.

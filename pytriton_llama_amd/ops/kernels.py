@@ -696,7 +696,13 @@ def gemm_rows_add_rmsnorm(x: torch.Tensor, w: torch.Tensor, blocked: torch.Tenso
 # kernel behind it (its first proposal, which steps launched kernel by kernel run). Measured inside a step of two prompts
 # of a model of 4 to 14 layers, one of the layer's three products at a time given to the library: by themselves, one
 # after the other, the library's kernels are faster than in a step (2,048 x 2,048 at 284 rows 16.4 us against the tile's 17.7,
-# level in a step). Below: what a layer of the step takes more (+) or less (-) with the tile, us, one MI355X.
+# level in a step). Below: what a layer of the step takes more (+) or less (-) with the tile, us, one MI355X, taken with two
+# loading waves in the tiles. With the four they have now, again at the edges of the rules: 2,048 x 8,192 at 96 / 277 / 576 / 768 rows
+# -5.5 / -9.0 / -15 / -8.9, 3,072 x 8,192 at 277 / 768 -4.6 / -14, 4,096 x 14,336 -27 / -15, 2,048 x 2,048 at 96 / 277 / 512 / 768 -5.9 / -1.4 /
+# -0.1 / +0.1, 3,072 x 3,072 at 448 / 512 / 576 / 640 / 768 -3.6 / +3.3 / -1.1 / +1.9 / -4.5, 4,096 x 4,096 at 576 / 640 / 768 -7.3 / -7.3 /
+# +2.9; gate-up 2 x 8,192 x 2,048 at 277 / 448 / 480 / 512 / 576 / 768 -3.1 / +1.2 / +0.5 / +1.3 / -0.1 / +5.4, 2 x 8,192 x 3,072 at 277 / 448 /
+# 512 / 576 / 640 -3.1 / -1.8 / -0.2 / -0.2 / +11, 2 x 14,336 x 4,096 at 96 / 128 / 160 / 277 / 448 -2.9 / +0.1 / +0.8 / +0.4 / +21: the
+# rules stand.
 # A product with the norm behind it. A deep K gains most: 2,048 x 8,192 at 96 / 277 / 576 / 768 rows -6.1 / -9.1 / -15 / -8.4,
 # 3,072 x 8,192 -17 / -3.5 / -11 / -14, 4,096 x 14,336 -35 / -27 / -41 / -13, 768 x 2,048 -3.4 / -3.5 / -2.3 / -1.4; 5,120 x 13,824
 # at 900 / 1,024 -12 / +29 and 8,192 x 28,672 by itself at 560 / 640 253 / 326 against 256 / 265, so the bound falls with N.

@@ -24,9 +24,9 @@ BUILD_DIR = os.path.join(CSRC_DIR, "_build")
 ARCH = "gfx950"
 # packed float32 instructions are switched off for every kernel of this package. The first 14 words of a kernel's arguments
 # (up to the first struct) come in registers with the wave, not by a load from memory that the first addresses wait for: a decode step is
-# a chain of some hundred kernels of 4 to 15 us, and 0.6 to 1.4 % of it (batch 8 of the Llama-3.2-1B shape 984 -> 976 us, batch 64
-# 1,840 -> 1,814, float32 1,465 -> 1,445). The kernels of such a step name first what the first loads need (with the
-# widths of a product's share behind the 14 words, batch 1 and 8 were level or slower).
+# a chain of some hundred kernels of 4 to 15 us. The kernels of such a step name first what the first loads need. Both builds in turn
+# on one card, without and with: batch 64 of the Llama-3.2-1B shape 1,845 -> 1,814 us, 4 requests in float32 1,464 -> 1,440, 8 long
+# contexts at the 8B shape 4,382 -> 4,359; batch 1 and 8 (809, 1,000) differ by no more than the runs of one build, 1.5 to 1.9 %.
 HIPCC_FLAGS = ["--offload-arch=" + ARCH, "-O3", "-fPIC", "-shared", "-std=c++17",
                "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
                "-mllvm", "-amdgpu-kernarg-preload-count=16"]
