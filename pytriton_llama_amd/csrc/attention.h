@@ -56,6 +56,19 @@ __device__ __forceinline__ float tanh_exp2(float x2) {
   return fmaf(-2.0f, __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(x2)), 1.0f);
 }
 
+// Memory that another workgroup of the launch has written or will read.
+__device__ __forceinline__ void put_shared(float* p, float v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+__device__ __forceinline__ float get_shared(const float* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+// Workgroups that share a (sequence, kv head) pair's keys count in a ticket who is done. Tickets lie 16 bytes apart: those of one
+// line are counted one after the other (one sequence, 8 pairs of 16 parts: 8.8 us side by side, 8.1 so and as 128 bytes apart).
+constexpr int TICKET = 4;
+// One more part of a pair is done (its writes have reached memory): whether it was the last one. The counter is zero again then.
+__device__ __forceinline__ bool last_part(int* ticket, int parts) {
+  const bool last = __hip_atomic_fetch_add(ticket, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == parts - 1;
+  if (last) __hip_atomic_store(ticket, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return last;
+}
+
 static inline bool extras_ok(const AttnExtras& ex) {
   return ex.softcap >= 0.f && !(ex.chunk > 0 && (ex.window > 0 || ex.keep_first > 0));
 }

@@ -477,10 +477,8 @@ attn_decode_kernel(TO* __restrict__ out, long out_stride, const T* __restrict__ 
 template <typename T>
 __global__ void __launch_bounds__(64)
 attn_decode_merge_kernel(const float* __restrict__ part_acc, const float* __restrict__ part_ml,
-                         const int32_t* __restrict__ ctx_len, int Hq, int D, int num_splits, int tile,
-                         const int32_t* __restrict__ q_start, T* __restrict__ out, long out_stride, AttnExtras ex) {
-  // tile (0: every split left a part): keys a split is a multiple of; splits without keys left none, and a
-  // sequence that one split answered for is done.
+                         int Hq, int D, int num_splits, const int32_t* __restrict__ q_start,
+                         T* __restrict__ out, long out_stride, AttnExtras ex) {
   // one wave per (sequence, head): lanes take the splits' (max, denominator) side by side,
   // then the head dimension, with the splits' weights in LDS. The partial results come from
   // other compute units' writes, a long way off: the first 16 splits of the lane's first
@@ -495,11 +493,6 @@ attn_decode_merge_kernel(const float* __restrict__ part_acc, const float* __rest
 #pragma unroll
   for (int s = 0; s < AHEAD; ++s) first[s] = (s < num_splits && lane < D) ? pa0[(size_t)s * D] : 0.f;
   const int row = q_start[seq];
-  if (tile) {
-    const int span = walk_of(ex, ctx_len[seq]), per = keys_a_split(span, num_splits, tile);
-    num_splits = (span + per - 1) / per;
-    if (num_splits <= 1) return;
-  }
   float mn = -INFINITY;
   for (int s = lane; s < num_splits; s += 64) mn = fmaxf(mn, part_ml[(base + s) * 2]);
   mn = wave_max(mn);
@@ -550,8 +543,8 @@ static int launch_decode(void* out, long out_stride, const void* q, long q_strid
   if (hipGetLastError() != hipSuccess) return PTL_ERR_LAUNCH;
   if (num_splits > 1) {
     dim3 mgrid(n_seq, Hq);
-    attn_decode_merge_kernel<TO><<<mgrid, 64, 0, stream>>>(part_acc, part_ml, nullptr, Hq, Dv, num_splits, 0, q_start,
-                                                          (TO*)out, out_stride, ex);
+    attn_decode_merge_kernel<TO><<<mgrid, 64, 0, stream>>>(part_acc, part_ml, Hq, Dv, num_splits, q_start, (TO*)out,
+                                                          out_stride, ex);
   }
   return ptl_launch_status();
 }
@@ -560,12 +553,13 @@ static int launch_decode(void* out, long out_stride, const void* q, long q_strid
 // with Hq = heads * maps, k_cache [pages, Hkv * maps, page_size, Dk], v_cache [pages, Hkv,
 // page_size, Dv], out [T, Hq, Dv] of the caches' type or (out_f32) float32.
 // part_acc [n_seq, Hq, num_splits, Dv] and part_ml [n_seq, Hq, num_splits, 2] are
-// float32 workspaces of the caller (unused when num_splits == 1).
+// float32 workspaces of the caller (unused when num_splits == 1), and so are, for float32 caches, TICKET * n_seq * Hkv tickets: zeros,
+// which they are again after the launch.
 extern "C" int ptl_attention_decode_kv(void* out, long out_stride, int out_f32, const void* q,
                                        long q_stride, const void* k_cache, const void* v_cache,
                                        const int32_t* q_start, const int32_t* ctx_len,
                                        const int32_t* block_table, int bt_stride, float* part_acc,
-                                       float* part_ml, int n_seq, int Hq, int Hkv, int maps, int Dk,
+                                       float* part_ml, int* tickets, int n_seq, int Hq, int Hkv, int maps, int Dk,
                                        int Dv, int page_size, int window, int keep_first, int chunk,
                                        const float* sink, const float* gate, long gate_stride,
                                        float softcap, float scale, int num_splits, int dtype, hipStream_t stream) {
@@ -576,15 +570,11 @@ extern "C" int ptl_attention_decode_kv(void* out, long out_stride, int out_f32, 
       num_splits > 1024 || (num_splits > 1 && (!part_acc || !part_ml)) || !extras_ok(ex))
     return PTL_ERR_ARG;
   if (dtype == PTL_DTYPE_F32 && attn_f32_decodes(Hq, Hkv, maps, Dk, Dv) &&
-      attn_f32_fits(out, out_stride, q, q_stride, k_cache, v_cache, Dk, Dv) && (num_splits == 1 || (uintptr_t)part_acc % 16 == 0)) {
-    const int rc = attention_f32_decode((float*)out, out_stride, (const float*)q, q_stride, (const float*)k_cache,
+      attn_f32_fits(out, out_stride, q, q_stride, k_cache, v_cache, Dk, Dv) && (num_splits == 1 || tickets)) {
+    return attention_f32_decode((float*)out, out_stride, (const float*)q, q_stride, (const float*)k_cache,
                                         (const float*)v_cache, q_start, ctx_len, block_table, bt_stride,
-                                        SplitArgs{part_acc, part_ml, num_splits}, n_seq, Hq, Hkv, Dk, Dv, page_size, ex,
-                                        scale, stream);
-    if (rc != PTL_OK || num_splits == 1) return rc;
-    attn_decode_merge_kernel<float><<<dim3(n_seq, Hq), 64, 0, stream>>>(part_acc, part_ml, ctx_len, Hq, Dv, num_splits,
-                                                                       AF_DECODE_TILE, q_start, (float*)out, out_stride, ex);
-    return ptl_launch_status();
+                                        SplitArgs{part_acc, part_ml, tickets, num_splits}, n_seq, Hq, Hkv, Dk, Dv, page_size,
+                                        ex, scale, stream);
   }
   const int chunks = (Dk > Dv ? Dk : Dv) / 16;
   int lpk = 1;
@@ -616,12 +606,12 @@ extern "C" int ptl_attention_decode(void* out, long out_stride, const void* q, l
                                     const void* k_cache, const void* v_cache,
                                     const int32_t* q_start, const int32_t* ctx_len,
                                     const int32_t* block_table, int bt_stride, float* part_acc,
-                                    float* part_ml, int n_seq, int Hq, int Hkv, int D, int page_size,
+                                    float* part_ml, int* tickets, int n_seq, int Hq, int Hkv, int D, int page_size,
                                     int window, int keep_first, int chunk, const float* sink,
                                     const float* gate, long gate_stride, float softcap, float scale, int num_splits,
                                     int dtype, hipStream_t stream) {
   return ptl_attention_decode_kv(out, out_stride, 0, q, q_stride, k_cache, v_cache, q_start, ctx_len,
-                                 block_table, bt_stride, part_acc, part_ml, n_seq, Hq, Hkv, 1, D, D,
+                                 block_table, bt_stride, part_acc, part_ml, tickets, n_seq, Hq, Hkv, 1, D, D,
                                  page_size, window, keep_first, chunk, sink, gate, gate_stride, softcap, scale,
                                  num_splits, dtype, stream);
 }
@@ -629,30 +619,28 @@ extern "C" int ptl_attention_decode(void* out, long out_stride, const void* q, l
 // ===========================================================================
 // ptl_attention_decode_mfma: the bfloat16 decode case on the matrix cores.
 //
-// num_splits workgroups a (sequence, kv head) pair, each with an equal part of that pair's keys; those without keys
-// leave at once, and a pair that the first one covers is done. The parts of the others meet in a second kernel.
+// The keys of a (sequence, kv head) pair are cut into equal parts of whole turns, one a workgroup. A pair of one part is
+// done with it; the parts of others are merged by the workgroup that is done last, which a counter of the pair says (tickets,
+// zero before and after the launch): a second kernel for that costs 4 to 5 us a layer, also where no pair of the
+// step has more than one part. Parts and counters are written and read past the XCDs' own L2 (agent scope); nothing waits for
+// another workgroup.
 //
-// What bounds the kernel is the memory a compute unit keeps on its way (about 26 GB/s a unit, hardly more with two
-// workgroups than with one; 6.6 TB/s in all), so its time is that of the unit with the most keys. Workgroups go to the
-// units in turn, so with the sequences fastest in the grid the splits of a pair meet on one unit as soon as
-// n_seq * Hkv is a multiple of the units: the longest sequence's unit gets it num_splits times. Where contexts
-// differ (each workgroup finds that out from ctx_len, a recorded step does not know it) workgroups therefore take
-// their pairs by length, the longest first, every second turn of the units from the other end: a unit's second
-// workgroup is short where its first is long. Who computes a part is all that changes: a sequence's bits do not
-// depend on the others. From DECODE_ORDER_KEYS keys a split on (of the longest), where some context is a quarter
-// longer or shorter than the first, for 9 to 64 sequences and up to 4 splits: with more splits the parts are short and
-// the order costs 0.5 to 1.5 us (16 sequences, 2 heads of 96, 16 splits: 300 to 3,000 keys 15.0 -> 16.6, 500 each 10.2 ->
-// 11.4); equal contexts keep the order in which a pair's parts lie in the L2 that the second kernel reads them from
-// (48 of 1,000, 8 x 128: 40.9 against 45.0); at 400 keys a split it gains nothing yet (20 of 800 beside 12 empty rows,
-// 8 x 64: 14.5 against 15.8). One split, where there are more workgroups than units, from DECODE_ORDER_KEYS_ONE keys on
-// (of the longest): 64 of 61 to 2,610 keys, 8 kv heads of 64, 47 -> 40, 8 x 128 96 -> 70; 64 of 1,000 to 2,000 42 -> 40 and 82 ->
-// 73; one of 3,000 beside 63 of 100 46 -> 39 and 90 -> 61; at 400 to 600 keys it costs (16.5 -> 19.0, 28.7 -> 29.9).
-// Measured (one MI355X, us with the second kernel; the sequences fastest in brackets): 20 of 130 to 2,900 keys
-// beside 12 empty rows, 8 kv heads of 128, 42 (55); 32 of 300 to 3,000, 8 x 128, 48 (60), 8 x 64, 29 (34); 16 of 300 to
-// 3,000, 8 x 128, 30 (36); 48 of 300 to 3,000, 8 x 128, 68 (86); 32 of 1,000 to 2,000, 8 x 128, 42 (45.5); one of 3,000
-// beside 31 of 100, 8 x 128, 39 (53); 32 of 2,048, 8 x 64, 27.5 (28.0).
-// (Cutting all pairs' keys as one list into equal shares gave 35, 52, 29, 31, 92, 49, 19 and 29: better only where a few
-// sequences have nearly all keys, worse by up to 1.4 times where a share crosses many short pairs.)
+// What bounds the kernel is the memory a compute unit keeps on its way (about 26 GB/s a unit in all, 17 one workgroup), so its
+// time is that of the unit with the most keys, and of the longest part. A pair has num_splits parts of one turn at least, and
+// more where they would be longer than ``piece`` keys (up to DECODE_MOST_PARTS): one of 3,000 keys beside 31 of 100, 8 kv heads
+// of 128, 2 splits 38.2 -> 29.2, 20 of 130 to 2,900 beside 12 empty rows 41.6 -> 33.4, but 32 of 300 to 3,000 48.1 -> 51.1 and, at
+// one split, 64 of 61 to 2,610 69.5 -> 79.9 with parts of at most 1,024 keys (hence 2,048 there); a part costs 4 to 7 us to begin and to end,
+// so shorter ones lose (64 of 61 to 2,610, 8 x 64, at most 1,536 / 1,024 / 512 / 256 keys 40 / 45 / 46 / 56). How a pair is
+// cut depends on its own keys and num_splits alone, so a sequence's bits do not depend on the others.
+// Where the contexts of 9 to 64 sequences differ by more than a quarter (each workgroup finds that out from ctx_len, a recorded step
+// does not know it) the parts of all pairs are one list, the longest first, every second turn of the units from the other
+// end: a unit's second workgroup is short where its first is long. Equal ones keep the grid's order (64 of 1,400, 8 x 64, 36.1
+// against 38.0 in the list).
+// Measured (one MI355X, us; with the second kernel and without the list in brackets): one of 45 keys, 8 x 64, 4.8 (6.7); one of
+// 2,048 8.2 (8.4); 8 of 2,048 12.2 (13.3); 8 of 100 to 1,000 8.5 (10.2); 16 of 500 9.6 (10.6); 64 of 61 to 2,610 41 (43); 20
+// of 130 to 2,900 beside 12 empty rows 21 (23), 8 x 128 33 (44); 32 of 2,000, 8 x 128, 53 (53); 48 of 300 to 3,000 37 (39),
+// 8 x 128 76 (72). Eight waves a workgroup instead of four: 64 of 1,400, 8 x 64, 36 -> 40. A persistent grid that walks the list
+// costs the start of every part again: 64 of 1,400 in two parts 42.7, one workgroup a part 41.6.
 //
 // A wave takes UNR tiles of 16 keys per turn and all query heads of a kv head at once (up to 16 of them
 // are the N side of the MFMA tiles, so grouped heads cost nothing extra):
@@ -669,8 +657,7 @@ extern "C" int ptl_attention_decode(void* out, long out_stride, const void* q, l
 // are on their way from global memory while this turn is computed, and the page
 // numbers of the turn after that are read one turn earlier still.
 // The softmax state of a head (running max, denominator) lives in the lanes of
-// that head's column; the waves are merged at the end of a pair, the parts of a pair by the
-// second kernel. Needs D % 32 == 0, D <= 128, Hq/Hkv <= 16, a page size
+// that head's column; the waves are merged at the end of a part. Needs D % 32 == 0, D <= 128, Hq/Hkv <= 16, a page size
 // that is a power of two, pages (of all kv heads) below 4 GiB.
 // ===========================================================================
 __device__ __forceinline__ void wave_lds_fence() {
@@ -681,24 +668,27 @@ __device__ __forceinline__ void wave_lds_fence() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-#define DECODE_ORDER_SEQS 64       // sequences of an ordered launch (one a lane)
-#define DECODE_ORDER_KEYS 512      // keys a split from which on the order matters
-#define DECODE_ORDER_KEYS_ONE 1024 // ... where there is one split
+#define DECODE_LIST_SEQS 64        // sequences of a listed launch (one a lane)
+#define DECODE_MOST_PARTS 16       // parts that ``piece`` cuts a pair into at most
 
-// A grid of one dimension: workgroups (sequence, kv head, split), the sequences fastest. ORDERED: by length where
-// contexts differ (above); cus: the compute units.
+// What parts of a pair the workgroups leave for the one that merges them.
+struct DecodeParts {
+  float *acc, *ml;                 // [sequence][head][most][D] results, [..][2] their maximum (of scores times log2 e) and denominator
+  int* tickets;                    // [sequence][kv head][TICKET]: parts that are done
+  int most;                        // parts a pair has room for
+};
+
+// LISTED: a list of parts (above), cus: the compute units, the grid a multiple of them; else a grid of workgroups
+// (sequence, kv head, split), the sequences fastest.
 // KEPT: a window that keeps the sequence's first keys (keep_first > 0). CAP: scores are capped; then
 // scale_log2 is softcap * log2 e and cap_in takes a raw score to tanh_exp2's argument.
-// part_acc [sequence][head][num_splits][D], part_ml [sequence][head][num_splits][2]: the results of the splits of a
-// pair that has several, and their (max, denominator).
-template <int NDT, int UNR, bool ORDERED, bool KEPT, bool CAP>
+template <int NDT, int UNR, bool LISTED, bool KEPT, bool CAP>
 __global__ void __launch_bounds__(256, NDT <= 2 ? 3 : 2)
 attn_decode_mfma_kernel(const int32_t* __restrict__ ctx_len, const int32_t* __restrict__ block_table,
                         const bf16_t* __restrict__ k_cache, const bf16_t* __restrict__ v_cache, int n_seq, int Hkv,
                         int num_splits, int bt_stride, int page_size, int page_shift, const bf16_t* __restrict__ q, long q_stride,
-                        int Hq, int cus, bf16_t* __restrict__ out, long out_stride, const int32_t* __restrict__ q_start,
-                        float* __restrict__ part_acc, float* __restrict__ part_ml, AttnExtras ex, float scale_log2,
-                        float cap_in) {
+                        int Hq, int cus, int piece, bf16_t* __restrict__ out, long out_stride,
+                        const int32_t* __restrict__ q_start, DecodeParts parts, AttnExtras ex, float scale_log2, float cap_in) {
   constexpr int D = 32 * NDT;
   constexpr int NT = 2 * NDT;             // 16-wide tiles of the head dimension
   constexpr int WAVES = 4;
@@ -722,24 +712,40 @@ attn_decode_mfma_kernel(const int32_t* __restrict__ ctx_len, const int32_t* __re
     vrow[i] = c / CPR;
     vcol[i] = (c - vrow[i] * CPR) * 8;
   }
-  int seq = blockIdx.x % n_seq, kvh = blockIdx.x / n_seq % Hkv, split = blockIdx.x / (n_seq * Hkv);
-  if (ORDERED) {
+  int seq = blockIdx.x % n_seq, kvh = blockIdx.x / n_seq % Hkv, split = blockIdx.x / (n_seq * Hkv), per, n_parts;
+  if (LISTED) {
+    // lane s has sequence s: the keys of its parts, and how many of them a pair has
     const int c = lane < n_seq ? ctx_len[lane] : 0, keys = c > 0 ? walk_of(ex, c) : 0;
+    const int lane_per = keys_a_split(keys, min(max(num_splits, (keys + piece - 1) / piece), parts.most), TILE);   // (below too)
+    const int lane_parts = lane < n_seq ? max(1, (keys + lane_per - 1) / lane_per) : 0;
     const unsigned long long some = __ballot(keys > 0);
     const int one = some ? __builtin_amdgcn_readlane(keys, __ffsll(some) - 1) : 0;
-    if (__any(keys > (num_splits == 1 ? DECODE_ORDER_KEYS_ONE : DECODE_ORDER_KEYS * num_splits)) && __any(keys > 0 && abs(keys - one) > one / 4)) {
-      // unit u: the workgroups of a sequence's split (one a kv head); turn: the units that all compute units take
-      const int u = blockIdx.x / Hkv, turn = max(1, cus / Hkv), first = u / turn * turn;
-      const int at = u / turn % 2 ? first + min(turn, n_seq * num_splits - first) - 1 - (u - first) : u;
-      kvh = blockIdx.x - u * Hkv;
-      split = at % num_splits;
-      int place = 0;                                      // of sequence ``lane``, the longest first
-      for (int s = 0; s < n_seq; ++s) {
-        const int other = __builtin_amdgcn_readlane(keys, s);
-        place += (other > keys || (other == keys && s < lane)) ? 1 : 0;
-      }
-      seq = __ffsll((unsigned long long)__ballot(lane < n_seq && place == at / num_splits)) - 1;
+    if (__any(keys > 0 && abs(keys - one) > one / 4)) {
+      const int turn = blockIdx.x / cus, unit = blockIdx.x - turn * cus, at = turn * cus + (turn % 2 ? cus - 1 - unit : unit);
+      const int group = at / (8 * Hkv), in_group = at - group * 8 * Hkv, u = 8 * group + in_group % 8;
+      int all = lane_parts;
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) all += __shfl_xor(all, o, 64);
+      if (u >= all) return;
+      // the longest parts first: every wave counts a quarter of the sequences that come before the lane's
+      const int packed = (keys > 0 ? min(lane_per, 1 << 24) : 0) << 6 | (63 - lane);
+      int start = 0;
+      for (int s = __builtin_amdgcn_readfirstlane(wave); s < n_seq; s += WAVES)
+        start += __builtin_amdgcn_readlane(packed, s) > packed ? __builtin_amdgcn_readlane(lane_parts, s) : 0;
+      int* counts = reinterpret_cast<int*>(lds);
+      counts[wave * 64 + lane] = start;
+      __syncthreads();
+      start = 0;
+#pragma unroll
+      for (int w = 0; w < WAVES; ++w) start += counts[w * 64 + lane];
+      __syncthreads();
+      seq = __ffsll((unsigned long long)__ballot(u >= start && u < start + lane_parts)) - 1;
+      kvh = in_group / 8;
+      split = u - __builtin_amdgcn_readlane(start, seq);
     }
+    per = __builtin_amdgcn_readlane(lane_per, seq);
+    n_parts = __builtin_amdgcn_readlane(lane_parts, seq);
+    if (split >= n_parts) return;
   }
   const int head0 = kvh * G;
   const int row = q_start[seq];
@@ -750,10 +756,13 @@ attn_decode_mfma_kernel(const int32_t* __restrict__ ctx_len, const int32_t* __re
   const int n_kept = KEPT ? min(max(ex.keep_first, 0), k_lo) : 0;
   const int shift = k_lo - n_kept;
   const int span = ctx - shift;
-  const int per = keys_a_split(span, num_splits, TILE);
+  if (!LISTED) {
+    per = keys_a_split(span, min(max(num_splits, (span + piece - 1) / piece), parts.most), TILE);
+    n_parts = max(1, (span + per - 1) / per);
+    if (split >= n_parts) return;
+  }
   const int k_begin = split * per;
   const int k_end = min(span, k_begin + per);
-  if (split > 0 && k_begin >= k_end) return;              // (the first split answers for a row without keys)
   const int turns = (k_end - k_begin + TILE - 1) / TILE;
   auto key_at = [&](int kw) { return (KEPT && kw < n_kept) ? kw : kw + shift; };
   const int32_t* bt = block_table + (size_t)seq * bt_stride;
@@ -885,6 +894,20 @@ attn_decode_mfma_kernel(const int32_t* __restrict__ ctx_len, const int32_t* __re
   float l = l_part + __shfl_xor(l_part, 16, 64);
   l += __shfl_xor(l, 32, 64);
 
+  // column d of the h-th head's result: the weighted sum a of values and the denominator ll to the maximum mn
+  auto write = [&](int h, int d, float mn, float ll, float a) {
+    const int head = head0 + h;
+    if (ex.sink) {                         // one more term of the denominator: exp(sink)
+      const float sk = ex.sink[head] * 1.4426950408889634f;
+      const float mx = fmaxf(mn, sk);
+      const float f = __builtin_amdgcn_exp2f(mn - mx);
+      ll = ll * f + __builtin_amdgcn_exp2f(sk - mx);
+      a *= f;
+    }
+    out[(size_t)row * out_stride + (size_t)head * D + d] =
+        float_to_bf16(ll > 0.f ? a / ll * head_gate(ex, row, head) : 0.f);
+  };
+
   // merge the waves: [wave][head][D] accumulators, [wave][head][2] (max, denominator);
   // the region takes the place of the value tiles, which every wave has left by now
   __syncthreads();
@@ -910,105 +933,133 @@ attn_decode_mfma_kernel(const int32_t* __restrict__ ctx_len, const int32_t* __re
       ll += w_ml[(w * 16 + h) * 2 + 1] * f;
       a += w_acc[(w * 16 + h) * D + d] * f;
     }
-    const int head = head0 + h;
-    if (num_splits == 1) {
-      if (ex.sink) {                       // one more term of the denominator: exp(sink)
-        const float sk = ex.sink[head] * 1.4426950408889634f;
-        const float mx = fmaxf(mn, sk);
-        const float f = __builtin_amdgcn_exp2f(mn - mx);
-        ll = ll * f + __builtin_amdgcn_exp2f(sk - mx);
-        a *= f;
-      }
-      out[(size_t)row * out_stride + (size_t)head * D + d] =
-          float_to_bf16(ll > 0.f ? a / ll * head_gate(ex, row, head) : 0.f);
-    } else if (per >= span) {              // the only split with keys: what the second kernel makes of it, bit for bit
-      const float m = mn * 0.6931471805599453f, sk = ex.sink ? ex.sink[head] : -INFINITY, mx = fmaxf(m, sk);
-      const float w = expf(m - (mx == -INFINITY ? 0.f : mx));
-      ll *= w;
-      if (ex.sink) ll += expf(sk - mx);
-      out[(size_t)row * out_stride + (size_t)head * D + d] =
-          float_to_bf16(a * w * (ll > 0.f ? head_gate(ex, row, head) / ll : 0.f));
+    if (n_parts == 1) {
+      write(h, d, mn, ll, a);
     } else {
-      const size_t p = ((size_t)seq * Hq + head) * num_splits + split;
-      part_acc[p * D + d] = a;
-      // the merge works with natural exponents
-      if (d == 0) { part_ml[p * 2] = mn * 0.6931471805599453f; part_ml[p * 2 + 1] = ll; }
+      const size_t p = ((size_t)seq * Hq + head0 + h) * parts.most + split;
+      put_shared(parts.acc + p * D + d, a);
+      if (d == 0) { put_shared(parts.ml + p * 2, mn); put_shared(parts.ml + p * 2 + 1, ll); }
+    }
+  }
+  if (n_parts > 1) {
+    int* done = reinterpret_cast<int*>(w_ml + WAVES * 16 * 2);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // this wave's part of the part has reached memory
+    __syncthreads();
+    if (tid == 0) *done = last_part(parts.tickets + ((size_t)seq * Hkv + kvh) * TICKET, n_parts);
+    __syncthreads();
+    if (*done) {
+      // (the parts lie a long way off: eight of them are asked for at once)
+      constexpr int AHEAD = 8;
+      for (int i = tid; i < G * D; i += 64 * WAVES) {
+        const int h = i / D, d = i - h * D;
+        const size_t p = ((size_t)seq * Hq + head0 + h) * parts.most;
+        const float *acc = parts.acc + p * D + d, *ml = parts.ml + p * 2;
+        float mn = -INFINITY, ll = 0.f, a = 0.f;
+        for (int s0 = 0; s0 < n_parts; s0 += AHEAD) {
+          float av[AHEAD], mv[AHEAD], lv[AHEAD];
+#pragma unroll
+          for (int s = 0; s < AHEAD; ++s) {
+            const int at = min(s0 + s, n_parts - 1);
+            mv[s] = get_shared(ml + 2 * at);
+            lv[s] = get_shared(ml + 2 * at + 1);
+            av[s] = get_shared(acc + (size_t)at * D);
+          }
+          float m_new = mn;
+#pragma unroll
+          for (int s = 0; s < AHEAD; ++s) m_new = fmaxf(m_new, mv[s]);
+          const float ms = m_new == -INFINITY ? 0.f : m_new, f0 = __builtin_amdgcn_exp2f(mn - ms);
+          ll *= f0;
+          a *= f0;
+#pragma unroll
+          for (int s = 0; s < AHEAD; ++s) {
+            const float f = s0 + s < n_parts ? __builtin_amdgcn_exp2f(mv[s] - ms) : 0.f;
+            ll = fmaf(lv[s], f, ll);
+            a = fmaf(av[s], f, a);
+          }
+          mn = m_new;
+        }
+        write(h, d, mn, ll, a);
+      }
     }
   }
 }
 
-static bool decode_ordered(int n_seq, int Hkv, int num_splits) {
-  return num_splits <= 4 && n_seq > 8 && n_seq <= DECODE_ORDER_SEQS && (num_splits > 1 || n_seq * Hkv > compute_units());
-}
+// Whether the parts of all pairs are one list.
+static bool decode_listed(int n_seq) { return n_seq > 8 && n_seq <= DECODE_LIST_SEQS; }
+// The keys beyond which a part is cut again (figures above).
+static int decode_piece(int D, int num_splits) { return D <= 64 ? 1536 : num_splits == 1 ? 2048 : 1024; }
 
-template <int NDT, int UNR, bool ORDERED>
+template <int NDT, int UNR, bool LISTED>
 static int launch_decode_mfma(void* out, long out_stride, const void* q, long q_stride,
                               const void* k_cache, const void* v_cache, const int32_t* q_start,
                               const int32_t* ctx_len, const int32_t* block_table, int bt_stride,
-                              float* parts, int n_seq, int Hq, int Hkv, int page_size, const AttnExtras& ex,
-                              float scale, int num_splits, hipStream_t stream) {
-  constexpr int D = 32 * NDT, WAVES = 4, TILE = 16 * UNR * WAVES;
-  const long groups = (long)n_seq * Hkv * num_splits;
+                              float* parts, int* tickets, int n_seq, int Hq, int Hkv, int page_size, const AttnExtras& ex,
+                              float scale, int num_splits, int most, int piece, hipStream_t stream) {
+  constexpr int D = 32 * NDT, WAVES = 4;
+  const int cus = compute_units();
+  long groups = (long)n_seq * Hkv * most;
+  if (LISTED) groups = ((long)(n_seq * most + 7) / 8 * 8 * Hkv + cus - 1) / cus * cus;   // (whole turns of the units)
   if (groups > 0x7fffffff) return PTL_ERR_ARG;
-  float* part_ml = parts ? parts + (long)n_seq * Hq * num_splits * D : nullptr;
+  const DecodeParts dp{parts, parts ? parts + (long)n_seq * Hq * most * D : nullptr, tickets, most};
   int page_shift = 0;
   while ((1 << page_shift) < page_size) ++page_shift;
-  const size_t lds_merge = (size_t)WAVES * 16 * (D + 2) * sizeof(float);
+  const size_t lds_merge = (size_t)WAVES * 16 * (D + 2) * sizeof(float) + 16;
   const size_t lds_values = (size_t)WAVES * UNR * 16 * (D + 16) * sizeof(bf16_t);
   const size_t lds = lds_merge > lds_values ? lds_merge : lds_values;
   const bool kept = ex.window > 0 && ex.keep_first > 0, cap = ex.softcap > 0.f;
   const float log2e = 1.4426950408889634f;
   const float scale_log2 = (cap ? ex.softcap : scale) * log2e, cap_in = cap ? 2.0f * log2e * scale / ex.softcap : 0.f;
 #define GO(KEPT, CAP)                                                                                              \
-  attn_decode_mfma_kernel<NDT, UNR, ORDERED, KEPT, CAP><<<(unsigned)groups, 64 * WAVES, lds, stream>>>(            \
+  attn_decode_mfma_kernel<NDT, UNR, LISTED, KEPT, CAP><<<(unsigned)groups, 64 * WAVES, lds, stream>>>(             \
       ctx_len, block_table, (const bf16_t*)k_cache, (const bf16_t*)v_cache, n_seq, Hkv, num_splits, bt_stride, page_size, \
-      page_shift, (const bf16_t*)q, q_stride, Hq, compute_units(), (bf16_t*)out, out_stride, q_start, parts, part_ml, ex, \
-      scale_log2, cap_in)
+      page_shift, (const bf16_t*)q, q_stride, Hq, cus, piece, (bf16_t*)out, out_stride, q_start, dp, ex, scale_log2, cap_in)
   if (kept) {
     if (cap) GO(true, true); else GO(true, false);
   } else {
     if (cap) GO(false, true); else GO(false, false);
   }
 #undef GO
-  if (hipGetLastError() != hipSuccess) return PTL_ERR_LAUNCH;
-  if (num_splits > 1)
-    attn_decode_merge_kernel<bf16_t><<<dim3(n_seq, Hq), 64, 0, stream>>>(
-        parts, part_ml, ctx_len, Hq, D, num_splits, TILE, q_start, (bf16_t*)out, out_stride, ex);
   return ptl_launch_status();
 }
 
-// floats of workspace that ptl_attention_decode_mfma wants
-extern "C" long ptl_attention_decode_mfma_workspace(int n_seq, int Hq, int Hkv, int D, int num_splits) {
-  if (n_seq <= 0 || Hkv <= 0 || Hq % Hkv || num_splits <= 1) return 0;
-  return (long)n_seq * Hq * num_splits * (D + 2);
+// The most parts a pair of at most ``keys`` keys has. Where they are more than one, ptl_attention_decode_mfma wants
+// n_seq * Hq * parts * (D + 2) floats of workspace and TICKET * n_seq * Hkv tickets.
+extern "C" int ptl_attention_decode_mfma_parts(int D, int num_splits, long keys, int piece) {
+  if (D <= 0 || num_splits < 1 || keys <= 0 || piece < 0) return 1;
+  if (piece == 0) piece = decode_piece(D, num_splits);
+  return max(num_splits, (int)min((keys + piece - 1) / piece, (long)DECODE_MOST_PARTS));
 }
 
-// parts: ptl_attention_decode_mfma_workspace floats. unroll: 16-key tiles a wave takes per turn, 1 or 2 (0: the
-// kernel's choice).
+// parts: floats of workspace for ``most`` parts a pair (ptl_attention_decode_mfma_parts for at least the keys of the longest
+// sequence); tickets: zeros, which they are again after the launch. unroll: 16-key tiles a wave takes per turn, 1 or 2 (0:
+// the kernel's choice). piece: keys beyond which a part is cut again (0: the kernel's choice).
 extern "C" int ptl_attention_decode_mfma(void* out, long out_stride, const void* q, long q_stride,
                                          const void* k_cache, const void* v_cache,
                                          const int32_t* q_start, const int32_t* ctx_len,
-                                         const int32_t* block_table, int bt_stride, float* parts,
+                                         const int32_t* block_table, int bt_stride, float* parts, int* tickets, int most,
                                          int n_seq, int Hq, int Hkv, int D,
                                          int page_size, int window, int keep_first, int chunk,
                                          const float* sink, const float* gate, long gate_stride,
-                                         float softcap, float scale, int num_splits, int unroll, hipStream_t stream) {
+                                         float softcap, float scale, int num_splits, int unroll, int piece,
+                                         hipStream_t stream) {
   if (n_seq <= 0) return PTL_OK;
   const AttnExtras ex{window, keep_first, chunk, sink, gate, gate_stride, softcap};
   if (Hq <= 0 || Hkv <= 0 || Hq % Hkv || Hq / Hkv > 16 || D <= 0 || D % 32 || D > 128 ||
       page_size <= 0 || (page_size & (page_size - 1)) || Hq > 65535 ||
       (long)Hkv * page_size * D * 2 >= (1L << 32) || q_stride % 8 || num_splits < 1 ||
-      num_splits > 1024 || (num_splits > 1 && !parts) || unroll < 0 || unroll > 2 || !extras_ok(ex))
+      num_splits > 1024 || most < num_splits || (most > 1 && (!parts || !tickets)) || unroll < 0 || unroll > 2 || piece < 0 ||
+      !extras_ok(ex))
     return PTL_ERR_ARG;
   if (unroll == 0) unroll = 2;
+  if (piece == 0) piece = decode_piece(D, num_splits);
 #define GO(N, U)                                                                                                \
-  (decode_ordered(n_seq, Hkv, num_splits)                                                                            \
+  (decode_listed(n_seq)                                                                                              \
        ? launch_decode_mfma<N, U, true>(out, out_stride, q, q_stride, k_cache, v_cache, q_start, ctx_len,       \
-                                        block_table, bt_stride, parts, n_seq, Hq, Hkv, page_size, ex, scale,    \
-                                        num_splits, stream)                                                     \
+                                        block_table, bt_stride, parts, tickets, n_seq, Hq, Hkv, page_size, ex, scale, \
+                                        num_splits, most, piece, stream)                                        \
        : launch_decode_mfma<N, U, false>(out, out_stride, q, q_stride, k_cache, v_cache, q_start, ctx_len,      \
-                                         block_table, bt_stride, parts, n_seq, Hq, Hkv, page_size, ex, scale,   \
-                                         num_splits, stream))
+                                         block_table, bt_stride, parts, tickets, n_seq, Hq, Hkv, page_size, ex, scale, \
+                                         num_splits, most, piece, stream))
   if (unroll == 1) {
     switch (D / 32) {
       case 1: return GO(1, 1);

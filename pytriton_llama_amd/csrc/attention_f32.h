@@ -33,11 +33,13 @@
 #define AF_DECODE_TILE 128
 struct SplitArgs {
   float *part_acc, *part_ml;     // [sequence][head][num_splits][Dv] and [2]
+  int* tickets;                  // [sequence][kv head][TICKET]: parts that are done, zero before and after the launch
   int num_splits;
 };
 
 // DECODE: sequence blockIdx.x brings one token, and the rows of the block are the query heads (up to 16) of kv head
-// blockIdx.y; the keys are shared by blockIdx.z workgroups as well. (HPW 1, maps 1.)
+// blockIdx.y; the keys are shared by blockIdx.z workgroups as well, of which the one that is done last merges the parts (a
+// second kernel for that took 4.9 us, also where one part has all keys). (HPW 1, maps 1.)
 template <int HPW, int NK, int BN, bool DECODE>
 __global__ void __launch_bounds__(256)
 attn_f32_kernel(float* __restrict__ out, long out_stride, const float* __restrict__ q, long q_stride,
@@ -69,12 +71,13 @@ attn_f32_kernel(float* __restrict__ out, long out_stride, const float* __restric
   const int k_end = DECODE ? ctx : min(ctx, first_q + rows), k_lo = first_seen(ex, first_q), row_lo = first_seen(ex, qpos);
   // the walk: the kept first keys left of the window, then the keys from the window's start on
   const int n_kept = min(max(ex.keep_first, 0), k_lo), shift = k_lo - n_kept, n_all = n_kept + (k_end - k_lo);
-  int k_first = 0, n_walk = n_all;
+  int k_first = 0, n_walk = n_all, n_parts = 1;
   if (DECODE) {
     const int per = keys_a_split(n_all, sp.num_splits, AF_DECODE_TILE);
     k_first = blockIdx.z * per;
     n_walk = min(n_all, k_first + per);
-    if (blockIdx.z > 0 && k_first >= n_walk) return;     // (the first answers for a row without keys)
+    n_parts = max(1, (n_all + per - 1) / per);
+    if (blockIdx.z >= n_parts) return;                   // (the first answers for a row without keys)
   }
   const bool row_valid = ln < rows;
 
@@ -223,21 +226,80 @@ attn_f32_kernel(float* __restrict__ out, long out_stride, const float* __restric
         acc[t] = acc[t] * a + *reinterpret_cast<const f32x4_t*>(other + (t * 64 + lane) * 4) * b;
     }
   }
+  if (DECODE && n_parts > 1) {                   // (one wave is left)
+    const size_t place = ((size_t)seq * Hq + head) * sp.num_splits + blockIdx.z;
+    if (row_valid) {
+      if (lg == 0) {
+        put_shared(sp.part_ml + place * 2, m_run);
+        put_shared(sp.part_ml + place * 2 + 1, l_run);
+      }
+      float* o = sp.part_acc + place * Dv;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        if (NK >= 4) {
+#pragma unroll
+          for (int v = 0; v < NK / 4; ++v) {
+            const int d = 64 * v + 16 * lg + 4 * r;
+            if (d < Dv) {
+#pragma unroll
+              for (int t = 0; t < 4; ++t) put_shared(o + d + t, acc[4 * v + t][r]);
+            }
+          }
+        } else {
+          const int d = 8 * lg + 2 * r;
+          if (d < Dv) { put_shared(o + d, acc[0][r]); put_shared(o + d + 1, acc[NK > 1 ? 1 : 0][r]); }
+        }
+      }
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // the part has reached memory
+    int last = 0;
+    if (lane == 0) last = last_part(sp.tickets + ((size_t)seq * Hkv + vh) * TICKET, n_parts);
+    if (!__builtin_amdgcn_readfirstlane(last)) return;
+    constexpr int AHEAD = 8;
+    for (int i = lane; i < G * Dv / 4; i += 64) {        // four columns a lane
+      const int h = 4 * i / Dv, d = 4 * i - h * Dv, hd = vh * G + h;
+      const size_t p = ((size_t)seq * Hq + hd) * sp.num_splits;
+      const float *pa = sp.part_acc + p * Dv + d, *ml = sp.part_ml + p * 2;
+      f32x4_t a = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      float mn = ex.sink ? ex.sink[hd] : -INFINITY, den = ex.sink ? 1.f : 0.f;   // (the denominator's term without a key)
+      for (int s0 = 0; s0 < n_parts; s0 += AHEAD) {      // (they lie a long way off: eight of them are asked for at once)
+        f32x4_t av[AHEAD];
+        float mv[AHEAD], lv[AHEAD], m_new = mn;
+#pragma unroll
+        for (int s = 0; s < AHEAD; ++s) {
+          const int at = min(s0 + s, n_parts - 1);
+          const float* v = pa + (size_t)at * Dv;
+          mv[s] = get_shared(ml + 2 * at);
+          lv[s] = get_shared(ml + 2 * at + 1);
+          av[s] = f32x4_t{get_shared(v), get_shared(v + 1), get_shared(v + 2), get_shared(v + 3)};
+        }
+#pragma unroll
+        for (int s = 0; s < AHEAD; ++s) m_new = fmaxf(m_new, mv[s]);
+        const float ms = m_new == -INFINITY ? 0.f : m_new, f0 = expf(mn - ms);
+        den *= f0;
+        a *= f0;
+#pragma unroll
+        for (int s = 0; s < AHEAD; ++s) {
+          const float f = s0 + s < n_parts ? expf(mv[s] - ms) : 0.f;
+          den = fmaf(lv[s], f, den);
+          a += av[s] * f;
+        }
+        mn = m_new;
+      }
+      const float inv = den > 0.f ? head_gate(ex, row, hd) / den : 0.f;
+      *reinterpret_cast<f32x4_t*>(out + (size_t)row * out_stride + (size_t)hd * Dv + d) = a * inv;
+    }
+    return;
+  }
   if (!row_valid) return;
-  const bool split = DECODE && n_all > n_walk - k_first;     // a part of the keys: the merge kernel does the rest
-  const size_t place = DECODE ? ((size_t)seq * Hq + head) * sp.num_splits + blockIdx.z : 0;
   float den = l_run, f = 1.f;
-  if (ex.sink && !split) {                                 // one more term of the denominator: exp(sink)
+  if (ex.sink) {                                 // one more term of the denominator: exp(sink)
     const float sk = ex.sink[head], mx = fmaxf(m_run, sk);
     f = expf(m_run - mx);
     den = l_run * f + expf(sk - mx);
   }
-  const float inv = split ? 1.f : den > 0.f ? f / den * head_gate(ex, row, head) : 0.f;
-  float* o = split ? sp.part_acc + place * Dv : out + (size_t)row * out_stride + (size_t)head * Dv;
-  if (split && lg == 0) {
-    sp.part_ml[place * 2] = m_run;
-    sp.part_ml[place * 2 + 1] = l_run;
-  }
+  const float inv = den > 0.f ? f / den * head_gate(ex, row, head) : 0.f;
+  float* o = out + (size_t)row * out_stride + (size_t)head * Dv;
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     if (NK >= 4) {
@@ -288,7 +350,7 @@ static int attention_f32(float* out, long out_stride, const float* q, long q_str
 #define GO(HPW, NK, BN)                                                                                            \
   return launch_attn_f32<HPW, NK, BN, false>(dim3(n_work, Hq / HPW), st, out, out_stride, q, q_stride, k_cache, v_cache, \
                                              q_start, ctx_len, block_table, bt_stride, work_seq, work_qoff, Hq, Hkv,    \
-                                             maps, Dk, Dv, page_size, ex, scale, SplitArgs{nullptr, nullptr, 1})
+                                             maps, Dk, Dv, page_size, ex, scale, SplitArgs{nullptr, nullptr, nullptr, 1})
 #define GO_HEADS(NK)             \
   {                              \
     if (hpw == 2) GO(2, NK, 32); \
@@ -315,7 +377,7 @@ static bool attn_f32_decodes(int Hq, int Hkv, int maps, int Dk, int Dv) {
 }
 
 // One token a sequence (arguments as ptl_attention_decode_kv, of attn_f32_fits and attn_f32_decodes). Splits without
-// keys leave at once; the caller merges what sequences of several splits left.
+// keys leave at once.
 static int attention_f32_decode(float* out, long out_stride, const float* q, long q_stride, const float* k_cache,
                                 const float* v_cache, const int32_t* q_start, const int32_t* ctx_len,
                                 const int32_t* block_table, int bt_stride, const SplitArgs& sp, int n_seq, int Hq, int Hkv,

@@ -23,6 +23,7 @@ from typing import Dict, Hashable, List, Optional, Sequence, Tuple
 import numpy as np
 import torch
 
+from .. import ops
 from ..parts.base import WorkList
 
 
@@ -79,6 +80,8 @@ class StepContext:
     ctx_lens: List[int] = field(default_factory=list)     # upper bounds of its size class)
     max_q_len: int = 0
     max_ctx_len: int = 0
+    tickets: Optional[torch.Tensor] = None     # int32 zeros, ops.TICKET a single-token sequence and kv head: the workgroups of
+                                               # a launch that share a sequence's keys count in them who is done, and leave zeros
 
 
 def order_entries(entries: Sequence[StepEntry]) -> List[int]:
@@ -152,8 +155,8 @@ class SeqInput:
 
 class StepLayout:
     """Every integer array of a step in one int32 buffer: token ids, positions, q_start,
-    ctx_len, state slots, logit rows, the work lists the parts asked for, and per cache group
-    the slot of every token and the block table.
+    ctx_len, state slots, logit rows, the work lists the parts asked for, per cache group
+    the slot of every token and the block table, and zeros for the tickets of decoding rows.
 
     ``sizes`` fixes what the buffer holds at most; ``fill`` writes a step into it and pads
     what the step leaves: token 0 at position 0 with cache slot -1 for rows, no context and
@@ -176,6 +179,8 @@ class StepLayout:
             fields += [(f"work_seq{i}", most), (f"work_row{i}", most)]
         for g in range(len(manager.paged)):
             fields += [(f"slots{g}", rows), (f"table{g}", S * sizes.table_width)]
+        kv_heads = max((t.shape[0] for g in manager.paged for t in g.spec.tensors if len(t.shape) == 2), default=0)
+        fields.append(("tickets", ops.TICKET * B * kv_heads))
         self.spans, n = {}, 0
         for name, k in fields:
             self.spans[name] = (n, k)
@@ -227,7 +232,7 @@ class StepLayout:
             work=work, groups=groups, num_tokens=sz.decode_rows + sz.multi_tokens, num_seqs=S,
             num_logit_rows=sz.logit_rows, logit_rows_are_identity=logit_rows_are_identity,
             num_decode_seqs=sz.decode_rows, q_lens=list(q_lens), ctx_lens=list(ctx_lens),
-            max_q_len=max(q_lens, default=0), max_ctx_len=max(ctx_lens, default=0))
+            max_q_len=max(q_lens, default=0), max_ctx_len=max(ctx_lens, default=0), tickets=self.view("tickets"))
 
     # ---- writing a step ----------------------------------------------------------
     def fill(self, decode: Sequence[SeqInput], multi: Sequence[SeqInput],

@@ -1016,18 +1016,34 @@ def attention_decode_mfma_fits(dtype, Hq: int, Hkv: int, D: int, page_size: int 
             and Hkv * page_size * D * 2 < 2 ** 32)
 
 
+TICKET = 4          # int32 zeros that one (sequence, kv head) pair counts in (csrc/attention.h)
+
+
+def _tickets(tickets: Optional[torch.Tensor], n: int, like: torch.Tensor, what: str) -> torch.Tensor:
+    """``n`` zeros that the workgroups of a launch count their parts in (zeros again after it): the caller's, or new ones."""
+    if tickets is None or tickets.numel() < n:
+        return torch.zeros(n, dtype=torch.int32, device=like.device)
+    if tickets.dtype != torch.int32 or not tickets.is_contiguous() or tickets.device != like.device:
+        raise KernelError(f"{what}: tickets must be a contiguous int32 tensor on {like.device}")
+    return tickets
+
+
 def attention_decode(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor,
                      v_cache: torch.Tensor, q_start: torch.Tensor, ctx_len: torch.Tensor,
                      block_table: torch.Tensor, n_seq: int, scale: float, window: int = 0,
                      num_splits: int = 1, matrix_cores: bool = False, unroll: int = 0,
                      keep_first: int = 0, sink: Optional[torch.Tensor] = None, chunk: int = 0,
-                     gate: Optional[torch.Tensor] = None, softcap: float = 0.0) -> None:
+                     gate: Optional[torch.Tensor] = None, softcap: float = 0.0,
+                     tickets: Optional[torch.Tensor] = None, piece: int = 0) -> None:
     """Split-KV attention of the first ``n_seq`` sequences of the tables, each of
     which brings exactly one query token (see csrc/attention.hip). Head sizes in
     steps of 16 up to 256, float32 or bfloat16. ``matrix_cores``: the MFMA
     variant (bfloat16, head sizes 32/64/96/128, at most 16 heads a kv head, a page
     size that is a power of two); ``unroll``: its 16-key tiles per wave and turn
-    (1 or 2; 0 leaves the choice to the kernel)."""
+    (1 or 2; 0 leaves the choice to the kernel); ``piece``: the keys beyond which it cuts one of the
+    ``num_splits`` parts of a sequence again, up to 16 parts (0: the kernel's choice).
+    ``tickets``: an int32 tensor of zeros that launches on one stream may share (StepContext.tickets):
+    TICKET * n_seq * kv heads of them are counted in, and zero again afterwards; without it one is made."""
     T, Hq, Hkv, D, page_size = _attention_common(out, q, k_cache, v_cache, q_start, ctx_len,
                                                  block_table, "attention_decode")
     if D % 16 or D > 256:
@@ -1044,24 +1060,33 @@ def attention_decode(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor,
             raise KernelError("attention_decode: the matrix-core variant needs bfloat16, a head "
                               "size of 32/64/96/128, at most 16 heads a kv head, a page size that "
                               "is a power of two, aligned q rows")
-        lib.ptl_attention_decode_mfma_workspace.restype = ctypes.c_long
-        parts = torch.empty(lib.ptl_attention_decode_mfma_workspace(int(n_seq), Hq, Hkv, D, int(num_splits)),
-                            dtype=torch.float32, device=q.device)
+        keys = block_table.shape[1] * page_size
+        if window:
+            keys = min(keys, window + keep_first)
+        elif chunk:
+            keys = min(keys, chunk)
+        most = lib.ptl_attention_decode_mfma_parts(D, int(num_splits), ctypes.c_long(max(1, keys)), int(piece))
+        parts = None
+        if most > 1:
+            parts = torch.empty(n_seq * Hq * most * (D + 2), dtype=torch.float32, device=q.device)
+            tickets = _tickets(tickets, TICKET * n_seq * Hkv, q, "attention_decode")
         _check(lib.ptl_attention_decode_mfma(
             _ptr(out), ctypes.c_long(out.stride(0)), _ptr(q), ctypes.c_long(q.stride(0)),
             _ptr(k_cache), _ptr(v_cache), _ptr(q_start), _ptr(ctx_len), _ptr(block_table),
-            int(block_table.stride(0)), _ptr(parts), int(n_seq), Hq, Hkv, D,
-            page_size, *extras, ctypes.c_float(scale), int(num_splits), int(unroll),
+            int(block_table.stride(0)), _ptr(parts), _ptr(tickets), int(most), int(n_seq), Hq, Hkv, D,
+            page_size, *extras, ctypes.c_float(scale), int(num_splits), int(unroll), int(piece),
             _stream()), "attention_decode_mfma")
         return
     part_acc = part_ml = None
     if num_splits > 1:
         part_acc = torch.empty((n_seq, Hq, num_splits, D), dtype=torch.float32, device=q.device)
         part_ml = torch.empty((n_seq, Hq, num_splits, 2), dtype=torch.float32, device=q.device)
+        if q.dtype == torch.float32:
+            tickets = _tickets(tickets, TICKET * n_seq * Hkv, q, "attention_decode")
     _check(lib.ptl_attention_decode(
         _ptr(out), ctypes.c_long(out.stride(0)), _ptr(q), ctypes.c_long(q.stride(0)),
         _ptr(k_cache), _ptr(v_cache), _ptr(q_start), _ptr(ctx_len), _ptr(block_table),
-        int(block_table.stride(0)), _ptr(part_acc), _ptr(part_ml), int(n_seq), Hq, Hkv, D, page_size,
+        int(block_table.stride(0)), _ptr(part_acc), _ptr(part_ml), _ptr(tickets), int(n_seq), Hq, Hkv, D, page_size,
         *extras, ctypes.c_float(scale), int(num_splits), _dtype_code(q), _stream()),
         "attention_decode")
 
@@ -1687,10 +1712,11 @@ def attention_decode_kv(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tenso
                         q_start: torch.Tensor, ctx_len: torch.Tensor, block_table: torch.Tensor, n_seq: int,
                         scale: float, maps: int = 1, num_splits: int = 1, window: int = 0,
                         keep_first: int = 0, sink: Optional[torch.Tensor] = None, chunk: int = 0,
-                        gate: Optional[torch.Tensor] = None, softcap: float = 0.0) -> None:
+                        gate: Optional[torch.Tensor] = None, softcap: float = 0.0,
+                        tickets: Optional[torch.Tensor] = None) -> None:
     """Split-KV attention of the first ``n_seq`` sequences of the tables, each of which brings one
     query token, with keys and values of different sizes and ``maps`` score maps a head (shapes as
-    for attention_generic_kv; sizes in steps of 16 up to 256)."""
+    for attention_generic_kv; sizes in steps of 16 up to 256). ``tickets``: as for attention_decode."""
     _need_gpu(out, q, k_cache, v_cache, q_start, ctx_len, block_table)
     if q.dim() != 3 or k_cache.dim() != 4 or v_cache.dim() != 4:
         raise KernelError("attention_decode_kv: q [T, Hq, Dk], caches [pages, heads, page_size, size]")
@@ -1719,10 +1745,12 @@ def attention_decode_kv(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tenso
     if num_splits > 1:
         part_acc = torch.empty((n_seq, Hq, num_splits, Dv), dtype=torch.float32, device=q.device)
         part_ml = torch.empty((n_seq, Hq, num_splits, 2), dtype=torch.float32, device=q.device)
+        if q.dtype == torch.float32:
+            tickets = _tickets(tickets, TICKET * n_seq * Hkv, q, "attention_decode_kv")
     _check(library.load("attention").ptl_attention_decode_kv(
         _ptr(out), ctypes.c_long(out.stride(0)), int(out.dtype == torch.float32 and q.dtype != torch.float32),
         _ptr(q), ctypes.c_long(q.stride(0)), _ptr(k_cache), _ptr(v_cache), _ptr(q_start), _ptr(ctx_len),
-        _ptr(block_table), int(block_table.stride(0)), _ptr(part_acc), _ptr(part_ml), int(n_seq), Hq, Hkv,
+        _ptr(block_table), int(block_table.stride(0)), _ptr(part_acc), _ptr(part_ml), _ptr(tickets), int(n_seq), Hq, Hkv,
         int(maps), Dk, Dv, page_size, *extras, ctypes.c_float(scale), int(num_splits),
         _dtype_code(q), _stream()), "attention_decode_kv")
 

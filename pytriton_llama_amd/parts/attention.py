@@ -196,7 +196,7 @@ class PagedAttention(Part):
             ops.attention_decode(out, q, k, v, ctx.q_start, ctx.ctx_len,
                                  group.block_table, n_dec, self.scale, window,
                                  self.decode_splits(ctx, n_dec, mfma, q.device), matrix_cores=mfma,
-                                 sink=self.sink)
+                                 sink=self.sink, tickets=ctx.tickets)
         if n_dec == ctx.num_seqs:
             return
         if (ops.attention_prefill_mfma_fits(q.dtype, self.num_kv_heads, D, cache.page_size)

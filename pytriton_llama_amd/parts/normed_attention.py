@@ -208,6 +208,7 @@ class NormedAttention(Part):
         window = self.window or 0
         extras = dict(keep_first=self.keep_first, sink=self.sink, chunk=self.chunk or 0, gate=gate,
                       softcap=self.softcap)
+        decode = dict(extras, tickets=ctx.tickets)
         # one map and keys as large as values: the matrix-core form of the split-KV kernel takes them
         mfma = (n_dec and self.maps == 1 and self.dim == self.vdim and q.stride(0) % 8 == 0
                 and ops.attention_decode_mfma_fits(q.dtype, self.num_heads, self.num_kv_heads, self.dim,
@@ -215,11 +216,11 @@ class NormedAttention(Part):
         if mfma:
             ops.attention_decode(a, q, cache.k, cache.v, ctx.q_start, ctx.ctx_len, group.block_table, n_dec,
                                  self.scale, window, self.decode_splits(ctx, n_dec, q.device, True),
-                                 matrix_cores=True, **extras)
+                                 matrix_cores=True, **decode)
         elif n_dec:
             ops.attention_decode_kv(a, q, cache.k, cache.v, ctx.q_start, ctx.ctx_len, group.block_table, n_dec,
                                     self.scale, self.maps, self.decode_splits(ctx, n_dec, q.device), window,
-                                    **extras)
+                                    **decode)
         if n_dec == ctx.num_seqs:
             return
         if n_dec == ctx.num_decode_seqs and ops.attention_prefill_mfma_kv_fits(

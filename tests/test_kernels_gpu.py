@@ -1489,6 +1489,39 @@ def test_attention_decode_mfma_one_split_in_order(ops, n, Hkv, D, longest):
         assert torch.equal(out[r], run([r])[0]), f"sequence {r}"
 
 
+@pytest.mark.parametrize("dtype,D,Hq,Hkv", [(torch.bfloat16, 64, 8, 2), (torch.bfloat16, 128, 3, 3), (torch.float32, 64, 8, 2)])
+@pytest.mark.parametrize("n", [1, 9, 64, 65])
+def test_attention_decode_parts_meet_in_the_last_workgroup(ops, n, dtype, D, Hq, Hkv):
+    """Sequences of no, one and up to 16 parts (of 128 keys at least): the plain result, the same bits from every launch over one
+    set of tickets, which are zero again each time."""
+    P, pages = 16, 135
+    edges = [3000, 0, 128, 129, 2047, 2048, 2049, 2150, 1]
+    g = torch.Generator().manual_seed(n)
+    ctx = [edges[i] if i < len(edges) else 1 + 97 * i % 700 for i in range(n)]
+    ctx = [min(c, pages * P) for c in ctx]
+    kc, vc = (torch.randn(pages, Hkv, P, D, generator=g).to(dtype) for _ in range(2))
+    bt = torch.stack([torch.randperm(pages, generator=g) for _ in range(n)]).to(torch.int32)
+    q = torch.randn(n, Hq, D, generator=g).to(dtype)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")
+    tickets = torch.zeros(ops.TICKET * n * Hkv, dtype=torch.int32, device="cuda")
+    mfma = dtype == torch.bfloat16
+    outs = []
+    for _ in range(3):
+        out = torch.full((n, Hq, D), 9.0, dtype=dtype, device="cuda")
+        ops.attention_decode(out, q.cuda(), kc.cuda(), vc.cuda(), i32(list(range(n + 1))), i32(ctx), bt.cuda(), n, D ** -0.5,
+                             num_splits=1 if mfma else 16, matrix_cores=mfma, tickets=tickets, piece=128 if mfma else 0)
+        assert int(tickets.abs().max()) == 0
+        outs.append(out)
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
+    for r in range(min(n, len(edges))):
+        if not ctx[r]:
+            assert bool((outs[0][r] == 0).all())
+            continue
+        rows = [t[bt[r].long()].transpose(1, 2).reshape(pages * P, Hkv, D)[:ctx[r]] for t in (kc, vc)]
+        want = _masked_attention(q[r], *rows, ctx[r] - 1, D ** -0.5)
+        torch.testing.assert_close(outs[0][r].float().cpu(), want.float(), **tol(dtype))
+
+
 @pytest.mark.parametrize("D", [16, 32, 48, 64, 80, 128])
 @pytest.mark.parametrize("heads", [3, 4, 8, 16])
 def test_attention_decode_float32_form_by_head_size(ops, D, heads):
