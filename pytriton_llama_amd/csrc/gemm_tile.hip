@@ -6,6 +6,8 @@
 //                        projections) has too few tiles for the compute units otherwise
 //   ptl_tile_gate_up     act(x Wg^T) * (x Wu^T) for W = [Wg; Wu]: the rows of a gate and of its up lie in one wave's
 //                        tile, so the [M, 2 I] product is never stored
+//   ptl_tile_qkv_rope_store  q | k | v: the two rows of W of a rotated pair lie in one wave's tile; q is stored rotated, k (rotated)
+//                        and v go to their pages
 // The reference runs these products through cuBLAS and the rest as kernels of their own
 // (lite_llama/models/llama.py:107-120, lite_llama/kernels/swiglu.py, skip_rmsnorm.py).
 //
@@ -24,7 +26,13 @@
 // sum, residual and norm, 2,048 x 8,192, 80 / 285 / 532 / 1,024 rows: 17.6 / 27.0 / 32.6 / 50.6 (24.6 / 36.2 / 47.8 / 55.2);
 // 3,072 x 8,192 20.8 / 34.8 / 44.2 / 63.2 (43.8 / 38.5 / 54.8 / 72.5); 4,096 x 14,336 32.1 / 52.7 / 74.2 / 120 (47.4 / 83.2 /
 // 120 / 139); output projection, 2,048 x 2,048 10.0 / 16.1 / 18.5 / 21.1 (11.5 / 14.1 / 17.1 / 21.3). Gate-up with SiLU-multiply,
-// 2 x 8,192 x 2,048, 80 / 285 / 532 / 700 rows: 20.5 / 29.6 / 40.7 / 54.3 (22.4 / 34.2 / 47.3 / 53.5).
+// 2 x 8,192 x 2,048, 80 / 285 / 532 / 700 rows: 20.5 / 29.6 / 40.7 / 54.3 (22.4 / 34.2 / 47.3 / 53.5). q | k | v with rotation and cache
+// write, 3,072 x 2,048 at 277 / 532 / 1,024 / 2,048 rows 11.8 / 15.9 / 25.3 / 31.8 (18.5 / 22.4 / 30.2 / 37.1), 5,120 x 3,072 at 277 /
+// 532 / 1,024 20.9 / 29.8 / 45.1 (26.5 / 33.0 / 46.7), 6,144 x 4,096 28.9 / 39.0 / 53.6 (35.1 / 46.4 / 61.6).
+// What bounds the loads: a compute unit has some 64 KB under way, which come back in order, so what lies in L2 waits for what comes from
+// HBM: 160 rows of x and 128 of W a tile, 277 x 16,384 x 2,048, loads alone 24 us (the whole product 28.6), 14 with W in the
+// memory-side cache, whatever the depth, the layout of W or the kind of load; x alone 26 TB/s from L2. Products alone 18 us.
+// W fetched ahead through the scalar cache: 24 -> 31 us.
 #include "common.h"
 #include "device.h"
 #include "mfma.h"
@@ -32,7 +40,7 @@
 
 namespace {
 
-enum { OUT_SUMS = 0, OUT_GLU = 1 };
+enum { OUT_SUMS = 0, OUT_GLU = 1, OUT_QKV = 2 };
 
 constexpr int KC = TILE_ROW / 2;           // columns of a chunk
 
@@ -55,14 +63,24 @@ __device__ __forceinline__ float pair_value(const GluArgs& a, float g, float u) 
   return glu(a, g, u);
 }
 
+// Where q | k | v go (ptl_tile_qkv_rope_store).
+struct QkvArgs {
+  const float2* table;       // [M][D / 2] cosines and sines, or null
+  const int32_t* slots;
+  bf16_t *k_cache, *v_cache;
+  int Hq, Hkv, D, page_size;
+  long ldq;
+};
+
 struct TileArgs {
-  void* y;                   // OUT_SUMS: float32 [splits, M, N]; OUT_GLU: bfloat16 [M, N]
+  void* y;                   // OUT_SUMS: float32 [splits, M, N]; OUT_GLU: bfloat16 [M, N]; OUT_QKV: q
   const bf16_t* x;
   const bf16_t* w;
-  int M, N, K;               // N: columns of y
+  int M, N, K;               // N: columns of y (OUT_QKV: pairs of columns of q | k | v)
   long ldx;
   int splits, tiles_m, tiles_n;
   GluArgs act;
+  QkvArgs qkv;
 };
 
 struct Tile {
@@ -92,9 +110,10 @@ gemm_tile_kernel(const TileArgs a) {
   constexpr int WAVES = WGM * WGN;
   constexpr int WM = BM / WGM, WN = BN / WGN;                // the wave's part of the tile
   constexpr int TM = WM / 16, TN = WN / 16;
-  constexpr int COLS = MODE == OUT_GLU ? BN / 2 : BN;        // columns of y a tile gives
+  constexpr bool PAIRS = MODE != OUT_SUMS;                   // rows of W that meet in a result: half a wave's each
+  constexpr int COLS = PAIRS ? BN / 2 : BN;                  // columns of y a tile gives
   constexpr int CHUNK = (BM + BN) * TILE_ROW;                // rows of x, then rows of W
-  static_assert(MODE != OUT_GLU || TN % 2 == 0, "the two of a pair meet in a wave");
+  static_assert(!PAIRS || TN % 2 == 0, "the two of a pair meet in a wave");
   extern __shared__ __align__(16) unsigned char lds[];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
@@ -114,9 +133,15 @@ gemm_tile_kernel(const TileArgs a) {
       if (r < BM) return reinterpret_cast<const char*>(a.x + (size_t)min(t.m0 + r, M - 1) * a.ldx + k0);
       const int q = r - BM;
       int row;
-      if (MODE == OUT_GLU) {                                 // a wave's rows: one half gate, the other half up
+      if (PAIRS) {                                           // a wave's rows: one half gate, the other half up
         const int part = q / WN, at = q - part * WN, up = at >= WN / 2;
-        row = min(t.n0 + part * (WN / 2) + (up ? at - WN / 2 : at), N - 1) + (up ? N : 0);
+        row = min(t.n0 + part * (WN / 2) + (up ? at - WN / 2 : at), N - 1);
+        if (MODE == OUT_QKV) {                               // ... one half of a head and the other
+          const int half = a.qkv.D >> 1, head = row / half;
+          row += head * half + (up ? half : 0);
+        } else {
+          row += up ? N : 0;
+        }
       } else {
         row = min(t.n0 + q, N - 1);
       }
@@ -187,6 +212,35 @@ gemm_tile_kernel(const TileArgs a) {
         for (int j = 0; j < TN; ++j) {
           const int col = t.n0 + wn * WN + 16 * j + 4 * lg;
           if (col < N) *reinterpret_cast<f32x4_t*>(row + col) = acc[j][i];
+        }
+      } else if (MODE == OUT_QKV) {
+        const int half = a.qkv.D >> 1, slot = a.qkv.slots ? a.qkv.slots[m] : -1;
+        const int page = slot / a.qkv.page_size, off = slot - page * a.qkv.page_size;
+#pragma unroll
+        for (int j = 0; j < TN / 2; ++j) {
+          const int pair = t.n0 + wn * (WN / 2) + 16 * j + 4 * lg, head = pair / half, at = pair - head * half;
+          if (pair >= N) continue;
+          const int kv = head - a.qkv.Hq, v = kv >= a.qkv.Hkv;
+          if (kv >= 0 && slot < 0) continue;
+          f32x4_t c01 = f32x4_t{1.f, 0.f, 1.f, 0.f}, c23 = c01;    // cosine, sine of two pairs
+          if (!v && a.qkv.table) {
+            const f32x4_t* cs = reinterpret_cast<const f32x4_t*>(a.qkv.table + (size_t)m * half + at);
+            c01 = cs[0];
+            c23 = cs[1];
+          }
+          union { uint2 u; bf16_t e[4]; } lo, hi;
+#pragma unroll
+          for (int k = 0; k < 4; ++k) {
+            const float c = k < 2 ? c01[2 * k] : c23[2 * k - 4], s = k < 2 ? c01[2 * k + 1] : c23[2 * k - 3];
+            const float x1 = rounded(acc[j][i][k]), x2 = rounded(acc[j + TN / 2][i][k]);
+            lo.e[k] = to_bf16(x1 * c - x2 * s);
+            hi.e[k] = to_bf16(x2 * c + x1 * s);
+          }
+          bf16_t* to = kv < 0 ? reinterpret_cast<bf16_t*>(a.y) + (size_t)m * a.qkv.ldq + (size_t)head * a.qkv.D
+                              : (v ? a.qkv.v_cache : a.qkv.k_cache) +
+                                    (((size_t)page * a.qkv.Hkv + (v ? kv - a.qkv.Hkv : kv)) * a.qkv.page_size + off) * a.qkv.D;
+          *reinterpret_cast<uint2*>(to + at) = lo.u;
+          *reinterpret_cast<uint2*>(to + at + half) = hi.u;
         }
       } else {
         bf16_t* row = reinterpret_cast<bf16_t*>(a.y) + (size_t)m * N;
@@ -270,7 +324,7 @@ int launch(TileArgs a, hipStream_t stream) {
   auto kernel = gemm_tile_kernel<BM, BN, WGM, WGN, NB, LOADERS, MODE>;
   static LdsAllowance allowance;
   if (!allowance.ask(reinterpret_cast<const void*>(kernel), lds)) return PTL_ERR_LAUNCH;
-  const int cols = MODE == OUT_GLU ? BN / 2 : BN;
+  const int cols = MODE == OUT_SUMS ? BN : BN / 2;
   a.tiles_m = (a.M + BM - 1) / BM;
   a.tiles_n = (a.N + cols - 1) / cols;
   const long total = (long)a.tiles_m * a.tiles_n * a.splits, most = (long)OCC * compute_units();
@@ -309,7 +363,7 @@ extern "C" int ptl_tile_gemm_splits(int M, int N, int K) {
 extern "C" int ptl_tile_product(void* y, const void* x, const void* w, int M, int N, int K, long ldx, int sums, int tile,
                                 int splits, int act, float limit, hipStream_t stream) {
   if (bad(y, x, w, M, N, K, ldx) || splits < 1 || (K / KC) % splits) return PTL_ERR_ARG;
-  TileArgs a{y, (const bf16_t*)x, (const bf16_t*)w, M, N, K, ldx, splits, 0, 0, GluArgs{act, limit}};
+  TileArgs a{y, (const bf16_t*)x, (const bf16_t*)w, M, N, K, ldx, splits, 0, 0, GluArgs{act, limit}, QkvArgs{}};
   if (sums) return run<OUT_SUMS>(tile, a, stream);
   if (splits != 1 || !(glu_ok(act) || act == TILE_SILU_HW)) return PTL_ERR_ARG;
   return run<OUT_GLU>(tile, a, stream);
@@ -332,4 +386,27 @@ extern "C" int ptl_tile_gate_up(void* out, const void* x, const void* w, int M, 
   if (bad(out, x, w, M, I, K, ldx) || !glu_ok(act) || (hw_silu && act != GLU_SILU)) return PTL_ERR_ARG;
   return ptl_tile_product(out, x, w, M, I, K, ldx, 0, plan_for(M, 2 * I, K, false).shape, 1, hw_silu ? TILE_SILU_HW : act,
                           limit, stream);
+}
+
+// q, k, v = x W^T (rows of W: q | k | v, heads of D), q and k rotated by ``table`` ([M][D / 2] cosines and sines as pairs of
+// floats, null: not at all): q [M, ldq], k and v into pages [pages, Hkv, page_size, D] at slots[m] = page * page_size + offset (below 0,
+// or slots null: nowhere). The products are rounded to bfloat16 before the rotation, as stored ones are (rope.hip). K a multiple of
+// 64, D of 32, 16-byte aligned rows, tables and pages. tile: -1: the plan's, else one of the caller's, for tests (two more than ptl_tile_shapes()).
+extern "C" int ptl_tile_qkv_rope_store(void* q, long ldq, const void* x, const void* w, int M, int K, long ldx, const void* table,
+                                       const int32_t* slots, void* k_cache, void* v_cache, int Hq, int Hkv, int D,
+                                       int page_size, int tile, hipStream_t stream) {
+  if (Hq <= 0 || Hkv <= 0 || D <= 0 || D % 32 || page_size <= 0 || (long)(Hq + 2 * Hkv) * D > 0x3fffffff) return PTL_ERR_ARG;
+  const int rows_w = (Hq + 2 * Hkv) * D;
+  if (bad(q, x, w, M, rows_w / 2, K, ldx) || ldq % 8 || ldq < (long)Hq * D || !aligned(table) || !aligned(k_cache) ||
+      !aligned(v_cache) || (slots && (!k_cache || !v_cache)) || tile < -1 || tile >= N_SHAPES + 2)
+    return PTL_ERR_ARG;
+  const TileArgs a{q, (const bf16_t*)x, (const bf16_t*)w, M, rows_w / 2, K, ldx, 1, 0, 0, GluArgs{},
+                   QkvArgs{(const float2*)table, slots, (bf16_t*)k_cache, (bf16_t*)v_cache, Hq, Hkv, D, page_size, ldq}};
+  // Few rows of a narrow W: the smallest tiles as long as each finds a compute unit of its own. 3,072 x 2,048 at 48 / 64 / 96 / 128
+  // rows 9.6 / 9.6 / 10.3 / 10.6 us (tiles of 64 x 64 12.5 / 13.3 / 11.8 / 13.2), 5,120 x 3,072 at 48 / 64 13.8 / 14.5 (16.3 /
+  // 17.4), 6,144 x 4,096 17.3 / 18.1 (20.7 / 22.1); beyond one tile a unit 5,120 x 3,072 at 80 rows 18.3 (15.0).
+  const int units = compute_units(), cols = (rows_w + 31) / 32;
+  if (tile == N_SHAPES || (tile < 0 && (M + 31) / 32 * cols <= units)) return launch<32, 32, 2, 1, 5, 2, OUT_QKV>(a, stream);
+  if (tile == N_SHAPES + 1 || (tile < 0 && (M + 63) / 64 * cols <= units)) return launch<64, 32, 4, 1, 5, 2, OUT_QKV>(a, stream);
+  return run<OUT_QKV>(tile < 0 ? plan_for(M, rows_w, K, false).shape : tile, a, stream);
 }

@@ -17,9 +17,11 @@ struct PtlPromptEntries {
   int (*add_norm)(void*, const void*, void*, const float*, int, int, float, int, hipStream_t);
   int (*gate_up)(void*, const void*, const void*, int, int, int, long, int, float, int, hipStream_t);
   int (*act_mul)(void*, const void*, int, int, int, int, hipStream_t);
+  int (*qkv)(void*, long, const void*, const void*, int, int, long, const void*, const int32_t*, void*, void*, int, int, int,
+             int, int, hipStream_t);
 };
 
-enum Entry { PRODUCT, ROPE_STORE, SUMS, SUM_NORM, ADD_NORM, GATE_UP, ACT_MUL };
+enum Entry { PRODUCT, ROPE_STORE, SUMS, SUM_NORM, ADD_NORM, GATE_UP, ACT_MUL, QKV };
 
 // Of the whole step. failed: which Entry a call that returned an error got it from (-1: its own arguments). o_splits, down_splits: slices of K of the tile product, 0: the library's product and the norm by
 // itself. gate_up_tile: whether gate and up go through the tile product.
@@ -31,6 +33,7 @@ struct PtlPromptStep {
   // partial sums, or a product [T, H]; gate_up [T, 2 I] (not used where the tile product takes it). qkv, product and
   // gate_up may be one place: none is read any more when the next of them is written.
   void *y, *residual, *qkv, *mixed, *product, *gate_up, *a;
+  int qkv_tile;                                  // q | k | v with rotation and cache write in tiles (of qkv only the columns of q are written)
 };
 
 struct PtlPromptLayer {
@@ -38,9 +41,10 @@ struct PtlPromptLayer {
   const float *inv_freq, *post_norm, *next_norm; // next_norm: of the layer behind this one
   void *k_cache, *v_cache;
   float post_eps, next_eps;
+  const void* turns;                             // cosines and sines of the step's rows (qkv_tile)
 };
 
-static_assert(sizeof(PtlPromptStep) == 120 && sizeof(PtlPromptLayer) == 80, "as ops/prompt.py lays them out");
+static_assert(sizeof(PtlPromptStep) == 128 && sizeof(PtlPromptLayer) == 88, "as ops/prompt.py lays them out");
 
 // What is behind the attention of ``before`` (null: none) up to the norm in front of ``after``, then what is in
 // front of the attention of ``after`` (null: the down projection of ``before`` and the norm are left to the caller).
@@ -77,7 +81,11 @@ extern "C" int ptl_prompt_between(const PtlPromptEntries* e, PtlPromptStep* s, c
     }
     if (after && (rc = product_norm(s->a, before->down, s->I, s->down_splits, before->next_norm, before->next_eps))) return rc;
   }
-  if (after) {
+  if (after && s->qkv_tile) {
+    if ((rc = of(QKV, e->qkv(s->qkv, width, s->y, after->qkv, T, H, H, after->turns, s->slots, after->k_cache, after->v_cache,
+                             s->Hq, s->Hkv, D, s->page_size, -1, st))))
+      return rc;
+  } else if (after) {
     if ((rc = of(PRODUCT, e->product(s->qkv, s->y, after->qkv, T, width, H, H, width, PTL_DTYPE_BF16, 1, 0, 0, 0, 0, st))))
       return rc;
     bf16_t* q = reinterpret_cast<bf16_t*>(s->qkv);

@@ -120,3 +120,23 @@ extern "C" int ptl_rope_store(void* q, void* k, const void* v, long row_stride,
     return PTL_ERR_ARG;
   return ptl_launch_status();
 }
+
+// table [T][half]: cosine and sine of positions[t] * inv_freq[j], as rope_store_kernel has them: for products that
+// rotate what they give themselves, once for all layers of a step.
+__global__ void rope_table_kernel(float2* __restrict__ table, const int32_t* __restrict__ positions,
+                                  const float* __restrict__ inv_freq, int total, int half) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= total) return;
+  const int t = i / half;
+  float s, c;
+  sincosf((float)positions[t] * inv_freq[i - t * half], &s, &c);
+  table[i] = make_float2(c, s);
+}
+
+extern "C" int ptl_rope_table(void* table, const int32_t* positions, const float* inv_freq, int T, int half,
+                              hipStream_t stream) {
+  if (T <= 0) return PTL_OK;
+  if (half <= 0 || (long)T * half > 0x3fffffff || !table || !positions || !inv_freq || (uintptr_t)table % 8) return PTL_ERR_ARG;
+  rope_table_kernel<<<(T * half + 255) / 256, 256, 0, stream>>>((float2*)table, positions, inv_freq, T * half, half);
+  return ptl_launch_status();
+}

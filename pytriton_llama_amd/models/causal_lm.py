@@ -134,6 +134,13 @@ class CausalLM:
     # ---- the forward pass of one step ------------------------------------------
     def forward(self, ctx, storage) -> torch.Tensor:
         """Float32 logits [len(ctx.logit_rows), vocab] for the flat batch ``ctx``."""
+        ctx.rotations = {}                  # (a recorded step's context is there for several passes, its positions change)
+        try:
+            return self._forward(ctx, storage)
+        finally:
+            ctx.rotations = None
+
+    def _forward(self, ctx, storage) -> torch.Tensor:
         if getattr(self.embedding, "takes_positions", False):
             h = self.embedding.forward(ctx.token_ids, ctx.positions)
         else:

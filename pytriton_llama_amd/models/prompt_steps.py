@@ -24,6 +24,10 @@ from ..parts.norm import RMSNorm
 from ..parts.rotary import RotaryEncoding
 
 
+# Up to 64 rows some products go to kernels that read the decode copies of the weights.
+LEAST_ROWS = 65
+
+
 def _plain(block) -> bool:
     """Whether the block is the plain decoder's, and what its parts do in such a step is what their classes say: a part
     whose forward somebody replaced (to watch or to change what goes through it) is asked, not passed by."""
@@ -50,7 +54,7 @@ def run(model, h: torch.Tensor, ctx, storage) -> Optional[Tuple[PendingProduct, 
     None where the step or a block is not of this kind."""
     T = h.shape[0]
     calls = model.schedule[:-1]
-    if (T < ops.TILE_MIN_ROWS or not calls or h.dtype != torch.bfloat16 or h.dim() != 2
+    if (T < LEAST_ROWS or not calls or h.dtype != torch.bfloat16 or h.dim() != 2
             or not h.is_cuda or not h.is_contiguous() or h.data_ptr() % 16 or kernels._timed_products):
         return None
     if not getattr(model.blocks[model.schedule[-1].block], "takes_pending_product", False):
@@ -92,6 +96,8 @@ def run(model, h: torch.Tensor, ctx, storage) -> Optional[Tuple[PendingProduct, 
     o_splits = ops.gemm_tile_splits(T, H, Hq * D) if ops.gemm_tile_add_rmsnorm_fits(mixed, mixer.o, residual, norm) else 0
     down_splits = ops.gemm_tile_splits(T, H, I) if ops.gemm_tile_add_rmsnorm_fits(a, ffn.down, residual, norm) else 0
     tile = ops.gate_up_tile_fits(y, ffn.gate_up)
+    qkv_tile = (ops.qkv_rope_store_tile_fits(y, mixer.qkv, D) and all(t.data_ptr() % 16 == 0 for c in caches for t in (c.k, c.v)))
+    tables = [m.position.table(ctx) for m in (b.mixer for b in blocks)] if qkv_tile else [None] * len(blocks)
     # q | k | v, a product (or its float32 sums) and gate | up, one after the other in one place: each has been read when
     # the next is written, so a long step takes no more memory than by the parts, which hold the activation of the block
     # before where ``mixed`` is held here
@@ -99,17 +105,18 @@ def run(model, h: torch.Tensor, ctx, storage) -> Optional[Tuple[PendingProduct, 
                        dtype=torch.bfloat16, device=h.device)
     step = prompt.PromptStep(
         T, H, I, Hq, Hkv, D, page_size, act, o_splits, down_splits, int(tile), 0, ctx.positions.data_ptr(), slots.data_ptr(),
-        y.data_ptr(), residual.data_ptr(), wide.data_ptr(), mixed.data_ptr(), wide.data_ptr(), wide.data_ptr(), a.data_ptr())
+        y.data_ptr(), residual.data_ptr(), wide.data_ptr(), mixed.data_ptr(), wide.data_ptr(), wide.data_ptr(), a.data_ptr(),
+        int(qkv_tile))
     table = prompt.entries()
     q, out = wide[:T * width].view(T, Hq + 2 * Hkv, D)[:, :Hq], mixed.view(T, Hq, D)
     before = None
-    for i, (b, cache) in enumerate(zip(blocks, caches)):
+    for i, (b, cache, turns) in enumerate(zip(blocks, caches, tables)):
         m, f = b.mixer, b.feed_forward
         behind = blocks[i + 1].input_norm if i + 1 < len(blocks) else b.post_norm     # (of the last one: not read)
         layer = prompt.PromptLayer(
             m.qkv.data_ptr(), m.o.data_ptr(), f.gate_up.data_ptr(), f.down.data_ptr(), m.position.inv_freq.data_ptr(),
             b.post_norm.weight.data_ptr(), behind.weight.data_ptr(), cache.k.data_ptr(), cache.v.data_ptr(),
-            b.post_norm.eps, behind.eps)
+            b.post_norm.eps, behind.eps, turns.data_ptr() if turns is not None else 0)
         prompt.prompt_between(table, step, before, layer)
         m.attend(out, q, cache, ctx, ctx.groups[cache.group])
         before = layer

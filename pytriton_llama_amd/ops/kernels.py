@@ -678,7 +678,8 @@ def sum_add_rmsnorm(partials: torch.Tensor, residual: torch.Tensor, weight: torc
 def gemm_rows_add_rmsnorm_fits(x: torch.Tensor, w: torch.Tensor, blocked: Optional[torch.Tensor],
                                residual: torch.Tensor, norm_weight: torch.Tensor) -> bool:
     N = w.shape[0]
-    return _rows_x_ok(x, w, blocked, "add_norm") and _sum_norm_ok(x, N, residual, norm_weight)
+    return (_rows_x_ok(x, w, blocked, "add_norm") and _sum_norm_ok(x, N, residual, norm_weight)
+            and not gemm_tile_add_rmsnorm_fits(x, w, residual, norm_weight))
 
 
 def gemm_rows_add_rmsnorm(x: torch.Tensor, w: torch.Tensor, blocked: torch.Tensor, residual: torch.Tensor,
@@ -710,7 +711,18 @@ def gemm_rows_add_rmsnorm(x: torch.Tensor, w: torch.Tensor, blocked: torch.Tenso
 # -3.1 / +0.6 / +1.3 / +1.6, 3,072 x 3,072 at 96 / 277 / 448 / 512 / 560 / 640 / 768 -5.0 / -1.5 / -3.3 / +3.8 / -1.4 / +3.2 /
 # -4.4, 1,536 x 1,536 at 277 / 448 / 768 -0.5 / +2.1 / -0.8, 4,096 x 4,096 at 277 / 576 / 640 / 768 -4.2 / -6.2 / -5.5 / +5.9, 5,120 x 5,120 at 448 / 512 /
 # 532 -5.4 / -5.1 / +6.2, 1,024 x 1,024 at 277 / 576 / 768 -3.3 / -1.7 / -1.1.
-TILE_MIN_ROWS = 65
+# From 33 rows on they are ahead of the kernels for tens of rows too (csrc/gemm_rows.hip, whose waves read every x fragment from LDS for 16
+# rows of W), us at 48 and 64 rows, those in brackets: 2,048 x 2,048 with norm 9.2, 9.6 (10.1, 10.8), 3,072 x 3,072 12.5, 13.4 (14.6,
+# 16.6), 4,096 x 4,096 15.3, 16.0 (15.2, 16.0); 2,048 x 8,192 14.3, 14.8 (14.9, 15.8), 3,072 x 8,192 18.0, 18.7 (21.5, 23.9), 4,096 x
+# 14,336 28.5, 29.3 (30.7, 32.7); q | k | v with rotation 3,072 x 2,048 9.6, 9.6 (11.3, 13.5), 5,120 x 3,072 13.8, 14.5 (16.2, 18.4), 6,144 x
+# 4,096 17.3, 18.1 (20.1, 22.3); at 32 rows level. Gate-up with SiLU 2 x 8,192 x 2,048 18.5, 18.9 (17.8, 19.6), 2 x 8,192 x 3,072 22.2,
+# 23.7 (24.5, 26.7), 2 x 14,336 x 4,096 50.1, 50.6 (53.6, 61.1).
+TILE_MIN_ROWS = 33
+
+
+def tile_least_rows_gate_up(rows_w: int, K: int) -> int:
+    """Rows from which ``gate_up_tile`` is the faster way for w [rows_w, K]."""
+    return TILE_MIN_ROWS if rows_w * K >= 3 << 24 else 49
 
 
 def tile_most_rows_sums(N: int, K: int) -> int:
@@ -788,9 +800,65 @@ def gemm_tile_add_rmsnorm(x: torch.Tensor, w: torch.Tensor, residual: torch.Tens
     return sum_add_rmsnorm(gemm_tile_sums(x, w), residual, norm_weight, eps)
 
 
+def rope_table(positions: torch.Tensor, inv_freq: torch.Tensor) -> torch.Tensor:
+    """Float32 [T, D / 2, 2]: cosines and sines of positions * inv_freq, as ``rope_store`` has them."""
+    _need_gpu(positions, inv_freq)
+    _i32(positions, "positions")
+    if inv_freq.dtype != torch.float32 or inv_freq.dim() != 1 or not inv_freq.is_contiguous():
+        raise KernelError("rope_table: inv_freq must be contiguous float32 [D / 2]")
+    table = torch.empty((positions.numel(), inv_freq.numel(), 2), dtype=torch.float32, device=positions.device)
+    _check(library.load("rope").ptl_rope_table(_ptr(table), _ptr(positions), _ptr(inv_freq), positions.numel(),
+                                               inv_freq.numel(), _stream()), "rope_table")
+    return table
+
+
+# q | k | v with rotation and cache write against the library's product and rope_store: as long as tiles of 128 x 192 all lie on the
+# chip at once. us, those in brackets: 3,072 x 2,048 at 2,048 rows 31.8 (37.1), 5,120 x 3,072 at 1,024 / 1,536 / 2,048 45.1 / 57.5 /
+# 81.1 (46.7 / 55.1 / 69.7), 6,144 x 4,096 53.6 / 89.4 / 98.8 (61.6 / 82.2 / 92.8); fewer rows in csrc/gemm_tile.hip.
+def tile_most_rows_qkv(rows_w: int, units: int) -> int:
+    """Rows up to which ``qkv_rope_store_tile`` is the faster way for w of rows_w rows on a chip of ``units`` compute units."""
+    return 128 * 192 * units // max(1, rows_w)
+
+
+def qkv_rope_store_tile_fits(x: torch.Tensor, w: torch.Tensor, head_dim: int) -> bool:
+    """Whether ``qkv_rope_store_tile`` takes x and is the faster way for it."""
+    return (x.shape[0] >= TILE_MIN_ROWS and head_dim % 32 == 0 and _tile_x_ok(x, w)
+            and x.shape[0] <= tile_most_rows_qkv(w.shape[0], compute_units(x.device)))
+
+
+def qkv_rope_store_tile(x: torch.Tensor, w: torch.Tensor, table: Optional[torch.Tensor], slots: Optional[torch.Tensor],
+                        k_cache: Optional[torch.Tensor], v_cache: Optional[torch.Tensor], num_heads: int, num_kv_heads: int,
+                        head_dim: int, page_size: int, tile: int = -1) -> torch.Tensor:
+    """As ``qkv_rope_store``, for some hundred rows (csrc/gemm_tile.hip). ``table``: ``rope_table`` of the rows' positions, None: no
+    rotation; ``tile``: one of the kernel's tiles, for tests."""
+    if not (_tile_x_ok(x, w) and head_dim % 32 == 0):
+        raise KernelError("qkv_rope_store_tile: needs bfloat16 x [M, K] and contiguous w [N, K], K a multiple of 64, a head size "
+                          "in steps of 32, 16-byte aligned rows")
+    M, K = x.shape
+    Hq, Hkv, D = num_heads, num_kv_heads, head_dim
+    if w.shape[0] != (Hq + 2 * Hkv) * D:
+        raise KernelError(f"qkv_rope_store_tile: weight has {w.shape[0]} rows, ({Hq} + 2*{Hkv}) * {D} expected")
+    _need_gpu(table, slots, k_cache, v_cache)
+    if table is not None and (table.dtype != torch.float32 or table.shape != (M, D // 2, 2) or not table.is_contiguous()
+                              or table.data_ptr() % 16):
+        raise KernelError(f"qkv_rope_store_tile: table must be contiguous float32 [{M}, {D // 2}, 2]")
+    if slots is not None:
+        if slots.dtype != torch.int32 or slots.numel() != M or not slots.is_contiguous():
+            raise KernelError("qkv_rope_store_tile: slots must be contiguous int32 [M]")
+        for name, c in (("k_cache", k_cache), ("v_cache", v_cache)):
+            if c is None or c.dim() != 4 or c.shape[1:] != (Hkv, page_size, D) or c.dtype != torch.bfloat16 \
+                    or not c.is_contiguous() or c.data_ptr() % 16:
+                raise KernelError(f"qkv_rope_store_tile: {name} must be contiguous bfloat16 [pages, {Hkv}, {page_size}, {D}]")
+    q = torch.empty((M, Hq, D), dtype=torch.bfloat16, device=x.device)
+    _check(library.load("gemm_tile").ptl_tile_qkv_rope_store(
+        _ptr(q), ctypes.c_long(Hq * D), _ptr(x), _ptr(w), M, K, ctypes.c_long(x.stride(0)), _ptr(table), _ptr(slots),
+        _ptr(k_cache), _ptr(v_cache), Hq, Hkv, D, int(page_size), int(tile), _stream()), "qkv_rope_store_tile")
+    return q
+
+
 def gate_up_tile_fits(x: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether ``gate_up_tile`` takes x and is the faster way for it."""
-    return (x.shape[0] >= TILE_MIN_ROWS and _tile_x_ok(x, w)
+    return (x.shape[0] >= tile_least_rows_gate_up(w.shape[0], w.shape[1]) and _tile_x_ok(x, w)
             and x.shape[0] <= tile_most_rows_gate_up(w.shape[0], w.shape[1], compute_units(x.device)))
 
 
@@ -815,7 +883,7 @@ def gate_up_silu_fits(x: torch.Tensor, w: torch.Tensor, blocked: Optional[torch.
     """Whether ``gate_up_silu`` is the way to go for x. ``blocked``: the blocked copy of w, which
     the kernel for some tens of rows reads."""
     if _rows_x_ok(x, w, blocked, "gate_up") and w.shape[0] % 64 == 0:
-        return True
+        return not gate_up_tile_fits(x, w)
     return _fused_x_ok(x, w) and w.shape[0] % 32 == 0
 
 

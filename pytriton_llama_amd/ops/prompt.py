@@ -13,18 +13,19 @@ _P, _I, _F = ctypes.c_void_p, ctypes.c_int, ctypes.c_float
 # the entries a layer calls, in the order of PtlPromptEntries
 ENTRIES = (("blaslt", "ptl_blaslt_gemm_bf16"), ("rope", "ptl_rope_store"), ("gemm_tile", "ptl_tile_gemm_sums"),
            ("gemm_rows", "ptl_rows_sum_add_rmsnorm"), ("norm", "ptl_add_rmsnorm"), ("gemm_tile", "ptl_tile_gate_up"),
-           ("activation", "ptl_silu_mul"))
+           ("activation", "ptl_silu_mul"), ("gemm_tile", "ptl_tile_qkv_rope_store"))
 
 
 class PromptStep(ctypes.Structure):
     _fields_ = ([(n, _I) for n in ("T", "H", "I", "Hq", "Hkv", "D", "page_size", "act", "o_splits", "down_splits",
                                    "gate_up_tile", "failed")]
-                + [(n, _P) for n in ("positions", "slots", "y", "residual", "qkv", "mixed", "product", "gate_up", "a")])
+                + [(n, _P) for n in ("positions", "slots", "y", "residual", "qkv", "mixed", "product", "gate_up", "a")]
+                + [("qkv_tile", _I)])
 
 
 class PromptLayer(ctypes.Structure):
     _fields_ = ([(n, _P) for n in ("qkv", "o", "gate_up", "down", "inv_freq", "post_norm", "next_norm", "k_cache", "v_cache")]
-                + [("post_eps", _F), ("next_eps", _F)])
+                + [("post_eps", _F), ("next_eps", _F), ("turns", _P)])
 
 
 def entries():

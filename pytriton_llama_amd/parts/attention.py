@@ -10,6 +10,7 @@ from .. import ops
 from .base import (ParamSource, Part, PendingProduct, PendingScale, WorkList, as_tensor,
                    paged_kv_spec, place, register_part)
 from .linear import LINEAR_LIBRARIES, decode_copy, linear
+from .rotary import RotaryEncoding
 
 
 # How the attention kernels cut the query rows of a step: 16 rows a work item for the vector-FMA
@@ -99,6 +100,12 @@ class PagedAttention(Part):
     takes_pending_scale = True
     can_defer_output = True
 
+    @property
+    def _in_tiles(self) -> bool:
+        """Whether the tiles know this part's position encoding: none, or the plain rotation."""
+        return self.position is None or (type(self.position) is RotaryEncoding
+                                         and "rotary_inv_freq" not in vars(self.position))
+
     def forward(self, x, ctx, cache, defer_output: bool = False):
         T = x.shape[0]
         Hq, Hkv, D = self.num_heads, self.num_kv_heads, self.head_dim
@@ -109,6 +116,12 @@ class PagedAttention(Part):
         if isinstance(x, PendingScale) and fused and ops.qkv_rope_store_fits(x.values, self.qkv, D):
             x, scale = x.values, x.scale
         x = as_tensor(x)
+        if (self._in_tiles and ops.qkv_rope_store_tile_fits(x, self.qkv, D)
+                and (cache.k.data_ptr() | cache.v.data_ptr()) % 16 == 0):
+            # some tens to hundreds of rows: projection, rotation (the step's cosines and sines) and cache write in tiles
+            q = ops.qkv_rope_store_tile(x, self.qkv, self.position.table(ctx) if self.position is not None else None,
+                                        group.slots if cache.writable else None, cache.k, cache.v, Hq, Hkv, D, cache.page_size)
+            return self._attended(q, ctx, cache, group, defer_output)
         if fused and ops.qkv_rope_store_fits(x, self.qkv, D, self.qkv_blocked):
             # the few rows of a decode step: projection, rotation and cache write in one kernel
             q = ops.qkv_rope_store(x, self.qkv, ctx.positions, rotary,

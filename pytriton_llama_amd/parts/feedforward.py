@@ -66,7 +66,8 @@ class SwiGLU(Part):
         elif ops.gate_up_f32_tiles_fits(x, self.gate_up):   # ... and of a prompt in float32
             a = ops.gate_up_f32_tiles(x, self.gate_up, self.act)
         elif ops.gate_up_tile_fits(x, self.gate_up):        # some hundred rows: the same in tiles
-            a = ops.gate_up_tile(x, self.gate_up, self.act, hw_silu=True)
+            # (SiLU as the other kernels for as many rows have it)
+            a = ops.gate_up_tile(x, self.gate_up, self.act, hw_silu=x.shape[0] > ops.ROWS_MAX["gate_up"])
         else:
             a = ops.silu_mul(linear(x, self.gate_up, blocked=self.gate_up_blocked), self.act)
         if defer_output:                    # (the norm that follows picks the kernels by the rows)

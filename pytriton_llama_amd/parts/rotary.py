@@ -97,6 +97,15 @@ class RotaryEncoding(Part):
     def rotary_inv_freq(self) -> Optional[torch.Tensor]:
         return self.inv_freq
 
+    def table(self, ctx) -> torch.Tensor:
+        """``ops.rope_table`` of the step's rows: one for all parts of the same frequencies in a model's pass over ``ctx``."""
+        if ctx.rotations is None:
+            return ops.rope_table(ctx.positions, self.inv_freq)
+        key = self.inv_freq_host.numpy().tobytes()
+        if key not in ctx.rotations:
+            ctx.rotations[key] = ops.rope_table(ctx.positions, self.inv_freq)
+        return ctx.rotations[key]
+
     def apply(self, q: torch.Tensor, k: torch.Tensor, positions: torch.Tensor) -> None:
         """Rotate q and k ([T, heads, D] views of one buffer) in place."""
         ops.rope_store(q, k, k, positions, self.inv_freq, None, None, None, 1, k_in_place=True)

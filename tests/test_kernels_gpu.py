@@ -1379,6 +1379,32 @@ def test_attention_decode_mfma_shares(ops, case, unroll):
                     **case)
 
 
+@pytest.mark.parametrize("Hq,Hkv,D", [(4, 1, 32), (3, 1, 64), (2, 2, 96), (5, 2, 128)])
+@pytest.mark.parametrize("tile", range(-1, 14))
+def test_qkv_rope_store_tile(ops, tile, Hq, Hkv, D):
+    """Every tile, rows and heads that do not fill it, rows that are stored nowhere: what the product (float32, rounded once) and
+    rope_store give, a bfloat16 rounding apart where the product's last bit differs by the order of its sum."""
+    P, pages, K = 8, 40, 192
+    torch.manual_seed(100 * D + tile)
+    for M in (1, 37, 150):
+        x = torch.randn(M, K, device="cuda").to(torch.bfloat16)
+        w = (torch.randn((Hq + 2 * Hkv) * D, K, device="cuda") * K ** -0.5).to(torch.bfloat16)
+        pos = torch.randint(0, 100000, (M,), device="cuda").int()
+        inv = (500000.0 ** (-torch.arange(0, D, 2, device="cuda").double() / D)).float()
+        slots = torch.randperm(P * pages, device="cuda")[:M].int()
+        slots[M // 2] = -1
+        caches = [torch.zeros(pages, Hkv, P, D, dtype=torch.bfloat16, device="cuda") for _ in range(4)]
+        for table in (ops.rope_table(pos, inv), None):
+            q = ops.qkv_rope_store_tile(x, w, table, slots, *caches[:2], Hq, Hkv, D, P, tile=tile)
+            y = (x.float() @ w.float().T).to(torch.bfloat16)
+            parts = [t.view(M, -1, D) for t in y.split([Hq * D, Hkv * D, Hkv * D], 1)]
+            ops.rope_store(*parts, pos, inv if table is not None else None, slots, *caches[2:], P)
+            for got, want in ((q, parts[0]), (caches[0], caches[2]), (caches[1], caches[3])):
+                torch.testing.assert_close(got.float(), want.float(), **tol(torch.bfloat16))
+        none = ops.qkv_rope_store_tile(x, w, None, None, None, None, Hq, Hkv, D, P, tile=tile)
+        assert torch.equal(none, q)
+
+
 @pytest.mark.parametrize("n", [12, 80])
 def test_attention_decode_mfma_shares_beside_empty_rows(ops, n):
     """Rows without keys (padding of a recorded step) between sequences of very different lengths: zeros

@@ -19,3 +19,15 @@ def test_products_with_the_norm_behind_them(N, K, most):
 def test_gate_up(I, K, most):
     """As for the sums; and as long as the largest tiles lie on the chip at once."""
     assert ops.tile_most_rows_gate_up(2 * I, K, 256) == most
+
+
+@pytest.mark.parametrize("rows_w,most", [(3072, 2048), (5120, 1228), (6144, 1024), (98304, 64)])
+def test_qkv(rows_w, most):
+    """As long as tiles of 128 x 192 lie on the chip at once."""
+    assert ops.tile_most_rows_qkv(rows_w, 256) == most
+
+
+@pytest.mark.parametrize("I,K,least", [(8192, 2048, 49), (8192, 3072, 33), (14336, 4096, 33), (5632, 2048, 49)])
+def test_gate_up_from(I, K, least):
+    """Below, the kernel for tens of rows was faster."""
+    assert ops.tile_least_rows_gate_up(2 * I, K) == least
