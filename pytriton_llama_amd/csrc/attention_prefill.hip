@@ -72,7 +72,13 @@ template <> __device__ __forceinline__ void store4<float>(float* p, const float*
 // tanh_exp2(raw score * cap_in) takes the place of the raw score and scale_log2 is softcap * log2 e.
 // SIDES: groups of four waves in the workgroup. Two sides take the key tiles of a block in turn, each
 // with buffers, maxima and sums of its own, which meet through LDS at the end.
-template <int NDK, int NDV, int RT, typename TO, bool KEPT, bool CAP, int SIDES>
+// PAGED: the rows that one load instruction brings (64 lanes of 16 bytes) lie in one page: sizes of 32, 64 and 128, pages of at least 16
+// rows, no kept keys. The page's number then comes by a scalar load and an address is a scalar base and the lane's
+// place: what a tile's loads cost the waves in instructions is most of what the loads cost (2,048 rows, 32 heads of 64, 43.3 us,
+// without any loads 30; a third buffer, which lets a tile take two turns to arrive, changes nothing). us before and with it: 38.7; 24 heads
+// of 128, 512 rows on 1,536 / 3,072 keys 32.4, 58.8 -> 31.6, 56.0, 2,048 rows 64.4 -> 58.3; 32 heads of 128, 2,048 rows on
+// 8,192 keys 284 -> 262; 16 heads, 1,531 rows 45.3 -> 41.8.
+template <int NDK, int NDV, int RT, typename TO, bool KEPT, bool CAP, int SIDES, bool PAGED>
 __global__ void __launch_bounds__(256 * SIDES, SIDES == 1 && (NDK + NDV) <= 4 ? 3 : 2)
 attn_prefill_mfma_kernel(TO* __restrict__ out, long out_stride, const bf16_t* __restrict__ q,
                          long q_stride, const bf16_t* __restrict__ k_cache,
@@ -227,9 +233,18 @@ attn_prefill_mfma_kernel(TO* __restrict__ out, long out_stride, const bf16_t* __
     const int k0 = k_begin + t * PF_BN;
     return t < n_tiles && k0 >= k_lo && k0 + PF_BN <= k_end;
   };
+  auto page_at = [&](int row) {                 // of a row that is the same in all lanes
+    const int kp = __builtin_amdgcn_readfirstlane(min(max(row, k_lo), k_end - 1)) >> page_shift;
+    return *(const __attribute__((address_space(4))) int32_t*)(uintptr_t)(bt + kp);
+  };
   auto load_pages = [&](int t) {
     const int k0 = k_begin + t * PF_BN;
-    if (whole(t)) {
+    if constexpr (PAGED) {
+#pragma unroll
+      for (int i = 0; i < NCHK; ++i) pgk[i] = page_at(k0 + 64 / CPRK * (wave_u * NCHK + i));
+#pragma unroll
+      for (int i = 0; i < NCHV; ++i) pgv[i] = page_at(k0 + 64 / CPRV * (wave_u * NCHV + i));
+    } else if (whole(t)) {
 #pragma unroll
       for (int i = 0; i < NCHK; ++i) pgk[i] = bt[key_at(k0 + crowk[i]) >> page_shift];
 #pragma unroll
@@ -265,18 +280,32 @@ attn_prefill_mfma_kernel(TO* __restrict__ out, long out_stride, const bf16_t* __
     const bool all = whole(t);
 #pragma unroll
     for (int i = 0; i < NCHK; ++i) {
-      if (all || pgk[i] >= 0) {
-        const uint32_t in_page = (uint32_t)((key_at(k0 + crowk[i]) & page_mask) * DK + ccolk[i]) * 2;
-        to_lds(k_head, (uint64_t)(uint32_t)pgk[i] * page_bytes_k + in_page, Kb, wave_u * NCHK + i);
+      if (PAGED ? all || (k0 + crowk[i] >= k_lo && k0 + crowk[i] < k_end) : all || pgk[i] >= 0) {
+        if constexpr (PAGED) {
+          const int first_row = 64 / CPRK * (wave_u * NCHK + i);
+          const uint64_t at = (uint64_t)(uint32_t)pgk[i] * page_bytes_k + (uint32_t)(((k0 + first_row) & page_mask) * (DK * 2));
+          to_lds(reinterpret_cast<const bf16_t*>(reinterpret_cast<const char*>(k_head) + at),
+                 (uint32_t)((crowk[i] - first_row) * DK + ccolk[i]) * 2, Kb, wave_u * NCHK + i);
+        } else {
+          const uint32_t in_page = (uint32_t)((key_at(k0 + crowk[i]) & page_mask) * DK + ccolk[i]) * 2;
+          to_lds(k_head, (uint64_t)(uint32_t)pgk[i] * page_bytes_k + in_page, Kb, wave_u * NCHK + i);
+        }
       } else {                                    // rows outside the keys read as zeros
         *reinterpret_cast<uint4*>(Kb + 8 * (64 * (wave_u * NCHK + i) + lane)) = make_uint4(0, 0, 0, 0);
       }
     }
 #pragma unroll
     for (int i = 0; i < NCHV; ++i) {
-      if (all || pgv[i] >= 0) {
-        const uint32_t in_page = (uint32_t)((key_at(k0 + crowv[i]) & page_mask) * DV + ccolv[i]) * 2;
-        to_lds(v_head, (uint64_t)(uint32_t)pgv[i] * page_bytes_v + in_page, Vb, wave_u * NCHV + i);
+      if (PAGED ? all || (k0 + crowv[i] >= k_lo && k0 + crowv[i] < k_end) : all || pgv[i] >= 0) {
+        if constexpr (PAGED) {
+          const int first_row = 64 / CPRV * (wave_u * NCHV + i);
+          const uint64_t at = (uint64_t)(uint32_t)pgv[i] * page_bytes_v + (uint32_t)(((k0 + first_row) & page_mask) * (DV * 2));
+          to_lds(reinterpret_cast<const bf16_t*>(reinterpret_cast<const char*>(v_head) + at),
+                 (uint32_t)((crowv[i] - first_row) * DV + ccolv[i]) * 2, Vb, wave_u * NCHV + i);
+        } else {
+          const uint32_t in_page = (uint32_t)((key_at(k0 + crowv[i]) & page_mask) * DV + ccolv[i]) * 2;
+          to_lds(v_head, (uint64_t)(uint32_t)pgv[i] * page_bytes_v + in_page, Vb, wave_u * NCHV + i);
+        }
       } else {
         *reinterpret_cast<uint4*>(Vb + 8 * (64 * (wave_u * NCHV + i) + lane)) = make_uint4(0, 0, 0, 0);
       }
@@ -489,14 +518,16 @@ static int launch_prefill_mfma(void* out, long out_stride, const void* q, long q
   if (kept && cap) return PTL_ERR_ARG;
   const float log2e = 1.4426950408889634f;
   const float scale_log2 = (cap ? ex.softcap : scale) * log2e, cap_in = cap ? 2.0f * log2e * scale / ex.softcap : 0.f;
-#define GO(KEPT, CAP)                                                                                       \
-  attn_prefill_mfma_kernel<NDK, NDV, RT, TO, KEPT, CAP, SIDES><<<grid, 256 * SIDES, 0, stream>>>(           \
+  constexpr bool SIZES = NDK != 3 && NDV != 3;
+#define GO(KEPT, CAP, PAGED)                                                                                \
+  attn_prefill_mfma_kernel<NDK, NDV, RT, TO, KEPT, CAP, SIDES, PAGED><<<grid, 256 * SIDES, 0, stream>>>(    \
       (TO*)out, out_stride, (const bf16_t*)q, q_stride, (const bf16_t*)k_cache, (const bf16_t*)v_cache,     \
       q_start, ctx_len, block_table, bt_stride, work_seq, work_qoff, n_work, Hq, Hkv, maps, page_size,      \
       page_shift, ex, scale_log2, cap_in)
-  if (kept) GO(true, false);
-  else if (cap) GO(false, true);
-  else GO(false, false);
+  if (kept) GO(true, false, false);
+  else if (cap) GO(false, true, false);
+  else if (SIZES && page_size >= 16) GO(false, false, SIZES);
+  else GO(false, false, false);
 #undef GO
   return ptl_launch_status();
 }

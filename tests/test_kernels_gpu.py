@@ -1608,6 +1608,44 @@ def test_attention_prefill_mfma_window(ops, kernel):
                     P=8, window=70, kernel=kernel)
 
 
+@pytest.mark.parametrize("masks", [dict(), dict(window=70), dict(chunk=96)], ids=["all", "window", "chunk"])
+@pytest.mark.parametrize("D", [32, 64, 96, 128])
+@pytest.mark.parametrize("rows", [64, 128])
+def test_attention_prefill_mfma_page_numbers_of_a_wave(ops, D, masks, rows):
+    """Pages of 16 rows and more have their numbers read once for the rows of a load instruction: the bits that pages of 8 rows
+    give, whose numbers every lane reads, at portions that begin and end inside pages, with pages left of a window given back."""
+    torch.manual_seed(D)
+    q_lens, lens, Hq, Hkv = [1, 65, 130, 200], [77, 300, 130, 513], 6, 2
+    first = [0] * 4
+    if "window" in masks:
+        first = [max(0, n - q - masks["window"] + 1) for q, n in zip(q_lens, lens)]
+    if "chunk" in masks:
+        first = [(n - q) // masks["chunk"] * masks["chunk"] for q, n in zip(q_lens, lens)]
+    keys = [torch.randn(2, n, Hkv, D).to(torch.bfloat16) for n in lens]
+    q = torch.randn(sum(q_lens), Hq, D, device="cuda").to(torch.bfloat16)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")
+    from pytriton_llama_amd.engine.batch import work_items
+    lists = [i32(t.tolist()) for t in work_items(q_lens, lens, 0, rows)]
+    outs = []
+    for P in (8, 16, 32, 128):
+        pages = [-(-n // P) for n in lens]
+        table = torch.full((4, max(pages)), -1, dtype=torch.int32)
+        pool = torch.full((2, sum(pages), Hkv, P, D), float("nan"), dtype=torch.bfloat16)
+        order, at = torch.randperm(sum(pages)), 0
+        for i, n in enumerate(lens):
+            for p in range(pages[i]):
+                page, take = int(order[at]), keys[i][:, p * P:(p + 1) * P]
+                pool[:, page, :, :take.shape[1]] = take.transpose(1, 2)
+                table[i, p] = page if (p + 1) * P > first[i] else -1
+                at += 1
+        out = torch.zeros_like(q)
+        ops.attention_prefill_mfma(out, q, pool[0].cuda(), pool[1].cuda(), i32([0, 1, 66, 196, 396]), i32(lens), table.cuda(),
+                                   *lists, D ** -0.5, block_rows=rows, **masks)
+        outs.append(out)
+    assert bool(torch.isfinite(outs[0].float()).all())
+    assert all(torch.equal(o, outs[0]) for o in outs[1:])
+
+
 def test_attention_prefill_mfma_refuses_odd_page_size(ops):
     """A page size that is no power of two is for the general kernel; the fast one says so."""
     assert not ops.attention_prefill_mfma_fits(torch.bfloat16, 1, 32, 5)
