@@ -575,7 +575,7 @@ extern "C" int ptl_attention_prefill_mfma(void* out, long out_stride, const void
       Hq > 65535 || n_groups < 1 || n_groups > n_work || q_stride % 8 || out_stride % 4 ||
       (block_rows != 64 && block_rows != 128) || !extras_ok(ex))
     return PTL_ERR_ARG;
-  // Two sides where there are no more workgroups than compute units and portions are long enough to have long
+  // Two sides where there are few workgroups a compute unit and portions are long enough to have long
   // chains of key tiles by themselves. A block's time is that of its
   // chain of key tiles, and a compute unit with one workgroup of four waves has one wave a SIMD, which
   // nothing covers: eight waves on two chains of half the length hold the unit as well as a second
@@ -587,7 +587,18 @@ extern "C" int ptl_attention_prefill_mfma(void* out, long out_stride, const void
   // prompt would pay in every layer; a short portion behind a long prefix gains (64 rows on 320 keys 12.1 ->
   // 11.3, on 1,088 29.9 -> 22.8). How many keys a recorded step will have is not known at its launch: callers give
   // the rows of what is most likely a prompt of its own, and 0 where a prefix is as likely.
-  if (block_rows == 64 && (longest <= 0 || longest > 256) && (long)n_groups * Hq <= compute_units())
+  // Up to two workgroups a unit: at head sizes up to 64 two of eight waves fit as well, so two sides win for lists of more than
+  // 256 rows (longest not known) or with a portion of 512; above, a unit holds one at a time, and they win for a
+  // prompt by itself only, whose workgroups are of all lengths (us with one side and two; 32 heads of 64: 700 rows 13.9 / 11.7,
+  // 1,024 18.4 / 15.7, 700 on 3,072 keys 48.5 / 40.9, 1,024 on 4,096 64.5 / 53.5, twice 512 11.5 / 11.1, but three times 260 8.7 /
+  // 9.5; 16 heads of 128: 1,531 rows 40.7 / 30.8, 2,048 53.0 / 45.6; 24 of 128: 700 rows 21.4 / 18.2, 1,024 29.0 / 25.2, but
+  // 700 on 3,072 keys 78 / 91 and 300 + 200 + 257 + 100 12.6 / 15.6; 32 of 128: twice 512 17.8 / 21.1). Three workgroups a unit are
+  // level at head size 64 (1,531 rows of 32 heads 25.9 / 26.4) and lose above (42.1 / 48.0).
+  const long groups = (long)n_groups * Hq, units = compute_units();
+  const bool both = groups <= units ||
+                    (groups <= 2 * units && (D <= 64 ? (longest <= 0 ? n_groups > 4 : longest >= 512)
+                                                     : longest > 0 && longest > 64L * (n_work - 2)));
+  if (block_rows == 64 && (longest <= 0 || longest > 256) && both)
     return prefill_same_size<1, 2>(D / 32, out, out_stride, q, q_stride, k_cache, v_cache, q_start, ctx_len,
                                    block_table, bt_stride, work_seq, work_qoff, n_work, n_groups, Hq, Hkv,
                                    page_size, ex, scale, stream);
