@@ -679,7 +679,7 @@ def gemm_rows_add_rmsnorm_fits(x: torch.Tensor, w: torch.Tensor, blocked: Option
                                residual: torch.Tensor, norm_weight: torch.Tensor) -> bool:
     N = w.shape[0]
     return (_rows_x_ok(x, w, blocked, "add_norm") and _sum_norm_ok(x, N, residual, norm_weight)
-            and not gemm_tile_add_rmsnorm_fits(x, w, residual, norm_weight))
+            and (x.shape[0] < TILE_MIN_ROWS or not gemm_tile_add_rmsnorm_fits(x, w, residual, norm_weight)))
 
 
 def gemm_rows_add_rmsnorm(x: torch.Tensor, w: torch.Tensor, blocked: torch.Tensor, residual: torch.Tensor,

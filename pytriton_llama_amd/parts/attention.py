@@ -116,7 +116,7 @@ class PagedAttention(Part):
         if isinstance(x, PendingScale) and fused and ops.qkv_rope_store_fits(x.values, self.qkv, D):
             x, scale = x.values, x.scale
         x = as_tensor(x)
-        if (self._in_tiles and ops.qkv_rope_store_tile_fits(x, self.qkv, D)
+        if (T >= ops.TILE_MIN_ROWS and self._in_tiles and ops.qkv_rope_store_tile_fits(x, self.qkv, D)
                 and (cache.k.data_ptr() | cache.v.data_ptr()) % 16 == 0):
             # some tens to hundreds of rows: projection, rotation (the step's cosines and sines) and cache write in tiles
             q = ops.qkv_rope_store_tile(x, self.qkv, self.position.table(ctx) if self.position is not None else None,
@@ -209,7 +209,7 @@ class PagedAttention(Part):
             ops.attention_decode(out, q, k, v, ctx.q_start, ctx.ctx_len,
                                  group.block_table, n_dec, self.scale, window,
                                  self.decode_splits(ctx, n_dec, mfma, q.device), matrix_cores=mfma,
-                                 sink=self.sink, tickets=ctx.tickets)
+                                 sink=self.sink, tickets=getattr(ctx, "tickets", None))
         if n_dec == ctx.num_seqs:
             return
         if (ops.attention_prefill_mfma_fits(q.dtype, self.num_kv_heads, D, cache.page_size)

@@ -42,15 +42,16 @@ class RMSNorm(Part):
 
     def forward(self, x, residual: Optional[torch.Tensor], scale_ok: bool = False):
         if isinstance(x, PendingProduct):
-            # some tens of rows (from ops.ROWS_MIN on): the product as partial sums over slices of
-            # K, then one kernel that adds them up, adds the residual and normalises
+            # some tens to hundreds of rows: the product as partial sums over slices of K, in tiles of rows of x and of
+            # W, then one kernel that adds them up, adds the residual and normalises
+            if (residual is not None and x.x.shape[0] >= ops.TILE_MIN_ROWS
+                    and ops.gemm_tile_add_rmsnorm_fits(x.x, x.w, residual, self.weight)):
+                y = ops.gemm_tile_add_rmsnorm(x.x, x.w, residual, self.weight, self.eps)
+                return y, residual
+            # fewer rows (from ops.ROWS_MIN on): the same by the kernel that streams the blocked copy of W
             if (residual is not None and x.blocked is not None
                     and ops.gemm_rows_add_rmsnorm_fits(x.x, x.w, x.blocked, residual, self.weight)):
                 y = ops.gemm_rows_add_rmsnorm(x.x, x.w, x.blocked, residual, self.weight, self.eps)
-                return y, residual
-            # some hundred rows (a portion of a prompt): the same, in tiles of rows of x and of W
-            if residual is not None and ops.gemm_tile_add_rmsnorm_fits(x.x, x.w, residual, self.weight):
-                y = ops.gemm_tile_add_rmsnorm(x.x, x.w, residual, self.weight, self.eps)
                 return y, residual
             # the few rows of a decode step: the product, the residual sum and the weight in one
             # kernel; the rsqrt factor is left to the part that takes the result

@@ -208,7 +208,7 @@ class NormedAttention(Part):
         window = self.window or 0
         extras = dict(keep_first=self.keep_first, sink=self.sink, chunk=self.chunk or 0, gate=gate,
                       softcap=self.softcap)
-        decode = dict(extras, tickets=ctx.tickets)
+        decode = dict(extras, tickets=getattr(ctx, "tickets", None))
         # one map and keys as large as values: the matrix-core form of the split-KV kernel takes them
         mfma = (n_dec and self.maps == 1 and self.dim == self.vdim and q.stride(0) % 8 == 0
                 and ops.attention_decode_mfma_fits(q.dtype, self.num_heads, self.num_kv_heads, self.dim,

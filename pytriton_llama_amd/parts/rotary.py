@@ -99,7 +99,7 @@ class RotaryEncoding(Part):
 
     def table(self, ctx) -> torch.Tensor:
         """``ops.rope_table`` of the step's rows: one for all parts of the same frequencies in a model's pass over ``ctx``."""
-        if ctx.rotations is None:
+        if getattr(ctx, "rotations", None) is None:
             return ops.rope_table(ctx.positions, self.inv_freq)
         key = self.inv_freq_host.numpy().tobytes()
         if key not in ctx.rotations:
