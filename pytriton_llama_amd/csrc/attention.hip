@@ -28,6 +28,7 @@
 // (float32 or bfloat16), any page size, any D up to 640 (beyond 256 with more LDS than a
 // kernel gets unasked: the launcher asks for it).
 #include "attention.h"
+#include "attention_decode.h"
 #include "attention_f32.h"
 #include "common.h"
 #include "device.h"
@@ -660,28 +661,6 @@ extern "C" int ptl_attention_decode(void* out, long out_stride, const void* q, l
 // that head's column; the waves are merged at the end of a part. Needs D % 32 == 0, D <= 128, Hq/Hkv <= 16, a page size
 // that is a power of two, pages (of all kv heads) below 4 GiB.
 // ===========================================================================
-__device__ __forceinline__ void wave_lds_fence() {
-  // orders this wave's LDS writes and reads for the compiler; the LDS itself runs a wave's
-  // instructions in order
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-#define DECODE_LIST_SEQS 64        // sequences of a listed launch (one a lane)
-#define DECODE_MOST_PARTS 16       // parts that ``piece`` cuts a pair into at most
-
-// What parts of a pair the workgroups leave for the one that merges them.
-struct DecodeParts {
-  float *acc, *ml;                 // [sequence][head][most][D] results, [..][2] their maximum (of scores times log2 e) and denominator
-  int* tickets;                    // [sequence][kv head][TICKET]: parts that are done
-  int most;                        // parts a pair has room for
-};
-
-// LISTED: a list of parts (above), cus: the compute units, the grid a multiple of them; else a grid of workgroups
-// (sequence, kv head, split), the sequences fastest.
-// KEPT: a window that keeps the sequence's first keys (keep_first > 0). CAP: scores are capped; then
-// scale_log2 is softcap * log2 e and cap_in takes a raw score to tanh_exp2's argument.
 template <int NDT, int UNR, bool LISTED, bool KEPT, bool CAP>
 __global__ void __launch_bounds__(256, NDT <= 2 ? 3 : 2)
 attn_decode_mfma_kernel(const int32_t* __restrict__ ctx_len, const int32_t* __restrict__ block_table,
@@ -689,305 +668,12 @@ attn_decode_mfma_kernel(const int32_t* __restrict__ ctx_len, const int32_t* __re
                         int num_splits, int bt_stride, int page_size, int page_shift, const bf16_t* __restrict__ q, long q_stride,
                         int Hq, int cus, int piece, bf16_t* __restrict__ out, long out_stride,
                         const int32_t* __restrict__ q_start, DecodeParts parts, AttnExtras ex, float scale_log2, float cap_in) {
-  constexpr int D = 32 * NDT;
-  constexpr int NT = 2 * NDT;             // 16-wide tiles of the head dimension
-  constexpr int WAVES = 4;
-  constexpr int UNIT = 16 * UNR;          // keys of a wave's turn
-  constexpr int TILE = UNIT * WAVES;      // ... of the workgroup's
-  constexpr int VS = D + 16;              // row stride of a value tile in LDS, in elements
-  constexpr int CPR = D / 8;              // 16-byte chunks per row
-  constexpr int VCH = 16 * CPR / 64;      // chunks of a tile per lane
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int ln = lane & 15, lg = lane >> 4;
-  const int G = Hq / Hkv;
-  const int page_mask = page_size - 1;
-  const uint32_t page_bytes = (uint32_t)Hkv * page_size * D * 2;
   extern __shared__ float lds[];
-  bf16_t* vl = reinterpret_cast<bf16_t*>(lds) + (size_t)wave * UNR * 16 * VS;
-  // this lane's chunks of a value tile: row vrow[i], elements vcol[i] .. +7
-  int vrow[VCH], vcol[VCH];
-#pragma unroll
-  for (int i = 0; i < VCH; ++i) {
-    const int c = lane + 64 * i;
-    vrow[i] = c / CPR;
-    vcol[i] = (c - vrow[i] * CPR) * 8;
-  }
-  int seq = blockIdx.x % n_seq, kvh = blockIdx.x / n_seq % Hkv, split = blockIdx.x / (n_seq * Hkv), per, n_parts;
-  if (LISTED) {
-    // lane s has sequence s: the keys of its parts, and how many of them a pair has
-    const int c = lane < n_seq ? ctx_len[lane] : 0, keys = c > 0 ? walk_of(ex, c) : 0;
-    const int lane_per = keys_a_split(keys, min(max(num_splits, (keys + piece - 1) / piece), parts.most), TILE);   // (below too)
-    const int lane_parts = lane < n_seq ? max(1, (keys + lane_per - 1) / lane_per) : 0;
-    const unsigned long long some = __ballot(keys > 0);
-    const int one = some ? __builtin_amdgcn_readlane(keys, __ffsll(some) - 1) : 0;
-    if (__any(keys > 0 && abs(keys - one) > one / 4)) {
-      const int turn = blockIdx.x / cus, unit = blockIdx.x - turn * cus, at = turn * cus + (turn % 2 ? cus - 1 - unit : unit);
-      const int group = at / (8 * Hkv), in_group = at - group * 8 * Hkv, u = 8 * group + in_group % 8;
-      int all = lane_parts;
-#pragma unroll
-      for (int o = 1; o < 64; o <<= 1) all += __shfl_xor(all, o, 64);
-      if (u >= all) return;
-      // the longest parts first: every wave counts a quarter of the sequences that come before the lane's
-      const int packed = (keys > 0 ? min(lane_per, 1 << 24) : 0) << 6 | (63 - lane);
-      int start = 0;
-      for (int s = __builtin_amdgcn_readfirstlane(wave); s < n_seq; s += WAVES)
-        start += __builtin_amdgcn_readlane(packed, s) > packed ? __builtin_amdgcn_readlane(lane_parts, s) : 0;
-      int* counts = reinterpret_cast<int*>(lds);
-      counts[wave * 64 + lane] = start;
-      __syncthreads();
-      start = 0;
-#pragma unroll
-      for (int w = 0; w < WAVES; ++w) start += counts[w * 64 + lane];
-      __syncthreads();
-      seq = __ffsll((unsigned long long)__ballot(u >= start && u < start + lane_parts)) - 1;
-      kvh = in_group / 8;
-      split = u - __builtin_amdgcn_readlane(start, seq);
-    }
-    per = __builtin_amdgcn_readlane(lane_per, seq);
-    n_parts = __builtin_amdgcn_readlane(lane_parts, seq);
-    if (split >= n_parts) return;
-  }
-  const int head0 = kvh * G;
-  const int row = q_start[seq];
-  const int ctx = ctx_len[seq];
-  const int k_lo = first_seen(ex, ctx - 1);
-  // the walk: the kept first keys left of the window, then the window; k_begin, k_end and the
-  // keys of a turn are indices of the walk, key_at gives the position
-  const int n_kept = KEPT ? min(max(ex.keep_first, 0), k_lo) : 0;
-  const int shift = k_lo - n_kept;
-  const int span = ctx - shift;
-  if (!LISTED) {
-    per = keys_a_split(span, min(max(num_splits, (span + piece - 1) / piece), parts.most), TILE);
-    n_parts = max(1, (span + per - 1) / per);
-    if (split >= n_parts) return;
-  }
-  const int k_begin = split * per;
-  const int k_end = min(span, k_begin + per);
-  const int turns = (k_end - k_begin + TILE - 1) / TILE;
-  auto key_at = [&](int kw) { return (KEPT && kw < n_kept) ? kw : kw + shift; };
-  const int32_t* bt = block_table + (size_t)seq * bt_stride;
-  const char* k_head = reinterpret_cast<const char*>(k_cache) + (size_t)kvh * page_size * D * 2;
-  const char* v_head = reinterpret_cast<const char*>(v_cache) + (size_t)kvh * page_size * D * 2;
-
-  Frag8 qf[NDT];
-#pragma unroll
-  for (int kk = 0; kk < NDT; ++kk) {
-    qf[kk].u = make_uint4(0, 0, 0, 0);
-    if (ln < G)
-      qf[kk].u = *reinterpret_cast<const uint4*>(q + (size_t)row * q_stride +
-                                                 (size_t)(head0 + ln) * D + 32 * kk + 8 * lg);
-  }
-  f32x4_t o[NT];
-#pragma unroll
-  for (int t = 0; t < NT; ++t) o[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  float m_run = -INFINITY, l_part = 0.f;
-
-  int pk[UNR], pv[UNR][VCH];            // pages of the key row and of the value chunks' rows
-  uint4 vg[UNR][VCH];                   // values on their way to LDS
-  auto first_key = [&](int turn) { return k_begin + turn * TILE + 16 * UNR * wave; };
-  auto load_pages = [&](int turn) {
-    const int kc = first_key(turn);
-#pragma unroll
-    for (int u = 0; u < UNR; ++u) {
-      const int kp = kc + 16 * u + ln;
-      pk[u] = (turn < turns && kp < k_end) ? bt[key_at(kp) >> page_shift] : -1;
-#pragma unroll
-      for (int i = 0; i < VCH; ++i) {
-        const int vp = kc + 16 * u + vrow[i];
-        pv[u][i] = (turn < turns && vp < k_end) ? bt[key_at(vp) >> page_shift] : -1;
-      }
-    }
-  };
-  auto issue_loads = [&](int turn, Frag8 (&kf)[UNR][NDT]) {
-    const int kc = first_key(turn);
-#pragma unroll
-    for (int u = 0; u < UNR; ++u) {
-      const int kp = key_at(kc + 16 * u + ln);
-      const char* kr = k_head + (size_t)(uint32_t)max(pk[u], 0) * page_bytes +
-                       (uint32_t)(((kp & page_mask) * D + 8 * lg) * 2);
-#pragma unroll
-      for (int kk = 0; kk < NDT; ++kk)
-        kf[u][kk].u = pk[u] >= 0 ? load_once(kr + 64 * kk) : make_uint4(0, 0, 0, 0);
-#pragma unroll
-      for (int i = 0; i < VCH; ++i) {
-        const int vp = key_at(kc + 16 * u + vrow[i]);
-        vg[u][i] = make_uint4(0, 0, 0, 0);              // rows past the end read as zeros
-        if (pv[u][i] >= 0)
-          vg[u][i] = load_once(v_head + (size_t)(uint32_t)pv[u][i] * page_bytes +
-                               (uint32_t)(((vp & page_mask) * D + vcol[i]) * 2));
-      }
-    }
-  };
-  // one turn: the values that arrived go to LDS, the next turn's loads are issued, this
-  // turn's keys (in kf) and values (in LDS) are used
-  auto step = [&](int turn, Frag8 (&kf)[UNR][NDT], Frag8 (&kf_next)[UNR][NDT]) {
-    wave_lds_fence();                                   // the last turn's reads are done
-#pragma unroll
-    for (int u = 0; u < UNR; ++u)
-#pragma unroll
-      for (int i = 0; i < VCH; ++i)
-        *reinterpret_cast<uint4*>(vl + (u * 16 + vrow[i]) * VS + vcol[i]) = vg[u][i];
-    wave_lds_fence();
-    if (turn + 1 < turns) {
-      issue_loads(turn + 1, kf_next);
-      load_pages(turn + 2);
-    }
-    const int kc = first_key(turn);
-    if (kc >= k_end) return;                            // wave-uniform: nothing of this turn is ours
-    f32x4_t st[UNR];
-#pragma unroll
-    for (int u = 0; u < UNR; ++u) {
-      st[u] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int kk = 0; kk < NDT; ++kk)
-        st[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[u][kk].v, qf[kk].v, st[u], 0, 0, 0);
-    }
-    float tmax = -INFINITY;
-#pragma unroll
-    for (int u = 0; u < UNR; ++u)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        float sc = (CAP ? tanh_exp2(st[u][i] * cap_in) : st[u][i]) * scale_log2;
-        sc = (kc + 16 * u + 4 * lg + i < k_end) ? sc : -INFINITY;
-        st[u][i] = sc;
-        tmax = fmaxf(tmax, sc);
-      }
-    tmax = max_with_lane_xor16(tmax);
-    tmax = max_with_lane_xor32(tmax);
-    if (tmax > m_run) {                                 // (finite: key kc is in range)
-      const float alpha = __builtin_amdgcn_exp2f(m_run - tmax);
-      m_run = tmax;
-      l_part *= alpha;
-#pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        o[t][0] *= alpha; o[t][1] *= alpha; o[t][2] *= alpha; o[t][3] *= alpha;
-      }
-    }
-    s16x4_t pb[UNR];
-#pragma unroll
-    for (int u = 0; u < UNR; ++u)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float p = __builtin_amdgcn_exp2f(st[u][i] - m_run);
-        l_part += p;
-        pb[u][i] = (short)float_to_bf16(p);
-      }
-    const bf16_t* vp = vl + (4 * lg + (ln >> 2)) * VS + 4 * (ln & 3);
-#pragma unroll
-    for (int u = 0; u < UNR; ++u)
-#pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        const s16x4_t vf = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-            (__attribute__((address_space(3))) s16x4_t*)(vp + u * 16 * VS + 16 * t));
-        o[t] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(vf, pb[u], o[t], 0, 0, 0);
-      }
-  };
-
-  Frag8 kfa[UNR][NDT], kfb[UNR][NDT];
-  load_pages(0);
-  issue_loads(0, kfa);
-  load_pages(1);
-  for (int turn = 0; turn < turns; turn += 2) {
-    step(turn, kfa, kfb);
-    if (turn + 1 < turns) step(turn + 1, kfb, kfa);
-  }
-  float l = l_part + __shfl_xor(l_part, 16, 64);
-  l += __shfl_xor(l, 32, 64);
-
-  // column d of the h-th head's result: the weighted sum a of values and the denominator ll to the maximum mn
-  auto write = [&](int h, int d, float mn, float ll, float a) {
-    const int head = head0 + h;
-    if (ex.sink) {                         // one more term of the denominator: exp(sink)
-      const float sk = ex.sink[head] * 1.4426950408889634f;
-      const float mx = fmaxf(mn, sk);
-      const float f = __builtin_amdgcn_exp2f(mn - mx);
-      ll = ll * f + __builtin_amdgcn_exp2f(sk - mx);
-      a *= f;
-    }
-    out[(size_t)row * out_stride + (size_t)head * D + d] =
-        float_to_bf16(ll > 0.f ? a / ll * head_gate(ex, row, head) : 0.f);
-  };
-
-  // merge the waves: [wave][head][D] accumulators, [wave][head][2] (max, denominator);
-  // the region takes the place of the value tiles, which every wave has left by now
-  __syncthreads();
-  float* w_acc = lds;
-  float* w_ml = lds + WAVES * 16 * D;
-  if (ln < G) {
-#pragma unroll
-    for (int t = 0; t < NT; ++t)
-      *reinterpret_cast<f32x4_t*>(w_acc + (wave * 16 + ln) * D + 16 * t + 4 * lg) = o[t];
-    if (lg == 0) { w_ml[(wave * 16 + ln) * 2] = m_run; w_ml[(wave * 16 + ln) * 2 + 1] = l; }
-  }
-  __syncthreads();
-  for (int i = tid; i < G * D; i += 64 * WAVES) {
-    const int h = i / D, d = i - h * D;
-    float mn = -INFINITY;
-#pragma unroll
-    for (int w = 0; w < WAVES; ++w) mn = fmaxf(mn, w_ml[(w * 16 + h) * 2]);
-    const float ms = mn == -INFINITY ? 0.f : mn;
-    float ll = 0.f, a = 0.f;
-#pragma unroll
-    for (int w = 0; w < WAVES; ++w) {
-      const float f = __builtin_amdgcn_exp2f(w_ml[(w * 16 + h) * 2] - ms);
-      ll += w_ml[(w * 16 + h) * 2 + 1] * f;
-      a += w_acc[(w * 16 + h) * D + d] * f;
-    }
-    if (n_parts == 1) {
-      write(h, d, mn, ll, a);
-    } else {
-      const size_t p = ((size_t)seq * Hq + head0 + h) * parts.most + split;
-      put_shared(parts.acc + p * D + d, a);
-      if (d == 0) { put_shared(parts.ml + p * 2, mn); put_shared(parts.ml + p * 2 + 1, ll); }
-    }
-  }
-  if (n_parts > 1) {
-    int* done = reinterpret_cast<int*>(w_ml + WAVES * 16 * 2);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // this wave's part of the part has reached memory
-    __syncthreads();
-    if (tid == 0) *done = last_part(parts.tickets + ((size_t)seq * Hkv + kvh) * TICKET, n_parts);
-    __syncthreads();
-    if (*done) {
-      // (the parts lie a long way off: eight of them are asked for at once)
-      constexpr int AHEAD = 8;
-      for (int i = tid; i < G * D; i += 64 * WAVES) {
-        const int h = i / D, d = i - h * D;
-        const size_t p = ((size_t)seq * Hq + head0 + h) * parts.most;
-        const float *acc = parts.acc + p * D + d, *ml = parts.ml + p * 2;
-        float mn = -INFINITY, ll = 0.f, a = 0.f;
-        for (int s0 = 0; s0 < n_parts; s0 += AHEAD) {
-          float av[AHEAD], mv[AHEAD], lv[AHEAD];
-#pragma unroll
-          for (int s = 0; s < AHEAD; ++s) {
-            const int at = min(s0 + s, n_parts - 1);
-            mv[s] = get_shared(ml + 2 * at);
-            lv[s] = get_shared(ml + 2 * at + 1);
-            av[s] = get_shared(acc + (size_t)at * D);
-          }
-          float m_new = mn;
-#pragma unroll
-          for (int s = 0; s < AHEAD; ++s) m_new = fmaxf(m_new, mv[s]);
-          const float ms = m_new == -INFINITY ? 0.f : m_new, f0 = __builtin_amdgcn_exp2f(mn - ms);
-          ll *= f0;
-          a *= f0;
-#pragma unroll
-          for (int s = 0; s < AHEAD; ++s) {
-            const float f = s0 + s < n_parts ? __builtin_amdgcn_exp2f(mv[s] - ms) : 0.f;
-            ll = fmaf(lv[s], f, ll);
-            a = fmaf(av[s], f, a);
-          }
-          mn = m_new;
-        }
-        write(h, d, mn, ll, a);
-      }
-    }
-  }
+  attn_decode_part<NDT, UNR, LISTED, KEPT, CAP>(
+      blockIdx.x, [](int w) { return lds + w * (decode_region<NDT, UNR>() / 4); }, ctx_len, block_table, k_cache, v_cache, n_seq,
+      Hkv, num_splits, bt_stride, page_size, page_shift, q, q_stride, Hq, cus, piece, out, out_stride, q_start, parts, ex,
+      scale_log2, cap_in);
 }
-
-// Whether the parts of all pairs are one list.
-static bool decode_listed(int n_seq) { return n_seq > 8 && n_seq <= DECODE_LIST_SEQS; }
-// The keys beyond which a part is cut again (figures above).
-static int decode_piece(int D, int num_splits) { return D <= 64 ? 1536 : num_splits == 1 ? 2048 : 1024; }
 
 template <int NDT, int UNR, bool LISTED>
 static int launch_decode_mfma(void* out, long out_stride, const void* q, long q_stride,
@@ -997,15 +683,12 @@ static int launch_decode_mfma(void* out, long out_stride, const void* q, long q_
                               float scale, int num_splits, int most, int piece, hipStream_t stream) {
   constexpr int D = 32 * NDT, WAVES = 4;
   const int cus = compute_units();
-  long groups = (long)n_seq * Hkv * most;
-  if (LISTED) groups = ((long)(n_seq * most + 7) / 8 * 8 * Hkv + cus - 1) / cus * cus;   // (whole turns of the units)
+  const long groups = decode_groups(n_seq, Hkv, most, LISTED, cus);
   if (groups > 0x7fffffff) return PTL_ERR_ARG;
   const DecodeParts dp{parts, parts ? parts + (long)n_seq * Hq * most * D : nullptr, tickets, most};
   int page_shift = 0;
   while ((1 << page_shift) < page_size) ++page_shift;
-  const size_t lds_merge = (size_t)WAVES * 16 * (D + 2) * sizeof(float) + 16;
-  const size_t lds_values = (size_t)WAVES * UNR * 16 * (D + 16) * sizeof(bf16_t);
-  const size_t lds = lds_merge > lds_values ? lds_merge : lds_values;
+  const size_t lds = (size_t)WAVES * decode_region<NDT, UNR>();
   const bool kept = ex.window > 0 && ex.keep_first > 0, cap = ex.softcap > 0.f;
   const float log2e = 1.4426950408889634f;
   const float scale_log2 = (cap ? ex.softcap : scale) * log2e, cap_in = cap ? 2.0f * log2e * scale / ex.softcap : 0.f;

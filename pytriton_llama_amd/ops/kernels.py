@@ -1243,6 +1243,55 @@ def attention_prefill_mfma(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Te
         *extras, ctypes.c_float(scale), _stream()), "attention_prefill_mfma")
 
 
+def attention_step_fits(dtype: torch.dtype, num_heads: int, num_kv_heads: int, head_dim: int, page_size: int) -> bool:
+    """Whether ``attention_step`` takes this case: what both of its kernels take, of head size 64 or 128, pages of 16 and more."""
+    return (head_dim in (64, 128) and page_size >= 16
+            and attention_decode_mfma_fits(dtype, num_heads, num_kv_heads, head_dim, page_size)
+            and attention_prefill_mfma_fits(dtype, num_kv_heads, head_dim, page_size))
+
+
+def attention_step(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, q_start: torch.Tensor,
+                   ctx_len: torch.Tensor, block_table: torch.Tensor, n_seq: int, work_seq: torch.Tensor,
+                   work_qoff: torch.Tensor, scale: float, window: int = 0, num_splits: int = 1, groups: int = 0,
+                   sink: Optional[torch.Tensor] = None, chunk: int = 0, gate: Optional[torch.Tensor] = None,
+                   tickets: Optional[torch.Tensor] = None) -> None:
+    """attention_decode (matrix cores) of the first ``n_seq`` sequences and attention_prefill_mfma of the 64-row blocks that the
+    work list names, in one launch (csrc/attention_step.hip); arguments as there."""
+    T, Hq, Hkv, D, page_size = _attention_common(out, q, k_cache, v_cache, q_start, ctx_len, block_table, "attention_step")
+    if not attention_step_fits(q.dtype, Hq, Hkv, D, page_size):
+        raise KernelError("attention_step: bfloat16, head size 64 or 128, at most 16 heads a kv head, a page size from 16 on "
+                          "that is a power of two")
+    if q.stride(0) % 8 or out.stride(0) % 4 or q.data_ptr() % 16 or out.data_ptr() % 8:
+        raise KernelError("attention_step: q rows must be 16-byte aligned, out rows 8-byte")
+    if not 0 < n_seq < ctx_len.numel() or q_start.numel() < ctx_len.numel() + 1 or block_table.shape[0] < ctx_len.numel():
+        raise KernelError("attention_step: the tables hold decoding sequences and others behind them")
+    if num_splits < 1:
+        raise KernelError("attention_step: num_splits must be >= 1")
+    _need_gpu(work_seq, work_qoff)
+    _i32(work_seq, "work_seq")
+    _i32(work_qoff, "work_qoff")
+    n_work = int(work_seq.numel())
+    if n_work == 0 or work_qoff.numel() != n_work:
+        raise KernelError("attention_step: inconsistent work list")
+    window, _, chunk, sink_p, gate_p, gate_stride, _ = _mask_extras("attention_step", T, Hq, window, 0, chunk, sink, gate, 0.0)
+    keys = block_table.shape[1] * page_size
+    if window:
+        keys = min(keys, window)
+    elif chunk:
+        keys = min(keys, chunk)
+    most = library.load("attention").ptl_attention_decode_mfma_parts(D, int(num_splits), ctypes.c_long(max(1, keys)), 0)
+    parts = None
+    if most > 1:
+        parts = torch.empty(n_seq * Hq * most * (D + 2), dtype=torch.float32, device=q.device)
+        tickets = _tickets(tickets, TICKET * n_seq * Hkv, q, "attention_step")
+    _check(library.load("attention_step").ptl_attention_step(
+        _ptr(out), ctypes.c_long(out.stride(0)), _ptr(q), ctypes.c_long(q.stride(0)), _ptr(k_cache), _ptr(v_cache),
+        _ptr(q_start), _ptr(ctx_len), _ptr(block_table), int(block_table.stride(0)), _ptr(work_seq), _ptr(work_qoff), n_work,
+        min(n_work, int(groups)) if groups > 0 else n_work, _ptr(parts), _ptr(tickets), int(most), int(n_seq), Hq, Hkv, D,
+        page_size, window, chunk, sink_p, gate_p, gate_stride, ctypes.c_float(scale), int(num_splits), _stream()),
+        "attention_step")
+
+
 def argmax(logits: torch.Tensor, host_out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """Greedy token per row of float32 logits [R, V]; ties go to the lowest id. ``host_out``:
     pinned int32 host memory (at least R long) that the kernel fills as well, over the bus;
@@ -1728,10 +1777,11 @@ def attention_prefill_mfma_kv(out: torch.Tensor, q: torch.Tensor, k_cache: torch
                               work_seq: torch.Tensor, work_qoff: torch.Tensor, scale: float, maps: int = 1,
                               groups: int = 1, window: int = 0, keep_first: int = 0,
                               sink: Optional[torch.Tensor] = None, chunk: int = 0,
-                              gate: Optional[torch.Tensor] = None, softcap: float = 0.0) -> None:
+                              gate: Optional[torch.Tensor] = None, softcap: float = 0.0, longest: int = 0) -> None:
     """The matrix-core kernel for prompt portions in its general form (csrc/attention_prefill.hip):
     shapes as for attention_generic_kv, bfloat16 q and caches, out bfloat16 or float32; the work
-    list names 64-row blocks, ``groups`` workgroups a head share it."""
+    list names 64-row blocks, ``groups`` workgroups a head share it. ``longest``: as for attention_prefill_mfma
+    (keys and values of one size, one map, bfloat16 out)."""
     _need_gpu(out, q, k_cache, v_cache, q_start, ctx_len, block_table, work_seq, work_qoff)
     if q.dim() != 3 or k_cache.dim() != 4 or v_cache.dim() != 4:
         raise KernelError("attention_prefill_mfma_kv: q [T, Hq, Dk], caches [pages, heads, page_size, size]")
@@ -1767,7 +1817,7 @@ def attention_prefill_mfma_kv(out: torch.Tensor, q: torch.Tensor, k_cache: torch
         _ptr(out), ctypes.c_long(out.stride(0)), int(out.dtype == torch.float32), _ptr(q),
         ctypes.c_long(q.stride(0)), _ptr(k_cache), _ptr(v_cache), _ptr(q_start), _ptr(ctx_len),
         _ptr(block_table), int(block_table.stride(0)), _ptr(work_seq), _ptr(work_qoff), n_work,
-        max(1, min(int(groups), n_work)), Hq, Hkv, int(maps), Dk, Dv, page_size, *extras,
+        max(1, min(int(groups), n_work)), int(longest), Hq, Hkv, int(maps), Dk, Dv, page_size, *extras,
         ctypes.c_float(scale), _stream()), "attention_prefill_mfma_kv")
 
 

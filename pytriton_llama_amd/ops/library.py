@@ -31,12 +31,12 @@ HIPCC_FLAGS = ["--offload-arch=" + ARCH, "-O3", "-fPIC", "-shared", "-std=c++17"
                "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
                "-mllvm", "-amdgpu-kernarg-preload-count=16"]
 
-KERNEL_LIBRARIES = ("embedding", "norm", "rope", "attention", "attention_prefill", "activation",
+KERNEL_LIBRARIES = ("embedding", "norm", "rope", "attention", "attention_prefill", "attention_step", "activation",
                     "gemm", "gemm_f32", "gemm_rows", "gemm_tile", "blaslt", "sampling", "probe", "stream", "latent", "moe", "prepare", "prompt",
                     "recurrent", "selective", "linear_scan")
-# options of single sources. attention_prefill: no value there is a NaN unless an input is, and
+# options of single sources. attention_prefill, attention_step: no value there is a NaN unless an input is, and
 # without the promise every maximum of scores is preceded by instructions that quiet its inputs
-EXTRA_FLAGS = {"attention_prefill": ["-fno-honor-nans"]}
+EXTRA_FLAGS = {"attention_prefill": ["-fno-honor-nans"], "attention_step": ["-fno-honor-nans"]}
 # libraries a source is linked with (after the source on the command line)
 LINK_FLAGS = {"blaslt": ["-lhipblaslt"]}
 

@@ -20,6 +20,7 @@ ALL_16 = WorkList(16)
 PORTIONS_16 = WorkList(16, after_decode=True)
 PORTIONS_64 = WorkList(64, after_decode=True)
 PORTIONS_128 = WorkList(128, after_decode=True)
+STEP_DECODES = 3, 8        # decoding requests from which portions beside them go into their launch, head sizes 64 and 128
 
 
 @register_part("mixer", "paged_attention")
@@ -62,7 +63,7 @@ class PagedAttention(Part):
         self.o_blocked: Optional[torch.Tensor] = None
         libs = ("attention", "rope", "prompt") + LINEAR_LIBRARIES    # (prompt: steps of prompts, any head size)
         if self.head_dim % 32 == 0 and self.head_dim <= 128:
-            libs += ("attention_prefill",)          # the matrix-core kernel for prompt portions
+            libs += ("attention_prefill", "attention_step")     # the matrix-core kernels for prompt portions
         if position is not None:
             libs += tuple(position.kernel_libraries)
         self.kernel_libraries = tuple(dict.fromkeys(libs))
@@ -194,6 +195,15 @@ class PagedAttention(Part):
             want = -(-4 * cus // base)
         return max(1, min(want, -(-span // turn), 64))
 
+    def _one_launch(self, n_dec: int, q, ctx, page_size: int) -> bool:
+        """Whether decoding requests and the portions beside them are one launch (csrc/attention_step.hip has the figures): some of
+        the former at least, and few blocks of the latter."""
+        if n_dec < STEP_DECODES[self.head_dim > 64] or n_dec == ctx.num_seqs or not ops.attention_step_fits(
+                q.dtype, self.num_heads, self.num_kv_heads, self.head_dim, page_size) or q.stride(0) % 8:
+            return False
+        blocks = ctx.work[PORTIONS_64][0].numel()
+        return 0 < blocks * self.num_heads <= ops.compute_units(q.device) * (2 if self.head_dim <= 64 else 1)
+
     def attend(self, out, q, cache, ctx, group, k=None, v=None) -> None:
         """``k`` / ``v``: the pools of keys and of values, [pages, Hkv, page_size, D] each, when
         they are not the cache layer's "k" and "v" (a mixer that keeps one tensor a token and
@@ -202,6 +212,11 @@ class PagedAttention(Part):
         v = cache.v if v is None else v
         D, window = self.head_dim, self.window or 0
         n_dec = ctx.num_decode_seqs if D % 16 == 0 and D <= 256 else 0      # (else: the vector kernel)
+        if n_dec and self._one_launch(n_dec, q, ctx, cache.page_size):
+            ops.attention_step(out, q, k, v, ctx.q_start, ctx.ctx_len, group.block_table, n_dec, *ctx.work[PORTIONS_64],
+                               self.scale, window, self.decode_splits(ctx, n_dec, True, q.device), sink=self.sink,
+                               tickets=getattr(ctx, "tickets", None))
+            return
         if n_dec:
             mfma = (ops.attention_decode_mfma_fits(q.dtype, self.num_heads, self.num_kv_heads, D,
                                                    cache.page_size)

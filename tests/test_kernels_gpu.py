@@ -1802,6 +1802,84 @@ def test_attention_prefill_mfma_short_portions_keep_one_side(ops, D):
         torch.testing.assert_close(run(2).float(), one.float(), atol=2e-2, rtol=2e-2)
 
 
+@pytest.mark.parametrize("D,Hkv,G,P", [(64, 8, 4, 16), (64, 1, 2, 64), (128, 2, 3, 16), (128, 8, 16, 32)])
+@pytest.mark.parametrize("masks", [dict(), dict(window=70), dict(chunk=96)], ids=["all", "window", "chunk"])
+@pytest.mark.parametrize("contexts", [[1], [40, 0, 700, 129, 0], [17, 1100, 0, 256, 33, 512, 90, 1, 300], [31 + 7 * i for i in range(65)]],
+                         ids=["one", "five", "listed", "many"])
+def test_attention_of_a_step_in_one_launch(ops, D, Hkv, G, P, masks, contexts):
+    """The bits of the decode kernel and of one group of waves for the portions (which portions of few rows always take), with
+    rows without keys, an empty work item, shared blocks, sinks and gates, twice over the same tickets, and in a replayed graph."""
+    torch.manual_seed(D + len(contexts))
+    n, q_lens, lens = len(contexts), [70, 200], [130, 460]
+    Hq, rows, seqs = Hkv * G, [1] * n + q_lens, contexts + lens
+    T, pages = sum(rows), [-(-k // P) for k in seqs]
+    order, at = torch.randperm(sum(pages) + 1).tolist(), 0
+    table = torch.full((len(seqs), max(pages)), -1, dtype=torch.int32)
+    for i, k in enumerate(pages):
+        table[i, :k] = torch.tensor(order[at:at + k], dtype=torch.int32)
+        at += k
+    k, v = (torch.randn(sum(pages) + 1, Hkv, P, D, device="cuda").to(torch.bfloat16) for _ in range(2))
+    q = torch.randn(T, Hq, D, device="cuda").to(torch.bfloat16)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")
+    start = i32([0] + torch.tensor(rows).cumsum(0).tolist())
+    from pytriton_llama_amd.engine.batch import work_items
+    ws, wo = (t.tolist() for t in work_items(rows, seqs, n, 64))
+    ws, wo = i32(ws + [n + 1]), i32(wo + [256])
+    extras = dict(masks, sink=torch.randn(Hq, device="cuda"), gate=torch.randn(T, Hq, device="cuda"))
+    tables = (start, i32(seqs), table.cuda())
+    tickets = torch.zeros(ops.TICKET * n * Hkv, dtype=torch.int32, device="cuda")
+    for splits, groups in ((1, 0), (3, 2)):
+        apart = torch.zeros_like(q)
+        ops.attention_decode(apart, q, k, v, *tables, n, D ** -0.5, num_splits=splits, matrix_cores=True, **extras)
+        ops.attention_prefill_mfma(apart, q, k, v, *tables, ws, wo, D ** -0.5, groups=groups, longest=1, **extras)
+
+        def step(out):
+            ops.attention_step(out, q, k, v, *tables, n, ws, wo, D ** -0.5, num_splits=splits, groups=groups, tickets=tickets,
+                               **extras)
+            return out
+        for _ in range(2):
+            assert torch.equal(step(torch.zeros_like(q)), apart)
+        assert not bool(tickets.any())
+        out, graph = torch.zeros_like(q), torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            step(out)
+        for _ in range(3):
+            out.fill_(float("nan"))
+            graph.replay()
+            assert torch.equal(out, apart)
+
+
+def test_attention_of_a_step_refuses(ops):
+    """What one of the two kernels does not take, and steps without one kind of rows."""
+    bf = lambda *s: torch.zeros(*s, dtype=torch.bfloat16, device="cuda")
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")
+
+    def call(D=64, Hq=2, P=16, dtype=torch.bfloat16, n_seq=1, work=1, rows=3):
+        q, kv = bf(rows, Hq, D).to(dtype), bf(2, 1, P, D).to(dtype)
+        ops.attention_step(torch.empty_like(q), q, kv, kv, i32([0, 1, rows]), i32([1, 2]), i32([[0], [1]]), n_seq, i32([1] * work),
+                           i32([0] * work), 0.1)
+    call()
+    for wrong in (dict(D=32), dict(D=96), dict(P=8), dict(P=24), dict(Hq=17), dict(dtype=torch.float32), dict(n_seq=0),
+                  dict(n_seq=2), dict(work=0)):
+        with pytest.raises(ops.KernelError, match="attention_step"):
+            call(**wrong)
+
+
+@pytest.mark.parametrize("D,n_dec,rows,one", [(64, 2, 70, False), (64, 3, 70, True), (128, 7, 70, False), (128, 8, 70, True),
+                                              (96, 8, 70, False), (64, 8, 64 * 257, False), (128, 8, 64 * 129, False)])
+def test_which_steps_take_one_launch(ops, D, n_dec, rows, one):
+    """Two heads on 256 compute units: up to two workgroups a unit at head size 64, one above; from three and eight decoding
+    requests on."""
+    from types import SimpleNamespace
+
+    from pytriton_llama_amd.parts import attention as part
+    if ops.compute_units(torch.device("cuda", 0)) != 256:
+        pytest.skip("the sizes are for 256 compute units")
+    ctx = SimpleNamespace(num_seqs=n_dec + 1, work={part.PORTIONS_64: (torch.zeros(-(-rows // 64)), None)})
+    q = torch.zeros(1, 2, D, dtype=torch.bfloat16, device="cuda")
+    assert part.PagedAttention(128, 2, 1, D)._one_launch(n_dec, q, ctx, 16) == one
+
+
 def test_attention_prefill_mfma_plan(ops):
     """128-row blocks once there are 1.25 t of them (t: workgroups a head can have resident);
     a workgroup a block up to 2 t blocks, t workgroups beyond; never more workgroups than blocks."""
