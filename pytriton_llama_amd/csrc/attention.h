@@ -59,6 +59,11 @@ __device__ __forceinline__ float tanh_exp2(float x2) {
 // Memory that another workgroup of the launch has written or will read.
 __device__ __forceinline__ void put_shared(float* p, float v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 __device__ __forceinline__ float get_shared(const float* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+// two of them, 8-byte aligned
+__device__ __forceinline__ float2 get_shared2(const float* p) {
+  return __builtin_bit_cast(float2, __hip_atomic_load(reinterpret_cast<const unsigned long long*>(p), __ATOMIC_RELAXED,
+                                                      __HIP_MEMORY_SCOPE_AGENT));
+}
 // Workgroups that share a (sequence, kv head) pair's keys count in a ticket who is done. Tickets lie 16 bytes apart: those of one
 // line are counted one after the other (one sequence, 8 pairs of 16 parts: 8.8 us side by side, 8.1 so and as 128 bytes apart).
 constexpr int TICKET = 4;

@@ -26,6 +26,7 @@
 #include "device.h"
 #include "mfma.h"
 #include "mfma_f32.h"
+#include <type_traits>
 
 #define AF_ROWS 16
 
@@ -212,23 +213,26 @@ attn_f32_kernel(float* __restrict__ out, long out_stride, const float* __restric
       mine[NK * 256 + 64 + lane] = l_run;
     }
     __syncthreads();
-    if (part > 0) return;
+    if (part > 0 && !(DECODE && n_parts > 1)) return;
+    if (part == 0) {
 #pragma unroll
-    for (int p = 1; p < KS; ++p) {
-      const float* other = lds + (size_t)(wave + p * HPW) * (NK * 256 + 128);
-      const float m_o = other[NK * 256 + lane], l_o = other[NK * 256 + 64 + lane];
-      const float m_new = fmaxf(m_run, m_o), m_safe = m_new == -INFINITY ? 0.f : m_new;
-      const float a = expf(m_run - m_safe), b = expf(m_o - m_safe);
-      l_run = l_run * a + l_o * b;
-      m_run = m_new;
+      for (int p = 1; p < KS; ++p) {
+        const float* other = lds + (size_t)(wave + p * HPW) * (NK * 256 + 128);
+        const float m_o = other[NK * 256 + lane], l_o = other[NK * 256 + 64 + lane];
+        const float m_new = fmaxf(m_run, m_o), m_safe = m_new == -INFINITY ? 0.f : m_new;
+        const float a = expf(m_run - m_safe), b = expf(m_o - m_safe);
+        l_run = l_run * a + l_o * b;
+        m_run = m_new;
 #pragma unroll
-      for (int t = 0; t < NK; ++t)
-        acc[t] = acc[t] * a + *reinterpret_cast<const f32x4_t*>(other + (t * 64 + lane) * 4) * b;
+        for (int t = 0; t < NK; ++t)
+          acc[t] = acc[t] * a + *reinterpret_cast<const f32x4_t*>(other + (t * 64 + lane) * 4) * b;
+      }
     }
   }
-  if (DECODE && n_parts > 1) {                   // (one wave is left)
+  if (DECODE && n_parts > 1) {
     const size_t place = ((size_t)seq * Hq + head) * sp.num_splits + blockIdx.z;
-    if (row_valid) {
+    int* done = reinterpret_cast<int*>(lds);     // (the first wave has left nothing there)
+    if (part == 0 && row_valid) {
       if (lg == 0) {
         put_shared(sp.part_ml + place * 2, m_run);
         put_shared(sp.part_ml + place * 2 + 1, l_run);
@@ -252,43 +256,49 @@ attn_f32_kernel(float* __restrict__ out, long out_stride, const float* __restric
       }
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // the part has reached memory
-    int last = 0;
-    if (lane == 0) last = last_part(sp.tickets + ((size_t)seq * Hkv + vh) * TICKET, n_parts);
-    if (!__builtin_amdgcn_readfirstlane(last)) return;
-    constexpr int AHEAD = 8;
-    for (int i = lane; i < G * Dv / 4; i += 64) {        // four columns a lane
-      const int h = 4 * i / Dv, d = 4 * i - h * Dv, hd = vh * G + h;
-      const size_t p = ((size_t)seq * Hq + hd) * sp.num_splits;
-      const float *pa = sp.part_acc + p * Dv + d, *ml = sp.part_ml + p * 2;
-      f32x4_t a = f32x4_t{0.f, 0.f, 0.f, 0.f};
-      float mn = ex.sink ? ex.sink[hd] : -INFINITY, den = ex.sink ? 1.f : 0.f;   // (the denominator's term without a key)
-      for (int s0 = 0; s0 < n_parts; s0 += AHEAD) {      // (they lie a long way off: eight of them are asked for at once)
-        f32x4_t av[AHEAD];
-        float mv[AHEAD], lv[AHEAD], m_new = mn;
+    if (tid == 0) *done = last_part(sp.tickets + ((size_t)seq * Hkv + vh) * TICKET, n_parts);
+    __syncthreads();
+    if (!*done) return;
+    // Four columns a thread. The parts lie a long way off: up to eight are asked for at once, in loads of eight bytes (32 rows of 16
+    // heads of 96 on one kv head, two parts each: one wave with loads of four bytes, eight parts always, cost a step of eight
+    // layers 50 us more than a second kernel).
+    auto merge = [&](auto at_once) __attribute__((always_inline)) {
+      constexpr int AHEAD = decltype(at_once)::value;
+      for (int i = tid; i < G * Dv / 4; i += 256) {
+        const int h = 4 * i / Dv, d = 4 * i - h * Dv, hd = vh * G + h;
+        const size_t p = ((size_t)seq * Hq + hd) * sp.num_splits;
+        const float *pa = sp.part_acc + p * Dv + d, *ml = sp.part_ml + p * 2;
+        f32x4_t a = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        float mn = ex.sink ? ex.sink[hd] : -INFINITY, den = ex.sink ? 1.f : 0.f;   // (the denominator's term without a key)
+        for (int s0 = 0; s0 < n_parts; s0 += AHEAD) {
+          float2 lo[AHEAD], hi[AHEAD], ends[AHEAD];
+          float m_new = mn;
 #pragma unroll
-        for (int s = 0; s < AHEAD; ++s) {
-          const int at = min(s0 + s, n_parts - 1);
-          const float* v = pa + (size_t)at * Dv;
-          mv[s] = get_shared(ml + 2 * at);
-          lv[s] = get_shared(ml + 2 * at + 1);
-          av[s] = f32x4_t{get_shared(v), get_shared(v + 1), get_shared(v + 2), get_shared(v + 3)};
+          for (int s = 0; s < AHEAD; ++s) {
+            const int at = min(s0 + s, n_parts - 1);
+            ends[s] = get_shared2(ml + 2 * at);
+            lo[s] = get_shared2(pa + (size_t)at * Dv);
+            hi[s] = get_shared2(pa + (size_t)at * Dv + 2);
+          }
+#pragma unroll
+          for (int s = 0; s < AHEAD; ++s) m_new = fmaxf(m_new, ends[s].x);
+          const float ms = m_new == -INFINITY ? 0.f : m_new, f0 = expf(mn - ms);
+          den *= f0;
+          a *= f0;
+#pragma unroll
+          for (int s = 0; s < AHEAD; ++s) {
+            const float f = s0 + s < n_parts ? expf(ends[s].x - ms) : 0.f;
+            den = fmaf(ends[s].y, f, den);
+            a += f32x4_t{lo[s].x, lo[s].y, hi[s].x, hi[s].y} * f;
+          }
+          mn = m_new;
         }
-#pragma unroll
-        for (int s = 0; s < AHEAD; ++s) m_new = fmaxf(m_new, mv[s]);
-        const float ms = m_new == -INFINITY ? 0.f : m_new, f0 = expf(mn - ms);
-        den *= f0;
-        a *= f0;
-#pragma unroll
-        for (int s = 0; s < AHEAD; ++s) {
-          const float f = s0 + s < n_parts ? expf(mv[s] - ms) : 0.f;
-          den = fmaf(lv[s], f, den);
-          a += av[s] * f;
-        }
-        mn = m_new;
+        const float inv = den > 0.f ? head_gate(ex, row, hd) / den : 0.f;
+        *reinterpret_cast<f32x4_t*>(out + (size_t)row * out_stride + (size_t)hd * Dv + d) = a * inv;
       }
-      const float inv = den > 0.f ? head_gate(ex, row, hd) / den : 0.f;
-      *reinterpret_cast<f32x4_t*>(out + (size_t)row * out_stride + (size_t)hd * Dv + d) = a * inv;
-    }
+    };
+    if (n_parts <= 2) merge(std::integral_constant<int, 2>{});
+    else merge(std::integral_constant<int, 8>{});
     return;
   }
   if (!row_valid) return;
