@@ -77,8 +77,11 @@ template <int N> __device__ __forceinline__ void wait_loads_but() {
 // DEPTH: chunks of W a wave has under way. MODE_PLAIN: wave w owns rows r0 + 16 w, y (or the
 // partial sums of this workgroup's slice of K) gets the product. MODE_SILU: waves 0, 1 own gate
 // rows r0 .. r0 + 31, waves 2, 3 the up rows r0 + I ..; out = act(gate) * up.
+// (WT 2: two waves a SIMD by order, for two workgroups a compute unit: with four tiles of x the compiler took 214 registers and
+// 48 accumulation registers, six more than that leaves room for. 64 rows of 128,256 x 2,048 / 3,072 / 4,096 144 / 220 / 292 -> 106 / 161 /
+// 219 us, fewer tiles level.)
 template <int MT, int KC, int DEPTH, int WT, int MODE, typename TY>
-__global__ void __launch_bounds__((4 / WT + 1) * 64)
+__global__ void __launch_bounds__((4 / WT + 1) * 64, WT == 2 && MT <= 4 ? 2 : 1)
 gemm_rows_kernel(TY* __restrict__ y, const bf16_t* __restrict__ x, const bf16_t* __restrict__ wb,
                  int M, int N_out, int w_rows, int K, long ldx, long ldy, int k_per_split,
                  int pair_offset, GluArgs act) {
