@@ -596,7 +596,7 @@ def _fused_x_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
 # 9.8 / 11.2 / 14.8 against 11.9 / 12.5 / 12.2; down projection + norm 15.8 / 17.2 / 21.7 against
 # 19.5 / 25.9 / 25.1; gate-up + SiLU-multiply 19.5 / 22.7 / 31.2 against 21.5 / 22.3 / 25.5; q|k|v +
 # rotation + cache write 10.0 / 13.7 / 18.5 against 13.7 / 14.1 / 17.1; the head of 128,256 columns
-# 101 / 112 / 206 against 131 / 137 / 150. Against the fused kernels for at most 16 rows, whole
+# 96 / 106 / 206 against 131 / 137 / 150. Against the fused kernels for at most 16 rows, whole
 # decode steps of 16 rows: 1.287 -> 1.243 ms at the 1B widths, 4.73 -> 4.58 ms at the 8B widths,
 # 3.04 -> 3.07 ms at the 3B widths (product by product the faster one depends on the shape): from
 # 9 rows on a step takes these kernels, where they fit.
