@@ -254,8 +254,8 @@ attn_decode_part(int block, Region region, const int32_t* __restrict__ ctx_len, 
       ll = ll * f + __builtin_amdgcn_exp2f(sk - mx);
       a *= f;
     }
-    out[(size_t)row * out_stride + (size_t)head * D + d] =
-        float_to_bf16(ll > 0.f ? a / ll * head_gate(ex, row, head) : 0.f);
+    // (by the inverse: where a score is a NaN or an infinity, a and ll are NaNs, and so is the result)
+    out[(size_t)row * out_stride + (size_t)head * D + d] = float_to_bf16(a * (ll > 0.f ? head_gate(ex, row, head) / ll : 0.f));
   };
 
   // merge the waves: [head][D] accumulators and [head][2] (max, denominator) take the place of

@@ -1,5 +1,5 @@
 // Prompt portions over the paged cache on the matrix cores: what a workgroup does, for the kernels of attention_prefill.hip and
-// attention_step.hip. Compiled with -fno-honor-nans (max2).
+// attention_step.hip.
 #pragma once
 #include "attention.h"
 #include "common.h"
@@ -8,12 +8,10 @@
 
 #define PF_BN 64
 
-
-// (This file is compiled with -fno-honor-nans: fmaxf then is one v_max, or half a v_max3,
-// without a quieting v_max(x, x) in front of every score that comes out of an MFMA. No inline
-// assembly for it: the compiler inserts the wait states between an MFMA and the first read of
-// its result only for instructions it knows.)
-__device__ __forceinline__ float max2(float a, float b) { return fmaxf(a, b); }
+// The maximum that is a NaN where an operand is: half a v_maximum3. fmaxf, which has to drop NaNs, is preceded by
+// a quieting v_max(x, x) for every score that comes out of an MFMA. (No inline assembly for it: the compiler
+// inserts the wait states between an MFMA and the first read of its result only for instructions it knows.)
+__device__ __forceinline__ float max2(float a, float b) { return __builtin_elementwise_maximum(a, b); }
 __device__ __forceinline__ s16x4_t lds_read_tr16(const bf16_t* p) {
   return __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4_t*)p);
 }

@@ -1,7 +1,6 @@
 // Attention of prompt portions over the paged cache on the matrix cores (bfloat16).
 // The cache layout, the meaning of the arguments and the reference formulas are those of
-// attention.hip; this kernel has a source file of its own because it is compiled with one more
-// option (see max2 below).
+// attention.hip.
 #include "attention_prefill.h"
 #include "common.h"
 #include "device.h"

@@ -34,9 +34,6 @@ HIPCC_FLAGS = ["--offload-arch=" + ARCH, "-O3", "-fPIC", "-shared", "-std=c++17"
 KERNEL_LIBRARIES = ("embedding", "norm", "rope", "attention", "attention_prefill", "attention_step", "activation",
                     "gemm", "gemm_f32", "gemm_rows", "gemm_tile", "blaslt", "sampling", "probe", "stream", "latent", "moe", "prepare", "prompt",
                     "recurrent", "selective", "linear_scan")
-# options of single sources. attention_prefill, attention_step: no value there is a NaN unless an input is, and
-# without the promise every maximum of scores is preceded by instructions that quiet its inputs
-EXTRA_FLAGS = {"attention_prefill": ["-fno-honor-nans"], "attention_step": ["-fno-honor-nans"]}
 # libraries a source is linked with (after the source on the command line)
 LINK_FLAGS = {"blaslt": ["-lhipblaslt"]}
 
@@ -96,7 +93,7 @@ def _headers() -> List[str]:
 def _options(name: str) -> str:
     """What the file beside a library says of how it was compiled: the options, without the compiler's and the sources' places
     (a checkout may be built in one and used in another)."""
-    return " ".join(HIPCC_FLAGS + EXTRA_FLAGS.get(name, []) + LINK_FLAGS.get(name, [])) + "\n"
+    return " ".join(HIPCC_FLAGS + LINK_FLAGS.get(name, [])) + "\n"
 
 
 def _options_path(lib: str) -> str:
@@ -118,7 +115,7 @@ def is_stale(name: str) -> bool:
 
 
 def compile_command(name: str, out: str) -> List[str]:
-    return ([_hipcc()] + HIPCC_FLAGS + EXTRA_FLAGS.get(name, []) +
+    return ([_hipcc()] + HIPCC_FLAGS +
             ["-I", CSRC_DIR, "-o", out, source_path(name)] + LINK_FLAGS.get(name, []))
 
 

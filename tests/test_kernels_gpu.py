@@ -1849,6 +1849,47 @@ def test_attention_of_a_step_in_one_launch(ops, D, Hkv, G, P, masks, contexts):
             assert torch.equal(out, apart)
 
 
+@pytest.mark.parametrize("D,Hkv,G", [(64, 2, 4), (128, 3, 2)])
+@pytest.mark.parametrize("where,value", [("key", math.nan), ("key", math.inf), ("value", math.nan), ("query", math.nan)])
+def test_attention_gives_nans_for_scores_that_are_no_numbers(ops, D, Hkv, G, where, value):
+    """Decode attention with one part a sequence and with several, and both kinds of rows in one launch: NaNs where the plain
+    attention has them, the other heads' and sequences' numbers as it has them, zeros for a row without keys."""
+    torch.manual_seed(D)
+    P, Hq, contexts, rows = 16, Hkv * G, [300, 0, 5, 700], [1, 1, 1, 1, 40]
+    lens, n = contexts + [90], 4
+    pages = [-(-c // P) for c in lens]
+    table, at = torch.full((5, max(pages)), -1, dtype=torch.int32), 0
+    for i, k in enumerate(pages):
+        table[i, :k] = torch.arange(at, at + k)
+        at += k
+    k, v = (torch.randn(at, Hkv, P, D).to(torch.bfloat16) for _ in range(2))
+    q = torch.randn(sum(rows), Hq, D).abs().to(torch.bfloat16)          # (an infinite key then is an infinite score)
+    for seq, key in ((0, 10), (3, 650), (4, 20)):
+        page, off = int(table[seq, key // P]), key % P
+        if where == "query":
+            q[seq, 1, 3] = value
+        else:
+            (k if where == "key" else v)[page, 0, off, 3] = value
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")
+    starts = [0, 1, 2, 3, 4, 44]
+    want = torch.zeros(44, Hq, D, dtype=torch.float64)
+    for seq, c in enumerate(lens):
+        keys, values = (t[table[seq, :pages[seq]].long()].transpose(1, 2).reshape(-1, Hkv, D)[:c] for t in (k, v))
+        for i in range(rows[seq] if c else 0):
+            pos = c - rows[seq] + i
+            want[starts[seq] + i] = _masked_attention(q[starts[seq] + i], keys[:pos + 1], values[:pos + 1], pos, D ** -0.5)
+    assert 0 < int(want[:4].isnan().sum()) < want[:4].numel() // 2
+    tables, dev = (i32(starts), i32(lens), table.cuda()), (q.cuda(), k.cuda(), v.cuda())
+    for splits, piece in ((1, 1 << 20), (1, 128), (4, 0)):
+        out = torch.full((44, Hq, D), 9.0, dtype=torch.bfloat16, device="cuda")
+        ops.attention_decode(out, *dev, *tables, n, D ** -0.5, num_splits=splits, matrix_cores=True, piece=piece)
+        torch.testing.assert_close(out[:n].double().cpu(), want[:n], equal_nan=True, **tol(torch.bfloat16))
+    for splits in (1, 4):
+        out = torch.full((44, Hq, D), 9.0, dtype=torch.bfloat16, device="cuda")
+        ops.attention_step(out, *dev, *tables, n, i32([4]), i32([0]), D ** -0.5, num_splits=splits)
+        torch.testing.assert_close(out.double().cpu(), want, equal_nan=True, **tol(torch.bfloat16))
+
+
 def test_attention_of_a_step_refuses(ops):
     """What one of the two kernels does not take, and steps without one kind of rows."""
     bf = lambda *s: torch.zeros(*s, dtype=torch.bfloat16, device="cuda")
