@@ -222,8 +222,9 @@ gemm_tile_kernel(const TileArgs a) {
           if (pair >= N) continue;
           const int kv = head - a.qkv.Hq, v = kv >= a.qkv.Hkv;
           if (kv >= 0 && slot < 0) continue;
+          const bool turned = !v && a.qkv.table;
           f32x4_t c01 = f32x4_t{1.f, 0.f, 1.f, 0.f}, c23 = c01;    // cosine, sine of two pairs
-          if (!v && a.qkv.table) {
+          if (turned) {
             const f32x4_t* cs = reinterpret_cast<const f32x4_t*>(a.qkv.table + (size_t)m * half + at);
             c01 = cs[0];
             c23 = cs[1];
@@ -233,8 +234,9 @@ gemm_tile_kernel(const TileArgs a) {
           for (int k = 0; k < 4; ++k) {
             const float c = k < 2 ? c01[2 * k] : c23[2 * k - 4], s = k < 2 ? c01[2 * k + 1] : c23[2 * k - 3];
             const float x1 = rounded(acc[j][i][k]), x2 = rounded(acc[j + TN / 2][i][k]);
-            lo.e[k] = to_bf16(x1 * c - x2 * s);
-            hi.e[k] = to_bf16(x2 * c + x1 * s);
+            // (a copy where nothing is turned: times 1 less times 0 is a NaN beside an infinity)
+            lo.e[k] = to_bf16(turned ? x1 * c - x2 * s : x1);
+            hi.e[k] = to_bf16(turned ? x2 * c + x1 * s : x2);
           }
           bf16_t* to = kv < 0 ? reinterpret_cast<bf16_t*>(a.y) + (size_t)m * a.qkv.ldq + (size_t)head * a.qkv.D
                               : (v ? a.qkv.v_cache : a.qkv.k_cache) +

@@ -1405,6 +1405,30 @@ def test_qkv_rope_store_tile(ops, tile, Hq, Hkv, D):
         assert torch.equal(none, q)
 
 
+@pytest.mark.parametrize("value", [math.inf, -math.inf, math.nan])
+@pytest.mark.parametrize("turned", [False, True])
+@pytest.mark.parametrize("M", [37, 150])
+def test_qkv_rope_store_tile_copies_what_is_not_turned(ops, value, turned, M):
+    """An infinity or a NaN in one column of a value (and, without a rotation, of q and k) stays in that column: the other of the
+    pair keeps its number, as a stored product does."""
+    P, pages, K, Hq, Hkv, D = 8, 40, 192, 3, 2, 64
+    torch.manual_seed(M)
+    x = torch.randn(M, K, device="cuda").to(torch.bfloat16)
+    w = (torch.randn((Hq + 2 * Hkv) * D, K, device="cuda") * K ** -0.5).to(torch.bfloat16)
+    for head, col in ((Hq + Hkv, 5), (Hq + 2 * Hkv - 1, 40)) + (() if turned else ((1, 40), (Hq, 5), (Hq + 1, 63))):
+        w[head * D + col, 7] = value
+    pos = torch.arange(M, device="cuda").int()
+    inv = (500000.0 ** (-torch.arange(0, D, 2, device="cuda").double() / D)).float()
+    slots = torch.randperm(P * pages, device="cuda")[:M].int()
+    caches = [torch.zeros(pages, Hkv, P, D, dtype=torch.bfloat16, device="cuda") for _ in range(4)]
+    q = ops.qkv_rope_store_tile(x, w, ops.rope_table(pos, inv) if turned else None, slots, *caches[:2], Hq, Hkv, D, P)
+    parts = [t.view(M, -1, D) for t in (x.float() @ w.float().T).to(torch.bfloat16).split([Hq * D, Hkv * D, Hkv * D], 1)]
+    ops.rope_store(*parts, pos, inv if turned else None, slots, *caches[2:], P)
+    for got, want in ((q, parts[0]), (caches[0], caches[2]), (caches[1], caches[3])):
+        torch.testing.assert_close(got.float(), want.float(), equal_nan=True, **tol(torch.bfloat16))
+    assert int((~torch.isfinite(caches[1].float())).sum()) == 2 * M
+
+
 @pytest.mark.parametrize("n", [12, 80])
 def test_attention_decode_mfma_shares_beside_empty_rows(ops, n):
     """Rows without keys (padding of a recorded step) between sequences of very different lengths: zeros
