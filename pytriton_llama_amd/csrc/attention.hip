@@ -555,7 +555,8 @@ static int launch_decode(void* out, long out_stride, const void* q, long q_strid
 // page_size, Dv], out [T, Hq, Dv] of the caches' type or (out_f32) float32.
 // part_acc [n_seq, Hq, num_splits, Dv] and part_ml [n_seq, Hq, num_splits, 2] are
 // float32 workspaces of the caller (unused when num_splits == 1), and so are, for float32 caches, TICKET * n_seq * Hkv tickets: zeros,
-// which they are again after the launch.
+// which they are again after the launch. (Without tickets, or with workspaces that are not 8-byte aligned, which is how the matrix-core
+// form reads the parts, the general one takes float32 as well.)
 extern "C" int ptl_attention_decode_kv(void* out, long out_stride, int out_f32, const void* q,
                                        long q_stride, const void* k_cache, const void* v_cache,
                                        const int32_t* q_start, const int32_t* ctx_len,
@@ -571,12 +572,12 @@ extern "C" int ptl_attention_decode_kv(void* out, long out_stride, int out_f32, 
       num_splits > 1024 || (num_splits > 1 && (!part_acc || !part_ml)) || !extras_ok(ex))
     return PTL_ERR_ARG;
   if (dtype == PTL_DTYPE_F32 && attn_f32_decodes(Hq, Hkv, maps, Dk, Dv) &&
-      attn_f32_fits(out, out_stride, q, q_stride, k_cache, v_cache, Dk, Dv) && (num_splits == 1 || tickets)) {
+      attn_f32_fits(out, out_stride, q, q_stride, k_cache, v_cache, Dk, Dv) &&
+      (num_splits == 1 || (tickets && ((uintptr_t)part_acc | (uintptr_t)part_ml) % 8 == 0)))
     return attention_f32_decode((float*)out, out_stride, (const float*)q, q_stride, (const float*)k_cache,
-                                        (const float*)v_cache, q_start, ctx_len, block_table, bt_stride,
-                                        SplitArgs{part_acc, part_ml, tickets, num_splits}, n_seq, Hq, Hkv, Dk, Dv, page_size,
-                                        ex, scale, stream);
-  }
+                                (const float*)v_cache, q_start, ctx_len, block_table, bt_stride,
+                                SplitArgs{part_acc, part_ml, tickets, num_splits}, n_seq, Hq, Hkv, Dk, Dv, page_size, ex,
+                                scale, stream);
   const int chunks = (Dk > Dv ? Dk : Dv) / 16;
   int lpk = 1;
   while (lpk < chunks) lpk <<= 1;

@@ -101,3 +101,17 @@ def test_small_f32_products_have_no_kernel_that_splits_x(tmp_path, M, N, K, part
     wants = took[0]["code"] != 0
     assert wants == (parts or any("gemm_f32_sum_kernel" in k for k in kernels))
     assert took[2] == ({"code": -1, "launches": []} if wants else took[1])
+
+
+@pytest.mark.parametrize("splits,acc,ml,tickets,matrix_cores", [(4, 0, 0, 1, True), (4, 8, 8, 1, True), (4, 4, 0, 1, False),
+                                                                (4, 0, 4, 1, False), (4, 0, 0, 0, False), (1, 4, 4, 0, True)])
+def test_float32_decode_attention_by_its_workspaces(tmp_path, splits, acc, ml, tickets, matrix_cores):
+    """The last workgroup of a sequence reads the parts eight bytes at a time: workspaces that do not lie so, like a call
+    without tickets, go to the general kernel and its merge."""
+    at = lambda off: ("p", (1 << 20) + off)
+    took = run(tmp_path, "attention", [(0, "ptl_attention_decode", [
+        P, ("l", 512), P, ("l", 512), P, P, P, P, P, *i(64), at(acc), at(ml), P if tickets else NO, *i(3, 8, 2, 64, 16), *EXTRAS,
+        *i(splits, 0), NO])])[0]
+    names = [k["kernel"] for k in took["launches"]]
+    assert took["code"] == 0 and any("attn_f32_kernel" in n for n in names) == matrix_cores
+    assert [any(part in n for n in names) for part in ("attn_decode_kernel", "attn_decode_merge_kernel")] == [not matrix_cores] * 2
