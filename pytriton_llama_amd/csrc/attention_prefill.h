@@ -190,8 +190,11 @@ attn_prefill_blocks(bf16_t* const Ks0, bf16_t* const Ks1, bf16_t* const Vs0, bf1
     const int k0 = k_begin + t * PF_BN;
     return t < n_tiles && k0 >= k_lo && k0 + PF_BN <= k_end;
   };
-  auto page_at = [&](int row) {                 // of a row that is the same in all lanes
-    const int kp = __builtin_amdgcn_readfirstlane(min(max(row, k_lo), k_end - 1)) >> page_shift;
+  // of a row that is the same in all lanes; a row that is no key gets the page of one that is (the table's first, for
+  // a portion without any)
+  const int last_key = max(k_end - 1, 0);
+  auto page_at = [&](int row) {
+    const int kp = __builtin_amdgcn_readfirstlane(min(max(row, k_lo), last_key)) >> page_shift;
     return *(const __attribute__((address_space(4))) int32_t*)(uintptr_t)(bt + kp);
   };
   auto load_pages = [&](int t) {

@@ -1670,6 +1670,27 @@ def test_attention_prefill_mfma_page_numbers_of_a_wave(ops, D, masks, rows):
     assert all(torch.equal(o, outs[0]) for o in outs[1:])
 
 
+@pytest.mark.parametrize("D", [32, 64, 128])
+@pytest.mark.parametrize("rows", [64, 128])
+def test_attention_prefill_mfma_portion_without_keys(ops, D, rows):
+    """A portion whose context says that there are no keys: zeros, and nothing is read in front of the table; the one beside it as
+    by itself. Pages whose numbers are read once for a load instruction's rows and pages whose numbers every lane reads."""
+    torch.manual_seed(D)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")
+    q = torch.randn(45, 4, D, device="cuda").to(torch.bfloat16)
+    for P in (8, 16):
+        k, v = (torch.randn(5 * 16 // P, 2, P, D, device="cuda").to(torch.bfloat16) for _ in range(2))
+        table = torch.full((2, 80 // P), -1, dtype=torch.int32)
+        table[1] = torch.arange(80 // P)
+        outs = []
+        for ctx, work in ((0, [0, 1]), (0, [1])):
+            out = torch.full((45, 4, D), 9.0, dtype=torch.bfloat16, device="cuda")
+            ops.attention_prefill_mfma(out, q, k, v, i32([0, 5, 45]), i32([ctx, 75]), table.cuda(), i32(work), i32([0] * len(work)),
+                                       D ** -0.5, block_rows=rows)
+            outs.append(out)
+        assert bool((outs[0][:5] == 0).all()) and torch.equal(outs[0][5:], outs[1][5:])
+
+
 def test_attention_prefill_mfma_refuses_odd_page_size(ops):
     """A page size that is no power of two is for the general kernel; the fast one says so."""
     assert not ops.attention_prefill_mfma_fits(torch.bfloat16, 1, 32, 5)
