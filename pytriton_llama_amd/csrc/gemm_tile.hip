@@ -65,7 +65,7 @@ __device__ __forceinline__ float pair_value(const GluArgs& a, float g, float u) 
 
 // Where q | k | v go (ptl_tile_qkv_rope_store).
 struct QkvArgs {
-  const float2* table;       // [M][D / 2] cosines and sines, or null
+  const float2* const* turns;      // where it says where the cosines and sines [M][D / 2] lie, or null
   const int32_t* slots;
   bf16_t *k_cache, *v_cache;
   int Hq, Hkv, D, page_size;
@@ -125,6 +125,7 @@ gemm_tile_kernel(const TileArgs a) {
   const int first_tile = xcd * run + min(xcd, rest) + (blockIdx.x >> 3);
   const int my_tiles = (total - first_tile + G - 1) / G;     // (the grid has no more workgroups than there are tiles)
   const int k_per_split = K / a.splits, chunks = k_per_split / KC;
+  const float2* const table = MODE == OUT_QKV && a.qkv.turns ? *a.qkv.turns : nullptr;
 
   if (wave >= WAVES) {
     tile_bring<BM + BN, NB, PW>(lds, wave - WAVES, lane, my_tiles, chunks, [&](int i, int r) {
@@ -222,10 +223,10 @@ gemm_tile_kernel(const TileArgs a) {
           if (pair >= N) continue;
           const int kv = head - a.qkv.Hq, v = kv >= a.qkv.Hkv;
           if (kv >= 0 && slot < 0) continue;
-          const bool turned = !v && a.qkv.table;
+          const bool turned = !v && table;
           f32x4_t c01 = f32x4_t{1.f, 0.f, 1.f, 0.f}, c23 = c01;    // cosine, sine of two pairs
           if (turned) {
-            const f32x4_t* cs = reinterpret_cast<const f32x4_t*>(a.qkv.table + (size_t)m * half + at);
+            const f32x4_t* cs = reinterpret_cast<const f32x4_t*>(table + (size_t)m * half + at);
             c01 = cs[0];
             c23 = cs[1];
           }
@@ -390,20 +391,20 @@ extern "C" int ptl_tile_gate_up(void* out, const void* x, const void* w, int M, 
                           limit, stream);
 }
 
-// q, k, v = x W^T (rows of W: q | k | v, heads of D), q and k rotated by ``table`` ([M][D / 2] cosines and sines as pairs of
-// floats, null: not at all): q [M, ldq], k and v into pages [pages, Hkv, page_size, D] at slots[m] = page * page_size + offset (below 0,
+// q, k, v = x W^T (rows of W: q | k | v, heads of D), q and k rotated by a table of cosines and sines (pairs of floats [M][D / 2],
+// 16-byte aligned; ``turns``: the place in device memory that holds its address, null: not at all): q [M, ldq], k and v into pages [pages, Hkv, page_size, D] at slots[m] = page * page_size + offset (below 0,
 // or slots null: nowhere). The products are rounded to bfloat16 before the rotation, as stored ones are (rope.hip). K a multiple of
 // 64, D of 32, 16-byte aligned rows, tables and pages. tile: -1: the plan's, else one of the caller's, for tests (two more than ptl_tile_shapes()).
-extern "C" int ptl_tile_qkv_rope_store(void* q, long ldq, const void* x, const void* w, int M, int K, long ldx, const void* table,
+extern "C" int ptl_tile_qkv_rope_store(void* q, long ldq, const void* x, const void* w, int M, int K, long ldx, const void* turns,
                                        const int32_t* slots, void* k_cache, void* v_cache, int Hq, int Hkv, int D,
                                        int page_size, int tile, hipStream_t stream) {
   if (Hq <= 0 || Hkv <= 0 || D <= 0 || D % 32 || page_size <= 0 || (long)(Hq + 2 * Hkv) * D > 0x3fffffff) return PTL_ERR_ARG;
   const int rows_w = (Hq + 2 * Hkv) * D;
-  if (bad(q, x, w, M, rows_w / 2, K, ldx) || ldq % 8 || ldq < (long)Hq * D || !aligned(table) || !aligned(k_cache) ||
+  if (bad(q, x, w, M, rows_w / 2, K, ldx) || ldq % 8 || ldq < (long)Hq * D || (uintptr_t)turns % 8 || !aligned(k_cache) ||
       !aligned(v_cache) || (slots && (!k_cache || !v_cache)) || tile < -1 || tile >= N_SHAPES + 2)
     return PTL_ERR_ARG;
   const TileArgs a{q, (const bf16_t*)x, (const bf16_t*)w, M, rows_w / 2, K, ldx, 1, 0, 0, GluArgs{},
-                   QkvArgs{(const float2*)table, slots, (bf16_t*)k_cache, (bf16_t*)v_cache, Hq, Hkv, D, page_size, ldq}};
+                   QkvArgs{(const float2* const*)turns, slots, (bf16_t*)k_cache, (bf16_t*)v_cache, Hq, Hkv, D, page_size, ldq}};
   // Few rows of a narrow W: the smallest tiles as long as each finds a compute unit of its own. 3,072 x 2,048 at 48 / 64 / 96 / 128
   // rows 9.6 / 9.6 / 10.3 / 10.6 us (tiles of 64 x 64 12.5 / 13.3 / 11.8 / 13.2), 5,120 x 3,072 at 48 / 64 13.8 / 14.5 (16.3 /
   // 17.4), 6,144 x 4,096 17.3 / 18.1 (20.7 / 22.1); beyond one tile a unit 5,120 x 3,072 at 80 rows 18.3 (15.0).

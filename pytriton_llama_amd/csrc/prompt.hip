@@ -41,7 +41,7 @@ struct PtlPromptLayer {
   const float *inv_freq, *post_norm, *next_norm; // next_norm: of the layer behind this one
   void *k_cache, *v_cache;
   float post_eps, next_eps;
-  const void* turns;                             // cosines and sines of the step's rows (qkv_tile)
+  const void* turns;                             // where it says where the cosines and sines of the step's rows lie (qkv_tile)
 };
 
 static_assert(sizeof(PtlPromptStep) == 128 && sizeof(PtlPromptLayer) == 88, "as ops/prompt.py lays them out");

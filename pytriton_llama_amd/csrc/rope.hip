@@ -121,22 +121,44 @@ extern "C" int ptl_rope_store(void* q, void* k, const void* v, long row_stride,
   return ptl_launch_status();
 }
 
-// table [T][half]: cosine and sine of positions[t] * inv_freq[j], as rope_store_kernel has them: for products that
-// rotate what they give themselves, once for all layers of a step.
-__global__ void rope_table_kernel(float2* __restrict__ table, const int32_t* __restrict__ positions,
-                                  const float* __restrict__ inv_freq, int total, int half) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= total) return;
+// tables [n][T][half]: cosine and sine of positions[t] * inv_freq[j], as rope_store_kernel has them, for n arrays of
+// frequencies: for products that rotate what they give themselves, all layers of a step by one launch. An array that holds the
+// same bits as the first has its table: at[i] says where the table of array i lies. (One launch a layer is 2 us each. Tables of
+// their own for layers with equal frequencies come from memory instead of L2: the products of 277 rows 10.9 -> 11.1 us.)
+constexpr int ROPE_TABLES = 64;
+struct RopeFrequencies { const float* of[ROPE_TABLES]; };
+
+__global__ void __launch_bounds__(256)
+rope_tables_kernel(float2* __restrict__ tables, const float2** __restrict__ at, const int32_t* __restrict__ positions, int total,
+                   int half, RopeFrequencies inv_freq) {
+  const int y = blockIdx.y, i = blockIdx.x * 256 + threadIdx.x;
+  const float *own = inv_freq.of[y], *first = inv_freq.of[0];
+  bool same = true;
+  for (int j = threadIdx.x; j < half; j += 256) same &= __float_as_uint(own[j]) == __float_as_uint(first[j]);
+  same = __syncthreads_and(same) && y > 0;
+  float2* table = tables + (same ? 0 : (size_t)y * total);
+  if (i == 0) at[y] = table;
+  if (same || i >= total) return;
   const int t = i / half;
   float s, c;
-  sincosf((float)positions[t] * inv_freq[i - t * half], &s, &c);
+  sincosf((float)positions[t] * own[i - t * half], &s, &c);
   table[i] = make_float2(c, s);
 }
 
-extern "C" int ptl_rope_table(void* table, const int32_t* positions, const float* inv_freq, int T, int half,
-                              hipStream_t stream) {
-  if (T <= 0) return PTL_OK;
-  if (half <= 0 || (long)T * half > 0x3fffffff || !table || !positions || !inv_freq || (uintptr_t)table % 8) return PTL_ERR_ARG;
-  rope_table_kernel<<<(T * half + 255) / 256, 256, 0, stream>>>((float2*)table, positions, inv_freq, T * half, half);
+// at: n pointers in device memory, written by the launch. inv_freq: n (up to ROPE_TABLES) pointers in host memory, read before
+// the call returns.
+extern "C" int ptl_rope_tables(void* tables, void* at, const int32_t* positions, const float* const* inv_freq, int n, int T,
+                               int half, hipStream_t stream) {
+  if (n <= 0 || T <= 0) return PTL_OK;
+  if (n > ROPE_TABLES || half <= 0 || (long)T * half > 0x3fffffff || !tables || !at || !positions || !inv_freq ||
+      ((uintptr_t)tables | (uintptr_t)at) % 8)
+    return PTL_ERR_ARG;
+  RopeFrequencies all{};
+  for (int i = 0; i < n; ++i) {
+    if (!inv_freq[i]) return PTL_ERR_ARG;
+    all.of[i] = inv_freq[i];
+  }
+  rope_tables_kernel<<<dim3((T * half + 255) / 256, n), 256, 0, stream>>>((float2*)tables, (const float2**)at, positions, T * half,
+                                                                         half, all);
   return ptl_launch_status();
 }

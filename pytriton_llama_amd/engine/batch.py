@@ -25,6 +25,7 @@ import torch
 
 from .. import ops
 from ..parts.base import WorkList
+from ..parts.rotary import Rotations
 
 
 def work_items(q_lens, ctx_lens, first_seq: int, block_rows: int):
@@ -82,8 +83,7 @@ class StepContext:
     max_ctx_len: int = 0
     tickets: Optional[torch.Tensor] = None     # int32 zeros, ops.TICKET a single-token sequence and kv head: the workgroups of
                                                # a launch that share a sequence's keys count in them who is done, and leave zeros
-    rotations: Optional[Dict[bytes, torch.Tensor]] = None      # while a model's forward runs: the cosines and sines of the rows,
-                                               # by the bytes of the frequencies (parts.rotary)
+    rotations: Optional[Rotations] = None      # while a model's forward runs: the cosines and sines of the rows
 
 
 def order_entries(entries: Sequence[StepEntry]) -> List[int]:

@@ -10,6 +10,7 @@ import torch
 
 from .. import ops
 from ..parts.base import ParamSource, Part, as_tensor, run_norm, says
+from ..parts.rotary import Rotations
 from . import prompt_steps
 
 
@@ -134,7 +135,8 @@ class CausalLM:
     # ---- the forward pass of one step ------------------------------------------
     def forward(self, ctx, storage) -> torch.Tensor:
         """Float32 logits [len(ctx.logit_rows), vocab] for the flat batch ``ctx``."""
-        ctx.rotations = {}                  # (a recorded step's context is there for several passes, its positions change)
+        # (of this pass only: a recorded step's context is there for several, and its positions change)
+        ctx.rotations = Rotations(self.blocks)
         try:
             return self._forward(ctx, storage)
         finally:

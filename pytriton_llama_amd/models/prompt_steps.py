@@ -21,7 +21,7 @@ from ..parts.base import PendingProduct
 from ..parts.block import PreNormBlock
 from ..parts.feedforward import SwiGLU
 from ..parts.norm import RMSNorm
-from ..parts.rotary import RotaryEncoding
+from ..parts.rotary import RotaryEncoding, Rotations
 
 
 # Up to 64 rows some products go to kernels that read the decode copies of the weights.
@@ -97,7 +97,8 @@ def run(model, h: torch.Tensor, ctx, storage) -> Optional[Tuple[PendingProduct, 
     down_splits = ops.gemm_tile_splits(T, H, I) if ops.gemm_tile_add_rmsnorm_fits(a, ffn.down, residual, norm) else 0
     tile = ops.gate_up_tile_fits(y, ffn.gate_up)
     qkv_tile = (ops.qkv_rope_store_tile_fits(y, mixer.qkv, D) and all(t.data_ptr() % 16 == 0 for c in caches for t in (c.k, c.v)))
-    tables = [m.position.table(ctx) for m in (b.mixer for b in blocks)] if qkv_tile else [None] * len(blocks)
+    rotations = getattr(ctx, "rotations", None) or Rotations(blocks)
+    tables = [rotations.table(b.mixer.position, ctx.positions) for b in blocks] if qkv_tile else [None] * len(blocks)
     # q | k | v, a product (or its float32 sums) and gate | up, one after the other in one place: each has been read when
     # the next is written, so a long step takes no more memory than by the parts, which hold the activation of the block
     # before where ``mixed`` is held here
@@ -116,7 +117,7 @@ def run(model, h: torch.Tensor, ctx, storage) -> Optional[Tuple[PendingProduct, 
         layer = prompt.PromptLayer(
             m.qkv.data_ptr(), m.o.data_ptr(), f.gate_up.data_ptr(), f.down.data_ptr(), m.position.inv_freq.data_ptr(),
             b.post_norm.weight.data_ptr(), behind.weight.data_ptr(), cache.k.data_ptr(), cache.v.data_ptr(),
-            b.post_norm.eps, behind.eps, turns.data_ptr() if turns is not None else 0)
+            b.post_norm.eps, behind.eps, turns.of.address(turns.index) if turns is not None else 0)
         prompt.prompt_between(table, step, before, layer)
         m.attend(out, q, cache, ctx, ctx.groups[cache.group])
         before = layer

@@ -11,7 +11,7 @@ import contextlib
 import ctypes
 import functools
 import itertools
-from typing import Optional
+from typing import NamedTuple, Optional, Sequence
 
 import torch
 
@@ -800,16 +800,48 @@ def gemm_tile_add_rmsnorm(x: torch.Tensor, w: torch.Tensor, residual: torch.Tens
     return sum_add_rmsnorm(gemm_tile_sums(x, w), residual, norm_weight, eps)
 
 
-def rope_table(positions: torch.Tensor, inv_freq: torch.Tensor) -> torch.Tensor:
-    """Float32 [T, D / 2, 2]: cosines and sines of positions * inv_freq, as ``rope_store`` has them."""
-    _need_gpu(positions, inv_freq)
+ROPE_TABLES = 64        # tables of one launch (csrc/rope.hip)
+
+
+class RopeTables:
+    """The cosines and sines of a step's rows for n arrays of frequencies, on the GPU: ``address(i)`` is a place in its memory that
+    says where the table of array i, float32 [rows, half, 2], lies (equal arrays share one); as long as this object is there."""
+
+    def __init__(self, n: int, rows: int, half: int, device):
+        self.n, self.rows, self.half = n, rows, half
+        self.tables = torch.empty((n, rows, half, 2), dtype=torch.float32, device=device)
+        self.at = torch.empty(n, dtype=torch.int64, device=device)
+        self._at = self.at.data_ptr()
+
+    def address(self, i: int) -> int:
+        return self._at + 8 * i
+
+
+class RopeTable(NamedTuple):
+    """Table ``index`` of some."""
+    of: RopeTables
+    index: int
+
+
+def rope_tables(positions: torch.Tensor, inv_freqs: Sequence[torch.Tensor]) -> RopeTables:
+    """Cosines and sines of positions * inv_freq, as ``rope_store`` has them, for each of n arrays of frequencies of one size."""
+    _need_gpu(positions, *inv_freqs)
     _i32(positions, "positions")
-    if inv_freq.dtype != torch.float32 or inv_freq.dim() != 1 or not inv_freq.is_contiguous():
-        raise KernelError("rope_table: inv_freq must be contiguous float32 [D / 2]")
-    table = torch.empty((positions.numel(), inv_freq.numel(), 2), dtype=torch.float32, device=positions.device)
-    _check(library.load("rope").ptl_rope_table(_ptr(table), _ptr(positions), _ptr(inv_freq), positions.numel(),
-                                               inv_freq.numel(), _stream()), "rope_table")
-    return table
+    T, half = positions.numel(), inv_freqs[0].numel()
+    if any(f.dtype != torch.float32 or f.shape != (half,) or not f.is_contiguous() for f in inv_freqs):
+        raise KernelError("rope_tables: every inv_freq must be contiguous float32 [D / 2]")
+    made = RopeTables(len(inv_freqs), T, half, positions.device)
+    for i in range(0, made.n, ROPE_TABLES):
+        some = inv_freqs[i:i + ROPE_TABLES]
+        freqs = (ctypes.c_void_p * len(some))(*(f.data_ptr() for f in some))
+        _check(library.load("rope").ptl_rope_tables(_ptr(made.tables[i]), ctypes.c_void_p(made.address(i)), _ptr(positions), freqs,
+                                                    len(some), T, half, _stream()), "rope_tables")
+    return made
+
+
+def rope_table(positions: torch.Tensor, inv_freq: torch.Tensor) -> RopeTable:
+    """``rope_tables`` of one array of frequencies."""
+    return RopeTable(rope_tables(positions, [inv_freq]), 0)
 
 
 # q | k | v with rotation and cache write against the library's product and rope_store: as long as tiles of 128 x 192 all lie on the
@@ -826,7 +858,7 @@ def qkv_rope_store_tile_fits(x: torch.Tensor, w: torch.Tensor, head_dim: int) ->
             and x.shape[0] <= tile_most_rows_qkv(w.shape[0], compute_units(x.device)))
 
 
-def qkv_rope_store_tile(x: torch.Tensor, w: torch.Tensor, table: Optional[torch.Tensor], slots: Optional[torch.Tensor],
+def qkv_rope_store_tile(x: torch.Tensor, w: torch.Tensor, table: Optional[RopeTable], slots: Optional[torch.Tensor],
                         k_cache: Optional[torch.Tensor], v_cache: Optional[torch.Tensor], num_heads: int, num_kv_heads: int,
                         head_dim: int, page_size: int, tile: int = -1) -> torch.Tensor:
     """As ``qkv_rope_store``, for some hundred rows (csrc/gemm_tile.hip). ``table``: ``rope_table`` of the rows' positions, None: no
@@ -838,10 +870,9 @@ def qkv_rope_store_tile(x: torch.Tensor, w: torch.Tensor, table: Optional[torch.
     Hq, Hkv, D = num_heads, num_kv_heads, head_dim
     if w.shape[0] != (Hq + 2 * Hkv) * D:
         raise KernelError(f"qkv_rope_store_tile: weight has {w.shape[0]} rows, ({Hq} + 2*{Hkv}) * {D} expected")
-    _need_gpu(table, slots, k_cache, v_cache)
-    if table is not None and (table.dtype != torch.float32 or table.shape != (M, D // 2, 2) or not table.is_contiguous()
-                              or table.data_ptr() % 16):
-        raise KernelError(f"qkv_rope_store_tile: table must be contiguous float32 [{M}, {D // 2}, 2]")
+    _need_gpu(slots, k_cache, v_cache)
+    if table is not None and (table.of.rows, table.of.half) != (M, D // 2):
+        raise KernelError(f"qkv_rope_store_tile: the table is for {table.of.rows} rows of head size {2 * table.of.half}")
     if slots is not None:
         if slots.dtype != torch.int32 or slots.numel() != M or not slots.is_contiguous():
             raise KernelError("qkv_rope_store_tile: slots must be contiguous int32 [M]")
@@ -851,7 +882,8 @@ def qkv_rope_store_tile(x: torch.Tensor, w: torch.Tensor, table: Optional[torch.
                 raise KernelError(f"qkv_rope_store_tile: {name} must be contiguous bfloat16 [pages, {Hkv}, {page_size}, {D}]")
     q = torch.empty((M, Hq, D), dtype=torch.bfloat16, device=x.device)
     _check(library.load("gemm_tile").ptl_tile_qkv_rope_store(
-        _ptr(q), ctypes.c_long(Hq * D), _ptr(x), _ptr(w), M, K, ctypes.c_long(x.stride(0)), _ptr(table), _ptr(slots),
+        _ptr(q), ctypes.c_long(Hq * D), _ptr(x), _ptr(w), M, K, ctypes.c_long(x.stride(0)),
+        ctypes.c_void_p(table.of.address(table.index) if table is not None else 0), _ptr(slots),
         _ptr(k_cache), _ptr(v_cache), Hq, Hkv, D, int(page_size), int(tile), _stream()), "qkv_rope_store_tile")
     return q
 

@@ -97,15 +97,35 @@ class RotaryEncoding(Part):
     def rotary_inv_freq(self) -> Optional[torch.Tensor]:
         return self.inv_freq
 
-    def table(self, ctx) -> torch.Tensor:
-        """``ops.rope_table`` of the step's rows: one for all parts of the same frequencies in a model's pass over ``ctx``."""
+    def table(self, ctx) -> ops.RopeTable:
+        """``ops.rope_table`` of the step's rows; in a model's pass over ``ctx`` made once for all of its encodings."""
         if getattr(ctx, "rotations", None) is None:
             return ops.rope_table(ctx.positions, self.inv_freq)
-        key = self.inv_freq_host.numpy().tobytes()
-        if key not in ctx.rotations:
-            ctx.rotations[key] = ops.rope_table(ctx.positions, self.inv_freq)
-        return ctx.rotations[key]
+        return ctx.rotations.table(self, ctx.positions)
 
     def apply(self, q: torch.Tensor, k: torch.Tensor, positions: torch.Tensor) -> None:
         """Rotate q and k ([T, heads, D] views of one buffer) in place."""
         ops.rope_store(q, k, k, positions, self.inv_freq, None, None, None, 1, k_in_place=True)
+
+
+class Rotations:
+    """The cosines and sines of a step's rows for the rotary encodings of a model, while its forward runs: each from the
+    frequencies that its part has on the GPU then, all by one launch."""
+
+    def __init__(self, blocks):
+        self._blocks = blocks
+        self._made = {}
+
+    def table(self, encoding: RotaryEncoding, positions: torch.Tensor) -> ops.RopeTable:
+        if encoding not in self._made:
+            own = encoding.inv_freq
+            parts = {encoding: None}
+            for block in self._blocks:
+                part = getattr(getattr(block, "mixer", None), "position", None)
+                if type(part) is RotaryEncoding and part not in self._made and part.inv_freq is not None \
+                        and part.inv_freq.shape == own.shape and part.inv_freq.device == own.device:
+                    parts[part] = None
+            tables = ops.rope_tables(positions, [p.inv_freq for p in parts])
+            for i, part in enumerate(parts):
+                self._made[part] = ops.RopeTable(tables, i)
+        return self._made[encoding]

@@ -1405,6 +1405,27 @@ def test_qkv_rope_store_tile(ops, tile, Hq, Hkv, D):
         assert torch.equal(none, q)
 
 
+@pytest.mark.parametrize("n,rows,half", [(1, 1, 16), (3, 40, 32), (16, 277, 64), (65, 9, 16), (130, 3, 144)])
+def test_rope_tables(ops, n, rows, half):
+    """Cosines and sines for many arrays of frequencies, more than a launch takes among them: arrays of other bits (in the last
+    number, or a sign of zero) have tables of their own, equal ones share that of their launch's first."""
+    pos = torch.randint(0, 5000, (rows,), device="cuda").int()
+    base = (10000.0 ** (-torch.arange(half, device="cuda").double() / half)).float()
+    base[0] = 0.0
+    other, signed = base.clone(), base.clone()
+    other[-1] *= 0.5
+    signed[0] = -0.0
+    freqs = [{2: other, 5: signed, 64: other, 66: other}.get(i, base.clone()) for i in range(n)]
+    made = ops.rope_tables(pos, freqs)
+    at = [(a - made.tables.data_ptr()) // (8 * rows * half) for a in made.at.tolist()]
+    bits = lambda f: f.view(torch.int32).tolist()
+    first = [i // ops.ROPE_TABLES * ops.ROPE_TABLES for i in range(n)]
+    assert at == [first[i] if bits(freqs[i]) == bits(freqs[first[i]]) else i for i in range(n)]
+    for i in range(n):
+        angle = (pos[:, None].float() * freqs[i]).double()
+        torch.testing.assert_close(made.tables[at[i]].double(), torch.stack([angle.cos(), angle.sin()], 2), atol=3e-7, rtol=0)
+
+
 @pytest.mark.parametrize("value", [math.inf, -math.inf, math.nan])
 @pytest.mark.parametrize("turned", [False, True])
 @pytest.mark.parametrize("M", [37, 150])

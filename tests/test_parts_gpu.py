@@ -590,3 +590,41 @@ def test_rmsnorm_part_takes_any_width(gpu_device, dtype):
         torch.testing.assert_close(res.float().cpu(), wr.to(dtype).float(), atol=0, rtol=0)
         y0, _ = n.forward(x.cuda(), None)
         torch.testing.assert_close(y0.float().cpu(), plain_llama.rms_norm(x.float(), w, 1e-5), atol=tol, rtol=tol)
+
+
+def test_rotations_of_a_pass_are_its_own_and_each_part_s(gpu_device, monkeypatch):
+    """Steps whose products rotate by tables (from 33 rows on): one launch a pass makes those of all layers, from the frequencies
+    that a part has on the GPU (of one layer they were changed there), for the positions of this pass: prompts, then recorded
+    decode steps of 48 rows replayed at the next positions. The logits are those of the separate rotation."""
+    from pytriton_llama_amd import ops
+    from pytriton_llama_amd.config import build_model
+    from pytriton_llama_amd.engine.batch import StepEntry
+    from pytriton_llama_amd.engine.runner import ModelRunner
+    from pytriton_llama_amd.weights import load_random_weights
+    from tiny_configs import tiny
+    model = build_model(tiny("B")[0])
+    load_random_weights(model, 4, torch.bfloat16, gpu_device, norm_std=0.1, std=0.12)
+    g = torch.Generator().manual_seed(2)
+    seqs = [torch.randint(0, 384, (40 + i % 5 + 4,), generator=g).tolist() for i in range(48)]
+    made = []
+    tables = ops.rope_tables
+    monkeypatch.setattr(ops, "rope_tables", lambda positions, freqs: made.append(len(freqs)) or tables(positions, freqs))
+
+    def run():
+        runner = ModelRunner(model, 16, 48 * 4, 48, max_model_len=64, use_graphs=True)
+        out = [runner.step([StepEntry(i, s[:-4], [len(s) - 5]) for i, s in enumerate(seqs)]).float().cpu()]
+        for k in range(4):
+            out.append(runner.step([StepEntry(i, [s[len(s) - 4 + k]], [0]) for i, s in enumerate(seqs)]).float().cpu())
+        return torch.stack(out)
+
+    equal = run()
+    assert set(made) == {3} and len(made) == 3          # the prompts, the warm-up of the recorded step, the recording
+    own = model.blocks[1].mixer.position.inv_freq
+    own.mul_(0.25)
+    got = run()
+    monkeypatch.setattr(ops, "qkv_rope_store_tile_fits", lambda *args: False)
+    want = run()
+    apart = (got - want).norm() / want.norm()
+    assert apart < 1e-2 and (equal - want).norm() / want.norm() > 8e-2, (apart, (equal - want).norm() / want.norm())
+    own.mul_(4.0)
+    assert (equal - run()).norm() / equal.norm() < 1e-2
