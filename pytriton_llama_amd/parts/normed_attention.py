@@ -232,7 +232,8 @@ class NormedAttention(Part):
             blocks = ws.numel()
             ops.attention_prefill_mfma_kv(a, q, cache.k, cache.v, ctx.q_start, ctx.ctx_len, group.block_table,
                                           ws, wo, self.scale, self.maps, blocks if blocks <= 2 * t else t,
-                                          window, longest=0 if n_dec else max(ctx.q_lens), **extras)
+                                          window, longest=0 if n_dec else max(getattr(ctx, "q_lens", ()), default=0),
+                                          **extras)             # (0: not known, as in a context that has no lengths)
             return
         ws, wo = ctx.work[PORTIONS_16 if n_dec else ALL_16]
         ops.attention_generic_kv(a, q, cache.k, cache.v, ctx.q_start, ctx.ctx_len, group.block_table,

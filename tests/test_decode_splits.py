@@ -2,9 +2,12 @@
 from types import SimpleNamespace
 
 import pytest
+import torch
 
 from pytriton_llama_amd import ops
+from pytriton_llama_amd.parts import attention
 from pytriton_llama_amd.parts.attention import PagedAttention
+from pytriton_llama_amd.parts.normed_attention import NormedAttention
 
 
 def splits(rows, kv_heads, head_dim, longest, monkeypatch, window=None):
@@ -33,3 +36,18 @@ def test_about_one_workgroup_a_unit(rows, kv_heads, monkeypatch):
 def test_other_batches(rows, kv_heads, want, head_dim, monkeypatch):
     """Two workgroups a unit, none finer than a turn of 128 keys; one from 1.75 for each on."""
     assert splits(rows, kv_heads, head_dim, 4096, monkeypatch) == want
+
+
+@pytest.mark.parametrize("lengths,longest", [(dict(q_lens=[30, 300]), 300), (dict(q_lens=[]), 0), (dict(), 0)])
+def test_portions_of_a_context_without_lengths(lengths, longest, monkeypatch):
+    """The rows of the longest portion choose between two forms of the kernel: a context need not have them."""
+    monkeypatch.setattr(ops, "compute_units", lambda device: 256)
+    took = {}
+    monkeypatch.setattr(ops, "attention_prefill_mfma_kv", lambda *args, **kwargs: took.update(kwargs))
+    part = NormedAttention(256, 4, 2, 64, 64)
+    blocks = torch.zeros(6, dtype=torch.int32)
+    ctx = SimpleNamespace(num_decode_seqs=0, num_seqs=2, q_start=None, ctx_len=None, work={attention.PORTIONS_64: (blocks, blocks)},
+                          **lengths)
+    q = torch.zeros(330, 4, 64, dtype=torch.bfloat16)
+    part.attend(torch.empty_like(q), q, SimpleNamespace(k=None, v=None, page_size=16), ctx, SimpleNamespace(block_table=None))
+    assert took["longest"] == longest
