@@ -629,20 +629,35 @@ extern "C" int ptl_attention_decode(void* out, long out_stride, const void* q, l
 //
 // What bounds the kernel is the memory a compute unit keeps on its way (about 26 GB/s a unit in all, 17 one workgroup), so its
 // time is that of the unit with the most keys, and of the longest part. A pair has num_splits parts of one turn at least, and
-// more where they would be longer than ``piece`` keys (up to DECODE_MOST_PARTS): one of 3,000 keys beside 31 of 100, 8 kv heads
-// of 128, 2 splits 38.2 -> 29.2, 20 of 130 to 2,900 beside 12 empty rows 41.6 -> 33.4, but 32 of 300 to 3,000 48.1 -> 51.1 and, at
-// one split, 64 of 61 to 2,610 69.5 -> 79.9 with parts of at most 1,024 keys (hence 2,048 there); a part costs 4 to 7 us to begin and to end,
-// so shorter ones lose (64 of 61 to 2,610, 8 x 64, at most 1,536 / 1,024 / 512 / 256 keys 40 / 45 / 46 / 56). How a pair is
-// cut depends on its own keys and num_splits alone, so a sequence's bits do not depend on the others.
+// more where they would be longer than ``piece`` keys: the longest sequence of a batch otherwise decides the time of the
+// launch. How a pair is cut depends on its own keys and on the launch (num_splits, rows, heads) alone, so a sequence's bits do
+// not depend on the others; and so it cannot know whether it is an outlier or one of many equals, for which more parts are more work
+// (a part costs 4 to 7 us to begin and to end) and, where some lie above the line and some below, an uneven load.
+// Hence the lines (us; cut at 2,048 keys, at the line, not at all; 8 kv heads):
+//   one split (two workgroups a unit or about that: the batch fills the chip), 4,096. 64 of 2,062 keys of 64 54.5, 49.0, 49.0, of 128
+//   100, 92.7, 92.7; 61 to 2,610 39.1, 40.0, 40.0 and 69.0, 66.6, 66.6; 3,500 to 5,000 109, 114, 95.5 and 193, 213, 183 (at 8,192 as not
+//   at all); 64 of 4,500 105, 105, 99.5 and 200, 200, 194; 7,000 to 10,000 192, 192, 182 and 364, 364, 355; 61 to 8,000 100, 96, 108 and
+//   189, 191, 186; one of 8,000 beside 63 of 100 52.8, 52.5, 92.5 and 80, 80, 141 (16 parts 24.7 and 48: a workgroup more for each
+//   of the short ones then), 8 of 4,000 beside 56 of 300 34, 53, 53.
+//   two and three splits, sizes above 64, 1,024: 20 of 130 to 2,900 beside 12 empty rows 40.5, 32.4, 40.8; one of 3,000 beside 31 of 100
+//   37.7, 28.8, 37.7, of 8,000 47, 47, 80; 32 of 2,000 51.0, 50.7, 51.3, of 4,000 93.3, 96.3, 93.9, of 8,000 176, 176, 176; 32 of 130 to
+//   8,000 108, 110, 102.
+//   else 2,048: sizes up to 64, 32 of 130 to 8,000 51.9, not at all 54.7 (at 1,536 54.3), 32 of 8,000 93.2, 91.6, one of 8,000 beside 31 of
+//   100 29.3, 36.3; 8 of 16,384 49.6, 49.6 (at 1,536 55.8), 16 of 130 to 8,000 33.2, 33.3 (31.2); of 128 at four splits and more, 8 of 16,384
+//   93.9, 93.9 (at 1,024 101), 16 of 130 to 8,000 56.0, 55.8 (61.5).
+// And no pair has more parts than a launch of DECODE_MOST_GROUPS workgroups a unit has room for: the grid is made for the
+// longest context that the block table can hold, and workgroups without keys take their place in the queue. 64 of 300 keys, 8 kv heads of
+// 64, with a table of 131,072 tokens 19.3 -> 12.0, of 128 29.9 -> 18.7, 256 of 300 55 -> 31 and 96 -> 61, 32 of 100 to 500 15.3 -> 12.3
+// and 24.4 -> 18.1: as with a table of 4,096, and with a grid without those workgroups.
 // Where the contexts of 9 to 64 sequences differ by more than a quarter (each workgroup finds that out from ctx_len, a recorded step
 // does not know it) the parts of all pairs are one list, the longest first, every second turn of the units from the other
 // end: a unit's second workgroup is short where its first is long. Equal ones keep the grid's order (64 of 1,400, 8 x 64, 36.1
 // against 38.0 in the list).
-// Measured (one MI355X, us; with the second kernel and without the list in brackets): one of 45 keys, 8 x 64, 4.8 (6.7); one of
-// 2,048 8.2 (8.4); 8 of 2,048 12.2 (13.3); 8 of 100 to 1,000 8.5 (10.2); 16 of 500 9.6 (10.6); 64 of 61 to 2,610 41 (43); 20
-// of 130 to 2,900 beside 12 empty rows 21 (23), 8 x 128 33 (44); 32 of 2,000, 8 x 128, 53 (53); 48 of 300 to 3,000 37 (39),
-// 8 x 128 76 (72). Eight waves a workgroup instead of four: 64 of 1,400, 8 x 64, 36 -> 40. A persistent grid that walks the list
-// costs the start of every part again: 64 of 1,400 in two parts 42.7, one workgroup a part 41.6.
+// Measured (one MI355X, us; with the parts merged by a second kernel and without the list in brackets): one of 45 keys, 8 x 64, 4.8 (6.7);
+// one of 2,048 7.7 (8.7); 8 of 2,048 11.9 (12.7), of 300 7.0 (8.4); 16 of 2,000 18.1 (18.8); 64 of 61 to 2,610 40.1 (41.2), of 2,062 49.0
+// (50.6), 8 x 128 66.6 (68.0) and 92.7 (96.6); 20 of 130 to 2,900 beside 12 empty rows 20.3 (23.0), 8 x 128 32.4 (44.1); 32 of 2,000, 8 x
+// 128, 50.7 (52.5); 48 of 300 to 3,000 35.9 (39.0), 73.1 (72.3). Eight waves a workgroup instead of four: 64 of 1,400, 8 x 64, 36 -> 40. A
+// persistent grid that walks the list costs the start of every part again: 64 of 1,400 in two parts 42.7, one workgroup a part 41.6.
 //
 // A wave takes UNR tiles of 16 keys per turn and all query heads of a kv head at once (up to 16 of them
 // are the N side of the MFMA tiles, so grouped heads cost nothing extra):
@@ -706,12 +721,13 @@ static int launch_decode_mfma(void* out, long out_stride, const void* q, long q_
   return ptl_launch_status();
 }
 
-// The most parts a pair of at most ``keys`` keys has. Where they are more than one, ptl_attention_decode_mfma wants
-// n_seq * Hq * parts * (D + 2) floats of workspace and TICKET * n_seq * Hkv tickets.
-extern "C" int ptl_attention_decode_mfma_parts(int D, int num_splits, long keys, int piece) {
-  if (D <= 0 || num_splits < 1 || keys <= 0 || piece < 0) return 1;
-  if (piece == 0) piece = decode_piece(D, num_splits);
-  return max(num_splits, (int)min((keys + piece - 1) / piece, (long)DECODE_MOST_PARTS));
+// The most parts a pair of at most ``keys`` keys has, of n_seq * Hkv pairs. Where they are more than one, ptl_attention_decode_mfma
+// wants n_seq * Hq * parts * (D + 2) floats of workspace and TICKET * n_seq * Hkv tickets. piece: as there; the caller's own is
+// not limited by what the launch has room for.
+extern "C" int ptl_attention_decode_mfma_parts(int D, int num_splits, long keys, long pairs, int piece) {
+  if (D <= 0 || num_splits < 1 || keys <= 0 || pairs <= 0 || piece < 0) return 1;
+  if (piece > 0) return max(num_splits, (int)min((keys + piece - 1) / piece, (long)DECODE_MOST_PARTS));
+  return decode_most(D, num_splits, keys, pairs, compute_units());
 }
 
 // parts: floats of workspace for ``most`` parts a pair (ptl_attention_decode_mfma_parts for at least the keys of the longest

@@ -16,6 +16,7 @@ __device__ __forceinline__ void wave_lds_fence() {
 
 #define DECODE_LIST_SEQS 64        // sequences of a listed launch (one a lane)
 #define DECODE_MOST_PARTS 16       // parts that ``piece`` cuts a pair into at most
+#define DECODE_MOST_GROUPS 4       // ... as long as the launch has no more workgroups a compute unit than that
 
 // What parts of a pair the workgroups leave for the one that merges them.
 struct DecodeParts {
@@ -336,8 +337,14 @@ attn_decode_part(int block, Region region, const int32_t* __restrict__ ctx_len, 
 
 // Whether the parts of all pairs are one list.
 static bool decode_listed(int n_seq) { return n_seq > 8 && n_seq <= DECODE_LIST_SEQS; }
-// The keys beyond which a part is cut again (figures above).
-static int decode_piece(int D, int num_splits) { return D <= 64 ? 1536 : num_splits == 1 ? 2048 : 1024; }
+// The keys beyond which a part is cut again, and the most parts that a pair of at most ``keys`` keys then has (figures in
+// attention.hip).
+static int decode_piece(int D, int num_splits) { return num_splits == 1 ? 4096 : D > 64 && num_splits <= 3 ? 1024 : 2048; }
+static int decode_most(int D, int num_splits, long keys, long pairs, int cus) {
+  const int piece = decode_piece(D, num_splits);
+  const long cut = min((keys + piece - 1) / piece, (long)DECODE_MOST_PARTS);
+  return max(num_splits, (int)min(cut, (long)DECODE_MOST_GROUPS * cus / pairs));
+}
 // Workgroups of a launch with room for ``most`` parts a pair.
 static long decode_groups(int n_seq, int Hkv, int most, bool listed, int cus) {
   if (!listed) return (long)n_seq * Hkv * most;

@@ -1165,7 +1165,8 @@ def attention_decode(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor,
             keys = min(keys, window + keep_first)
         elif chunk:
             keys = min(keys, chunk)
-        most = lib.ptl_attention_decode_mfma_parts(D, int(num_splits), ctypes.c_long(max(1, keys)), int(piece))
+        most = lib.ptl_attention_decode_mfma_parts(D, int(num_splits), ctypes.c_long(max(1, keys)), ctypes.c_long(n_seq * Hkv),
+                                                   int(piece))
         parts = None
         if most > 1:
             parts = torch.empty(n_seq * Hq * most * (D + 2), dtype=torch.float32, device=q.device)
@@ -1311,7 +1312,8 @@ def attention_step(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor, v_
         keys = min(keys, window)
     elif chunk:
         keys = min(keys, chunk)
-    most = library.load("attention").ptl_attention_decode_mfma_parts(D, int(num_splits), ctypes.c_long(max(1, keys)), 0)
+    most = library.load("attention").ptl_attention_decode_mfma_parts(D, int(num_splits), ctypes.c_long(max(1, keys)),
+                                                                     ctypes.c_long(n_seq * Hkv), 0)
     parts = None
     if most > 1:
         parts = torch.empty(n_seq * Hq * most * (D + 2), dtype=torch.float32, device=q.device)

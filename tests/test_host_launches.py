@@ -115,3 +115,27 @@ def test_float32_decode_attention_by_its_workspaces(tmp_path, splits, acc, ml, t
     names = [k["kernel"] for k in took["launches"]]
     assert took["code"] == 0 and any("attn_f32_kernel" in n for n in names) == matrix_cores
     assert [any(part in n for n in names) for part in ("attn_decode_kernel", "attn_decode_merge_kernel")] == [not matrix_cores] * 2
+
+
+@pytest.mark.parametrize("rows,kv_heads,head_dim,splits", [(1, 8, 64, 32), (8, 8, 128, 8), (16, 8, 64, 4), (32, 8, 64, 3), (32, 8, 128, 2),
+                                                           (48, 8, 128, 2), (64, 8, 64, 1), (64, 8, 128, 1), (65, 8, 64, 1),
+                                                           (256, 8, 64, 1), (200, 32, 128, 1)])
+def test_decode_attention_is_not_launched_for_the_longest_table(tmp_path, rows, kv_heads, head_dim, splits):
+    """However long the contexts that a block table can hold: no more workgroups than four a compute unit, or than the splits
+    ask for; a table of short contexts has no parts beyond them; a piece of the caller's own is taken as it is."""
+    pairs = rows * kv_heads
+    keys = [128, 4096, 32768, 131072, 1 << 20]
+    parts = [t["code"] for t in run(tmp_path, "attention", [
+        (0, "ptl_attention_decode_mfma_parts", [*i(head_dim, splits), ("l", k), ("l", pairs), ("i", piece)])
+        for piece in (0, 128) for k in keys])]
+    assert parts[0] == splits and parts == sorted(parts[:5]) + parts[5:]
+    assert splits > 1 or parts[1] == 1              # (a batch that fills the chip is not cut up to 4,096 keys)
+    assert all(m == splits or m * pairs <= 4 * 256 for m in parts[:5]) and parts[4] <= max(splits, 16)
+    assert parts[5:] == [max(splits, m) for m in (1, 16, 16, 16, 16)]
+    took = run(tmp_path, "attention", [(0, "ptl_attention_decode_mfma", [
+        P, ("l", 4096), P, ("l", 4096), P, P, P, P, P, *i(8192), P, P, *i(most, rows, 2 * kv_heads, kv_heads, head_dim, 16), *EXTRAS,
+        *i(splits, 0, 0), NO]) for most in parts[:5]])
+    for most, t in zip(parts, took):
+        assert t["code"] == 0 and len(t["launches"]) == 1
+        # (a list of parts is in whole turns of eight and of the units)
+        assert rows * kv_heads * most <= t["launches"][0]["grid"][0] < pairs * most + 8 * kv_heads + 256
