@@ -139,3 +139,29 @@ def test_decode_attention_is_not_launched_for_the_longest_table(tmp_path, rows, 
         assert t["code"] == 0 and len(t["launches"]) == 1
         # (a list of parts is in whole turns of eight and of the units)
         assert rows * kv_heads * most <= t["launches"][0]["grid"][0] < pairs * most + 8 * kv_heads + 256
+
+
+@pytest.mark.parametrize("heads,head_dim,blocks,longest,two", [
+    (64, 64, 8, 0, True),              # 512 workgroups on 256 units
+    (65, 64, 8, 0, False),
+    (65, 64, 4, 0, False),             # four blocks: as likely short portions
+    (64, 64, 4, 0, True),              # ... which find a unit each
+    (64, 64, 4, 256, False),           # ... and are known to be short
+    (33, 32, 8, 512, True),
+    (33, 32, 8, 511, False),
+    (40, 128, 8, 450, True),           # a prompt by itself
+    (40, 96, 9, 450, True),            # ... with one more (empty, in a recorded step) block
+    (40, 128, 8, 321, False),          # with two more
+    (65, 128, 8, 450, False)])
+def test_prompt_attention_with_one_group_of_waves_or_two(tmp_path, heads, head_dim, blocks, longest, two):
+    """Both sides of the lines, for the entry of one head size and for the general one."""
+    step = [P, P, P, P, P, *i(40), P, P]
+    masks = [*EXTRAS, NO]
+    took = run(tmp_path, "attention_prefill", [
+        (0, "ptl_attention_prefill_mfma", [P, ("l", heads * head_dim), P, ("l", heads * head_dim), *step,
+                                           *i(blocks, blocks, 64, longest, heads, 1, head_dim, 16), *masks]),
+        (0, "ptl_attention_prefill_mfma_kv", [P, ("l", heads * head_dim), *i(0), P, ("l", heads * head_dim), *step,
+                                              *i(blocks, blocks, longest, heads, 1, 1, head_dim, head_dim, 16), *masks])])
+    for t in took:
+        assert t["code"] == 0 and len(t["launches"]) == 1 and t["launches"][0]["threads"] == (512 if two else 256)
+        assert t["launches"][0]["grid"][0] * t["launches"][0]["grid"][1] == heads * blocks
