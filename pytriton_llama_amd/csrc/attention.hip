@@ -633,18 +633,23 @@ extern "C" int ptl_attention_decode(void* out, long out_stride, const void* q, l
 // launch. How a pair is cut depends on its own keys and on the launch (num_splits, rows, heads) alone, so a sequence's bits do
 // not depend on the others; and so it cannot know whether it is an outlier or one of many equals, for which more parts are more work
 // (a part costs 4 to 7 us to begin and to end) and, where some lie above the line and some below, an uneven load.
-// Hence the lines (us; cut at 2,048 keys, at the line, not at all; 8 kv heads):
-//   one split (two workgroups a unit or about that: the batch fills the chip), 4,096. 64 of 2,062 keys of 64 54.5, 49.0, 49.0, of 128
-//   100, 92.7, 92.7; 61 to 2,610 39.1, 40.0, 40.0 and 69.0, 66.6, 66.6; 3,500 to 5,000 109, 114, 95.5 and 193, 213, 183 (at 8,192 as not
-//   at all); 64 of 4,500 105, 105, 99.5 and 200, 200, 194; 7,000 to 10,000 192, 192, 182 and 364, 364, 355; 61 to 8,000 100, 96, 108 and
-//   189, 191, 186; one of 8,000 beside 63 of 100 52.8, 52.5, 92.5 and 80, 80, 141 (16 parts 24.7 and 48: a workgroup more for each
-//   of the short ones then), 8 of 4,000 beside 56 of 300 34, 53, 53.
-//   two and three splits, sizes above 64, 1,024: 20 of 130 to 2,900 beside 12 empty rows 40.5, 32.4, 40.8; one of 3,000 beside 31 of 100
-//   37.7, 28.8, 37.7, of 8,000 47, 47, 80; 32 of 2,000 51.0, 50.7, 51.3, of 4,000 93.3, 96.3, 93.9, of 8,000 176, 176, 176; 32 of 130 to
-//   8,000 108, 110, 102.
-//   else 2,048: sizes up to 64, 32 of 130 to 8,000 51.9, not at all 54.7 (at 1,536 54.3), 32 of 8,000 93.2, 91.6, one of 8,000 beside 31 of
-//   100 29.3, 36.3; 8 of 16,384 49.6, 49.6 (at 1,536 55.8), 16 of 130 to 8,000 33.2, 33.3 (31.2); of 128 at four splits and more, 8 of 16,384
-//   93.9, 93.9 (at 1,024 101), 16 of 130 to 8,000 56.0, 55.8 (61.5).
+// Hence the lines (us, 8 kv heads of 64 and of 128): contexts that fill the chip with num_splits parts each lose 5 to 17 % just
+// beyond a line, so it lies where such batches are rare, and an outlier is cut as well as a later line allows.
+//   one split (two workgroups a unit or about that), 8,192; at 4,096, at the line, not at all: 64 of 3,500 to 5,000 keys 119, 100, 100 and 213,
+//   189, 183; of 4,500 110, 105, 101 and 205, 195, 195; 61 to 8,000 98.8, 109, 109 and 192, 186, 187; 7,000 to 10,000 201, 201, 186 and
+//   404, 404, 358; 61 to 16,000 184, 186, 209 and 354, 364, 362; one of 8,000 beside 63 of 100 53.1, 93.2, 93.1 and 81, 143, 143, of 16,000
+//   54.7, 96.3, 178 and 83, 148, 274. (At 2,048 64 of 2,062, a batch behind prompts of that length, took 54.5 for 49.0, 100 for 92.7.)
+//   two and three splits, 2,048 up to 64; at 2,048 and not at all: 32 of 130 to 8,000 51.9, 54.7, of 8,000 93.2, 91.6, of 6,200 78.3, 72.5;
+//   one of 8,000 beside 31 of 100 30.4, 37.2. Above 64 1,024; at 2,048, at the line, not at all: 20 of 130 to 2,900 beside 12 empty rows
+//   40.5, 32.4, 40.8; one of 3,000 beside 31 of 100 37.7, 28.8, 37.7, of 8,000 47, 47, 80; 32 of 2,000 51.0, 50.7, 51.3, of 2,100 54.5, 58.9,
+//   54.0, of 4,000 93.3, 96.3, 93.9, of 8,000 176, 176, 176; 32 of 130 to 4,300 60, 66, 60, to 8,000 108, 110, 102.
+//   four (16 requests), 3,072 up to 64 and 4,096 above; at 2,048, 3,072, 4,096, not at all: 16 of 8,300 58.9, 54.4, 52.4, 52.5 and 112, 103,
+//   103, 98.9; of 12,300 81.8, 81.5, 77.1, 77.3 and 153, 157, 141, 141; of 16,400 99.4, 98.7, 108, 99.7 and 186, 182, 200, 184; 130 to
+//   16,000 54.0, 53.6, 56.2, 56.4 and 111, 105, 101, 96.8; one of 16,000 beside 15 of 100 30.4, 37.4, 52.4, 52.4 and 48.7, 59.9, 82.6, 83.1,
+//   of 32,000 beside 15 of 2,000 59, 59, 59, 100 and 94, 94, 94, 160.
+//   more (up to 12 requests or so), not at all: a part is short beside the launch. At 2,048 and not at all: 8 of 16,400 56.2, 54.1 and 109, 98.1;
+//   of 20,000 69.9, 63.1 and 135, 115; of 32,800 101, 95.1 and 196, 183; 130 to 32,000 76.1, 70.6 and 148, 134; one of 32,000 beside 7 of
+//   100 68.5, 71.3 and 136, 135.
 // And no pair has more parts than a launch of DECODE_MOST_GROUPS workgroups a unit has room for: the grid is made for the
 // longest context that the block table can hold, and workgroups without keys take their place in the queue. 64 of 300 keys, 8 kv heads of
 // 64, with a table of 131,072 tokens 19.3 -> 12.0, of 128 29.9 -> 18.7, 256 of 300 55 -> 31 and 96 -> 61, 32 of 100 to 500 15.3 -> 12.3

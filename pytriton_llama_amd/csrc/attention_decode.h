@@ -339,7 +339,11 @@ attn_decode_part(int block, Region region, const int32_t* __restrict__ ctx_len, 
 static bool decode_listed(int n_seq) { return n_seq > 8 && n_seq <= DECODE_LIST_SEQS; }
 // The keys beyond which a part is cut again, and the most parts that a pair of at most ``keys`` keys then has (figures in
 // attention.hip).
-static int decode_piece(int D, int num_splits) { return num_splits == 1 ? 4096 : D > 64 && num_splits <= 3 ? 1024 : 2048; }
+static int decode_piece(int D, int num_splits) {
+  if (num_splits > 4) return 1 << 30;
+  if (num_splits == 4) return D > 64 ? 4096 : 3072;
+  return num_splits == 1 ? 8192 : D > 64 ? 1024 : 2048;
+}
 static int decode_most(int D, int num_splits, long keys, long pairs, int cus) {
   const int piece = decode_piece(D, num_splits);
   const long cut = min((keys + piece - 1) / piece, (long)DECODE_MOST_PARTS);

@@ -124,12 +124,14 @@ def test_decode_attention_is_not_launched_for_the_longest_table(tmp_path, rows, 
     """However long the contexts that a block table can hold: no more workgroups than four a compute unit, or than the splits
     ask for; a table of short contexts has no parts beyond them; a piece of the caller's own is taken as it is."""
     pairs = rows * kv_heads
-    keys = [128, 4096, 32768, 131072, 1 << 20]
+    keys = [128, 8192, 32768, 131072, 1 << 20]
     parts = [t["code"] for t in run(tmp_path, "attention", [
         (0, "ptl_attention_decode_mfma_parts", [*i(head_dim, splits), ("l", k), ("l", pairs), ("i", piece)])
         for piece in (0, 128) for k in keys])]
     assert parts[0] == splits and parts == sorted(parts[:5]) + parts[5:]
-    assert splits > 1 or parts[1] == 1              # (a batch that fills the chip is not cut up to 4,096 keys)
+    # a batch that fills the chip is not cut up to 8,192 keys, nor one whose requests have many parts
+    assert splits > 1 or parts[1] == 1
+    assert splits < 5 or parts[:5] == [splits] * 5
     assert all(m == splits or m * pairs <= 4 * 256 for m in parts[:5]) and parts[4] <= max(splits, 16)
     assert parts[5:] == [max(splits, m) for m in (1, 16, 16, 16, 16)]
     took = run(tmp_path, "attention", [(0, "ptl_attention_decode_mfma", [
