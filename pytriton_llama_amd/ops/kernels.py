@@ -715,14 +715,19 @@ def gemm_rows_add_rmsnorm(x: torch.Tensor, w: torch.Tensor, blocked: torch.Tenso
 # rows of W), us at 48 and 64 rows, those in brackets: 2,048 x 2,048 with norm 9.2, 9.6 (10.1, 10.8), 3,072 x 3,072 12.5, 13.4 (14.6,
 # 16.6), 4,096 x 4,096 15.3, 16.0 (15.2, 16.0); 2,048 x 8,192 14.3, 14.8 (14.9, 15.8), 3,072 x 8,192 18.0, 18.7 (21.5, 23.9), 4,096 x
 # 14,336 28.5, 29.3 (30.7, 32.7); q | k | v with rotation 3,072 x 2,048 9.6, 9.6 (11.3, 13.5), 5,120 x 3,072 13.8, 14.5 (16.2, 18.4), 6,144 x
-# 4,096 17.3, 18.1 (20.1, 22.3); at 32 rows level. Gate-up with SiLU 2 x 8,192 x 2,048 18.5, 18.9 (17.8, 19.6), 2 x 8,192 x 3,072 22.2,
-# 23.7 (24.5, 26.7), 2 x 14,336 x 4,096 50.1, 50.6 (53.6, 61.1).
+# 4,096 17.3, 18.1 (20.1, 22.3); at 32 rows level. Gate-up with SiLU at 33, 48 and 64 rows, W from HBM: 2 x 8,192 x 2,048 18.7, 18.9, 19.1
+# (18.4, 18.2, 20.3), 2 x 8,704 x 2,048 25.9, 26.3, 27.5 (28.8, 28.5, 34.8), 2 x 8,192 x 2,304 18.1, 18.9, 20.0 (22.1, 21.7, 23.7),
+# 2 x 9,728 x 2,048 25.9, 26.9, 27.4 (29.3, 28.9, 35.1), 2 x 7,168 x 3,072 21.5, 23.3, 23.5 (26.0, 25.6, 26.2), 2 x 8,192 x 3,072 23.1, 24.1,
+# 24.5 (26.8, 26.2, 27.5), 2 x 6,144 x 4,096 24.6, 25.8, 27.7 (29.3, 29.0, 31.5), 2 x 14,336 x 4,096 at 48 and 64 50.1, 50.6 (53.6, 61.1): the
+# line lies on the one matrix of them where the other kernel is level or ahead up to 48 rows. Smaller ones, below the line, would
+# take the tiles 3 to 15 % faster there too (2 x 7,168 x 2,048 17.0, 17.4 against 18.2, 17.8, 2 x 5,632 x 2,048 14.4, 15.0 against 16.9, 16.6,
+# 2 x 4,096 x 1,024 8.7, 9.0 against 10.3, 9.9).
 TILE_MIN_ROWS = 33
 
 
 def tile_least_rows_gate_up(rows_w: int, K: int) -> int:
     """Rows from which ``gate_up_tile`` is the faster way for w [rows_w, K]."""
-    return TILE_MIN_ROWS if rows_w * K >= 3 << 24 else 49
+    return TILE_MIN_ROWS if rows_w * K > 1 << 25 else 49
 
 
 def tile_most_rows_sums(N: int, K: int) -> int:

@@ -27,7 +27,8 @@ def test_qkv(rows_w, most):
     assert ops.tile_most_rows_qkv(rows_w, 256) == most
 
 
-@pytest.mark.parametrize("I,K,least", [(8192, 2048, 49), (8192, 3072, 33), (14336, 4096, 33), (5632, 2048, 49)])
+@pytest.mark.parametrize("I,K,least", [(8192, 2048, 49), (8192, 3072, 33), (14336, 4096, 33), (5632, 2048, 49), (8704, 2048, 33),
+                                       (8192, 2304, 33), (7168, 3072, 33), (9728, 2048, 33)])
 def test_gate_up_from(I, K, least):
-    """Below, the kernel for tens of rows was faster."""
+    """Matrices up to that of 2 x 8,192 x 2,048, where the kernel for tens of rows is the faster one below, and larger ones."""
     assert ops.tile_least_rows_gate_up(2 * I, K) == least
